@@ -17,15 +17,15 @@
     X(gemm_pp64, 1, "1: whole-line ping-pong kernel (gemm_tn_pp64_kernel); 0: the 32-wide K-tile body it replaced")         \
     X(gemm_tall, 1, "whole-line kernel: 1 a ragged column block of <= 128 columns as 384x128 tiles (round 6), 0 as padded 256x256 tiles") \
     X(gemm_even_grid, 0, "whole-line kernel: 1 the fewest persistent workgroups that keep the round count (every workgroup the same number of tiles), 0 always 256") \
-    X(gemm_pingpong, 1, "0: never take a ping-pong kernel (256x128 ring / 128x128 kernels only)")                          \
-    X(gemm_small, 0, "1: always the 128x128 kernel")                                                                        \
+    X(gemm_pingpong, 1, "0: never take a ping-pong kernel (mid-size kernel only)")                          \
+    X(gemm_small, 0, "1: fp32 always through the 128x128 kernel")                                                                        \
     X(gemm_wgs, 256, "persistent workgroups of the 256x128 ring kernel (0: one tile per workgroup)")                        \
     X(gemm_pad_pct, 112, "ping-pong kernel is taken while N padded to 256 <= this percentage of N")                         \
     X(gemm_rope_lut, 1, "K-tile body only: rotary factors from the LDS position LUT when the caller supplies one")          \
     X(gemm_group_m, 0, "> 0: row blocks per group of the ping-pong tile walk (0: chosen per shape)")                        \
+    X(gemm_mid, 0, "> 0: this tile size of the mid-size kernel for every bf16 product of two or more rows (0: chosen per shape)") \
     X(gemm_split, 1, "0: no round-aligned / few-tile split of a launch")                                                    \
-    X(gemm_co_streams, 0, "> 0: overrides the co-running-streams hint of the few-tile choice")                              \
-    X(gemm_ring_cost_permille, 720, "few-tile choice: cost of a round of ring tiles relative to a round of ping-pong tiles") \
+    X(gemm_co_streams, 0, "> 0: overrides the co-running-streams hint of the many-tile split")                              \
     X(gemm_epi_serial, 0, "1: the two wave groups' epilogues in separate intervals (the order before round 4)")             \
     X(gemm_nostore, 0, "1: timing only -- K loops without epilogues (results are NOT written)")                             \
     X(gemm_trace, 0, "1: per-tile s_memtime stamps of workgroup 0 printed to stderr (synchronises)")                        \
@@ -60,7 +60,7 @@ struct CogsDebug {
     COGS_DEBUG_SWITCHES(COGS_DBG_FIELD)
 #undef COGS_DBG_FIELD
     // read-only reports (cogs_debug_get): what the last cogs_gemm of this process dispatched to
-    // 0 none yet, 1 128x128, 2 256x128 ring, 3 K-tile ping-pong, 4 whole-line ping-pong, 5 ping-pong + ring (split), 6 GEMV, 7 few-row GEMM
+    // 0 none yet, 1 128x128 (fp32), 2 mid-size (fp32: 256x128), 3 K-tile ping-pong, 4 whole-line ping-pong, 5 ping-pong + mid-size (split), 6 GEMV, 7 few-row GEMM
     std::atomic<long long> gemm_last_body{0};
     // ... and the last cogs_attention: 1 general MFMA kernel, 2 ViT unpipelined, 3 ViT pipelined (row-major K/V), 4 single-token
     // decode (+ combine), 5 prompt LDS-DMA kernel, 7 row-wise fp32 kernel, 8 ViT pipelined, head-major K/V (6 and 9 were the archived

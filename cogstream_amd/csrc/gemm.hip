@@ -8,20 +8,19 @@
 //   model/cogreasoner_chat.py:179-211 (projector); the Qwen2 linears of
 //   transformers' modeling_qwen2 (q/k/v(+bias), o, gate/up, down, lm_head).
 //
-// Design (gfx950):
-//   * 128x128 output tile per 256-thread workgroup (4 waves as 2x2, 64x64 per wave,
-//     4x4 MFMA tiles of 16x16), 128-byte K slab per step (64 bf16 / 32 fp32).
-//   * both operands staged HBM->LDS by direct LDS-DMA (global_load_lds_dwordx4),
-//     two LDS buffers; the LDS image is lane-linear, the XOR swizzle lives on the
-//     per-lane SOURCE address and on the ds_read address (chunk ^= row&7), which
-//     makes every ds_read_b128 fragment read conflict free.
+// This file has the ping-pong kernels of large bf16 products, the fp32 kernels of the parity mode and the choice among all bodies;
+// gemm_mid.hip has the tiles of mid-size bf16 products, gemv.hip the single row.
+//
+// Common to the tiled kernels (gfx950):
+//   * both operands staged HBM->LDS by direct LDS-DMA (global_load_lds_dwordx4) as 128-byte rows (64 bf16 / 32 fp32 of K);
+//     the LDS image is lane-linear, the XOR swizzle lives on the per-lane SOURCE address and on the ds_read address
+//     (chunk ^= row&7), which makes every ds_read_b128 fragment read conflict free.
 //   * weights are the MFMA A operand, activations the B operand, so that a lane ends
 //     up holding 4 CONSECUTIVE output columns of one row: bias / residual / rope /
 //     swiglu epilogues and the 8-byte stores are all lane-local.
-//   * the fp32 instantiation (parity mode) keeps the same byte layout and uses the
-//     exact-f32 MFMA (v_mfma_f32_16x16x4_f32).
 //   * blocks are remapped XCD-aware (bijective) and walked in groups of 8 row tiles
 //     so that co-resident blocks of one XCD share A/W panels in its L2.
+// fp32 keeps the same byte layout and uses the exact-f32 MFMA (v_mfma_f32_16x16x4_f32).
 #include "common.h"
 #include "kernels.h"
 #include "gemm_epilogue.h"
@@ -36,9 +35,7 @@ constexpr int ROW_BYTES = 128;               // one tile row of the K slab
 constexpr int TILE_BYTES = BM * ROW_BYTES;   // 16 KiB per operand per buffer
 constexpr int GROUP_M = 8;
 
-template <typename T> struct ElemCfg;
-template <> struct ElemCfg<bf16_t> { static constexpr int BK = 64; };
-template <> struct ElemCfg<float> { static constexpr int BK = 32; };
+constexpr int BK32 = 32;                     // K slab of the fp32 kernels: 128 bytes
 
 struct GemmArgs {
     const char* A; long lda;   // bytes per row
@@ -59,10 +56,10 @@ __device__ __forceinline__ void glds16(const char* g, char* l) {
                                      (__attribute__((address_space(3))) void*)l, 16, 0, 0);
 }
 
-template <typename T, int EPI>
+template <int EPI>
 __global__ __launch_bounds__(256, 2) void gemm_tn_kernel(GemmArgs p) {
     extern __shared__ __attribute__((aligned(16))) char smem[];
-    constexpr int BK = ElemCfg<T>::BK;
+    typedef float T;
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -110,7 +107,7 @@ __global__ __launch_bounds__(256, 2) void gemm_tn_kernel(GemmArgs p) {
 #pragma unroll
         for (int j = 0; j < 4; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-    const int KT = p.K / BK;
+    const int KT = p.K / BK32;
 
     // fragment sets are register double buffered (see the 256x128 kernel below for the TOUCH rationale)
     u32x4 af[2][4], wf[2][4];
@@ -124,25 +121,15 @@ __global__ __launch_bounds__(256, 2) void gemm_tn_kernel(GemmArgs p) {
         }
     };
     auto mma = [&](int set) {
-        if constexpr (sizeof(T) == 2) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
 #pragma unroll
             for (int mi = 0; mi < 4; ++mi)
 #pragma unroll
                 for (int ni = 0; ni < 4; ++ni)
-                    acc[mi][ni] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-                        __builtin_bit_cast(bf16x8, wf[set][ni]), __builtin_bit_cast(bf16x8, af[set][mi]),
+                    acc[mi][ni] = __builtin_amdgcn_mfma_f32_16x16x4f32(
+                        __uint_as_float(wf[set][ni][e]), __uint_as_float(af[set][mi][e]),
                         acc[mi][ni], 0, 0, 0);
-        } else {
-#pragma unroll
-            for (int e = 0; e < 4; ++e)
-#pragma unroll
-                for (int mi = 0; mi < 4; ++mi)
-#pragma unroll
-                    for (int ni = 0; ni < 4; ++ni)
-                        acc[mi][ni] = __builtin_amdgcn_mfma_f32_16x16x4f32(
-                            __uint_as_float(wf[set][ni][e]), __uint_as_float(af[set][mi][e]),
-                            acc[mi][ni], 0, 0, 0);
-        }
     };
 #define COGS_TOUCH1(S)                                                                                       \
     asm volatile("" : "+v"(af[S][0]), "+v"(af[S][1]), "+v"(af[S][2]), "+v"(af[S][3]), "+v"(wf[S][0]), \
@@ -188,7 +175,7 @@ __global__ __launch_bounds__(256, 2) void gemm_tn_kernel(GemmArgs p) {
 
 
 // ---------------------------------------------------------------------------------------------
-// Large-M variant: 256x128 output tile, 8 waves (4x2, 64x64 each), 3-deep LDS ring (3 x 48 KiB),
+// fp32, 512 rows and more: 256x128 output tile, 8 waves (4x2, 64x64 each), 3-deep LDS ring (3 x 48 KiB),
 // LDS-DMA prefetch two K slabs ahead that stays in flight ACROSS the barrier: one raw s_barrier per
 // K step, counted s_waitcnt vmcnt(6) (= the 6 pieces of the next slab may still be in flight), all
 // LDS in one array (guide section 5, "Pipelining across barriers"). One workgroup per CU.
@@ -197,16 +184,16 @@ constexpr int SLAB2 = (BM2 + BN) * ROW_BYTES;   // 48 KiB per K slab (A 32 KiB t
 constexpr int PIECES2 = SLAB2 / 1024 / 8;       // 6 LDS-DMA pieces per wave per slab
 constexpr int PERSISTENT_WGS = 256;             // one workgroup per CU (MI355X: 256 CUs)
 
-template <typename T, int EPI>
+template <int EPI>
 __global__ __launch_bounds__(512, 2) void gemm_tn_256x128_kernel(GemmArgs p) {
     extern __shared__ __attribute__((aligned(16))) char smem[];
-    constexpr int BK = ElemCfg<T>::BK;
+    typedef float T;
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wm = wid >> 1, wn = wid & 1;
     const int nb = p.nbm * p.nbn;
-    const int KT = p.K / BK;
+    const int KT = p.K / BK32;
 
     // PERSISTENT: this workgroup walks tiles t = blockIdx.x, +gridDim.x, ... of the XCD-aware order; the
     // K-slab ring runs continuously ACROSS tiles, so the next tile's first slabs stream in while the
@@ -273,25 +260,15 @@ __global__ __launch_bounds__(512, 2) void gemm_tn_256x128_kernel(GemmArgs p) {
         }
     };
     auto mma = [&](int set) {
-        if constexpr (sizeof(T) == 2) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
 #pragma unroll
             for (int mi = 0; mi < 4; ++mi)
 #pragma unroll
                 for (int ni = 0; ni < 4; ++ni)
-                    acc[mi][ni] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-                        __builtin_bit_cast(bf16x8, wf[set][ni]), __builtin_bit_cast(bf16x8, af[set][mi]),
+                    acc[mi][ni] = __builtin_amdgcn_mfma_f32_16x16x4f32(
+                        __uint_as_float(wf[set][ni][e]), __uint_as_float(af[set][mi][e]),
                         acc[mi][ni], 0, 0, 0);
-        } else {
-#pragma unroll
-            for (int e = 0; e < 4; ++e)
-#pragma unroll
-                for (int mi = 0; mi < 4; ++mi)
-#pragma unroll
-                    for (int ni = 0; ni < 4; ++ni)
-                        acc[mi][ni] = __builtin_amdgcn_mfma_f32_16x16x4f32(
-                            __uint_as_float(wf[set][ni][e]), __uint_as_float(af[set][mi][e]),
-                            acc[mi][ni], 0, 0, 0);
-        }
     };
     // TOUCH(set): makes the compiler place its wait for that fragment set HERE (before newer ds_reads are
     // issued): hipcc cannot count lgkmcnt across the loop back-edge and would otherwise wait lgkmcnt(0) right
@@ -312,7 +289,6 @@ __global__ __launch_bounds__(512, 2) void gemm_tn_256x128_kernel(GemmArgs p) {
     asm volatile("" ::: "memory");
     load_frags(0, 0, 0);
     int buf = 0;
-    int epi_stores = 0;   // store instructions the previous tile's epilogue left in flight
 
     for (int t = blockIdx.x; t < nb; t += gridDim.x) {
         int m0, n0;
@@ -334,11 +310,8 @@ __global__ __launch_bounds__(512, 2) void gemm_tn_256x128_kernel(GemmArgs p) {
                 // the next slab must have landed (own pieces: counted vmcnt -- at most the 6 pieces of the slab
                 // after it may stay in flight; everyone's: barrier); after the barrier nobody reads the current
                 // slab any more, so its ring slot is restaged
-                // the 8 stores of the previous tile's (wide, interior) epilogue are newer than the pieces this wait is
-                // about for the first two slabs of a tile: leave them in flight (see the ping-pong kernel)
-                const bool relaxed = epi_stores == 8 && kt < 2;
-                if (staged > 1) { if (relaxed) asm volatile("s_waitcnt vmcnt(14)" ::: "memory"); else asm volatile("s_waitcnt vmcnt(6)" ::: "memory"); }
-                else { if (relaxed) asm volatile("s_waitcnt vmcnt(8)" ::: "memory"); else asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
+                if (staged > 1) asm volatile("s_waitcnt vmcnt(6)" ::: "memory");
+                else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
                 __builtin_amdgcn_s_barrier();
                 asm volatile("" ::: "memory");
                 staged += stage_next(buf) ? 1 : 0;
@@ -350,8 +323,6 @@ __global__ __launch_bounds__(512, 2) void gemm_tn_256x128_kernel(GemmArgs p) {
             buf = nbuf;
         }
         epilogue_wave<T, EPI>(p.epi, m0 + wm * 64, n0 + wn * 64, p.M, p.N, lane, acc);
-        epi_stores = (sizeof(T) == 2 && (EPI & (EPI_SWIGLU | EPI_F32OUT | EPI_GENERIC | EPI_NOSTORE)) == 0 &&
-                      (p.N & 31) == 0 && m0 + BM2 <= p.M && n0 + BN <= p.N) ? 8 : 0;
     }
 #undef COGS_TOUCH
 }
@@ -956,8 +927,7 @@ __global__ __launch_bounds__(512, 2) void gemm_tn_pp64_kernel(GemmArgs p) {
 // report per-KERNEL averages that can be compared with rocprofv3's kernel stats
 static thread_local long g_gemm_launches = 0;
 // how many streams the caller is feeding with GEMMs of this size at the same time (cogs_vit_encode's two-stream mode: 2).
-// Only the few-tile choice below reads it: with a second stream filling the CUs a launch leaves idle, a partly filled
-// round costs its share of the chip, not a whole round.
+// Only the many-tile split below reads it: a second stream fills the CUs that a launch's last round leaves idle.
 static thread_local int g_co_streams = 1;
 void cogs_k_gemm_co_streams(int streams) { g_co_streams = streams < 1 ? 1 : streams; }
 long cogs_k_gemm_launch_count() { return g_gemm_launches; }
@@ -966,25 +936,25 @@ int cogs_k_gemv(hipStream_t st, const CogsGemm& g);
 
 namespace {
 
-template <typename T, int EPI>
+template <int EPI>
 void launch_small(hipStream_t st, const GemmArgs& p, int grid) {
     const size_t lds = 4 * TILE_BYTES;
     static std::atomic<uint64_t> attr_done{0};
-    cogs_ensure_dyn_lds((const void*)gemm_tn_kernel<T, EPI>, (int)lds, attr_done);
+    cogs_ensure_dyn_lds((const void*)gemm_tn_kernel<EPI>, (int)lds, attr_done);
     ++g_gemm_launches;
     g_cogs_debug.gemm_last_body = 1;
-    hipLaunchKernelGGL((gemm_tn_kernel<T, EPI>), dim3(grid), dim3(256), lds, st, p);
+    hipLaunchKernelGGL((gemm_tn_kernel<EPI>), dim3(grid), dim3(256), lds, st, p);
 }
-template <typename T, int EPI>
+template <int EPI>
 void launch_big(hipStream_t st, const GemmArgs& p, int grid) {
     const size_t lds = 3 * SLAB2;
     static std::atomic<uint64_t> attr_done{0};
-    cogs_ensure_dyn_lds((const void*)gemm_tn_256x128_kernel<T, EPI>, (int)lds, attr_done);
+    cogs_ensure_dyn_lds((const void*)gemm_tn_256x128_kernel<EPI>, (int)lds, attr_done);
     const int dbg_wgs = (int)g_cogs_debug.gemm_wgs;
     const int wgs = dbg_wgs <= 0 ? grid : (grid < dbg_wgs ? grid : dbg_wgs);   // 0 = one tile per workgroup
     ++g_gemm_launches;
     g_cogs_debug.gemm_last_body = 2;
-    hipLaunchKernelGGL((gemm_tn_256x128_kernel<T, EPI>), dim3(wgs), dim3(512), lds, st, p);
+    hipLaunchKernelGGL((gemm_tn_256x128_kernel<EPI>), dim3(wgs), dim3(512), lds, st, p);
 }
 // debug switch gemm_pp64 = 0 keeps the 32-wide K-tile kernel (A/B runs); default: the whole-line kernel wherever it exists
 // (every epilogue but the rotary LUT one, for which it has no LDS left -- cogs_k_gemm then takes the rotary factors from
@@ -1096,10 +1066,9 @@ void dispatch_pp(hipStream_t st, const GemmArgs& p, int grid, int mask) {
 #undef COGS_PP_CASE
 }
 
-template <typename T>
-void dispatch(hipStream_t st, const GemmArgs& p, int grid, int mask, bool big) {
+void dispatch_f32(hipStream_t st, const GemmArgs& p, int grid, int mask, bool big) {
 #define COGS_EPI_CASE(E) \
-    case E: if (big) launch_big<T, E>(st, p, grid); else launch_small<T, E>(st, p, grid); break;
+    case E: if (big) launch_big<E>(st, p, grid); else launch_small<E>(st, p, grid); break;
     switch (mask) {
         COGS_EPI_CASE(0)
         COGS_EPI_CASE(EPI_BIAS)
@@ -1120,12 +1089,44 @@ void dispatch(hipStream_t st, const GemmArgs& p, int grid, int mask, bool big) {
         COGS_EPI_CASE(EPI_SWIGLU | EPI_BIAS)
         COGS_EPI_CASE(EPI_GELU_ERF)
         COGS_EPI_CASE(EPI_F32OUT)
-        default: if (big) launch_big<T, EPI_GENERIC>(st, p, grid); else launch_small<T, EPI_GENERIC>(st, p, grid); break;
+        default: if (big) launch_big<EPI_GENERIC>(st, p, grid); else launch_small<EPI_GENERIC>(st, p, grid); break;
     }
 #undef COGS_EPI_CASE
 }
 
 }  // namespace
+
+// ---- which kernel a bf16 product of two or more rows gets -------------------------------------------------------------------
+// All of them walk K in the same order, so the choice is by time alone. Time of a launch = rounds of tiles over the chip x (slabs x
+// time of a slab + the rest of a tile: prologue, epilogue), with a slab's time measured per tile size for one and, where the LDS
+// has room for them, two workgroups on a CU (MI355X, weights from HBM, K = 1152 .. 18 944; the sums below are within 15 % of every
+// shape that was measured). The small tiles are bound by a slab's LDS traffic and barrier, not by MFMAs: they pay while the
+// larger ones leave CUs without a tile.
+struct TileCost { int tile, tm, tn; float one, two, rest; };     // us; two = 0: one workgroup per CU
+static constexpr TileCost MID_TILES[] = {
+    {1, 32, 64, 0.22f, 0.36f, 2.5f}, {2, 64, 64, 0.26f, 0.48f, 2.5f}, {3, 128, 64, 0.38f, 0.71f, 2.5f},
+    {4, 128, 128, 0.55f, 0.f, 3.f},  {5, 128, 256, 0.85f, 0.f, 4.f}};
+static constexpr float PP_SLAB = 1.13f, PP_REST = 8.f, SECOND_LAUNCH = 2.f;
+
+static float tile_time(int tiles, int slabs, float one, float two, float rest) {
+    const float t1 = slabs * one + rest, t2 = slabs * two + rest;
+    if (two == 0.f) return (float)((tiles + PERSISTENT_WGS - 1) / PERSISTENT_WGS) * t1;
+    const int full = tiles / (2 * PERSISTENT_WGS), left = tiles % (2 * PERSISTENT_WGS);
+    return full * t2 + (left == 0 ? 0.f : left <= PERSISTENT_WGS ? t1 : t2);
+}
+static int best_mid_tile(int M, int N, int K, float* time) {
+    int best = 0;
+    for (const TileCost& t : MID_TILES) {
+        const float c = tile_time((M + t.tm - 1) / t.tm * ((N + t.tn - 1) / t.tn), K / 64, t.one, t.two, t.rest);
+        if (best == 0 || c < *time) { best = t.tile; *time = c; }
+    }
+    return best;
+}
+static int launch_mid(hipStream_t st, const CogsGemm& g, int tile) {
+    ++g_gemm_launches;
+    g_cogs_debug.gemm_last_body = 2;
+    return cogs_k_gemm_mid(st, g, tile);
+}
 
 int cogs_k_gemm(hipStream_t st, const CogsGemm& g) {
     const int es = g.dtype == COGS_DT_BF16 ? 2 : 4;
@@ -1139,6 +1140,16 @@ int cogs_k_gemm(hipStream_t st, const CogsGemm& g) {
     if (g.hm_rows > 0 && (g.M == 1 || g.dtype != COGS_DT_BF16)) return COGS_E_UNSUPPORTED;       // head-major output: bf16 MFMA kernels only
     if (g.M == 1) { ++g_gemm_launches; g_cogs_debug.gemm_last_body = 6; return cogs_k_gemv(st, g); }
     if (g.rms_gamma) return COGS_E_UNSUPPORTED;   // fused RMSNorm exists for the single-token GEMV only
+    const int env_co = (int)g_cogs_debug.gemm_co_streams;   // A/B runs
+    const int S = env_co > 0 ? env_co : g_co_streams;
+    float mid_time = 0.f;
+    const int env_mid = (int)g_cogs_debug.gemm_mid;
+    const int mid = g.dtype != COGS_DT_BF16 ? 0 : env_mid > 0 ? env_mid : best_mid_tile(g.M, g.N, g.K, &mid_time);
+    const int n_pad = (g.N + BN3 - 1) / BN3 * BN3;
+    const bool pp_fits = n_pad * 100 <= g.N * (int)g_cogs_debug.gemm_pad_pct;   // default: <= 12 % of the MFMAs spent on N padding
+    // (the ping-pong kernel wants two slabs and, below a row block, wastes its tiles' rows)
+    const bool pp = mid > 0 && env_mid == 0 && g_cogs_debug.gemm_pingpong != 0 && pp_fits && g.K >= 128 && g.M >= 256 && !g.force_mid_tile;
+    if (mid > 0 && !pp) return launch_mid(st, g, mid);
     GemmArgs p;
     p.trace = nullptr; p.rope_lut = nullptr; p.rope_lut_bytes = 0; p.group_m = GROUP_M;
     p.epi_serial = (int)g_cogs_debug.gemm_epi_serial;
@@ -1147,13 +1158,7 @@ int cogs_k_gemm(hipStream_t st, const CogsGemm& g) {
     p.A = (const char*)g.A; p.lda = g.lda * es;
     p.W = (const char*)g.W; p.ldw = g.ldw * es;
     p.M = g.M; p.N = g.N; p.K = g.K;
-    const bool env_small = g_cogs_debug.gemm_small != 0;
-    const bool env_nopp = g_cogs_debug.gemm_pingpong == 0;
-    const int n_pad = (g.N + BN3 - 1) / BN3 * BN3;
-    const int env_waste = (int)g_cogs_debug.gemm_pad_pct;
-    const bool pp_fits = n_pad * 100 <= g.N * env_waste;   // default: <= 12 % of the MFMAs spent on N padding (N = 1152 -> 1280 measured faster than the 256x128 ring kernel)
-    if (!env_nopp && !env_small && g.dtype == COGS_DT_BF16 && g.M >= 1024 && pp_fits && !g.force_small_tile &&
-        !g.force_mid_tile) {
+    if (pp) {
         p.nbm = (g.M + BM3 - 1) / BM3;
         p.nbn = (g.N + BN3 - 1) / BN3;
         const bool env_nostore = g_cogs_debug.gemm_nostore != 0;
@@ -1196,49 +1201,33 @@ int cogs_k_gemm(hipStream_t st, const CogsGemm& g) {
         }
         // Round-aligned split. The persistent kernel walks nbm*nbn tiles with 256 workgroups; when the last round
         // is mostly empty (N = 1152 at cfg2: 1155 tiles = 4.5 rounds, half the CUs idle for a whole tile time) the
-        // leading row blocks that make up WHOLE rounds stay here and the remaining rows go to the 256x128 kernel,
-        // whose half-size tiles fill the chip again (rows are independent: same arithmetic per row, same K order, so
+        // leading row blocks that make up WHOLE rounds stay here and the remaining rows go to the mid-size kernel,
+        // whose smaller tiles fill the chip again (rows are independent: same arithmetic per row, same K order, so
         // a row's result does not depend on which kernel computed it).
         const bool env_nosplit = g_cogs_debug.gemm_split == 0;
         const int nb = count_tiles(g.M);
         p.ntiles = nb;
         const int rounds = nb / PERSISTENT_WGS, rem = nb % PERSISTENT_WGS;
-        int mb_main = -1;      // >= 0: row blocks that stay in this kernel (0 = none: the whole GEMM goes to the ring kernel)
-        // (calibrated on K = 1152 .. 4352, the ViT shapes; longer K -- the Qwen2 prompt pass at M = 2048 -- keeps the
-        // plain ping-pong launch)
-        const int env_co = (int)g_cogs_debug.gemm_co_streams;   // A/B runs
-        const int S = env_co > 0 ? env_co : g_co_streams;
-        if (!env_nosplit && !env_nostore && nb <= 2 * PERSISTENT_WGS && g.K <= 4352) {
-            // Few tiles (one rank's share of a frame-sharded clip: M = 6 400 is 125 tiles for N = 1152 and 350 = 1.37
-            // rounds for QKV): the time is rounds x one tile, so the choice is by rounds. Calibrated on the four ViT
-            // shapes at M = 3 200 .. 14 784 (tools/cal_tiles.sh, rocprofv3; round 4 with the whole-line kernel,
-            // tools/experiments/cring_sweep.sh): a round of 256x128 ring tiles takes 0.72 of a round of ping-pong tiles of
-            // the same K; a second launch costs about 0.08 of one. With a second stream running the other half of the clip
-            // (S = 2) the CUs a launch leaves idle are not lost, so a launch costs max(1, its share of the chip) and is never
-            // split: measured at 3 200 / 3 696 / 6 400 / 14 784 rows per stream, the ring kernel wins the first two (65 and
-            // 75 ping-pong tiles: -2 %, -7 % of the step), the ping-pong kernel the third (125 tiles: -12 %) and the unsplit
-            // launch the last (-4 %).
-            const int rbm = (g.M + BM2 - 1) / BM2, rbn = (g.N + BN - 1) / BN;
-            auto launch_cost = [&](int tiles) {
-                return S == 1 ? (float)((tiles + PERSISTENT_WGS - 1) / PERSISTENT_WGS)
-                              : fmaxf(1.f, (float)S * (float)tiles / (float)PERSISTENT_WGS);
-            };
-            const float c_ring = (float)g_cogs_debug.gemm_ring_cost_permille * 1e-3f;   // 0.72; the switch is for calibration sweeps
-            const float c_launch = 0.08f;
-            const float cost_pp = launch_cost(nb);
-            const float cost_ring = c_ring * launch_cost(rbm * rbn);
-            float best = cost_pp;
-            if (cost_ring < best) { best = cost_ring; mb_main = 0; }
-            if (S == 1 && rounds == 1 && rem > 0) {
+        int mb_main = -1;      // >= 0: row blocks that stay in this kernel (0 = none: all of the GEMM goes to the mid-size kernel)
+        if (!env_nosplit && !env_nostore && nb <= 2 * PERSISTENT_WGS) {
+            // Few tiles (a short clip, one rank's share of a frame-sharded one, a short prompt): the cheapest of this kernel, the
+            // mid-size one and one round here with the rest there -- each timed as if alone also when the encoder feeds two
+            // streams. (Counting both streams' tiles as one launch picked larger tiles, which leave less for the other stream's
+            // launch to run beside: 4 x 256 patches 3.09 against 2.58 ms, 16 x 256 5.46 / 4.92, 8 x 924 8.52 / 7.95.)
+            const int slabs = g.K / 64;
+            float best = tile_time(nb, slabs, PP_SLAB, 0.f, PP_REST);
+            if (mid_time < best) { best = mid_time; mb_main = 0; }
+            if (rounds == 1 && rem > 0) {
                 const int mb = whole_blocks(PERSISTENT_WGS);           // whole row blocks inside the first round
                 const int rows_rem = g.M - mb * BM3;
-                if (mb > 0 && rows_rem >= 512) {     // the remainder must reach the 256x128 ring kernel the cost model prices
-                    const float cost_split = 1.f + c_ring * launch_cost(((rows_rem + BM2 - 1) / BM2) * rbn) + c_launch;
-                    if (cost_split < best) { best = cost_split; mb_main = mb; }
+                if (mb > 0 && rows_rem > 0) {
+                    float rest;
+                    best_mid_tile(rows_rem, g.N, g.K, &rest);
+                    if (slabs * PP_SLAB + PP_REST + rest + SECOND_LAUNCH < best) mb_main = mb;
                 }
             }
         } else if (S == 1 && !env_nosplit && !env_nostore && g.K >= 2048 && rounds >= 2 && rem > 0 && rem * 100 < PERSISTENT_WGS * 45) {
-            // (many tiles: pays when a tile is long against a second launch and the last round is less than ~45 % full:
+            // (many tiles, one stream -- beside a second one a split launch costs the 64-frame clip 1 %: pays when a tile is long against a second launch and the last round is less than ~45 % full:
             // measured with the two-segment K loop at K = 1152: -2 %; K = 3584, last round 34 % full: +2 %; K = 18944,
             // 34 %: +6 %; K = 4352, 51 % full (ViT fc2): -2 %, so it no longer splits)
             const int mb = whole_blocks(rounds * PERSISTENT_WGS);    // whole row blocks within the full rounds
@@ -1275,12 +1264,10 @@ int cogs_k_gemm(hipStream_t st, const CogsGemm& g) {
         dispatch_pp(st, p, nb, env_nostore ? EPI_NOSTORE : pp_mask);
         return COGS_LAUNCH_CHECK();
     }
-    const bool big = g.M >= 512 && !g.force_small_tile && !env_small;
+    // fp32
+    const bool big = g.M >= 512 && !g.force_small_tile && g_cogs_debug.gemm_small == 0;
     p.nbm = (g.M + (big ? BM2 : BM) - 1) / (big ? BM2 : BM);
     p.nbn = (g.N + BN - 1) / BN;
-    const int grid = p.nbm * p.nbn;
-    const int mask = cogs_epi_mask(g);
-    if (g.dtype == COGS_DT_BF16) dispatch<bf16_t>(st, p, grid, mask, big);
-    else dispatch<float>(st, p, grid, mask, big);
+    dispatch_f32(st, p, p.nbm * p.nbn, cogs_epi_mask(g), big);
     return COGS_LAUNCH_CHECK();
 }

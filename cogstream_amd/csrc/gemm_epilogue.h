@@ -158,34 +158,35 @@ template <> struct RawVec<float> {
     static __device__ __forceinline__ f32x4 to_f32(f32x4 w) { return w; }
 };
 
-// Epilogue of one wave's 64x64 tile held as acc[mi][ni] (lane: row mb + 16 mi + (lane&15), columns
-// nb + 16 ni + 4 (lane>>4) .. +3). Loads first, then math + stores.
-template <typename T, int EPI>
+// Epilogue of one wave's 16 MI x 16 NI tile held as acc[mi][ni] (lane: row mb + 16 mi + (lane&15), columns
+// nb + 16 ni + 4 (lane>>4) .. +3). Loads first, then math + stores. EPI_ROWSTAT over a 32-column tile (NI == 2) cannot close a
+// 64-column block: the lanes' sums of row block mi go to half_stats[mi] instead and the caller joins the two halves.
+template <typename T, int EPI, int MI = 4, int NI = 4>
 __device__ __forceinline__ void epilogue_tile(const EpiArgs& p, int mb, int nb, int M, int N, int lane,
-                                              f32x4 (&acc)[4][4]) {
+                                              f32x4 (&acc)[MI][NI], f32x2* half_stats = nullptr) {
     const int mrow = mb + (lane & 15);
     const int ncol = nb + ((lane >> 4) << 2);
     if constexpr ((EPI & EPI_NOSTORE) != 0) {
 #pragma unroll
-        for (int mi = 0; mi < 4; ++mi)
+        for (int mi = 0; mi < MI; ++mi)
 #pragma unroll
-            for (int ni = 0; ni < 4; ++ni) asm volatile("" ::"v"(acc[mi][ni]));
+            for (int ni = 0; ni < NI; ++ni) asm volatile("" ::"v"(acc[mi][ni]));
         return;
     } else if constexpr ((EPI & EPI_GENERIC) != 0) {
 #pragma unroll
-        for (int mi = 0; mi < 4; ++mi) {
+        for (int mi = 0; mi < MI; ++mi) {
             const int m = mrow + mi * 16;
             if (m >= M) continue;
 #pragma unroll
-            for (int ni = 0; ni < 4; ++ni) {
+            for (int ni = 0; ni < NI; ++ni) {
                 const int n = ncol + ni * 16;
                 if (n < N) epilogue4<T>(p, m, n, acc[mi][ni]);
             }
         }
         return;
     } else {
-        // Two half tiles (mi pairs): per half, phase 1 issues every load (clamped addresses keep the loads
-        // unconditional), phase 2 does math + stores. Batching per half caps the live registers so hipcc does
+        // Pairs of row blocks: per half, phase 1 issues every load (clamped addresses keep the loads
+        // unconditional), phase 2 does math + stores. Batching per pair caps the live registers so hipcc does
         // not fall back to load->use round trips when the persistent loop keeps next-tile fragments live.
         //
         // WIDE path (bf16 output, N % 32 == 0): an MFMA lane owns 4 consecutive columns = 8 bytes, so a plain
@@ -197,24 +198,27 @@ __device__ __forceinline__ void epilogue_tile(const EpiArgs& p, int mb, int nb, 
         using raw_t = typename RawVec<T>::type;
         constexpr bool CAN_WIDE = sizeof(T) == 2 && (EPI & (EPI_SWIGLU | EPI_F32OUT)) == 0;
         const bool wide = CAN_WIDE && (N & 31) == 0;
+        // SwiGLU rows in whole 8- or 16-byte units: the wave's outputs all inside the row, rows and base aligned
+        constexpr bool CAN_PACK = sizeof(T) == 2 && (EPI & ~EPI_BIAS) == EPI_SWIGLU;
+        const bool packed = CAN_PACK && nb + 16 * NI <= N && (p.ldc & 7) == 0 && (reinterpret_cast<unsigned long>(p.C) & 15) == 0;
         const int g4 = lane >> 4;
         const int wcol = 16 * (g4 & 1) + 8 * (g4 >> 1);   // this lane's 8 columns inside a 32-column tile pair
-        f32x4 bias_v[4];
-        int nn[4];
+        f32x4 bias_v[NI];
+        int nn[NI];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) nn[i] = min(ncol + i * 16, N - 4);
+        for (int i = 0; i < NI; ++i) nn[i] = min(ncol + i * 16, N - 4);
         if constexpr ((EPI & EPI_LNFOLD) != 0) {
 #pragma unroll
-            for (int ni = 0; ni < 4; ++ni) bias_v[ni] = *reinterpret_cast<const f32x4*>(p.col_c + nn[ni]);
+            for (int ni = 0; ni < NI; ++ni) bias_v[ni] = *reinterpret_cast<const f32x4*>(p.col_c + nn[ni]);
         } else if constexpr ((EPI & EPI_BIAS) != 0) {
 #pragma unroll
-            for (int ni = 0; ni < 4; ++ni) bias_v[ni] = ld4_f<T>(reinterpret_cast<const T*>(p.bias) + nn[ni]);
+            for (int ni = 0; ni < NI; ++ni) bias_v[ni] = ld4_f<T>(reinterpret_cast<const T*>(p.bias) + nn[ni]);
         }
 #pragma unroll
-        for (int half = 0; half < 2; ++half) {
-            raw_t res_raw[2][4];
-            u32x4 res_wide[2][2];
-            f32x2 cs[2][4], sn[2][4];
+        for (int half = 0; half < MI / 2; ++half) {
+            raw_t res_raw[2][NI];
+            u32x4 res_wide[2][NI / 2];
+            f32x2 cs[2][NI], sn[2][NI];
             int mm[2];
             float rs2[2];
 #pragma unroll
@@ -229,7 +233,7 @@ __device__ __forceinline__ void epilogue_tile(const EpiArgs& p, int mb, int nb, 
 #pragma unroll
                         for (int i = 0; i < 2; ++i)
 #pragma unroll
-                            for (int pr = 0; pr < 2; ++pr)
+                            for (int pr = 0; pr < NI / 2; ++pr)
                                 res_wide[i][pr] = *reinterpret_cast<const u32x4*>(
                                     reinterpret_cast<const T*>(p.R) + (long)mm[i] * p.ldr + min(nb + 32 * pr, N - 32) + wcol);
                     }
@@ -237,7 +241,7 @@ __device__ __forceinline__ void epilogue_tile(const EpiArgs& p, int mb, int nb, 
 #pragma unroll
                     for (int i = 0; i < 2; ++i)
 #pragma unroll
-                        for (int ni = 0; ni < 4; ++ni)
+                        for (int ni = 0; ni < NI; ++ni)
                             res_raw[i][ni] = *reinterpret_cast<const raw_t*>(reinterpret_cast<const T*>(p.R) + (long)mm[i] * p.ldr + nn[ni]);
                 }
             }
@@ -245,7 +249,7 @@ __device__ __forceinline__ void epilogue_tile(const EpiArgs& p, int mb, int nb, 
 #pragma unroll
                 for (int i = 0; i < 2; ++i)
 #pragma unroll
-                    for (int ni = 0; ni < 4; ++ni) {
+                    for (int ni = 0; ni < NI; ++ni) {
                         rope_load(p, mm[i], (nn[ni] % p.head_dim) >> 1, cs[i][ni], sn[i][ni]);
                     }
             }
@@ -253,10 +257,10 @@ __device__ __forceinline__ void epilogue_tile(const EpiArgs& p, int mb, int nb, 
             for (int i = 0; i < 2; ++i) {
                 const int mi = 2 * half + i;
                 const int m = mrow + mi * 16;
-                f32x4 v[4];
+                f32x4 v[NI];
                 float st1 = 0.f, st2 = 0.f;   // EPI_ROWSTAT: this lane's share of (sum x, sum x^2) of row m in this tile
 #pragma unroll
-                for (int ni = 0; ni < 4; ++ni) {
+                for (int ni = 0; ni < NI; ++ni) {
                     const int n = ncol + ni * 16;
                     v[ni] = acc[mi][ni];
                     if constexpr ((EPI & EPI_LNFOLD) != 0) {
@@ -281,7 +285,7 @@ __device__ __forceinline__ void epilogue_tile(const EpiArgs& p, int mb, int nb, 
                 if (wide) {
                     if constexpr (CAN_WIDE) {
 #pragma unroll
-                        for (int pr = 0; pr < 2; ++pr) {
+                        for (int pr = 0; pr < NI / 2; ++pr) {
                             f32x4 va = v[2 * pr], vb = v[2 * pr + 1];
                             if constexpr ((EPI & EPI_RES) != 0) {
                                 // residual arrives in the exchanged layout: exchange back, then add in fp32
@@ -318,9 +322,27 @@ __device__ __forceinline__ void epilogue_tile(const EpiArgs& p, int mb, int nb, 
                                     u32x4{s0[0], s1[0], s0[1], s1[1]};
                         }
                     }
+                } else if (packed) {
+                    if constexpr (CAN_PACK) {
+                        // the lane's two outputs of every n-tile as one dword; the dwords of the lanes that share a row are
+                        // transposed so that a lane stores 8 (NI = 4) or 4 (NI = 2) consecutive outputs (see epilogue_pair_swiglu)
+                        unsigned d[NI];
+#pragma unroll
+                        for (int ni = 0; ni < NI; ++ni) d[ni] = pack_bf2(silu_f(v[ni][0]) * v[ni][1], silu_f(v[ni][2]) * v[ni][3]);
+                        const auto e = __builtin_amdgcn_permlane16_swap(d[0], d[1], false, false);
+                        T* row = reinterpret_cast<T*>(p.C) + (long)m * p.ldc + (nb >> 1);
+                        if constexpr (NI == 4) {
+                            const auto f = __builtin_amdgcn_permlane16_swap(d[2], d[3], false, false);
+                            const auto x = __builtin_amdgcn_permlane32_swap((unsigned)e[0], (unsigned)f[0], false, false);
+                            const auto y = __builtin_amdgcn_permlane32_swap((unsigned)e[1], (unsigned)f[1], false, false);
+                            if (m < M) *reinterpret_cast<u32x4*>(row + 8 * g4) = u32x4{(unsigned)x[0], (unsigned)y[0], (unsigned)x[1], (unsigned)y[1]};
+                        } else {
+                            if (m < M) *reinterpret_cast<u32x2*>(row + 8 * (g4 & 1) + 4 * (g4 >> 1)) = u32x2{(unsigned)e[0], (unsigned)e[1]};
+                        }
+                    }
                 } else {
 #pragma unroll
-                    for (int ni = 0; ni < 4; ++ni) {
+                    for (int ni = 0; ni < NI; ++ni) {
                         const int n = ncol + ni * 16;
                         if constexpr ((EPI & EPI_RES) != 0) v[ni] += RawVec<T>::to_f32(res_raw[i][ni]);
                         if constexpr ((EPI & EPI_ROWSTAT) != 0) {
@@ -342,7 +364,9 @@ __device__ __forceinline__ void epilogue_tile(const EpiArgs& p, int mb, int nb, 
                         }
                     }
                 }
-                if constexpr ((EPI & EPI_ROWSTAT) != 0) {
+                if constexpr ((EPI & EPI_ROWSTAT) != 0 && NI == 2) {
+                    half_stats[mi] = f32x2{st1, st2};
+                } else if constexpr ((EPI & EPI_ROWSTAT) != 0) {
                     st1 = rowgroup_sum(st1);
                     st2 = rowgroup_sum(st2);
                     if (g4 == 0 && m < M && nb < N)

@@ -48,6 +48,7 @@ struct CogsGemm {
                                              //   (include/cogs.h, cogs_gemm_desc.ln_ab, has the contract)
 };
 int cogs_k_gemm(hipStream_t st, const CogsGemm& g);
+int cogs_k_gemm_mid(hipStream_t st, const CogsGemm& g, int tile);     // gemm_mid.hip; the caller (cogs_k_gemm) has checked the operands
 void cogs_k_gemm_co_streams(int streams);   // hint for the few-tile choice: streams fed with GEMMs of this size at once (thread-local)
 // (a, b) = (rstd, -rstd * mean) per row from the EPI_ROWSTAT partials [rows][tiles][2]: ab [rows][2]
 int cogs_k_ln_finalize(hipStream_t st, const float* stat_part, int rows, int tiles, int H, float eps, float* ab);

@@ -1029,3 +1029,46 @@ def test_attention_head_major_inputs_equal_token_major_bit_for_bit(dev, heads, l
     assert torch.isfinite(out.float()).all()
     assert torch.equal(out, tok), float((out.float() - tok.float()).abs().max())
     assert torch.equal(outg, tok), "guard rows behind a head's rows were read: %g" % float((outg.float() - tok.float()).abs().max())
+
+
+@pytest.mark.parametrize("tile", [1, 2, 3, 4, 5])
+def test_mid_size_gemm_tiles_equal_each_other_and_fp64(dev, tile):
+    """gemm_mid.hip: every tile size, forced, at the edges of its tiles (rows and columns one short of and past a tile, a ragged
+    last one, fewer slabs than the ring has slots, odd slab counts), with each fused epilogue. Against float64 products of the same bf16
+    operands: the output's rounding is half a bf16 step (8 significant bits: spacing 2^-7 in [1, 2), half of it 2^-8 of the value at the
+    most), the fp32 sums of up to 1152 products add at most 2^-20 of the sum of |a||w|; fp32 outputs only have the latter. And bit for bit against the kernel that the dispatch picks: a row's
+    bits must not depend on the tile."""
+    from cogstream_amd import _lib as L2
+    ops = _ops()
+    g = torch.Generator(device=dev).manual_seed(tile)
+    rnd = lambda *s: (torch.randn(*s, generator=g, device=dev) * 0.5).bfloat16()
+    for M, N, K in ((2, 4, 64), (31, 60, 128), (33, 64, 192), (63, 132, 320), (65, 128, 384), (127, 260, 448), (129, 384, 512), (300, 700, 1152), (640, 1152, 640)):
+        a, w, b, r = rnd(M, K), rnd(N, K), rnd(N), rnd(M, N)
+        cases = [("plain", {}), ("bias", dict(bias=b)), ("residual", dict(bias=b, residual=r)), ("fp32", dict(out_f32=True)),
+                 ("gelu", dict(bias=b, act=L2.ACT_GELU_TANH)), ("swiglu", dict(act=L2.ACT_SWIGLU))]
+        if N % 64 == 0:
+            cases.append(("statistics", dict(bias=b, residual=r, row_stats=torch.empty(M, N // 64, 2, device=dev))))
+            table = torch.randn(M, 32, 2, generator=g, device=dev)
+            fold = dict(ln_ab=torch.rand(M, 2, generator=g, device=dev) + 0.5, col_c=torch.randn(N, generator=g, device=dev))
+            cases += [("rotary", dict(bias=b, rope_cos=table, rope_cols=64, head_dim=64)), ("folded norm", fold),
+                      ("rotary, head-major, folded norm", dict(rope_cos=table, rope_cols=64, head_dim=64, hm_cols=N, **fold))]
+        for name, kw in cases:
+            outs = []
+            for t in (tile, 0):
+                with L2.debug_switch("gemm_mid", t):
+                    stats = kw.get("row_stats")
+                    if stats is not None:
+                        stats.fill_(-7.0)
+                    outs.append((ops.gemm(a, w, **kw).clone(), None if stats is None else stats.clone()))
+            (x, sx), (y, sy) = outs
+            assert torch.equal(x, y), (M, N, K, name)
+            assert sx is None or torch.equal(sx, sy), (M, N, K, name)
+            if name in ("plain", "bias", "residual", "fp32"):
+                ref = a.double() @ w.double().t()
+                size = a.double().abs() @ w.double().abs().t()
+                if "bias" in kw:
+                    ref += b.double()
+                if "residual" in kw:
+                    ref += r.double()
+                bound = size * 2.0 ** -20 + (0 if name == "fp32" else ref.abs() * 2.0 ** -8 + 1e-30)
+                assert bool(((x.double() - ref).abs() <= bound * 1.01).all()), (M, N, K, name)
