@@ -17,9 +17,17 @@ from .runtime import get_handle
 
 
 @lru_cache(maxsize=64)
-def _tables(in_size: int, out_size: int):
+def _tables(in_size: int, out_size: int, device: int):
+    """tap tables of a resize on a device. Kept by size, not copied up on every call: four copies that wait for the device each
+    took as long as the kernel. The copies are complete when the tables enter the cache, so any stream may read them."""
     b, k, ks = resample_coeffs(in_size, out_size)
-    return np.ascontiguousarray(b), np.ascontiguousarray(k), ks
+    dev = torch.device("cuda", device)
+    return torch.from_numpy(np.ascontiguousarray(b)).to(dev), torch.from_numpy(np.ascontiguousarray(k)).to(dev), ks
+
+
+@lru_cache(maxsize=64)
+def _value_table(device: int):
+    return torch.from_numpy(pixel_value_table()).to(torch.device("cuda", device))
 
 
 def preprocess_media_gpu(items: Sequence[torch.Tensor], merge_sizes: Sequence[int], min_tokens: int = 16,
@@ -32,15 +40,14 @@ def preprocess_media_gpu(items: Sequence[torch.Tensor], merge_sizes: Sequence[in
     shapes = [(int(v.shape[0]), int(v.shape[1]), int(v.shape[2])) for v in items]
     targets = media_target_sizes(shapes, list(merge_sizes), min_tokens, max_tokens)
     handle = get_handle(dev)
-    table = torch.from_numpy(pixel_value_table()).to(dev)
+    index = dev.index if dev.index is not None else torch.cuda.current_device()
+    table = _value_table(index)
     outs, grids = [], []
     for v, merge_size, (th, tw) in zip(items, merge_sizes, targets):
         assert v.dtype == torch.uint8 and v.is_contiguous() and v.shape[-1] == 3
         t, H, W = int(v.shape[0]), int(v.shape[1]), int(v.shape[2])
-        bx, kx, ksx = _tables(W, tw)
-        by, ky, ksy = _tables(H, th)
-        dbx, dkx = torch.from_numpy(bx).to(dev), torch.from_numpy(kx).to(dev)
-        dby, dky = torch.from_numpy(by).to(dev), torch.from_numpy(ky).to(dev)
+        dbx, dkx, ksx = _tables(W, tw, index)
+        dby, dky, ksy = _tables(H, th, index)
         gh, gw = th // PATCH, tw // PATCH
         out = torch.empty(t * gh * gw, 3 * PATCH * PATCH, device=dev, dtype=out_dtype)
         n = C.c_size_t()

@@ -3,6 +3,7 @@ restatement of the same op on the same seeded inputs. Tolerances are stated per 
 bf16 storage => ~2^-8 relative per rounding; fp32 parity mode => 1e-4 or tighter."""
 import math
 
+import numpy as np
 import pytest
 import torch
 import torch.nn.functional as F
@@ -1072,3 +1073,29 @@ def test_mid_size_gemm_tiles_equal_each_other_and_fp64(dev, tile):
                     ref += r.double()
                 bound = size * 2.0 ** -20 + (0 if name == "fp32" else ref.abs() * 2.0 ** -8 + 1e-30)
                 assert bool(((x.double() - ref).abs() <= bound * 1.01).all()), (M, N, K, name)
+
+
+@pytest.mark.parametrize("t,h,w,merge,max_tokens,offset", [
+    (1, 28, 28, 2, 16384, 0),        # one window, enlarged: the smallest
+    (1, 45, 61, 1, 16384, 1),        # odd grid (bands of one patch), frames that start off a word
+    (2, 120, 214, 2, 16384, 2),      # a last tile of fewer than six patches
+    (3, 333, 517, 2, 300, 3),        # shrunk by less than 2 (9 taps) and the clip's last bytes read one by one
+    (2, 480, 854, 2, 120, 0),        # shrunk by about 3 (16 taps)
+    (1, 700, 640, 2, 40, 1),         # by about 4 (24 taps)
+    (1, 1024, 1500, 2, 16, 0),       # by about 10: the two-pass kernels
+])
+def test_fused_resize_equals_the_host_path(dev, t, h, w, merge, max_tokens, offset):
+    """csrc/preprocess.hip: the one-kernel resize and patchify, and the two-pass kernels behind it, give the bytes of the host
+    path (Pillow's arithmetic) through the value table: fp32 equal, bf16 that rounded once"""
+    from cogstream_amd import processing as pr
+    from cogstream_amd.preprocess_gpu import preprocess_videos_gpu
+    rng = np.random.default_rng(h)
+    frames = rng.integers(0, 256, (t, h, w, 3), dtype=np.uint8)
+    ref = pr.preprocess_videos([frames], merge_size=merge, max_tokens=max_tokens)
+    room = torch.empty(frames.size + offset, dtype=torch.uint8, device=dev)
+    room[offset:].copy_(torch.from_numpy(frames).reshape(-1))
+    clip = room[offset:].view(t, h, w, 3)
+    for dtype in (torch.float32, torch.bfloat16):
+        got = preprocess_videos_gpu([clip], merge_size=merge, max_tokens=max_tokens, out_dtype=dtype)
+        assert got["grid_sizes"].tolist() == ref["grid_sizes"].tolist()
+        assert torch.equal(got["pixel_values"].cpu(), torch.from_numpy(ref["pixel_values"]).to(dtype))
