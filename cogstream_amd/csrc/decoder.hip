@@ -60,7 +60,7 @@ namespace {
 
 struct Work {
     float* x; void *h, *y, *cq, *q, *att, *act, *hn, *ctx, *kvx, *qlat, *olat;
-    float *t32, *gate, *rope, *part, *dq, *dk, *dv, *dbg, *dout, *drec;
+    float *ypart, *t32, *gate, *rope, *part, *dq, *dk, *dv, *dbg, *dout, *drec;
     CogsSeq* seqs; int *rowseq, *rowpos, *want;
     size_t bytes;
 };
@@ -76,6 +76,7 @@ Work carve(const CogsDecoder& d, int S, int nseq, int64_t C, int n_want, void* w
     k.x = (float*)c.take(n * d.wp * 4 * (d.w.streams > 0 ? d.w.streams : 1));
     k.h = c.take(n * d.wp * es);
     k.y = c.take(n * d.wp * es);
+    if (S <= 64) k.ypart = (float*)c.take(n * d.wp * 4 * COGS_SKINNY_MAX_PARTS);     // few-row products into the residual stream
     k.t32 = (float*)c.take(n * d.max_t32 * 4);
     k.cq = c.take(n * d.max_cq * es);
     k.q = c.take(n * d.max_q * es);
@@ -126,6 +127,7 @@ struct Step {
     cogs_handle h; hipStream_t st; const CogsDecoder& d; Work k;
     const std::vector<CogsSeq>& seqs;
     int S, nseq, max_new, max_ctx; int64_t C;
+    int y_parts = 0;           // the sublayer's output is k.y, or so many partial sums in k.ypart
 
     const void* at(const void* p, size_t elems) const { return (const char*)p + elems * esize(d.w.dtype); }
 
@@ -136,6 +138,17 @@ struct Step {
         if (g_cogs_debug.gemm_skinny != 0 && cogs_k_gemm_skinny_fits(g)) return cogs_k_gemm_skinny(st, g);
         if (g.K < 128) g.force_small_tile = 1;      // the deep-pipelined kernels want at least two 64-wide slabs
         return cogs_k_gemm(st, g);
+    }
+
+    // a sublayer's last product, C = k.y: partial sums where few rows leave too few workgroups otherwise
+    int lin_out(CogsGemm& g) {
+        g.C = k.y; g.ldc = d.wp; g.M = S; g.N = d.wp;
+        g.dtype = d.w.dtype;
+        const int parts = g_cogs_debug.gemm_skinny != 0 && cogs_k_gemm_skinny_fits(g) ? cogs_k_gemm_skinny_parts(g.M, g.N, g.K) : 1;
+        y_parts = parts > 1 ? parts : 0;
+        if (parts < 2) return lin(g);
+        PROF(COGS_PROF_GEMM);
+        return cogs_k_gemm_skinny(st, g, k.ypart);
     }
 
     int latent_attention(const Run& run) {
@@ -214,8 +227,8 @@ struct Step {
     // attention rows -> sublayer output
     int project(const void* o_w, int oin) {
         CogsGemm g;
-        g.A = k.att; g.lda = oin; g.W = o_w; g.ldw = oin; g.C = k.y; g.ldc = d.wp; g.M = S; g.N = d.wp; g.K = oin;
-        return lin(g);
+        g.A = k.att; g.lda = oin; g.W = o_w; g.ldw = oin; g.K = oin;
+        return lin_out(g);
     }
 
     int attention(const Run& run) {
@@ -284,14 +297,14 @@ struct Step {
         g.N = m.act == COGS_ACT_SWIGLU ? 2 * ffp : ffp; g.K = d.wp; g.act = m.act;
         COGS_TRY(lin(g));
         CogsGemm g2;
-        g2.A = k.act; g2.lda = ffp; g2.W = m.down_w; g2.ldw = ffp; g2.C = k.y; g2.ldc = d.wp; g2.bias = m.down_b; g2.M = S; g2.N = d.wp; g2.K = ffp;
-        return lin(g2);
+        g2.A = k.act; g2.lda = ffp; g2.W = m.down_w; g2.ldw = ffp; g2.bias = m.down_b; g2.K = ffp;
+        return lin_out(g2);
     }
 
     // x from the embeddings, or x += norm(y) through the sublayer's (`from`) hyper-connections; then h = norm of what `to` reads
     int stream(const void* embeds, const float* y_gamma, const cogs_hyper* from, const cogs_hyper* to, const float* out_gamma, float* sum) {
         CogsStreamNorm a;
-        a.x = k.x; a.embeds = embeds; a.y = embeds ? nullptr : k.y; a.y_gamma = y_gamma; a.out = out_gamma ? k.h : nullptr; a.out_gamma = out_gamma;
+        a.x = k.x; a.embeds = embeds; a.y = embeds ? nullptr : y_parts ? (const void*)k.ypart : k.y; a.y_parts = embeds ? 0 : y_parts; a.y_gamma = y_gamma; a.out = out_gamma ? k.h : nullptr; a.out_gamma = out_gamma;
         a.rows = S; a.H = d.w.width; a.Hp = d.wp; a.eps = d.w.eps;
         if (embeds) { a.embed_scale = d.w.embed_scale; a.pos = d.w.pos; a.rowpos = k.rowpos; }
         a.streams = d.w.streams; a.sum = sum;

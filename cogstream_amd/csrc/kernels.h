@@ -83,7 +83,10 @@ int cogs_k_attention_decode(hipStream_t st, const struct CogsAttn& a, float* par
 int cogs_k_attention(hipStream_t st, const CogsAttn& a);
 // few-row GEMM (gemm_skinny.hip): bf16, 2 <= M <= 64; opt-in per call site (its summation order differs from cogs_k_gemm's)
 bool cogs_k_gemm_skinny_fits(const CogsGemm& g);
-int cogs_k_gemm_skinny(hipStream_t st, const CogsGemm& g);
+#define COGS_SKINNY_MAX_PARTS 8
+int cogs_k_gemm_skinny_parts(int M, int N, int K);
+// part != nullptr (plain products, with or without a bias): cogs_k_gemm_skinny_parts(..) (2, 4 or 8) partial sums fp32 [parts][M][N] instead of C
+int cogs_k_gemm_skinny(hipStream_t st, const CogsGemm& g, float* part = nullptr);
 long cogs_k_gemm_launch_count();   // kernels launched by cogs_k_gemm so far on this thread
 
 
@@ -189,6 +192,7 @@ int cogs_k_rope_sets(hipStream_t st, float* table, const CogsRopeSet* sets_dev, 
 // (in_w null: the sum of the streams), and sum (nullable) [rows][Hp] receives the sum of the streams
 struct CogsStreamNorm {
     float* x = nullptr; const void* embeds = nullptr; const void* y = nullptr; const float* y_gamma = nullptr;
+    int y_parts = 0;           // 2, 4, 8: y is the sum of so many fp32 [rows][Hp] arrays, one behind the other (added in order)
     void* out = nullptr; const float* out_gamma = nullptr; const int* pick = nullptr;
     int rows = 0, H = 0, Hp = 0; float eps = 0.f;
     float embed_scale = 1.f; const void* pos = nullptr; const int* rowpos = nullptr;

@@ -203,6 +203,25 @@ __global__ __launch_bounds__(256) void ln_finalize_kernel(const float* __restric
     *reinterpret_cast<f32x2*>(ab + 2 * (long)r) = f32x2{rstd, (float)(-(double)rstd * mean)};
 }
 
+// the sum of NP partial arrays at q, `step` apart: all loads out before the first addition
+template <int NP>
+__device__ __forceinline__ f32x4 sum_parts(const float* q, long step) {
+    f32x4 part[NP];
+#pragma unroll
+    for (int s = 0; s < NP; ++s) part[s] = *reinterpret_cast<const f32x4*>(q + s * step);
+#pragma unroll
+    for (int s = 1; s < NP; ++s) part[0] += part[s];
+    return part[0];
+}
+// four columns of a sublayer's output
+template <typename T>
+__device__ __forceinline__ f32x4 stream_y(const CogsStreamNorm& p, long row, int i) {
+    if (p.y_parts == 0) return ld4_f<T>(reinterpret_cast<const T*>(p.y) + row * p.Hp + i);
+    const float* q = reinterpret_cast<const float*>(p.y) + row * p.Hp + i;
+    const long step = (long)p.rows * p.Hp;
+    return p.y_parts == 2 ? sum_parts<2>(q, step) : p.y_parts == 4 ? sum_parts<4>(q, step) : sum_parts<8>(q, step);
+}
+
 // fp32 residual stream around a sublayer (kernels.h, CogsStreamNorm): one workgroup of TPB threads per row, the row in
 // registers (C chunks of four columns per thread). Norms entirely in fp32, one rounding of the normed row.
 template <typename T, int C, int TPB>
@@ -235,7 +254,7 @@ __global__ __launch_bounds__(TPB) void stream_norm_kernel(CogsStreamNorm p) {
         for (int c = 0; c < C; ++c) {
             const int i = (tid + TPB * c) * 4;
             y[c] = f32x4{0.f, 0.f, 0.f, 0.f};
-            if (i < p.Hp) y[c] = ld4_f<T>(reinterpret_cast<const T*>(p.y) + row * p.Hp + i);
+            if (i < p.Hp) y[c] = stream_y<T>(p, row, i);
 #pragma unroll
             for (int e = 0; e < 4; ++e) ss += y[c][e] * y[c][e];
         }
@@ -304,7 +323,7 @@ __global__ __launch_bounds__(TPB) void stream_mix_kernel(CogsStreamNorm p) {
         for (int c = 0; c < C; ++c) {
             const int i = (tid + TPB * c) * 4;
             y[c] = f32x4{0.f, 0.f, 0.f, 0.f};
-            if (i < p.Hp) y[c] = ld4_f<T>(reinterpret_cast<const T*>(p.y) + row * p.Hp + i);
+            if (i < p.Hp) y[c] = stream_y<T>(p, row, i);
 #pragma unroll
             for (int e = 0; e < 4; ++e) ss += y[c][e] * y[c][e];
         }
@@ -418,6 +437,7 @@ int launch_stream_norm(hipStream_t st, const CogsStreamNorm& a) {
 int cogs_k_stream_norm(hipStream_t st, int dtype, const CogsStreamNorm& a) {
     if (a.rows <= 0) return COGS_OK;
     if ((a.pos && !a.rowpos) || (a.y && a.streams > 0 && (!a.mix || !a.out_w)) || (a.streams <= 0 && (a.mix || a.in_w))) return COGS_E_INVALID;
+    if (a.y_parts != 0 && a.y_parts != 2 && a.y_parts != 4 && a.y_parts != 8) return COGS_E_INVALID;
     if (!a.x || a.Hp % 4 || a.H <= 0 || a.H > a.Hp || (a.out && !a.out_gamma) || (a.pick && (!a.out || a.y || a.embeds))) return COGS_E_INVALID;
     return dtype == COGS_DT_BF16 ? launch_stream_norm<bf16_t>(st, a) : launch_stream_norm<float>(st, a);
 }

@@ -375,6 +375,17 @@ def test_forms_and_kernels_agree(dev):
             assert rms_err(run(e, toks, [20, 380, *range(381, 400)]), lg) < TOL[torch.bfloat16], (name, value)
 
 
+@pytest.mark.parametrize("rows", [3, 16, 31, 64])
+@pytest.mark.parametrize("width,ff", [(70, 4100), (1100, 1030), (2120, 4100)])
+def test_sublayer_outputs_in_partial_sums(dev, rows, width, ff):
+    """as in test_gpu_pabalix.py, through the hyper-connected streams"""
+    cfg = config([attention(heads=8, kv_heads=2, dim=32, vdim=130), delta(heads=8, kv_heads=4, dim=16, vdim=130)], width=width, ff=ff, vocab=97)
+    st = state(cfg)
+    toks = tokens(cfg, rows)
+    got = run(engine(cfg, st, torch.bfloat16), toks)
+    assert rms_err(got, lo.forward(cfg, double(st), toks)[0]) < TOL[torch.bfloat16]
+
+
 def test_unsupported_calls_are_refused(dev):
     from cogstream_amd import _lib as L
     cfg, st, e, toks, _, _ = named("peaked", torch.bfloat16)

@@ -260,6 +260,18 @@ def test_forms_and_kernels_agree(dev):
             assert rms_err(run(e, toks, [20, 380, *range(381, 400)]), lg) < TOL[torch.bfloat16], (name, value)
 
 
+@pytest.mark.parametrize("rows", [2, 16, 17, 32, 33, 64])
+@pytest.mark.parametrize("width,ff", [(70, 4100), (1100, 1030), (3140, 4100)])
+def test_sublayer_outputs_in_partial_sums(dev, rows, width, ff):
+    """up to 64 rows: the products into the residual stream are stored as 2, 4 or 8 partial sums (a bias in the first) that the
+    stream's norm adds up; odd widths, K on both sides of the line between two ways to cut it, against the oracle"""
+    cfg = config([mixer(G, heads=8, dim=32, rot=16, vdim=130)], width=width, ff=ff, vocab=97)
+    st = state(cfg)
+    toks = tokens(cfg, rows)
+    got = run(engine(cfg, st, torch.bfloat16), toks)
+    assert rms_err(got, po.forward(cfg, double(st), toks)[0]) < TOL[torch.bfloat16]
+
+
 def test_unsupported_calls_are_refused(dev):
     from cogstream_amd import _lib as L
     cfg, st, e, toks, _, _ = named("peaked", torch.bfloat16, dev, 150)
