@@ -651,13 +651,12 @@ cogs_status VitRange::layer(int l) {
     char* qkv = (char*)big;
     char* att = qkv + (size_t)N * 3 * H * es;
     const cogs_vit_layer& L = h->vit_layers[l];
-    if (fold) { PROF(COGS_PROF_NORM); COGS_TRY(cogs_k_ln_finalize(st, stat_part, (int)N, H / 64, H, w.ln_eps, ln_ab)); }
-    else { PROF(COGS_PROF_NORM); COGS_TRY(cogs_k_layernorm(st, dt, x, ln, L.ln1_g, L.ln1_b, (int)N, H, w.ln_eps)); }
+    if (!fold) { PROF(COGS_PROF_NORM); COGS_TRY(cogs_k_layernorm(st, dt, x, ln, L.ln1_g, L.ln1_b, (int)N, H, w.ln_eps)); }
     {
         CogsGemm g; g.dtype = dt;
         g.A = fold ? x : ln; g.lda = H; g.W = L.qkv_w; g.ldw = H; g.C = qkv; g.ldc = 3 * H;
         g.M = (int)N; g.N = 3 * H; g.K = H;
-        if (fold) { g.ln_ab = ln_ab; g.col_c = L.qkv_c; }
+        if (fold) { g.ln_ab = ln_ab; g.ln_part = stat_part; g.ln_eps = w.ln_eps; g.col_c = L.qkv_c; }
         else g.bias = L.qkv_b;
         g.rope_cos = rc; g.rope_sin = rs; g.rope_cols = 2 * H; g.head_dim = hd;
         if (prescale_q) { g.q_scale = scale * 1.4426950408889634f; g.q_cols = H; }
@@ -689,13 +688,12 @@ cogs_status VitRange::layer(int l) {
         if (fold) g.row_stats = stat_part;
         { PROF(COGS_PROF_GEMM); COGS_TRY(cogs_k_gemm(st, g)); }
     }
-    if (fold) { PROF(COGS_PROF_NORM); COGS_TRY(cogs_k_ln_finalize(st, stat_part, (int)N, H / 64, H, w.ln_eps, ln_ab)); }
-    else { PROF(COGS_PROF_NORM); COGS_TRY(cogs_k_layernorm(st, dt, x, ln, L.ln2_g, L.ln2_b, (int)N, H, w.ln_eps)); }
+    if (!fold) { PROF(COGS_PROF_NORM); COGS_TRY(cogs_k_layernorm(st, dt, x, ln, L.ln2_g, L.ln2_b, (int)N, H, w.ln_eps)); }
     {
         CogsGemm g; g.dtype = dt;
         g.A = fold ? x : ln; g.lda = H; g.W = L.fc1_w; g.ldw = H; g.C = big; g.ldc = w.inter_pad;
         g.M = (int)N; g.N = w.inter_pad; g.K = H; g.act = COGS_ACT_GELU_TANH;
-        if (fold) { g.ln_ab = ln_ab; g.col_c = L.fc1_c; }
+        if (fold) { g.ln_ab = ln_ab; g.ln_part = stat_part; g.ln_eps = w.ln_eps; g.col_c = L.fc1_c; }
         else g.bias = L.fc1_b;
         { PROF(COGS_PROF_GEMM); COGS_TRY(cogs_k_gemm(st, g)); }
     }

@@ -153,6 +153,25 @@ __device__ __forceinline__ float wave_min(float v) {
     return wave_butterfly(v, [](float a, float b) { return fminf(a, b); });
 }
 
+// (rstd, -rstd * mean) of a row from its 64-column partial sums (sum, sum of squares): fp64, in order, biased variance like
+// nn.LayerNorm. The loads go out a batch ahead of the additions.
+__device__ __forceinline__ f32x2 ln_row_factors(const f32x2* part, int tiles, float inv_h, float eps) {
+    constexpr int B = 18;
+    double s1 = 0.0, s2 = 0.0;
+    for (int t0 = 0; t0 < tiles; t0 += B) {
+        f32x2 v[B];
+#pragma unroll
+        for (int i = 0; i < B; ++i) v[i] = part[min(t0 + i, tiles - 1)];
+#pragma unroll
+        for (int i = 0; i < B; ++i)
+            if (t0 + i < tiles) { s1 += (double)v[i][0]; s2 += (double)v[i][1]; }
+    }
+    const double mean = s1 * inv_h;
+    const double var = fmax(s2 * inv_h - mean * mean, 0.0);
+    const float rstd = (float)(1.0 / sqrt(var + (double)eps));
+    return f32x2{rstd, (float)(-(double)rstd * mean)};
+}
+
 // activations (fp32)
 __device__ __forceinline__ float gelu_tanh_f(float x) {
     // 0.5*x*(1+tanh(u)), u = sqrt(2/pi)*(x+0.044715x^3)   (ACT2FN["gelu_pytorch_tanh"])

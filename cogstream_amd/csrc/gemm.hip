@@ -1122,6 +1122,10 @@ static int best_mid_tile(int M, int N, int K, float* time) {
     }
     return best;
 }
+// the row factors of a folded LayerNorm for the kernels that read them finished (the mid-size one forms its rows' own)
+static int finish_ln(hipStream_t st, const CogsGemm& g) {
+    return g.ln_part ? cogs_k_ln_finalize(st, g.ln_part, g.M, g.K / 64, g.K, g.ln_eps, const_cast<float*>(g.ln_ab)) : COGS_OK;
+}
 static int launch_mid(hipStream_t st, const CogsGemm& g, int tile) {
     ++g_gemm_launches;
     g_cogs_debug.gemm_last_body = 2;
@@ -1137,6 +1141,7 @@ int cogs_k_gemm(hipStream_t st, const CogsGemm& g) {
     // the fused-LayerNorm features exist in the specialised MFMA epilogues only: the single-row GEMV and the run-time
     // (EPI_GENERIC) epilogue know neither, and silently dropping them would return un-normalised rows
     if ((g.row_stats || g.ln_ab) && (g.M == 1 || cogs_epi_mask(g) == EPI_GENERIC)) return COGS_E_UNSUPPORTED;
+    if (g.ln_part && (!g.ln_ab || g.K % 64 != 0)) return COGS_E_INVALID;
     if (g.hm_rows > 0 && (g.M == 1 || g.dtype != COGS_DT_BF16)) return COGS_E_UNSUPPORTED;       // head-major output: bf16 MFMA kernels only
     if (g.M == 1) { ++g_gemm_launches; g_cogs_debug.gemm_last_body = 6; return cogs_k_gemv(st, g); }
     if (g.rms_gamma) return COGS_E_UNSUPPORTED;   // fused RMSNorm exists for the single-token GEMV only
@@ -1245,12 +1250,14 @@ int cogs_k_gemm(hipStream_t st, const CogsGemm& g) {
             if (g.rope_rowpos) b.rope_rowpos = g.rope_rowpos + rows_main;
             if (g.row_stats) b.row_stats = g.row_stats + (size_t)rows_main * (g.N / 64) * 2;
             if (g.ln_ab) b.ln_ab = g.ln_ab + (size_t)rows_main * 2;
+            if (mb_main > 0) b.ln_part = nullptr;      // (finished below, in front of the first launch)
             if (g.rope_cos) {
                 const size_t per_row = (size_t)(g.head_dim / 2) * (g.rope_sin ? 1 : 2);
                 b.rope_cos = g.rope_cos + (size_t)rows_main * per_row;
                 if (g.rope_sin) b.rope_sin = g.rope_sin + (size_t)rows_main * per_row;
             }
             if (mb_main > 0) {
+                if (const int rc_ln = finish_ln(st, g)) return rc_ln;
                 p.M = rows_main; p.nbm = mb_main;
                 p.ntiles = count_tiles(rows_main);
                 dispatch_pp(st, p, p.ntiles, pp_mask);
@@ -1261,10 +1268,12 @@ int cogs_k_gemm(hipStream_t st, const CogsGemm& g) {
             if (mb_main > 0) g_cogs_debug.gemm_last_body = 5;
             return rc3;
         }
+        if (const int rc_ln = finish_ln(st, g)) return rc_ln;
         dispatch_pp(st, p, nb, env_nostore ? EPI_NOSTORE : pp_mask);
         return COGS_LAUNCH_CHECK();
     }
     // fp32
+    if (const int rc_ln = finish_ln(st, g)) return rc_ln;
     const bool big = g.M >= 512 && !g.force_small_tile && g_cogs_debug.gemm_small == 0;
     p.nbm = (g.M + (big ? BM2 : BM) - 1) / (big ? BM2 : BM);
     p.nbn = (g.N + BN - 1) / BN;

@@ -160,10 +160,11 @@ template <> struct RawVec<float> {
 
 // Epilogue of one wave's 16 MI x 16 NI tile held as acc[mi][ni] (lane: row mb + 16 mi + (lane&15), columns
 // nb + 16 ni + 4 (lane>>4) .. +3). Loads first, then math + stores. EPI_ROWSTAT over a 32-column tile (NI == 2) cannot close a
-// 64-column block: the lanes' sums of row block mi go to half_stats[mi] instead and the caller joins the two halves.
+// 64-column block: the lanes' sums of row block mi go to half_stats[mi] instead and the caller joins the two halves. row_scale: EPI_LNFOLD's factor of
+// row block mi's row, where the caller has it (else from ln_ab).
 template <typename T, int EPI, int MI = 4, int NI = 4>
 __device__ __forceinline__ void epilogue_tile(const EpiArgs& p, int mb, int nb, int M, int N, int lane,
-                                              f32x4 (&acc)[MI][NI], f32x2* half_stats = nullptr) {
+                                              f32x4 (&acc)[MI][NI], f32x2* half_stats = nullptr, const float* row_scale = nullptr) {
     const int mrow = mb + (lane & 15);
     const int ncol = nb + ((lane >> 4) << 2);
     if constexpr ((EPI & EPI_NOSTORE) != 0) {
@@ -225,7 +226,7 @@ __device__ __forceinline__ void epilogue_tile(const EpiArgs& p, int mb, int nb, 
             for (int i = 0; i < 2; ++i) mm[i] = min(mrow + (2 * half + i) * 16, M - 1);
             if constexpr ((EPI & EPI_LNFOLD) != 0) {
 #pragma unroll
-                for (int i = 0; i < 2; ++i) rs2[i] = p.ln_ab[2 * (long)mm[i]];
+                for (int i = 0; i < 2; ++i) rs2[i] = row_scale ? row_scale[2 * half + i] : p.ln_ab[2 * (long)mm[i]];
             }
             if constexpr ((EPI & EPI_RES) != 0) {
                 if (wide) {

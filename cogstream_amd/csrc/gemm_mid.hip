@@ -27,6 +27,7 @@ struct MidArgs {
     const char* W; long ldw;
     int M, N, KT;              // KT: 64-wide K slabs
     int nbm, nbn;
+    const float* ln_part; int ln_tiles; float ln_inv_h, ln_eps;     // EPI_LNFOLD: row statistics still in partial sums (or null)
     EpiArgs epi;
 };
 
@@ -135,6 +136,13 @@ __global__ __launch_bounds__(64 * WM * WN, WPE) void gemm_mid_kernel(MidArgs p) 
     };
 
     for (int i = 0; i < S && i < KT; ++i) stage(i);
+    // EPI_LNFOLD: the factors of this wave's rows while the ring fills; lane l has row l of its 16 MI
+    float factor = 0.f;
+    if constexpr ((EPI & EPI_LNFOLD) != 0) {
+        const long r = min(m0 + wm * 16 * MI + (lane & (16 * MI - 1)), p.M - 1);
+        factor = p.ln_part ? ln_row_factors(reinterpret_cast<const f32x2*>(p.ln_part) + r * p.ln_tiles, p.ln_tiles, p.ln_inv_h, p.ln_eps)[0]
+                           : p.epi.ln_ab[2 * r];
+    }
     wait_slabs<P, S - 1>(min(S, KT) - 1);
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
@@ -177,7 +185,12 @@ __global__ __launch_bounds__(64 * WM * WN, WPE) void gemm_mid_kernel(MidArgs p) 
     }
 
     const int mb = m0 + wm * 16 * MI, nb = n0 + wn * 16 * NI;
-    if constexpr (MI == 4 && NI == 4) {
+    if constexpr ((EPI & EPI_LNFOLD) != 0) {
+        float rs[MI];
+#pragma unroll
+        for (int mi = 0; mi < MI; ++mi) rs[mi] = __shfl(factor, 16 * mi + (lane & 15));
+        epilogue_tile<bf16_t, EPI, MI, NI>(p.epi, mb, nb, p.M, p.N, lane, acc, nullptr, rs);
+    } else if constexpr (MI == 4 && NI == 4) {
         epilogue_wave<bf16_t, EPI>(p.epi, mb, nb, p.M, p.N, lane, acc);
     } else if constexpr ((EPI & EPI_ROWSTAT) != 0 && NI == 2) {
         // a 64-column block's sums come from two waves; the pair is added lane by lane in the order of one 64-column wave, then
@@ -237,6 +250,7 @@ int cogs_k_gemm_mid(hipStream_t st, const CogsGemm& g, int tile) {
     p.A = (const char*)g.A; p.lda = g.lda * 2;
     p.W = (const char*)g.W; p.ldw = g.ldw * 2;
     p.M = g.M; p.N = g.N; p.KT = g.K / 64;
+    p.ln_part = g.ln_part; p.ln_tiles = g.K / 64; p.ln_inv_h = 1.0f / (float)g.K; p.ln_eps = g.ln_eps;
 #define COGS_MID_CASE(E) case E: dispatch_tile<E>(st, p, tile); break;
     switch (cogs_epi_mask(g)) {
         COGS_MID_CASE(0)

@@ -46,13 +46,14 @@ struct CogsGemm {
     const float* ln_ab = nullptr;            // != null: y = ln_ab[r][0] * acc + col_c[n] instead of acc + bias. W = rows of
     const float* col_c = nullptr;            //   W0*diag(gamma) made ZERO-SUM over k, col_c = bias + W0.beta; bias must be null
                                              //   (include/cogs.h, cogs_gemm_desc.ln_ab, has the contract)
+    // != null: ln_ab (then [M][2] of scratch) is not filled in yet, the statistics are in these partials [M][K/64][2]: the kernel
+    // forms each row's factor itself, or cogs_k_ln_finalize runs first
+    const float* ln_part = nullptr; float ln_eps = 0.f;
 };
 int cogs_k_gemm(hipStream_t st, const CogsGemm& g);
 int cogs_k_gemm_mid(hipStream_t st, const CogsGemm& g, int tile);     // gemm_mid.hip; the caller (cogs_k_gemm) has checked the operands
 void cogs_k_gemm_co_streams(int streams);   // hint for the few-tile choice: streams fed with GEMMs of this size at once (thread-local)
 // (a, b) = (rstd, -rstd * mean) per row from the EPI_ROWSTAT partials [rows][tiles][2]: ab [rows][2]
-int cogs_k_ln_finalize(hipStream_t st, const float* stat_part, int rows, int tiles, int H, float eps, float* ab);
-// (a, b) = (rstd, -rstd * mean) per row from the EPI_ROWSTAT partials: ab [rows][2]
 int cogs_k_ln_finalize(hipStream_t st, const float* stat_part, int rows, int tiles, int H, float eps, float* ab);
 
 struct CogsAttn {
