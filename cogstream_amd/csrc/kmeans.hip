@@ -288,23 +288,25 @@ __global__ __launch_bounds__(256) void reduce_assign_kernel(const float* __restr
 // normalised by their sum; torch.multinomial(probs, 1) on the CPU IS argmax(probs / q), q ~ Exponential(1) one draw per
 // element from the CPU generator (ATen multinomial, n_sample == 1) -- the host hands those draws over. A zero sum (every
 // row coincides with a chosen centre) is the reference's random.randint branch: flagged, the host then takes the step-wise
-// path. One workgroup; the sum runs in fp64 in a fixed order (torch's own fp32 summation order is not reproduced: the sum
+// path. The sum runs in fp64 in a fixed order (torch's own fp32 summation order is not reproduced: the sum
 // is a common divisor of all ratios and only moves the argmax between ratios closer than a few ulps).
-__global__ __launch_bounds__(256) void kpp_select_kernel(const float* __restrict__ nearest2, const float* __restrict__ q, int Tn,
-                                                         int* __restrict__ idx_out, int* __restrict__ zero_flag, int first_row) {
-    __shared__ double red[4];
-    __shared__ float rv[4];
-    __shared__ int ri[4];
-    const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
-    if (first_row >= 0 && tid == 0) idx_out[-1] = first_row;      // step 1 also records the caller's first centre
+// Run by 256 threads of the workgroup that measured the last row (others wrote nearest2: read past the caches).
+__device__ __forceinline__ void kpp_select(float* nearest2, const float* __restrict__ q, int Tn, int* __restrict__ idx_out, int* __restrict__ zero_flag,
+                                           int tid, double* red, float* rv, int* ri) {
+    const int lane = tid & 63, wid = tid >> 6;
+    const bool on = tid < 256;
+    auto load = [&](int t) { return __hip_atomic_load(nearest2 + t, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); };
+    const float own = on && tid < Tn ? load(tid) : 0.f;          // a thread's first row; further ones are read twice
+    auto near_of = [&](int t) { return t == tid ? own : load(t); };
+    const float own_q = on && tid < Tn ? q[tid] : 1.f;
     double sum = 0.0;
-    for (int t = tid; t < Tn; t += 256) {
-        const float d = sqrtf(nearest2[t]);
+    for (int t = on ? tid : Tn; t < Tn; t += 256) {
+        const float d = sqrtf(near_of(t));
         sum += (double)__fmul_rn(d, d);
     }
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) sum += __shfl_xor(sum, o, 64);
-    if (lane == 0) red[wid] = sum;
+    if (on && lane == 0) red[wid] = sum;
     __syncthreads();
     const float total = (float)((red[0] + red[1]) + (red[2] + red[3]));
     if (total == 0.f) {
@@ -313,9 +315,9 @@ __global__ __launch_bounds__(256) void kpp_select_kernel(const float* __restrict
     }
     float best = -INFINITY;
     int bi = 0x7fffffff;
-    for (int t = tid; t < Tn; t += 256) {                 // ascending t per thread: the first maximum is kept
-        const float d = sqrtf(nearest2[t]);
-        const float r = __fdiv_rn(__fdiv_rn(__fmul_rn(d, d), total), q[t]);
+    for (int t = on ? tid : Tn; t < Tn; t += 256) {       // ascending t per thread: the first maximum is kept
+        const float d = sqrtf(near_of(t));
+        const float r = __fdiv_rn(__fdiv_rn(__fmul_rn(d, d), total), t == tid ? own_q : q[t]);
         if (r > best || (r != r && best == best)) { best = r; bi = t; }      // NaN counts as the maximum, like torch.argmax
     }
 #pragma unroll
@@ -325,7 +327,7 @@ __global__ __launch_bounds__(256) void kpp_select_kernel(const float* __restrict
         const bool take = (ob > best) || (ob != ob && best == best) || ((ob == best || (ob != ob && best != best)) && oi < bi);
         if (take) { best = ob; bi = oi; }
     }
-    if (lane == 0) { rv[wid] = best; ri[wid] = bi; }
+    if (on && lane == 0) { rv[wid] = best; ri[wid] = bi; }
     __syncthreads();
     if (tid == 0) {
         float b = rv[0]; int i = ri[0];
@@ -336,6 +338,75 @@ __global__ __launch_bounds__(256) void kpp_select_kernel(const float* __restrict
         }
         *idx_out = i == 0x7fffffff ? 0 : i;
     }
+}
+
+// One k-means++ step (:46-60) of the whole-seeding call: workgroup t measures row t against the newest centre, a slice of 512
+// columns per wave at a time, folds the distance into nearest2[t], and the workgroup that finishes last draws the next centre. The sums are
+// those of sqdist_kernel and reduce_min_kernel, value by value: fp32 within a slice (lanes 32, 16, then 1, 2, 4, 8 apart), the
+// slices in fp64 by one wave's lanes. Bound by what a CU takes in (its row and the centre's, 60 bytes a nanosecond): a step of
+// [256, 179 200] bf16 is 23 us; partial sums by slices (sqdist), their reduction and the draw were three launches, 31 us.
+constexpr int KPP_T = 1024;
+template <typename T>
+__global__ __launch_bounds__(KPP_T) void kpp_step_kernel(const T* __restrict__ x, int Tn, long PD, int nslices, const int* __restrict__ centre_from,
+                                                         int centre_row, int first, float* nearest2, const float* __restrict__ q, int* idx_out,
+                                                         int* zero_flag, int* done, float* spill) {
+    extern __shared__ __attribute__((aligned(16))) char smem_raw[];
+    float* const sums = spill ? spill + (long)blockIdx.x * nslices : reinterpret_cast<float*>(smem_raw);       // [nslices]
+    __shared__ double red[4];
+    __shared__ float rv[4];
+    __shared__ int ri[4], last;
+    const int tid = threadIdx.x, lane = tid & 63, wid = __builtin_amdgcn_readfirstlane(tid >> 6);
+    constexpr int NW = KPP_T / 64, U = 4;
+    const T* xr = x + (long)blockIdx.x * PD + lane * 8;
+    const T* cr = x + (long)(centre_from ? *centre_from : centre_row) * PD + lane * 8;
+    // a row is a whole number of memory interleaves away from the next as often as not: every workgroup starts at another slice
+    const int turn = (int)((unsigned)blockIdx.x * 61u % (unsigned)nslices);
+    auto slice = [&](int i) { const int sl = i + turn; return sl < nslices ? sl : sl - nslices; };
+    for (int s0 = wid; s0 < nslices; s0 += NW * U) {
+        float a[U][8], c[U][8];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {                            // (slices and columns past the end repeat what is there and are not used)
+            const long j = (long)slice(min(s0 + NW * u, nslices - 1)) * SL;
+            const long at = j + lane * 8 < PD ? j : PD - 8 - lane * 8;
+            ld8_f<T>(xr + at, a[u]);
+            ld8_f<T>(cr + at, c[u]);
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            if (s0 + NW * u >= nslices) break;
+            const int sl = slice(s0 + NW * u);
+            float s = 0.f;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const float d0 = a[u][e] - c[u][e], d1 = a[u][4 + e] - c[u][4 + e];
+                s = fmaf(d0, d0, s);
+                s = fmaf(d1, d1, s);
+            }
+            if ((long)sl * SL + lane * 8 >= PD) s = 0.f;
+            s = swap32_sum(s, s);
+            s = row16_sum(swap16_sum(s, s));
+            if (lane == 0) sums[sl] = s;
+        }
+    }
+    __syncthreads();
+    if (wid == 0) {
+        double d = 0.0;
+        for (int sl = lane; sl < nslices; sl += 64) d += (double)sums[sl];
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) d += __shfl_xor(d, o, 64);
+        if (lane == 0) {
+            const float d2 = (float)d;
+            __hip_atomic_store(nearest2 + blockIdx.x, first ? d2 : fminf(nearest2[blockIdx.x], d2), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            last = __hip_atomic_fetch_add(done, 1, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) == Tn - 1;
+        }
+    }
+    __syncthreads();
+    if (!last) return;
+    if (tid == 0) {
+        *done = 0;                                               // for the next step's launch
+        if (first) idx_out[-1] = centre_row;                     // step 1 also records the caller's first centre
+    }
+    kpp_select(nearest2, q, Tn, idx_out, zero_flag, tid, red, rv, ri);
 }
 
 // k-means++ step (:46-60): nearest2[t] = min(nearest2[t], dist2 to the newest centre) (first: plain store)
@@ -491,7 +562,8 @@ __global__ __launch_bounds__(256) void update_kernel(const T* __restrict__ x, lo
 
 // one workgroup: centre times, shift norms (scratch [2K]: feature-shift norm, squared time shift), total movement.
 // status (nullable, host-mapped): {shift, reseeds used, abort, empty clusters} for the Lloyd loop's one read per iteration
-__global__ __launch_bounds__(256) void update_final_kernel(const float* __restrict__ ts, int K,
+constexpr int UF_T = 1024;
+__global__ __launch_bounds__(UF_T) void update_final_kernel(const float* __restrict__ ts, int K,
                                                            const int* __restrict__ offs, const int* __restrict__ members,
                                                            const int* __restrict__ reseed_rows, int* __restrict__ ctl,
                                                            float* __restrict__ cts,
@@ -505,25 +577,25 @@ __global__ __launch_bounds__(256) void update_final_kernel(const float* __restri
     const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
     if (!aborted) {
         if (Tn_lds > 0) {
-            for (int i = threadIdx.x; i < Tn_lds; i += 256) mts[i] = ts[members[i]];     // one dependent pair per thread, in parallel
+            for (int i = threadIdx.x; i < Tn_lds; i += UF_T) mts[i] = ts[members[i]];     // one dependent pair per thread, in parallel
             __syncthreads();
         }
-        for (int k = wid; k < K; k += 4) {                  // one wave per cluster
+        for (int k = wid; k < K; k += UF_T / 64) {          // shift: one wave per cluster
             double s = 0.0;
             for (int b = lane; b < nblk; b += 64) s += (double)shift_partial[(long)b * K + k];
 #pragma unroll
             for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
-            if (lane == 0) {
-                scratch[k] = sqrtf((float)s);
-                float tsum = 0.f;
-                const int b0 = offs[k], e0 = offs[k + 1];
-                if (Tn_lds > 0) { for (int i = b0; i < e0; ++i) tsum += mts[i]; }
-                else { for (int i = b0; i < e0; ++i) tsum += ts[members[i]]; }
-                const float nt = e0 > b0 ? tsum / (float)(e0 - b0) : ts[reseed_rows[k]];
-                const float d = nt - cts[k];
-                scratch[K + k] = d * d;
-                cts[k] = nt;
-            }
+            if (lane == 0) scratch[k] = sqrtf((float)s);
+        }
+        for (int k = UF_T - 1 - (int)threadIdx.x; k < K; k += UF_T) {      // times: one thread per cluster, its members in order (the last waves first: they
+            float tsum = 0.f;                                                       // have the fewest shifts to sum)
+            const int b0 = offs[k], e0 = offs[k + 1];
+            if (Tn_lds > 0) { for (int i = b0; i < e0; ++i) tsum += mts[i]; }
+            else { for (int i = b0; i < e0; ++i) tsum += ts[members[i]]; }
+            const float nt = e0 > b0 ? tsum / (float)(e0 - b0) : ts[reseed_rows[k]];
+            const float d = nt - cts[k];
+            scratch[K + k] = d * d;
+            cts[k] = nt;
         }
     }
     __syncthreads();
@@ -737,7 +809,7 @@ int launch_update(hipStream_t st, int dtype, const void* feats, const float* ts,
         hipLaunchKernelGGL(update_kernel<float>, dim3(nblk, K), dim3(256), 0, st, (const float*)feats, PD, K, w.offs, w.members,
                            w.reseed, ctl, centres, w.partial);
     const int t_lds = T <= MEMB_T ? T : 0;       // member-ordered time stamps staged in LDS (64 KiB at most)
-    hipLaunchKernelGGL(update_final_kernel, dim3(1), dim3(256), (size_t)t_lds * 4, st, ts, K, w.offs, w.members, w.reseed, ctl,
+    hipLaunchKernelGGL(update_final_kernel, dim3(1), dim3(UF_T), (size_t)t_lds * 4, st, ts, K, w.offs, w.members, w.reseed, ctl,
                        centre_ts, w.partial, nblk, w.scratch, shift_out, status, t_lds, tol);
     return COGS_LAUNCH_CHECK();
 }
@@ -791,7 +863,7 @@ int cogs_k_kmeans_pp_step(hipStream_t st, int dtype, const void* feats, int T, l
 
 // The whole k-means++ seeding (kmeans_with_time.py:41-62) in one call, no host round trip per centre: step m measures
 // every row against the newest centre (row idx[m-1], read from device memory), folds it into nearest2 and draws centre m
-// as argmax(probs / q[m-1]) (kpp_select_kernel). q: device fp32 [K-1][T], the Exponential(1) draws the reference's K-1
+// as argmax(probs / q[m-1]) (kpp_select). q: device fp32 [K-1][T], the Exponential(1) draws the reference's K-1
 // torch.multinomial calls would make on the CPU generator, made ahead by the host. idx: device int32 [K], idx[0] given.
 // *zero_flag (device int, zeroed here) is set when a step found all probabilities zero -- the reference's
 // random.randint branch; the indices from that step on are then meaningless and the caller redoes the seeding step by step.
@@ -799,16 +871,22 @@ int cogs_k_kmeans_pp(hipStream_t st, int dtype, const void* feats, int T, long P
                      int* zero_flag, float* nearest2, float* ws, int nslices) {
     if (T <= 0 || K <= 0 || PD % 8 || !q || !idx || !zero_flag || !nearest2 || first_row < 0 || first_row >= T) return COGS_E_INVALID;
     const KmWs w = carve(ws, T, PD, 1);
-    if (hipMemsetAsync(zero_flag, 0, sizeof(int), st) != hipSuccess) return COGS_E_HIP;
+    if (nslices != (int)((PD + SL - 1) / SL)) return COGS_E_WORKSPACE;
+    if (hipMemsetAsync(zero_flag, 0, sizeof(int), st) != hipSuccess || hipMemsetAsync(w.ctl, 0, sizeof(int), st) != hipSuccess) return COGS_E_HIP;
+    size_t lds = (size_t)nslices * 4;
+    float* spill = nullptr;
+    if (lds > 48 * 1024) { lds = 0; spill = w.partial; }         // more than six million columns: a row's sums in the workspace
     for (int m = 1; m < K; ++m) {
         // step 1 measures against the caller's first centre (a kernel argument: nothing is uploaded), later steps against
         // the row the previous step drew (read from device memory)
-        const int rc = m == 1 ? sqdist_partials(st, dtype, feats, T, PD, nullptr, nullptr, first_row, 1, w.partial, nslices)
-                              : sqdist_partials(st, dtype, feats, T, PD, nullptr, idx + (m - 1), -1, 1, w.partial, nslices);
-        if (rc != COGS_OK) return rc;
-        hipLaunchKernelGGL(reduce_min_kernel, dim3((T + 3) / 4), dim3(256), 0, st, w.partial, nslices, T, m == 1 ? 1 : 0, nearest2);
-        hipLaunchKernelGGL(kpp_select_kernel, dim3(1), dim3(256), 0, st, nearest2, q + (size_t)(m - 1) * T, T, idx + m, zero_flag,
-                           m == 1 ? first_row : -1);
+        const int* from = m == 1 ? nullptr : idx + (m - 1);
+        const float* qm = q + (size_t)(m - 1) * T;
+        if (dtype == COGS_DT_BF16)
+            hipLaunchKernelGGL(kpp_step_kernel<bf16_t>, dim3(T), dim3(KPP_T), lds, st, (const bf16_t*)feats, T, PD, nslices, from, first_row, m == 1, nearest2,
+                               qm, idx + m, zero_flag, w.ctl, spill);
+        else
+            hipLaunchKernelGGL(kpp_step_kernel<float>, dim3(T), dim3(KPP_T), lds, st, (const float*)feats, T, PD, nslices, from, first_row, m == 1, nearest2,
+                               qm, idx + m, zero_flag, w.ctl, spill);
     }
     if (K == 1 && hipMemcpyAsync(idx, &first_row, sizeof(int), hipMemcpyHostToDevice, st) != hipSuccess) return COGS_E_HIP;
     return COGS_LAUNCH_CHECK();

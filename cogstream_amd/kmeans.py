@@ -77,7 +77,9 @@ def kmeans_with_time_min_max(features: torch.Tensor, timestamp, cluster_num: int
     # redone step by step (the round-3 path: one pinned read of the [T] distances per centre) ----
     first = random.randint(0, T - 1)
     py_state, torch_state = random.getstate(), torch.get_rng_state()
-    q = torch.stack([torch.empty(T, dtype=torch.float32).exponential_(1) for _ in range(K - 1)])
+    q = torch.empty(K - 1, T, dtype=torch.float32)
+    for row in q.unbind(0):
+        row.exponential_(1)
     idx_d, flag = ops.kmeans_pp(x, first, K, q.to(dev, non_blocking=True), ws)
     # (no host read here: the Lloyd loop below starts from the device-resident rows; the flag is looked at after its
     # first synchronisation, and in the rare flagged case everything is redone step by step)

@@ -1099,3 +1099,28 @@ def test_fused_resize_equals_the_host_path(dev, t, h, w, merge, max_tokens, offs
         got = preprocess_videos_gpu([clip], merge_size=merge, max_tokens=max_tokens, out_dtype=dtype)
         assert got["grid_sizes"].tolist() == ref["grid_sizes"].tolist()
         assert torch.equal(got["pixel_values"].cpu(), torch.from_numpy(ref["pixel_values"]).to(dtype))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("T,PD,K", [(2, 8, 2), (5, 520, 4), (257, 1000, 9), (300, 4096, 12), (3, 6_300_000, 3)])
+def test_whole_seeding_equals_the_steps(dev, T, PD, K, dtype):
+    """cogs_kmeans_pp (one launch a centre) draws the rows that distances of cogs_kmeans_pp_step and the same exponentials give on the
+    host: one slice and fewer, a ragged last slice, more rows than a workgroup's threads draw from at once, rows whose slice sums no
+    longer fit the LDS; rows that all coincide raise the flag"""
+    ops = _ops()
+    g = torch.Generator(device=dev).manual_seed(T)
+    x = torch.randn(T, PD, generator=g, device=dev).to(dtype)
+    q = torch.empty(K - 1, T).exponential_(1)
+    first = T // 2
+    ws = ops.kmeans_workspace(T, PD, K, x.device)
+    idx, flag = ops.kmeans_pp(x, first, K, q.to(dev), ws)
+    want, near = [first], torch.empty(T, device=dev)
+    probs = torch.empty(T).pin_memory()
+    for m in range(K - 1):
+        ops.kmeans_pp_step(x, want[-1], m == 0, near, probs, ws)
+        p = probs.sqrt() ** 2
+        want.append(int((p / p.double().sum().float() / q[m]).argmax()))
+    assert idx.tolist() == want and int(flag) == 0
+    same = x[:1].expand(T, PD).contiguous()
+    _, flag = ops.kmeans_pp(same, first, K, q.to(dev), ws)
+    assert int(flag) == 1
