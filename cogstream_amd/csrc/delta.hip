@@ -9,15 +9,19 @@
 // A token-by-token kernel (delta_recur) serves the sizes the chunked pair has no instance for.
 //
 // Chunks. With G_i = sum of ln g over the chunk's tokens 0 .. i and S0 the state in front of it,
-//   u_i = beta_i (v_i - e^{G_i} S0^T k_i - sum_{j<i} e^{G_i - G_j} (k_i . k_j) u_j),  i.e.  U = T diag(beta) (V - diag(e^G) K S0)
+//   u_i = beta_i (v_i - e^{G_i} S0^T k_i - sum_{j<i} e^{G_i - G_j} (k_i . k_j) u_j),  i.e.  U = T diag(beta) (V - diag(e^G) K S0) = T diag(beta) V + W S0
 //   with T = (I + L)^-1, L_ij = beta_i e^{G_i - G_j} k_i . k_j (j < i);   O = diag(e^G) Q S0 + P U with P_ij = e^{G_i - G_j} q_i . k_j (j <= i);
 //   S = e^{G_last} S0 + K^T diag(e^{G_last - G_j}) U.
-// Only exponentials of differences of later minus earlier sums appear (<= 1); the sums themselves are fp64. T diag(beta), P and the
+// Only exponentials of differences of later minus earlier sums appear (<= 1); the sums themselves are fp64. T diag(beta), W, P and the
 // exponentials do not depend on S: delta_chunk forms them for all chunks at once, T by forward substitution. delta_scan walks a
 // sequence's chunks: a workgroup owns 16 columns of S, its four waves the 16-row tiles of S in turn.
+// The scan's chunks follow one another, so what counts is the length of one: W S0, a sum over the waves, the new state. W (33 MB at
+// 4096 tokens and 16 heads, in place of a product with T behind the sum) and operands in the order of the lanes took it from 2.2 to
+// 1.2 us a chunk: 285 -> 155 us for the scan, 26 -> 39 us for delta_chunk. Two thirds of that are matrix instructions (54 of 14 ns), the
+// rest LDS exchange and the loads' share of issue. delta_chunk is bound by its phases: all workgroups load, then multiply, then store.
 // MFMA layout: a 16x16 accumulator holds rows 4 g + r in register r of lane group g, which is the B operand of the r-th of four
-// 4-deep steps if k is taken in the order 4 g + r -- so S, R and U go from product to product in their registers, and A operands
-// are 16-byte loads of four neighbouring k.
+// 4-deep steps if k is taken in the order 4 g + r -- so S and U go from product to product in their registers, and A operands are
+// 16-byte loads of four neighbouring k.
 #include "common.h"
 #include "kernels.h"
 #include "debug.h"
@@ -26,7 +30,9 @@ namespace {
 
 constexpr int CH = 32;                        // tokens of a chunk
 constexpr int TILE = 256;                     // floats of a 16x16 tile, row-major
-constexpr int REC = 6 * TILE + 3 * CH;        // per chunk and head: T beta tiles (0,0) (1,0) (1,1) | P tiles | e^G | e^{G_last - G} | e^{G_last}, ..
+constexpr int EXPS = 6 * TILE;                 // per chunk and head: P tiles (0,0) (1,0) (1,1) | T beta tiles | e^G | e^{G_last - G} | e^{G_last}, .. | W [2][dkp / 16][64 lanes][4];
+constexpr int REC = EXPS + 3 * CH;            // P and T beta as A operands [4 steps][64 lanes], W as A operands too
+__host__ __device__ constexpr int rec_floats(int dkp) { return REC + CH * dkp; }
 
 __device__ __forceinline__ float unit_scale(float ss) { return 1.f / sqrtf(ss + 1e-6f); }
 __device__ __forceinline__ float sigmoid_f(float x) { return 1.f / (1.f + expf(-x)); }
@@ -200,87 +206,105 @@ __device__ __forceinline__ f32x4 mfma4(const f32x4& a, const f32x4& b, f32x4 c) 
 }
 
 __device__ __forceinline__ float* chunk_rec(const CogsDelta& p, const CogsSeq& s, int seq, int chunk, int h) {
-    return p.rec + ((long)(s.row0 / CH + seq + chunk) * p.heads + h) * REC;      // (a later sequence starts behind the chunks of an earlier one)
+    return p.rec + ((long)(s.row0 / CH + seq + chunk) * p.heads + h) * rec_floats(p.dkp);      // (a later sequence starts behind the chunks of an earlier one)
 }
 
-// what a chunk needs besides S: three waves, one per tile (0,0), (1,0), (1,1) of the 32 x 32 matrices
-__global__ __launch_bounds__(192) void delta_chunk_kernel(CogsDelta p) {
+// What a chunk needs besides S and V: P, T diag(beta), the exponentials and W = -T diag(beta) diag(e^G) K. Three waves take a tile
+// (0,0), (1,0), (1,1) each of the 32 x 32 matrices, then four waves the 16-column pieces of W.
+__global__ __launch_bounds__(256) void delta_chunk_kernel(CogsDelta p) {
     __shared__ double cum[CH];
-    __shared__ float beta_s[CH];
-    __shared__ __attribute__((aligned(16))) float Ls[3][16][20], Ts[3][16][20];
+    __shared__ __attribute__((aligned(16))) float beta_s[CH], eg_s[CH];
+    __shared__ __attribute__((aligned(16))) float L10[16][20], Ts[3][16][20];
     const int chunk = blockIdx.x, h = blockIdx.y, seq = blockIdx.z;
     const CogsSeq s = p.seqs[seq];
     const int n = min(CH, s.len - chunk * CH);
     if (n <= 0) return;
     const int tid = threadIdx.x, lane = tid & 63, li = lane & 15, g = lane >> 4;
-    const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
+    // the waves' roles go round from workgroup to workgroup: the k-th waves of all of a compute unit's workgroups share a SIMD
+    const int turn = (blockIdx.y * gridDim.x + blockIdx.x) >> 8;
+    const int wid = (__builtin_amdgcn_readfirstlane(tid >> 6) + turn + blockIdx.x) & 3;
     const long row0 = s.row0 + chunk * CH;
     const int kh = h / (p.heads / p.kv_heads);
-    const long k0 = ((long)kh * p.rows + row0) * p.dkp + 4 * g;
+    const float* K = p.k + ((long)kh * p.rows + row0) * p.dkp;
+    const float* Q = p.q + ((long)kh * p.rows + row0) * p.dkp;
+    float* rec = chunk_rec(p, s, seq, chunk, h);
     const int ta = wid > 0 ? 1 : 0, tb = wid == 2 ? 1 : 0;
-    if (tid < CH) {
-        const int r = min(tid, n - 1);
+    if (wid == 3 && lane < CH) {
+        const int r = min(lane, n - 1);
         const float* bg = p.bg + ((row0 + r) * p.heads + h) * 2;
-        beta_s[tid] = bg[0];
-        double sum = tid < n ? (double)bg[1] : 0.0;
+        beta_s[lane] = bg[0];
+        double sum = lane < n ? (double)bg[1] : 0.0;
 #pragma unroll
         for (int o = 1; o < CH; o *= 2) {
             const double before = __shfl_up(sum, o, CH);
-            if (tid >= o) sum += before;
+            if (lane >= o) sum += before;
         }
-        cum[tid] = sum;
+        cum[lane] = sum;
+        eg_s[lane] = expf((float)sum);
     }
     f32x4 kk = {0.f, 0.f, 0.f, 0.f}, qk = kk;
-    const long ra = min(16 * ta + li, n - 1), rb = min(16 * tb + li, n - 1);
-    const float* ka = p.k + k0 + ra * p.dkp;
-    const float* qa = p.q + k0 + ra * p.dkp;
-    const float* kb = p.k + k0 + rb * p.dkp;
-    for (int d = 0; d < p.dkp; d += 64) {              // four 16-wide steps in flight; steps past the end are not multiplied
-        f32x4 a[4], b[4], q[4];
+    if (wid < 3) {
+        const long ra = min(16 * ta + li, n - 1), rb = min(16 * tb + li, n - 1);
+        const float *ka = K + ra * p.dkp + 4 * g, *qa = Q + ra * p.dkp + 4 * g, *kb = K + rb * p.dkp + 4 * g;
+        for (int d = 0; d < p.dkp; d += 64) {          // four 16-wide steps in flight; steps past the end are not multiplied
+            f32x4 a[4], b[4], q[4];
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            const int o = min(d + 16 * e, p.dkp - 16);
-            a[e] = *reinterpret_cast<const f32x4*>(ka + o);
-            b[e] = *reinterpret_cast<const f32x4*>(kb + o);
-            q[e] = *reinterpret_cast<const f32x4*>(qa + o);
-        }
-        __builtin_amdgcn_sched_barrier(0);
+            for (int e = 0; e < 4; ++e) {
+                const int o = min(d + 16 * e, p.dkp - 16);
+                a[e] = *reinterpret_cast<const f32x4*>(ka + o);
+                b[e] = *reinterpret_cast<const f32x4*>(kb + o);
+                q[e] = *reinterpret_cast<const f32x4*>(qa + o);
+            }
+            __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            if (d + 16 * e >= p.dkp) break;
-            kk = mfma4(a[e], b[e], kk);
-            qk = mfma4(q[e], b[e], qk);
+            for (int e = 0; e < 4; ++e) {
+                if (d + 16 * e >= p.dkp) break;
+                kk = mfma4(a[e], b[e], kk);
+                qk = mfma4(q[e], b[e], qk);
+            }
         }
     }
+    const int kt = p.dkp >> 4;
+    auto piece = [&](int t, f32x4 (&x)[2]) {           // 16 columns of K, as the operand of tokens 4 g + r (0 .. 15) and 16 + 4 g + r
+#pragma unroll
+        for (int a = 0; a < 2; ++a)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) x[a][r] = K[(long)min(16 * a + 4 * g + r, n - 1) * p.dkp + 16 * t + li];
+    };
+    f32x4 x[2][2];                                     // two pieces on the way
+    piece(min(wid, kt - 1), x[0]);
+    piece(min(wid + 4, kt - 1), x[1]);
     __syncthreads();
-    float* rec = chunk_rec(p, s, seq, chunk, h);
-    const int j = 16 * tb + li;
+    if (wid < 3) {
+        const int j = 16 * tb + li;
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-        const int i = 16 * ta + 4 * g + r;
-        const float e = j <= i ? expf((float)(cum[i] - cum[j])) : 0.f;
-        const bool in = i < n && j < n;
-        Ls[wid][4 * g + r][li] = in && j < i ? beta_s[i] * e * kk[r] : 0.f;
-        rec[(3 + wid) * TILE + (4 * g + r) * 16 + li] = in && j <= i ? e * qk[r] : 0.f;
-    }
-    if (tid < CH) {
-        rec[6 * TILE + tid] = expf((float)cum[tid]);
-        rec[6 * TILE + CH + tid] = tid < n ? expf((float)(cum[CH - 1] - cum[tid])) : 0.f;
-        if (tid == 0) rec[6 * TILE + 2 * CH] = expf((float)cum[CH - 1]);
-    }
-    __syncthreads();
-    // inverses of the two diagonal blocks: a lane per column
-    if (wid == 0 && lane < 32) {
-        const int blk = lane >> 4, b = blk * 2, c = li;
-        float x[16];
-#pragma unroll
-        for (int i = 0; i < 16; ++i) {
-            float v = i == c ? 1.f : 0.f;
-#pragma unroll
-            for (int m = 0; m < i; ++m) v = fmaf(-Ls[b][i][m], x[m], v);
-            x[i] = v;
-            Ts[b][i][c] = v;
+        for (int r = 0; r < 4; ++r) {
+            const int i = 16 * ta + 4 * g + r;
+            const float e = j <= i ? expf((float)(cum[i] - cum[j])) : 0.f;
+            const bool in = i < n && j < n;
+            kk[r] = in && j < i ? beta_s[i] * e * kk[r] : 0.f;                   // L
+            rec[wid * TILE + (li & 3) * 64 + (li >> 2) * 16 + 4 * g + r] = in && j <= i ? e * qk[r] : 0.f;      // [step][lane] of the scan's A operands
         }
+    } else if (lane < CH) {
+        rec[EXPS + lane] = eg_s[lane];
+        rec[EXPS + CH + lane] = lane < n ? expf((float)(cum[CH - 1] - cum[lane])) : 0.f;
+        if (lane == 0) rec[EXPS + 2 * CH] = eg_s[CH - 1];
+    }
+    if (wid == 1) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) L10[4 * g + r][li] = kk[r];
+    } else if (wid < 3) {                              // inverse of a diagonal block: a lane per column, L from its registers
+        float z[16];
+#pragma unroll
+        for (int i = 0; i < 16; ++i) z[i] = i == li ? 1.f : 0.f;
+#pragma unroll
+        for (int m = 0; m < 15; ++m)
+#pragma unroll
+            for (int i = m + 1; i < 16; ++i)
+                z[i] = fmaf(-__uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(kk[i & 3]), (i >> 2) * 16 + m)), z[m], z[i]);
+        if (lane < 16)
+#pragma unroll
+            for (int i = 0; i < 16; ++i) Ts[wid][i][lane] = z[i];
     }
     __syncthreads();
     // T(1,0) = -T(1,1) L(1,0) T(0,0)
@@ -288,225 +312,249 @@ __global__ __launch_bounds__(192) void delta_chunk_kernel(CogsDelta p) {
         f32x4 b, m = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int r = 0; r < 4; ++r) b[r] = Ts[0][4 * g + r][li];
-        m = mfma4(frag(&Ls[1][0][0], 20, li, g), b, m);
+        m = mfma4(frag(&L10[0][0], 20, li, g), b, m);
         f32x4 t = mfma4(frag(&Ts[2][0][0], 20, li, g), m, f32x4{0.f, 0.f, 0.f, 0.f});
 #pragma unroll
         for (int r = 0; r < 4; ++r) Ts[1][4 * g + r][li] = -t[r];
     }
     __syncthreads();
+    // T diag(beta) for the scan, and -that diag(e^G): row li, tokens 4 g + r
+    f32x4 te[3];
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-        const int i = 16 * ta + 4 * g + r;
-        rec[wid * TILE + (4 * g + r) * 16 + li] = i < n && j < n ? Ts[wid][4 * g + r][li] * beta_s[j] : 0.f;
+    for (int w = 0; w < 3; ++w) {
+        const int i = (w > 0 ? 16 : 0) + li, j = (w == 2 ? 16 : 0) + 4 * g;
+        const f32x4 t = frag(&Ts[w][0][0], 20, li, g), be = *reinterpret_cast<const f32x4*>(beta_s + j), e = *reinterpret_cast<const f32x4*>(eg_s + j);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const float v = i < n && j + r < n ? t[r] * be[r] : 0.f;
+            te[w][r] = -v * e[r];
+            if (wid == w) rec[(3 + w) * TILE + r * 64 + lane] = v;
+        }
+    }
+    const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+    auto product = [&](int t, const f32x4 (&v)[2]) {   // transposed: a lane ends with four neighbours of a row of W
+        float* o = rec + REC + (t * 64 + lane) * 4;
+        *reinterpret_cast<f32x4*>(o) = mfma4(v[0], te[0], zero);
+        *reinterpret_cast<f32x4*>(o + kt * TILE) = mfma4(v[1], te[2], zero) + mfma4(v[0], te[1], zero);
+    };
+    for (int t = wid; t < kt; t += 8) {
+        product(t, x[0]);
+        piece(min(t + 8, kt - 1), x[0]);
+        if (t + 4 < kt) product(t + 4, x[1]);
+        piece(min(t + 12, kt - 1), x[1]);
     }
 }
 
-// what a wave needs of one chunk; loaded one chunk ahead
+// what a wave needs of one chunk
 template <int NK>
 struct ScanIn {
-    f32x4 tm[3], pm[2], eg[2], ec[2], v[2], k[2][NK], q[2][NK], kt[2][NK];
-    float gl;
+    f32x4 w[2][NK], q[2][NK], kt[2][NK], eg[2], ec[2];
+    float pm[3], tm[3], v[2], gl;
 };
 
-// NK: 16-row tiles of S per wave. A chunk: S^T k from the state (partial sums of the waves meet in LDS: one barrier), then, while they
-// do, S^T q; U; the new state beside P U. The read-outs' partial sums ride on the next chunk's barrier, and waves 0 and 1 finish and
-// store 16 rows of them each behind it (waves 2 and 3 form copies of P U that nobody reads: they would wait otherwise). One wave per
-// SIMD issues in order, so the next chunk's loads are spread between the matrix instructions, and no product is one long chain.
+// NK: 16-row tiles of S per wave. A chunk: U = T diag(beta) V + W S, in partial sums over the waves' rows of S (and a quarter of
+// T diag(beta) V each) that meet in LDS (one barrier); while they do, Q S; then the new state and, beside it, a quarter of P U per wave
+// into the partial read-outs. Those ride on the next chunk's barrier, and every wave finishes a quarter of them behind it. One wave per
+// SIMD issues in order, so everything else -- the next chunk's loads, scaling, sums -- stands between matrix instructions that do not
+// need it (sched_barrier keeps it there). T diag(beta) V, P U and the state's growth are sums of their own: chained to what they are
+// added to, they were rounded at its size (error of the read-outs against fp64 2.5e-7 of them instead of 2.0e-7).
 template <int NK>
-__global__ __launch_bounds__(256, 1) void delta_scan_kernel(CogsDelta p) {
+__global__ __launch_bounds__(256, NK > 2 ? 1 : 2) void delta_scan_kernel(CogsDelta p) {
     __shared__ __attribute__((aligned(16))) f32x4 red[2][4][4][64];
-    // workgroups go round the XCDs: the columns of a head stay on one, whose L2 then serves its K and Q once
+    // workgroups go round the XCDs: the columns of a head stay on one, whose L2 then serves its W, K and Q once
     const int ng = p.dvp >> 4, place = blockIdx.x >> 3, h = (blockIdx.x & 7) + 8 * (place / ng), col0 = (place % ng) * 16, seq = blockIdx.z;
     if (h >= p.heads) return;
     const CogsSeq s = p.seqs[seq];
     const int tid = threadIdx.x, lane = tid & 63, li = lane & 15, g = lane >> 4;
-    const int wid = __builtin_amdgcn_readfirstlane(tid >> 6), half = wid & 1;
+    const int wid = __builtin_amdgcn_readfirstlane(tid >> 6), half = wid & 1, fin = wid >> 1;
     const int kh = h / (p.heads / p.kv_heads);
     const int ld = p.dkp, ldv = p.dvp;
-    const float* K = p.k + ((long)kh * p.rows + s.row0) * ld;
-    const float* Q = p.q + ((long)kh * p.rows + s.row0) * ld;
-    const float* V = p.v + ((long)h * p.rows + s.row0) * ldv + col0;
     float* O = p.o + ((long)h * p.rows + s.row0) * ldv + col0;
     float* S = s.state + p.state_off + (long)h * p.dkp * p.dvp + col0 + li;
     const int tiles = p.dkp >> 4;
     f32x4 st[NK];
-    int tn[NK];                                  // tiles past the end repeat the last one, and their S is kept at zero
-    float live[NK];
+    int tn[NK];                                  // tiles past the end repeat the last one, and their S stays zero
 #pragma unroll
     for (int n = 0; n < NK; ++n) {
         st[n] = f32x4{0.f, 0.f, 0.f, 0.f};
         const int t = wid + 4 * n;
-        tn[n] = 16 * min(t, tiles - 1);
-        live[n] = t < tiles ? 1.f : 0.f;
+        tn[n] = min(t, tiles - 1);
         if (t < tiles && s.pos0 > 0)
 #pragma unroll
             for (int r = 0; r < 4; ++r) st[n][r] = S[(long)(16 * t + 4 * g + r) * p.dvp];
     }
     const int nc = (s.len + CH - 1) / CH;
-    // a lane's places in a chunk's rows (bytes); a ragged last chunk repeats its last row
-    unsigned ko[2], to[2][4], vo[2][4], oo[4];
+    // a lane's places in a chunk's rows (bytes)
+    int qo[2], to[2][4], vo[2], oo[2];
+    const int wo = lane * 16, po = lane * 4 + wid * 256, ego = 16 * g;
+    int zo = 0;
+    asm("" : "+v"(zo));                          // (a scalar load would share its counter with LDS)
 #pragma unroll
-    for (int r = 0; r < 4; ++r) oo[r] = ((16 * half + 4 * g + r) * ldv + li) * 4;
-    const unsigned ro = (li * 16 + 4 * g) * 4, ego = 16 * g;
-    auto places = [&](int valid) {
+    for (int r = 0; r < 2; ++r) oo[r] = ((16 * fin + 4 * g + 2 * half + r) * ldv + li) * 4;
 #pragma unroll
-        for (int a = 0; a < 2; ++a) {
-            ko[a] = (min(16 * a + li, valid - 1) * ld + 4 * g) * 4;
+    for (int a = 0; a < 2; ++a) {
+        vo[a] = ((16 * a + 4 * g + wid) * ldv + li) * 4;
+        qo[a] = ((16 * a + li) * ld + 4 * g) * 4;
 #pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int row = min(16 * a + 4 * g + r, valid - 1);
-                to[a][r] = (row * ld + li) * 4;
-                vo[a][r] = (row * ldv + li) * 4;
-            }
-        }
+        for (int r = 0; r < 4; ++r) to[a][r] = ((16 * a + 4 * g + r) * ld + li) * 4;
+    }
+    // buffer loads: a scalar base per array and chunk, a lane's place, a scalar piece -- no address arithmetic per load; rows past the
+    // sequence's end, and K's columns of a tile past S's end, lie behind the buffer's size and read as zero
+    struct From { float *k, *q, *v, *rec; };
+    const From f0{p.k + ((long)kh * p.rows + s.row0) * ld, p.q + ((long)kh * p.rows + s.row0) * ld, p.v + ((long)h * p.rows + s.row0) * ldv + col0, chunk_rec(p, s, seq, 0, h)};
+    From f = f0;
+    const int bytes_rec = rec_floats(ld) * 4;
+    int bytes_q, bytes_v, bytes_k[NK];
+    auto sizes = [&](int rows) {
+        bytes_q = rows * ld * 4;
+        bytes_v = (rows - 1) * ldv * 4 + 64;
+#pragma unroll
+        for (int n = 0; n < NK; ++n) bytes_k[n] = wid + 4 * n < tiles ? bytes_q : 0;
     };
-    places(CH);
-    auto at4 = [](const float* base, unsigned bytes) { return *reinterpret_cast<const f32x4*>(reinterpret_cast<const char*>(base) + bytes); };
-    auto at1 = [](const float* base, unsigned bytes) { return *reinterpret_cast<const float*>(reinterpret_cast<const char*>(base) + bytes); };
-    // load i of a chunk: the 12 NK + 18 of them in the order of their use
-    struct From { const float *k, *q, *v, *rec; };
-    From f{K, Q, V, chunk_rec(p, s, seq, 0, h)};
-    const long step_k = (long)CH * ld, step_v = (long)CH * ldv, step_rec = (long)p.heads * REC;
+    sizes(min(CH, s.len));
+    auto at4 = [](float* base, int size, int lane_off, int off) {
+        return __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(__builtin_amdgcn_make_buffer_rsrc(base, 0, size, 0x00020000), lane_off, off, 0));
+    };
+    auto at1 = [](float* base, int size, int lane_off, int off) {
+        return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(__builtin_amdgcn_make_buffer_rsrc(base, 0, size, 0x00020000), lane_off, off, 0));
+    };
+    const long step_k = (long)CH * ld, step_v = (long)CH * ldv, step_rec = (long)p.heads * rec_floats(ld);
     int at = 0;                                                // the chunk f points to
     auto advance = [&] {                                       // (the last chunk is loaded again rather than nothing)
-        if (at + 1 >= nc) return;
-        ++at;
-        f.k += step_k; f.q += step_k; f.v += step_v; f.rec += step_rec;
-        if ((at + 1) * CH > s.len) places(s.len - at * CH);
+        at = min(at + 1, nc - 1);
+        f = From{f0.k + at * step_k, f0.q + at * step_k, f0.v + at * step_v, f0.rec + at * step_rec};
+        sizes(min(CH, s.len - at * CH));
     };
-    constexpr int L_K = 2 * NK, L_V = L_K + 8, L_TM = L_V + 3, L_EG = L_TM + 2, L_Q = L_EG + 2 * NK, L_EC = L_Q + 2, L_KT = L_EC + 8 * NK, L_ALL = L_KT + 3;
+    // load i of a chunk, in the order of their use
+    constexpr int L_U = 5, L_W = L_U + 2 * NK, L_Q = L_W + 2 * NK, L_E = L_Q + 4, L_G = L_E + 1, L_KT = L_G + 8 * NK, L_ALL = L_KT + 3;
     auto load = [&](ScanIn<NK>& in, int i) {
-        if (i < L_K) in.k[i & 1][i >> 1] = at4(f.k + tn[i >> 1], ko[i & 1]);
-        else if (i < L_V) in.v[(i - L_K) >> 2][(i - L_K) & 3] = at1(f.v, vo[(i - L_K) >> 2][(i - L_K) & 3]);
-        else if (i < L_TM) in.tm[i - L_V] = at4(f.rec + (i - L_V) * TILE, ro);
-        else if (i < L_EG) in.eg[i - L_TM] = at4(f.rec + 6 * TILE + 16 * (i - L_TM), ego);
-        else if (i < L_Q) in.q[(i - L_EG) & 1][(i - L_EG) >> 1] = at4(f.q + tn[(i - L_EG) >> 1], ko[(i - L_EG) & 1]);
-        else if (i < L_EC) in.ec[i - L_Q] = at4(f.rec + 6 * TILE + CH + 16 * (i - L_Q), ego);
-        else if (i < L_KT) in.kt[((i - L_EC) >> 2) & 1][(i - L_EC) >> 3][(i - L_EC) & 3] = at1(f.k + tn[(i - L_EC) >> 3], to[((i - L_EC) >> 2) & 1][(i - L_EC) & 3]);
-        else if (i < L_ALL - 1) in.pm[i - L_KT] = at4(f.rec + (3 + half + (i - L_KT)) * TILE, ro);      // half 0: P(0,0) and one without use; 1: P(1,0), P(1,1)
-        else if (i < L_ALL) in.gl = f.rec[6 * TILE + 2 * CH];
+        if (i < 2) in.v[i] = at1(f.v, bytes_v, vo[i], 0);
+        else if (i < L_U) in.tm[i - 2] = at1(f.rec, bytes_rec, po, (1 + i) * TILE * 4);
+        else if (i < L_W) { const int j = i - L_U; in.w[j / NK][j % NK] = at4(f.rec, bytes_rec, wo, (REC + ((j / NK) * tiles + tn[j % NK]) * TILE) * 4); }
+        else if (i < L_Q) { const int j = i - L_W; in.q[j / NK][j % NK] = at4(f.q, bytes_q, qo[j / NK], 64 * tn[j % NK]); }
+        else if (i < L_E) { const int j = i - L_Q; (j & 2 ? in.eg : in.ec)[j & 1] = at4(f.rec, bytes_rec, ego, (EXPS + (j & 2 ? 0 : CH) + 16 * (j & 1)) * 4); }
+        else if (i < L_G) in.gl = at1(f.rec, bytes_rec, zo, (EXPS + 2 * CH) * 4);
+        else if (i < L_KT) { const int j = i - L_G; in.kt[(j >> 2) & 1][j >> 3][j & 3] = at1(f.k, bytes_k[j >> 3], to[(j >> 2) & 1][j & 3], 64 * tn[j >> 3]); }
+        else if (i < L_ALL) in.pm[i - L_KT] = at1(f.rec, bytes_rec, po, (i - L_KT) * TILE * 4);
     };
     const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
-    const float second = half ? 1.f : 0.f;                     // rows 0 .. 15 have no P(0,1)
-    f32x4 y[2] = {zero, zero}, po = zero, peg = zero;          // the previous chunk's: partial S^T q, P U and e^G of this wave's rows
-    auto sum4 = [&](f32x4 (*rd)[4][64], int a) { return (rd[0][a][lane] + rd[1][a][lane]) + (rd[2][a][lane] + rd[3][a][lane]); };
-    auto store = [&](int c, const f32x4& o, bool ragged) {
-        float* oc = O + (long)c * CH * ldv;
+    f32x4 y[2] = {zero, zero};                                 // the previous chunk's read-outs, this wave's part of the sums
+    auto gather = [&](f32x2 (&o)[4], f32x4 (*rd)[4][64]) {
 #pragma unroll
-        for (int r = 0; r < 4; ++r)
-            if (!ragged || c * CH + 16 * half + 4 * g + r < s.len) *reinterpret_cast<float*>(reinterpret_cast<char*>(oc) + oo[r]) = o[r];
+        for (int w = 0; w < 4; ++w) o[w] = *(reinterpret_cast<const f32x2*>(&rd[w][2 + fin][lane]) + half);
     };
-    auto meet = [&] {                                          // (loads of the next chunk stay in flight)
+    auto finish = [&](int c, const f32x2 (&o)[4], bool ragged) {
+        float* oc = O + (long)c * CH * ldv;
+        const f32x2 t = (o[0] + o[1]) + (o[2] + o[3]);
+#pragma unroll
+        for (int r = 0; r < 2; ++r)
+            if (!ragged || c * CH + 16 * fin + 4 * g + 2 * half + r < s.len) *reinterpret_cast<float*>(reinterpret_cast<char*>(oc) + oo[r]) = t[r];
+    };
+    auto meet = [&] {                                          // (loads of later chunks stay in flight)
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
     };
     auto mfma = [](float a, float b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); };
+    auto mine = [&](const f32x4& v) { return wid < 2 ? (wid == 0 ? v[0] : v[1]) : (wid == 2 ? v[2] : v[3]); };
+    auto pin = [](f32x4 (&v)[4]) { asm volatile("" : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]), "+v"(v[3])); };      // (used from here on, no earlier)
     // chunk c from `in`, the next one into nx
     auto chunk = [&](int c, const ScanIn<NK>& in, ScanIn<NK>& nx) {
-        advance();
-        constexpr int STEPS = 8 * NK + 8 * NK / 2 + 6;         // pairs of matrix instructions
-        int step = 0, done = 0;
-        auto feed = [&] {                                      // this pair's share of the loads
+        constexpr int STEPS = 24 * NK;                         // matrix instructions that bring loads with them
+        static_assert(L_ALL + L_E - L_U <= 2 * STEPS);
+        constexpr int LONG = L_E - L_U, WORK = L_ALL + LONG;   // the four waves' 16-byte loads take the time of two matrix instructions, the others half
+        int step = 0, next = 0;
+        auto due = [&] { return next < L_ALL && (next + (next > L_U ? min(next - L_U, LONG) : 0)) * STEPS < (step + 1) * WORK; };
+        auto feed = [&] {
+            if (due()) load(nx, next++);
+            if (due()) load(nx, next++);
             ++step;
-#pragma unroll
-            for (int i = 0; i < L_ALL; ++i)
-                if (i >= done && i < (L_ALL * step + STEPS - 1) / STEPS) load(nx, i);
-            done = (L_ALL * step + STEPS - 1) / STEPS;
             __builtin_amdgcn_sched_barrier(0);
         };
-        f32x4 x[2][2] = {{zero, zero}, {zero, zero}};          // [16 rows][half of the depth]
-#pragma unroll
-        for (int n = 0; n < NK; ++n)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-#pragma unroll
-                for (int a = 0; a < 2; ++a) x[a][r & 1] = mfma(in.k[a][n][r], st[n][r], x[a][r & 1]);
-                feed();
-            }
         f32x4 (*rd)[4][64] = red[c & 1];
+        f32x4 x[2], o[2], odd, tv[2];
+        auto qs = [&](int a, int i) {
+            o[a] = mfma(in.q[a][i >> 2][i & 3], st[i >> 2][i & 3], i < 1 ? zero : o[a]);
+            feed();
+        };
 #pragma unroll
-        for (int a = 0; a < 2; ++a) {
-            rd[wid][2 + a][lane] = y[a];
-            rd[wid][a][lane] = x[a][0] + x[a][1];
-        }
-        meet();
-        f32x4 part[3][4];
+        for (int a = 0; a < 2; ++a) {                          // (one 16 rows after the other: the first ones' sums travel meanwhile)
+            if (a == 0) {
+                tv[0] = mfma(in.tm[0], in.v[0], zero);
+                advance();
+                tv[1] = mfma(in.tm[1], in.v[0], zero);
+                tv[1] = mfma(in.tm[2], in.v[1], tv[1]);
+                __builtin_amdgcn_sched_barrier(0);
+            }
 #pragma unroll
-        for (int a = 0; a < 3; ++a)
-#pragma unroll
-            for (int w = 0; w < 4; ++w) part[a][w] = rd[w][a < 2 ? a : 2 + half][lane];
-        __builtin_amdgcn_sched_barrier(0);
-        y[0] = y[1] = zero;
-        f32x4 y2[2] = {zero, zero};
-#pragma unroll
-        for (int n = 0; n < NK; ++n)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-#pragma unroll
-                for (int a = 0; a < 2; ++a) {
-                    f32x4& t = (r & 1) ? y2[a] : y[a];
-                    t = mfma(in.q[a][n][r], st[n][r], t);
-                }
+            for (int i = 0; i < 4 * NK; ++i) {
+                x[a] = mfma(in.w[a][i >> 2][i & 3], st[i >> 2][i & 3], i < 1 ? zero : x[a]);
+                if (i == 1) rd[wid][a == 0 ? 2 : 3][lane] = y[a];
+                if (i == 2 && a == 1) rd[wid][0][lane] = x[0];
                 feed();
             }
-        f32x4 rr[2], u[2] = {zero, zero}, u1 = zero;
+            x[a] += tv[a];
+        }
+        qs(0, 0);
+        rd[wid][1][lane] = x[1];
+        qs(0, 1);
+        qs(0, 2);
+        meet();
+        f32x4 part[2][4], u[2], ue[2], grow[NK];
+        f32x2 fo[4];
 #pragma unroll
         for (int a = 0; a < 2; ++a) {
-            rr[a] = in.v[a] - in.eg[a] * ((part[a][0] + part[a][1]) + (part[a][2] + part[a][3]));
-            y[a] += y2[a];
+#pragma unroll
+            for (int w = 0; w < 4; ++w) part[a][w] = rd[w][a][lane];
+            __builtin_amdgcn_sched_barrier(0);
         }
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {                          // three chains
-            u[0] = mfma(in.tm[0][r], rr[0][r], u[0]);
-            u[1] = mfma(in.tm[1][r], rr[0][r], u[1]);
-            if (r & 1) feed();
-            u1 = mfma(in.tm[2][r], rr[1][r], u1);
+        for (int i = 3; i < 8 * NK; ++i) {
+            qs(i / (4 * NK), i % (4 * NK));
+            if (i == 8 * NK - 3) { pin(part[0]); u[0] = (part[0][0] + part[0][1]) + (part[0][2] + part[0][3]); }
+            if (i == 8 * NK - 2) { ue[0] = u[0] * in.ec[0]; gather(fo, rd); }
+        }
+        pin(part[1]);
+#pragma unroll
+        for (int i = 0; i < 8 * NK; ++i) {
+            // rows of the chunk's first half before the second's, so that U's second half has time
+            const int n = (i >> 2) % NK, a = (i >> 2) / NK, r = i & 3;
+            if (i == 1) u[1] = (part[1][0] + part[1][1]) + (part[1][2] + part[1][3]);
+            if (i == 2) ue[1] = u[1] * in.ec[1];
+            grow[n] = mfma(in.kt[a][n][r], ue[a][r], a == 0 && r == 0 ? zero : grow[n]);
+            if (a == 1 && n > 0 && r == 1) st[n - 1] = st[n - 1] * in.gl + grow[n - 1];        // (summed by itself: one rounding of S per chunk)
+            if (i == 3) { const float m = mine(u[0]); y[0] = mfma(in.pm[0], m, zero); y[1] = mfma(in.pm[1], m, zero); }
+            if (i == 4) y[1] = mfma(in.pm[2], mine(u[1]), y[1]);
+            if (i == 5) y[0] += o[0] * in.eg[0];
+            if (i == 6) y[1] += o[1] * in.eg[1];
+            if (i == 6 && c > 0) finish(c - 1, fo, false);
             feed();
         }
-        u[1] += u1;
-        const f32x4 o = po + peg * ((part[2][0] + part[2][1]) + (part[2][2] + part[2][3]));
-        f32x4 ue[2], pa = zero, pb = zero, s2[NK];
-        const f32x4 up = u[1] * second;
-#pragma unroll
-        for (int a = 0; a < 2; ++a) ue[a] = u[a] * in.ec[a];
-#pragma unroll
-        for (int n = 0; n < NK; ++n) {
-            st[n] *= in.gl;
-            s2[n] = zero;
-        }
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-#pragma unroll
-            for (int n = 0; n < NK; ++n) {
-                st[n] = mfma(in.kt[0][n][r], ue[0][r], st[n]);
-                s2[n] = mfma(in.kt[1][n][r], ue[1][r], s2[n]);
-                feed();
-            }
-            pa = mfma(in.pm[0][r], u[0][r], pa);
-            pb = mfma(in.pm[1][r], up[r], pb);
-        }
-#pragma unroll
-        for (int n = 0; n < NK; ++n) st[n] = (st[n] + s2[n]) * live[n];
-        po = pa + pb;
-        peg = half ? in.eg[1] : in.eg[0];
-        if (c > 0 && wid < 2) store(c - 1, o, false);
+        st[NK - 1] = st[NK - 1] * in.gl + grow[NK - 1];
     };
     ScanIn<NK> in0, in1;
-    if (s.len < CH) places(s.len);
 #pragma unroll
-    for (int i = 0; i < L_ALL; ++i) load(in0, i);
-    for (int c = 0; c < nc; c += 2) {
-        chunk(c, in0, in1);
-        if (c + 1 >= nc) break;
-        chunk(c + 1, in1, in0);
+    for (int i = 0; i < L_ALL; ++i) {
+        load(in0, i);
+        __builtin_amdgcn_sched_barrier(0);                     // (in this order: the waits count on it)
     }
+    // the first chunk in front of the loop, and no exit in the loop's middle: the loads then stand in the same order on every way to a
+    // wait, and none waits for all of them
+    chunk(0, in0, in1);
+    int c = 1;
+    for (; c + 1 < nc; c += 2) {
+        chunk(c, in1, in0);
+        chunk(c + 1, in0, in1);
+    }
+    if (c < nc) chunk(c, in1, in0);
     {
         f32x4 (*rd)[4][64] = red[nc & 1];
+        f32x2 fo[4];
 #pragma unroll
         for (int a = 0; a < 2; ++a) rd[wid][2 + a][lane] = y[a];
         meet();
-        if (wid < 2) store(nc - 1, po + peg * sum4(rd, 2 + half), true);
+        gather(fo, rd);
+        finish(nc - 1, fo, true);
     }
 #pragma unroll
     for (int n = 0; n < NK; ++n) {
@@ -675,7 +723,7 @@ bool sizes_ok(const CogsDelta& a) {
 
 }  // namespace
 
-size_t cogs_k_delta_rec_floats(int rows, int nseq, int heads) { return (size_t)(rows / CH + nseq) * heads * REC; }
+size_t cogs_k_delta_rec_floats(int rows, int nseq, int heads, int dkp) { return (size_t)(rows / CH + nseq) * heads * rec_floats(dkp); }
 
 int cogs_k_delta_prompt(hipStream_t st, int dtype, const CogsDelta& a, int rows, int nseq, int max_new) {
     if (!sizes_ok(a) || rows <= 0 || nseq <= 0 || nseq > 65535 || a.heads > 65535) return COGS_E_INVALID;
@@ -683,7 +731,7 @@ int cogs_k_delta_prompt(hipStream_t st, int dtype, const CogsDelta& a, int rows,
     const int keep = (max_new < a.taps ? max_new : a.taps) * a.channels;
     hipLaunchKernelGGL(delta_tail_kernel, dim3((keep + 1023) / 1024, nseq), dim3(256), 0, st, a);
     if (a.dkp <= 256 && g_cogs_debug.delta_chunk != 0) {
-        hipLaunchKernelGGL(delta_chunk_kernel, dim3((max_new + CH - 1) / CH, a.heads, nseq), dim3(192), 0, st, a);
+        hipLaunchKernelGGL(delta_chunk_kernel, dim3((max_new + CH - 1) / CH, a.heads, nseq), dim3(256), 0, st, a);
         const dim3 grid((a.heads + 7) / 8 * 8 * (a.dvp / 16), 1, nseq);
         if (a.dkp <= 64) hipLaunchKernelGGL(delta_scan_kernel<1>, grid, dim3(256), 0, st, a);
         else if (a.dkp <= 128) hipLaunchKernelGGL(delta_scan_kernel<2>, grid, dim3(256), 0, st, a);

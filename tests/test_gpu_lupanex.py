@@ -386,6 +386,28 @@ def test_sublayer_outputs_in_partial_sums(dev, rows, width, ff):
     assert rms_err(got, lo.forward(cfg, double(st), toks)[0]) < TOL[torch.bfloat16]
 
 
+@pytest.mark.parametrize("dim,vdim", [(16, 16), (64, 48), (80, 16), (128, 128), (144, 32), (256, 16)])
+def test_chunked_delta_rule_at_the_edges_of_its_tiles(dev, dim, vdim):
+    """every number of row tiles per wave, whole and ragged; chunks of one token, whole and ragged ones, one to four of them, from nothing
+    and from a state, unequal prompts together: within the tolerance of the oracle, and as close to it as the token-by-token form (both
+    sum in fp32, in another order: a quarter more at most, of errors that vary by a tenth from one sequence of words to the next)"""
+    from cogstream_amd import _lib as L
+    cfg = config([delta(heads=4, kv_heads=2, dim=dim, vdim=vdim, conv=4, ff=None)], width=64)
+    st = state(cfg)
+    toks = tokens(cfg, 130)
+    lg = lo.forward(cfg, double(st), toks)[0]
+    e = engine(cfg, st, torch.float32)
+    for cuts in ((), [1, 33, 64], [31], [32, 65, 97], [96], [128, 129]):
+        got = rms_err(run(e, toks, cuts), lg)
+        with L.debug_switch("delta_chunk", 0):
+            want = rms_err(run(e, toks, cuts), lg)
+        assert got < TOL[torch.float32] and got < 1.25 * want + 1e-7, (cuts, got, want)
+    s = sequences(e)
+    lens = [1, 33, 96, 130, 32]
+    out = s.step([(i, toks[:n], [n - 1]) for i, n in enumerate(lens)])
+    assert rms_err(out, lg[[n - 1 for n in lens]]) < TOL[torch.float32]
+
+
 def test_unsupported_calls_are_refused(dev):
     from cogstream_amd import _lib as L
     cfg, st, e, toks, _, _ = named("peaked", torch.bfloat16)
