@@ -158,13 +158,44 @@ template <> struct RawVec<float> {
     static __device__ __forceinline__ f32x4 to_f32(f32x4 w) { return w; }
 };
 
+// What epilogue_tile reads besides the accumulators, for a caller that asks for it in front of its product: behind the product these
+// loads are a round trip to memory of their own (1 to 2 us, twice for MI = 4) that nothing overlaps.
+template <typename T, int EPI, int MI, int NI>
+struct EpiOperands {
+    f32x4 bias[NI];
+    f32x2 cs[MI][NI], sn[MI][NI];
+    u32x4 res[MI][NI / 2];                       // where rows are stored in 16-byte units (see WIDE path below)
+    __device__ __forceinline__ void load(const EpiArgs& p, int mb, int nb, int M, int N, int lane) {
+        const int g4 = lane >> 4, wcol = 16 * (g4 & 1) + 8 * (g4 >> 1);
+#pragma unroll
+        for (int ni = 0; ni < NI; ++ni) {
+            const int n = min(nb + 4 * g4 + 16 * ni, N - 4);
+            if constexpr ((EPI & EPI_LNFOLD) != 0) bias[ni] = *reinterpret_cast<const f32x4*>(p.col_c + n);
+            else if constexpr ((EPI & EPI_BIAS) != 0) bias[ni] = ld4_f<T>(reinterpret_cast<const T*>(p.bias) + n);
+        }
+#pragma unroll
+        for (int mi = 0; mi < MI; ++mi) {
+            const int m = min(mb + (lane & 15) + 16 * mi, M - 1);
+            if constexpr ((EPI & EPI_ROPE) != 0)
+#pragma unroll
+                for (int ni = 0; ni < NI; ++ni) rope_load(p, m, (min(nb + 4 * g4 + 16 * ni, N - 4) % p.head_dim) >> 1, cs[mi][ni], sn[mi][ni]);
+            if constexpr ((EPI & EPI_RES) != 0)
+                if ((N & 31) == 0)
+#pragma unroll
+                    for (int pr = 0; pr < NI / 2; ++pr)
+                        res[mi][pr] = *reinterpret_cast<const u32x4*>(reinterpret_cast<const T*>(p.R) + (long)m * p.ldr + min(nb + 32 * pr, N - 32) + wcol);
+        }
+    }
+};
+
 // Epilogue of one wave's 16 MI x 16 NI tile held as acc[mi][ni] (lane: row mb + 16 mi + (lane&15), columns
 // nb + 16 ni + 4 (lane>>4) .. +3). Loads first, then math + stores. EPI_ROWSTAT over a 32-column tile (NI == 2) cannot close a
 // 64-column block: the lanes' sums of row block mi go to half_stats[mi] instead and the caller joins the two halves. row_scale: EPI_LNFOLD's factor of
-// row block mi's row, where the caller has it (else from ln_ab).
+// row block mi's row, where the caller has it (else from ln_ab). early: operands that are there already.
 template <typename T, int EPI, int MI = 4, int NI = 4>
 __device__ __forceinline__ void epilogue_tile(const EpiArgs& p, int mb, int nb, int M, int N, int lane,
-                                              f32x4 (&acc)[MI][NI], f32x2* half_stats = nullptr, const float* row_scale = nullptr) {
+                                              f32x4 (&acc)[MI][NI], f32x2* half_stats = nullptr, const float* row_scale = nullptr,
+                                              const EpiOperands<T, EPI, MI, NI>* early = nullptr) {
     const int mrow = mb + (lane & 15);
     const int ncol = nb + ((lane >> 4) << 2);
     if constexpr ((EPI & EPI_NOSTORE) != 0) {
@@ -208,7 +239,10 @@ __device__ __forceinline__ void epilogue_tile(const EpiArgs& p, int mb, int nb, 
         int nn[NI];
 #pragma unroll
         for (int i = 0; i < NI; ++i) nn[i] = min(ncol + i * 16, N - 4);
-        if constexpr ((EPI & EPI_LNFOLD) != 0) {
+        if (early) {
+#pragma unroll
+            for (int ni = 0; ni < NI; ++ni) bias_v[ni] = early->bias[ni];
+        } else if constexpr ((EPI & EPI_LNFOLD) != 0) {
 #pragma unroll
             for (int ni = 0; ni < NI; ++ni) bias_v[ni] = *reinterpret_cast<const f32x4*>(p.col_c + nn[ni]);
         } else if constexpr ((EPI & EPI_BIAS) != 0) {
@@ -235,7 +269,7 @@ __device__ __forceinline__ void epilogue_tile(const EpiArgs& p, int mb, int nb, 
                         for (int i = 0; i < 2; ++i)
 #pragma unroll
                             for (int pr = 0; pr < NI / 2; ++pr)
-                                res_wide[i][pr] = *reinterpret_cast<const u32x4*>(
+                                res_wide[i][pr] = early ? early->res[2 * half + i][pr] : *reinterpret_cast<const u32x4*>(
                                     reinterpret_cast<const T*>(p.R) + (long)mm[i] * p.ldr + min(nb + 32 * pr, N - 32) + wcol);
                     }
                 } else {
@@ -251,7 +285,8 @@ __device__ __forceinline__ void epilogue_tile(const EpiArgs& p, int mb, int nb, 
                 for (int i = 0; i < 2; ++i)
 #pragma unroll
                     for (int ni = 0; ni < NI; ++ni) {
-                        rope_load(p, mm[i], (nn[ni] % p.head_dim) >> 1, cs[i][ni], sn[i][ni]);
+                        if (early) { cs[i][ni] = early->cs[2 * half + i][ni]; sn[i][ni] = early->sn[2 * half + i][ni]; }
+                        else rope_load(p, mm[i], (nn[ni] % p.head_dim) >> 1, cs[i][ni], sn[i][ni]);
                     }
             }
 #pragma unroll

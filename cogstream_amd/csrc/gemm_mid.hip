@@ -135,6 +135,13 @@ __global__ __launch_bounds__(64 * WM * WN, WPE) void gemm_mid_kernel(MidArgs p) 
         }
     };
 
+    // what the epilogue reads, in front of the product where the registers are there to hold it (NI = 4 has none to spare):
+    // M = 256 of the vision encoder, N x K = 1152 x 4304 / 1152 with residual 13.5 -> 13.0 us, 4304 x 1152 14.6 -> 14.2; M = 1024
+    // 28.1 -> 27.0
+    const int mb = m0 + wm * 16 * MI, nb = n0 + wn * 16 * NI;
+    constexpr bool EARLY = NI == 2 && (EPI & EPI_GENERIC) == 0;
+    EpiOperands<bf16_t, EPI, MI, NI> early;
+    if constexpr (EARLY) early.load(p.epi, mb, nb, p.M, p.N, lane);
     for (int i = 0; i < S && i < KT; ++i) stage(i);
     // EPI_LNFOLD: the factors of this wave's rows while the ring fills; lane l has row l of its 16 MI
     float factor = 0.f;
@@ -184,19 +191,19 @@ __global__ __launch_bounds__(64 * WM * WN, WPE) void gemm_mid_kernel(MidArgs p) 
         if (kt < KT) tail(f1, f0);
     }
 
-    const int mb = m0 + wm * 16 * MI, nb = n0 + wn * 16 * NI;
+    const auto* operands = EARLY ? &early : nullptr;
     if constexpr ((EPI & EPI_LNFOLD) != 0) {
         float rs[MI];
 #pragma unroll
         for (int mi = 0; mi < MI; ++mi) rs[mi] = __shfl(factor, 16 * mi + (lane & 15));
-        epilogue_tile<bf16_t, EPI, MI, NI>(p.epi, mb, nb, p.M, p.N, lane, acc, nullptr, rs);
+        epilogue_tile<bf16_t, EPI, MI, NI>(p.epi, mb, nb, p.M, p.N, lane, acc, nullptr, rs, operands);
     } else if constexpr (MI == 4 && NI == 4) {
         epilogue_wave<bf16_t, EPI>(p.epi, mb, nb, p.M, p.N, lane, acc);
     } else if constexpr ((EPI & EPI_ROWSTAT) != 0 && NI == 2) {
         // a 64-column block's sums come from two waves; the pair is added lane by lane in the order of one 64-column wave, then
         // over the lanes, so the statistics have the same bits
         f32x2 st[MI];
-        epilogue_tile<bf16_t, EPI, MI, NI>(p.epi, mb, nb, p.M, p.N, lane, acc, st);
+        epilogue_tile<bf16_t, EPI, MI, NI>(p.epi, mb, nb, p.M, p.N, lane, acc, st, nullptr, operands);
         __syncthreads();                         // the ring is free
         f32x2* xch = reinterpret_cast<f32x2*>(smem) + (wid & ~1) * MI * 64 + lane;
         static_assert(WN % 2 == 0, "the two halves of a 64-column block are neighbouring waves");
@@ -216,7 +223,7 @@ __global__ __launch_bounds__(64 * WM * WN, WPE) void gemm_mid_kernel(MidArgs p) 
             }
         }
     } else {
-        epilogue_tile<bf16_t, EPI, MI, NI>(p.epi, mb, nb, p.M, p.N, lane, acc);
+        epilogue_tile<bf16_t, EPI, MI, NI>(p.epi, mb, nb, p.M, p.N, lane, acc, nullptr, nullptr, operands);
     }
 }
 
