@@ -299,7 +299,8 @@ __global__ __launch_bounds__(64) void mla_rowwise_kernel(CogsMla p) {
 }
 
 // ------------------------------------------------------------------------------------------------ prompt attention (bf16)
-// 4 waves x 32 query rows of one (sequence, head) against 64-key tiles. Staging as in attn.hip's prompt kernel: a tile's pieces
+// 4 waves x 32 query rows of one (sequence, head) against 64-key tiles; NH = 2: 8 waves, each half with every second tile, whose sums
+// meet at the end. Staging as in attn.hip's prompt kernel: a tile's pieces
 // (1 KiB = 64 lanes x 16 bytes) go global -> LDS by LDS-DMA into a double buffer, one tile ahead, one barrier per tile. Keys come
 // from two places -- the head's expanded part and the rotated part all heads share -- so a K tile is two LDS regions of KN and KR
 // 32-dimension steps. LDS-DMA writes lane-linear images: the bank swizzles live on the source address.
@@ -329,8 +330,8 @@ template <int DT> __device__ __forceinline__ int mla_vswz(int row) {
     else return b3;
 }
 
-template <int KN, int KR, int DT, int WGS>
-__global__ __launch_bounds__(256, WGS) void mla_prefill_kernel(CogsMla p, int nqt, int group) {
+template <int KN, int KR, int DT, int WPE, int NH>
+__global__ __launch_bounds__(256 * NH, WPE) void mla_prefill_kernel(CogsMla p, int nqt, int group) {
     constexpr int NQ = 2, KS = KN + KR;
     constexpr bool HEADS = KR == 0;
     constexpr int N_LDS = 64 * KN * 64, R_LDS = 64 * KR * 64, V_LDS = 64 * DT * 32, BUF = N_LDS + R_LDS + V_LDS;
@@ -338,8 +339,9 @@ __global__ __launch_bounds__(256, WGS) void mla_prefill_kernel(CogsMla p, int nq
     static_assert(DT % 2 == 0, "whole pieces per wave");
     extern __shared__ __attribute__((aligned(16))) char smem[];
 
-    const int tid = threadIdx.x, lane = tid & 63;
+    const int tid = threadIdx.x & 255, lane = tid & 63;
     const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int kh = NH == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x >> 8);         // this wave's share of the key tiles: kh, kh + NH, ..
     const int li = lane & 15, g = lane >> 4;
     // launch order -> (sequence, head) and query tile. An XCD gets a contiguous run, `group` (sequence, head) pairs at a time (their
     // K / V meet in its L2), long query tiles first; where a group is two waves of one workgroup per CU (<= 64), the second
@@ -351,7 +353,7 @@ __global__ __launch_bounds__(256, WGS) void mla_prefill_kernel(CogsMla p, int nq
         const int per = group * nqt, grp = bid / per, np = total / nqt;
         int i = bid - grp * per;
         const int gsz = min(group, np - grp * group), n = gsz * nqt;
-        if (n <= 64 && i >= 32) i = n - 1 - (i - 32);
+        if (NH == 1 && n <= 64 && i >= 32) i = n - 1 - (i - 32);
         qt = nqt - 1 - i / gsz;
         pair = grp * group + i % gsz;
     }
@@ -392,7 +394,8 @@ __global__ __launch_bounds__(256, WGS) void mla_prefill_kernel(CogsMla p, int nq
     const int p0 = s.pos0 + q0;                                                     // position of the workgroup's first row
     float b_far = 0.f;
     int t_far = 0;                                                                  // tiles [0, t_far) lie past the bias table's end
-    float* const win = reinterpret_cast<float*>(smem + 2 * BUF);
+    float* const win = reinterpret_cast<float*>(smem + 2 * NH * BUF);
+    auto slot = [&](int t) { return NH == 1 ? t & 1 : 2 * kh + ((t >> 1) & 1); };           // a tile's buffer
     if constexpr (HEADS) {
         if (p.bias) {
             b_far = p.bias[(long)h * p.nb + p.nb - 1];
@@ -456,7 +459,7 @@ __global__ __launch_bounds__(256, WGS) void mla_prefill_kernel(CogsMla p, int nq
         const bf16_t* kp = uniform_ptr(K + (long)kb * p.ldk);
         const bf16_t* rp = HEADS ? nullptr : uniform_ptr(KRp + (long)kb * p.ldkr);
         const bf16_t* vp = uniform_ptr(V + (long)kb * p.ldv);
-        const unsigned st = __builtin_amdgcn_readfirstlane(smem_lds + (t & 1) * BUF);
+        const unsigned st = __builtin_amdgcn_readfirstlane(smem_lds + slot(t) * BUF);
         const bool ragged = valid < 64;
 #pragma unroll
         for (int i = 0; i < KN; ++i) {
@@ -483,8 +486,8 @@ __global__ __launch_bounds__(256, WGS) void mla_prefill_kernel(CogsMla p, int nq
     // bias window of tile t: entry i is distance p0 - 63 - 64 t + i (queries below p0 + 128, keys 64 t .. 64 t + 63)
     auto stage_window = [&](int t) {
         if constexpr (HEADS)
-            if (t >= t_far && tid < MLA_WIN)
-                win[(t & 1) * MLA_WIN + tid] = p.bias[(long)h * p.nb + min(max(p0 - 63 - 64 * t + tid, 0), p.nb - 1)];
+            if (p.bias && t + NH > t_far && tid < MLA_WIN)     // (a round's tiles take one form)
+                win[slot(t) * MLA_WIN + tid] = p.bias[(long)h * p.nb + min(max(p0 - 63 - 64 * t + tid, 0), p.nb - 1)];
     };
 
     const int krow0 = 8 * (li >> 2) + (li & 3);
@@ -497,11 +500,11 @@ __global__ __launch_bounds__(256, WGS) void mla_prefill_kernel(CogsMla p, int nq
         constexpr bool NEAR = HEADS && decltype(near_tag)::value;
         const int kb = t * 64;
         if (!wave_active || (MASKED && kb > wave_hi)) return;
-        const char* Ns = smem + (t & 1) * BUF;
+        const char* Ns = smem + slot(t) * BUF;
         const char* Rs = Ns + N_LDS;
         const char* Vs = Rs + R_LDS;
         f32x4 sacc[4][NQ];
-        __builtin_amdgcn_s_setprio(0);
+        if (NH == 1) __builtin_amdgcn_s_setprio(0);
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
             const int krow = 32 * (u >> 1) + 4 * (u & 1) + krow0;
@@ -512,7 +515,7 @@ __global__ __launch_bounds__(256, WGS) void mla_prefill_kernel(CogsMla p, int nq
                 const float nm = HEADS && !NEAR ? b_far - m_ref[i] : -m_ref[i];
                 start[i] = f32x4{nm, nm, nm, nm};
                 if constexpr (NEAR) {
-                    const float* b = win + (t & 1) * MLA_WIN + (qpos[i] - p0 + 63 - (32 * (u >> 1) + 8 * g + 4 * (u & 1)));
+                    const float* b = win + slot(t) * MLA_WIN + (qpos[i] - p0 + 63 - (32 * (u >> 1) + 8 * g + 4 * (u & 1)));
 #pragma unroll
                     for (int r = 0; r < 4; ++r) start[i][r] += b[-r];
                 }
@@ -536,7 +539,7 @@ __global__ __launch_bounds__(256, WGS) void mla_prefill_kernel(CogsMla p, int nq
             }
             __builtin_amdgcn_sched_group_barrier(0x008, 12, 0);
         }
-        __builtin_amdgcn_s_setprio(1);
+        if (NH == 1) __builtin_amdgcn_s_setprio(1);
         bf16x8 pf[2][NQ][2];                           // [32-key step][row group][head, remainder]
 #pragma unroll
         for (int i = 0; i < NQ; ++i) {
@@ -549,8 +552,9 @@ __global__ __launch_bounds__(256, WGS) void mla_prefill_kernel(CogsMla p, int nq
                         if (kb + 32 * (u >> 1) + 8 * g + 4 * (u & 1) + r > qpos[i]) sacc[u][i][r] = -INFINITY;
                     d = fmaxf(d, sacc[u][i][r]);
                 }
-            if constexpr (FIRST) {                     // key 0 is visible to every row: finite
+            if constexpr (FIRST) {                     // key 0 is visible to every row: finite; a share that starts behind it may see nothing
                 d = col_max4(d);
+                if constexpr (NH > 1 && MASKED) d = d == -INFINITY ? 0.f : d;
 #pragma unroll
                 for (int u = 0; u < 4; ++u)
 #pragma unroll
@@ -582,7 +586,7 @@ __global__ __launch_bounds__(256, WGS) void mla_prefill_kernel(CogsMla p, int nq
                 pf[u][i][1] = __builtin_bit_cast(bf16x8, x);
             }
         }
-        __builtin_amdgcn_s_setprio(0);
+        if (NH == 1) __builtin_amdgcn_s_setprio(0);
 #pragma unroll
         for (int u = 0; u < 2; ++u)
 #pragma unroll
@@ -617,8 +621,12 @@ __global__ __launch_bounds__(256, WGS) void mla_prefill_kernel(CogsMla p, int nq
 
     // tiles [0, t_mid) lie left of the diagonal of every row
     const int t_mid = min((s.pos0 + q0 + 1) >> 6, nt);
-    issue_tile(0);
-    stage_window(0);
+    auto next_tile = [&](int t) {
+        if (t >= nt) return;
+        issue_tile(t);
+        stage_window(t);
+    };
+    next_tile(kh);
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 #pragma unroll
     for (int i = 0; i < NQ; ++i)
@@ -632,46 +640,68 @@ __global__ __launch_bounds__(256, WGS) void mla_prefill_kernel(CogsMla p, int nq
         else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         __builtin_amdgcn_s_barrier();
     };
-    auto next_tile = [&](int t) {
-        if (t >= nt) return;
-        issue_tile(t);
-        stage_window(t);
-    };
     typedef std::true_type yes;
     typedef std::false_type no;
-    next_tile(1);
     // masked tiles look the bias up, unless there is none
     const bool no_bias = HEADS && t_far >= nt;
-    if (t_mid <= 0) {
-        if (no_bias) process_tile(0, yes{}, yes{}, no{});
-        else process_tile(0, yes{}, yes{}, yes{});
-    } else if (!HEADS || 0 < t_far) process_tile(0, no{}, yes{}, no{});
-    else process_tile(0, no{}, yes{}, yes{});
-    tile_tail();
-    int t = 1;
     const int t_plain = HEADS ? min(t_mid, t_far) : t_mid;
-    for (; t < t_plain; ++t) {
-        next_tile(t + 1);
+    next_tile(kh + NH);
+    if (kh >= nt) {
+    } else if (kh >= t_mid) {
+        if (no_bias) process_tile(kh, yes{}, yes{}, no{});
+        else process_tile(kh, yes{}, yes{}, yes{});
+    } else if (!HEADS || kh < t_far) process_tile(kh, no{}, yes{}, no{});
+    else process_tile(kh, no{}, yes{}, yes{});
+    tile_tail();
+    int t = kh + NH;                                   // (as many rounds for every share)
+    for (; t - kh + NH <= t_plain; t += NH) {
+        next_tile(t + NH);
         process_tile(t, no{}, no{}, no{});
         tile_tail();
     }
     if constexpr (HEADS) {
-        for (; t < t_mid; ++t) {
-            next_tile(t + 1);
+        for (; t - kh + NH <= t_mid; t += NH) {
+            next_tile(t + NH);
             process_tile(t, no{}, no{}, yes{});
             tile_tail();
         }
     }
-    for (; t < nt; ++t) {
-        next_tile(t + 1);
-        if (no_bias) process_tile(t, yes{}, no{}, no{});
-        else process_tile(t, yes{}, no{}, yes{});
+    for (; t - kh < nt; t += NH) {
+        next_tile(t + NH);
+        if (t < nt) {
+            if (no_bias) process_tile(t, yes{}, no{}, no{});
+            else process_tile(t, yes{}, no{}, yes{});
+        }
         tile_tail();
     }
 
+    // the shares' sums meet in LDS: wave (w, kh) hands over rows of group 1 - kh and finishes those of group kh
+    auto join = [&](auto mine_tag) {
+        constexpr int MINE = decltype(mine_tag)::value, OTHER = 1 - MINE;
+        f32x4* x = reinterpret_cast<f32x4*>(smem) + (wid * 2 + OTHER) * (DT + 1) * 64 + lane;
+#pragma unroll
+        for (int d = 0; d < DT; ++d) x[d * 64] = oacc[d][OTHER];
+        x[DT * 64] = f32x4{lacc[OTHER][0], m_ref[OTHER], 0.f, 0.f};
+        __syncthreads();
+        const f32x4* y = reinterpret_cast<const f32x4*>(smem) + (wid * 2 + MINE) * (DT + 1) * 64 + lane;
+        const f32x4 lm = y[DT * 64];
+        // a share that saw no key has a sum of zero and takes no part in the reference
+        const float m = lm[0] == 0.f ? m_ref[MINE] : lacc[MINE][0] == 0.f ? lm[1] : fmaxf(m_ref[MINE], lm[1]);
+        const float fa = lacc[MINE][0] == 0.f ? 0.f : __builtin_amdgcn_exp2f(m_ref[MINE] - m), fb = lm[0] == 0.f ? 0.f : __builtin_amdgcn_exp2f(lm[1] - m);
+#pragma unroll
+        for (int d = 0; d < DT; ++d) oacc[d][MINE] = oacc[d][MINE] * fa + y[d * 64] * fb;
+        lacc[MINE] = lacc[MINE] * fa + lm[0] * fb;
+        m_ref[MINE] = m;
+    };
+    static_assert(NH == 1 || 8 * (DT + 1) * 1024 <= 2 * NH * BUF, "the exchange fits the tiles' buffers");
+    if constexpr (NH == 2) {
+        if (kh == 0) join(std::integral_constant<int, 0>{});
+        else join(std::integral_constant<int, 1>{});
+    }
     const int dt = p.dv >> 4;
 #pragma unroll
     for (int i = 0; i < NQ; ++i) {
+        if (NH == 2 && i != kh) continue;
         const int qrow = q0 + wid * 32 + 16 * i + li;
         if (qrow >= s.len) continue;
         float f = 1.f / (lacc[i][0] + (p.sink ? exp2f(p.sink[h] - m_ref[i]) : 0.f));
@@ -911,17 +941,27 @@ __global__ __launch_bounds__(256) void mla_combine_kernel(const float* __restric
     }
 }
 
-template <int KN, int KR, int DT, int WGS>
+template <int KN, int KR, int DT, int WPE, int NH>
 int launch_prefill(hipStream_t st, const CogsMla& a) {
     static std::atomic<uint64_t> attr_done{0};
-    constexpr int lds = 2 * (64 * KN * 64 + 64 * KR * 64 + 64 * DT * 32) + (KR == 0 ? 2 * MLA_WIN * 4 : 0);
-    cogs_ensure_dyn_lds((const void*)mla_prefill_kernel<KN, KR, DT, WGS>, lds, attr_done);
+    constexpr int lds = 2 * NH * (64 * KN * 64 + 64 * KR * 64 + 64 * DT * 32) + (KR == 0 ? 2 * NH * MLA_WIN * 4 : 0);
+    cogs_ensure_dyn_lds((const void*)mla_prefill_kernel<KN, KR, DT, WPE, NH>, lds, attr_done);
     const int nqt = (a.max_new + 127) / 128;
     const long grid = (long)nqt * a.heads * a.nseq;
     if (grid > 0x7fffffffL) return COGS_E_INVALID;
-    const int group = nqt >= 64 ? 1 : 64 / nqt;
-    hipLaunchKernelGGL((mla_prefill_kernel<KN, KR, DT, WGS>), dim3((unsigned)grid), dim3(256), lds, st, a, nqt, group);
+    const int group = nqt >= 64 ? 1 : 64 / nqt;            // (NH = 2: one workgroup per CU, the next longest to the CU that is done first)
+    hipLaunchKernelGGL((mla_prefill_kernel<KN, KR, DT, WPE, NH>), dim3((unsigned)grid), dim3(256 * NH), lds, st, a, nqt, group);
     return COGS_LAUNCH_CHECK();
+}
+
+// One query tile's keys are a chain of 2.3 us a tile for a wave that has its SIMD to itself, and the longest chain lasted 146 of the
+// 190 us of 4096 rows x 16 heads (192 + 128 columns). With two waves per tile and half the chain each it takes 99 us, and the whole 147:
+// 1800 rows 77 -> 53 us, 1000 rows 44 -> 33, 300 rows 17 -> 16; 4096 rows x 32 heads 330 -> 299. Many short chains fill the chip by
+// themselves and only pay for the join: 8 sequences x 16 heads of 64 to 512 keys 33 us, and 36 in halves.
+template <int KN, int KR, int DT>
+int launch_prefill_split(hipStream_t st, const CogsMla& a) {
+    const long tiles = (long)((a.max_new + 127) / 128) * a.heads * a.nseq;
+    return tiles <= 256 || a.max_ctx >= 1024 ? launch_prefill<KN, KR, DT, 2, 2>(st, a) : launch_prefill<KN, KR, DT, 2, 1>(st, a);
 }
 
 template <int DTW, int PER, int WGS>
@@ -987,21 +1027,21 @@ int cogs_k_mla_attention(hipStream_t st, int dtype, const CogsMla& a) {
         a.q_head % 32 == 0 && a.q_head >= a.dn && a.q_rot == a.q_head && a.ldo % 4 == 0 && a.o_head % 4 == 0 && g_cogs_debug.mla_rowwise == 0 &&
         a.kvw < (1 << 23)) {
         const int kn = a.dn / 32, dt = a.dv / 16;
-        if (kn <= 1 && dt <= 2) return launch_prefill<1, 0, 2, 2>(st, a);
-        if (kn <= 2 && dt <= 4) return launch_prefill<2, 0, 4, 2>(st, a);
-        if (kn <= 4 && dt <= 8) return launch_prefill<4, 0, 8, 2>(st, a);
-        if (kn <= 8 && dt <= 16) return launch_prefill<8, 0, 16, 1>(st, a);
+        if (kn <= 1 && dt <= 2) return launch_prefill_split<1, 0, 2>(st, a);
+        if (kn <= 2 && dt <= 4) return launch_prefill_split<2, 0, 4>(st, a);
+        if (kn <= 4 && dt <= 8) return launch_prefill_split<4, 0, 8>(st, a);
+        if (kn <= 8 && dt <= 16) return launch_prefill<8, 0, 16, 1, 1>(st, a);
     }
     if (dtype == COGS_DT_BF16 && !a.kvw && !a.absorbed && a.dn % 8 == 0 && a.dr % 8 == 0 && a.dv % 16 == 0 && a.ldq % 8 == 0 && a.q_head % 32 == 0 &&
         a.q_rot % 32 == 0 && a.q_rot >= a.dn && a.q_head - a.q_rot >= a.dr && a.ldk % 8 == 0 && a.k_head % 8 == 0 && a.ldkr % 8 == 0 &&
         a.ldv % 8 == 0 && a.v_head % 8 == 0 && a.ldo % 4 == 0 && a.o_head % 4 == 0 && g_cogs_debug.mla_rowwise == 0 &&
         a.ldk < (1 << 23) && a.ldkr < (1 << 23) && a.ldv < (1 << 23)) {       // (a tile's byte offsets are 32 bits)
         const int kn = a.q_rot / 32, kr = (a.q_head - a.q_rot) / 32, dt = a.dv / 16;
-        if (kn <= 1 && kr <= 1 && dt <= 2) return launch_prefill<1, 1, 2, 2>(st, a);
-        if (kn <= 2 && kr <= 1 && dt <= 4) return launch_prefill<2, 1, 4, 2>(st, a);
-        if (kn <= 4 && kr <= 1 && dt <= 8) return launch_prefill<4, 1, 8, 2>(st, a);
-        if (kn <= 4 && kr <= 2 && dt <= 8) return launch_prefill<4, 2, 8, 2>(st, a);
-        if (kn <= 8 && kr <= 4 && dt <= 16) return launch_prefill<8, 4, 16, 1>(st, a);
+        if (kn <= 1 && kr <= 1 && dt <= 2) return launch_prefill_split<1, 1, 2>(st, a);
+        if (kn <= 2 && kr <= 1 && dt <= 4) return launch_prefill_split<2, 1, 4>(st, a);
+        if (kn <= 4 && kr <= 1 && dt <= 8) return launch_prefill_split<4, 1, 8>(st, a);
+        if (kn <= 4 && kr <= 2 && dt <= 8) return launch_prefill_split<4, 2, 8>(st, a);
+        if (kn <= 8 && kr <= 4 && dt <= 16) return launch_prefill<8, 4, 16, 1, 1>(st, a);
     }
     if (a.dn + a.dr > RW_DIM || a.dv > 64 * RW_VREG) return COGS_E_UNSUPPORTED;
     if (dtype == COGS_DT_BF16) hipLaunchKernelGGL(mla_rowwise_kernel<bf16_t>, dim3(a.rows, a.heads), dim3(64), 0, st, a);

@@ -408,6 +408,22 @@ def test_chunked_delta_rule_at_the_edges_of_its_tiles(dev, dim, vdim):
     assert rms_err(out, lg[[n - 1 for n in lens]]) < TOL[torch.float32]
 
 
+@pytest.mark.parametrize("name", ["peaked", "mixed"])
+def test_a_query_tile_by_one_wave_or_by_two(dev, name):
+    """many prompts at once (each query tile's keys are one wave's) and few (every second key tile is another wave's): prompts that end
+    at the edges of the 64-key tiles and of the 128-row tiles, from nothing and behind cached tokens, against the oracle"""
+    cfg, st, e, toks, lg, _ = named(name, torch.bfloat16, 400)
+    lens = [1, 63, 64, 65, 127, 128, 129, 191, 192, 193, 257]
+    for times in (1, 20):
+        for cut in (0, 30):
+            s = sequences(e)
+            jobs = [(i, n) for i, n in enumerate(lens * times) if n > cut]
+            if cut:
+                s.step([(i, toks[:cut], []) for i, _ in jobs])
+            out = s.step([(i, toks[cut:n], [n - 1 - cut]) for i, n in jobs])
+            assert rms_err(out, lg[[n - 1 for _, n in jobs]]) < TOL[torch.bfloat16], (times, cut)
+
+
 def test_unsupported_calls_are_refused(dev):
     from cogstream_amd import _lib as L
     cfg, st, e, toks, _, _ = named("peaked", torch.bfloat16)
