@@ -48,7 +48,7 @@ for M in (3696, 7392):
         a2 = torch.cat([a[:, s * kc:(s + 1) * kc] for s in range(split)], 0).contiguous()
         w2 = w[:, :kc].contiguous()
         part = torch.empty(split * M, N, device=dev, dtype=torch.float32)
-        with L.debug_switch("gemm_ring_cost_permille", 4000), L.debug_switch("gemm_split", 0):
+        with L.debug_switch("gemm_split", 0):
             t1 = med(lambda: ops.gemm(a2, w2, out=part, out_f32=True))
             body = L.debug_get("gemm_last_body")
         t2 = med(lambda: part.view(split, M, N).sum(0).add_(res.float()).bfloat16())
