@@ -1153,7 +1153,7 @@ int cogs_k_gemm(hipStream_t st, const CogsGemm& g) {
     const int n_pad = (g.N + BN3 - 1) / BN3 * BN3;
     const bool pp_fits = n_pad * 100 <= g.N * (int)g_cogs_debug.gemm_pad_pct;   // default: <= 12 % of the MFMAs spent on N padding
     // (the ping-pong kernel wants two slabs and, below a row block, wastes its tiles' rows)
-    const bool pp = mid > 0 && env_mid == 0 && g_cogs_debug.gemm_pingpong != 0 && pp_fits && g.K >= 128 && g.M >= 256 && !g.force_mid_tile;
+    const bool pp = mid > 0 && env_mid == 0 && g_cogs_debug.gemm_pingpong != 0 && pp_fits && g.K >= 128 && g.M >= 256;
     if (mid > 0 && !pp) return launch_mid(st, g, mid);
     GemmArgs p;
     p.trace = nullptr; p.rope_lut = nullptr; p.rope_lut_bytes = 0; p.group_m = GROUP_M;
@@ -1243,7 +1243,7 @@ int cogs_k_gemm(hipStream_t st, const CogsGemm& g) {
         if (mb_main >= 0) {
             const int rows_main = mb_main * BM3;
             CogsGemm b = g;
-            b.M = g.M - rows_main; b.force_mid_tile = 1;
+            b.M = g.M - rows_main;
             b.A = (const char*)g.A + (size_t)rows_main * g.lda * es;
             b.C = (char*)g.C + (size_t)rows_main * (g.hm_rows > 0 ? g.head_dim : g.ldc) * (g.out_f32 ? 4 : es);   // head-major: rows advance by head_dim inside every head block
             if (g.residual) b.residual = (const char*)g.residual + (size_t)rows_main * g.ldr * es;
@@ -1264,7 +1264,9 @@ int cogs_k_gemm(hipStream_t st, const CogsGemm& g) {
                 const int rc2 = COGS_LAUNCH_CHECK();
                 if (rc2 != COGS_OK) return rc2;
             }
-            const int rc3 = cogs_k_gemm(st, b);
+            // (straight to the kernel: a remainder may be one row, which cogs_k_gemm would take for a single-row product)
+            float rest = 0.f;
+            const int rc3 = launch_mid(st, b, mb_main > 0 ? best_mid_tile(b.M, b.N, b.K, &rest) : mid);
             if (mb_main > 0) g_cogs_debug.gemm_last_body = 5;
             return rc3;
         }

@@ -1124,3 +1124,36 @@ def test_whole_seeding_equals_the_steps(dev, T, PD, K, dtype):
     same = x[:1].expand(T, PD).contiguous()
     _, flag = ops.kmeans_pp(same, first, K, q.to(dev), ws)
     assert int(flag) == 1
+
+
+@pytest.mark.parametrize("M,N,K,form", [
+    (4609, 3456, 1152, "rotary, head-major, folded norm"), (3841, 4352, 1152, "folded norm, gelu"), (13825, 1152, 1152, "residual, statistics"),
+    (13825, 1152, 4352, "residual, statistics"), (3585, 4608, 3584, "rotary"), (4609, 3584, 3584, "residual"), (2049, 8192, 2048, "plain"),
+    (1281, 11264, 2048, "swiglu"), (2049, 8192, 2048, "fp32")])
+def test_a_split_product_whose_remainder_is_one_row(dev, M, N, K, form):
+    """a product cut into whole rounds of 256x256 tiles and one more row: that row gets its fused epilogue and the bits of the unsplit
+    launch, like every other"""
+    from cogstream_amd import _lib as L2
+    ops = _ops()
+    g = torch.Generator(device=dev).manual_seed(M)
+    rnd = lambda *s: (torch.randn(*s, generator=g, device=dev) * 0.5).bfloat16()
+    a, w = rnd(M, K), rnd(N, K)
+    table = lambda: torch.randn(M, 36, 2, generator=g, device=dev)
+    fold = lambda: dict(ln_ab=torch.rand(M, 2, generator=g, device=dev) + 0.5, col_c=torch.randn(N, generator=g, device=dev))
+    kw = {"rotary, head-major, folded norm": lambda: dict(rope_cos=table(), rope_cols=2304, head_dim=72, hm_cols=1152, **fold()),
+          "folded norm, gelu": lambda: dict(act=L2.ACT_GELU_TANH, **fold()),
+          "residual, statistics": lambda: dict(bias=rnd(N), residual=rnd(M, N), row_stats=torch.empty(M, N // 64, 2, device=dev)),
+          "rotary": lambda: dict(bias=rnd(N), rope_cos=torch.randn(M, 64, 2, generator=g, device=dev), rope_cols=4096, head_dim=128),
+          "residual": lambda: dict(residual=rnd(M, N)), "plain": dict, "swiglu": lambda: dict(act=L2.ACT_SWIGLU),
+          "fp32": lambda: dict(out_f32=True)}[form]()
+    outs = []
+    for split, body in ((1, 5), (0, 4)):
+        stats = kw.get("row_stats")
+        if stats is not None:
+            stats.fill_(-7.0)
+        with L2.debug_switch("gemm_split", split):
+            out = ops.gemm(a, w, **kw)
+        assert L2.debug_get("gemm_last_body") == body
+        outs.append((out, None if stats is None else stats.clone()))
+    (x, sx), (y, sy) = outs
+    assert torch.equal(x, y) and (sx is None or torch.equal(sx, sy))
