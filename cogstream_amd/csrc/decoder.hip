@@ -45,7 +45,7 @@ struct CogsDecoder {
     // largest row widths over the layers
     int max_t32 = 0, max_cq = 0, max_q = 0, max_o = 0, max_ff = 0, max_kvcols = 0, max_kvw = 0, max_heads = 0;
     long max_qlat = 0, max_olat = 0;
-    int max_dqk = 0, max_dv = 0, max_dheads = 0, max_ddk = 0;       // gated delta rule: kv_heads x dim, heads x vdim, heads, dim
+    int max_dqk = 0, max_dv = 0, max_dheads = 0;       // gated delta rule: kv_heads x dim, heads x vdim, heads
     bool att_tail = false;
 };
 
@@ -117,7 +117,7 @@ Work carve(const CogsDecoder& d, int S, int nseq, int64_t C, int n_want, void* w
         k.dv = (float*)c.take(n * d.max_dv * 4);
         k.dout = (float*)c.take(n * d.max_dv * 4);
         k.dbg = (float*)c.take(n * d.max_dheads * 2 * 4);
-        k.drec = (float*)c.take(cogs_k_delta_rec_floats(S, nseq, d.max_dheads, d.max_ddk) * 4);
+        k.drec = (float*)c.take(cogs_k_delta_rec_floats(S, nseq, d.max_dheads) * 4);
     }
     k.bytes = c.off;
     return k;
@@ -400,7 +400,7 @@ cogs_status cogs_decoder_load(cogs_handle h, const cogs_decoder_weights* w) {
             g.channels = 2 * m.kv_heads * g.dk + m.heads * g.dv;
             g.ldt = g.channels + m.heads * g.dv + 2 * g.headsp;
             G.state = (long)m.heads * g.dk * g.dv + (long)m.taps * g.channels;
-            mx(d->max_t32, g.ldt); mx(d->max_dqk, m.kv_heads * g.dk); mx(d->max_dv, m.heads * g.dv); mx(d->max_dheads, m.heads); mx(d->max_ddk, g.dk);
+            mx(d->max_t32, g.ldt); mx(d->max_dqk, m.kv_heads * g.dk); mx(d->max_dv, m.heads * g.dv); mx(d->max_dheads, m.heads);
             oin = g.oin; ocols = m.heads * g.dv;
         } else {
             return fail(COGS_E_INVALID);

@@ -9,18 +9,18 @@
 // A token-by-token kernel (delta_recur) serves the sizes the chunked pair has no instance for.
 //
 // Chunks. With G_i = sum of ln g over the chunk's tokens 0 .. i and S0 the state in front of it,
-//   u_i = beta_i (v_i - e^{G_i} S0^T k_i - sum_{j<i} e^{G_i - G_j} (k_i . k_j) u_j),  i.e.  U = T diag(beta) (V - diag(e^G) K S0) = T diag(beta) V + W S0
+//   u_i = beta_i (v_i - e^{G_i} S0^T k_i - sum_{j<i} e^{G_i - G_j} (k_i . k_j) u_j),  i.e.  U = T diag(beta) (V - diag(e^G) K S0)
 //   with T = (I + L)^-1, L_ij = beta_i e^{G_i - G_j} k_i . k_j (j < i);   O = diag(e^G) Q S0 + P U with P_ij = e^{G_i - G_j} q_i . k_j (j <= i);
 //   S = e^{G_last} S0 + K^T diag(e^{G_last - G_j}) U.
-// Only exponentials of differences of later minus earlier sums appear (<= 1); the sums themselves are fp64. T diag(beta), W, P and the
+// Only exponentials of differences of later minus earlier sums appear (<= 1); the sums themselves are fp64. T diag(beta), P and the
 // exponentials do not depend on S: delta_chunk forms them for all chunks at once, T by forward substitution. delta_scan walks a
 // sequence's chunks: a workgroup owns 16 columns of S, its four waves the 16-row tiles of S in turn.
-// The scan's chunks follow one another, so what counts is the length of one: W S0, a sum over the waves, the new state. W (33 MB at
-// 4096 tokens and 16 heads, in place of a product with T behind the sum) and operands in the order of the lanes took it from 2.2 to
-// 1.2 us a chunk: 285 -> 155 us for the scan, 26 -> 39 us for delta_chunk. Two thirds of that are matrix instructions (54 of 14 ns), the
-// rest LDS exchange and the loads' share of issue. delta_chunk is bound by its phases: all workgroups load, then multiply, then store.
+// The scan's chunks follow one another, so what counts is the length of one: K S, a sum over the waves, the product with T, the new
+// state. Operands in the order of the lanes and buffer loads without address arithmetic took it from 2.1 to 1.45 us a chunk (4096
+// tokens, 16 heads of 128: scan 273 -> 188 us, delta_chunk 30). Two thirds of that are matrix instructions (63 of 14 ns), the rest LDS
+// exchange and the loads' share of issue.
 // MFMA layout: a 16x16 accumulator holds rows 4 g + r in register r of lane group g, which is the B operand of the r-th of four
-// 4-deep steps if k is taken in the order 4 g + r -- so S and U go from product to product in their registers, and A operands are
+// 4-deep steps if k is taken in the order 4 g + r -- so S, V - diag(e^G) K S and U go from product to product in their registers, and A operands are
 // 16-byte loads of four neighbouring k.
 #include "common.h"
 #include "kernels.h"
@@ -30,9 +30,8 @@ namespace {
 
 constexpr int CH = 32;                        // tokens of a chunk
 constexpr int TILE = 256;                     // floats of a 16x16 tile, row-major
-constexpr int EXPS = 6 * TILE;                 // per chunk and head: P tiles (0,0) (1,0) (1,1) | T beta tiles | e^G | e^{G_last - G} | e^{G_last}, .. | W [2][dkp / 16][64 lanes][4];
-constexpr int REC = EXPS + 3 * CH;            // P and T beta as A operands [4 steps][64 lanes], W as A operands too
-__host__ __device__ constexpr int rec_floats(int dkp) { return REC + CH * dkp; }
+constexpr int EXPS = 6 * TILE;                // per chunk and head: P tiles (0,0) (1,0) (1,1) | T beta tiles | e^G | e^{G_last - G} | e^{G_last}, ..;
+constexpr int REC = EXPS + 3 * CH;            // P as A operands [4 steps][64 lanes], T beta as [64 lanes][4 steps]
 
 __device__ __forceinline__ float unit_scale(float ss) { return 1.f / sqrtf(ss + 1e-6f); }
 __device__ __forceinline__ float sigmoid_f(float x) { return 1.f / (1.f + expf(-x)); }
@@ -206,11 +205,11 @@ __device__ __forceinline__ f32x4 mfma4(const f32x4& a, const f32x4& b, f32x4 c) 
 }
 
 __device__ __forceinline__ float* chunk_rec(const CogsDelta& p, const CogsSeq& s, int seq, int chunk, int h) {
-    return p.rec + ((long)(s.row0 / CH + seq + chunk) * p.heads + h) * rec_floats(p.dkp);      // (a later sequence starts behind the chunks of an earlier one)
+    return p.rec + ((long)(s.row0 / CH + seq + chunk) * p.heads + h) * REC;      // (a later sequence starts behind the chunks of an earlier one)
 }
 
-// What a chunk needs besides S and V: P, T diag(beta), the exponentials and W = -T diag(beta) diag(e^G) K. Three waves take a tile
-// (0,0), (1,0), (1,1) each of the 32 x 32 matrices, then four waves the 16-column pieces of W.
+// What a chunk needs besides S and V: P, T diag(beta) and the exponentials. Three waves take a tile (0,0), (1,0), (1,1) each of the
+// 32 x 32 matrices.
 __global__ __launch_bounds__(256) void delta_chunk_kernel(CogsDelta p) {
     __shared__ double cum[CH];
     __shared__ __attribute__((aligned(16))) float beta_s[CH], eg_s[CH];
@@ -264,16 +263,6 @@ __global__ __launch_bounds__(256) void delta_chunk_kernel(CogsDelta p) {
             }
         }
     }
-    const int kt = p.dkp >> 4;
-    auto piece = [&](int t, f32x4 (&x)[2]) {           // 16 columns of K, as the operand of tokens 4 g + r (0 .. 15) and 16 + 4 g + r
-#pragma unroll
-        for (int a = 0; a < 2; ++a)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) x[a][r] = K[(long)min(16 * a + 4 * g + r, n - 1) * p.dkp + 16 * t + li];
-    };
-    f32x4 x[2][2];                                     // two pieces on the way
-    piece(min(wid, kt - 1), x[0]);
-    piece(min(wid + 4, kt - 1), x[1]);
     __syncthreads();
     if (wid < 3) {
         const int j = 16 * tb + li;
@@ -318,50 +307,35 @@ __global__ __launch_bounds__(256) void delta_chunk_kernel(CogsDelta p) {
         for (int r = 0; r < 4; ++r) Ts[1][4 * g + r][li] = -t[r];
     }
     __syncthreads();
-    // T diag(beta) for the scan, and -that diag(e^G): row li, tokens 4 g + r
-    f32x4 te[3];
+    if (wid < 3) {                                     // T diag(beta): row li, tokens 4 g + r
+        const int i = 16 * ta + li, j = 16 * tb + 4 * g;
+        f32x4 t = frag(&Ts[wid][0][0], 20, li, g) * *reinterpret_cast<const f32x4*>(beta_s + j);
 #pragma unroll
-    for (int w = 0; w < 3; ++w) {
-        const int i = (w > 0 ? 16 : 0) + li, j = (w == 2 ? 16 : 0) + 4 * g;
-        const f32x4 t = frag(&Ts[w][0][0], 20, li, g), be = *reinterpret_cast<const f32x4*>(beta_s + j), e = *reinterpret_cast<const f32x4*>(eg_s + j);
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const float v = i < n && j + r < n ? t[r] * be[r] : 0.f;
-            te[w][r] = -v * e[r];
-            if (wid == w) rec[(3 + w) * TILE + r * 64 + lane] = v;
-        }
-    }
-    const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
-    auto product = [&](int t, const f32x4 (&v)[2]) {   // transposed: a lane ends with four neighbours of a row of W
-        float* o = rec + REC + (t * 64 + lane) * 4;
-        *reinterpret_cast<f32x4*>(o) = mfma4(v[0], te[0], zero);
-        *reinterpret_cast<f32x4*>(o + kt * TILE) = mfma4(v[1], te[2], zero) + mfma4(v[0], te[1], zero);
-    };
-    for (int t = wid; t < kt; t += 8) {
-        product(t, x[0]);
-        piece(min(t + 8, kt - 1), x[0]);
-        if (t + 4 < kt) product(t + 4, x[1]);
-        piece(min(t + 12, kt - 1), x[1]);
+        for (int r = 0; r < 4; ++r) t[r] = i < n && j + r < n ? t[r] : 0.f;
+        *reinterpret_cast<f32x4*>(rec + (3 + wid) * TILE + 4 * lane) = t;
     }
 }
 
 // what a wave needs of one chunk
 template <int NK>
 struct ScanIn {
-    f32x4 w[2][NK], q[2][NK], kt[2][NK], eg[2], ec[2];
-    float pm[3], tm[3], v[2], gl;
+    f32x4 k[2][NK], q[2][NK], kt[2][NK], eg[2], ec[2], tm[3], v[2];
+    float pm[3], gl;
 };
 
-// NK: 16-row tiles of S per wave. A chunk: U = T diag(beta) V + W S, in partial sums over the waves' rows of S (and a quarter of
-// T diag(beta) V each) that meet in LDS (one barrier); while they do, Q S; then the new state and, beside it, a quarter of P U per wave
-// into the partial read-outs. Those ride on the next chunk's barrier, and every wave finishes a quarter of them behind it. One wave per
+// NK: 16-row tiles of S per wave. A chunk: K S in partial sums over the waves' rows of S that meet in LDS (one barrier); while they do,
+// Q S; then R = V - diag(e^G) K S and U = T diag(beta) R, which every wave forms whole, the new state and, beside it, a quarter of P U per
+// wave into the partial read-outs. Those ride on the next chunk's barrier, and every wave finishes a quarter of them behind it. One wave per
 // SIMD issues in order, so everything else -- the next chunk's loads, scaling, sums -- stands between matrix instructions that do not
-// need it (sched_barrier keeps it there). T diag(beta) V, P U and the state's growth are sums of their own: chained to what they are
-// added to, they were rounded at its size (error of the read-outs against fp64 2.5e-7 of them instead of 2.0e-7).
+// need it (sched_barrier keeps it there). R comes first and is multiplied then: where keys recur the state already predicts V, R is small
+// against both, and so is what rounding T and the product add. (As T diag(beta) V + W S, with W = -T diag(beta) diag(e^G) K ahead of the
+// scan, 54 instead of 63 matrix instructions, two terms of V's size were rounded and cancelled: read-outs of 8 recurring pairs were off
+// by 1.2e-7 of them instead of 8.2e-8, values read back from the state by 1.2e-7 instead of 3.5e-8.) K S and Q S are two chains each, and
+// P U and the state's growth sums of their own: chained to what they are added to, they were rounded at its size.
 template <int NK>
 __global__ __launch_bounds__(256, NK > 2 ? 1 : 2) void delta_scan_kernel(CogsDelta p) {
     __shared__ __attribute__((aligned(16))) f32x4 red[2][4][4][64];
-    // workgroups go round the XCDs: the columns of a head stay on one, whose L2 then serves its W, K and Q once
+    // workgroups go round the XCDs: the columns of a head stay on one, whose L2 then serves its K and Q once
     const int ng = p.dvp >> 4, place = blockIdx.x >> 3, h = (blockIdx.x & 7) + 8 * (place / ng), col0 = (place % ng) * 16, seq = blockIdx.z;
     if (h >= p.heads) return;
     const CogsSeq s = p.seqs[seq];
@@ -385,25 +359,27 @@ __global__ __launch_bounds__(256, NK > 2 ? 1 : 2) void delta_scan_kernel(CogsDel
     }
     const int nc = (s.len + CH - 1) / CH;
     // a lane's places in a chunk's rows (bytes)
-    int qo[2], to[2][4], vo[2], oo[2];
-    const int wo = lane * 16, po = lane * 4 + wid * 256, ego = 16 * g;
+    int qo[2], to[2][4], vo[2][4], oo[2];
+    const int tmo = lane * 16, po = lane * 4 + wid * 256, ego = 16 * g;
     int zo = 0;
     asm("" : "+v"(zo));                          // (a scalar load would share its counter with LDS)
 #pragma unroll
     for (int r = 0; r < 2; ++r) oo[r] = ((16 * fin + 4 * g + 2 * half + r) * ldv + li) * 4;
 #pragma unroll
     for (int a = 0; a < 2; ++a) {
-        vo[a] = ((16 * a + 4 * g + wid) * ldv + li) * 4;
         qo[a] = ((16 * a + li) * ld + 4 * g) * 4;
 #pragma unroll
-        for (int r = 0; r < 4; ++r) to[a][r] = ((16 * a + 4 * g + r) * ld + li) * 4;
+        for (int r = 0; r < 4; ++r) {
+            to[a][r] = ((16 * a + 4 * g + r) * ld + li) * 4;
+            vo[a][r] = ((16 * a + 4 * g + r) * ldv + li) * 4;
+        }
     }
     // buffer loads: a scalar base per array and chunk, a lane's place, a scalar piece -- no address arithmetic per load; rows past the
     // sequence's end, and K's columns of a tile past S's end, lie behind the buffer's size and read as zero
     struct From { float *k, *q, *v, *rec; };
     const From f0{p.k + ((long)kh * p.rows + s.row0) * ld, p.q + ((long)kh * p.rows + s.row0) * ld, p.v + ((long)h * p.rows + s.row0) * ldv + col0, chunk_rec(p, s, seq, 0, h)};
     From f = f0;
-    const int bytes_rec = rec_floats(ld) * 4;
+    constexpr int bytes_rec = REC * 4;
     int bytes_q, bytes_v, bytes_k[NK];
     auto sizes = [&](int rows) {
         bytes_q = rows * ld * 4;
@@ -418,24 +394,24 @@ __global__ __launch_bounds__(256, NK > 2 ? 1 : 2) void delta_scan_kernel(CogsDel
     auto at1 = [](float* base, int size, int lane_off, int off) {
         return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(__builtin_amdgcn_make_buffer_rsrc(base, 0, size, 0x00020000), lane_off, off, 0));
     };
-    const long step_k = (long)CH * ld, step_v = (long)CH * ldv, step_rec = (long)p.heads * rec_floats(ld);
+    const long step_k = (long)CH * ld, step_v = (long)CH * ldv, step_rec = (long)p.heads * REC;
     int at = 0;                                                // the chunk f points to
     auto advance = [&] {                                       // (the last chunk is loaded again rather than nothing)
         at = min(at + 1, nc - 1);
         f = From{f0.k + at * step_k, f0.q + at * step_k, f0.v + at * step_v, f0.rec + at * step_rec};
         sizes(min(CH, s.len - at * CH));
     };
-    // load i of a chunk, in the order of their use
-    constexpr int L_U = 5, L_W = L_U + 2 * NK, L_Q = L_W + 2 * NK, L_E = L_Q + 4, L_G = L_E + 1, L_KT = L_G + 8 * NK, L_ALL = L_KT + 3;
+    // load i of a chunk, in the order of their use, the 16-byte ones first
+    constexpr int L_Q = 2 * NK, L_E = L_Q + 2 * NK, L_T = L_E + 4, L_V = L_T + 3, L_G = L_V + 8, L_KT = L_G + 1, L_PM = L_KT + 8 * NK, L_ALL = L_PM + 3;
     auto load = [&](ScanIn<NK>& in, int i) {
-        if (i < 2) in.v[i] = at1(f.v, bytes_v, vo[i], 0);
-        else if (i < L_U) in.tm[i - 2] = at1(f.rec, bytes_rec, po, (1 + i) * TILE * 4);
-        else if (i < L_W) { const int j = i - L_U; in.w[j / NK][j % NK] = at4(f.rec, bytes_rec, wo, (REC + ((j / NK) * tiles + tn[j % NK]) * TILE) * 4); }
-        else if (i < L_Q) { const int j = i - L_W; in.q[j / NK][j % NK] = at4(f.q, bytes_q, qo[j / NK], 64 * tn[j % NK]); }
-        else if (i < L_E) { const int j = i - L_Q; (j & 2 ? in.eg : in.ec)[j & 1] = at4(f.rec, bytes_rec, ego, (EXPS + (j & 2 ? 0 : CH) + 16 * (j & 1)) * 4); }
-        else if (i < L_G) in.gl = at1(f.rec, bytes_rec, zo, (EXPS + 2 * CH) * 4);
-        else if (i < L_KT) { const int j = i - L_G; in.kt[(j >> 2) & 1][j >> 3][j & 3] = at1(f.k, bytes_k[j >> 3], to[(j >> 2) & 1][j & 3], 64 * tn[j >> 3]); }
-        else if (i < L_ALL) in.pm[i - L_KT] = at1(f.rec, bytes_rec, po, (i - L_KT) * TILE * 4);
+        if (i < L_Q) in.k[i / NK][i % NK] = at4(f.k, bytes_q, qo[i / NK], 64 * tn[i % NK]);
+        else if (i < L_E) { const int j = i - L_Q; in.q[j / NK][j % NK] = at4(f.q, bytes_q, qo[j / NK], 64 * tn[j % NK]); }
+        else if (i < L_T) { const int j = i - L_E; (j & 2 ? in.ec : in.eg)[j & 1] = at4(f.rec, bytes_rec, ego, (EXPS + (j & 2 ? CH : 0) + 16 * (j & 1)) * 4); }
+        else if (i < L_V) in.tm[i - L_T] = at4(f.rec, bytes_rec, tmo, (3 + i - L_T) * TILE * 4);
+        else if (i < L_G) { const int j = i - L_V; in.v[j >> 2][j & 3] = at1(f.v, bytes_v, vo[j >> 2][j & 3], 0); }
+        else if (i < L_KT) in.gl = at1(f.rec, bytes_rec, zo, (EXPS + 2 * CH) * 4);
+        else if (i < L_PM) { const int j = i - L_KT; in.kt[(j >> 2) & 1][j >> 3][j & 3] = at1(f.k, bytes_k[j >> 3], to[(j >> 2) & 1][j & 3], 64 * tn[j >> 3]); }
+        else if (i < L_ALL) in.pm[i - L_PM] = at1(f.rec, bytes_rec, po, (i - L_PM) * TILE * 4);
     };
     const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
     f32x4 y[2] = {zero, zero};                                 // the previous chunk's read-outs, this wave's part of the sums
@@ -460,11 +436,11 @@ __global__ __launch_bounds__(256, NK > 2 ? 1 : 2) void delta_scan_kernel(CogsDel
     auto pin = [](f32x4 (&v)[4]) { asm volatile("" : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]), "+v"(v[3])); };      // (used from here on, no earlier)
     // chunk c from `in`, the next one into nx
     auto chunk = [&](int c, const ScanIn<NK>& in, ScanIn<NK>& nx) {
-        constexpr int STEPS = 24 * NK;                         // matrix instructions that bring loads with them
-        static_assert(L_ALL + L_E - L_U <= 2 * STEPS);
-        constexpr int LONG = L_E - L_U, WORK = L_ALL + LONG;   // the four waves' 16-byte loads take the time of two matrix instructions, the others half
+        constexpr int STEPS = 24 * NK + 12;                    // matrix instructions that bring loads with them
+        constexpr int LONG = L_V, WORK = L_ALL + LONG;         // the four waves' 16-byte loads take the time of two matrix instructions, the others half
+        static_assert(WORK <= 2 * STEPS);
         int step = 0, next = 0;
-        auto due = [&] { return next < L_ALL && (next + (next > L_U ? min(next - L_U, LONG) : 0)) * STEPS < (step + 1) * WORK; };
+        auto due = [&] { return next < L_ALL && (next + min(next, LONG)) * STEPS < (step + 1) * WORK; };
         auto feed = [&] {
             if (due()) load(nx, next++);
             if (due()) load(nx, next++);
@@ -472,35 +448,32 @@ __global__ __launch_bounds__(256, NK > 2 ? 1 : 2) void delta_scan_kernel(CogsDel
             __builtin_amdgcn_sched_barrier(0);
         };
         f32x4 (*rd)[4][64] = red[c & 1];
-        f32x4 x[2], o[2], odd, tv[2];
+        f32x4 x[2], o[2], odd;
         auto qs = [&](int a, int i) {
-            o[a] = mfma(in.q[a][i >> 2][i & 3], st[i >> 2][i & 3], i < 1 ? zero : o[a]);
+            f32x4& t = i & 1 ? odd : o[a];
+            t = mfma(in.q[a][i >> 2][i & 3], st[i >> 2][i & 3], i < 2 ? zero : t);
+            if (i == 4 * NK - 1) o[a] += odd;
             feed();
         };
 #pragma unroll
         for (int a = 0; a < 2; ++a) {                          // (one 16 rows after the other: the first ones' sums travel meanwhile)
-            if (a == 0) {
-                tv[0] = mfma(in.tm[0], in.v[0], zero);
-                advance();
-                tv[1] = mfma(in.tm[1], in.v[0], zero);
-                tv[1] = mfma(in.tm[2], in.v[1], tv[1]);
-                __builtin_amdgcn_sched_barrier(0);
-            }
 #pragma unroll
             for (int i = 0; i < 4 * NK; ++i) {
-                x[a] = mfma(in.w[a][i >> 2][i & 3], st[i >> 2][i & 3], i < 1 ? zero : x[a]);
+                f32x4& t = i & 1 ? odd : x[a];
+                t = mfma(in.k[a][i >> 2][i & 3], st[i >> 2][i & 3], i < 2 ? zero : t);
+                if (i == 0 && a == 0) advance();
                 if (i == 1) rd[wid][a == 0 ? 2 : 3][lane] = y[a];
                 if (i == 2 && a == 1) rd[wid][0][lane] = x[0];
                 feed();
             }
-            x[a] += tv[a];
+            x[a] += odd;
         }
         qs(0, 0);
         rd[wid][1][lane] = x[1];
         qs(0, 1);
         qs(0, 2);
         meet();
-        f32x4 part[2][4], u[2], ue[2], grow[NK];
+        f32x4 part[2][4], rr[2], u[2], u10, ue[2], grow[NK];
         f32x2 fo[4];
 #pragma unroll
         for (int a = 0; a < 2; ++a) {
@@ -511,15 +484,25 @@ __global__ __launch_bounds__(256, NK > 2 ? 1 : 2) void delta_scan_kernel(CogsDel
 #pragma unroll
         for (int i = 3; i < 8 * NK; ++i) {
             qs(i / (4 * NK), i % (4 * NK));
-            if (i == 8 * NK - 3) { pin(part[0]); u[0] = (part[0][0] + part[0][1]) + (part[0][2] + part[0][3]); }
-            if (i == 8 * NK - 2) { ue[0] = u[0] * in.ec[0]; gather(fo, rd); }
+            if (i == 8 * NK - 3) { pin(part[0]); rr[0] = in.v[0] - in.eg[0] * ((part[0][0] + part[0][1]) + (part[0][2] + part[0][3])); }
+            if (i == 8 * NK - 2) { pin(part[1]); rr[1] = in.v[1] - in.eg[1] * ((part[1][0] + part[1][1]) + (part[1][2] + part[1][3])); }
+            if (i == 8 * NK - 1) gather(fo, rd);
         }
-        pin(part[1]);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) { u[0] = mfma(in.tm[0][r], rr[0][r], r < 1 ? zero : u[0]); feed(); }
+#pragma unroll
+        for (int r = 0; r < 4; ++r) { u10 = mfma(in.tm[1][r], rr[0][r], r < 1 ? zero : u10); feed(); }
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            u[1] = mfma(in.tm[2][r], rr[1][r], r < 1 ? zero : u[1]);
+            if (r == 0) ue[0] = u[0] * in.ec[0];
+            feed();
+        }
 #pragma unroll
         for (int i = 0; i < 8 * NK; ++i) {
             // rows of the chunk's first half before the second's, so that U's second half has time
             const int n = (i >> 2) % NK, a = (i >> 2) / NK, r = i & 3;
-            if (i == 1) u[1] = (part[1][0] + part[1][1]) + (part[1][2] + part[1][3]);
+            if (i == 1) u[1] += u10;
             if (i == 2) ue[1] = u[1] * in.ec[1];
             grow[n] = mfma(in.kt[a][n][r], ue[a][r], a == 0 && r == 0 ? zero : grow[n]);
             if (a == 1 && n > 0 && r == 1) st[n - 1] = st[n - 1] * in.gl + grow[n - 1];        // (summed by itself: one rounding of S per chunk)
@@ -723,7 +706,7 @@ bool sizes_ok(const CogsDelta& a) {
 
 }  // namespace
 
-size_t cogs_k_delta_rec_floats(int rows, int nseq, int heads, int dkp) { return (size_t)(rows / CH + nseq) * heads * rec_floats(dkp); }
+size_t cogs_k_delta_rec_floats(int rows, int nseq, int heads) { return (size_t)(rows / CH + nseq) * heads * REC; }
 
 int cogs_k_delta_prompt(hipStream_t st, int dtype, const CogsDelta& a, int rows, int nseq, int max_new) {
     if (!sizes_ok(a) || rows <= 0 || nseq <= 0 || nseq > 65535 || a.heads > 65535) return COGS_E_INVALID;

@@ -264,6 +264,6 @@ struct CogsDelta {
     void* att; long ldo;                 // [rows][heads x dvp], in `dtype`
     const CogsSeq* seqs; const int* rowseq; const int* rowpos; long state_off;      // floats
 };
-size_t cogs_k_delta_rec_floats(int rows, int nseq, int heads, int dkp);     // dkp: of the largest layer
+size_t cogs_k_delta_rec_floats(int rows, int nseq, int heads);
 int cogs_k_delta_prompt(hipStream_t st, int dtype, const CogsDelta& a, int rows, int nseq, int max_new);
 int cogs_k_delta_step(hipStream_t st, int dtype, const CogsDelta& a, int nseq);      // one new row per sequence, row i = sequence i

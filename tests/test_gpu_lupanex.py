@@ -408,6 +408,57 @@ def test_chunked_delta_rule_at_the_edges_of_its_tiles(dev, dim, vdim):
     assert rms_err(out, lg[[n - 1 for n in lens]]) < TOL[torch.float32]
 
 
+@pytest.mark.parametrize("dim", [64, 128, 256])
+def test_the_chunked_delta_rule_keeps_what_recurs(dev, dim):
+    """a few (key, value) pairs that come again and again: the state already predicts every value, so what a chunk writes is the rounding of
+    its own sums. Read back at the stored keys, against 64-bit arithmetic on the very same inputs, the chunked form must be as exact as the
+    token-by-token one, and off by no more than its last write is: an entry of S is rounded by at most 2^-24 of itself, V - K S by at most
+    half of that of V (measured 3.4e-8 to 6.8e-8; two terms of V's size that cancel 1.2e-7 to 1.9e-7). The inputs are exact: one-hot
+    tokens, whole values (silu returns them as they are), beta and g equal to one; the keys come out of one-token states, in the column
+    whose value is a power of two"""
+    from cogstream_amd import _lib as L
+    H, P, width, vdim = 4, 4, 64, 64
+    cfg = config([delta(heads=H, kv_heads=2, dim=dim, vdim=vdim, conv=1, ff=None)], width=width, vocab=P, scale=1.0, streams=None, eps=1e-30)
+    st = state(cfg)
+    g = torch.Generator().manual_seed(dim)
+    st["embed"].copy_(torch.eye(P, width))               # normed: 8 in one column
+    st["pos"].zero_()
+    st["l0.norm1"].fill_(1.0)
+    for n in "qkv":
+        st[f"l0.mix.{n}.conv"].fill_(1.0)
+    st["l0.mix.k"].normal_(generator=g)
+    values = torch.randint(18, 64, (H, vdim, P), generator=g).float()
+    values[:, 0] = 32.0
+    st["l0.mix.v"].zero_()[:, :P] = values.view(H * vdim, P) / 8
+    st["l0.mix.b"].fill_(25.0)                           # sigmoid(200)
+    st["l0.mix.A_log"].fill_(-100.0)
+    e = engine(cfg, st, torch.float32)
+
+    def state_of(toks):
+        s = sequences(e)
+        s.step([("r", toks, [])])
+        return s.caches["r"].state[:H * dim * vdim].view(H, dim, vdim).cpu()
+
+    keys = []
+    for t in range(P):
+        one = state_of([t])
+        keys.append(one[:, :, 0] / 32)
+        assert torch.equal(one, keys[-1][:, :, None] * values[:, None, :, t])
+    toks = torch.randint(0, P, (500,), generator=g).tolist()
+    exact = torch.zeros(H, dim, vdim, dtype=torch.float64)
+    for t in toks:
+        k, v = keys[t].double()[:, :, None], values[:, :, t].double()[:, None]
+        exact += k * (v - (k * exact).sum(1, keepdim=True))
+    at = torch.stack(keys, 1).double()
+    want = at @ exact
+    err = []
+    for chunked in (1, 0):
+        with L.debug_switch("delta_chunk", chunked):
+            got = at @ state_of(toks).double()
+        err.append(float((got - want).norm() / want.norm()))
+    assert err[0] < err[1] and err[0] < 1.5 * 2.0 ** -24, err
+
+
 @pytest.mark.parametrize("name", ["peaked", "mixed"])
 def test_a_query_tile_by_one_wave_or_by_two(dev, name):
     """many prompts at once (each query tile's keys are one wave's) and few (every second key tile is another wave's): prompts that end
