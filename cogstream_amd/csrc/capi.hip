@@ -80,6 +80,7 @@ cogs_status cogs_debug_get(const char* name, int64_t* value) {
 #undef COGS_DBG_GET
     if (strcmp(name, "gemm_last_body") == 0) { *value = g_cogs_debug.gemm_last_body; return COGS_OK; }
     if (strcmp(name, "attn_last_kernel") == 0) { *value = g_cogs_debug.attn_last_kernel; return COGS_OK; }
+    if (strcmp(name, "km_pp_last_launches") == 0) { *value = g_cogs_debug.km_pp_last_launches; return COGS_OK; }
     if (strcmp(name, "attn_vit_last_end") == 0) { *value = g_cogs_debug.attn_vit_last_end; return COGS_OK; }
     return COGS_E_INVALID;
 }
@@ -94,7 +95,8 @@ const char* cogs_debug_list(void) {
         "attn_last_kernel (read only): kernel of the last cogs_attention -- 1 general MFMA, 2 ViT unpipelined, 3 ViT pipelined, "
         "4 single-token decode, 5 prompt LDS-DMA, 7 row-wise fp32, 8 ViT pipelined on head-major K/V\n"
         "attn_vit_last_end (read only): ragged end of the last pipelined ViT attention launch -- 10 x tiles behind the four-tile loop + "
-        "32-key blocks of the last tile (41 .. 72: compile-time shape), 0 the run-time form\n";
+        "32-key blocks of the last tile (41 .. 72: compile-time shape), 0 the run-time form\n"
+        "km_pp_last_launches (read only): kernels per centre of the last cogs_kmeans_pp, 1 or 3\n";
 }
 
 cogs_status cogs_create(int device, cogs_handle* out) {

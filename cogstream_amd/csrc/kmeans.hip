@@ -290,7 +290,7 @@ __global__ __launch_bounds__(256) void reduce_assign_kernel(const float* __restr
 // row coincides with a chosen centre) is the reference's random.randint branch: flagged, the host then takes the step-wise
 // path. The sum runs in fp64 in a fixed order (torch's own fp32 summation order is not reproduced: the sum
 // is a common divisor of all ratios and only moves the argmax between ratios closer than a few ulps).
-// Run by 256 threads of the workgroup that measured the last row (others wrote nearest2: read past the caches).
+// Run by 256 threads, of kpp_select_kernel or of the workgroup that measured the last row (others wrote nearest2: read past the caches).
 __device__ __forceinline__ void kpp_select(float* nearest2, const float* __restrict__ q, int Tn, int* __restrict__ idx_out, int* __restrict__ zero_flag,
                                            int tid, double* red, float* rv, int* ri) {
     const int lane = tid & 63, wid = tid >> 6;
@@ -339,6 +339,13 @@ __device__ __forceinline__ void kpp_select(float* nearest2, const float* __restr
         *idx_out = i == 0x7fffffff ? 0 : i;
     }
 }
+__global__ __launch_bounds__(256) void kpp_select_kernel(float* nearest2, const float* __restrict__ q, int Tn, int* idx_out, int* zero_flag, int first_row) {
+    __shared__ double red[4];
+    __shared__ float rv[4];
+    __shared__ int ri[4];
+    if (first_row >= 0 && threadIdx.x == 0) idx_out[-1] = first_row;      // step 1 also records the caller's first centre
+    kpp_select(nearest2, q, Tn, idx_out, zero_flag, threadIdx.x, red, rv, ri);
+}
 
 // One k-means++ step (:46-60) of the whole-seeding call: workgroup t measures row t against the newest centre, a slice of 512
 // columns per wave at a time, folds the distance into nearest2[t], and the workgroup that finishes last draws the next centre. The sums are
@@ -349,9 +356,9 @@ constexpr int KPP_T = 1024;
 template <typename T>
 __global__ __launch_bounds__(KPP_T) void kpp_step_kernel(const T* __restrict__ x, int Tn, long PD, int nslices, const int* __restrict__ centre_from,
                                                          int centre_row, int first, float* nearest2, const float* __restrict__ q, int* idx_out,
-                                                         int* zero_flag, int* done, float* spill) {
+                                                         int* zero_flag, int* done) {
     extern __shared__ __attribute__((aligned(16))) char smem_raw[];
-    float* const sums = spill ? spill + (long)blockIdx.x * nslices : reinterpret_cast<float*>(smem_raw);       // [nslices]
+    float* const sums = reinterpret_cast<float*>(smem_raw);                                                     // [nslices]
     __shared__ double red[4];
     __shared__ float rv[4];
     __shared__ int ri[4], last;
@@ -861,6 +868,23 @@ int cogs_k_kmeans_pp_step(hipStream_t st, int dtype, const void* feats, int T, l
     return COGS_OK;
 }
 
+// Which form a centre of the whole seeding takes. One launch has a workgroup, and so a CU's intake, per row: it wins where rows are
+// about as many as CUs, or short. Fewer long rows leave CUs idle, more rows than CUs read the centre again for every round, where
+// sqdist keeps it in LDS. Time of three launches a centre over one (K = 18), by rows:        (MI355X; fp32 rows are twice as long)
+//                     T = 24    48    80   120   160   200   256   257   320   400
+//   bf16,  28 KB          1.7   1.6   1.6   1.4   1.2   1.2   1.1   1.2   1.05  1.1
+//   bf16,  84 KB          1.5   1.3   1.2   1.2   1.2   1.1   1.1   1.1   1.05  1.0
+//   bf16, 168 KB          1.2   1.0   1.1   1.1   1.2   1.2   1.1   0.95  0.88  0.94
+//   bf16, 350 KB          0.85  0.83  0.89  1.07  1.13  1.18  1.18  0.92  0.87  0.94
+//   bf16, 896 KB          0.55  0.69  0.82  1.01  1.11  1.20  1.18  0.82  0.77  0.86
+//   fp32, 168 KB          1.18  1.08  1.03  1.05  1.01  0.99  0.95  0.76  0.74  0.80
+//   fp32, 700 KB          0.65  0.63  0.81  0.94  1.02  1.09  1.09  0.78  0.80  0.75
+static bool kpp_in_one_launch(int dtype, int T, long PD) {
+    const long kb = PD * (dtype == COGS_DT_BF16 ? 2 : 4) >> 10;
+    if (dtype == COGS_DT_BF16) return T <= 256 ? kb <= 128 || (kb <= 1024 && T >= 120) : T <= 300 && kb <= 88;
+    return T <= 160 ? kb <= 176 : T <= 256 && kb >= 256 && kb <= 1024;
+}
+
 // The whole k-means++ seeding (kmeans_with_time.py:41-62) in one call, no host round trip per centre: step m measures
 // every row against the newest centre (row idx[m-1], read from device memory), folds it into nearest2 and draws centre m
 // as argmax(probs / q[m-1]) (kpp_select). q: device fp32 [K-1][T], the Exponential(1) draws the reference's K-1
@@ -872,21 +896,27 @@ int cogs_k_kmeans_pp(hipStream_t st, int dtype, const void* feats, int T, long P
     if (T <= 0 || K <= 0 || PD % 8 || !q || !idx || !zero_flag || !nearest2 || first_row < 0 || first_row >= T) return COGS_E_INVALID;
     const KmWs w = carve(ws, T, PD, 1);
     if (nslices != (int)((PD + SL - 1) / SL)) return COGS_E_WORKSPACE;
-    if (hipMemsetAsync(zero_flag, 0, sizeof(int), st) != hipSuccess || hipMemsetAsync(w.ctl, 0, sizeof(int), st) != hipSuccess) return COGS_E_HIP;
-    size_t lds = (size_t)nslices * 4;
-    float* spill = nullptr;
-    if (lds > 48 * 1024) { lds = 0; spill = w.partial; }         // more than six million columns: a row's sums in the workspace
+    const bool one = kpp_in_one_launch(dtype, T, PD);
+    if (hipMemsetAsync(zero_flag, 0, sizeof(int), st) != hipSuccess) return COGS_E_HIP;
+    if (one && hipMemsetAsync(w.ctl, 0, sizeof(int), st) != hipSuccess) return COGS_E_HIP;      // the counter of finished rows
+    g_cogs_debug.km_pp_last_launches = one ? 1 : 3;
+    const size_t lds = (size_t)nslices * 4;
     for (int m = 1; m < K; ++m) {
         // step 1 measures against the caller's first centre (a kernel argument: nothing is uploaded), later steps against
         // the row the previous step drew (read from device memory)
         const int* from = m == 1 ? nullptr : idx + (m - 1);
         const float* qm = q + (size_t)(m - 1) * T;
-        if (dtype == COGS_DT_BF16)
+        if (!one) {
+            const int rc = sqdist_partials(st, dtype, feats, T, PD, nullptr, from, m == 1 ? first_row : -1, 1, w.partial, nslices);
+            if (rc != COGS_OK) return rc;
+            hipLaunchKernelGGL(reduce_min_kernel, dim3((T + 3) / 4), dim3(256), 0, st, w.partial, nslices, T, m == 1 ? 1 : 0, nearest2);
+            hipLaunchKernelGGL(kpp_select_kernel, dim3(1), dim3(256), 0, st, nearest2, qm, T, idx + m, zero_flag, m == 1 ? first_row : -1);
+        } else if (dtype == COGS_DT_BF16)
             hipLaunchKernelGGL(kpp_step_kernel<bf16_t>, dim3(T), dim3(KPP_T), lds, st, (const bf16_t*)feats, T, PD, nslices, from, first_row, m == 1, nearest2,
-                               qm, idx + m, zero_flag, w.ctl, spill);
+                               qm, idx + m, zero_flag, w.ctl);
         else
             hipLaunchKernelGGL(kpp_step_kernel<float>, dim3(T), dim3(KPP_T), lds, st, (const float*)feats, T, PD, nslices, from, first_row, m == 1, nearest2,
-                               qm, idx + m, zero_flag, w.ctl, spill);
+                               qm, idx + m, zero_flag, w.ctl);
     }
     if (K == 1 && hipMemcpyAsync(idx, &first_row, sizeof(int), hipMemcpyHostToDevice, st) != hipSuccess) return COGS_E_HIP;
     return COGS_LAUNCH_CHECK();

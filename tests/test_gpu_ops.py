@@ -1102,11 +1102,13 @@ def test_fused_resize_equals_the_host_path(dev, t, h, w, merge, max_tokens, offs
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
-@pytest.mark.parametrize("T,PD,K", [(2, 8, 2), (5, 520, 4), (257, 1000, 9), (300, 4096, 12), (3, 6_300_000, 3)])
+@pytest.mark.parametrize("T,PD,K", [(2, 8, 2), (5, 520, 4), (257, 1000, 9), (300, 4096, 12), (3, 6_300_000, 3), (130, 179_200, 4), (24, 179_200, 4),
+                                    (256, 65_536, 3), (257, 65_536, 3), (160, 65_544, 3), (161, 65_536, 3)])
 def test_whole_seeding_equals_the_steps(dev, T, PD, K, dtype):
-    """cogs_kmeans_pp (one launch a centre) draws the rows that distances of cogs_kmeans_pp_step and the same exponentials give on the
-    host: one slice and fewer, a ragged last slice, more rows than a workgroup's threads draw from at once, rows whose slice sums no
-    longer fit the LDS; rows that all coincide raise the flag"""
+    """cogs_kmeans_pp draws the rows that distances of cogs_kmeans_pp_step and the same exponentials give on the host, with one launch a
+    centre and with three: one slice and fewer, a ragged last slice, more rows than a workgroup's threads draw from at once, sizes on
+    both sides of the lines between the two; rows that all coincide raise the flag"""
+    from cogstream_amd import _lib as L2
     ops = _ops()
     g = torch.Generator(device=dev).manual_seed(T)
     x = torch.randn(T, PD, generator=g, device=dev).to(dtype)
@@ -1114,6 +1116,11 @@ def test_whole_seeding_equals_the_steps(dev, T, PD, K, dtype):
     first = T // 2
     ws = ops.kmeans_workspace(T, PD, K, x.device)
     idx, flag = ops.kmeans_pp(x, first, K, q.to(dev), ws)
+    kb = PD * x.element_size() >> 10
+    if T > 400 or kb > 1024 or (T < 100 and kb > 256) or (T > 256 and kb > 100):     # few long rows, more rows than CUs: the slower form of 0.5 to 0.9
+        assert L2.debug_get("km_pp_last_launches") == 3
+    elif T <= 160 and kb <= 128:
+        assert L2.debug_get("km_pp_last_launches") == 1
     want, near = [first], torch.empty(T, device=dev)
     probs = torch.empty(T).pin_memory()
     for m in range(K - 1):
