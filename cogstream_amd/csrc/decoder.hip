@@ -195,7 +195,7 @@ struct Step {
                 CogsMla a{};
                 a.Q = k.qlat; a.ldq = (long)m.heads * G.kvw; a.q_head = G.kvw; a.q_rot = G.kvp; a.ldk = a.ldkr = a.ldv = G.kvw;
                 a.O = k.olat; a.ldo = (long)m.heads * G.kvp; a.o_head = G.kvp; a.dn = G.kvp; a.dr = G.rotc; a.dv = G.kvp; a.heads = m.heads;
-                a.sink = m.sink; a.seqs = k.seqs; a.nseq = nseq; a.rowseq = k.rowseq; a.rows = S; a.max_new = 1; a.max_ctx = max_ctx;
+                a.sink = m.sink; a.seqs = k.seqs; a.nseq = nseq; a.rowseq = k.rowseq; a.rows = S; a.max_new = 1;
                 a.absorbed = 1; a.layer_off = run.cache_off; a.kr_col = G.kvp;
                 PROF(COGS_PROF_ATTN);
                 COGS_TRY(cogs_k_mla_attention(st, dt, a));
@@ -217,7 +217,7 @@ struct Step {
             a.Q = k.q; a.ldq = qcols; a.q_head = G.dq; a.q_rot = G.dk; a.K = k.kvx; a.ldk = G.kvcols; a.k_head = G.dn;
             a.KR = at(ctx, G.kvp); a.ldkr = G.kvw; a.V = at(k.kvx, (size_t)m.heads * G.dn); a.ldv = G.kvcols; a.v_head = G.dv;
             a.O = k.att; a.ldo = G.oin; a.o_head = G.dv; a.dn = G.dn; a.dr = G.dr; a.dv = G.dv; a.heads = m.heads;
-            a.sink = m.sink; a.gate = gate; a.seqs = k.seqs; a.nseq = nseq; a.rowseq = k.rowseq; a.rows = S; a.max_new = max_new; a.max_ctx = max_ctx;
+            a.sink = m.sink; a.gate = gate; a.seqs = k.seqs; a.nseq = nseq; a.rowseq = k.rowseq; a.rows = S; a.max_new = max_new;
             PROF(COGS_PROF_ATTN);
             COGS_TRY(cogs_k_mla_attention(st, dt, a));
         }
@@ -254,7 +254,7 @@ struct Step {
         } else {
             CogsMla a{};
             a.Q = k.q; a.ldq = (long)m.heads * G.dk; a.q_head = a.q_rot = G.dk; a.ldk = a.ldv = G.kvw; a.O = k.att; a.ldo = G.oin; a.o_head = G.dv;
-            a.dn = G.dk; a.dv = G.dv; a.heads = m.heads; a.seqs = k.seqs; a.nseq = nseq; a.rowseq = k.rowseq; a.rows = S; a.max_new = max_new; a.max_ctx = max_ctx;
+            a.dn = G.dk; a.dv = G.dv; a.heads = m.heads; a.seqs = k.seqs; a.nseq = nseq; a.rowseq = k.rowseq; a.rows = S; a.max_new = max_new;
             a.layer_off = run.cache_off; a.kvw = G.kvw; a.v_col = G.dk; a.rep = rep; a.bias = m.dist_bias; a.nb = m.dist_n;
             PROF(COGS_PROF_ATTN);
             COGS_TRY(cogs_k_mla_attention(st, dt, a));

@@ -225,7 +225,7 @@ struct CogsMla {
     int dn, dr, dv, heads;
     const float* sink;                           // [heads] in log2 units, or null
     const float* gate;                           // [rows][heads], or null
-    const CogsSeq* seqs; int nseq; const int* rowseq; int rows, max_new, max_ctx;     // (new rows and keys of the longest sequence)
+    const CogsSeq* seqs; int nseq; const int* rowseq; int rows, max_new;     // (new rows of the longest sequence)
     int absorbed; long layer_off; int kr_col;
     // kvw != 0: keys and values per head from the sequence's cache (K / KR / V unused): blocks [max_len][kvw] of heads / rep key / value
     // heads from column layer_off on, rows [key | value from v_col]; ldk = ldv = kvw, dr = 0, q_rot = q_head

@@ -288,6 +288,21 @@ def test_a_query_tile_by_one_wave_or_by_two(dev, name):
             assert rms_err(out, lg[[n - 1 for _, n in jobs]]) < TOL[torch.bfloat16], (times, cut)
 
 
+def test_short_prompts_beside_a_long_one(dev):
+    """a prompt of many key tiles by itself has each query tile's keys shared by two waves; short ones beside it, most of whose query tiles are
+    empty, take that away (every workgroup would wait for a whole CU) and none of the result"""
+    from cogstream_amd import _lib as L
+    cfg, st, e, toks, _, _ = named("peaked", torch.bfloat16, dev, 150)
+    toks = tokens(cfg, 1100, seed=3)
+    lens = [1100] + [64] * 15
+    alone = [sequences(e).step([("r", toks[:n], [n - 1])]).cpu() for n in (64, 1100)]
+    assert L.debug_get("mla_last_waves") == 8
+    out = sequences(e).step([(i, toks[:n], [n - 1]) for i, n in enumerate(lens)])
+    assert L.debug_get("mla_last_waves") == 4
+    for i, n in enumerate(lens):
+        assert rms_err(out[i:i + 1], alone[n == 1100]) < TOL[torch.bfloat16]
+
+
 def test_unsupported_calls_are_refused(dev):
     from cogstream_amd import _lib as L
     cfg, st, e, toks, _, _ = named("peaked", torch.bfloat16, dev, 150)
