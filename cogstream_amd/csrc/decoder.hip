@@ -76,7 +76,8 @@ Work carve(const CogsDecoder& d, int S, int nseq, int64_t C, int n_want, void* w
     k.x = (float*)c.take(n * d.wp * 4 * (d.w.streams > 0 ? d.w.streams : 1));
     k.h = c.take(n * d.wp * es);
     k.y = c.take(n * d.wp * es);
-    if (S <= 64) k.ypart = (float*)c.take(n * d.wp * 4 * COGS_SKINNY_MAX_PARTS);     // few-row products into the residual stream
+    // few-row products into the residual stream; there for more rows too, so that a workspace sized for them serves fewer
+    if (d.w.dtype == COGS_DT_BF16) k.ypart = (float*)c.take((size_t)(S < 64 ? S : 64) * d.wp * 4 * COGS_SKINNY_MAX_PARTS);
     k.t32 = (float*)c.take(n * d.max_t32 * 4);
     k.cq = c.take(n * d.max_cq * es);
     k.q = c.take(n * d.max_q * es);

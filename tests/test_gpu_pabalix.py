@@ -303,6 +303,21 @@ def test_short_prompts_beside_a_long_one(dev):
         assert rms_err(out[i:i + 1], alone[n == 1100]) < TOL[torch.bfloat16]
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_a_workspace_serves_every_smaller_step(dev, dtype):
+    """of one sequence, from two rows on: few rows need partial sums of their own, and no more memory for them than more rows do"""
+    import ctypes as C
+    from cogstream_amd import _lib as L
+    cfg, st, e, toks, _, _ = named("mixed", dtype, dev, 150)
+    e._activate()
+    sizes = []
+    for rows in range(2, 140):
+        n = C.c_size_t()
+        L.check(L.lib.cogs_decoder_workspace_bytes(e.handle.h, rows, 1, 200, 1, C.byref(n)))
+        sizes.append(n.value)
+    assert sizes == sorted(sizes)
+
+
 def test_unsupported_calls_are_refused(dev):
     from cogstream_amd import _lib as L
     cfg, st, e, toks, _, _ = named("peaked", torch.bfloat16, dev, 150)
