@@ -19,7 +19,8 @@ from .runtime import get_handle
 @lru_cache(maxsize=64)
 def _tables(in_size: int, out_size: int, device: int):
     """tap tables of a resize on a device. Kept by size, not copied up on every call: four copies that wait for the device each
-    took as long as the kernel. The copies are complete when the tables enter the cache, so any stream may read them."""
+    took as long as the kernel. The copies are complete when the tables enter the cache; a stream that reads them is recorded with them
+    (the caller's part), so that an entry that leaves the cache is not reused under a queued kernel."""
     b, k, ks = resample_coeffs(in_size, out_size)
     dev = torch.device("cuda", device)
     return torch.from_numpy(np.ascontiguousarray(b)).to(dev), torch.from_numpy(np.ascontiguousarray(k)).to(dev), ks
@@ -42,12 +43,16 @@ def preprocess_media_gpu(items: Sequence[torch.Tensor], merge_sizes: Sequence[in
     handle = get_handle(dev)
     index = dev.index if dev.index is not None else torch.cuda.current_device()
     table = _value_table(index)
+    stream = torch.cuda.current_stream(dev)
+    table.record_stream(stream)
     outs, grids = [], []
     for v, merge_size, (th, tw) in zip(items, merge_sizes, targets):
         assert v.dtype == torch.uint8 and v.is_contiguous() and v.shape[-1] == 3
         t, H, W = int(v.shape[0]), int(v.shape[1]), int(v.shape[2])
         dbx, dkx, ksx = _tables(W, tw, index)
         dby, dky, ksy = _tables(H, th, index)
+        for taps in (dbx, dkx, dby, dky):
+            taps.record_stream(stream)
         gh, gw = th // PATCH, tw // PATCH
         out = torch.empty(t * gh * gw, 3 * PATCH * PATCH, device=dev, dtype=out_dtype)
         n = C.c_size_t()

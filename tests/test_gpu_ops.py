@@ -1101,6 +1101,28 @@ def test_fused_resize_equals_the_host_path(dev, t, h, w, merge, max_tokens, offs
         assert torch.equal(got["pixel_values"].cpu(), torch.from_numpy(ref["pixel_values"]).to(dtype))
 
 
+def test_tap_tables_outlive_their_place_in_the_cache(dev):
+    """a resize queued on a side stream, and tables that leave the cache before it runs: their memory, asked for again on the stream that
+    made them, is not theirs until the resize is done. (Zeros in it would be tables of no taps: a black clip, no read out of place)"""
+    from cogstream_amd import preprocess_gpu as pg
+    frames = torch.randint(1, 256, (1, 300, 400, 3), device=dev, dtype=torch.uint8)
+    want = pg.preprocess_videos_gpu([frames])["pixel_values"].clone()
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        torch.cuda._sleep(200_000_000)
+        got = pg.preprocess_videos_gpu([frames])["pixel_values"]
+    tables = [(t.data_ptr(), t.numel() * 4) for key in ((400, 392), (300, 308)) for t in pg._tables(*key, 0)[:2]] + [(pg._value_table(0).data_ptr(), 3072)]
+    pg._tables.cache_clear()
+    pg._value_table.cache_clear()
+    reused = [torch.zeros(1 << 14, device=dev, dtype=torch.int32) for _ in range(64)]      # more than the small blocks' segments hold
+    assert not side.query(), "the resize must still be queued here"
+    for x in reused:
+        assert not any(p < x.data_ptr() + x.numel() * 4 and x.data_ptr() < p + n for p, n in tables)
+    torch.cuda.synchronize()
+    assert torch.equal(got, want)
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("T,PD,K", [(2, 8, 2), (5, 520, 4), (257, 1000, 9), (300, 4096, 12), (3, 6_300_000, 3), (130, 179_200, 4), (24, 179_200, 4),
                                     (256, 65_536, 3), (257, 65_536, 3), (160, 65_544, 3), (161, 65_536, 3)])
