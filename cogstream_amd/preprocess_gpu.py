@@ -38,6 +38,8 @@ def preprocess_media_gpu(items: Sequence[torch.Tensor], merge_sizes: Sequence[in
     dev = items[0].device
     if dev.type != "cuda":
         raise L.CogsError("preprocess_media_gpu needs frames on the GPU")
+    if torch.cuda.is_current_stream_capturing():       # a replay would read tap tables that the cache may have given back
+        raise L.CogsError("preprocess_media_gpu cannot be captured in a graph")
     shapes = [(int(v.shape[0]), int(v.shape[1]), int(v.shape[2])) for v in items]
     targets = media_target_sizes(shapes, list(merge_sizes), min_tokens, max_tokens)
     handle = get_handle(dev)

@@ -1123,6 +1123,17 @@ def test_tap_tables_outlive_their_place_in_the_cache(dev):
     assert torch.equal(got, want)
 
 
+def test_preprocessing_is_not_captured(dev):
+    """also when the size's tables are there already: they are the cache's, not the graph's"""
+    from cogstream_amd import _lib as L2
+    from cogstream_amd.preprocess_gpu import preprocess_videos_gpu
+    frames = torch.randint(0, 256, (1, 56, 84, 3), device=dev, dtype=torch.uint8)
+    want = preprocess_videos_gpu([frames])["pixel_values"].clone()
+    with pytest.raises(L2.CogsError), torch.cuda.graph(torch.cuda.CUDAGraph()):
+        preprocess_videos_gpu([frames])
+    assert torch.equal(preprocess_videos_gpu([frames])["pixel_values"], want)
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("T,PD,K", [(2, 8, 2), (5, 520, 4), (257, 1000, 9), (300, 4096, 12), (3, 6_300_000, 3), (130, 179_200, 4), (24, 179_200, 4),
                                     (256, 65_536, 3), (257, 65_536, 3), (160, 65_544, 3), (161, 65_536, 3)])
