@@ -207,10 +207,10 @@ __device__ __forceinline__ f32x4 sum_parts(const float* q, long step) {
     for (int s = 1; s < NP; ++s) part[0] += part[s];
     return part[0];
 }
-// four columns of a sublayer's output
-template <typename T>
+// four columns of a sublayer's output; PARTS: in partial sums
+template <typename T, bool PARTS>
 __device__ __forceinline__ f32x4 stream_y(const CogsStreamNorm& p, long row, int i) {
-    if (p.y_parts == 0) return ld4_f<T>(reinterpret_cast<const T*>(p.y) + row * p.Hp + i);
+    if constexpr (!PARTS) return ld4_f<T>(reinterpret_cast<const T*>(p.y) + row * p.Hp + i);
     const float* q = reinterpret_cast<const float*>(p.y) + row * p.Hp + i;
     const long step = (long)p.rows * p.Hp;
     return p.y_parts == 2 ? sum_parts<2>(q, step) : p.y_parts == 4 ? sum_parts<4>(q, step) : sum_parts<8>(q, step);
@@ -218,7 +218,7 @@ __device__ __forceinline__ f32x4 stream_y(const CogsStreamNorm& p, long row, int
 
 // fp32 residual stream around a sublayer (kernels.h, CogsStreamNorm): one workgroup of TPB threads per row, the row in
 // registers (C chunks of four columns per thread). Norms entirely in fp32, one rounding of the normed row.
-template <typename T, int C, int TPB>
+template <typename T, int C, int TPB, bool PARTS>
 __global__ __launch_bounds__(TPB) void stream_norm_kernel(CogsStreamNorm p) {
     constexpr int NW = TPB / 64;
     __shared__ float red[2][NW];
@@ -248,7 +248,7 @@ __global__ __launch_bounds__(TPB) void stream_norm_kernel(CogsStreamNorm p) {
         for (int c = 0; c < C; ++c) {
             const int i = (tid + TPB * c) * 4;
             y[c] = f32x4{0.f, 0.f, 0.f, 0.f};
-            if (i < p.Hp) y[c] = stream_y<T>(p, row, i);
+            if (i < p.Hp) y[c] = stream_y<T, PARTS>(p, row, i);
 #pragma unroll
             for (int e = 0; e < 4; ++e) ss += y[c][e] * y[c][e];
         }
@@ -292,7 +292,7 @@ __global__ __launch_bounds__(TPB) void stream_norm_kernel(CogsStreamNorm p) {
 
 // the same with a scaled embedding and a position table at the start and hyper-connected streams (x [row][stream][Hp]). NS: streams
 // rounded up; a chunk's old streams are in registers together, only the combination that is normed stays there for the row.
-template <typename T, int C, int TPB, int NS>
+template <typename T, int C, int TPB, int NS, bool PARTS>
 __global__ __launch_bounds__(TPB) void stream_mix_kernel(CogsStreamNorm p) {
     constexpr int NW = TPB / 64;
     __shared__ float red[2][NW];
@@ -317,7 +317,7 @@ __global__ __launch_bounds__(TPB) void stream_mix_kernel(CogsStreamNorm p) {
         for (int c = 0; c < C; ++c) {
             const int i = (tid + TPB * c) * 4;
             y[c] = f32x4{0.f, 0.f, 0.f, 0.f};
-            if (i < p.Hp) y[c] = stream_y<T>(p, row, i);
+            if (i < p.Hp) y[c] = stream_y<T, PARTS>(p, row, i);
 #pragma unroll
             for (int e = 0; e < 4; ++e) ss += y[c][e] * y[c][e];
         }
@@ -386,15 +386,23 @@ __global__ __launch_bounds__(TPB) void stream_mix_kernel(CogsStreamNorm p) {
 template <typename T, int NS>
 int launch_stream_mix(hipStream_t st, const CogsStreamNorm& a) {
     const dim3 grid(a.rows);
-#define COGS_STREAM(C, TPB) hipLaunchKernelGGL((stream_mix_kernel<T, C, TPB, NS>), grid, dim3(TPB), 0, st, a)
+#define COGS_STREAM(C, TPB) hipLaunchKernelGGL((stream_mix_kernel<T, C, TPB, NS, false>), grid, dim3(TPB), 0, st, a)
+// (partial sums come of products of at most 64 rows)
+#define COGS_STREAM_FEW(C, TPB)                                                                                                     \
+    do {                                                                                                                            \
+        if (a.y_parts > 0) hipLaunchKernelGGL((stream_mix_kernel<T, C, TPB, NS, true>), grid, dim3(TPB), 0, st, a);                 \
+        else COGS_STREAM(C, TPB);                                                                                                   \
+    } while (0)
     if (a.rows <= 64 && a.Hp > 1024) {
-        if (a.Hp <= 4096) COGS_STREAM(1, 1024);
-        else if (a.Hp <= 16384) COGS_STREAM(4, 1024);
+        if (a.Hp <= 4096) COGS_STREAM_FEW(1, 1024);
+        else if (a.Hp <= 16384) COGS_STREAM_FEW(4, 1024);
         else return COGS_E_UNSUPPORTED;
-    } else if (a.Hp <= 1024) COGS_STREAM(1, 256);
+    } else if (a.Hp <= 1024) COGS_STREAM_FEW(1, 256);
+    else if (a.y_parts > 0) return COGS_E_UNSUPPORTED;
     else if (a.Hp <= 4096) COGS_STREAM(4, 256);
     else if (a.Hp <= 16384) COGS_STREAM(16, 256);
     else return COGS_E_UNSUPPORTED;
+#undef COGS_STREAM_FEW
 #undef COGS_STREAM
     return COGS_LAUNCH_CHECK();
 }
@@ -410,18 +418,25 @@ int launch_stream_norm(hipStream_t st, const CogsStreamNorm& a) {
         return COGS_E_UNSUPPORTED;
     }
     const dim3 grid(a.rows);
-#define COGS_STREAM(C, TPB) hipLaunchKernelGGL((stream_norm_kernel<T, C, TPB>), grid, dim3(TPB), 0, st, a)
+#define COGS_STREAM(C, TPB) hipLaunchKernelGGL((stream_norm_kernel<T, C, TPB, false>), grid, dim3(TPB), 0, st, a)
+#define COGS_STREAM_FEW(C, TPB)                                                                                                     \
+    do {                                                                                                                            \
+        if (a.y_parts > 0) hipLaunchKernelGGL((stream_norm_kernel<T, C, TPB, true>), grid, dim3(TPB), 0, st, a);                    \
+        else COGS_STREAM(C, TPB);                                                                                                   \
+    } while (0)
     if (a.rows <= 64 && a.Hp > 1024) {           // few rows: latency, not bandwidth -- more threads on each
-        if (a.Hp <= 4096) COGS_STREAM(1, 1024);
-        else if (a.Hp <= 8192) COGS_STREAM(2, 1024);
-        else if (a.Hp <= 16384) COGS_STREAM(4, 1024);
+        if (a.Hp <= 4096) COGS_STREAM_FEW(1, 1024);
+        else if (a.Hp <= 8192) COGS_STREAM_FEW(2, 1024);
+        else if (a.Hp <= 16384) COGS_STREAM_FEW(4, 1024);
         else return COGS_E_UNSUPPORTED;
-    } else if (a.Hp <= 1024) COGS_STREAM(1, 256);
+    } else if (a.Hp <= 1024) COGS_STREAM_FEW(1, 256);
+    else if (a.y_parts > 0) return COGS_E_UNSUPPORTED;
     else if (a.Hp <= 2048) COGS_STREAM(2, 256);
     else if (a.Hp <= 4096) COGS_STREAM(4, 256);
     else if (a.Hp <= 8192) COGS_STREAM(8, 256);
     else if (a.Hp <= 16384) COGS_STREAM(16, 256);
     else return COGS_E_UNSUPPORTED;
+#undef COGS_STREAM_FEW
 #undef COGS_STREAM
     return COGS_LAUNCH_CHECK();
 }
