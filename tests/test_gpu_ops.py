@@ -23,6 +23,13 @@ def _L():
     return _lib
 
 
+@pytest.fixture(params=[1, 0], ids=["dispatched", "unsplit"])
+def gemm_split(request):
+    """products as the dispatch takes them, and (0) wholly by the ping-pong kernel from 256 rows on where N pads to 256 by at most 12 %"""
+    with _L().debug_switch("gemm_split", request.param):
+        yield request.param
+
+
 @pytest.mark.parametrize("dtype,tol", [(torch.bfloat16, 1.2e-2), (torch.float32, 2e-5)])
 @pytest.mark.parametrize("M,N,K", [(128, 128, 64), (300, 256, 192), (1, 512, 256), (77, 132, 128), (1024, 1152, 1152),
                                    (515, 132, 64), (777, 384, 704)])
@@ -42,7 +49,7 @@ def test_gemm_bias_residual(dev, dtype, tol, M, N, K):
 def test_gemm_integer_exact(dev):
     """MFMA fragment/layout check with exactly representable data and an asymmetric W"""
     run_gemm_integer_exact(dev, 256, 256, 128)
-    run_gemm_integer_exact(dev, 1024 + 40, 384, 448)   # 256x128 ring-buffered variant, ragged M
+    run_gemm_integer_exact(dev, 1024 + 40, 384, 448)   # fp32: 256x128 ring-buffered variant, ragged M
 
 
 def run_gemm_integer_exact(dev, M, N, K):
@@ -86,9 +93,9 @@ def test_gemm_swiglu(dev, M):
 
 @pytest.mark.parametrize("M,heads,interleaved", [(1, 2, False), (96, 2, False), (96, 2, True), (1300, 2, True),
                                                  (1300, 7, True), (1300, 7, False)])
-def test_gemm_rope_epilogue(dev, M, heads, interleaved):
+def test_gemm_rope_epilogue(dev, gemm_split, M, heads, interleaved):
     """columns [0, rope_cols) rotated as rotate_half pairs after the (d, d+hd/2) row interleave; both table
-    formats; M = 1300 reaches the 256x128 (heads 2) and ping-pong (heads 7) kernels, whose interior wave tiles
+    formats; M = 1300 reaches the mid-size (heads 2, and 7 as dispatched) and ping-pong (heads 7) kernels, whose interior wave tiles
     take the lean epilogue while the tile straddling rope_cols and the ragged last row block take the general one"""
     ops = _ops()
     torch.manual_seed(3)
@@ -119,13 +126,13 @@ def test_gemm_rope_epilogue(dev, M, heads, interleaved):
     assert rel_err(out.float().view(M, 3 * heads, hd), refp) < 1.2e-2
 
 
-def test_gemm_rope_position_lut_equals_row_table(dev):
+def test_gemm_rope_position_lut_equals_row_table(dev, gemm_split):
     """the ping-pong GEMM's LDS position LUT (2-D rotary: first half of a head's pairs uses the row's h, second half
     its w) must give bit-identical outputs to the per-row (cos, sin) table built from the same angles -- and both
     must match the plain reference"""
     ops = _ops()
     torch.manual_seed(17)
-    hd, heads, K, M = 72, 7, 128, 1500            # N = 1512: ping-pong kernel; ragged last row block; rope straddle
+    hd, heads, K, M = 72, 7, 128, 1500            # N = 1512: unsplit, the ping-pong kernel; ragged last row block; rope straddle
     nf, maxpos = hd // 4, 45
     N = 3 * heads * hd
     x = torch.randn(M, K).bfloat16()
@@ -615,7 +622,8 @@ def test_whole_line_gemm_equals_the_k_tile_gemm_bit_for_bit(dev):
     """gemm_tn_pp64_kernel (round 4: 64-wide slabs of whole 128-byte lines in a five-unit ring, three kinds of slab, the
     two wave groups' epilogues in one interval) must produce the bits of gemm_tn_pp_kernel (32-wide K-tiles): same tile,
     same MFMA order, same epilogues. The second kernel is reached through the debug switch gemm_pp64 = 0 (the dispatch
-    is asked which body ran). Shapes: the cfg2 ViT GEMMs at a quarter of the clip (several rounds of the persistent grid,
+    is asked which body ran), as the dispatch takes them -- where it sends a shape, or a split's remainder, to the mid-size kernel both
+    sides have that part in common -- and with gemm_split = 0, where all of the product is theirs. Shapes: the cfg2 ViT GEMMs at a quarter of the clip (several rounds of the persistent grid,
     ragged last row block), a frame-sharded share (few tiles), the Qwen2 gate/up and down projections at 2 100 rows
     (SwiGLU epilogue; K = 18 944: 296 slabs per tile)."""
     from cogstream_amd import _lib as L2
@@ -637,6 +645,15 @@ def test_whole_line_gemm_equals_the_k_tile_gemm_bit_for_bit(dev):
             out = _gemm(**kw)
             assert L2.debug_get("gemm_last_body") in (2, 3, 5), L2.debug_get("gemm_last_body")
         return out
+
+    def both_whole(tag, **kw):
+        with L2.debug_switch("gemm_split", 0):
+            a = _gemm(**kw)
+            assert L2.debug_get("gemm_last_body") == 4, tag
+            with L2.debug_switch("gemm_pp64", 0):
+                b = _gemm(**kw)
+                assert L2.debug_get("gemm_last_body") == 3, tag
+        assert torch.equal(a, b), tag
 
     class _Ops:
         gemm = staticmethod(gemm_ab)
@@ -664,6 +681,7 @@ def test_whole_line_gemm_equals_the_k_tile_gemm_bit_for_bit(dev):
                 b = ops.gemm(**kw, lib=alt)
                 torch.cuda.synchronize()
                 assert torch.equal(a, b), (M, name, rep, float((a.float() - b.float()).abs().max()))
+            both_whole((M, name), **kw)
     xq, inter = rnd(2100, 3584), rnd(2100, 18944)
     for name, kw in (("gate/up swiglu", dict(a=xq, w=rnd(2 * 18944, 3584), act=L2.ACT_SWIGLU)),
                      ("down+res", dict(a=inter, w=rnd(3584, 18944), residual=rnd(2100, 3584)))):
@@ -671,6 +689,7 @@ def test_whole_line_gemm_equals_the_k_tile_gemm_bit_for_bit(dev):
         b = ops.gemm(**kw, lib=alt)
         torch.cuda.synchronize()
         assert torch.equal(a, b), (name, float((a.float() - b.float()).abs().max()))
+        both_whole(name, **kw)
 
 
 def test_tall_ragged_column_tiles_equal_padded_tiles_bit_for_bit(dev):
@@ -680,7 +699,8 @@ def test_tall_ragged_column_tiles_equal_padded_tiles_bit_for_bit(dev):
     gemm_tall = 0). Shapes: row counts that are / are not multiples of 384 and of 256, fewer rows than one tall tile's second
     and third row group, a ragged block narrower than 128 columns (generic epilogue in its second column group), every fused
     ViT epilogue of an N = 1152 / 3456 GEMM (bias + residual + row statistics, rotary + head-major), walk groups forced to
-    3 / 6 / 9 row blocks, and the few-tile split choices of a frame-sharded share (gemm_split)."""
+    3 / 6 / 9 row blocks, and the few-tile split choices of a frame-sharded share. The dispatch sends most of these shapes, or part of
+    them, to the mid-size kernel: with gemm_split = 0 every shape that pads to whole column blocks by at most 12 % is all theirs."""
     from cogstream_amd import _lib as L2
     ops = _ops()
     g = torch.Generator(device=dev).manual_seed(17)
@@ -728,12 +748,12 @@ def test_tall_ragged_column_tiles_equal_padded_tiles_bit_for_bit(dev):
         ]
         for name, kw in cases:
             bodies.add(both((M, name), **kw))
+            with L2.debug_switch("gemm_split", 0):
+                n = kw["w"].shape[0]
+                assert both((M, name, "unsplit"), **kw) == (4 if -(-n // 256) * 256 * 100 <= n * 112 else 2)
         for gm in (3, 4, 9):
-            with L2.debug_switch("gemm_group_m", gm):
+            with L2.debug_switch("gemm_group_m", gm), L2.debug_switch("gemm_split", 0):
                 bodies.add(both((M, "group_m", gm), **cases[0][1]))
-        with L2.debug_switch("gemm_split", 0):
-            bodies.add(both((M, "unsplit"), **cases[0][1]))
-            bodies.add(both((M, "unsplit fc2"), **cases[1][1]))
     assert 4 in bodies, bodies          # the whole-line kernel (and with it the tall walk) did run
 
 
@@ -815,12 +835,12 @@ def test_round5_prompt_attention_kernel_is_as_close_to_fp32_as_the_round4_kernel
 
 
 @pytest.mark.parametrize("M", [300, 1300, 4096])
-def test_gemm_row_stats_and_ln_fold(dev, M):
+def test_gemm_row_stats_and_ln_fold(dev, gemm_split, M):
     """LayerNorm fused around the GEMMs: (1) a residual-stream GEMM (N = hidden) also writes per-row partial sums,
     cogs_ln_finalize turns them into (rstd, -rstd * mean); (2) the consuming GEMM reads x itself with W * diag(gamma)
     (rows centred) and applies rstd_r * acc + c_n -- together LN(x) W^T + bias of nn.LayerNorm + nn.Linear
-    (model/modeling_videollama3_encoder.py:382-391). M = 300 / 1300 / 4096 reach the 128x128, 256x128 + ragged ping-pong
-    and the full ping-pong kernels."""
+    (model/modeling_videollama3_encoder.py:382-391). The mid-size kernel (as dispatched) and the ping-pong kernel with
+    ragged last row blocks."""
     ops = _ops()
     torch.manual_seed(M)
     H, N2, eps = 1152, 1472, 1e-6
@@ -957,13 +977,13 @@ def L_ACT_GELU():
 
 @pytest.mark.parametrize("M,heads,fold", [(96, 2, False), (1300, 2, True), (1300, 7, True), (2048 + 40, 16, True), (6400, 16, False),
                                           (14824, 16, True)])
-def test_gemm_head_major_output_equals_row_major_bit_for_bit(dev, M, heads, fold):
+def test_gemm_head_major_output_equals_row_major_bit_for_bit(dev, gemm_split, M, heads, fold):
     """cogs_gemm_desc.hm_rows (round 5: the encoder's QKV GEMM stores q | k | v as [block][head][row][hd] so that the
     attention kernel streams whole 128-byte lines): the same epilogue arithmetic, only the store address changes -- the
     head-major result must be the row-major result re-arranged, bit for bit. heads = 2 / 7: hm_cols is not a multiple of
     64, so a wave tile straddles q / k / v and every tile takes the general epilogue; heads = 16 (the production width):
-    interior tiles take the lean paired epilogue; M covers the 128x128, 256x128 ring and ping-pong kernels, a ragged last
-    row block, and the round-aligned split (14 824 rows)."""
+    interior tiles take the lean paired epilogue; M covers the mid-size and ping-pong kernels, a ragged last
+    row block, and the round-aligned split (6 400 rows as dispatched)."""
     ops = _ops()
     g = torch.Generator(device=dev).manual_seed(M + heads)
     hd, K = 72, 1152 if heads == 16 else 128
@@ -1037,8 +1057,10 @@ def test_mid_size_gemm_tiles_equal_each_other_and_fp64(dev, tile):
     """gemm_mid.hip: every tile size, forced, at the edges of its tiles (rows and columns one short of and past a tile, a ragged
     last one, fewer slabs than the ring has slots, odd slab counts), with each fused epilogue. Against float64 products of the same bf16
     operands: the output's rounding is half a bf16 step (8 significant bits: spacing 2^-7 in [1, 2), half of it 2^-8 of the value at the
-    most), the fp32 sums of up to 1152 products add at most 2^-20 of the sum of |a||w|; fp32 outputs only have the latter. And bit for bit against the kernel that the dispatch picks: a row's
-    bits must not depend on the tile."""
+    most), the fp32 sums of up to 1152 products add at most 2^-20 of the sum of |a||w|; fp32 outputs only have the latter; behind an
+    activation (slope 1.13 at the most) the sums' part grows by that and its exponential and reciprocal add 2^-18 of the value; the
+    statistics are sums of the stored values. And bit for bit against the tile that the dispatch picks and, from 256 rows on and where N
+    pads to 256 by at most 12 %, the ping-pong kernel: a row's bits must not depend on either."""
     from cogstream_amd import _lib as L2
     ops = _ops()
     g = torch.Generator(device=dev).manual_seed(tile)
@@ -1055,18 +1077,39 @@ def test_mid_size_gemm_tiles_equal_each_other_and_fp64(dev, tile):
                       ("rotary, head-major, folded norm", dict(rope_cos=table, rope_cols=64, head_dim=64, hm_cols=N, **fold))]
         for name, kw in cases:
             outs = []
-            for t in (tile, 0):
-                with L2.debug_switch("gemm_mid", t):
+            for t, split in ((tile, 1), (0, 1)) + (((0, 0),) if M >= 256 and -(-N // 256) * 256 * 100 <= N * 112 else ()):
+                with L2.debug_switch("gemm_mid", t), L2.debug_switch("gemm_split", split):
                     stats = kw.get("row_stats")
                     if stats is not None:
                         stats.fill_(-7.0)
                     outs.append((ops.gemm(a, w, **kw).clone(), None if stats is None else stats.clone()))
-            (x, sx), (y, sy) = outs
-            assert torch.equal(x, y), (M, N, K, name)
-            assert sx is None or torch.equal(sx, sy), (M, N, K, name)
+                    assert split or L2.debug_get("gemm_last_body") == 4
+            x, sx = outs[0]
+            for y, sy in outs[1:]:
+                assert torch.equal(x, y), (M, N, K, name)
+                assert sx is None or torch.equal(sx, sy), (M, N, K, name)
+            ref = a.double() @ w.double().t()
+            size = a.double().abs() @ w.double().abs().t()
+            if sx is not None:
+                blocks = x.double().view(M, N // 64, 64)
+                for got, terms in ((sx[..., 0], blocks), (sx[..., 1], blocks ** 2)):
+                    assert bool(((got.double() - terms.sum(-1)).abs() <= terms.abs().sum(-1) * 2.0 ** -18).all()), (M, N, K, name)
+            if name == "gelu":
+                z = ref + b.double()
+                want = F.gelu(z, approximate="tanh")
+                bound = size * 1.13 * 2.0 ** -20 + z.abs() * 2.0 ** -18 + want.abs() * 2.0 ** -8 + 1e-30
+                assert bool(((x.double() - want).abs() <= bound * 1.01).all()), (M, N, K, name)
+            if name == "swiglu":
+                gate, up, eg, eu = ref[:, 0::2], ref[:, 1::2], size[:, 0::2] * 2.0 ** -20, size[:, 1::2] * 2.0 ** -20
+                want = F.silu(gate) * up
+                bound = 1.13 * up.abs() * eg + F.silu(gate).abs() * eu + 1.13 * eg * eu + (gate * up).abs() * 2.0 ** -18 + want.abs() * 2.0 ** -8 + 1e-30
+                assert bool(((x.double() - want).abs() <= bound * 1.01).all()), (M, N, K, name)
+            if name == "folded norm":
+                ab, cc = kw["ln_ab"].double()[:, :1], kw["col_c"].double()
+                want = ab * ref + cc
+                bound = ab * size * 2.0 ** -20 + (want.abs() + cc.abs()) * 2.0 ** -22 + want.abs() * 2.0 ** -8
+                assert bool(((x.double() - want).abs() <= bound * 1.01).all()), (M, N, K, name)
             if name in ("plain", "bias", "residual", "fp32"):
-                ref = a.double() @ w.double().t()
-                size = a.double().abs() @ w.double().abs().t()
                 if "bias" in kw:
                     ref += b.double()
                 if "residual" in kw:
