@@ -957,14 +957,15 @@ int launch_prefill(hipStream_t st, const CogsMla& a) {
 // One query tile's keys are a chain of 2.3 us a tile for a wave that has its SIMD to itself, and the longest chain lasted 146 of the
 // 190 us of 4096 rows x 16 heads (192 + 128 columns). With two waves per tile and half the chain each it takes 99 us, and the whole 147:
 // 1800 rows 77 -> 53 us, 1000 rows 44 -> 33, 300 rows 17 -> 16. That needs workgroups that have a CU to themselves: up to one per CU, or two
-// whose chains are of all lengths (one sequence). More of them, or shorter sequences beside the longest, whose empty query tiles wait
-// for a whole CU's LDS too, are slower in halves. Whole passes of 9 layers of 16 heads, / of 6 of 32, four waves against eight: one prompt of 4000 rows
-// 4.90 / 4.82 ms (32 heads 8.54 / 8.59), 4 x 512 rows behind 2000 3.63 / 3.51 (32 heads 5.49 / 5.60), 8 x 16 behind 1000 1.54 / 1.50,
+// where one sequence's chains are longer than a CU's share of the work (as many query tiles as heads). More of them, or shorter sequences beside the longest, whose empty query tiles wait
+// for a whole CU's LDS too, are slower in halves. Whole passes of 9 layers of 16 heads, / of 6 of 32, four waves against eight: one prompt of 4096 rows
+// 4.91 / 4.79 ms (32 heads 8.76 / 8.84, 28 heads x 2048 5.75 / 5.86), 4 x 512 rows behind 2000 3.63 / 3.51 (32 heads 5.49 / 5.60), 8 x 16 behind 1000 1.54 / 1.50,
 // 32 x 16 behind 1000 2.98 / 3.15, 1 x 2048 + 3 x 64 3.94 / 4.04, + 63 x 32 5.83 / 6.63, 8 x 300 3.07 / 3.13.
 template <int KN, int KR, int DT>
 int launch_prefill_split(hipStream_t st, const CogsMla& a) {
-    const long tiles = (long)((a.max_new + 127) / 128) * a.heads * a.nseq;
-    const bool halves = tiles <= (a.nseq == 1 ? 512 : 256);
+    const int nqt = (a.max_new + 127) / 128;
+    const long tiles = (long)nqt * a.heads * a.nseq;
+    const bool halves = tiles <= 256 || (tiles <= 512 && a.nseq == 1 && nqt >= a.heads);
     g_cogs_debug.mla_last_waves = halves ? 8 : 4;
     return halves ? launch_prefill<KN, KR, DT, 2, 2>(st, a) : launch_prefill<KN, KR, DT, 2, 1>(st, a);
 }
