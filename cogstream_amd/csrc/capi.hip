@@ -91,8 +91,8 @@ const char* cogs_debug_list(void) {
 #define COGS_DBG_DOC(n, dflt, doc) #n " = " #dflt ": " doc "\n"
         COGS_DEBUG_SWITCHES(COGS_DBG_DOC)
 #undef COGS_DBG_DOC
-        "gemm_last_body (read only): body the last cogs_gemm dispatched to -- 1 128x128, 2 256x128 ring, 3 K-tile ping-pong, "
-        "4 whole-line ping-pong, 5 ping-pong + ring (split launch), 6 GEMV, 7 few-row GEMM\n"
+        "gemm_last_body (read only): body the last cogs_gemm dispatched to -- 1 128x128 (fp32), 2 mid-size (fp32: 256x128), 3 K-tile ping-pong, "
+        "4 whole-line ping-pong, 5 ping-pong + mid-size (split launch), 6 GEMV, 7 few-row GEMM\n"
         "attn_last_kernel (read only): kernel of the last cogs_attention -- 1 general MFMA, 2 ViT unpipelined, 3 ViT pipelined, "
         "4 single-token decode, 5 prompt LDS-DMA, 7 row-wise fp32, 8 ViT pipelined on head-major K/V\n"
         "attn_vit_last_end (read only): ragged end of the last pipelined ViT attention launch -- 10 x tiles behind the four-tile loop + "

@@ -24,7 +24,7 @@
     X(gemm_rope_lut, 1, "K-tile body only: rotary factors from the LDS position LUT when the caller supplies one")          \
     X(gemm_group_m, 0, "> 0: row blocks per group of the ping-pong tile walk (0: chosen per shape)")                        \
     X(gemm_mid, 0, "> 0: this tile size of the mid-size kernel for every bf16 product of two or more rows (0: chosen per shape)") \
-    X(gemm_split, 1, "0: no round-aligned / few-tile split of a launch")                                                    \
+    X(gemm_split, 1, "0: what the ping-pong kernel can take is all its (no split, no mid-size kernel for few tiles)")                                                    \
     X(gemm_co_streams, 0, "> 0: overrides the co-running-streams hint of the many-tile split")                              \
     X(gemm_epi_serial, 0, "1: the two wave groups' epilogues in separate intervals (the order before round 4)")             \
     X(gemm_nostore, 0, "1: timing only -- K loops without epilogues (results are NOT written)")                             \

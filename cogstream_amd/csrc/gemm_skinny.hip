@@ -3,7 +3,8 @@
 // HBM-bound like the single-row GEMV (gemv.hip): every weight byte is read once, straight into MFMA A fragments. A workgroup owns
 // 16 NT output columns; its NW waves take alternate 64-element slices of K (a row's slice is one whole 128-byte line), the batch rows
 // are the columns of v_mfma_f32_16x16x32_bf16 (MT groups of 16), and the waves' partial tiles are summed through LDS in a fixed
-// order. The batch rows come from L2 once per workgroup -- as many bytes as the weights with NT = 1 and M = 16 -- so columns are
+// order. (How many waves and partial sums there are depends on M as well as on N and K: a row's bits may differ between steps of
+// other numbers of rows.) The batch rows come from L2 once per workgroup -- as many bytes as the weights with NT = 1 and M = 16 -- so columns are
 // taken 64 or 32 at a time where that still makes 160 workgroups.
 //
 // A sublayer's last product has few columns and a long K: 2048 columns are 128 workgroups of 16, each a quarter of what the chip

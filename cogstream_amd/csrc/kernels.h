@@ -24,7 +24,7 @@ struct CogsGemm {
     const float* rope_sin = nullptr;
     int rope_cols = 0;
     int head_dim = 0;
-    int force_small_tile = 0;                // testing: always use the 128x128 kernel
+    int force_small_tile = 0;                // fp32: always the 128x128 kernel
     const void* rms_gamma = nullptr;         // M == 1 only: RMS-normalise A on the fly with this weight
     float rms_eps = 0.f;
     // M == 1 only: output columns [kv_col0, kv_col0 + kv_dim) go to kv_k[0..kv_dim), the next kv_dim to kv_v
@@ -51,7 +51,7 @@ struct CogsGemm {
 };
 int cogs_k_gemm(hipStream_t st, const CogsGemm& g);
 int cogs_k_gemm_mid(hipStream_t st, const CogsGemm& g, int tile);     // gemm_mid.hip; the caller (cogs_k_gemm) has checked the operands
-void cogs_k_gemm_co_streams(int streams);   // hint for the few-tile choice: streams fed with GEMMs of this size at once (thread-local)
+void cogs_k_gemm_co_streams(int streams);   // streams fed with GEMMs of this size at once (thread-local): beside another stream a product of many tiles is not split
 // (a, b) = (rstd, -rstd * mean) per row from the EPI_ROWSTAT partials [rows][tiles][2]: ab [rows][2]
 int cogs_k_ln_finalize(hipStream_t st, const float* stat_part, int rows, int tiles, int H, float eps, float* ab);
 

@@ -536,7 +536,9 @@ cogs_status cogs_decoder_workspace_bytes(cogs_handle h, int rows, int nseq, int6
  * to back), at positions kv[i]->len ..; its cache rows are appended and kv[i]->len advances. No padding, any mix of lengths.
  * want (host [n_want], row numbers) -> logits fp32 [n_want][vocab_p]. streams, nullable: fp32 [layer runs][rows][width_p], the
  * residual stream (the sum of the streams) behind every layer run. Steps of one token per sequence take the absorbed form of
- * latent attention. */
+ * latent attention. The order of sums depends on the step's shape (rows, sequences, longest context): the same call gives the same
+ * bits, the same tokens in another step the same values to rounding. The workspace size is that of this step's shape; of one
+ * sequence, from two rows on, more rows never need less. */
 cogs_status cogs_decoder_forward(cogs_handle h, cogs_stream stream, const void* embeds, cogs_kv* const* kv, const int32_t* lens, int nseq,
                                  const int32_t* want, int n_want, float* logits, float* streams, void* ws, size_t ws_bytes);
 

@@ -294,7 +294,7 @@ def test_decode_gemvs_at_production_width_vs_oracle(dev, dot2):
 def test_share_sized_clip_is_bit_identical_on_1_to_4_streams(dev):
     """cogs_vit_set_streams accepts 1-4 contiguous frame ranges; rounds 4-5 checked 3 and 4 for bit identity on a small clip
     only. Here: a rank's 1/8 share of the cfg2 clip (8 frames of 22 x 42 patches, production width, 27
-    layers, random weights) -- the size at which the few-tile GEMM choice reads the co-stream hint S = 3 / 4 and the extra
+    layers, random weights) -- the size at which a range's products go to other kernels for every stream count and the extra
     workspace of the third and fourth range is used -- must come out the same bits on 1, 2, 3 and 4 streams (and the round-6
     tall tiles with them: an N = 1152 GEMM of a range takes a different tile walk for every stream count)."""
     from cogstream_amd import _lib as L

@@ -1,6 +1,6 @@
 #!/usr/bin/env python3
 """Would a fixed split-K pay for a frame-sharded share's fc2 (N = 1152, K = 4352, 3 696 rows per stream = 70 ping-pong tiles on 256
-CUs)? Emulation with what exists: the K = 4352 GEMM as shipped (ring kernel, residual + statistics) against `split` GEMMs of K / split
+CUs)? Emulation with what exists: the K = 4352 GEMM as dispatched (residual + statistics) against `split` GEMMs of K / split
 stacked as rows of ONE launch (M x split rows, fp32 output = the partial tiles) plus a torch sum over the partials as a stand-in for
 the reduce + epilogue kernel. Alone on the GPU, HIP events, medians."""
 import os

@@ -1,7 +1,7 @@
 #!/usr/bin/env python3
 """Would splitting the N = 1152 GEMMs by COLUMNS pay? 1152 = 4 x 256 + 128: the ping-pong kernel pads the fifth
 column tile to 256 (11 % of its MFMAs). Times, with the out-proj / fc2 epilogue (bias + residual + row statistics):
-the whole GEMM, its first 1024 columns (ping-pong kernel) and its last 128 columns (256x128 ring kernel)."""
+the whole GEMM, its first 1024 columns (ping-pong kernel) and its last 128 columns (mid-size kernel)."""
 import os, sys
 import torch
 sys.path.insert(0, os.path.dirname(os.path.dirname(os.path.abspath(__file__))))
