@@ -19,16 +19,19 @@ from .runtime import get_handle
 @lru_cache(maxsize=64)
 def _tables(in_size: int, out_size: int, device: int):
     """tap tables of a resize on a device. Kept by size, not copied up on every call: four copies that wait for the device each
-    took as long as the kernel. The copies are complete when the tables enter the cache; a stream that reads them is recorded with them
-    (the caller's part), so that an entry that leaves the cache is not reused under a queued kernel."""
+    took as long as the kernel. The copies are complete when the tables enter the cache; a stream that reads them and is not the one they
+    were made on (the last value) is recorded with them by the caller, so that an entry that leaves the cache is not reused under a queued
+    kernel."""
     b, k, ks = resample_coeffs(in_size, out_size)
     dev = torch.device("cuda", device)
-    return torch.from_numpy(np.ascontiguousarray(b)).to(dev), torch.from_numpy(np.ascontiguousarray(k)).to(dev), ks
+    return (torch.from_numpy(np.ascontiguousarray(b)).to(dev), torch.from_numpy(np.ascontiguousarray(k)).to(dev), ks,
+            torch.cuda.current_stream(dev).cuda_stream)
 
 
 @lru_cache(maxsize=64)
 def _value_table(device: int):
-    return torch.from_numpy(pixel_value_table()).to(torch.device("cuda", device))
+    dev = torch.device("cuda", device)
+    return torch.from_numpy(pixel_value_table()).to(dev), torch.cuda.current_stream(dev).cuda_stream
 
 
 def preprocess_media_gpu(items: Sequence[torch.Tensor], merge_sizes: Sequence[int], min_tokens: int = 16,
@@ -44,23 +47,29 @@ def preprocess_media_gpu(items: Sequence[torch.Tensor], merge_sizes: Sequence[in
     targets = media_target_sizes(shapes, list(merge_sizes), min_tokens, max_tokens)
     handle = get_handle(dev)
     index = dev.index if dev.index is not None else torch.cuda.current_device()
-    table = _value_table(index)
-    stream = torch.cuda.current_stream(dev)
-    table.record_stream(stream)
+    stream = L.current_stream()
+
+    def read_here(made_on, *tables):
+        if made_on != stream:
+            for t in tables:
+                t.record_stream(torch.cuda.current_stream())
+
+    table, made_on = _value_table(index)
+    read_here(made_on, table)
     outs, grids = [], []
     for v, merge_size, (th, tw) in zip(items, merge_sizes, targets):
         assert v.dtype == torch.uint8 and v.is_contiguous() and v.shape[-1] == 3
         t, H, W = int(v.shape[0]), int(v.shape[1]), int(v.shape[2])
-        dbx, dkx, ksx = _tables(W, tw, index)
-        dby, dky, ksy = _tables(H, th, index)
-        for taps in (dbx, dkx, dby, dky):
-            taps.record_stream(stream)
+        dbx, dkx, ksx, made_on = _tables(W, tw, index)
+        read_here(made_on, dbx, dkx)
+        dby, dky, ksy, made_on = _tables(H, th, index)
+        read_here(made_on, dby, dky)
         gh, gw = th // PATCH, tw // PATCH
         out = torch.empty(t * gh * gw, 3 * PATCH * PATCH, device=dev, dtype=out_dtype)
         n = C.c_size_t()
         L.check(L.lib.cogs_preprocess_workspace_bytes(t, H, tw, C.byref(n)))
         ws = handle.workspace("preprocess", n.value)
-        L.check(L.lib.cogs_preprocess_frames(L.current_stream(), v.data_ptr(), t, H, W, th, tw, int(merge_size),
+        L.check(L.lib.cogs_preprocess_frames(stream, v.data_ptr(), t, H, W, th, tw, int(merge_size),
                                              dbx.data_ptr(), dkx.data_ptr(), ksx, dby.data_ptr(), dky.data_ptr(), ksy,
                                              table.data_ptr(), out.data_ptr(), L.dtype_code(out_dtype), ws.data_ptr(), ws.numel()),
                 "cogs_preprocess_frames")

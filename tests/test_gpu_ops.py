@@ -1155,7 +1155,7 @@ def test_tap_tables_outlive_their_place_in_the_cache(dev):
     with torch.cuda.stream(side):
         torch.cuda._sleep(200_000_000)
         got = pg.preprocess_videos_gpu([frames])["pixel_values"]
-    tables = [(t.data_ptr(), t.numel() * 4) for key in ((400, 392), (300, 308)) for t in pg._tables(*key, 0)[:2]] + [(pg._value_table(0).data_ptr(), 3072)]
+    tables = [(t.data_ptr(), t.numel() * 4) for key in ((400, 392), (300, 308)) for t in pg._tables(*key, 0)[:2]] + [(pg._value_table(0)[0].data_ptr(), 3072)]
     pg._tables.cache_clear()
     pg._value_table.cache_clear()
     reused = [torch.zeros(1 << 14, device=dev, dtype=torch.int32) for _ in range(64)]      # more than the small blocks' segments hold
