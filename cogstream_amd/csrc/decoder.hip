@@ -137,7 +137,7 @@ struct Step {
         PROF(COGS_PROF_GEMM);
         g.dtype = d.w.dtype;
         if (g_cogs_debug.gemm_skinny != 0 && cogs_k_gemm_skinny_fits(g)) return cogs_k_gemm_skinny(st, g);
-        if (g.K < 128) g.force_small_tile = 1;      // (fp32: the ring of three slabs wants more than that)
+        if (g.K < 128) g.force_small_tile = 1;      // (fp32: products that short stay off the three-slab ring)
         return cogs_k_gemm(st, g);
     }
 
