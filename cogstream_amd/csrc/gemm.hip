@@ -1098,15 +1098,15 @@ void dispatch_f32(hipStream_t st, const GemmArgs& p, int grid, int mask, bool bi
 
 // ---- which kernel a bf16 product of two or more rows gets -------------------------------------------------------------------
 // All of them walk K in the same order, so the choice is by time alone. Time of a launch = rounds of tiles over the chip x (slabs x
-// time of a slab + the rest of a tile: prologue, epilogue), with a slab's time measured per tile size for one and, where the LDS
-// has room for them, two workgroups on a CU (MI355X, weights from HBM, K = 1152 .. 18 944; the sums below are within 15 % of every
-// shape that was measured). The small tiles are bound by a slab's LDS traffic and barrier, not by MFMAs: they pay while the
-// larger ones leave CUs without a tile.
+// time of a slab + the rest of a tile: prologue, epilogue), with a slab's time per tile size for one and, where the LDS has room for
+// them, two workgroups on a CU. The figures are a fit to launches of every tile at M = 48 .. 2048 and eleven weight shapes from 1152 x
+// 1152 to 37 888 x 3584 and 3584 x 18 944 (MI355X, weights from HBM); the tile they choose was the fastest or within 6 % of it at
+// each. They are those of a chip that is not full: three rounds of 128x256 take 0.95 us a slab, which no choice here depends on.
 struct TileCost { int tile, tm, tn; float one, two, rest; };     // us; two = 0: one workgroup per CU
 static constexpr TileCost MID_TILES[] = {
-    {1, 32, 64, 0.22f, 0.36f, 2.5f}, {2, 64, 64, 0.26f, 0.48f, 2.5f}, {3, 128, 64, 0.38f, 0.71f, 2.5f},
-    {4, 128, 128, 0.55f, 0.f, 3.f},  {5, 128, 256, 0.85f, 0.f, 4.f}};
-static constexpr float PP_SLAB = 1.13f, PP_REST = 8.f, SECOND_LAUNCH = 2.f;
+    {1, 32, 64, 0.165f, 0.f, 1.8f},   {2, 64, 64, 0.218f, 0.409f, 1.8f}, {3, 128, 64, 0.309f, 0.637f, 2.3f}, {4, 128, 128, 0.387f, 0.f, 3.6f},
+    {5, 128, 256, 0.629f, 0.f, 4.8f}, {6, 128, 64, 0.292f, 0.f, 2.9f},   {7, 160, 64, 0.332f, 0.f, 3.8f}};
+static constexpr float PP_SLAB = 1.14f, PP_REST = 6.f, SECOND_LAUNCH = 2.f;
 
 static float tile_time(int tiles, int slabs, float one, float two, float rest) {
     const float t1 = slabs * one + rest, t2 = slabs * two + rest;
@@ -1114,9 +1114,10 @@ static float tile_time(int tiles, int slabs, float one, float two, float rest) {
     const int full = tiles / (2 * PERSISTENT_WGS), left = tiles % (2 * PERSISTENT_WGS);
     return full * t2 + (left == 0 ? 0.f : left <= PERSISTENT_WGS ? t1 : t2);
 }
-static int best_mid_tile(int M, int N, int K, float* time) {
+static int best_mid_tile(int M, int N, int K, bool ln_fold, float* time) {
     int best = 0;
     for (const TileCost& t : MID_TILES) {
+        if (t.tile == 7 && ln_fold) continue;       // (its waves have more rows than lanes to hold their factors)
         const float c = tile_time((M + t.tm - 1) / t.tm * ((N + t.tn - 1) / t.tn), K / 64, t.one, t.two, t.rest);
         if (best == 0 || c < *time) { best = t.tile; *time = c; }
     }
@@ -1126,10 +1127,10 @@ static int best_mid_tile(int M, int N, int K, float* time) {
 static int finish_ln(hipStream_t st, const CogsGemm& g) {
     return g.ln_part ? cogs_k_ln_finalize(st, g.ln_part, g.M, g.K / 64, g.K, g.ln_eps, const_cast<float*>(g.ln_ab)) : COGS_OK;
 }
-static int launch_mid(hipStream_t st, const CogsGemm& g, int tile) {
+static int launch_mid(hipStream_t st, const CogsGemm& g, int tile, bool alone) {
     ++g_gemm_launches;
     g_cogs_debug.gemm_last_body = 2;
-    return cogs_k_gemm_mid(st, g, tile);
+    return cogs_k_gemm_mid(st, g, tile, alone);
 }
 
 int cogs_k_gemm(hipStream_t st, const CogsGemm& g) {
@@ -1149,12 +1150,12 @@ int cogs_k_gemm(hipStream_t st, const CogsGemm& g) {
     const int S = env_co > 0 ? env_co : g_co_streams;
     float mid_time = 0.f;
     const int env_mid = (int)g_cogs_debug.gemm_mid;
-    const int mid = g.dtype != COGS_DT_BF16 ? 0 : env_mid > 0 ? env_mid : best_mid_tile(g.M, g.N, g.K, &mid_time);
+    const int mid = g.dtype != COGS_DT_BF16 ? 0 : env_mid > 0 ? env_mid : best_mid_tile(g.M, g.N, g.K, g.ln_ab != nullptr, &mid_time);
     const int n_pad = (g.N + BN3 - 1) / BN3 * BN3;
     const bool pp_fits = n_pad * 100 <= g.N * (int)g_cogs_debug.gemm_pad_pct;   // default: <= 12 % of the MFMAs spent on N padding
     // (the ping-pong kernel wants two slabs and, below a row block, wastes its tiles' rows)
     const bool pp = mid > 0 && env_mid == 0 && g_cogs_debug.gemm_pingpong != 0 && pp_fits && g.K >= 128 && g.M >= 256;
-    if (mid > 0 && !pp) return launch_mid(st, g, mid);
+    if (mid > 0 && !pp) return launch_mid(st, g, mid, S == 1);
     GemmArgs p;
     p.trace = nullptr; p.rope_lut = nullptr; p.rope_lut_bytes = 0; p.group_m = GROUP_M;
     p.epi_serial = (int)g_cogs_debug.gemm_epi_serial;
@@ -1227,7 +1228,7 @@ int cogs_k_gemm(hipStream_t st, const CogsGemm& g) {
                 const int rows_rem = g.M - mb * BM3;
                 if (mb > 0 && rows_rem > 0) {
                     float rest;
-                    best_mid_tile(rows_rem, g.N, g.K, &rest);
+                    best_mid_tile(rows_rem, g.N, g.K, g.ln_ab != nullptr, &rest);
                     if (slabs * PP_SLAB + PP_REST + rest + SECOND_LAUNCH < best) mb_main = mb;
                 }
             }
@@ -1266,7 +1267,7 @@ int cogs_k_gemm(hipStream_t st, const CogsGemm& g) {
             }
             // (straight to the kernel: a remainder may be one row, which cogs_k_gemm would take for a single-row product)
             float rest = 0.f;
-            const int rc3 = launch_mid(st, b, mb_main > 0 ? best_mid_tile(b.M, b.N, b.K, &rest) : mid);
+            const int rc3 = launch_mid(st, b, mb_main > 0 ? best_mid_tile(b.M, b.N, b.K, g.ln_ab != nullptr, &rest) : mid, S == 1);
             if (mb_main > 0) g_cogs_debug.gemm_last_body = 5;
             return rc3;
         }

@@ -250,23 +250,23 @@ __device__ __forceinline__ void epilogue_tile(const EpiArgs& p, int mb, int nb, 
             for (int ni = 0; ni < NI; ++ni) bias_v[ni] = ld4_f<T>(reinterpret_cast<const T*>(p.bias) + nn[ni]);
         }
 #pragma unroll
-        for (int half = 0; half < MI / 2; ++half) {
+        for (int half = 0; half < (MI + 1) / 2; ++half) {
             raw_t res_raw[2][NI];
             u32x4 res_wide[2][NI / 2];
             f32x2 cs[2][NI], sn[2][NI];
             int mm[2];
             float rs2[2];
 #pragma unroll
-            for (int i = 0; i < 2; ++i) mm[i] = min(mrow + (2 * half + i) * 16, M - 1);
+            for (int i = 0; i < 2 && 2 * half + i < MI; ++i) mm[i] = min(mrow + (2 * half + i) * 16, M - 1);
             if constexpr ((EPI & EPI_LNFOLD) != 0) {
 #pragma unroll
-                for (int i = 0; i < 2; ++i) rs2[i] = row_scale ? row_scale[2 * half + i] : p.ln_ab[2 * (long)mm[i]];
+                for (int i = 0; i < 2 && 2 * half + i < MI; ++i) rs2[i] = row_scale ? row_scale[2 * half + i] : p.ln_ab[2 * (long)mm[i]];
             }
             if constexpr ((EPI & EPI_RES) != 0) {
                 if (wide) {
                     if constexpr (CAN_WIDE) {
 #pragma unroll
-                        for (int i = 0; i < 2; ++i)
+                        for (int i = 0; i < 2 && 2 * half + i < MI; ++i)
 #pragma unroll
                             for (int pr = 0; pr < NI / 2; ++pr)
                                 res_wide[i][pr] = early ? early->res[2 * half + i][pr] : *reinterpret_cast<const u32x4*>(
@@ -274,7 +274,7 @@ __device__ __forceinline__ void epilogue_tile(const EpiArgs& p, int mb, int nb, 
                     }
                 } else {
 #pragma unroll
-                    for (int i = 0; i < 2; ++i)
+                    for (int i = 0; i < 2 && 2 * half + i < MI; ++i)
 #pragma unroll
                         for (int ni = 0; ni < NI; ++ni)
                             res_raw[i][ni] = *reinterpret_cast<const raw_t*>(reinterpret_cast<const T*>(p.R) + (long)mm[i] * p.ldr + nn[ni]);
@@ -282,7 +282,7 @@ __device__ __forceinline__ void epilogue_tile(const EpiArgs& p, int mb, int nb, 
             }
             if constexpr ((EPI & EPI_ROPE) != 0) {
 #pragma unroll
-                for (int i = 0; i < 2; ++i)
+                for (int i = 0; i < 2 && 2 * half + i < MI; ++i)
 #pragma unroll
                     for (int ni = 0; ni < NI; ++ni) {
                         if (early) { cs[i][ni] = early->cs[2 * half + i][ni]; sn[i][ni] = early->sn[2 * half + i][ni]; }
@@ -290,7 +290,7 @@ __device__ __forceinline__ void epilogue_tile(const EpiArgs& p, int mb, int nb, 
                     }
             }
 #pragma unroll
-            for (int i = 0; i < 2; ++i) {
+            for (int i = 0; i < 2 && 2 * half + i < MI; ++i) {
                 const int mi = 2 * half + i;
                 const int m = mrow + mi * 16;
                 f32x4 v[NI];

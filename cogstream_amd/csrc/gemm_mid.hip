@@ -1,17 +1,23 @@
 // Mid-size GEMM (bf16):  C[M,N] = epilogue( A[M,K] . W[N,K]^T ), same sums in the same order as the kernels of gemm.hip.
 //
 // For products whose 256-wide tiles would leave most of the chip idle. One tile per workgroup, tiles from 32x64 to 128x256; the
-// K slabs (64 elements: one whole 128-byte line a row) go by LDS-DMA into a ring of S slots, S - 1 of them in flight ahead of the
-// slab being multiplied, one barrier and one counted vmcnt per slab. A slab's second half is read while the first half is multiplied,
-// the next slab's first half while the second is, so that LDS latency hides behind the wave's own matrix instructions; the small
-// tiles leave room for two workgroups per CU, which hide each other's barriers.
+// K slabs (64 elements: one whole 128-byte line a row; KS of them at a time) go by LDS-DMA into a ring of S slots, S - 1 of them in
+// flight ahead of the slabs being multiplied, one barrier and one counted vmcnt per KS slabs. While a slab is multiplied, the next
+// one's fragments are read and its slot is filled again.
 //
-// What bounds it: a CU takes in about 60 bytes a nanosecond of operand lines that miss its XCD's L2, whatever the tile, the ring
-// depth or the row stride (16 KiB slab 0.26 us, 32 KiB 0.53, 48 KiB 0.82), so a launch costs rounds x (TM + TN) x K x 2 / 60 ns and a
-// few us around it: the choice of a tile (gemm.hip) trades bytes per CU against CUs that have none. Products split over K would
-// need fewer bytes, and give other bits. Measured against the 128x128 / 256x128 tiles that were here before, one slab ahead or with
-// 256 rows per workgroup (weights from HBM): 256 x 1152 x 4352 80 -> 18 us, 256 x 3456 x 1152 24 -> 8.3, 1024 x 1152 x 4352 64 -> 31,
-// 621 x 3584 x 18944 250 -> 157, 160 x 3584 x 18944 306 -> 75, 400 x 2048 x 8192 127 -> 30, 4096 x 2048 x 5632 105 -> 83.
+// What bounds it, and what each part is there for (us per launch, weights from HBM, 27 of them in turn; before -> after):
+//   * A CU has about 60 KB of missing lines under way whatever the ring's depth, so weights that come from HBM arrive at 55 to 60 B/ns
+//     a CU, and at 105 to 115 B/ns from its XCD's L2. Where CUs are left over, workgroups behind the tiles' (prefetch_weights) ask
+//     for one dword of every weight line of their XCD's tiles, far ahead of the ring, on CUs whose own misses are free:
+//     256 x 1152 x 4352 13.6 -> 11.9, 1024 x 1152 x 4352 27.2 -> 23.8, 621 x 3584 x 18944 157 -> 137. (The tiles' own workgroups asking
+//     ahead gained a third of that: the same lines under way. A's lines asked for as well: no better, and worse for M = 1024.)
+//   * A slab of a small tile is multiplied faster than a barrier and the LDS round trip: two slabs per barrier where LDS is there for it
+//     (32x64: 13.6 -> 11.9 with the weights in L2; 128x64: 24.9 -> 23.8).
+//   * A wave issues in order, so fragment reads and DMA in front of the matrix instructions leave the matrix pipe idle meanwhile: they
+//     stand between them, one behind each (621 x 3584 x 18944 at 160x64: 121 -> 109; 4096 x 2048 x 5632 at 128x256: 87.5 -> 84.2).
+//     128x64 with two workgroups a CU has sixteen waves to fill the gaps, and is the slower for it (24.7 -> 26.1): not there.
+//   * 32x64 is four waves of 16x32 (two of 32x32: 13.7 instead of 11.9): every SIMD has one.
+// Products split over K would need fewer bytes per CU, and give other bits.
 //
 // K is walked in order by one accumulator per output: a row's bits do not depend on which tile size, or which kernel of gemm.hip,
 // computed it (frame ranges, prompts behind a kept prefix and whole prompts are compared bit for bit).
@@ -26,12 +32,12 @@ struct MidArgs {
     const char* A; long lda;   // bytes per row
     const char* W; long ldw;
     int M, N, KT;              // KT: 64-wide K slabs
-    int nbm, nbn;
+    int nbm, nbn;              // tiles; workgroups past them are prefetch_weights
     const float* ln_part; int ln_tiles; float ln_inv_h, ln_eps;     // EPI_LNFOLD: row statistics still in partial sums (or null)
     EpiArgs epi;
 };
 
-constexpr int ROW_BYTES = 128;
+constexpr int ROW_BYTES = 128, MID_CUS = 256;
 
 __device__ __forceinline__ void glds16(const char* g, char* l) {
     __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)g,
@@ -51,17 +57,42 @@ __device__ __forceinline__ void wait_slabs(int n) {
     else asm volatile("s_waitcnt vmcnt(%0)" ::"n"(MAX >= 6 ? 6 * P : 0) : "memory");
 }
 
-// WM x WN waves of 16 MI x 16 NI outputs, S ring slots
-template <int EPI, int MI, int NI, int WM, int WN, int S, int WPE>
+// workgroups (a multiple of 8: as many on each XCD) behind those of the tiles: one dword of every weight line that the tiles of this
+// XCD read, slabs in order, so that the tiles' DMA finds them in L2. Nothing waits for them and nothing is kept.
+__device__ __forceinline__ void prefetch_weights(const MidArgs& p, char* smem, int tm_group, int TN, int waves, int wid, int lane) {
+    const int nb = p.nbm * p.nbn, xcd = blockIdx.x & 7, q = nb >> 3, r = nb & 7;
+    const int x0 = xcd < r ? xcd * (q + 1) : r * (q + 1) + (xcd - r) * q, x1 = x0 + q + (xcd < r);
+    const int of = ((int)gridDim.x - nb) >> 3, me = ((int)blockIdx.x - nb) >> 3;
+    const int per_group = tm_group * p.nbn;
+    for (int k = me * waves + wid; k < p.KT; k += of * waves) {
+        for (int t = x0; t < x1;) {                              // columns of each group of row tiles (usually one)
+            const int g0 = t / per_group * per_group, gsz = min(p.nbm - g0 / p.nbn, tm_group), e = min(x1, g0 + gsz * p.nbn);
+            const int lo = (t - g0) / gsz * TN, hi = min(((e - 1 - g0) / gsz + 1) * TN, p.N);
+            for (int n = lo; n < hi; n += 64)
+                __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(p.W + (long)min(n + lane, hi - 1) * p.ldw + (long)k * ROW_BYTES),
+                                                 (__attribute__((address_space(3))) void*)smem, 4, 0, 0);
+            t = e;
+        }
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+}
+
+// WM x WN waves of 16 MI x 16 NI outputs, S ring slots of KS slabs; IL: reads and DMA between the matrix instructions
+template <int EPI, int MI, int NI, int WM, int WN, int S, int WPE, int KS, bool IL>
 __global__ __launch_bounds__(64 * WM * WN, WPE) void gemm_mid_kernel(MidArgs p) {
     extern __shared__ __attribute__((aligned(16))) char smem[];
-    constexpr int TM = 16 * MI * WM, TN = 16 * NI * WN, WAVES = WM * WN;
-    constexpr int SLAB = (TM + TN) * ROW_BYTES, P = SLAB / 1024 / WAVES;
-    static_assert(SLAB % (1024 * WAVES) == 0, "every wave stages the same number of pieces");
+    constexpr int TM = 16 * MI * WM, TN = 16 * NI * WN, WAVES = WM * WN, GROUP = 8;
+    constexpr int SUB = (TM + TN) * ROW_BYTES, SLAB = SUB * KS, P1 = SUB / 1024 / WAVES, P = P1 * KS;      // P: a wave's pieces per slot
+    static_assert(SUB % (1024 * WAVES) == 0, "every wave stages the same number of pieces");
     const int lane = threadIdx.x & 63;
     const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int wm = wid / WN, wn = wid % WN;
-    const int KT = p.KT;
+    if ((int)blockIdx.x >= p.nbm * p.nbn) {
+        prefetch_weights(p, smem, GROUP, TN, WAVES, wid, lane);
+        return;
+    }
+    const int KT = (p.KT + KS - 1) / KS;                         // slots' worth
+    const bool odd = KS == 2 && (p.KT & 1);                      // the last one holds one slab
 
     // block -> tile: XCD-aware, then groups of 8 row tiles with the rows running fastest, so that the row tiles that share a
     // panel of weights run on one XCD
@@ -69,26 +100,34 @@ __global__ __launch_bounds__(64 * WM * WN, WPE) void gemm_mid_kernel(MidArgs p) 
     {
         const int nb = p.nbm * p.nbn, xcd = blockIdx.x & 7, q = nb >> 3, r = nb & 7;
         const int bid = (xcd < r ? xcd * (q + 1) : r * (q + 1) + (xcd - r) * q) + (blockIdx.x >> 3);
-        const int per_group = 8 * p.nbn, first_m = bid / per_group * 8, gsz = min(p.nbm - first_m, 8);
+        const int per_group = GROUP * p.nbn, first_m = bid / per_group * GROUP, gsz = min(p.nbm - first_m, GROUP);
         m0 = (first_m + (bid % per_group) % gsz) * TM;
         n0 = ((bid % per_group) / gsz) * TN;
     }
     // piece pc of a slab: tile rows 8 pc .. +7 (A's rows, then W's); lane -> row + (lane >> 3), 16-byte chunk lane & 7, swizzled
-    const char* src[P];
+    const char* src[P1];
 #pragma unroll
-    for (int i = 0; i < P; ++i) {
-        const int r = (wid * P + i) * 8 + (lane >> 3);
+    for (int i = 0; i < P1; ++i) {
+        const int r = (wid * P1 + i) * 8 + (lane >> 3);
         const int c = (lane & 7) ^ (r & 7);
         src[i] = r < TM ? p.A + (long)min(m0 + r, p.M - 1) * p.lda + c * 16 : p.W + (long)min(n0 + r - TM, p.N - 1) * p.ldw + c * 16;
     }
-    char* const lds_wave = smem + wid * P * 1024;
-    auto stage = [&](int slot) {                 // the next slab of the stream
-        char* dst = lds_wave + slot * SLAB;
+    char* const lds_wave = smem + wid * P1 * 1024;
+    auto stage_piece = [&](int slot, int i, int u, int step) {
+        glds16(src[i] + u * step, lds_wave + slot * SLAB + u * SUB + i * 1024);
+    };
+    auto advance = [&]() {
 #pragma unroll
-        for (int i = 0; i < P; ++i) {
-            glds16(src[i], dst + i * 1024);
-            src[i] += ROW_BYTES;
-        }
+        for (int i = 0; i < P1; ++i) src[i] += ROW_BYTES * KS;
+    };
+    // the next KS slabs of the stream; alone: K ends behind the first (which then stands in for the second, not multiplied)
+    auto stage = [&](int slot, bool alone) {
+        const int step = KS == 2 && alone ? 0 : ROW_BYTES;
+#pragma unroll
+        for (int u = 0; u < KS; ++u)
+#pragma unroll
+            for (int i = 0; i < P1; ++i) stage_piece(slot, i, u, step);
+        advance();
     };
     int foff[2];
 #pragma unroll
@@ -100,34 +139,36 @@ __global__ __launch_bounds__(64 * WM * WN, WPE) void gemm_mid_kernel(MidArgs p) 
     for (int i = 0; i < MI; ++i)
 #pragma unroll
         for (int j = 0; j < NI; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-    struct Frags { u32x4 a[2][MI], w[2][NI]; } f0, f1;       // the halves of a slab
+    struct Frags { u32x4 a[2 * KS][MI], w[2 * KS][NI]; } f0, f1;       // half slabs
+    auto load_frag = [&](Frags& f, int slot, int s, int i) {           // half slab s: its NI weight fragments, then its MI others
+        const char* r = smem + slot * SLAB + (s >> 1) * SUB + foff[s & 1];
+        if (i < NI) f.w[s][i] = *reinterpret_cast<const u32x4*>(r + w_off + i * 16 * ROW_BYTES);
+        else f.a[s][i - NI] = *reinterpret_cast<const u32x4*>(r + a_off + (i - NI) * 16 * ROW_BYTES);
+    };
     auto load_frags = [&](Frags& f, int slot) {
 #pragma unroll
-        for (int s = 0; s < 2; ++s) {
-            const char* As = smem + slot * SLAB + a_off + foff[s];
-            const char* Ws = smem + slot * SLAB + w_off + foff[s];
+        for (int s = 0; s < 2 * KS; ++s)
 #pragma unroll
-            for (int i = 0; i < MI; ++i) f.a[s][i] = *reinterpret_cast<const u32x4*>(As + i * 16 * ROW_BYTES);
-#pragma unroll
-            for (int i = 0; i < NI; ++i) f.w[s][i] = *reinterpret_cast<const u32x4*>(Ws + i * 16 * ROW_BYTES);
-        }
+            for (int i = 0; i < MI + NI; ++i) load_frag(f, slot, s, i);
     };
-    auto mma = [&](Frags& f) {
+    auto mma1 = [&](Frags& f, int s, int mi, int ni) {
+        acc[mi][ni] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, f.w[s][ni]), __builtin_bit_cast(bf16x8, f.a[s][mi]),
+                                                              acc[mi][ni], 0, 0, 0);
+    };
+    auto mma = [&](Frags& f, int s0, int s1) {
         __builtin_amdgcn_s_setprio(1);
 #pragma unroll
-        for (int s = 0; s < 2; ++s)
+        for (int s = s0; s < s1; ++s)
 #pragma unroll
             for (int mi = 0; mi < MI; ++mi)
 #pragma unroll
-                for (int ni = 0; ni < NI; ++ni)
-                    acc[mi][ni] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, f.w[s][ni]),
-                                                                          __builtin_bit_cast(bf16x8, f.a[s][mi]), acc[mi][ni], 0, 0, 0);
+                for (int ni = 0; ni < NI; ++ni) mma1(f, s, mi, ni);
         __builtin_amdgcn_s_setprio(0);
     };
     // the wait for the fragments stands here, in front of newer LDS reads
     auto touch = [&](Frags& f) {
 #pragma unroll
-        for (int s = 0; s < 2; ++s) {
+        for (int s = 0; s < 2 * KS; ++s) {
 #pragma unroll
             for (int i = 0; i < MI; ++i) asm volatile("" : "+v"(f.a[s][i]));
 #pragma unroll
@@ -142,10 +183,11 @@ __global__ __launch_bounds__(64 * WM * WN, WPE) void gemm_mid_kernel(MidArgs p) 
     constexpr bool EARLY = NI == 2 && (EPI & EPI_GENERIC) == 0;
     EpiOperands<bf16_t, EPI, MI, NI> early;
     if constexpr (EARLY) early.load(p.epi, mb, nb, p.M, p.N, lane);
-    for (int i = 0; i < S && i < KT; ++i) stage(i);
+    for (int i = 0; i < S && i < KT; ++i) stage(i, odd && i == KT - 1);
     // EPI_LNFOLD: the factors of this wave's rows while the ring fills; lane l has row l of its 16 MI
     float factor = 0.f;
     if constexpr ((EPI & EPI_LNFOLD) != 0) {
+        static_assert(MI <= 4 && (MI & (MI - 1)) == 0, "a lane has one of the wave's rows");
         const long r = min(m0 + wm * 16 * MI + (lane & (16 * MI - 1)), p.M - 1);
         factor = p.ln_part ? ln_row_factors(reinterpret_cast<const f32x2*>(p.ln_part) + r * p.ln_tiles, p.ln_tiles, p.ln_inv_h, p.ln_eps)[0]
                            : p.epi.ln_ab[2 * r];
@@ -155,20 +197,38 @@ __global__ __launch_bounds__(64 * WM * WN, WPE) void gemm_mid_kernel(MidArgs p) 
     asm volatile("" ::: "memory");
     load_frags(f0, 0);
     int slot = 0, kt = 0;
-    // slab kt is in the fragments `cur`: once every wave has it there, its slot takes slab kt + S, and slab kt + 1 is read into the
+    // slot kt is in the fragments `cur`: once every wave has it there, its place takes slot kt + S, and slot kt + 1 is read into the
     // other set while this one is multiplied
     auto steady = [&](Frags& cur, Frags& nxt) {
         const int next = slot == S - 1 ? 0 : slot + 1;
         touch(cur);
-        asm volatile("s_waitcnt vmcnt(%0)" ::"n"((S - 2) * P) : "memory");       // slab kt + 1 has landed
+        asm volatile("s_waitcnt vmcnt(%0)" ::"n"((S - 2) * P) : "memory");       // slot kt + 1 has landed
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
-        stage(slot);
-        load_frags(nxt, next);
-        mma(cur);
+        if constexpr (!IL) {
+            stage(slot, false);
+            load_frags(nxt, next);
+            mma(cur, 0, 2 * KS);
+        } else {
+            constexpr int READS = 2 * KS * (MI + NI), OPS = READS + P, MMAS = 2 * KS * MI * NI;
+            __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+            for (int m = 0; m < MMAS; ++m) {
+                mma1(cur, m / (MI * NI), m / NI % MI, m % NI);
+#pragma unroll
+                for (int o = 0; o < OPS; ++o) {                  // one behind each; what is left behind the last
+                    if (o < m || (o > m && m < MMAS - 1)) continue;
+                    if (o < READS) load_frag(nxt, next, o / (MI + NI), o % (MI + NI));
+                    else stage_piece(slot, (o - READS) % P1, (o - READS) / P1, ROW_BYTES);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            __builtin_amdgcn_s_setprio(0);
+            advance();
+        }
         slot = next;
     };
-    for (; kt + 1 + S < KT; kt += 2) {
+    for (; kt + S + KS < KT; kt += 2) {
         steady(f0, f1);
         steady(f1, f0);
     }
@@ -179,10 +239,11 @@ __global__ __launch_bounds__(64 * WM * WN, WPE) void gemm_mid_kernel(MidArgs p) 
             wait_slabs<P, S - 1>(min(S - 2, KT - kt - 2));
             __builtin_amdgcn_s_barrier();
             asm volatile("" ::: "memory");
-            if (kt + S < KT) stage(slot);
             load_frags(nxt, next);
+            if (kt + S < KT) stage(slot, odd && kt + S == KT - 1);
         }
-        mma(cur);
+        mma(cur, 0, 2);
+        if (KS == 2 && !(odd && kt == KT - 1)) mma(cur, 2, 2 * KS);
         slot = next;
         ++kt;
     };
@@ -227,30 +288,39 @@ __global__ __launch_bounds__(64 * WM * WN, WPE) void gemm_mid_kernel(MidArgs p) 
     }
 }
 
-template <int EPI, int MI, int NI, int WM, int WN, int S, int WPE>
-void launch(hipStream_t st, MidArgs& p) {
-    constexpr int TM = 16 * MI * WM, TN = 16 * NI * WN, lds = S * (TM + TN) * ROW_BYTES;
+template <int EPI, int MI, int NI, int WM, int WN, int S, int WPE, int KS, bool IL>
+void launch(hipStream_t st, MidArgs& p, bool alone) {
+    constexpr int TM = 16 * MI * WM, TN = 16 * NI * WN, lds = S * KS * (TM + TN) * ROW_BYTES;
+    static_assert(lds <= 160 * 1024, "");
     static std::atomic<uint64_t> attr_done{0};
-    cogs_ensure_dyn_lds((const void*)gemm_mid_kernel<EPI, MI, NI, WM, WN, S, WPE>, lds, attr_done);
+    cogs_ensure_dyn_lds((const void*)gemm_mid_kernel<EPI, MI, NI, WM, WN, S, WPE, KS, IL>, lds, attr_done);
     p.nbm = (p.M + TM - 1) / TM;
     p.nbn = (p.N + TN - 1) / TN;
-    hipLaunchKernelGGL((gemm_mid_kernel<EPI, MI, NI, WM, WN, S, WPE>), dim3(p.nbm * p.nbn), dim3(64 * WM * WN), lds, st, p);
+    // CUs without a tile: up to four workgroups an XCD prefetch (32 or 112 in all made no difference)
+    const int tiles = p.nbm * p.nbn, left = alone ? (MID_CUS - tiles) / 8 * 8 : 0;
+    const int extra = left < 0 ? 0 : left > 32 ? 32 : left;
+    hipLaunchKernelGGL((gemm_mid_kernel<EPI, MI, NI, WM, WN, S, WPE, KS, IL>), dim3(tiles + extra), dim3(64 * WM * WN), lds, st, p);
 }
 
 template <int EPI>
-void dispatch_tile(hipStream_t st, MidArgs& p, int tile) {
+void dispatch_tile(hipStream_t st, MidArgs& p, int tile, bool alone) {
     switch (tile) {
-        case 1: launch<EPI, 2, 2, 1, 2, 6, 1>(st, p); break;          // 32 x 64
-        case 2: launch<EPI, 2, 2, 2, 2, 5, 2>(st, p); break;          // 64 x 64
-        case 3: launch<EPI, 2, 2, 4, 2, 3, 4>(st, p); break;          // 128 x 64
-        case 4: launch<EPI, 4, 2, 2, 4, 5, 2>(st, p); break;          // 128 x 128
-        default: launch<EPI, 4, 4, 2, 4, 3, 2>(st, p); break;         // 128 x 256
+        case 1: launch<EPI, 1, 2, 2, 2, 4, 2, 2, true>(st, p, alone); break;          // 32 x 64
+        case 2: launch<EPI, 2, 2, 2, 2, 4, 2, 1, true>(st, p, alone); break;          // 64 x 64, two a CU
+        case 3: launch<EPI, 2, 2, 4, 2, 3, 4, 1, false>(st, p, alone); break;         // 128 x 64, two a CU
+        case 4: launch<EPI, 4, 2, 2, 4, 4, 2, 1, true>(st, p, alone); break;          // 128 x 128
+        case 5: launch<EPI, 4, 4, 2, 4, 3, 2, 1, true>(st, p, alone); break;          // 128 x 256
+        case 6: launch<EPI, 2, 2, 4, 2, 3, 2, 2, true>(st, p, alone); break;          // 128 x 64, two slabs at a time
+        default:
+            if constexpr ((EPI & EPI_LNFOLD) == 0) launch<EPI, 5, 2, 2, 2, 5, 2, 1, true>(st, p, alone);          // 160 x 64
+            else launch<EPI, 2, 2, 4, 2, 3, 4, 1, false>(st, p, alone);
+            break;
     }
 }
 
 }  // namespace
 
-int cogs_k_gemm_mid(hipStream_t st, const CogsGemm& g, int tile) {
+int cogs_k_gemm_mid(hipStream_t st, const CogsGemm& g, int tile, bool alone) {
     MidArgs p;
     const int rc = cogs_fill_epi(g, &p.epi);
     if (rc != COGS_OK) return rc;
@@ -258,7 +328,7 @@ int cogs_k_gemm_mid(hipStream_t st, const CogsGemm& g, int tile) {
     p.W = (const char*)g.W; p.ldw = g.ldw * 2;
     p.M = g.M; p.N = g.N; p.KT = g.K / 64;
     p.ln_part = g.ln_part; p.ln_tiles = g.K / 64; p.ln_inv_h = 1.0f / (float)g.K; p.ln_eps = g.ln_eps;
-#define COGS_MID_CASE(E) case E: dispatch_tile<E>(st, p, tile); break;
+#define COGS_MID_CASE(E) case E: dispatch_tile<E>(st, p, tile, alone); break;
     switch (cogs_epi_mask(g)) {
         COGS_MID_CASE(0)
         COGS_MID_CASE(EPI_BIAS)
@@ -279,7 +349,7 @@ int cogs_k_gemm_mid(hipStream_t st, const CogsGemm& g, int tile) {
         COGS_MID_CASE(EPI_SWIGLU | EPI_BIAS)
         COGS_MID_CASE(EPI_GELU_ERF)
         COGS_MID_CASE(EPI_F32OUT)
-        default: dispatch_tile<EPI_GENERIC>(st, p, tile); break;
+        default: dispatch_tile<EPI_GENERIC>(st, p, tile, alone); break;
     }
 #undef COGS_MID_CASE
     return COGS_LAUNCH_CHECK();

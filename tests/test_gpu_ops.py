@@ -1118,6 +1118,12 @@ def test_mid_size_gemm_tiles_equal_each_other_and_fp64(dev, tile):
                 assert bool(((x.double() - ref).abs() <= bound * 1.01).all()), (M, N, K, name)
 
 
+@pytest.mark.parametrize("tile", [6, 7])
+def test_mid_size_gemm_tiles_of_two_slabs_and_of_160_rows(dev, tile):
+    """the same edges for 128x64 with two slabs a slot and 160x64 (five row blocks a wave; a folded norm falls back to 128x64)"""
+    test_mid_size_gemm_tiles_equal_each_other_and_fp64(dev, tile)
+
+
 @pytest.mark.parametrize("t,h,w,merge,max_tokens,offset", [
     (1, 28, 28, 2, 16384, 0),        # one window, enlarged: the smallest
     (1, 45, 61, 1, 16384, 1),        # odd grid (bands of one patch), frames that start off a word
