@@ -1,17 +1,24 @@
 // Few-row GEMM for batched decode:  C[M,N] = epilogue( A[M,K] . W[N,K]^T ),  2 <= M <= 64, bf16.
 //
-// HBM-bound like the single-row GEMV (gemv.hip): every weight byte is read once, straight into MFMA A fragments. A workgroup owns
-// 16 NT output columns; its NW waves take alternate 64-element slices of K (a row's slice is one whole 128-byte line), the batch rows
-// are the columns of v_mfma_f32_16x16x32_bf16 (MT groups of 16), and the waves' partial tiles are summed through LDS in a fixed
-// order. (How many waves and partial sums there are depends on M as well as on N and K: a row's bits may differ between steps of
-// other numbers of rows.) The batch rows come from L2 once per workgroup -- as many bytes as the weights with NT = 1 and M = 16 -- so columns are
-// taken 64 or 32 at a time where that still makes 160 workgroups.
+// HBM-bound like the single-row GEMV (gemv.hip): every weight byte is read once. A workgroup owns 16 NT output columns; its NW waves
+// take alternate 64-element slices of K, the batch rows are the columns of v_mfma_f32_16x16x32_bf16 (MT groups of 16), and the
+// waves' partial tiles are summed through LDS in a fixed order. (How many waves and partial sums there are depends on M as well as on N
+// and K: a row's bits may differ between steps of other numbers of rows.)
+//
+// Each wave streams its slices through a ring of its own, D slices of whole 128-byte lines by LDS-DMA: no barrier in the loop, the
+// wave waits for its own loads alone. Matrix fragments straight from memory put sixteen rows of 16 bytes into every quarter of a load: the
+// vector-memory path then took in 39 B/ns a CU whatever was in flight, also of weights that sat in L2 (8 x 8192 x 2048: 7.4 us from
+// L2, 9.8 from HBM); whole lines come at 110 (4.6 and 8.0). The weights are read with the streaming hint: nothing reads them again before
+// the next step, and 5 to 10 % less time (11 264 x 2048, 16 rows: 11.6 -> 10.9). Columns are taken 64 or 32 at a time where that still
+// makes 160 workgroups: the batch rows come from L2 once per workgroup, as many bytes as the weights with NT = 1 and M = 16. Fragments
+// from memory -> ring, weights from HBM (us):
+//      rows    6176 x 2048    8192 x 2048    11 264 x 2048    32 768 x 2048    2048 x 8192    2048 x 5632    4096 x 11 008
+//       16     9.9 -> 7.2     11.1 -> 8.6     14.8 -> 11.0     32.0 -> 26.6     9.5 -> 8.0     8.3 -> 6.4     21.9 -> 17.7
+//       64    14.7 -> 10.3    15.6 -> 11.6    20.5 -> 14.9     41.6 -> 35.0    13.2 -> 10.8   10.8 -> 9.1     27.9 -> 22.4
 //
 // A sublayer's last product has few columns and a long K: 2048 columns are 128 workgroups of 16, each a quarter of what the chip
 // could have in flight. Where the caller takes partial sums (cogs_k_stream_norm adds them up as it reads them), K is cut over
-// gridDim.y workgroups that each store an fp32 partial. 16 rows, weights from HBM: 2048 x 5632 15.1 -> 7.9 us (2.9 TB/s),
-// 2048 x 8192 18.6 -> 9.1, 2048 x 2048 6.6 -> 4.6, 4096 x 11008 30.1 -> 20.0 (4.5 TB/s); unsplit, 64 columns at a time and without the
-// streaming hint on the weight loads, 11264 x 2048 16.5 -> 12.9, 22016 x 4096 50.4 -> 43.
+// gridDim.y workgroups that each store an fp32 partial.
 #include "common.h"
 #include "kernels.h"
 #include "gemm_epilogue.h"
@@ -27,76 +34,124 @@ struct SkinnyArgs {
     EpiArgs epi;
 };
 
-// U slices in flight per wave
-template <int MT, int NT, int NW, int U>
+// at most n slices' pieces (P each) of this wave may stay in flight, n <= MAX
+template <int P, int MAX>
+__device__ __forceinline__ void wait_slices(int n) {
+    static_assert(MAX <= 3 && MAX * P < 64, "vmcnt is a 6-bit immediate");
+    if (n <= 0) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    else if (n == 1) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(P) : "memory");
+    else if (n == 2) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(MAX >= 2 ? 2 * P : 0) : "memory");
+    else asm volatile("s_waitcnt vmcnt(%0)" ::"n"(MAX >= 3 ? 3 * P : 0) : "memory");
+}
+
+// a piece: 8 rows x 128 bytes, 1 KiB of LDS; HINT: cache policy bits of the load (2: streaming)
+template <int HINT>
+__device__ __forceinline__ void piece16(const bf16_t* g, char* l) {
+    __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)g, (__attribute__((address_space(3))) void*)l, 16, 0, HINT);
+}
+
+// AP: pieces of batch rows a slice has (rows past M repeat the last), D: slices in a wave's ring
+template <int MT, int AP, int NT, int NW, int D>
 __global__ __launch_bounds__(64 * NW) void gemm_skinny_kernel(SkinnyArgs p) {
-    __shared__ __attribute__((aligned(16))) f32x4 red[NW][MT * NT][64];
+    extern __shared__ __attribute__((aligned(16))) char smem[];
+    constexpr int P = 2 * NT + AP, RING = D * P * 1024;
+    static_assert(MT * NT * 1024 <= RING, "a wave's partial tile takes its ring's place");
     const int lane = threadIdx.x & 63, li = lane & 15, g = lane >> 4;
     const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int n0 = blockIdx.x * (16 * NT);
-    const bf16_t *w[NT], *a[MT];
+    char* const ring = smem + wid * RING;
+    const int all = p.K >> 6, end = all * (blockIdx.y + 1) / gridDim.y, first = all * blockIdx.y / gridDim.y + wid;
+    const int n = first < end ? (end - first + NW - 1) / NW : 0;                // this wave's slices
+    // lane -> row lane >> 3 of a piece, 16-byte chunk lane & 7, swizzled
+    const int r = lane >> 3, c = (lane & 7) ^ r;
+    const bf16_t *w[2 * NT], *a[AP];
+#pragma unroll
+    for (int i = 0; i < 2 * NT; ++i) w[i] = p.W + (long)min(n0 + 8 * i + r, p.N - 1) * p.ldw + 64 * first + 8 * c;
+#pragma unroll
+    for (int i = 0; i < AP; ++i) a[i] = p.A + (long)min(8 * i + r, p.M - 1) * p.lda + 64 * first + 8 * c;
+    auto stage = [&](int slot) {                 // the next slice of the stream
+        char* d = ring + slot * (P * 1024);
+#pragma unroll
+        for (int i = 0; i < 2 * NT; ++i) { piece16<2>(w[i], d + i * 1024); w[i] += NW * 64; }
+#pragma unroll
+        for (int i = 0; i < AP; ++i) { piece16<0>(a[i], d + (2 * NT + i) * 1024); a[i] += NW * 64; }
+    };
+    for (int i = 0; i < D && i < n; ++i) stage(i);
     f32x4 acc[MT * NT];
 #pragma unroll
-    for (int t = 0; t < NT; ++t) w[t] = p.W + (long)min(n0 + 16 * t + li, p.N - 1) * p.ldw + 8 * g;
-#pragma unroll
-    for (int t = 0; t < MT; ++t) a[t] = p.A + (long)min(16 * t + li, p.M - 1) * p.lda + 8 * g;
-#pragma unroll
     for (int t = 0; t < MT * NT; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
-    const int all = p.K >> 6, ns = all * (blockIdx.y + 1) / gridDim.y;
-    for (int sl = all * blockIdx.y / gridDim.y + wid; sl < ns; sl += NW * U) {
-        u32x4 wf[U][NT][2], af[U][MT][2];
-        // (slices past the end repeat the last one and are not multiplied: every load of a batch goes out at once)
+    int off[2];                                  // row li of a 16-row group, 16-byte chunk 4 h + g
 #pragma unroll
-        for (int u = 0; u < U; ++u) {
-            const int k = 64 * min(sl + NW * u, ns - 1);
+    for (int h = 0; h < 2; ++h) off[h] = (li & 7) * 128 + (((4 * h + g) ^ (li & 7)) << 4);
+    int slot = 0;
+    for (int i = 0; i < n; ++i) {
+        wait_slices<P, D - 1>(min(D - 1, n - 1 - i));
+        const char* d = ring + slot * (P * 1024);
+        u32x4 wf[NT][2], af[MT][2];
 #pragma unroll
-            for (int t = 0; t < NT; ++t)
+        for (int h = 0; h < 2; ++h) {
 #pragma unroll
-                for (int hf = 0; hf < 2; ++hf) wf[u][t][hf] = *reinterpret_cast<const u32x4*>(w[t] + k + 32 * hf);
+            for (int t = 0; t < NT; ++t) wf[t][h] = *reinterpret_cast<const u32x4*>(d + (2 * t + (li >> 3)) * 1024 + off[h]);
+#pragma unroll
+            for (int t = 0; t < MT; ++t) af[t][h] = *reinterpret_cast<const u32x4*>(d + (2 * NT + min(2 * t + (li >> 3), AP - 1)) * 1024 + off[h]);
         }
+        // the wait for the fragments stands here, in front of the DMA into their slot
 #pragma unroll
-        for (int u = 0; u < U; ++u) {
-            const int k = 64 * min(sl + NW * u, ns - 1);
+        for (int t = 0; t < NT; ++t) asm volatile("" : "+v"(wf[t][0]), "+v"(wf[t][1]));
 #pragma unroll
-            for (int t = 0; t < MT; ++t)
+        for (int t = 0; t < MT; ++t) asm volatile("" : "+v"(af[t][0]), "+v"(af[t][1]));
+        asm volatile("" ::: "memory");
+        if (i + D < n) stage(slot);
 #pragma unroll
-                for (int hf = 0; hf < 2; ++hf) af[u][t][hf] = *reinterpret_cast<const u32x4*>(a[t] + k + 32 * hf);
-        }
-        __builtin_amdgcn_sched_barrier(0);          // (hipcc otherwise sinks the loads to their uses to save registers)
+        for (int t = 0; t < MT; ++t)
 #pragma unroll
-        for (int u = 0; u < U; ++u) {
-            if (sl + NW * u >= ns) break;
+            for (int q = 0; q < NT; ++q)
 #pragma unroll
-            for (int t = 0; t < MT; ++t)
-#pragma unroll
-                for (int q = 0; q < NT; ++q)
-#pragma unroll
-                    for (int hf = 0; hf < 2; ++hf)
-                        acc[t * NT + q] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, wf[u][q][hf]),
-                                                                                  __builtin_bit_cast(bf16x8, af[u][t][hf]), acc[t * NT + q], 0, 0, 0);
-        }
+                for (int h = 0; h < 2; ++h)
+                    acc[t * NT + q] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, wf[q][h]),
+                                                                              __builtin_bit_cast(bf16x8, af[t][h]), acc[t * NT + q], 0, 0, 0);
+        slot = slot == D - 1 ? 0 : slot + 1;
     }
+    // (every load into the ring has been waited for)
+    auto red = [&](int wave, int t) { return reinterpret_cast<f32x4*>(smem + wave * RING) + t * 64 + lane; };
 #pragma unroll
-    for (int t = 0; t < MT * NT; ++t) red[wid][t][lane] = acc[t];
+    for (int t = 0; t < MT * NT; ++t) *red(wid, t) = acc[t];
     __syncthreads();
     for (int t = wid; t < MT * NT; t += NW) {
-        f32x4 v = red[0][t][lane];
+        f32x4 v = *red(0, t);
 #pragma unroll
-        for (int s = 1; s < NW; ++s) v += red[s][t][lane];
-        const int m = 16 * (t / NT) + li, n = n0 + 16 * (t % NT) + 4 * g;
-        if (m >= p.M || n >= p.N) continue;
+        for (int s = 1; s < NW; ++s) v += *red(s, t);
+        const int m = 16 * (t / NT) + li, nn = n0 + 16 * (t % NT) + 4 * g;
+        if (m >= p.M || nn >= p.N) continue;
         if (gridDim.y == 1) {
-            epilogue4<bf16_t>(p.epi, m, n, v);
+            epilogue4<bf16_t>(p.epi, m, nn, v);
         } else {
-            if (p.epi.bias && blockIdx.y == 0) v += ld4_f<bf16_t>(reinterpret_cast<const bf16_t*>(p.epi.bias) + n);
-            *reinterpret_cast<f32x4*>(p.part + ((long)blockIdx.y * p.M + m) * p.N + n) = v;
+            if (p.epi.bias && blockIdx.y == 0) v += ld4_f<bf16_t>(reinterpret_cast<const bf16_t*>(p.epi.bias) + nn);
+            *reinterpret_cast<f32x4*>(p.part + ((long)blockIdx.y * p.M + m) * p.N + nn) = v;
         }
     }
 }
 
-template <int MT, int NT, int NW, int U>
+template <int MT, int AP, int NT, int NW, int D>
+void launch1(hipStream_t st, const SkinnyArgs& p, int splits) {
+    constexpr int lds = NW * D * (2 * NT + AP) * 1024;
+    static_assert(lds <= 160 * 1024, "");
+    static std::atomic<uint64_t> attr_done{0};
+    cogs_ensure_dyn_lds((const void*)gemm_skinny_kernel<MT, AP, NT, NW, D>, lds, attr_done);
+    hipLaunchKernelGGL((gemm_skinny_kernel<MT, AP, NT, NW, D>), dim3((p.N + 16 * NT - 1) / (16 * NT), splits), dim3(64 * NW), lds, st, p);
+}
+template <int MT, int NT, int NW, int D>
 void launch(hipStream_t st, const SkinnyArgs& p, int splits) {
-    hipLaunchKernelGGL((gemm_skinny_kernel<MT, NT, NW, U>), dim3((p.N + 16 * NT - 1) / (16 * NT), splits), dim3(64 * NW), 0, st, p);
+    if constexpr (MT == 1)
+        if (p.M <= 8) return launch1<MT, 1, NT, NW, D>(st, p, splits);
+    launch1<MT, 2 * MT, NT, NW, D>(st, p, splits);
+}
+// columns at a time; the ring takes 64 to 144 KB, two workgroups a CU for the most used sizes
+template <int MT>
+void launch_cols(hipStream_t st, const SkinnyArgs& p, int cols, int splits) {
+    if (cols == 64) launch<MT, 4, 4, 2>(st, p, splits);
+    else if (cols == 32) launch<MT, 2, MT == 1 ? 8 : 4, 3>(st, p, splits);
+    else launch<MT, 1, 4, MT == 1 ? 4 : MT == 2 ? 3 : 2>(st, p, splits);
 }
 
 }  // namespace
@@ -110,7 +165,7 @@ bool cogs_k_gemm_skinny_fits(const CogsGemm& g) {
 // (M <= 16) or four; else eight or four, so that the 64-column groups come to 256 workgroups.
 int cogs_k_gemm_skinny_parts(int M, int N, int K) {
     if (N > 4096 || K < 1024) return 1;
-    if (M <= 32 && K < 4096) return M <= 16 ? 2 : 4;
+    if (K < 4096) return M <= 16 ? 2 : 4;
     return N <= 2048 ? 8 : 4;
 }
 
@@ -124,29 +179,9 @@ int cogs_k_gemm_skinny(hipStream_t st, const CogsGemm& g, float* part) {
     g_cogs_debug.gemm_last_body = 7;
     const int parts = part ? cogs_k_gemm_skinny_parts(g.M, g.N, g.K) : 1;
     if (part && (g.act != COGS_ACT_NONE || g.residual || g.rope_cos || g.out_f32 || parts < 2)) return COGS_E_UNSUPPORTED;
-    if (parts > 1) {
-        const bool long_k = g.K >= 4096;
-        if (g.M <= 16) { if (long_k) launch<1, 4, 4, 2>(st, p, parts); else launch<1, 1, 4, 4>(st, p, parts); }
-        else if (g.M <= 32) { if (long_k) launch<2, 4, 4, 2>(st, p, parts); else launch<2, 2, 4, 2>(st, p, parts); }
-        else launch<4, 4, 4, 1>(st, p, parts);
-        return COGS_LAUNCH_CHECK();
-    }
-    const bool deep = g.K >= 1024;                  // else too few slices for eight waves
-    const int cols = g.N >= 64 * 160 ? 64 : g.N >= 32 * 160 ? 32 : 16;
-    if (g.M <= 16) {
-        if (!deep) launch<1, 1, 4, 4>(st, p, 1);
-        else if (cols == 64) launch<1, 4, 4, 2>(st, p, 1);
-        else if (cols == 32) launch<1, 2, 8, 2>(st, p, 1);
-        else launch<1, 1, 8, 4>(st, p, 1);
-    } else if (g.M <= 32) {
-        if (!deep) launch<2, 1, 4, 4>(st, p, 1);
-        else if (cols == 64) launch<2, 4, 8, 1>(st, p, 1);
-        else if (cols == 32) launch<2, 2, 8, 2>(st, p, 1);
-        else launch<2, 1, 8, 2>(st, p, 1);
-    } else {
-        if (!deep) launch<4, 1, 4, 2>(st, p, 1);
-        else if (cols > 16) launch<4, 2, 8, 1>(st, p, 1);
-        else launch<4, 1, 8, 2>(st, p, 1);
-    }
+    const int cols = parts > 1 ? (g.K >= 4096 ? 64 : g.M <= 16 ? 16 : 32) : g.N >= 64 * 160 ? 64 : g.N >= 32 * 160 ? 32 : 16;
+    if (g.M <= 16) launch_cols<1>(st, p, cols, parts);
+    else if (g.M <= 32) launch_cols<2>(st, p, cols, parts);
+    else launch_cols<4>(st, p, cols, parts);
     return COGS_LAUNCH_CHECK();
 }

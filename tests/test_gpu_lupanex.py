@@ -386,6 +386,18 @@ def test_sublayer_outputs_in_partial_sums(dev, rows, width, ff):
     assert rms_err(got, lo.forward(cfg, double(st), toks)[0]) < TOL[torch.bfloat16]
 
 
+@pytest.mark.parametrize("rows", [2, 8, 9, 17, 33])
+@pytest.mark.parametrize("width,ff", [(70, 10300), (1344, 5200)])
+def test_few_row_products_at_the_edges_of_their_rings(dev, rows, width, ff):
+    """rows at the edges of 8-row pieces and 16-row groups; waves with no, one and more slices than their ring holds (K = 128, 192, 1344,
+    5248, 10 304); 16, 32 and 64 columns at a time, ragged at the end; partial sums"""
+    cfg = config([attention(heads=4, kv_heads=2, dim=32, vdim=40)], width=width, ff=ff, vocab=97)
+    st = state(cfg)
+    toks = tokens(cfg, rows)
+    got = run(engine(cfg, st, torch.bfloat16), toks)
+    assert rms_err(got, lo.forward(cfg, double(st), toks)[0]) < TOL[torch.bfloat16]
+
+
 @pytest.mark.parametrize("dim,vdim", [(16, 16), (64, 48), (80, 16), (128, 128), (144, 32), (256, 16)])
 def test_chunked_delta_rule_at_the_edges_of_its_tiles(dev, dim, vdim):
     """every number of row tiles per wave, whole and ragged; chunks of one token, whole and ragged ones, one to four of them, from nothing
