@@ -575,11 +575,113 @@ __global__ __launch_bounds__(256) void delta_out_kernel(CogsDelta p) {
     }
 }
 
-// One new token per sequence: a workgroup per (head, sequence). S passes through registers once (NPER chunks of four columns per
+// One new token per sequence: a workgroup per (head, sequence), a wave per 16 columns of S: lane = (row group of 16, four columns), PER rows
+// a lane, so that both products with S close inside the wave and only the read-out's norm needs the others. S passes through registers
+// once; it is asked for behind the convolution's inputs (loads return in order) and arrives while they are worked on.
+// What is there besides the state is latency: a thread per column group with the row groups' sums in LDS had five barriers and sums of 16
+// in a row (8 sequences, 16 heads of 128: 10.6 us; this one 9.9, of which 33.6 MB of state in and out take 6.8).
+template <typename T, int PER, int TAPS>
+__global__ __launch_bounds__(1024) void delta_step_kernel(CogsDelta p) {
+    __shared__ __attribute__((aligned(16))) float z[3 * 256];           // q | k | v of this head behind the convolution
+    __shared__ float red[16];
+    const int h = blockIdx.x, row = blockIdx.y, tid = threadIdx.x, lane = tid & 63, wid = tid >> 6, threads = blockDim.x;
+    const int rep = p.heads / p.kv_heads, kh = h / rep, v0 = 2 * p.kv_heads * p.dkp, rg = lane >> 2, col = 16 * wid + 4 * (lane & 3);
+    const float* x = p.t + (long)row * p.ldt;
+    const float* gate = x + v0 + (long)p.heads * p.dvp + (long)h * p.dvp;
+    const float* tb = x + v0 + 2 * p.heads * p.dvp;
+    const CogsSeq s = p.seqs[row];
+    const int pos = s.pos0, at = pos % p.taps, n = 2 * p.dkp + p.dvp;
+    float* S = s.state + p.state_off + (long)h * p.dkp * p.dvp;
+    float* ring = s.state + p.state_off + (long)p.heads * p.dkp * p.dvp;
+    // channel of z[i]; its inputs, latest first, and their taps (zeros past the sequence's start)
+    auto channel = [&](int i) { return i < p.dkp ? kh * p.dkp + i : i < 2 * p.dkp ? (p.kv_heads + kh) * p.dkp + i - p.dkp : v0 + h * p.dvp + i - 2 * p.dkp; };
+    float in[TAPS], tap[TAPS];
+    auto request = [&](int i) {
+        const int c = channel(i);
+#pragma unroll
+        for (int j = 0; j < TAPS; ++j) {
+            const bool there = j < p.taps && j <= pos;
+            tap[j] = there ? p.conv[(long)(p.taps - 1 - j) * p.channels + c] : 0.f;
+            in[j] = j == 0 ? x[c] : there ? ring[(long)(at - j + (j > at ? p.taps : 0)) * p.channels + c] : 0.f;
+        }
+    };
+    auto finish = [&](int i) {
+        float y = tap[0] * in[0];
+#pragma unroll
+        for (int j = 1; j < TAPS; ++j) y = fmaf(tap[j], in[j], y);
+        z[(i < p.dkp ? 0 : i < 2 * p.dkp ? 256 - p.dkp : 512 - 2 * p.dkp) + i] = y / (1.f + expf(-y));
+        // the new input takes the oldest one's place, which no position reads any more
+        if (i >= 2 * p.dkp || h % rep == 0) ring[(long)at * p.channels + channel(i)] = in[0];
+    };
+    if (tid < n) request(tid);
+    const f32x4 zg = *reinterpret_cast<const f32x4*>(gate + col), wn = *reinterpret_cast<const f32x4*>(p.norm + col);
+    const float beta = sigmoid_f(tb[h]), g = expf(p.neg_a[h] * softplus_f(tb[p.headsp + h] + p.dt_bias[h]));
+    f32x4 sr[PER];
+#pragma unroll
+    for (int i = 0; i < PER; ++i)
+        sr[i] = pos > 0 && 16 * i < p.dkp ? *reinterpret_cast<const f32x4*>(S + (long)(16 * i + rg) * p.dvp + col) : f32x4{0.f, 0.f, 0.f, 0.f};
+    if (tid < n) finish(tid);
+    for (int i = tid + threads; i < n; i += threads) { request(i); finish(i); }
+    __syncthreads();
+    float sq = 0.f, sk = 0.f;
+    for (int d = lane; d < p.dkp; d += 64) { sq += z[d] * z[d]; sk += z[256 + d] * z[256 + d]; }
+    const float fq = unit_scale(wave_sum(sq)) * p.q_scale, fk = unit_scale(wave_sum(sk));
+    // the sum over the 16 row groups, in every lane
+    auto close = [](f32x4 a) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            float v = a[e];
+            v += lane_xor_dpp<4>(v);
+            v += lane_xor_dpp<8>(v);
+            const unsigned b = __builtin_bit_cast(unsigned, v);
+            const auto m = __builtin_amdgcn_permlane16_swap(b, b, false, false);
+            v = __builtin_bit_cast(float, (unsigned)m[0]) + __builtin_bit_cast(float, (unsigned)m[1]);
+            const unsigned c = __builtin_bit_cast(unsigned, v);
+            const auto o = __builtin_amdgcn_permlane32_swap(c, c, false, false);
+            a[e] = __builtin_bit_cast(float, (unsigned)o[0]) + __builtin_bit_cast(float, (unsigned)o[1]);
+        }
+        return a;
+    };
+    f32x4 a = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+        if (16 * i >= p.dkp) continue;
+        sr[i] *= g;
+        a += sr[i] * (z[256 + 16 * i + rg] * fk);
+    }
+    a = close(a);
+    const f32x4 u = beta * (*reinterpret_cast<const f32x4*>(z + 512 + col) - a);
+    a = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+        if (16 * i >= p.dkp) continue;
+        sr[i] += u * (z[256 + 16 * i + rg] * fk);
+        *reinterpret_cast<f32x4*>(S + (long)(16 * i + rg) * p.dvp + col) = sr[i];
+        a += sr[i] * (z[16 * i + rg] * fq);
+    }
+    a = close(a);
+    // read-out's norm and gate
+    float ss = (a[0] * a[0] + a[1] * a[1]) + (a[2] * a[2] + a[3] * a[3]);
+    ss += lane_xor_dpp<1>(ss);
+    ss += lane_xor_dpp<2>(ss);
+    if (lane == 0) red[wid] = ss;
+    __syncthreads();
+    ss = 0.f;
+    for (int w = 0; w < threads >> 6; ++w) ss += red[w];
+    const float f = 1.f / sqrtf(ss / (float)p.vdim + p.eps);
+    if (lane < 4) {
+        f32x4 y;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) y[e] = a[e] * f * wn[e] * (zg[e] / (1.f + expf(-zg[e])));
+        st4_f<T>(reinterpret_cast<T*>(p.att) + (long)row * p.ldo + (long)h * p.dvp + col, y);
+    }
+}
+
+// The same for heads of more than 256 rows or columns. S passes through registers once (NPER chunks of four columns per
 // thread; 0: read twice from memory): thread = (row group, four columns), the row groups' partial sums meet in LDS.
 constexpr int STEP_T = 512;
 template <typename T, int NPER>
-__global__ __launch_bounds__(STEP_T) void delta_step_kernel(CogsDelta p) {
+__global__ __launch_bounds__(STEP_T) void delta_step_wide_kernel(CogsDelta p) {
     extern __shared__ __attribute__((aligned(16))) float sm[];
     const int h = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
     const int row = blockIdx.y;
@@ -678,12 +780,19 @@ __global__ __launch_bounds__(STEP_T) void delta_step_kernel(CogsDelta p) {
 
 template <typename T>
 int launch_step(hipStream_t st, const CogsDelta& p, int nseq) {
+    const dim3 grid(p.heads, nseq);
+    if (p.dkp <= 256 && p.dvp <= 256 && p.taps <= 8) {
+#define COGS_STEP(N, TAPS) hipLaunchKernelGGL((delta_step_kernel<T, N, TAPS>), grid, dim3(4 * p.dvp), 0, st, p)
+        if (p.dkp <= 128) { if (p.taps <= 4) COGS_STEP(8, 4); else COGS_STEP(8, 8); }
+        else if (p.taps <= 4) COGS_STEP(16, 4);
+        else COGS_STEP(16, 8);
+#undef COGS_STEP
+        return COGS_LAUNCH_CHECK();
+    }
     const int nc = p.dvp / 4, groups = STEP_T / nc, nper = (p.dkp + groups - 1) / groups;
     const size_t lds = (size_t)(2 * p.dkp + 2 * p.dvp + 16) * 4 + (size_t)groups * nc * 16;
-    const dim3 grid(p.heads, nseq);
-#define COGS_STEP(N) hipLaunchKernelGGL((delta_step_kernel<T, N>), grid, dim3(STEP_T), lds, st, p)
-    if (nper <= 2) COGS_STEP(2);
-    else if (nper <= 8) COGS_STEP(8);
+#define COGS_STEP(N) hipLaunchKernelGGL((delta_step_wide_kernel<T, N>), grid, dim3(STEP_T), lds, st, p)
+    if (nper <= 8) COGS_STEP(8);
     else if (nper <= 32) COGS_STEP(32);
     else COGS_STEP(0);
 #undef COGS_STEP

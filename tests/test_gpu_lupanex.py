@@ -398,6 +398,20 @@ def test_few_row_products_at_the_edges_of_their_rings(dev, rows, width, ff):
     assert rms_err(got, lo.forward(cfg, double(st), toks)[0]) < TOL[torch.bfloat16]
 
 
+@pytest.mark.parametrize("dim,vdim,conv", [(16, 16, 1), (64, 256, 4), (256, 48, 5), (128, 128, 4), (130, 256, 8), (272, 16, 3), (16, 272, 9)])
+def test_one_token_delta_rule_at_the_edges_of_its_kernels(dev, dim, vdim, conv):
+    """one to sixteen waves of 16 columns, whole and ragged rows a lane, more channels than threads, windows of one to nine taps that start
+    empty and wrap around, shared q / k heads; above 256 rows or columns, or eight taps, the wide form: within the tolerance of the oracle"""
+    cfg = config([delta(heads=4, kv_heads=2, dim=dim, vdim=vdim, conv=conv, ff=None)], width=64)
+    st = state(cfg)
+    toks = tokens(cfg, 24)
+    lg = lo.forward(cfg, double(st), toks)[0]
+    for dtype in DTYPES:
+        e = engine(cfg, st, dtype)
+        for first in (1, 5):
+            assert rms_err(run(e, toks, range(first, 24), reserve=8), lg) < TOL[dtype], (dtype, first)
+
+
 @pytest.mark.parametrize("dim,vdim", [(16, 16), (64, 48), (80, 16), (128, 128), (144, 32), (256, 16)])
 def test_chunked_delta_rule_at_the_edges_of_its_tiles(dev, dim, vdim):
     """every number of row tiles per wave, whole and ragged; chunks of one token, whole and ragged ones, one to four of them, from nothing
