@@ -96,10 +96,10 @@ Work carve(const CogsDecoder& d, int S, int nseq, int64_t C, int n_want, void* w
             size_t b = 0;
             if (d.layers[l].mixer == COGS_MIX_LATENT && absorbed_step(S, nseq)) {
                 const int heads = d.layers[l].latent.heads;
-                b = (size_t)nseq * cogs_k_mla_decode_splits(nseq, heads, (int)C) * heads * (d.geom[l].lat.kvp + 2) * 4;
+                b = (size_t)cogs_k_mla_decode_parts(nseq, 1, heads, C) * heads * (d.geom[l].lat.kvp + 2) * 4;
             } else if (d.layers[l].mixer == COGS_MIX_ATTENTION) {
                 const cogs_attn_mixer& m = d.layers[l].attn;
-                b = (size_t)nseq * cogs_k_mla_decode_splits(nseq * m.kv_heads, m.heads / m.kv_heads, (int)C) * m.heads * (d.geom[l].att.dv + 2) * 4;
+                b = (size_t)cogs_k_mla_decode_parts(nseq, m.kv_heads, m.heads / m.kv_heads, C) * m.heads * (d.geom[l].att.dv + 2) * 4;
             }
             part = b > part ? b : part;
         }
@@ -189,7 +189,7 @@ struct Step {
             }
             if (dt == COGS_DT_BF16 && g_cogs_debug.mla_rowwise == 0 && cogs_k_mla_decode_fits(G.kvw, G.kvp)) {
                 CogsMlaDecode a{k.qlat, (long)m.heads * G.kvw, G.kvw, k.seqs, nseq, run.cache_off, G.kvw, G.kvw, 0, G.kvp, m.heads, m.heads,
-                                cogs_k_mla_decode_splits(nseq, m.heads, max_ctx), m.sink, k.part, k.olat, (long)m.heads * G.kvp, G.kvp, nullptr, 0};
+                                max_ctx, C, m.sink, k.part, k.olat, (long)m.heads * G.kvp, G.kvp, nullptr, 0};
                 PROF(COGS_PROF_ATTN);
                 COGS_TRY(cogs_k_mla_decode(st, a));
             } else {
@@ -249,7 +249,7 @@ struct Step {
         }
         if (token_step(S, nseq) && dt == COGS_DT_BF16 && g_cogs_debug.mla_rowwise == 0 && cogs_k_mla_decode_fits(G.kvw, G.dv)) {
             CogsMlaDecode a{k.q, (long)m.heads * G.dk, G.dk, k.seqs, nseq, run.cache_off, G.kvw, G.dk, G.dk, G.dv, m.heads, rep,
-                            cogs_k_mla_decode_splits(nseq * m.kv_heads, rep, max_ctx), nullptr, k.part, k.att, G.oin, G.dv, m.dist_bias, m.dist_n};
+                            max_ctx, C, nullptr, k.part, k.att, G.oin, G.dv, m.dist_bias, m.dist_n};
             PROF(COGS_PROF_ATTN);
             COGS_TRY(cogs_k_mla_decode(st, a));
         } else {

@@ -236,12 +236,13 @@ int cogs_k_mla_attention(hipStream_t st, int dtype, const CogsMla& a);
 struct CogsMlaDecode {
     // cache rows of kvw columns: the first kcols meet the query, kvp from vcol on are summed; `rep` query heads read one block of
     // rows (blocks of a sequence behind one another from column layer_off on)
-    const void* Q; long ldq; int q_head; const CogsSeq* seqs; int nseq; long layer_off; int kvw, kcols, vcol, kvp, heads, rep, nsplit;
-    const float* sink; float* part; void* out; long ldo; int o_head;     // part: nseq * nsplit * heads * (kvp + 2) floats
+    const void* Q; long ldq; int q_head; const CogsSeq* seqs; int nseq; long layer_off; int kvw, kcols, vcol, kvp, heads, rep;
+    int max_ctx; int64_t context;                // keys of the longest sequence, of all together (a sequence's ctx0: of those in front of it)
+    const float* sink; float* part; void* out; long ldo; int o_head;     // part: cogs_k_mla_decode_parts(..) * heads * (kvp + 2) floats
     const float* bias; int nb;                   // as in CogsMla
 };
 bool cogs_k_mla_decode_fits(int kvw, int kvp);
-int cogs_k_mla_decode_splits(int nseq, int heads, int max_ctx);
+int64_t cogs_k_mla_decode_parts(int nseq, int groups, int rep, int64_t context);
 int cogs_k_mla_decode(hipStream_t st, const CogsMlaDecode& a);
 
 // softmax attention with per-head keys and values: head rows behind the fused projection (attn_heads.hip), attention by CogsMla /

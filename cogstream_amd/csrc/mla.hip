@@ -715,99 +715,97 @@ __global__ __launch_bounds__(256 * NH, WPE) void mla_prefill_kernel(CogsMla p, i
 }
 
 // ------------------------------------------------------------------------------------------------ decode attention (bf16)
-// One new row per sequence. Workgroup = (split of the keys, 16 heads, sequence). A tile of 32 cache rows is one contiguous run in
-// memory; it goes through registers into LDS (the next tile's loads are in flight meanwhile) and is read twice there: as K rows
-// (A operand of S^T = C.Q^T; waves share the product as 2 key blocks x 2 halves of the row) and transposed as V (A operand of
-// O^T = C^T.P^T; wave w owns the latent columns 16 (w + 4 i)). The four partial score tiles meet in LDS in the accumulators' own
-// lane layout: every wave adds the halves of both blocks and has all 32 weights of its 16 query columns as the B operand.
+// One new row per sequence. Workgroup = (split of the keys, 16 heads, sequence): `tiles` tiles of 32 keys, as many for every
+// sequence, so that the longest does not have the longest splits. A tile of 32 cache rows is one contiguous run in memory; LDS-DMA
+// brings it into one of two slots (whole lines; 16-byte units beyond a row's end repeat its last, which pads the rows to an odd multiple of 32
+// bytes), both asked for before the first is waited for. It is read twice there: as K rows (A operand of S^T = C.Q^T; waves share the
+// product as 2 key blocks x 2 halves of the row, the queries in registers) and transposed as V (A operand of O^T = C^T.P^T; wave w owns
+// the latent columns 16 (w + 4 i)). The four partial score tiles meet in LDS in the accumulators' own lane layout: every wave adds the
+// halves of both blocks and has all 32 weights of its 16 query columns as the B operand.
+// Sixteen requests of 256 .. 4096 keys, rows of 576 columns, 16 heads: 20.7 us with 32 splits of each request, the next tile's loads in
+// registers and the queries in LDS -> 17.0; three tiles a split (two: 22, more workgroups than are resident; four: 18.9; six: 23). A tile
+// costs 2 us beside a second workgroup, the rest is latency around them: launch, table, first tile, partials out.
 struct MlaDecodeArgs {
     const bf16_t* Q; long ldq; int q_head;
     const CogsSeq* seqs; long layer_off;
     int kvw, kcols, vcol, kvp;              // cache row: columns [0, kcols) meet the query, [vcol, vcol + kvp) are summed
-    int heads, rep, groups, nht, nsplit;    // rep query heads read one cache block, `groups` blocks per sequence
+    int heads, rep, groups, nht, tiles;     // rep query heads read one cache block, `groups` blocks per sequence
     const float* bias; int nb;              // [heads][nb] added at distance min(n, nb - 1), or null
-    float* part_o; float* part_ml;          // [seq][split][head][kvp] relative to part_ml[..][0]; [..][2] = (max, sum)
+    float* part_o; float* part_ml;          // [part][head][kvp]; [..][2] = (max, sum)
 };
 
-template <int DTW, int PER, int WGS>
+constexpr int MLA_TK = 32;                  // keys of a tile
+// splits of sequence b and the place of its first partial: sequences one behind the other, with room for each one's rounding up
+__device__ __forceinline__ int mla_parts(const CogsSeq& s, int tiles) { return (s.pos0 / MLA_TK + tiles) / tiles; }
+__device__ __forceinline__ long mla_first_part(const CogsSeq& s, int b, int tiles) { return s.ctx0 / (MLA_TK * tiles) + b; }
+
+template <int DTW, int PER, int KH, int WGS>
 __global__ __launch_bounds__(256, WGS) void mla_decode_kernel(MlaDecodeArgs p) {
     extern __shared__ __attribute__((aligned(16))) char smem[];
-    constexpr int TK = 32;
+    constexpr int TK = MLA_TK;
     const int RS = p.kvw * 2 + 32;                               // an odd multiple of 32 bytes (kvw % 32 == 0)
-    f32x4* const Sx = reinterpret_cast<f32x4*>(smem);            // [key block][row half][lane]
-    char* const Ks = smem + 4 * 64 * 16;
-    char* const Qs = Ks + TK * RS;
+    f32x4* const Sx = reinterpret_cast<f32x4*>(smem + 2 * TK * RS);       // [key block][row half][lane]
 
     const int tid = threadIdx.x, lane = tid & 63;
     const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int li = lane & 15, g = lane >> 4;
     // the head tiles of a split sit 8 apart in the launch order = on one XCD: its L2 serves the second and later readers
-    const int bid = blockIdx.x, slot = bid & 7, rest = bid >> 3;
-    const int ht = rest % p.nht, split = (rest / p.nht) * 8 + slot;
-    if (split >= p.nsplit) return;
+    const int bid = blockIdx.x, rest = bid >> 3;
+    const int ht = rest % p.nht, split = (rest / p.nht) * 8 + (bid & 7);
     const int b = blockIdx.y / p.groups, grp = blockIdx.y - b * p.groups, h0 = grp * p.rep + ht * 16, h1 = (grp + 1) * p.rep;
     const CogsSeq s = p.seqs[b];
-    const int kend = s.pos0 + 1;
-    const unsigned nt_all = (unsigned)(kend + TK - 1) / TK;
-    const int t_begin = (int)(nt_all * (unsigned)split / (unsigned)p.nsplit);
-    const int t_end = (int)(nt_all * (unsigned)(split + 1) / (unsigned)p.nsplit);
-    const long slot0 = ((long)b * p.nsplit + split) * p.heads;
-    if (t_begin >= t_end) {                                        // nothing to do: an empty partial
-        if (tid < 16 && h0 + tid < h1) { p.part_ml[(slot0 + h0 + tid) * 2] = -INFINITY; p.part_ml[(slot0 + h0 + tid) * 2 + 1] = 0.f; }
-        return;
-    }
+    const int kend = s.pos0 + 1, t_begin = split * p.tiles, t_end = min(t_begin + p.tiles, (kend + TK - 1) / TK);
+    if (t_begin >= t_end) return;
+    const long slot0 = (mla_first_part(s, b, p.tiles) + split) * p.heads;
     const char* cache = s.cache + (p.layer_off + (long)grp * p.kvw) * s.max_len * 2;
-    const int row_bytes = p.kvw * 2, nch = p.kvw >> 3, nqc = p.kcols >> 3;      // 16-byte chunks of a row
-    const int tile_chunks = TK * nch;
-    const int dr_row = 256 / nch, dr_c = 256 % nch;
+    const int row_bytes = p.kvw * 2, nch = p.kvw >> 3, pieces = (nch + 2) >> 1;      // 16-byte units of a row; KiB of a slot
 
-    u32x4 reg[PER];
-    auto load_tile = [&](int t) {
-        const char* base = cache + (long)t * TK * row_bytes;
-        const int lim = min(TK, kend - t * TK) * nch - 1;           // chunks past the end repeat the last one (masked)
-#pragma unroll
-        for (int i = 0; i < PER; ++i)
-            reg[i] = *reinterpret_cast<const u32x4*>(base + min(tid + 256 * i, lim) * 16);
-    };
-    load_tile(t_begin);
-    const int row_t = tid / nch, c_t = tid - row_t * nch;
-    {
-        int r = row_t, c = c_t;
-#pragma unroll 1
-        while (r < 16) {
-            u32x4 v = {0, 0, 0, 0};
-            if (h0 + r < h1 && c < nqc) v = *reinterpret_cast<const u32x4*>(p.Q + (long)b * p.ldq + (long)(h0 + r) * p.q_head + c * 8);
-            *reinterpret_cast<u32x4*>(Qs + r * RS + c * 16) = v;
-            r += dr_row; c += dr_c;
-            if (c >= nch) { c -= nch; ++r; }
-        }
-    }
+    // queries as B operands: this wave's half of the row
     const int ks = p.kcols >> 5, dts = p.kvp >> 4, kh = (ks + 1) >> 1;
-    const int k_lo = (wid >> 1) ? kh : 0, k_hi = (wid >> 1) ? ks : kh;
+    const int k_lo = (wid >> 1) ? kh : 0, k_n = (wid >> 1) ? ks - kh : kh;
+    u32x4 qf[KH];
+    const bf16_t* q = p.Q + (long)b * p.ldq + (long)min(h0 + li, h1 - 1) * p.q_head + 32 * k_lo + 8 * g;
+#pragma unroll
+    for (int i = 0; i < KH; ++i) {
+        qf[i] = u32x4{0, 0, 0, 0};
+        if (i < k_n) qf[i] = *reinterpret_cast<const u32x4*>(q + 32 * i);
+    }
+    // piece i of this wave (past the last: the last again): where its lane's unit lies in the tile
+    int off[PER];
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+        const int j = min(wid + 4 * i, pieces - 1) * 64 + lane, row = j / (nch + 2);
+        off[i] = row * row_bytes + min(j - row * (nch + 2), nch - 1) * 16;
+    }
+    auto stage = [&](int t) {
+        const char* base = cache + (long)t * TK * row_bytes;
+        char* dst = smem + ((t - t_begin) & 1) * (TK * RS);
+        const int last = kend - t * TK - 1;                         // rows past the end repeat the last one (masked)
+#pragma unroll
+        for (int i = 0; i < PER; ++i) {
+            int o = off[i];
+            if (last < TK - 1) o -= max(o / row_bytes - last, 0) * row_bytes;
+            __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(base + o),
+                                             (__attribute__((address_space(3))) void*)(dst + min(wid + 4 * i, pieces - 1) * 1024), 16, 0, 0);
+        }
+    };
+    stage(t_begin);
+    if (t_begin + 1 < t_end) stage(t_begin + 1);
     f32x4 oacc[DTW], lacc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int d = 0; d < DTW; ++d) oacc[d] = f32x4{0.f, 0.f, 0.f, 0.f};
     float m = -INFINITY;
     const bf16x8 ones = __builtin_bit_cast(bf16x8, u32x4{0x3f803f80u, 0x3f803f80u, 0x3f803f80u, 0x3f803f80u});
-    const char* const qrd = Qs + li * RS + 16 * g;
-    const char* const krd = Ks + (16 * (wid & 1) + li) * RS + 16 * g;
-    const char* const vrd = Ks + (4 * g + (li >> 2)) * RS + (li & 3) * 8 + 32 * wid + p.vcol * 2;
+    const int krd = (16 * (wid & 1) + li) * RS + 16 * g + 64 * k_lo;
+    const int vrd = (4 * g + (li >> 2)) * RS + (li & 3) * 8 + 32 * wid + p.vcol * 2;
     const float* const bias = p.bias ? p.bias + (long)min(h0 + li, h1 - 1) * p.nb : nullptr;
     const float b_far = bias ? bias[p.nb - 1] : 0.f;
 
     for (int t = t_begin; t < t_end; ++t) {
-        __syncthreads();                                          // the previous tile's transposed reads are done
-        {
-            int r = row_t, c = c_t;
-#pragma unroll
-            for (int i = 0; i < PER; ++i) {
-                if (tid + 256 * i < tile_chunks) *reinterpret_cast<u32x4*>(Ks + r * RS + c * 16) = reg[i];
-                r += dr_row; c += dr_c;
-                if (c >= nch) { c -= nch; ++r; }
-            }
-        }
+        const char* const Ks = smem + ((t - t_begin) & 1) * (TK * RS);
+        if (t + 1 < t_end) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(PER) : "memory");
+        else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         __syncthreads();
-        if (t + 1 < t_end) load_tile(t + 1);
         const int nvalid = min(TK, kend - t * TK);
         f32x4 bias0 = {b_far, b_far, b_far, b_far}, bias1 = bias0;
         if (bias && s.pos0 - t * TK - (TK - 1) < p.nb - 1) {
@@ -822,23 +820,11 @@ __global__ __launch_bounds__(256, WGS) void mla_decode_kernel(MlaDecodeArgs p) {
             f32x4 acc[4];
 #pragma unroll
             for (int e = 0; e < 4; ++e) acc[e] = f32x4{0.f, 0.f, 0.f, 0.f};
-            int k = k_lo;
-#pragma unroll 1
-            for (; k + 3 < k_hi; k += 4) {
-                u32x4 kf[4], qv[4];
 #pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    kf[e] = *reinterpret_cast<const u32x4*>(krd + 64 * (k + e));
-                    qv[e] = *reinterpret_cast<const u32x4*>(qrd + 64 * (k + e));
-                }
-#pragma unroll
-                for (int e = 0; e < 4; ++e)
-                    acc[e] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, kf[e]), __builtin_bit_cast(bf16x8, qv[e]), acc[e], 0, 0, 0);
-            }
-#pragma unroll 1
-            for (; k < k_hi; ++k)
-                acc[0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, *reinterpret_cast<const u32x4*>(krd + 64 * k)),
-                                                                 __builtin_bit_cast(bf16x8, *reinterpret_cast<const u32x4*>(qrd + 64 * k)), acc[0], 0, 0, 0);
+            for (int i = 0; i < KH; ++i)
+                if (i < k_n)
+                    acc[i & 3] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, *reinterpret_cast<const u32x4*>(Ks + krd + 64 * i)),
+                                                                         __builtin_bit_cast(bf16x8, qf[i]), acc[i & 3], 0, 0, 0);
             Sx[((wid & 1) * 2 + (wid >> 1)) * 64 + lane] = (acc[0] + acc[1]) + (acc[2] + acc[3]);
         }
         __syncthreads();
@@ -865,16 +851,20 @@ __global__ __launch_bounds__(256, WGS) void mla_decode_kernel(MlaDecodeArgs p) {
         const bf16x8 ph = __builtin_bit_cast(bf16x8, u32x4{w[0], w[1], w[2], w[3]}), pl = __builtin_bit_cast(bf16x8, u32x4{x[0], x[1], x[2], x[3]});
         lacc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones, ph, lacc, 0, 0, 0);
         lacc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones, pl, lacc, 0, 0, 0);
-        // (no branch for columns past kvp: such a read stays inside Ks + Qs, and its accumulator is not stored)
+        // (no branch for columns past kvp: such a read stays inside the slots and Sx, and its accumulator is not stored)
 #pragma unroll
         for (int d = 0; d < DTW; ++d) {
-            const char* va = vrd + 128 * d;
+            const char* va = Ks + vrd + 128 * d;
             const i16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) i16x4*)(va));
             const i16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) i16x4*)(va + 16 * RS));
             const u32x2 l2 = __builtin_bit_cast(u32x2, lo), h2 = __builtin_bit_cast(u32x2, hi);
             const bf16x8 vf = __builtin_bit_cast(bf16x8, u32x4{l2[0], l2[1], h2[0], h2[1]});
             oacc[d] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, ph, oacc[d], 0, 0, 0);
             oacc[d] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, pl, oacc[d], 0, 0, 0);
+        }
+        if (t + 2 < t_end) {
+            __syncthreads();                                      // every wave is done with this slot
+            stage(t + 2);
         }
     }
     if (h0 + li < h1) {
@@ -890,17 +880,18 @@ __global__ __launch_bounds__(256, WGS) void mla_decode_kernel(MlaDecodeArgs p) {
 
 // splits of one (sequence, head) -> the head's weighted latent, bf16; 64 latent columns per workgroup, wave w sums every fourth split
 constexpr int MLA_MAX_SPLIT = 256;
-__global__ __launch_bounds__(256) void mla_combine_kernel(const float* __restrict__ part_o, const float* __restrict__ part_ml, int nsplit,
-                                                          int heads, int kvp, const float* __restrict__ sink, bf16_t* __restrict__ out,
-                                                          long ldo, int o_head) {
+__global__ __launch_bounds__(256) void mla_combine_kernel(const float* __restrict__ part_o, const float* __restrict__ part_ml,
+                                                          const CogsSeq* __restrict__ seqs, int tiles, int heads, int kvp,
+                                                          const float* __restrict__ sink, bf16_t* __restrict__ out, long ldo, int o_head) {
     __shared__ float w_sh[MLA_MAX_SPLIT];
     __shared__ float red[4];
     __shared__ float acc_sh[4][64];
     const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
     const int h = blockIdx.x, b = blockIdx.y, d = blockIdx.z * 64 + lane;
-    const long base = (long)b * nsplit * heads + h;
-    // the first 16 partial rows of this wave are requested before the weights are known (an empty split's row holds anything: its
-    // weight is tested, not multiplied)
+    const CogsSeq s = seqs[b];
+    const int nsplit = mla_parts(s, tiles);
+    const long base = mla_first_part(s, b, tiles) * heads + h;
+    // the first 16 partial rows of this wave are requested before the weights are known (past the last: the last again, not used)
     const float* po = part_o + base * kvp + min(d, kvp - 1);
     const long stride = (long)heads * kvp;
     float v[16];
@@ -970,12 +961,12 @@ int launch_prefill_split(hipStream_t st, const CogsMla& a) {
     return halves ? launch_prefill<KN, KR, DT, 2, 2>(st, a) : launch_prefill<KN, KR, DT, 2, 1>(st, a);
 }
 
-template <int DTW, int PER, int WGS>
-int launch_decode(hipStream_t st, const MlaDecodeArgs& p, int nblk) {
+template <int DTW, int PER, int KH, int WGS>
+int launch_decode(hipStream_t st, const MlaDecodeArgs& p, int nblk, int nsplit) {
     static std::atomic<uint64_t> attr_done{0};
-    const int lds = 48 * (p.kvw * 2 + 32) + 4 * 64 * 16;
-    cogs_ensure_dyn_lds((const void*)mla_decode_kernel<DTW, PER, WGS>, 160 * 1024, attr_done);
-    hipLaunchKernelGGL((mla_decode_kernel<DTW, PER, WGS>), dim3((unsigned)((p.nsplit + 7) / 8 * 8 * p.nht), nblk), dim3(256), lds, st, p);
+    const int lds = 2 * MLA_TK * (p.kvw * 2 + 32) + 4 * 64 * 16;
+    cogs_ensure_dyn_lds((const void*)mla_decode_kernel<DTW, PER, KH, WGS>, 160 * 1024, attr_done);
+    hipLaunchKernelGGL((mla_decode_kernel<DTW, PER, KH, WGS>), dim3((unsigned)((nsplit + 7) / 8 * 8 * p.nht), nblk), dim3(256), lds, st, p);
     return COGS_LAUNCH_CHECK();
 }
 
@@ -1055,43 +1046,48 @@ int cogs_k_mla_attention(hipStream_t st, int dtype, const CogsMla& a) {
     return COGS_LAUNCH_CHECK();
 }
 
-bool cogs_k_mla_decode_fits(int kvw, int kvp) {
-    return kvw % 32 == 0 && kvp % 16 == 0 && kvp <= 1024 && 48 * (kvw * 2 + 32) + 4096 <= 160 * 1024 && 32 * (kvw / 8) <= 256 * 18;
+bool cogs_k_mla_decode_fits(int kvw, int kvp) { return kvw % 32 == 0 && kvp % 16 == 0 && kvp <= 1024 && kvw <= 1152; }
+
+// Tiles of 32 keys per split: two workgroups a CU over the whole batch (context: keys of all sequences together), two tiles at the
+// least -- shorter splits cost more in the combine than they save here
+static int decode_tiles(int nseq, int groups, int rep, int64_t context) {
+    const int keys = (int)g_cogs_debug.mla_split_keys;
+    if (keys > 0) return (keys + MLA_TK - 1) / MLA_TK;
+    const int64_t units = (context / MLA_TK + nseq) * groups * ((rep + 15) / 16);
+    return units <= 1024 ? 2 : (int)((units + 511) / 512);
 }
 
-int cogs_k_mla_decode_splits(int nseq, int heads, int max_ctx) {
+// partials of all sequences together, at the most: as many as splits of the longest context up to this one have
+int64_t cogs_k_mla_decode_parts(int nseq, int groups, int rep, int64_t context) {
     const int keys = (int)g_cogs_debug.mla_split_keys;
-    int n;
-    if (keys > 0) n = (max_ctx + keys - 1) / keys;
-    else {
-        const int nht = (heads + 15) / 16;
-        n = 512 / (nseq * nht);                           // two workgroups per CU
-        const int most = (max_ctx + 63) / 64;             // shorter splits cost more in the combine than they save here
-        if (n > most) n = most;
-    }
-    if (n < 1) n = 1;
-    return n > MLA_MAX_SPLIT ? MLA_MAX_SPLIT : n;
+    int64_t n = context / (MLA_TK * (keys > 0 ? decode_tiles(nseq, groups, rep, context) : 2));
+    const int64_t full = 512 / (groups * ((rep + 15) / 16));
+    if (keys <= 0 && n > full) n = full;
+    return n + nseq + 1;
 }
 
 // one new row per sequence: queries of kcols columns per head -> per head the weighted sum of the cache rows' value columns
 int cogs_k_mla_decode(hipStream_t st, const CogsMlaDecode& a) {
     if (a.rep <= 0 || a.heads % a.rep || a.kcols % 32 || a.kcols > a.kvw || a.vcol % 16 || a.vcol + a.kvp > a.kvw || (a.bias && a.nb <= 0) ||
-        a.nseq <= 0 || (long)a.nseq * (a.heads / a.rep) > 65535 || a.nsplit < 1 || a.nsplit > MLA_MAX_SPLIT || !cogs_k_mla_decode_fits(a.kvw, a.kvp) ||
+        a.nseq <= 0 || (long)a.nseq * (a.heads / a.rep) > 65535 || a.max_ctx <= 0 || a.context < a.max_ctx || !cogs_k_mla_decode_fits(a.kvw, a.kvp) ||
         a.ldq % 8 || a.q_head % 8 || a.heads <= 0) return COGS_E_INVALID;
     MlaDecodeArgs p;
     p.Q = (const bf16_t*)a.Q; p.ldq = a.ldq; p.q_head = a.q_head; p.seqs = a.seqs; p.layer_off = a.layer_off;
-    p.kvw = a.kvw; p.kcols = a.kcols; p.vcol = a.vcol; p.kvp = a.kvp; p.nsplit = a.nsplit;
+    p.kvw = a.kvw; p.kcols = a.kcols; p.vcol = a.vcol; p.kvp = a.kvp;
     p.heads = a.heads; p.rep = a.rep; p.groups = a.heads / a.rep; p.nht = (a.rep + 15) / 16;
     p.bias = a.bias; p.nb = a.nb;
-    p.part_o = a.part; p.part_ml = a.part + (size_t)a.nseq * a.nsplit * a.heads * a.kvp;
-    const int dtw = (a.kvp / 16 + 3) / 4, chunks = 32 * (a.kvw / 8), nblk = a.nseq * p.groups;
+    const int all = (a.max_ctx + MLA_TK - 1) / MLA_TK;                // tiles of the longest sequence; the combine takes 256 splits
+    p.tiles = decode_tiles(a.nseq, p.groups, a.rep, a.context);
+    if ((all + p.tiles - 1) / p.tiles > MLA_MAX_SPLIT) p.tiles = (all + MLA_MAX_SPLIT - 1) / MLA_MAX_SPLIT;
+    p.part_o = a.part; p.part_ml = a.part + (size_t)cogs_k_mla_decode_parts(a.nseq, p.groups, a.rep, a.context) * a.heads * a.kvp;
+    const int dtw = (a.kvp / 16 + 3) / 4, nblk = a.nseq * p.groups, nsplit = (all + p.tiles - 1) / p.tiles;
     int rc;
-    if (dtw <= 2 && chunks <= 256 * 4) rc = launch_decode<2, 4, 4>(st, p, nblk);
-    else if (dtw <= 4 && chunks <= 256 * 6) rc = launch_decode<4, 6, 3>(st, p, nblk);
-    else if (dtw <= 8 && chunks <= 256 * 10) rc = launch_decode<8, 10, 2>(st, p, nblk);
-    else rc = launch_decode<16, 18, 1>(st, p, nblk);
+    if (dtw <= 2 && a.kvw <= 256) rc = launch_decode<2, 5, 4, 4>(st, p, nblk, nsplit);
+    else if (dtw <= 4 && a.kvw <= 384) rc = launch_decode<4, 7, 6, 2>(st, p, nblk, nsplit);
+    else if (dtw <= 8 && a.kvw <= 640) rc = launch_decode<8, 11, 10, 2>(st, p, nblk, nsplit);
+    else rc = launch_decode<16, 19, 18, 1>(st, p, nblk, nsplit);
     if (rc != COGS_OK) return rc;
-    hipLaunchKernelGGL(mla_combine_kernel, dim3(a.heads, a.nseq, (a.kvp + 63) / 64), dim3(256), 0, st, p.part_o, p.part_ml, a.nsplit, a.heads,
+    hipLaunchKernelGGL(mla_combine_kernel, dim3(a.heads, a.nseq, (a.kvp + 63) / 64), dim3(256), 0, st, p.part_o, p.part_ml, p.seqs, p.tiles, a.heads,
                        a.kvp, a.sink, (bf16_t*)a.out, a.ldo, a.o_head);
     return COGS_LAUNCH_CHECK();
 }
