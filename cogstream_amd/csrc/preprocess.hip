@@ -6,12 +6,17 @@
 // Pillow's fixed-point algorithm restated exactly (two passes, horizontal first, 22-bit integer coefficients
 // built on the host by cogstream_amd.processing.resample_coeffs, uint8 rounding after each pass), so the uint8
 // image -- and, through the [3,256] value table (processing.pixel_value_table), pixel_values -- is bit-identical to the reference's host path.
-// One kernel does both passes tile by tile; the two-pass kernels remain for shrinking by so much that a tile's intermediate rows
-// do not fit the LDS, and for outputs that are not aligned to a pair of elements.
+// resize_mfma_kernel does both passes as integer matrix products; resize_patchify_kernel does them with vector instructions where a patch's
+// taps span more than 48 source pixels or a band's more than 64 rows (shrinking by more than about 2.6), or a row has fewer pixels than the
+// products take; the two-pass kernels remain for shrinking by so much that a tile's intermediate rows do not fit the LDS, and for outputs
+// that are not aligned to a pair of elements.
 #include "common.h"
 #include "kernels.h"
 
 namespace {
+
+typedef int i32x4 __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));
 
 constexpr int PBITS = 22;
 
@@ -76,9 +81,8 @@ __global__ __launch_bounds__(256) void resize_v_patchify_kernel(const uint8_t* _
 // through memory. Horizontal: a thread keeps one output column, its taps in registers, and walks the rows; the 12 bytes of four
 // taps are one unaligned load. Vertical: a lane owns two neighbouring columns of a patch row -- the order of the output, so that
 // 98 lanes write 392 contiguous bytes -- and takes the three channels together, one tap at a time.
-// Bound by integer arithmetic (two instructions a product; the 22-bit taps leave no packed form) and byte traffic in LDS:
-// 64 frames 480 x 854 -> 308 x 588 in 102 us (1.5 TB/s of
-// frames and pixel_values); the two-pass kernels, a byte load per product, took 447.
+// Bound by loads off a word boundary, integer arithmetic (two instructions a product) and byte traffic in LDS: 64 frames 480 x 854 -> 308 x
+// 588 in 102 us; the two-pass kernels, a byte load per product, took 447.
 constexpr int TILE_P = 6, TILE_C = 14 * TILE_P;
 struct Bytes12 { unsigned w[3]; };
 
@@ -172,6 +176,239 @@ __global__ __launch_bounds__(256) void resize_patchify_kernel(const uint8_t* __r
     }
 }
 
+// ---- both passes as integer matrix products ----------------------------------------------------------------------------------
+// A resize is a banded matrix product, and the 22-bit taps are three signed bytes, so that v_mfma_i32_16x16x64_i8 computes it exactly:
+//   sum p k = sum (p - 128) k0 + 2^8 sum (p - 128) k1 + 2^16 sum (p - 128) k2 + 128 sum k,   k = k0 + 2^8 k1 + 2^16 k2  (|k| < 1.99 * 2^22).
+// A wave owns one patch column (14 output columns) of a band of one or two patch rows and walks over frames. Horizontal: 16 source rows
+// are the product's rows, the patch's columns its columns, and K is the interleaved source bytes as they lie in memory, 12 (four
+// pixels) to a lane's 16 -- a channel's taps are zero at the other channels' bytes. The result lies as four neighbouring rows of one column
+// in a lane: one dword of the wave's transposed [channel][column][64 rows] in LDS, which is the vertical product's operand; that product
+// leaves four neighbouring columns of one output row in a lane, the order of pixel_values. The taps of both passes are in registers in the
+// order of the lanes, built once per wave from the tables.
+// 64 frames 480 x 854 -> 308 x 588: 61 us (the vector form above: 109); 149 MB of frames and pixel_values
+// take 30. 8 of them 32 -> 22 us, 64 x 720 x 1280 192 -> 108. What is left: some 700 vector and 90 matrix instructions a frame and wave.
+constexpr int MM_ROWS = 64, MM_STRIDE = MM_ROWS + 16, MM_WAVES = 4, MM_RESIDENT = 2048;      // source rows of a band; bytes of a column of them in LDS
+
+// digits of a tap, each in the low byte
+__device__ __forceinline__ void tap_digits(int k, unsigned (&d)[3]) {
+    const int d0 = (int)(signed char)k, k1 = (k - d0) >> 8, d1 = (int)(signed char)k1;
+    d[0] = (unsigned)d0 & 255u;
+    d[1] = (unsigned)d1 & 255u;
+    d[2] = (unsigned)((k1 - d1) >> 8) & 255u;
+}
+__device__ __forceinline__ int join_digits(int d0, int d1, int d2) { return (((d2 << 8) + d1) << 8) + d0; }
+// four sums -> their bytes clip8(sum >> PBITS). v_ashr_pk_u8_i32 writes two and leaves the destination's upper half as it was, which hipcc
+// (7.2) takes for zero when it forms the instruction from shifts and ORs by itself: here only the lower halves are looked at
+__device__ __forceinline__ unsigned four_bytes(const i32x4 (&d)[3]) {
+    const unsigned lo = __builtin_amdgcn_ashr_pk_u8_i32(join_digits(d[0][0], d[1][0], d[2][0]), join_digits(d[0][1], d[1][1], d[2][1]), PBITS);
+    const unsigned hi = __builtin_amdgcn_ashr_pk_u8_i32(join_digits(d[0][2], d[1][2], d[2][2]), join_digits(d[0][3], d[1][3], d[2][3]), PBITS);
+    return __builtin_amdgcn_perm(hi, lo, 0x05040100u);
+}
+
+// sum over the lanes {r, r + 16, r + 32, r + 48}, in all four
+__device__ __forceinline__ int sum_groups(int v) {
+    const auto a = __builtin_amdgcn_permlane16_swap((unsigned)v, (unsigned)v, false, false);
+    const unsigned w = a[0] + a[1];
+    const auto b = __builtin_amdgcn_permlane32_swap(w, w, false, false);
+    return (int)(b[0] + b[1]);
+}
+
+// KS: 64-byte steps of K (16 pixels each); BP: patch rows of a band; RT: 16-row tiles of its source rows. The loop over the frames has no
+// branch: the next frame's loads are in flight while this one is worked on, and its stores are not waited for.
+template <typename TO, int KS, int BP, int RT>
+__global__ __launch_bounds__(64 * MM_WAVES, KS == 3 && RT == 4 ? 1 : 2) void resize_mfma_kernel(const uint8_t* __restrict__ in, TO* __restrict__ out, int T, int H, int W, int gh, int gw,
+                                                                       int ms, int frames, const int* __restrict__ bx, const int* __restrict__ kx, int ksx,
+                                                                       const int* __restrict__ by, const int* __restrict__ ky, int ksy,
+                                                                       const float* __restrict__ table) {
+    __shared__ float lut[768];
+    __shared__ __attribute__((aligned(16))) char mids[MM_WAVES][3 * 16 * MM_STRIDE];
+    const int tid = threadIdx.x, lane = tid & 63, li = lane & 15, g = lane >> 4;
+    const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
+    for (int i = tid; i < 768; i += 64 * MM_WAVES) lut[i] = table[i];
+    __syncthreads();
+    // neighbouring workgroups on one XCD: the lines that two patch columns share are in its L2
+    const int nwg = gridDim.x, xcd = blockIdx.x & 7, q8 = nwg >> 3, r8 = nwg & 7;
+    const int wg = (xcd < r8 ? xcd * (q8 + 1) : r8 * (q8 + 1) + (xcd - r8) * q8) + ((int)blockIdx.x >> 3);
+    const int bands = gh / BP, unit = wg * MM_WAVES + wid, pcol = unit % gw, bd = unit / gw % bands, f0 = unit / gw / bands * frames;
+    if (f0 >= T) return;
+    const int fend = min(f0 + frames, T);
+    char* const mid = mids[wid];
+    const int li14 = min(li, 13);                                   // (rows and columns 14 and 15 of the products repeat the last)
+
+    // horizontal: lane = column li of the patch, unit 4 s + g of K = the four pixels from base + 4 (4 s + g) on: the 16 bytes from the word
+    // that the first one starts in, shifted down to twelve (the fourth word has no taps). Loads off a word boundary are many times
+    // slower: with them a frame took 7 us a wave. The clip's last row is read byte by byte where a word behind it would be touched
+    const int x = pcol * 14 + li14, x0 = bx[2 * x], base = min(bx[2 * pcol * 14], W - 16 * KS);
+    const int y_first = bd * BP * 14, r0 = by[2 * y_first];
+    const bool at_end = fend == T && base + 16 * KS >= W - 1 && r0 + 16 * RT >= H;      // (one more pixel behind is three bytes)
+    long src_at[RT];
+#pragma unroll
+    for (int t = 0; t < RT; ++t) src_at[t] = (((long)f0 * H + min(r0 + 16 * t + li, H - 1)) * W + base + 4 * g) * 3;
+    const long words = (long)(reinterpret_cast<size_t>(in) & 3);     // (frames may start off a word)
+    const uint8_t* const in_w = in - words;
+    u32x4 src[RT][KS];
+    unsigned shift[RT];
+    auto load = [&](bool slow) {
+#pragma unroll
+        for (int t = 0; t < RT; ++t) {
+            const long at = src_at[t] + words;
+            shift[t] = (unsigned)at & 3u;
+            if (slow) {
+#pragma unroll
+                for (int s = 0; s < KS; ++s)
+#pragma unroll
+                    for (int w = 0; w < 3; ++w) {
+                        const uint8_t* q = in + src_at[t] + 48 * s + 4 * w;
+                        src[t][s][w] = q[0] | q[1] << 8 | q[2] << 16 | (unsigned)q[3] << 24;
+                    }
+                shift[t] = 0;
+            } else {
+#pragma unroll
+                for (int s = 0; s < KS; ++s) src[t][s] = *reinterpret_cast<const u32x4_a4*>(in_w + (at - shift[t]) + 48 * s);
+            }
+            src_at[t] += (long)H * W * 3;
+        }
+    };
+    load(at_end && f0 == T - 1);
+    u32x4 tx[KS][3][3];                                             // [step][channel][digit]
+    int sum_x = 0;
+#pragma unroll
+    for (int s = 0; s < KS; ++s) {
+#pragma unroll
+        for (int c = 0; c < 3; ++c)
+#pragma unroll
+            for (int d = 0; d < 3; ++d) tx[s][c][d] = u32x4{0, 0, 0, 0};
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const int t = base + 4 * (4 * s + g) + j - x0, k = t >= 0 && t < ksx ? kx[(long)x * ksx + t] : 0;
+            unsigned d[3];
+            sum_x += k;
+            tap_digits(k, d);
+#pragma unroll
+            for (int c = 0; c < 3; ++c)
+#pragma unroll
+                for (int e = 0; e < 3; ++e) tx[s][c][e][(3 * j + c) >> 2] |= d[e] << (8 * ((3 * j + c) & 3));
+        }
+    }
+    // vertical: lane = row li of the patch, source rows r0 + 16 g .. + 15
+    u32x4 ty[BP][3];
+    int start_y[BP];
+#pragma unroll
+    for (int pr = 0; pr < BP; ++pr) {
+        const int y = y_first + 14 * pr + li14, y0 = by[2 * y], n = by[2 * y + 1];
+        int sum = 0;
+#pragma unroll
+        for (int d = 0; d < 3; ++d) ty[pr][d] = u32x4{0, 0, 0, 0};
+#pragma unroll
+        for (int j = 0; j < 16; ++j) {
+            const int t = r0 + 16 * g + j - y0, k = t >= 0 && t < n ? ky[(long)y * ksy + t] : 0;
+            unsigned d[3];
+            sum += k;
+            tap_digits(k, d);
+#pragma unroll
+            for (int e = 0; e < 3; ++e) ty[pr][e][j >> 2] |= d[e] << (8 * (j & 3));
+        }
+        start_y[pr] = 128 * sum_groups(sum) + (1 << (PBITS - 1));
+    }
+    const int start_x = 128 * sum_groups(sum_x) + (1 << (PBITS - 1));
+
+    // The vertical product's rows are columns 0 .. 11 of the patch and 10 .. 13: a lane's four are neighbours in memory
+    const int wpr = gw / ms, px = g < 3 ? 4 * g : 10, xa = li < 12 ? li : li - 2;
+    const long frame = (long)gh * gw * 588;
+    TO* o[BP];
+#pragma unroll
+    for (int pr = 0; pr < BP; ++pr) {
+        const int prow = bd * BP + pr;
+        o[pr] = out + f0 * frame + (((prow / ms) * wpr + pcol / ms) * (ms * ms) + (prow % ms) * ms + pcol % ms) * 588l + li14 * 14 + px;
+    }
+    for (int f = f0; f < fend; ++f) {
+        u32x4 cur[RT][KS];
+#pragma unroll
+        for (int t = 0; t < RT; ++t)
+#pragma unroll
+            for (int s = 0; s < KS; ++s) {
+#pragma unroll
+                for (int w = 0; w < 3; ++w) cur[t][s][w] = __builtin_amdgcn_alignbyte(src[t][s][w + 1], src[t][s][w], shift[t]) ^ 0x80808080u;
+                cur[t][s][3] = 0;
+            }
+        if (f + 1 < fend) load(at_end && f + 1 == T - 1);
+#pragma unroll
+        for (int t = 0; t < RT; ++t) {
+#pragma unroll
+            for (int c = 0; c < 3; ++c) {
+                i32x4 acc[3] = {{start_x, start_x, start_x, start_x}, {0, 0, 0, 0}, {0, 0, 0, 0}};
+#pragma unroll
+                for (int s = 0; s < KS; ++s)
+#pragma unroll
+                    for (int d = 0; d < 3; ++d)
+                        acc[d] = __builtin_amdgcn_mfma_i32_16x16x64_i8(__builtin_bit_cast(i32x4, cur[t][s]), __builtin_bit_cast(i32x4, tx[s][c][d]), acc[d], 0, 0, 0);
+                *reinterpret_cast<unsigned*>(mid + (c * 16 + li) * MM_STRIDE + 16 * t + 4 * g) = four_bytes(acc) ^ 0x80808080u;
+            }
+        }
+        asm volatile("" ::: "memory");                             // (a wave's own LDS operations are in order)
+#pragma unroll
+        for (int c = 0; c < 3; ++c) {
+            const u32x4 a = *reinterpret_cast<const u32x4*>(mid + (c * 16 + xa) * MM_STRIDE + 16 * g);
+#pragma unroll
+            for (int pr = 0; pr < BP; ++pr) {
+                i32x4 acc[3] = {{start_y[pr], start_y[pr], start_y[pr], start_y[pr]}, {0, 0, 0, 0}, {0, 0, 0, 0}};
+#pragma unroll
+                for (int d = 0; d < 3; ++d)
+                    acc[d] = __builtin_amdgcn_mfma_i32_16x16x64_i8(__builtin_bit_cast(i32x4, a), __builtin_bit_cast(i32x4, ty[pr][d]), acc[d], 0, 0, 0);
+                // rescale + normalise through the host-built per-channel byte table (reference arithmetic, exact)
+                const unsigned b = four_bytes(acc);
+                float v[4];
+#pragma unroll
+                for (int r = 0; r < 4; ++r) v[r] = lut[c * 256 + (b >> (8 * r) & 255u)];
+                if constexpr (sizeof(TO) == 2) {
+                    const u32x2 w = {pack_bf2(v[0], v[1]), pack_bf2(v[2], v[3])};
+                    __builtin_memcpy(o[pr] + c * 196, &w, 8);
+                } else {
+                    __builtin_memcpy(o[pr] + c * 196, v, 16);
+                }
+            }
+        }
+        asm volatile("" ::: "memory");
+#pragma unroll
+        for (int pr = 0; pr < BP; ++pr) o[pr] += frame;
+    }
+}
+
+// pixels that a patch column's taps span (centres and a kernel's support, as for the bands' rows), rows that a band's do
+inline double tap_span(int in_size, int out_size, int outputs) {
+    const double scale = (double)in_size / out_size, wide = scale > 1.0 ? scale : 1.0;
+    return (outputs - 1) * scale + 4 * wide + 3;
+}
+// false: sizes this kernel does not take (columns above 48 source pixels or more than the row has, bands above 64 source rows)
+template <typename TO>
+bool launch_mfma(hipStream_t st, const uint8_t* frames, TO* out, int T, int H, int W, int th, int tw, int ms, const int* bx, const int* kx, int ksx,
+                 const int* by, const int* ky, int ksy, const float* table) {
+    const int gh = th / 14, gw = tw / 14;
+    const double px = tap_span(W, tw, 14);
+    const int steps = px <= 32 ? 2 : 3;
+    const int bp = steps == 2 && gh % 2 == 0 && tap_span(H, th, 28) <= MM_ROWS ? 2 : 1;       // (three steps leave no registers for two)
+    if (px > 48 || W < 16 * steps || tap_span(H, th, 14 * bp) > MM_ROWS) return false;
+    // frames in as many groups as give the shortest rounds of waves (two a SIMD); a wave's prologue costs one and a half frames
+    const long columns = (long)(gh / bp) * gw;
+    int each = T;
+    double best = 0;
+    for (int groups = 1; groups <= T && groups <= 64; ++groups) {
+        const int n = (T + groups - 1) / groups;
+        const double cost = (double)((columns * ((T + n - 1) / n) + MM_RESIDENT - 1) / MM_RESIDENT) * (n + 1.5);
+        if (groups == 1 || cost < best) { best = cost; each = n; }
+    }
+    const long units = columns * ((T + each - 1) / each), grid = (units + MM_WAVES - 1) / MM_WAVES;
+    if (grid > 0x7fffffff) return false;
+    const int tiles = (int)((tap_span(H, th, 14 * bp) + 15) / 16);
+#define COGS_MM(KS, BP, RT) hipLaunchKernelGGL((resize_mfma_kernel<TO, KS, BP, RT>), dim3((unsigned)grid), dim3(64 * MM_WAVES), 0, st, frames, out, T, H, W, gh, gw, ms, each, bx, kx, ksx, by, ky, ksy, table)
+    if (bp == 2) { if (tiles <= 3) COGS_MM(2, 2, 3); else COGS_MM(2, 2, 4); }
+    else if (steps == 2) { if (tiles <= 3) COGS_MM(2, 1, 3); else COGS_MM(2, 1, 4); }
+    else if (tiles <= 3) COGS_MM(3, 1, 3);
+    else COGS_MM(3, 1, 4);
+#undef COGS_MM
+    return true;
+}
+
 template <typename TO, int NG>
 void launch_fused(hipStream_t st, size_t lds, int grid, const uint8_t* frames, TO* out, int T, int H, int W, int gh, int gw, int ms, int band_p, int max_rows,
                   const int* bx, const int* kx, int ksx, const int* by, const int* ky, int ksy, const float* table) {
@@ -209,6 +446,10 @@ int cogs_k_preprocess(hipStream_t st, const uint8_t* frames, int T, int H, int W
         const size_t lds = 768 * 4 + (size_t)14 * band_p * (2 + ksy) * 4 + (size_t)3 * max_rows * TILE_C;
         const long grid = (long)T * (gh1 / band_p) * ((gw1 + TILE_P - 1) / TILE_P);
         const size_t pair = out_dtype == COGS_DT_BF16 ? 4 : 8;
+        if ((reinterpret_cast<size_t>(out) & (pair - 1)) == 0 &&
+            (out_dtype == COGS_DT_BF16 ? launch_mfma<bf16_t>(st, frames, (bf16_t*)out, T, H, W, th, tw, ms, bx, kx, ksx, by, ky, ksy, table)
+                                       : launch_mfma<float>(st, frames, (float*)out, T, H, W, th, tw, ms, bx, kx, ksx, by, ky, ksy, table)))
+            return COGS_LAUNCH_CHECK();
         if (lds <= 64 * 1024 && ksx <= 24 && (reinterpret_cast<size_t>(out) & (pair - 1)) == 0 && grid < 0x7fffffff) {
             if (out_dtype == COGS_DT_BF16)
                 dispatch_fused<bf16_t>(st, lds, (int)grid, frames, (bf16_t*)out, T, H, W, gh1, gw1, ms, band_p, max_rows, bx, kx, ksx, by, ky, ksy, table);

@@ -1150,6 +1150,19 @@ def test_fused_resize_equals_the_host_path(dev, t, h, w, merge, max_tokens, offs
         assert torch.equal(got["pixel_values"].cpu(), torch.from_numpy(ref["pixel_values"]).to(dtype))
 
 
+@pytest.mark.parametrize("t,h,w,merge,max_tokens,offset", [
+    (3, 70, 32, 1, 16384, 1),        # a row of exactly two steps of source bytes: the clip's last row is read byte by byte
+    (2, 57, 33, 1, 16384, 3),        # one pixel behind them
+    (2, 64, 34, 1, 16384, 2),        # two: whole words to the end
+    (3, 200, 300, 1, 90, 0),         # shrunk by about 1.8: three steps, bands of one patch
+    (70, 90, 120, 2, 2000, 1),       # frames in groups of several, the last one shorter
+    (1, 260, 90, 1, 40, 2),          # shrunk by about 1.7 one way, less the other
+])
+def test_resize_as_matrix_products_equals_the_host_path(dev, t, h, w, merge, max_tokens, offset):
+    """the sizes at which the matrix form's loads, steps and groups of frames change: the bytes of the host path"""
+    test_fused_resize_equals_the_host_path(dev, t, h, w, merge, max_tokens, offset)
+
+
 def test_tap_tables_outlive_their_place_in_the_cache(dev):
     """a resize queued on a side stream, and tables that leave the cache before it runs: their memory, asked for again on the stream that
     made them, is not theirs until the resize is done. (Zeros in it would be tables of no taps: a black clip, no read out of place)"""
