@@ -410,8 +410,14 @@ struct VitRange {
 // partly filled round of tiles). Same arithmetic per row, bit-identical tokens (tests/test_gpu_models.py). One rank's
 // share of a frame-sharded clip (8 frames of 22 x 42 patches: 145 tiles for the N = 1152 shapes) gains 10 %, the whole
 // 64-frame clip 2.7 % (round 4, same box, interleaved: 60.8 -> 59.2 ms; 256 frames at 140 x 280: 47.3 -> 46.5 ms).
+// Shorter clips run on one stream unless the caller has said how many: their products leave CUs idle anyway, which then fetch weights
+// ahead (gemm_mid.hip), one launch of twice the rows against two that share the chip. One stream / two, us, frames x patches:
+//   2 x 256 1722 / 1825, 4 x 256 2217 / 2308, 8 x 256 3206 / 3297, 16 x 256 4889 / 5178, 24 x 256 6453 / 6129, 32 x 256 8670 / 8002,
+//   2 x 924 2982 / 3378, 4 x 924 4881 / 5067, 6 x 924 6447 / 6330, 8 x 924 8803 / 7760, 12 x 924 11 179 / 11 254, 16 x 924 14 544 / 13 465
 // Not while the per-kernel profiler is on: overlapping launches stretch every bracket, so bench.py's `roofline` and
 // `breakdown_ms` describe the kernels one at a time. cogs_vit_set_streams(h, 1) or the debug switch vit_split_max switch it off.
+
+constexpr int64_t VIT_SPLIT_MIN = 5000;      // patches
 
 static cogs_status cogs_project_rows(cogs_handle h, hipStream_t st, const void* tokens, int M, void* out, void* ws);
 
@@ -443,7 +449,7 @@ static cogs_status vit_encode_impl(cogs_handle h, cogs_stream stream, const void
         return COGS_OK;
     };
     const int64_t split_max = g_cogs_debug.vit_split_max;
-    int S = h->vit_streams;
+    int S = h->vit_streams ? h->vit_streams : N >= VIT_SPLIT_MIN ? 2 : 1;
     if (S > nframes) S = (int)nframes;
     if (S < 2 || h->prof_on || attn_mode != COGS_ATTN_BLOCK_DIAG || N > split_max) return whole();
 
