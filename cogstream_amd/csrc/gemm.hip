@@ -1105,7 +1105,7 @@ void dispatch_f32(hipStream_t st, const GemmArgs& p, int grid, int mask, bool bi
 struct TileCost { int tile, tm, tn; float one, two, rest; };     // us; two = 0: one workgroup per CU
 static constexpr TileCost MID_TILES[] = {
     {1, 32, 64, 0.165f, 0.f, 1.8f},   {2, 64, 64, 0.218f, 0.409f, 1.8f}, {3, 128, 64, 0.309f, 0.637f, 2.3f}, {4, 128, 128, 0.387f, 0.f, 3.6f},
-    {5, 128, 256, 0.629f, 0.f, 4.8f}, {6, 128, 64, 0.292f, 0.f, 2.9f},   {7, 160, 64, 0.332f, 0.f, 3.8f}};
+    {5, 128, 256, 0.629f, 0.f, 4.8f}, {6, 128, 64, 0.292f, 0.f, 2.5f},   {7, 160, 64, 0.332f, 0.f, 3.8f}};
 static constexpr float PP_SLAB = 1.14f, PP_REST = 6.f, SECOND_LAUNCH = 2.f;
 
 static float tile_time(int tiles, int slabs, float one, float two, float rest) {

@@ -33,12 +33,13 @@ struct MidArgs {
     const char* W; long ldw;
     int M, N, KT;              // KT: 64-wide K slabs
     int nbm, nbn;              // tiles; workgroups past them are prefetch_weights
+    int group;                 // row tiles that share a panel of weights
     const float* ln_part; int ln_tiles; float ln_inv_h, ln_eps;     // EPI_LNFOLD: row statistics still in partial sums (or null)
     int ln_staged;             // a tile's fit a ring slot
     EpiArgs epi;
 };
 
-constexpr int ROW_BYTES = 128, MID_CUS = 256;
+constexpr int ROW_BYTES = 128, MID_CUS = 256, MAX_GROUP = 12;
 
 __device__ __forceinline__ void glds16(const char* g, char* l) {
     __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)g,
@@ -60,19 +61,35 @@ __device__ __forceinline__ void wait_slabs(int n) {
 
 // workgroups (a multiple of 8: as many on each XCD) behind those of the tiles: one dword of every weight line that the tiles of this
 // XCD read, slabs in order, so that the tiles' DMA finds them in L2. Nothing waits for them and nothing is kept.
-__device__ __forceinline__ void prefetch_weights(const MidArgs& p, char* smem, int tm_group, int TN, int waves, int wid, int lane) {
+__device__ __forceinline__ void prefetch_weights(const MidArgs& p, char* smem, int TM, int TN, int waves, int wid, int lane) {
     const int nb = p.nbm * p.nbn, xcd = blockIdx.x & 7, q = nb >> 3, r = nb & 7;
     const int x0 = xcd < r ? xcd * (q + 1) : r * (q + 1) + (xcd - r) * q, x1 = x0 + q + (xcd < r);
     const int of = ((int)gridDim.x - nb) >> 3, me = ((int)blockIdx.x - nb) >> 3;
-    const int per_group = tm_group * p.nbn;
-    for (int k = me * waves + wid; k < p.KT; k += of * waves) {
-        for (int t = x0; t < x1;) {                              // columns of each group of row tiles (usually one)
-            const int g0 = t / per_group * per_group, gsz = min(p.nbm - g0 / p.nbn, tm_group), e = min(x1, g0 + gsz * p.nbn);
-            const int lo = (t - g0) / gsz * TN, hi = min(((e - 1 - g0) / gsz + 1) * TN, p.N);
+    const int per_group = p.group * p.nbn;
+    auto columns = [&](int& t, int& lo, int& hi) {               // of the next group of row tiles (usually there is one)
+        const int g0 = t / per_group * per_group, gsz = min(p.nbm - g0 / p.nbn, p.group), e = min(x1, g0 + gsz * p.nbn);
+        lo = (t - g0) / gsz * TN;
+        hi = min(((e - 1 - g0) / gsz + 1) * TN, p.N);
+        t = e;
+    };
+    int cols = 0, lo, hi;
+    for (int t = x0; t < x1;) {
+        columns(t, lo, hi);
+        cols += hi - lo;
+    }
+    // A CU asks for missing lines at 55 to 60 B/ns and a tile takes in TM + TN rows of a slab at up to 110: where these workgroups have
+    // more columns than they can ask for in the tiles' time the launch would wait for them, so they take evenly spaced slabs, and none
+    // if that were less than half of them. 37 888 x 3584, M = 128 (a fifth): every slab 145 us, the fifth 75, none 68; 6176 x 2048,
+    // M = 1152 110 -> 32.5; 4608 x 3584, M = 1152 95 -> 46; where all can be had (3584 x 18 944, M = 621) 108, none 134.
+    const int slabs = (int)min((long)p.KT, (long)p.KT * of * (TM + TN) * 9 / (16L * max(cols, 1)));
+    if (2 * slabs < p.KT) return;
+    for (int j = me * waves + wid; j < slabs; j += of * waves) {
+        const int k = (int)((long)j * p.KT / slabs);
+        for (int t = x0; t < x1;) {
+            columns(t, lo, hi);
             for (int n = lo; n < hi; n += 64)
                 __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(p.W + (long)min(n + lane, hi - 1) * p.ldw + (long)k * ROW_BYTES),
                                                  (__attribute__((address_space(3))) void*)smem, 4, 0, 0);
-            t = e;
         }
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -82,26 +99,26 @@ __device__ __forceinline__ void prefetch_weights(const MidArgs& p, char* smem, i
 template <int EPI, int MI, int NI, int WM, int WN, int S, int WPE, int KS, bool IL>
 __global__ __launch_bounds__(64 * WM * WN, WPE) void gemm_mid_kernel(MidArgs p) {
     extern __shared__ __attribute__((aligned(16))) char smem[];
-    constexpr int TM = 16 * MI * WM, TN = 16 * NI * WN, WAVES = WM * WN, GROUP = 8;
+    constexpr int TM = 16 * MI * WM, TN = 16 * NI * WN, WAVES = WM * WN;
     constexpr int SUB = (TM + TN) * ROW_BYTES, SLAB = SUB * KS, P1 = SUB / 1024 / WAVES, P = P1 * KS;      // P: a wave's pieces per slot
     static_assert(SUB % (1024 * WAVES) == 0, "every wave stages the same number of pieces");
     const int lane = threadIdx.x & 63;
     const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int wm = wid / WN, wn = wid % WN;
     if ((int)blockIdx.x >= p.nbm * p.nbn) {
-        prefetch_weights(p, smem, GROUP, TN, WAVES, wid, lane);
+        prefetch_weights(p, smem, TM, TN, WAVES, wid, lane);
         return;
     }
     const int KT = (p.KT + KS - 1) / KS;                         // slots' worth
     const bool odd = KS == 2 && (p.KT & 1);                      // the last one holds one slab
 
-    // block -> tile: XCD-aware, then groups of 8 row tiles with the rows running fastest, so that the row tiles that share a
+    // block -> tile: XCD-aware, then groups of up to 12 row tiles with the rows running fastest, so that the row tiles that share a
     // panel of weights run on one XCD
     int m0, n0;
     {
         const int nb = p.nbm * p.nbn, xcd = blockIdx.x & 7, q = nb >> 3, r = nb & 7;
         const int bid = (xcd < r ? xcd * (q + 1) : r * (q + 1) + (xcd - r) * q) + (blockIdx.x >> 3);
-        const int per_group = GROUP * p.nbn, first_m = bid / per_group * GROUP, gsz = min(p.nbm - first_m, GROUP);
+        const int per_group = p.group * p.nbn, first_m = bid / per_group * p.group, gsz = min(p.nbm - first_m, p.group);
         m0 = (first_m + (bid % per_group) % gsz) * TM;
         n0 = ((bid % per_group) / gsz) * TN;
     }
@@ -319,6 +336,10 @@ void launch(hipStream_t st, MidArgs& p, bool alone) {
     cogs_ensure_dyn_lds((const void*)gemm_mid_kernel<EPI, MI, NI, WM, WN, S, WPE, KS, IL>, lds, attr_done);
     p.nbm = (p.M + TM - 1) / TM;
     p.nbn = (p.N + TN - 1) / TN;
+    // groups of row tiles as equal as they come: one row tile left over read every weight for itself, 9 row tiles of 1152 x 3456 x 1152
+    // 69.6 us (with its XCD's prefetch, below) against 14.1 in one group
+    const int groups = (p.nbm + MAX_GROUP - 1) / MAX_GROUP;
+    p.group = (p.nbm + groups - 1) / groups;
     p.ln_staged = (long)TM * p.ln_tiles * 8 <= KS * (TM + TN) * ROW_BYTES && ((long)p.M * p.ln_tiles) % 2 == 0;
     // CUs without a tile: up to four workgroups an XCD prefetch (one image 1561 us without, 1494 with two an XCD, 1371 with four, 1374 with eight)
     const int tiles = p.nbm * p.nbn, left = alone ? (MID_CUS - tiles) / 8 * 8 : 0;

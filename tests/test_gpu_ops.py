@@ -1052,6 +1052,22 @@ def test_attention_head_major_inputs_equal_token_major_bit_for_bit(dev, heads, l
     assert torch.equal(outg, tok), "guard rows behind a head's rows were read: %g" % float((outg.float() - tok.float()).abs().max())
 
 
+@pytest.mark.parametrize("tile", [1, 2, 3, 4, 5, 6, 7])
+@pytest.mark.parametrize("M,N,K", [(1147, 328, 192), (1537, 1544, 128), (100, 9000, 640)])
+def test_mid_size_gemm_groups_of_row_tiles(dev, tile, M, N, K):
+    """gemm_mid.hip: row tiles in groups of up to twelve, as equal as they come (9, 10 and 13 tiles of 128 rows, 8 to 49 of the other
+    heights, a shorter last group), with all, some and none of the weights fetched ahead by the workgroups behind the tiles'. Against
+    float64: half a bf16 step of the value and 2^-20 of the sum of |a||w| for fp32 sums of up to 640 products."""
+    from cogstream_amd import _lib as L2
+    ops = _ops()
+    g = torch.Generator(device=dev).manual_seed(M + tile)
+    a, w = (torch.randn(*s, generator=g, device=dev).bfloat16() for s in ((M, K), (N, K)))
+    with L2.debug_switch("gemm_mid", tile):
+        got = ops.gemm(a, w).double()
+    want, size = a.double() @ w.double().t(), a.double().abs() @ w.double().abs().t()
+    assert bool(((got - want).abs() <= want.abs() * 2.0 ** -8 + size * 2.0 ** -20).all())
+
+
 @pytest.mark.parametrize("tile", [1, 2, 3, 4, 5])
 def test_mid_size_gemm_tiles_equal_each_other_and_fp64(dev, tile):
     """gemm_mid.hip: every tile size, forced, at the edges of its tiles (rows and columns one short of and past a tile, a ragged
