@@ -412,12 +412,14 @@ struct VitRange {
 // 64-frame clip 2.7 % (round 4, same box, interleaved: 60.8 -> 59.2 ms; 256 frames at 140 x 280: 47.3 -> 46.5 ms).
 // Shorter clips run on one stream unless the caller has said how many: their products leave CUs idle anyway, which then fetch weights
 // ahead (gemm_mid.hip), one launch of twice the rows against two that share the chip. One stream / two, us, frames x patches:
-//   2 x 256 1722 / 1825, 4 x 256 2217 / 2308, 8 x 256 3206 / 3297, 16 x 256 4889 / 5178, 24 x 256 6453 / 6129, 32 x 256 8670 / 8002,
-//   2 x 924 2982 / 3378, 4 x 924 4881 / 5067, 6 x 924 6447 / 6330, 8 x 924 8803 / 7760, 12 x 924 11 179 / 11 254, 16 x 924 14 544 / 13 465
+//   8 x 256 3198 / 3314, 12 x 256 3776 / 4428, 18 x 256 5258 / 5395, 20 x 256 5767 / 5454, 2 x 924 3066 / 3355, 4 x 924 4924 / 5333,
+//   5 x 924 5853 / 5967, 6 x 924 6469 / 6366, 2 x 1200 4065 / 4094, 3 x 1200 4952 / 5189, 4 x 1200 6159 / 5926, 5 x 1200 7303 / 6799,
+//   2 x 1600 4495 / 4882, 3 x 1600 6456 / 5967, 8 x 576 5355 / 5397, 9 x 576 5939 / 5979, 2 x 1936 5563 / 5689, 3 x 1936 7628 / 7410,
+//   16 x 924 14 544 / 13 465
 // Not while the per-kernel profiler is on: overlapping launches stretch every bracket, so bench.py's `roofline` and
 // `breakdown_ms` describe the kernels one at a time. cogs_vit_set_streams(h, 1) or the debug switch vit_split_max switch it off.
 
-constexpr int64_t VIT_SPLIT_MIN = 5000;      // patches
+constexpr int64_t VIT_SPLIT_MIN = 4700;      // patches
 
 static cogs_status cogs_project_rows(cogs_handle h, hipStream_t st, const void* tokens, int M, void* out, void* ws);
 
