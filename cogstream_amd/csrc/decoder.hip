@@ -152,6 +152,23 @@ struct Step {
         return cogs_k_gemm_skinny(st, g, k.ypart);
     }
 
+    // the next product's weights, for the mix of streams in front of it
+    CogsAhead ahead(const void* W, int M, int N) const {
+        return d.w.dtype == COGS_DT_BF16 && d.w.streams > 0 ? cogs_k_gemm_skinny_ahead(W, d.wp, M, N, d.wp) : CogsAhead();
+    }
+    CogsAhead ahead_mixer(int l) const {
+        switch (d.layers[l].mixer) {
+            case COGS_MIX_ATTENTION: return ahead(d.layers[l].attn.in_w, S, d.geom[l].att.ldt);
+            case COGS_MIX_DELTA: return ahead(d.layers[l].delta.in_w, S, d.geom[l].del.ldt);
+            default: return ahead(d.layers[l].latent.in_w, S, d.geom[l].lat.ldt);
+        }
+    }
+    CogsAhead ahead_mlp(int l) const {
+        const cogs_decoder_mlp& m = d.layers[l].mlp;
+        const int ffp = up(m.ff, 64);
+        return ahead(m.up_w, S, m.act == COGS_ACT_SWIGLU ? 2 * ffp : ffp);
+    }
+
     int latent_attention(const Run& run) {
         const cogs_latent_mixer& m = d.layers[run.layer].latent;
         const LatentGeom& G = d.geom[run.layer].lat;
@@ -303,8 +320,9 @@ struct Step {
     }
 
     // x from the embeddings, or x += norm(y) through the sublayer's (`from`) hyper-connections; then h = norm of what `to` reads
-    int stream(const void* embeds, const float* y_gamma, const cogs_hyper* from, const cogs_hyper* to, const float* out_gamma, float* sum) {
+    int stream(const void* embeds, const float* y_gamma, const cogs_hyper* from, const cogs_hyper* to, const float* out_gamma, float* sum, const CogsAhead& next) {
         CogsStreamNorm a;
+        a.ahead = next;
         a.x = k.x; a.embeds = embeds; a.y = embeds ? nullptr : y_parts ? (const void*)k.ypart : k.y; a.y_parts = embeds ? 0 : y_parts; a.y_gamma = y_gamma; a.out = out_gamma ? k.h : nullptr; a.out_gamma = out_gamma;
         a.rows = S; a.H = d.w.width; a.Hp = d.wp; a.eps = d.w.eps;
         if (embeds) { a.embed_scale = d.w.embed_scale; a.pos = d.w.pos; a.rowpos = k.rowpos; }
@@ -499,7 +517,7 @@ cogs_status cogs_decoder_forward(cogs_handle h, cogs_stream stream, const void* 
         if (!d.sets.empty()) COGS_TRY(cogs_k_rope_sets(st, k.rope, d.sets_dev, (int)d.sets.size(), d.max_pairs, k.rowpos, S));
         if (d.att_tail) COGS_TRY(cogs_k_zero(st, k.att, align_up((size_t)S * d.max_o * esize(d.w.dtype))));
     }
-    COGS_TRY(s.stream(embeds, nullptr, nullptr, &d.layers[0].hyper1, d.layers[0].norm1, nullptr));
+    COGS_TRY(s.stream(embeds, nullptr, nullptr, &d.layers[0].hyper1, d.layers[0].norm1, nullptr, s.ahead_mixer(d.runs[0].layer)));
     for (size_t r = 0; r < d.runs.size(); ++r) {
         const cogs_decoder_layer& L = d.layers[d.runs[r].layer];
         const cogs_decoder_layer* next = r + 1 < d.runs.size() ? &d.layers[d.runs[r + 1].layer] : nullptr;
@@ -508,17 +526,18 @@ cogs_status cogs_decoder_forward(cogs_handle h, cogs_stream stream, const void* 
         const cogs_hyper* from = &L.hyper1;
         const float* gamma = L.norm1b;
         if (L.mlp.ff > 0) {
-            COGS_TRY(s.stream(nullptr, L.norm1b, &L.hyper1, &L.hyper2, L.norm2, nullptr));
+            COGS_TRY(s.stream(nullptr, L.norm1b, &L.hyper1, &L.hyper2, L.norm2, nullptr, s.ahead_mlp(d.runs[r].layer)));
             COGS_TRY(s.mlp(d.runs[r].layer));
             from = &L.hyper2;
             gamma = L.norm2b;
         }
-        COGS_TRY(s.stream(nullptr, gamma, from, next ? &next->hyper1 : nullptr, next ? next->norm1 : nullptr, sum));
+        COGS_TRY(s.stream(nullptr, gamma, from, next ? &next->hyper1 : nullptr, next ? next->norm1 : nullptr, sum, next ? s.ahead_mixer(d.runs[r + 1].layer) : CogsAhead()));
     }
     for (int i = 0; i < nseq; ++i) kv[i]->len += lens[i];
     if (n_want > 0) {
         CogsStreamNorm a;
         a.x = k.x; a.streams = d.w.streams; a.out = k.hn; a.out_gamma = d.w.final_norm; a.pick = k.want; a.rows = n_want; a.H = d.w.width; a.Hp = d.wp; a.eps = d.w.eps;
+        a.ahead = s.ahead(d.w.head, n_want, d.vocabp);
         { PROF(COGS_PROF_NORM); COGS_TRY(cogs_k_stream_norm(st, d.w.dtype, a)); }
         CogsGemm g;
         g.A = k.hn; g.lda = d.wp; g.W = d.w.head; g.ldw = d.wp; g.C = logits; g.ldc = d.vocabp; g.M = n_want; g.N = d.vocabp; g.K = d.wp; g.out_f32 = 1;

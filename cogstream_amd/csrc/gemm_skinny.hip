@@ -154,6 +154,9 @@ void launch_cols(hipStream_t st, const SkinnyArgs& p, int cols, int splits) {
     else launch<MT, 1, 4, MT == 1 ? 4 : MT == 2 ? 3 : 2>(st, p, splits);
 }
 
+// columns per workgroup of a product without partial sums
+int whole_cols(int N) { return N >= 64 * 160 ? 64 : N >= 32 * 160 ? 32 : 16; }
+
 }  // namespace
 
 bool cogs_k_gemm_skinny_fits(const CogsGemm& g) {
@@ -169,6 +172,22 @@ int cogs_k_gemm_skinny_parts(int M, int N, int K) {
     return N <= 2048 ? 8 : 4;
 }
 
+// how much of the next product's weights a mix of 4 us reads on idle CUs: what HBM gives meanwhile, or the mix takes the longer. Widths of 2048, 3 rows
+// stepped 24 times: none 11.57 ms, 5 MB 11.04, 8 MB 11.00, 12 MB 11.05, 18 MB 11.20, 40 MB 12.19; 8 rows 12.43 -> 12.06 with 8 MB; width
+// 3584, 16 rows, 12 steps 8.51 -> 8.36. (Norms of one stream are shorter and gained nothing.)
+constexpr long AHEAD_BYTES = 8000000;
+
+CogsAhead cogs_k_gemm_skinny_ahead(const void* W, long ldw, int M, int N, int K) {
+    CogsAhead a;
+    CogsGemm g;
+    g.dtype = COGS_DT_BF16; g.M = M; g.N = N; g.K = K; g.lda = K; g.ldw = ldw;
+    if (!W || g_cogs_debug.gemm_skinny == 0 || !cogs_k_gemm_skinny_fits(g)) return a;
+    const long lines = AHEAD_BYTES / (128L * N);
+    a.W = (const char*)W; a.ldw = ldw * 2; a.N = N; a.cols = whole_cols(N); a.groups = (N + a.cols - 1) / a.cols;
+    a.lines = (int)(lines < K / 64 ? lines : K / 64);
+    return a;
+}
+
 int cogs_k_gemm_skinny(hipStream_t st, const CogsGemm& g, float* part) {
     if (!cogs_k_gemm_skinny_fits(g)) return COGS_E_UNSUPPORTED;
     SkinnyArgs p;
@@ -179,7 +198,7 @@ int cogs_k_gemm_skinny(hipStream_t st, const CogsGemm& g, float* part) {
     g_cogs_debug.gemm_last_body = 7;
     const int parts = part ? cogs_k_gemm_skinny_parts(g.M, g.N, g.K) : 1;
     if (part && (g.act != COGS_ACT_NONE || g.residual || g.rope_cos || g.out_f32 || parts < 2)) return COGS_E_UNSUPPORTED;
-    const int cols = parts > 1 ? (g.K >= 4096 ? 64 : g.M <= 16 ? 16 : 32) : g.N >= 64 * 160 ? 64 : g.N >= 32 * 160 ? 32 : 16;
+    const int cols = parts > 1 ? (g.K >= 4096 ? 64 : g.M <= 16 ? 16 : 32) : whole_cols(g.N);
     if (g.M <= 16) launch_cols<1>(st, p, cols, parts);
     else if (g.M <= 32) launch_cols<2>(st, p, cols, parts);
     else launch_cols<4>(st, p, cols, parts);

@@ -81,6 +81,10 @@ struct CogsAttn {
 int cogs_k_attention_vit(hipStream_t st, const struct CogsAttn& a);   // attn_vit.hip: block-diagonal, hd 72, pre-scaled Q
 int cogs_k_attention_decode(hipStream_t st, const struct CogsAttn& a, float* part_o, float* part_ml);   // attn_decode.hip: one query row, hd 128, key-split partials
 int cogs_k_attention(hipStream_t st, const CogsAttn& a);
+// weights of a few-row GEMM that is launched next: a kernel of few workgroups reads the first `lines` 128-byte lines of every row into the
+// L2 caches on CUs it leaves idle (norm.hip, read_ahead). lines = 0: nothing to read
+struct CogsAhead { const char* W = nullptr; long ldw = 0; int N = 0, cols = 0, groups = 0, lines = 0; };
+CogsAhead cogs_k_gemm_skinny_ahead(const void* W, long ldw, int M, int N, int K);       // bf16, ldw in elements
 // few-row GEMM (gemm_skinny.hip): bf16, 2 <= M <= 64; opt-in per call site (its summation order differs from cogs_k_gemm's)
 bool cogs_k_gemm_skinny_fits(const CogsGemm& g);
 #define COGS_SKINNY_MAX_PARTS 8
@@ -197,6 +201,7 @@ struct CogsStreamNorm {
     int rows = 0, H = 0, Hp = 0; float eps = 0.f;
     float embed_scale = 1.f; const void* pos = nullptr; const int* rowpos = nullptr;
     int streams = 0; const float *mix = nullptr, *out_w = nullptr, *in_w = nullptr; float* sum = nullptr;
+    CogsAhead ahead;           // read beside hyper-connected streams of few rows (a workgroup of 1024 threads each), ignored elsewhere
 };
 int cogs_k_stream_norm(hipStream_t st, int dtype, const CogsStreamNorm& a);
 int cogs_k_zero(hipStream_t st, void* p, size_t bytes);      // 16-byte multiples

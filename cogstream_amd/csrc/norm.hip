@@ -305,10 +305,35 @@ __global__ __launch_bounds__(TPB) void stream_norm_kernel(CogsStreamNorm p) {
     }
 }
 
+// Workgroups behind those of a mix of few rows: lines of the next product's weights into the L2 caches (kernels.h, CogsAhead). Such a mix is 4 us
+// of latency on as many CUs as it has rows while HBM, which bounds the few-row product behind it (8 x 8192 x 2048: 8.0 us, 4.6 from L2), is
+// idle. Workgroup i runs on XCD i % 8, here and there, so each reads the lines of the column groups that its own XCD will want. How many:
+// cogs_k_gemm_skinny_ahead.
+constexpr int AHEAD_CUS = 256;
+
+int ahead_workgroups(const CogsAhead& p, int rows) { return p.lines > 0 && rows < AHEAD_CUS ? (AHEAD_CUS - rows) / 8 * 8 : 0; }
+
+__device__ __forceinline__ void read_ahead(const CogsAhead& p, int rows) {
+    const int xcd = blockIdx.x & 7, me = ((int)blockIdx.x - rows) >> 3, of = ((int)gridDim.x - rows) >> 3;
+    const int total = ((p.groups - xcd + 7) >> 3) * p.cols * p.lines, step = of * (int)blockDim.x;
+    for (int t = me * (int)blockDim.x + (int)threadIdx.x; t < total; t += step) {
+        const int row = t / p.lines, n = ((row / p.cols) * 8 + xcd) * p.cols + row % p.cols;
+        if (n >= p.N) continue;
+        const int v = *reinterpret_cast<const int*>(p.W + n * p.ldw + (long)(t - row * p.lines) * 128);
+        asm volatile("" ::"v"(v));
+    }
+}
+
 // the same with a scaled embedding and a position table at the start and hyper-connected streams (x [row][stream][Hp]). NS: streams
 // rounded up; a chunk's old streams are in registers together, only the combination that is normed stays there for the row.
 template <typename T, int C, int TPB, int NS, bool PARTS>
 __global__ __launch_bounds__(TPB) void stream_mix_kernel(CogsStreamNorm p) {
+    if constexpr (TPB == 1024) {
+        if ((int)blockIdx.x >= p.rows) {
+            read_ahead(p.ahead, p.rows);
+            return;
+        }
+    }
     constexpr int NW = TPB / 64;
     __shared__ float red[2][NW];
     const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
@@ -430,12 +455,12 @@ __global__ __launch_bounds__(TPB) void stream_mix_kernel(CogsStreamNorm p) {
 
 template <typename T, int NS>
 int launch_stream_mix(hipStream_t st, const CogsStreamNorm& a) {
-    const dim3 grid(a.rows);
-#define COGS_STREAM(C, TPB) hipLaunchKernelGGL((stream_mix_kernel<T, C, TPB, NS, false>), grid, dim3(TPB), 0, st, a)
+    const int rows = a.rows, more = ahead_workgroups(a.ahead, rows);
+#define COGS_STREAM(C, TPB) hipLaunchKernelGGL((stream_mix_kernel<T, C, TPB, NS, false>), dim3(rows + (TPB == 1024 ? more : 0)), dim3(TPB), 0, st, a)
 // (partial sums come of products of at most 64 rows)
 #define COGS_STREAM_FEW(C, TPB)                                                                                                     \
     do {                                                                                                                            \
-        if (a.y_parts > 0) hipLaunchKernelGGL((stream_mix_kernel<T, C, TPB, NS, true>), grid, dim3(TPB), 0, st, a);                 \
+        if (a.y_parts > 0) hipLaunchKernelGGL((stream_mix_kernel<T, C, TPB, NS, true>), dim3(rows + (TPB == 1024 ? more : 0)), dim3(TPB), 0, st, a); \
         else COGS_STREAM(C, TPB);                                                                                                   \
     } while (0)
     if (a.rows <= 64 && a.Hp > 1024) {

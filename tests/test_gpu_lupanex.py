@@ -412,6 +412,18 @@ def test_one_token_delta_rule_at_the_edges_of_its_kernels(dev, dim, vdim, conv):
             assert rms_err(run(e, toks, range(first, 24), reserve=8), lg) < TOL[dtype], (dtype, first)
 
 
+@pytest.mark.parametrize("rows", [2, 7, 64])
+@pytest.mark.parametrize("width,ff,vocab", [(1100, 200, 61), (1408, 10300, 40003)])
+def test_weights_read_beside_a_mix_of_streams(dev, rows, width, ff, vocab):
+    """all lines of the next product's rows and some of them (one of 22 of the head's); fewer column groups than XCDs, and numbers of them that
+    8 does not divide"""
+    cfg = config([attention(heads=4, kv_heads=2, dim=32, vdim=40)], width=width, ff=ff, vocab=vocab, streams=4)
+    st = state(cfg)
+    toks = tokens(cfg, rows)
+    got = run(engine(cfg, st, torch.bfloat16), toks)
+    assert rms_err(got, lo.forward(cfg, double(st), toks)[0]) < TOL[torch.bfloat16]
+
+
 @pytest.mark.parametrize("dim,vdim", [(16, 16), (64, 48), (80, 16), (128, 128), (144, 32), (256, 16)])
 def test_chunked_delta_rule_at_the_edges_of_its_tiles(dev, dim, vdim):
     """every number of row tiles per wave, whole and ragged; chunks of one token, whole and ragged ones, one to four of them, from nothing
