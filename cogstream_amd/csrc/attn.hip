@@ -22,7 +22,6 @@
 #include "common.h"
 #include "kernels.h"
 #include "debug.h"
-#include <stdlib.h>
 #include <type_traits>
 
 namespace {
@@ -546,11 +545,11 @@ __device__ __forceinline__ int v_swz(int row) { return ((row & 3) | (((row >> 3)
 // would take 0.75 ms -- the two ADD: SQ_VALU_MFMA_BUSY_CYCLES + the VALU's active cycles are ~95 % of the resident time,
 // bank conflicts 0, LDS array 21 % busy, 2.4 % of wave time waiting for LDS.
 constexpr float PREFILL_THR = 6.f;
-// PRIO: the wave-priority scheme (debug switch attn_prio) as a compile-time choice -- 2 = raised in the softmax phase (shipped), -1 =
+// NQ: 16-row query groups per wave. PRIO: the wave-priority scheme (debug switch attn_prio) as a compile-time choice -- 2 = raised in the softmax phase (shipped), -1 =
 // read p.prio_mode at run time (A/B runs: four s_cmp / s_cbranch pairs per tile, next to the MFMA blocks)
-template <int DEEP, int PRIO = -1>
+template <int DEEP, int PRIO = -1, int NQ = 2>
 __global__ __launch_bounds__(256, 2) void attn_prefill_dma_kernel(AttnArgs p) {
-    constexpr int HD = 128, NQ = 2, NT = 256, KS = 4, DT = 8;
+    constexpr int HD = 128, NT = 256, KS = 4, DT = 8, TQ = 64 * NQ;
     constexpr int K_LDS = 64 * 256, V_LDS = 64 * 256, BUF = K_LDS + V_LDS;     // 32 KiB per tile
     __shared__ __attribute__((aligned(16))) char smem[2 * BUF];
 
@@ -564,7 +563,7 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_dma_kernel(AttnArgs p) {
     int qs = 0, qe = p.q_len, ks = 0, ke = p.kv_len;
     if (p.cu) { qs = p.cu[seg]; qe = p.cu[seg + 1]; ks = qs; ke = qe; }
     const int qt = p.heavy_first ? (int)gridDim.x - 1 - (int)blockIdx.x : (int)blockIdx.x;
-    const int q0 = qs + qt * 128;
+    const int q0 = qs + qt * TQ;
     if (q0 >= qe) return;
 
     const bf16_t* Qp = reinterpret_cast<const bf16_t*>(p.Q);
@@ -576,7 +575,7 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_dma_kernel(AttnArgs p) {
     bool qok[NQ];
 #pragma unroll
     for (int qi = 0; qi < NQ; ++qi) {
-        qrow[qi] = q0 + wid * 32 + qi * 16 + li;
+        qrow[qi] = q0 + wid * 16 * NQ + qi * 16 + li;
         qok[qi] = qrow[qi] < qe;
 #pragma unroll
         for (int s = 0; s < KS; ++s) {
@@ -585,7 +584,7 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_dma_kernel(AttnArgs p) {
             qf[qi][s] = __builtin_bit_cast(bf16x8, v);
         }
     }
-    const int kend = min(ke, ks + (q0 - qs) + 127 + p.q_pos0 + 1);      // causal
+    const int kend = min(ke, ks + (q0 - qs) + TQ - 1 + p.q_pos0 + 1);      // causal
     const int nt = (kend - ks + 63) / 64;
 
     f32x4 oacc[DT][NQ];
@@ -648,7 +647,7 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_dma_kernel(AttnArgs p) {
     const int v_base = vr * 256 + ((li & 3) & 1) * 8;   // + 32u*256 (+4*256) + (((2d + ((li&3)>>1)) ^ v_sw) << 4)
     const int v_ch = (li & 3) >> 1;
 
-    const bool wave_active = q0 + wid * 32 < qe;
+    const bool wave_active = q0 + wid * 16 * NQ < qe;
 
     // first_tag: the wave's first tile (kt == 0: it subtracts its own maximum explicitly) -- a compile-time copy, so that the
     // other tiles carry no `first tile?` test (DEEP only; the round-4 form keeps the run-time flag)
@@ -689,14 +688,14 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_dma_kernel(AttnArgs p) {
             }
         }
         #if !defined(PF_ABL_NOQK) && !defined(PF_ABL_NOPV)
-        if constexpr (DEEP && !MASKED) {          // 16 reads, 32 MFMAs: 6 reads, then a read per pair of MFMAs
+        if constexpr (DEEP && !MASKED) {          // 16 reads, 16 NQ MFMAs: 6 reads, then a read per NQ MFMAs
             __builtin_amdgcn_sched_group_barrier(0x100, 6, 0);
 #pragma unroll
             for (int i = 0; i < 10; ++i) {
-                __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);
+                __builtin_amdgcn_sched_group_barrier(0x008, NQ, 0);
                 __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
             }
-            __builtin_amdgcn_sched_group_barrier(0x008, 12, 0);
+            __builtin_amdgcn_sched_group_barrier(0x008, 6 * NQ, 0);
         }
 #endif
         { const int pm = PRIO >= 0 ? PRIO : p.prio_mode; if (pm == 1) __builtin_amdgcn_s_setprio(0); else if (pm == 2) __builtin_amdgcn_s_setprio(1); }
@@ -816,14 +815,14 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_dma_kernel(AttnArgs p) {
             }
         }
         #if !defined(PF_ABL_NOQK) && !defined(PF_ABL_NOPV)
-        if constexpr (DEEP && !MASKED) {          // 32 transposed reads, 32 MFMAs: 8 reads lead (beside the exponentials)
+        if constexpr (DEEP && !MASKED) {          // 32 transposed reads, 16 NQ MFMAs: 8 reads lead (beside the exponentials)
             __builtin_amdgcn_sched_group_barrier(0x100, 8, 0);
 #pragma unroll
             for (int i = 0; i < 6; ++i) {
-                __builtin_amdgcn_sched_group_barrier(0x008, 4, 0);
+                __builtin_amdgcn_sched_group_barrier(0x008, 2 * NQ, 0);
                 __builtin_amdgcn_sched_group_barrier(0x100, 4, 0);
             }
-            __builtin_amdgcn_sched_group_barrier(0x008, 8, 0);
+            __builtin_amdgcn_sched_group_barrier(0x008, 4 * NQ, 0);
         }
 #endif
         if constexpr (!DEEP) {        // the deferred factor exists in the round-4 form only
@@ -1146,7 +1145,13 @@ int cogs_k_attention(hipStream_t st, const CogsAttn& a) {
             // (two more forms were built, tested at full size and measured slower -- a ping-pong form, 1.89 vs 1.81-1.86 ms per layer
             // at 15 395 tokens, and 64 query rows per wave, 2.94 vs 1.97 ms: tools/experiments/attn_prefill_variants.hip)
             g_cogs_debug.attn_last_kernel = 5;
-            if (g_cogs_debug.attn_prefill_deep && p.prio_mode == 2) hipLaunchKernelGGL((attn_prefill_dma_kernel<1, 2>), grid, dim3(256), 0, st, p);
+            // 64 query rows a workgroup where 128 leave CUs idle, or not many more than one to each: same bits, half the work in a key
+            // tile's chain. 28 heads, 128 rows a workgroup / 64, us: 100 rows 9.0 / 5.6, 256 12.2 / 7.9, 512 17.7 / 11.7, 621 19.9 / 15.8, 900
+            // 25.8 / 21.5, 1280 (280 workgroups) 39.1 / 32.2, 1600 (364) 45.6 / 44.4, 2048 (448) 60.9 / 78.1
+            const bool narrow = g_cogs_debug.attn_prefill_deep && p.prio_mode == 2 && (long)grid.x * grid.y * grid.z <= 320;
+            if (narrow)
+                hipLaunchKernelGGL((attn_prefill_dma_kernel<1, 2, 1>), dim3((max_len + 63) / 64, grid.y, grid.z), dim3(256), 0, st, p);
+            else if (g_cogs_debug.attn_prefill_deep && p.prio_mode == 2) hipLaunchKernelGGL((attn_prefill_dma_kernel<1, 2>), grid, dim3(256), 0, st, p);
             else if (g_cogs_debug.attn_prefill_deep) hipLaunchKernelGGL((attn_prefill_dma_kernel<1, -1>), grid, dim3(256), 0, st, p);
             else hipLaunchKernelGGL((attn_prefill_dma_kernel<0, -1>), grid, dim3(256), 0, st, p);
         } else if (a.head_dim == 128 && a.q_len == 1 && p.nsplit > 1 && p.gqa_pack && pre && !env_old_dec) {

@@ -1052,6 +1052,35 @@ def test_attention_head_major_inputs_equal_token_major_bit_for_bit(dev, heads, l
     assert torch.equal(outg, tok), "guard rows behind a head's rows were read: %g" % float((outg.float() - tok.float()).abs().max())
 
 
+@pytest.mark.parametrize("lens,hq,hkv,pos0", [((1,), 4, 2, 3), ((63,), 28, 4, 0), ((65,), 28, 4, 64), ((127,), 4, 4, 1), ((129,), 28, 4, 500), ((320,), 8, 1, 0),
+                                              ((621,), 28, 4, 0), ((1, 64, 130, 7), 4, 2, 0)])
+def test_prompt_attention_of_64_row_workgroups(dev, lens, hq, hkv, pos0):
+    """attn.hip, prompt kernel: query tiles of 64 rows (few of them) and of 128 (attn_prio 1 keeps to those) give the same bits, at the edges of
+    both and of key tiles, behind kept keys, and in segments; and the float64 result within the weights' and the output's bf16 rounding
+    (2^-8 each, of values up to the largest |v|)"""
+    from cogstream_amd import _lib as L2
+    ops = _ops()
+    g = torch.Generator(device=dev).manual_seed(sum(lens) + pos0)
+    n = sum(lens)
+    q = torch.randn(n, hq * 128, generator=g, device=dev).bfloat16() * 0.2
+    k, v = (torch.randn(n + pos0, hkv * 128, generator=g, device=dev).bfloat16() for _ in range(2))
+    kw = dict(hq=hq, hkv=hkv, head_dim=128, causal=True, q_prescaled=True, q_pos0=pos0)
+    if len(lens) > 1:
+        kw["cu_seqlens"] = torch.tensor([0, *torch.tensor(lens).cumsum(0).tolist()], dtype=torch.int32, device=dev)
+        kw["max_seqlen"] = max(lens)
+    got = ops.attention(q, k, v, **kw)
+    with L2.debug_switch("attn_prio", 1):
+        assert torch.equal(got, ops.attention(q, k, v, **kw))
+    at = 0
+    for m in lens:
+        K, V = (t[at:at + m + pos0].double().view(m + pos0, hkv, 128).repeat_interleave(hq // hkv, 1) for t in (k, v))
+        s = (q[at:at + m].double().view(m, hq, 128).transpose(0, 1) @ K.permute(1, 2, 0).contiguous()) * math.log(2.0)
+        s = s.masked_fill(torch.arange(m + pos0, device=dev)[None, None] > torch.arange(m, device=dev)[None, :, None] + pos0, -math.inf)
+        want = (s.softmax(-1) @ V.transpose(0, 1).contiguous()).transpose(0, 1).reshape(m, hq * 128)
+        assert float((got[at:at + m].double() - want).abs().max()) <= float(V.abs().max()) * 2.0 ** -7
+        at += m
+
+
 @pytest.mark.parametrize("tile", [1, 2, 3, 4, 5, 6, 7])
 @pytest.mark.parametrize("M,N,K", [(1147, 328, 192), (1537, 1544, 128), (100, 9000, 640)])
 def test_mid_size_gemm_groups_of_row_tiles(dev, tile, M, N, K):
