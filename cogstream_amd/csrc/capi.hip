@@ -923,7 +923,7 @@ static cogs_status llm_forward_impl(cogs_handle h, cogs_stream stream, const voi
             g.rope_cos = rc; g.rope_sin = rs; g.rope_cols = qd_q + kvd; g.head_dim = hd;
             if (prescale_q) { g.q_scale = scale * 1.4426950408889634f; g.q_cols = qd_q; }
             if (fuse_norm) { g.rms_gamma = L.in_ln; g.rms_eps = w.rms_eps; }
-            if (kv && S == 1) {   // single-token decode: the GEMV writes the new K / V row straight into the cache
+            if (kv) {             // new K / V rows go straight into the cache (or through C where the product's kernel cannot)
                 g.kv_k = (char*)kv->k + (((size_t)l * kv->max_len) + pos0) * kvd * es;
                 g.kv_v = (char*)kv->v + (((size_t)l * kv->max_len) + pos0) * kvd * es;
                 g.kv_col0 = qd_q; g.kv_dim = kvd;
@@ -936,11 +936,6 @@ static cogs_status llm_forward_impl(cogs_handle h, cogs_stream stream, const voi
         if (kv) {
             char* kc = (char*)kv->k + ((size_t)l * kv->max_len) * kvd * es;
             char* vc = (char*)kv->v + ((size_t)l * kv->max_len) * kvd * es;
-            if (S != 1) {
-                PROF(COGS_PROF_OTHER);
-                COGS_TRY(cogs_k_kv_append(st, dt, kp, vp, qd, kc + (size_t)pos0 * kvd * es, vc + (size_t)pos0 * kvd * es,
-                                          kvd, S, kvd));
-            }
             kp = kc; vp = vc; ldkv = kvd;
         }
         {

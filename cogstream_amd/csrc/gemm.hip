@@ -1133,7 +1133,14 @@ static int launch_mid(hipStream_t st, const CogsGemm& g, int tile, bool alone) {
     return cogs_k_gemm_mid(st, g, tile, alone);
 }
 
-int cogs_k_gemm(hipStream_t st, const CogsGemm& g) {
+// the mid-size kernel stores K and V columns straight into the cache where its waves' 32 or 64 columns do not straddle them
+static bool kv_in_epilogue(const CogsGemm& g) {
+    const int mask = cogs_epi_mask(g);
+    return g.kv_k && g.dtype == COGS_DT_BF16 && (mask == EPI_ROPE || mask == (EPI_BIAS | EPI_ROPE)) && g.kv_col0 % 64 == 0 && g.kv_dim % 64 == 0;
+}
+
+// kv_stored: K and V columns went to the cache (only where kv_in_epilogue)
+static int gemm_rows(hipStream_t st, const CogsGemm& g, bool* kv_stored) {
     const int es = g.dtype == COGS_DT_BF16 ? 2 : 4;
     const int BK = g.dtype == COGS_DT_BF16 ? 64 : 32;
     if (g.M <= 0 || g.N <= 0 || g.K <= 0) return COGS_E_INVALID;
@@ -1155,7 +1162,10 @@ int cogs_k_gemm(hipStream_t st, const CogsGemm& g) {
     const bool pp_fits = n_pad * 100 <= g.N * (int)g_cogs_debug.gemm_pad_pct;   // default: <= 12 % of the MFMAs spent on N padding
     // (the ping-pong kernel wants two slabs and, below a row block, wastes its tiles' rows)
     const bool pp = mid > 0 && env_mid == 0 && g_cogs_debug.gemm_pingpong != 0 && pp_fits && g.K >= 128 && g.M >= 256;
-    if (mid > 0 && !pp) return launch_mid(st, g, mid, S == 1);
+    if (mid > 0 && !pp) {
+        *kv_stored = kv_in_epilogue(g);
+        return launch_mid(st, g, mid, S == 1);
+    }
     GemmArgs p;
     p.trace = nullptr; p.rope_lut = nullptr; p.rope_lut_bytes = 0; p.group_m = GROUP_M;
     p.epi_serial = (int)g_cogs_debug.gemm_epi_serial;
@@ -1252,6 +1262,8 @@ int cogs_k_gemm(hipStream_t st, const CogsGemm& g) {
             if (g.row_stats) b.row_stats = g.row_stats + (size_t)rows_main * (g.N / 64) * 2;
             if (g.ln_ab) b.ln_ab = g.ln_ab + (size_t)rows_main * 2;
             if (mb_main > 0) b.ln_part = nullptr;      // (finished below, in front of the first launch)
+            if (mb_main > 0) b.kv_k = b.kv_v = nullptr;
+            else *kv_stored = kv_in_epilogue(g);
             if (g.rope_cos) {
                 const size_t per_row = (size_t)(g.head_dim / 2) * (g.rope_sin ? 1 : 2);
                 b.rope_cos = g.rope_cos + (size_t)rows_main * per_row;
@@ -1282,4 +1294,12 @@ int cogs_k_gemm(hipStream_t st, const CogsGemm& g) {
     p.nbn = (g.N + BN - 1) / BN;
     dispatch_f32(st, p, p.nbm * p.nbn, cogs_epi_mask(g), big);
     return COGS_LAUNCH_CHECK();
+}
+
+int cogs_k_gemm(hipStream_t st, const CogsGemm& g) {
+    bool kv_stored = g.M == 1 || !g.kv_k;
+    const int rc = gemm_rows(st, g, &kv_stored);
+    if (rc != COGS_OK || kv_stored) return rc;
+    const char* k = (const char*)g.C + (size_t)g.kv_col0 * (g.dtype == COGS_DT_BF16 ? 2 : 4);
+    return cogs_k_kv_append(st, g.dtype, k, k + (size_t)g.kv_dim * (g.dtype == COGS_DT_BF16 ? 2 : 4), g.ldc, g.kv_k, g.kv_v, g.kv_dim, g.M, g.kv_dim);
 }

@@ -27,8 +27,8 @@ struct CogsGemm {
     int force_small_tile = 0;                // fp32: always the 128x128 kernel
     const void* rms_gamma = nullptr;         // M == 1 only: RMS-normalise A on the fly with this weight
     float rms_eps = 0.f;
-    // M == 1 only: output columns [kv_col0, kv_col0 + kv_dim) go to kv_k[0..kv_dim), the next kv_dim to kv_v
-    // (single-token decode writes the new K/V row straight into the cache; no kv_append launch)
+    // output columns [kv_col0, kv_col0 + kv_dim) go to rows of kv_dim at kv_k, the next kv_dim to kv_v (C may be left without them)
+    // (the single-row and the mid-size bf16 kernel store them themselves, behind the others they are copied)
     void* kv_k = nullptr; void* kv_v = nullptr; int kv_col0 = 0; int kv_dim = 0;
     // rope epilogues only: columns [0, q_cols) (the Q heads) are multiplied by q_scale before rounding
     float q_scale = 1.f; int q_cols = 0;

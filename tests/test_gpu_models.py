@@ -127,6 +127,28 @@ def _llm(dev, dtype):
     return cfg, st, Qwen2Engine(st, cfg, dtype=dtype, device=dev)
 
 
+@pytest.mark.parametrize("tile,split", [(0, 1), (1, 1), (3, 1), (4, 1), (5, 1), (7, 1), (0, 0)])
+def test_keys_and_values_stored_by_the_qkv_product(dev, tile, split):
+    """the QKV product's waves store their K and V columns into the cache (the ping-pong kernel's, split = 0, are copied): the same bits
+    as without a cache, where attention reads the product's own rows, and behind a kept first part"""
+    from cogstream_amd import _lib as L2
+    from cogstream_amd.llm import Qwen2Engine
+    from cogstream_amd.weights import LlmConfig, random_llm_state
+    cfg = LlmConfig(hidden_size=768, intermediate_size=256, num_hidden_layers=2, num_attention_heads=6, num_key_value_heads=1, vocab_size=64,
+                    image_token_index=60, eos_token_id=59)
+    eng = Qwen2Engine(random_llm_state(cfg, seed=3, std=0.05), cfg, dtype=torch.bfloat16, device=dev)
+    for rows in (2, 33, 129, 300, 700):
+        g = torch.Generator(device=dev).manual_seed(rows)
+        x = torch.randn(rows, cfg.hidden_size, generator=g, device=dev).bfloat16()
+        with L2.debug_switch("gemm_mid", tile), L2.debug_switch("gemm_split", split):
+            want = eng.forward(x, None, want_logits=False, want_hidden=True)["hidden"]
+            cache, parts = eng.new_cache(rows + 3), eng.new_cache(rows + 1)
+            assert torch.equal(eng.forward(x, cache, want_logits=False, want_hidden=True)["hidden"], want)
+            n = rows // 2 + 1
+            got = [eng.forward(p, parts, want_logits=False, want_hidden=True)["hidden"] for p in (x[:n], x[n:]) if p.shape[0] > 1]
+            assert torch.equal(torch.cat(got), want[:sum(p.shape[0] for p in got)])
+
+
 @pytest.mark.parametrize("dtype,tol", [(torch.float32, 1e-4), (torch.bfloat16, 3e-2)])
 def test_llm_prefill_and_decode_vs_oracle(dev, dtype, tol):
     from oracle import qwen2 as oq
