@@ -299,7 +299,7 @@ __global__ __launch_bounds__(64) void mla_rowwise_kernel(CogsMla p) {
 }
 
 // ------------------------------------------------------------------------------------------------ prompt attention (bf16)
-// 4 waves x 32 query rows of one (sequence, head) against 64-key tiles; NH = 2: 8 waves, each half with every second tile, whose sums
+// 4 waves x 16 NQ query rows of one (sequence, head) against 64-key tiles; NH = 2: 8 waves, each half with every second tile, whose sums
 // meet at the end. Staging as in attn.hip's prompt kernel: a tile's pieces
 // (1 KiB = 64 lanes x 16 bytes) go global -> LDS by LDS-DMA into a double buffer, one tile ahead, one barrier per tile. Keys come
 // from two places -- the head's expanded part and the rotated part all heads share -- so a K tile is two LDS regions of KN and KR
@@ -330,9 +330,9 @@ template <int DT> __device__ __forceinline__ int mla_vswz(int row) {
     else return b3;
 }
 
-template <int KN, int KR, int DT, int WPE, int NH>
+template <int KN, int KR, int DT, int WPE, int NH, int NQ>
 __global__ __launch_bounds__(256 * NH, WPE) void mla_prefill_kernel(CogsMla p, int nqt, int group) {
-    constexpr int NQ = 2, KS = KN + KR;
+    constexpr int KS = KN + KR, WQ = 16 * NQ, TQ = 4 * WQ;              // query rows of a wave, of a workgroup
     constexpr bool HEADS = KR == 0;
     constexpr int N_LDS = 64 * KN * 64, R_LDS = 64 * KR * 64, V_LDS = 64 * DT * 32, BUF = N_LDS + R_LDS + V_LDS;
     constexpr int PV = DT / 2;                    // V pieces per wave (K: KN and KR)
@@ -359,7 +359,7 @@ __global__ __launch_bounds__(256 * NH, WPE) void mla_prefill_kernel(CogsMla p, i
     }
     const int h = pair % p.heads;
     const CogsSeq s = p.seqs[pair / p.heads];
-    const int q0 = qt * 128;
+    const int q0 = qt * TQ;
     if (q0 >= s.len) return;
 
     const bf16_t* Q = reinterpret_cast<const bf16_t*>(p.Q) + (long)s.row0 * p.ldq + (long)h * p.q_head;
@@ -377,7 +377,7 @@ __global__ __launch_bounds__(256 * NH, WPE) void mla_prefill_kernel(CogsMla p, i
     int qpos[NQ];
 #pragma unroll
     for (int i = 0; i < NQ; ++i) {
-        const int rc = min(q0 + wid * 32 + 16 * i + li, s.len - 1);
+        const int rc = min(q0 + wid * WQ + 16 * i + li, s.len - 1);
         qpos[i] = s.pos0 + rc;
 #pragma unroll
         for (int k = 0; k < KS; ++k) {
@@ -387,9 +387,9 @@ __global__ __launch_bounds__(256 * NH, WPE) void mla_prefill_kernel(CogsMla p, i
             qf[i][k] = __builtin_bit_cast(bf16x8, v);
         }
     }
-    const bool wave_active = q0 + wid * 32 < s.len;
-    const int wave_hi = s.pos0 + min(q0 + wid * 32 + 31, s.len - 1);               // last position of the wave's rows
-    const int kend = s.pos0 + min(q0 + 128, s.len);                                 // keys the workgroup needs
+    const bool wave_active = q0 + wid * WQ < s.len;
+    const int wave_hi = s.pos0 + min(q0 + wid * WQ + WQ - 1, s.len - 1);               // last position of the wave's rows
+    const int kend = s.pos0 + min(q0 + TQ, s.len);                                 // keys the workgroup needs
     const int nt = (kend + 63) >> 6;
     const int p0 = s.pos0 + q0;                                                     // position of the workgroup's first row
     float b_far = 0.f;
@@ -483,7 +483,7 @@ __global__ __launch_bounds__(256 * NH, WPE) void mla_prefill_kernel(CogsMla p, i
         }
     };
 
-    // bias window of tile t: entry i is distance p0 - 63 - 64 t + i (queries below p0 + 128, keys 64 t .. 64 t + 63)
+    // bias window of tile t: entry i is distance p0 - 63 - 64 t + i (queries below p0 + 128 at the most, keys 64 t .. 64 t + 63)
     auto stage_window = [&](int t) {
         if constexpr (HEADS)
             if (p.bias && t + NH > t_far && tid < MLA_WIN)     // (a round's tiles take one form)
@@ -530,14 +530,14 @@ __global__ __launch_bounds__(256 * NH, WPE) void mla_prefill_kernel(CogsMla p, i
                     sacc[u][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf, qf[i][k], k == 0 ? start[i] : sacc[u][i], 0, 0, 0);
             }
         }
-        if constexpr (!MASKED && !NEAR && KS >= 2) {   // 4 KS reads, 8 KS MFMAs: six reads lead, then a read per pair of MFMAs
+        if constexpr (!MASKED && !NEAR && KS >= 2) {   // 4 KS reads, 4 NQ KS MFMAs: six reads lead, then a read per NQ MFMAs
             __builtin_amdgcn_sched_group_barrier(0x100, 6, 0);
 #pragma unroll
             for (int i = 0; i < 4 * KS - 6; ++i) {
-                __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);
+                __builtin_amdgcn_sched_group_barrier(0x008, NQ, 0);
                 __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
             }
-            __builtin_amdgcn_sched_group_barrier(0x008, 12, 0);
+            __builtin_amdgcn_sched_group_barrier(0x008, 6 * NQ, 0);
         }
         if (NH == 1) __builtin_amdgcn_s_setprio(1);
         bf16x8 pf[2][NQ][2];                           // [32-key step][row group][head, remainder]
@@ -607,15 +607,15 @@ __global__ __launch_bounds__(256 * NH, WPE) void mla_prefill_kernel(CogsMla p, i
 #pragma unroll
                     for (int i = 0; i < NQ; ++i) oacc[d][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, pf[u][i][x], oacc[d][i], 0, 0, 0);
             }
-        if constexpr (!MASKED && DT >= 4) {            // 4 DT transposing reads, 8 + 8 DT MFMAs: eight reads lead
+        if constexpr (!MASKED && DT >= 4) {            // 4 DT transposing reads, 4 NQ (1 + DT) MFMAs: eight reads lead
             __builtin_amdgcn_sched_group_barrier(0x100, 8, 0);
-            __builtin_amdgcn_sched_group_barrier(0x008, 8, 0);
+            __builtin_amdgcn_sched_group_barrier(0x008, 4 * NQ, 0);
 #pragma unroll
             for (int i = 0; i < DT - 2; ++i) {
-                __builtin_amdgcn_sched_group_barrier(0x008, 8, 0);
+                __builtin_amdgcn_sched_group_barrier(0x008, 4 * NQ, 0);
                 __builtin_amdgcn_sched_group_barrier(0x100, 4, 0);
             }
-            __builtin_amdgcn_sched_group_barrier(0x008, 16, 0);
+            __builtin_amdgcn_sched_group_barrier(0x008, 8 * NQ, 0);
         }
     };
 
@@ -675,34 +675,42 @@ __global__ __launch_bounds__(256 * NH, WPE) void mla_prefill_kernel(CogsMla p, i
         tile_tail();
     }
 
-    // the shares' sums meet in LDS: wave (w, kh) hands over rows of group 1 - kh and finishes those of group kh
-    auto join = [&](auto mine_tag) {
-        constexpr int MINE = decltype(mine_tag)::value, OTHER = 1 - MINE;
-        f32x4* x = reinterpret_cast<f32x4*>(smem) + (wid * 2 + OTHER) * (DT + 1) * 64 + lane;
+    // the shares' sums meet in LDS: wave (w, kh) hands over rows of group 1 - kh and finishes those of group kh (one group: share 0 does)
+    auto at = [&](int grp) { return reinterpret_cast<f32x4*>(smem) + (wid * NQ + grp) * (DT + 1) * 64 + lane; };
+    auto hand_over = [&](auto tag) {
+        constexpr int G = decltype(tag)::value;
+        f32x4* x = at(G);
 #pragma unroll
-        for (int d = 0; d < DT; ++d) x[d * 64] = oacc[d][OTHER];
-        x[DT * 64] = f32x4{lacc[OTHER][0], m_ref[OTHER], 0.f, 0.f};
-        __syncthreads();
-        const f32x4* y = reinterpret_cast<const f32x4*>(smem) + (wid * 2 + MINE) * (DT + 1) * 64 + lane;
+        for (int d = 0; d < DT; ++d) x[d * 64] = oacc[d][G];
+        x[DT * 64] = f32x4{lacc[G][0], m_ref[G], 0.f, 0.f};
+    };
+    auto take = [&](auto tag) {
+        constexpr int G = decltype(tag)::value;
+        const f32x4* y = at(G);
         const f32x4 lm = y[DT * 64];
         // a share that saw no key has a sum of zero and takes no part in the reference
-        const float m = lm[0] == 0.f ? m_ref[MINE] : lacc[MINE][0] == 0.f ? lm[1] : fmaxf(m_ref[MINE], lm[1]);
-        const float fa = lacc[MINE][0] == 0.f ? 0.f : __builtin_amdgcn_exp2f(m_ref[MINE] - m), fb = lm[0] == 0.f ? 0.f : __builtin_amdgcn_exp2f(lm[1] - m);
+        const float m = lm[0] == 0.f ? m_ref[G] : lacc[G][0] == 0.f ? lm[1] : fmaxf(m_ref[G], lm[1]);
+        const float fa = lacc[G][0] == 0.f ? 0.f : __builtin_amdgcn_exp2f(m_ref[G] - m), fb = lm[0] == 0.f ? 0.f : __builtin_amdgcn_exp2f(lm[1] - m);
 #pragma unroll
-        for (int d = 0; d < DT; ++d) oacc[d][MINE] = oacc[d][MINE] * fa + y[d * 64] * fb;
-        lacc[MINE] = lacc[MINE] * fa + lm[0] * fb;
-        m_ref[MINE] = m;
+        for (int d = 0; d < DT; ++d) oacc[d][G] = oacc[d][G] * fa + y[d * 64] * fb;
+        lacc[G] = lacc[G] * fa + lm[0] * fb;
+        m_ref[G] = m;
     };
     static_assert(NH == 1 || 8 * (DT + 1) * 1024 <= 2 * NH * BUF, "the exchange fits the tiles' buffers");
     if constexpr (NH == 2) {
-        if (kh == 0) join(std::integral_constant<int, 0>{});
-        else join(std::integral_constant<int, 1>{});
+        typedef std::integral_constant<int, 0> first;
+        typedef std::integral_constant<int, NQ - 1> last;
+        if (kh == 1) hand_over(first{});
+        else if (NQ == 2) hand_over(last{});
+        __syncthreads();
+        if (kh == 0) take(first{});
+        else if (NQ == 2) take(last{});
     }
     const int dt = p.dv >> 4;
 #pragma unroll
     for (int i = 0; i < NQ; ++i) {
-        if (NH == 2 && i != kh) continue;
-        const int qrow = q0 + wid * 32 + 16 * i + li;
+        if (NH == 2 && (NQ == 2 ? i : 0) != kh) continue;
+        const int qrow = q0 + wid * WQ + 16 * i + li;
         if (qrow >= s.len) continue;
         float f = 1.f / (lacc[i][0] + (p.sink ? exp2f(p.sink[h] - m_ref[i]) : 0.f));
         const long row = s.row0 + qrow;
@@ -932,16 +940,16 @@ __global__ __launch_bounds__(256) void mla_combine_kernel(const float* __restric
     }
 }
 
-template <int KN, int KR, int DT, int WPE, int NH>
+template <int KN, int KR, int DT, int WPE, int NH, int NQ>
 int launch_prefill(hipStream_t st, const CogsMla& a) {
     static std::atomic<uint64_t> attr_done{0};
     constexpr int lds = 2 * NH * (64 * KN * 64 + 64 * KR * 64 + 64 * DT * 32) + (KR == 0 ? 2 * NH * MLA_WIN * 4 : 0);
-    cogs_ensure_dyn_lds((const void*)mla_prefill_kernel<KN, KR, DT, WPE, NH>, lds, attr_done);
-    const int nqt = (a.max_new + 127) / 128;
+    cogs_ensure_dyn_lds((const void*)mla_prefill_kernel<KN, KR, DT, WPE, NH, NQ>, lds, attr_done);
+    const int nqt = (a.max_new + 64 * NQ - 1) / (64 * NQ);
     const long grid = (long)nqt * a.heads * a.nseq;
     if (grid > 0x7fffffffL) return COGS_E_INVALID;
     const int group = nqt >= 64 ? 1 : 64 / nqt;            // (NH = 2: one workgroup per CU, the next longest to the CU that is done first)
-    hipLaunchKernelGGL((mla_prefill_kernel<KN, KR, DT, WPE, NH>), dim3((unsigned)grid), dim3(256 * NH), lds, st, a, nqt, group);
+    hipLaunchKernelGGL((mla_prefill_kernel<KN, KR, DT, WPE, NH, NQ>), dim3((unsigned)grid), dim3(256 * NH), lds, st, a, nqt, group);
     return COGS_LAUNCH_CHECK();
 }
 
@@ -952,13 +960,16 @@ int launch_prefill(hipStream_t st, const CogsMla& a) {
 // for a whole CU's LDS too, are slower in halves. Whole passes of 9 layers of 16 heads, / of 6 of 32, four waves against eight: one prompt of 4096 rows
 // 4.91 / 4.79 ms (32 heads 8.76 / 8.84, 28 heads x 2048 5.75 / 5.86), 4 x 512 rows behind 2000 3.63 / 3.51 (32 heads 5.49 / 5.60), 8 x 16 behind 1000 1.54 / 1.50,
 // 32 x 16 behind 1000 2.98 / 3.15, 1 x 2048 + 3 x 64 3.94 / 4.04, + 63 x 32 5.83 / 6.63, 8 x 300 3.07 / 3.13.
+// Up to 128 query tiles of 128 rows are taken as tiles of 64, half the work in a key tile's chain on twice the CUs: passes of 128 rows 863 -> 829 us,
+// 400 1121 -> 1076, 800 1601 -> 1572 (16 heads), 400 of 28 heads 2145 -> 2119, of 32 1682 -> 1656; delta rule, 400 rows 1260 -> 1246.
 template <int KN, int KR, int DT>
 int launch_prefill_split(hipStream_t st, const CogsMla& a) {
     const int nqt = (a.max_new + 127) / 128;
     const long tiles = (long)nqt * a.heads * a.nseq;
     const bool halves = tiles <= 256 || (tiles <= 512 && a.nseq == 1 && nqt >= a.heads);
     g_cogs_debug.mla_last_waves = halves ? 8 : 4;
-    return halves ? launch_prefill<KN, KR, DT, 2, 2>(st, a) : launch_prefill<KN, KR, DT, 2, 1>(st, a);
+    if (tiles <= 128) return launch_prefill<KN, KR, DT, 2, 2, 1>(st, a);
+    return halves ? launch_prefill<KN, KR, DT, 2, 2, 2>(st, a) : launch_prefill<KN, KR, DT, 2, 1, 2>(st, a);
 }
 
 template <int DTW, int PER, int KH, int WGS>
@@ -1027,7 +1038,7 @@ int cogs_k_mla_attention(hipStream_t st, int dtype, const CogsMla& a) {
         if (kn <= 1 && dt <= 2) return launch_prefill_split<1, 0, 2>(st, a);
         if (kn <= 2 && dt <= 4) return launch_prefill_split<2, 0, 4>(st, a);
         if (kn <= 4 && dt <= 8) return launch_prefill_split<4, 0, 8>(st, a);
-        if (kn <= 8 && dt <= 16) return launch_prefill<8, 0, 16, 1, 1>(st, a);
+        if (kn <= 8 && dt <= 16) return launch_prefill<8, 0, 16, 1, 1, 2>(st, a);
     }
     if (dtype == COGS_DT_BF16 && !a.kvw && !a.absorbed && a.dn % 8 == 0 && a.dr % 8 == 0 && a.dv % 16 == 0 && a.ldq % 8 == 0 && a.q_head % 32 == 0 &&
         a.q_rot % 32 == 0 && a.q_rot >= a.dn && a.q_head - a.q_rot >= a.dr && a.ldk % 8 == 0 && a.k_head % 8 == 0 && a.ldkr % 8 == 0 &&
@@ -1038,7 +1049,7 @@ int cogs_k_mla_attention(hipStream_t st, int dtype, const CogsMla& a) {
         if (kn <= 2 && kr <= 1 && dt <= 4) return launch_prefill_split<2, 1, 4>(st, a);
         if (kn <= 4 && kr <= 1 && dt <= 8) return launch_prefill_split<4, 1, 8>(st, a);
         if (kn <= 4 && kr <= 2 && dt <= 8) return launch_prefill_split<4, 2, 8>(st, a);
-        if (kn <= 8 && kr <= 4 && dt <= 16) return launch_prefill<8, 4, 16, 1, 1>(st, a);
+        if (kn <= 8 && kr <= 4 && dt <= 16) return launch_prefill<8, 4, 16, 1, 1, 2>(st, a);
     }
     if (a.dn + a.dr > RW_DIM || a.dv > 64 * RW_VREG) return COGS_E_UNSUPPORTED;
     if (dtype == COGS_DT_BF16) hipLaunchKernelGGL(mla_rowwise_kernel<bf16_t>, dim3(a.rows, a.heads), dim3(64), 0, st, a);

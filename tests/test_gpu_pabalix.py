@@ -288,6 +288,20 @@ def test_a_query_tile_by_one_wave_or_by_two(dev, name):
             assert rms_err(out, lg[[n - 1 for _, n in jobs]]) < TOL[torch.bfloat16], (times, cut)
 
 
+@pytest.mark.parametrize("name", ["peaked", "mixed"])
+@pytest.mark.parametrize("n", [2, 63, 64, 65, 127, 129, 191, 193, 300])
+def test_query_tiles_of_64_rows(dev, name, n):
+    """one prompt, few query tiles: they have 64 rows, one group of 16 a wave, whose second half of the keys another wave hands over; the edges of both
+    kinds of tiles, from nothing and behind cached tokens, against the oracle"""
+    cfg, st, e, toks, lg, _ = named(name, torch.bfloat16, dev, 400)
+    for cut in (0, 1, 70):
+        s = sequences(e)
+        if cut:
+            s.step([(0, toks[:cut], [])])
+        out = s.step([(0, toks[cut:cut + n], list(range(n)))])
+        assert rms_err(out, lg[cut:cut + n]) < TOL[torch.bfloat16], cut
+
+
 def test_short_prompts_beside_a_long_one(dev):
     """a prompt of many key tiles by itself has each query tile's keys shared by two waves; short ones beside it, most of whose query tiles are
     empty, take that away (every workgroup would wait for a whole CU) and none of the result"""
