@@ -1101,24 +1101,28 @@ void dispatch_f32(hipStream_t st, const GemmArgs& p, int grid, int mask, bool bi
 // time of a slab + the rest of a tile: prologue, epilogue), with a slab's time per tile size for one and, where the LDS has room for
 // them, two workgroups on a CU. The figures are a fit to launches of every tile at M = 48 .. 2048 and eleven weight shapes from 1152 x
 // 1152 to 37 888 x 3584 and 3584 x 18 944 (MI355X, weights from HBM); the tile they choose was the fastest or within 6 % of it at
-// each. They are those of a chip that is not full: three rounds of 128x256 take 0.95 us a slab, which no choice here depends on.
+// each. They are those of a chip that is not full; two and three rounds are slower a slab (1281 x 11 264 x 2048: two rounds of 128x256
+// 61.6 us, one of ping-pong tiles and a row of small ones 52; 320 x 22 016 x 4096: two of 128x256 95.6, one of ping-pong 88; 180 x 37 888
+// x 3584: 64x64 108.9, 128x128 96.6).
 struct TileCost { int tile, tm, tn; float one, two, rest; };     // us; two = 0: one workgroup per CU
 static constexpr TileCost MID_TILES[] = {
     {1, 32, 64, 0.165f, 0.f, 1.8f},   {2, 64, 64, 0.218f, 0.409f, 1.8f}, {3, 128, 64, 0.309f, 0.637f, 2.3f}, {4, 128, 128, 0.387f, 0.f, 3.6f},
     {5, 128, 256, 0.629f, 0.f, 4.8f}, {6, 128, 64, 0.292f, 0.f, 2.5f},   {7, 160, 64, 0.332f, 0.f, 3.8f}};
+static constexpr float MID_FULL = 1.25f, TWO_FULL = 1.15f, PP_FULL = 1.12f;         // slabs of launches of more than one round, against those
 static constexpr float PP_SLAB = 1.14f, PP_REST = 6.f, SECOND_LAUNCH = 2.f;
 
-static float tile_time(int tiles, int slabs, float one, float two, float rest) {
+static float tile_time(int tiles, int slabs, float one, float two, float rest, float full) {
     const float t1 = slabs * one + rest, t2 = slabs * two + rest;
-    if (two == 0.f) return (float)((tiles + PERSISTENT_WGS - 1) / PERSISTENT_WGS) * t1;
-    const int full = tiles / (2 * PERSISTENT_WGS), left = tiles % (2 * PERSISTENT_WGS);
-    return full * t2 + (left == 0 ? 0.f : left <= PERSISTENT_WGS ? t1 : t2);
+    const int rounds = (tiles + PERSISTENT_WGS - 1) / PERSISTENT_WGS;
+    if (two == 0.f) return rounds > 1 ? rounds * (slabs * one * full + rest) : t1;
+    const int whole = tiles / (2 * PERSISTENT_WGS), left = tiles % (2 * PERSISTENT_WGS);
+    return whole * (whole > 1 ? slabs * two * TWO_FULL + rest : t2) + (left == 0 ? 0.f : left <= PERSISTENT_WGS ? t1 : t2);
 }
 static int best_mid_tile(int M, int N, int K, bool ln_fold, float* time) {
     int best = 0;
     for (const TileCost& t : MID_TILES) {
         if (t.tile == 7 && ln_fold) continue;       // (its waves have more rows than lanes to hold their factors)
-        const float c = tile_time((M + t.tm - 1) / t.tm * ((N + t.tn - 1) / t.tn), K / 64, t.one, t.two, t.rest);
+        const float c = tile_time((M + t.tm - 1) / t.tm * ((N + t.tn - 1) / t.tn), K / 64, t.one, t.two, t.rest, MID_FULL);
         if (best == 0 || c < *time) { best = t.tile; *time = c; }
     }
     return best;
@@ -1231,7 +1235,7 @@ static int gemm_rows(hipStream_t st, const CogsGemm& g, bool* kv_stored) {
             // streams. (Counting both streams' tiles as one launch picked larger tiles, which leave less for the other stream's
             // launch to run beside: 4 x 256 patches 3.09 against 2.58 ms, 16 x 256 5.46 / 4.92, 8 x 924 8.52 / 7.95.)
             const int slabs = g.K / 64;
-            float best = tile_time(nb, slabs, PP_SLAB, 0.f, PP_REST);
+            float best = tile_time(nb, slabs, PP_SLAB, 0.f, PP_REST, PP_FULL);
             if (mid_time < best) { best = mid_time; mb_main = 0; }
             if (rounds == 1 && rem > 0) {
                 const int mb = whole_blocks(PERSISTENT_WGS);           // whole row blocks inside the first round
