@@ -1121,8 +1121,10 @@ static float tile_time(int tiles, int slabs, float one, float two, float rest, f
 static int best_mid_tile(int M, int N, int K, bool ln_fold, float* time) {
     int best = 0;
     for (const TileCost& t : MID_TILES) {
-        if (t.tile == 7 && ln_fold) continue;       // (its waves have more rows than lanes to hold their factors)
-        const float c = tile_time((M + t.tm - 1) / t.tm * ((N + t.tn - 1) / t.tn), K / 64, t.one, t.two, t.rest, MID_FULL);
+        const int tiles = (M + t.tm - 1) / t.tm * ((N + t.tn - 1) / t.tn);
+        // (160x64: its waves have more rows than lanes to hold their factors; three rounds of 150 x 37 888 x 3584 97 us, 128x128 88)
+        if (t.tile == 7 && (ln_fold || tiles > PERSISTENT_WGS)) continue;
+        const float c = tile_time(tiles, K / 64, t.one, t.two, t.rest, MID_FULL);
         if (best == 0 || c < *time) { best = t.tile; *time = c; }
     }
     return best;
