@@ -25,6 +25,7 @@
 // 32-multiple] = kvw columns.
 #include "common.h"
 #include "kernels.h"
+#include "mla_place.h"
 #include "debug.h"
 #include <type_traits>
 
@@ -757,14 +758,14 @@ __global__ __launch_bounds__(256, WGS) void mla_decode_kernel(MlaDecodeArgs p) {
     const int tid = threadIdx.x, lane = tid & 63;
     const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int li = lane & 15, g = lane >> 4;
-    // the head tiles of a split sit 8 apart in the launch order = on one XCD: its L2 serves the second and later readers
-    const int bid = blockIdx.x, rest = bid >> 3;
-    const int ht = rest % p.nht, split = (rest / p.nht) * 8 + (bid & 7);
-    const int b = blockIdx.y / p.groups, grp = blockIdx.y - b * p.groups, h0 = grp * p.rep + ht * 16, h1 = (grp + 1) * p.rep;
+    const int b = blockIdx.y / p.groups, grp = blockIdx.y - b * p.groups;
     const CogsSeq s = p.seqs[b];
+    const long part0 = mla_first_part(s, b, p.tiles);
+    const MlaPlace place = mla_place(blockIdx.x, blockIdx.y, gridDim.x, p.nht, part0);
+    const int split = place.split, h0 = grp * p.rep + place.head_tile * 16, h1 = (grp + 1) * p.rep;
     const int kend = s.pos0 + 1, t_begin = split * p.tiles, t_end = min(t_begin + p.tiles, (kend + TK - 1) / TK);
     if (t_begin >= t_end) return;
-    const long slot0 = (mla_first_part(s, b, p.tiles) + split) * p.heads;
+    const long slot0 = (part0 + split) * p.heads;
     const char* cache = s.cache + (p.layer_off + (long)grp * p.kvw) * s.max_len * 2;
     const int row_bytes = p.kvw * 2, nch = p.kvw >> 3, pieces = (nch + 2) >> 1;      // 16-byte units of a row; KiB of a slot
 
@@ -1060,7 +1061,9 @@ int cogs_k_mla_attention(hipStream_t st, int dtype, const CogsMla& a) {
 bool cogs_k_mla_decode_fits(int kvw, int kvp) { return kvw % 32 == 0 && kvp % 16 == 0 && kvp <= 1024 && kvw <= 1152; }
 
 // Tiles of 32 keys per split: two workgroups a CU over the whole batch (context: keys of all sequences together), two tiles at the
-// least -- shorter splits cost more in the combine than they save here
+// least -- shorter splits cost more in the combine than they save here. Rows of more than 592 columns leave LDS for one at a time: two
+// rounds, then. One of twice the tiles is the slower (32 x 256 .. 8192 keys, six layers, us, 9 tiles / 17: 640 columns 960 / 1070, 1088
+// 1156 / 1271), its last workgroups do not fit.
 static int decode_tiles(int nseq, int groups, int rep, int64_t context) {
     const int keys = (int)g_cogs_debug.mla_split_keys;
     if (keys > 0) return (keys + MLA_TK - 1) / MLA_TK;
