@@ -1145,10 +1145,14 @@ int cogs_k_attention(hipStream_t st, const CogsAttn& a) {
             // (two more forms were built, tested at full size and measured slower -- a ping-pong form, 1.89 vs 1.81-1.86 ms per layer
             // at 15 395 tokens, and 64 query rows per wave, 2.94 vs 1.97 ms: tools/experiments/attn_prefill_variants.hip)
             g_cogs_debug.attn_last_kernel = 5;
-            // 64 query rows a workgroup where 128 leave CUs idle, or not many more than one to each: same bits, half the work in a key
-            // tile's chain. 28 heads, 128 rows a workgroup / 64, us: 100 rows 9.0 / 5.6, 256 12.2 / 7.9, 512 17.7 / 11.7, 621 19.9 / 15.8, 900
-            // 25.8 / 21.5, 1280 (280 workgroups) 39.1 / 32.2, 1600 (364) 45.6 / 44.4, 2048 (448) 60.9 / 78.1
-            const bool narrow = g_cogs_debug.attn_prefill_deep && p.prio_mode == 2 && (long)grid.x * grid.y * grid.z <= 320;
+            // 64 query rows a workgroup where 128 leave CUs idle, or (prompts that begin here, mostly) not many more than one to each: same
+            // bits, half the work in a key tile's chain. 28 heads, 128 rows a workgroup / 64, us: 100 rows 9.0 / 5.6, 256 12.2 / 7.9, 512
+            // 17.7 / 11.7, 621 19.9 / 15.8, 900 25.8 / 21.5, 1280 (280 workgroups) 39.1 / 32.2, 1600 (364) 45.6 / 44.4, 2048 (448) 60.9 /
+            // 78.1. Above 256, half as wide ones are more than the chip holds (two a CU), and behind kept keys the late ones are no shorter:
+            // 1280 rows behind 500 keys 57.2 / 48.5, 2000 94.4 / 90.1, 4000 141 / 147, 15 000 394 / 454; 1152 rows (252) behind 15 000 309 / 295
+            const long wgs = (long)grid.x * grid.y * grid.z;
+            const bool narrow = g_cogs_debug.attn_prefill_deep && p.prio_mode == 2 && wgs <= (p.q_pos0 <= max_len ? 320 : 256);
+            g_cogs_debug.attn_last_rows = narrow ? 64 : 128;
             if (narrow)
                 hipLaunchKernelGGL((attn_prefill_dma_kernel<1, 2, 1>), dim3((max_len + 63) / 64, grid.y, grid.z), dim3(256), 0, st, p);
             else if (g_cogs_debug.attn_prefill_deep && p.prio_mode == 2) hipLaunchKernelGGL((attn_prefill_dma_kernel<1, 2>), grid, dim3(256), 0, st, p);

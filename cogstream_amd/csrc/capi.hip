@@ -80,6 +80,7 @@ cogs_status cogs_debug_get(const char* name, int64_t* value) {
 #undef COGS_DBG_GET
     if (strcmp(name, "gemm_last_body") == 0) { *value = g_cogs_debug.gemm_last_body; return COGS_OK; }
     if (strcmp(name, "attn_last_kernel") == 0) { *value = g_cogs_debug.attn_last_kernel; return COGS_OK; }
+    if (strcmp(name, "attn_last_rows") == 0) { *value = g_cogs_debug.attn_last_rows; return COGS_OK; }
     if (strcmp(name, "mla_last_waves") == 0) { *value = g_cogs_debug.mla_last_waves; return COGS_OK; }
     if (strcmp(name, "km_pp_last_launches") == 0) { *value = g_cogs_debug.km_pp_last_launches; return COGS_OK; }
     if (strcmp(name, "attn_vit_last_end") == 0) { *value = g_cogs_debug.attn_vit_last_end; return COGS_OK; }
@@ -95,6 +96,7 @@ const char* cogs_debug_list(void) {
         "4 whole-line ping-pong, 5 ping-pong + mid-size (split launch), 6 GEMV, 7 few-row GEMM\n"
         "attn_last_kernel (read only): kernel of the last cogs_attention -- 1 general MFMA, 2 ViT unpipelined, 3 ViT pipelined, "
         "4 single-token decode, 5 prompt LDS-DMA, 7 row-wise fp32, 8 ViT pipelined on head-major K/V\n"
+        "attn_last_rows (read only): query rows per workgroup of the last prompt attention (kernel 5), 64 or 128\n"
         "attn_vit_last_end (read only): ragged end of the last pipelined ViT attention launch -- 10 x tiles behind the four-tile loop + "
         "32-key blocks of the last tile (41 .. 72: compile-time shape), 0 the run-time form\n"
         "mla_last_waves (read only): waves per query tile of the last prompt attention of a described decoder in bf16, 4 or 8\n"

@@ -66,6 +66,8 @@ struct CogsDebug {
     // decode (+ combine), 5 prompt LDS-DMA kernel, 7 row-wise fp32 kernel, 8 ViT pipelined, head-major K/V (6 and 9 were the archived
     // ping-pong / 64-rows-per-wave prompt kernels: tools/experiments/attn_prefill_variants.hip)
     std::atomic<long long> attn_last_kernel{0};
+    // ... and query rows per workgroup of the last prompt LDS-DMA kernel, 64 or 128
+    std::atomic<long long> attn_last_rows{0};
     // ... and which ragged end the last pipelined ViT launch had: 10 R + blocks of the last tile (41 .. 72), 0 = the run-time form
     std::atomic<long long> attn_vit_last_end{0};
     // ... and the last prompt attention of a described decoder (bf16): waves per query tile, 4 or 8

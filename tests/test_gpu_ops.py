@@ -1081,6 +1081,24 @@ def test_prompt_attention_of_64_row_workgroups(dev, lens, hq, hkv, pos0):
         at += m
 
 
+@pytest.mark.parametrize("hq,hkv,rows,pos0,want", [(28, 4, 1280, 0, 64), (28, 4, 1280, 1281, 128), (28, 4, 1152, 9000, 64), (28, 4, 1500, 0, 128),
+                                                   (64, 8, 621, 4000, 128), (64, 8, 512, 4000, 64)])
+def test_prompt_attention_rows_behind_kept_keys(dev, hq, hkv, rows, pos0, want):
+    """query tiles of 64 rows are for prompts whose tiles of 128 leave CUs idle, and, up to 320 of those, for prompts that are not mostly
+    kept keys; the same bits either way"""
+    from cogstream_amd import _lib as L2
+    ops = _ops()
+    g = torch.Generator(device=dev).manual_seed(rows + pos0)
+    q = torch.randn(rows, hq * 128, generator=g, device=dev).bfloat16() * 0.2
+    k, v = (torch.randn(rows + pos0, hkv * 128, generator=g, device=dev).bfloat16() for _ in range(2))
+    kw = dict(hq=hq, hkv=hkv, head_dim=128, causal=True, q_prescaled=True, q_pos0=pos0)
+    got = ops.attention(q, k, v, **kw)
+    assert L2.debug_get("attn_last_rows") == want
+    with L2.debug_switch("attn_prio", 1):
+        assert torch.equal(got, ops.attention(q, k, v, **kw))
+        assert L2.debug_get("attn_last_rows") == 128
+
+
 @pytest.mark.parametrize("tile", [1, 2, 3, 4, 5, 6, 7])
 @pytest.mark.parametrize("M,N,K", [(1147, 328, 192), (1537, 1544, 128), (100, 9000, 640)])
 def test_mid_size_gemm_groups_of_row_tiles(dev, tile, M, N, K):
