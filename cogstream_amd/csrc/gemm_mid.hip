@@ -60,6 +60,9 @@ __device__ __forceinline__ void wait_slabs(int n) {
     else asm volatile("s_waitcnt vmcnt(%0)" ::"n"(MAX >= 6 ? 6 * P : 0) : "memory");
 }
 
+// columns whose weights `of` workgroups can ask for in the time of a tile (below)
+constexpr int read_ahead_cols(int TM, int TN, int of) { return of * (TM + TN) * 9 / 16; }
+
 // workgroups (a multiple of 8: as many on each XCD) behind those of the tiles: one dword of every weight line that the tiles of this
 // XCD read, slabs in order, so that the tiles' DMA finds them in L2. Nothing waits for them and nothing is kept.
 __device__ __forceinline__ void prefetch_weights(const MidArgs& p, char* smem, int TM, int TN, int waves, int wid, int lane) {
@@ -82,7 +85,7 @@ __device__ __forceinline__ void prefetch_weights(const MidArgs& p, char* smem, i
     // more columns than they can ask for in the tiles' time the launch would wait for them, so they take evenly spaced slabs, and none
     // if that were less than half of them. 37 888 x 3584, M = 128 (a fifth): every slab 145 us, the fifth 75, none 68; 6176 x 2048,
     // M = 1152 110 -> 32.5; 4608 x 3584, M = 1152 95 -> 46; where all can be had (3584 x 18 944, M = 621) 108, none 134.
-    const int slabs = (int)min((long)p.KT, (long)p.KT * of * (TM + TN) * 9 / (16L * max(cols, 1)));
+    const int slabs = (int)min((long)p.KT, (long)p.KT * read_ahead_cols(TM, TN, of) / max(cols, 1));
     if (2 * slabs < p.KT) return;
     for (int j = me * waves + wid; j < slabs; j += of * waves) {
         const int k = (int)((long)j * p.KT / slabs);
@@ -337,6 +340,9 @@ __global__ __launch_bounds__(64 * WM * WN, WPE) void gemm_mid_kernel(MidArgs p) 
     }
 }
 
+// CUs without a tile: up to four workgroups an XCD prefetch (one image 1561 us without, 1494 with two an XCD, 1371 with four, 1374 with eight)
+int read_ahead_workgroups(int tiles) { return tiles >= MID_CUS ? 0 : tiles > MID_CUS - 32 ? (MID_CUS - tiles) / 8 * 8 : 32; }
+
 template <int EPI, int MI, int NI, int WM, int WN, int S, int WPE, int KS, bool IL>
 void launch(hipStream_t st, MidArgs& p, bool alone) {
     constexpr int TM = 16 * MI * WM, TN = 16 * NI * WN, lds = S * KS * (TM + TN) * ROW_BYTES;
@@ -350,17 +356,29 @@ void launch(hipStream_t st, MidArgs& p, bool alone) {
     const int groups = (p.nbm + MAX_GROUP - 1) / MAX_GROUP;
     p.group = (p.nbm + groups - 1) / groups;
     p.ln_staged = (long)TM * p.ln_tiles * 8 <= KS * (TM + TN) * ROW_BYTES && ((long)p.M * p.ln_tiles) % 2 == 0;
-    // CUs without a tile: up to four workgroups an XCD prefetch (one image 1561 us without, 1494 with two an XCD, 1371 with four, 1374 with eight)
-    const int tiles = p.nbm * p.nbn, left = alone ? (MID_CUS - tiles) / 8 * 8 : 0;
-    const int extra = left < 0 ? 0 : left > 32 ? 32 : left;
+    const int tiles = p.nbm * p.nbn, extra = alone ? read_ahead_workgroups(tiles) : 0;
     hipLaunchKernelGGL((gemm_mid_kernel<EPI, MI, NI, WM, WN, S, WPE, KS, IL>), dim3(tiles + extra), dim3(64 * WM * WN), lds, st, p);
+}
+
+// 64x64 tiles, four ring slots or five: the fifth hides latency where the weights come from HBM -- the launch is slow for its lines, not
+// for its matrix instructions, and most of all where the last row tile is nearly empty: 200 x 3584 x 3584 17.0 -> 15.0 us, 129 x 4096 x 2048
+// 11.1 -> 10.1, 129 x 3584 x 1152 7.5 -> 7.1, whole row tiles 256 x 3584 x 3584 18.2 -> 17.4. It costs a slab's time in front of a short loop
+// (1024 x 1152 x 512 6.5 -> 6.9, 256 x 3584 x 768 level; up to twice as long a one with two workgroups on a CU, which hide each other's
+// latency: 1024 x 1152 x 1536 13.0 -> 13.5) and 1 to 4 % where every weight is read ahead into L2 (256 x 1152 x 1152 6.6 -> 6.8,
+// 256 x 1152 x 2560 10.3 -> 10.6).
+bool four_slots(const MidArgs& p, bool alone) {
+    const int nbm = (p.M + 63) / 64, tiles = nbm * ((p.N + 63) / 64), cols = ((tiles + 7) / 8 + nbm - 1) / nbm * 64;      // of an XCD
+    return p.KT <= (tiles > MID_CUS ? 24 : 12) || cols <= read_ahead_cols(64, 64, (alone ? read_ahead_workgroups(tiles) : 0) / 8);
 }
 
 template <int EPI>
 void dispatch_tile(hipStream_t st, MidArgs& p, int tile, bool alone) {
     switch (tile) {
         case 1: launch<EPI, 1, 2, 2, 2, 4, 2, 2, true>(st, p, alone); break;          // 32 x 64
-        case 2: launch<EPI, 2, 2, 2, 2, 4, 2, 1, true>(st, p, alone); break;          // 64 x 64, two a CU
+        case 2:                                                                       // 64 x 64, two a CU
+            if (four_slots(p, alone)) launch<EPI, 2, 2, 2, 2, 4, 2, 1, true>(st, p, alone);
+            else launch<EPI, 2, 2, 2, 2, 5, 2, 1, true>(st, p, alone);
+            break;
         case 3: launch<EPI, 2, 2, 4, 2, 3, 4, 1, false>(st, p, alone); break;         // 128 x 64, two a CU
         case 4: launch<EPI, 4, 2, 2, 4, 4, 2, 1, true>(st, p, alone); break;          // 128 x 128
         case 5: launch<EPI, 4, 4, 2, 4, 3, 2, 1, true>(st, p, alone); break;          // 128 x 256
