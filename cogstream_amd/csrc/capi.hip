@@ -79,6 +79,7 @@ cogs_status cogs_debug_get(const char* name, int64_t* value) {
     COGS_DEBUG_SWITCHES(COGS_DBG_GET)
 #undef COGS_DBG_GET
     if (strcmp(name, "gemm_last_body") == 0) { *value = g_cogs_debug.gemm_last_body; return COGS_OK; }
+    if (strcmp(name, "gemm_last_tile") == 0) { *value = g_cogs_debug.gemm_last_tile; return COGS_OK; }
     if (strcmp(name, "attn_last_kernel") == 0) { *value = g_cogs_debug.attn_last_kernel; return COGS_OK; }
     if (strcmp(name, "attn_last_rows") == 0) { *value = g_cogs_debug.attn_last_rows; return COGS_OK; }
     if (strcmp(name, "mla_last_waves") == 0) { *value = g_cogs_debug.mla_last_waves; return COGS_OK; }
@@ -94,6 +95,7 @@ const char* cogs_debug_list(void) {
 #undef COGS_DBG_DOC
         "gemm_last_body (read only): body the last cogs_gemm dispatched to -- 1 128x128 (fp32), 2 mid-size (fp32: 256x128), 3 K-tile ping-pong, "
         "4 whole-line ping-pong, 5 ping-pong + mid-size (split launch), 6 GEMV, 7 few-row GEMM\n"
+        "gemm_last_tile (read only): tile of the last mid-size bf16 product, numbered as in gemm_mid\n"
         "attn_last_kernel (read only): kernel of the last cogs_attention -- 1 general MFMA, 2 ViT unpipelined, 3 ViT pipelined, "
         "4 single-token decode, 5 prompt LDS-DMA, 7 row-wise fp32, 8 ViT pipelined on head-major K/V\n"
         "attn_last_rows (read only): query rows per workgroup of the last prompt attention (kernel 5), 64 or 128\n"

@@ -25,7 +25,7 @@
     X(gemm_group_m, 0, "> 0: row blocks per group of the ping-pong tile walk (0: chosen per shape)")                        \
     X(gemm_mid, 0, "> 0: this tile size of the mid-size kernel for every bf16 product of two or more rows (0: chosen per shape)") \
     X(gemm_split, 1, "0: what the ping-pong kernel can take is all its (no split, no mid-size kernel for few tiles)")                                                    \
-    X(gemm_co_streams, 0, "> 0: overrides the co-running-streams hint of the many-tile split")                              \
+    X(gemm_co_streams, 0, "> 0: overrides the co-running-streams hint (split, weights read ahead, choice of tile)")                              \
     X(gemm_epi_serial, 0, "1: the two wave groups' epilogues in separate intervals (the order before round 4)")             \
     X(gemm_nostore, 0, "1: timing only -- K loops without epilogues (results are NOT written)")                             \
     X(gemm_trace, 0, "1: per-tile s_memtime stamps of workgroup 0 printed to stderr (synchronises)")                        \
@@ -62,6 +62,8 @@ struct CogsDebug {
     // read-only reports (cogs_debug_get): what the last cogs_gemm of this process dispatched to
     // 0 none yet, 1 128x128 (fp32), 2 mid-size (fp32: 256x128), 3 K-tile ping-pong, 4 whole-line ping-pong, 5 ping-pong + mid-size (split), 6 GEMV, 7 few-row GEMM
     std::atomic<long long> gemm_last_body{0};
+    // ... and the tile of the last mid-size launch (the values of gemm_mid)
+    std::atomic<long long> gemm_last_tile{0};
     // ... and the last cogs_attention: 1 general MFMA kernel, 2 ViT unpipelined, 3 ViT pipelined (row-major K/V), 4 single-token
     // decode (+ combine), 5 prompt LDS-DMA kernel, 7 row-wise fp32 kernel, 8 ViT pipelined, head-major K/V (6 and 9 were the archived
     // ping-pong / 64-rows-per-wave prompt kernels: tools/experiments/attn_prefill_variants.hip)

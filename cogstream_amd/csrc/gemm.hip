@@ -927,7 +927,8 @@ __global__ __launch_bounds__(512, 2) void gemm_tn_pp64_kernel(GemmArgs p) {
 // report per-KERNEL averages that can be compared with rocprofv3's kernel stats
 static thread_local long g_gemm_launches = 0;
 // how many streams the caller is feeding with GEMMs of this size at the same time (cogs_vit_encode's two-stream mode: 2).
-// Only the many-tile split below reads it: a second stream fills the CUs that a launch's last round leaves idle.
+// A second stream fills the CUs that a launch's last round leaves idle: beside it a product of many tiles is not split, no workgroups
+// read weights ahead (gemm_mid.hip) and the choice leaves out the tile that wants every CU.
 static thread_local int g_co_streams = 1;
 void cogs_k_gemm_co_streams(int streams) { g_co_streams = streams < 1 ? 1 : streams; }
 long cogs_k_gemm_launch_count() { return g_gemm_launches; }
@@ -1118,12 +1119,15 @@ static float tile_time(int tiles, int slabs, float one, float two, float rest, f
     const int whole = tiles / (2 * PERSISTENT_WGS), left = tiles % (2 * PERSISTENT_WGS);
     return whole * (whole > 1 ? slabs * two * TWO_FULL + rest : t2) + (left == 0 ? 0.f : left <= PERSISTENT_WGS ? t1 : t2);
 }
-static int best_mid_tile(int M, int N, int K, bool ln_fold, float* time) {
+// alone: no other stream's products beside this one
+static int best_mid_tile(int M, int N, int K, bool ln_fold, bool alone, float* time) {
     int best = 0;
     for (const TileCost& t : MID_TILES) {
         const int tiles = (M + t.tm - 1) / t.tm * ((N + t.tn - 1) / t.tn);
-        // (160x64: its waves have more rows than lanes to hold their factors; three rounds of 150 x 37 888 x 3584 97 us, 128x128 88)
-        if (t.tile == 7 && (ln_fold || tiles > PERSISTENT_WGS)) continue;
+        // (160x64: its waves have more rows than lanes to hold their factors; three rounds of 150 x 37 888 x 3584 97 us, 128x128 88. Beside
+        // another stream, whose launch wants CUs too, its up to 256 workgroups of one to a CU leave none: 16 x 256 patches on two streams
+        // 5171 us with it, 4792 without; 5 x 924 5988 / 5604, 4 x 924 5283 / 4876, 8 x 924 7661 / 7663)
+        if (t.tile == 7 && (ln_fold || !alone || tiles > PERSISTENT_WGS)) continue;
         const float c = tile_time(tiles, K / 64, t.one, t.two, t.rest, MID_FULL);
         if (best == 0 || c < *time) { best = t.tile; *time = c; }
     }
@@ -1136,6 +1140,7 @@ static int finish_ln(hipStream_t st, const CogsGemm& g) {
 static int launch_mid(hipStream_t st, const CogsGemm& g, int tile, bool alone) {
     ++g_gemm_launches;
     g_cogs_debug.gemm_last_body = 2;
+    g_cogs_debug.gemm_last_tile = tile;
     return cogs_k_gemm_mid(st, g, tile, alone);
 }
 
@@ -1163,7 +1168,7 @@ static int gemm_rows(hipStream_t st, const CogsGemm& g, bool* kv_stored) {
     const int S = env_co > 0 ? env_co : g_co_streams;
     float mid_time = 0.f;
     const int env_mid = (int)g_cogs_debug.gemm_mid;
-    const int mid = g.dtype != COGS_DT_BF16 ? 0 : env_mid > 0 ? env_mid : best_mid_tile(g.M, g.N, g.K, g.ln_ab != nullptr, &mid_time);
+    const int mid = g.dtype != COGS_DT_BF16 ? 0 : env_mid > 0 ? env_mid : best_mid_tile(g.M, g.N, g.K, g.ln_ab != nullptr, S == 1, &mid_time);
     const int n_pad = (g.N + BN3 - 1) / BN3 * BN3;
     const bool pp_fits = n_pad * 100 <= g.N * (int)g_cogs_debug.gemm_pad_pct;   // default: <= 12 % of the MFMAs spent on N padding
     // (the ping-pong kernel wants two slabs and, below a row block, wastes its tiles' rows)
@@ -1244,7 +1249,7 @@ static int gemm_rows(hipStream_t st, const CogsGemm& g, bool* kv_stored) {
                 const int rows_rem = g.M - mb * BM3;
                 if (mb > 0 && rows_rem > 0) {
                     float rest;
-                    best_mid_tile(rows_rem, g.N, g.K, g.ln_ab != nullptr, &rest);
+                    best_mid_tile(rows_rem, g.N, g.K, g.ln_ab != nullptr, S == 1, &rest);
                     if (slabs * PP_SLAB + PP_REST + rest + SECOND_LAUNCH < best) mb_main = mb;
                 }
             }
@@ -1285,7 +1290,7 @@ static int gemm_rows(hipStream_t st, const CogsGemm& g, bool* kv_stored) {
             }
             // (straight to the kernel: a remainder may be one row, which cogs_k_gemm would take for a single-row product)
             float rest = 0.f;
-            const int rc3 = launch_mid(st, b, mb_main > 0 ? best_mid_tile(b.M, b.N, b.K, g.ln_ab != nullptr, &rest) : mid, S == 1);
+            const int rc3 = launch_mid(st, b, mb_main > 0 ? best_mid_tile(b.M, b.N, b.K, g.ln_ab != nullptr, S == 1, &rest) : mid, S == 1);
             if (mb_main > 0) g_cogs_debug.gemm_last_body = 5;
             return rc3;
         }

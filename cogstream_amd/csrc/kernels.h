@@ -51,7 +51,7 @@ struct CogsGemm {
 };
 int cogs_k_gemm(hipStream_t st, const CogsGemm& g);
 int cogs_k_gemm_mid(hipStream_t st, const CogsGemm& g, int tile, bool alone);     // gemm_mid.hip; the caller (cogs_k_gemm) has checked the operands. alone: no other stream's products beside it
-void cogs_k_gemm_co_streams(int streams);   // streams fed with GEMMs of this size at once (thread-local): beside another stream a product of many tiles is not split
+void cogs_k_gemm_co_streams(int streams);   // streams fed with GEMMs of this size at once (thread-local): beside another stream a product of many tiles is not split, weights are not read ahead
 // (a, b) = (rstd, -rstd * mean) per row from the EPI_ROWSTAT partials [rows][tiles][2]: ab [rows][2]
 int cogs_k_ln_finalize(hipStream_t st, const float* stat_part, int rows, int tiles, int H, float eps, float* ab);
 

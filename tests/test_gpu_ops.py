@@ -1181,6 +1181,21 @@ def test_mid_size_gemm_tiles_equal_each_other_and_fp64(dev, tile):
                 assert bool(((x.double() - ref).abs() <= bound * 1.01).all()), (M, N, K, name)
 
 
+@pytest.mark.parametrize("M,N,K", [(600, 3584, 3584), (600, 3584, 18944), (2048, 1152, 4352)])
+def test_tiles_that_want_every_cu_are_not_chosen_beside_another_stream(dev, M, N, K):
+    """160x64 is for a product that has the chip to itself; the bits do not depend on it"""
+    from cogstream_amd import _lib as L2
+    ops = _ops()
+    g = torch.Generator(device=dev).manual_seed(M + K)
+    a, w = (torch.randn(*s, generator=g, device=dev).bfloat16() for s in ((M, K), (N, K)))
+    alone = ops.gemm(a, w)
+    assert L2.debug_get("gemm_last_tile") == 7
+    with L2.debug_switch("gemm_co_streams", 2):
+        beside = ops.gemm(a, w)
+        assert L2.debug_get("gemm_last_tile") in (4, 5)
+    assert torch.equal(alone, beside)
+
+
 @pytest.mark.parametrize("tile", [6, 7])
 def test_mid_size_gemm_tiles_of_two_slabs_and_of_160_rows(dev, tile):
     """the same edges for 128x64 with two slabs a slot and 160x64 (five row blocks a wave; a folded norm falls back to 128x64)"""
