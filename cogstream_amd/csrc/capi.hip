@@ -79,6 +79,7 @@ cogs_status cogs_debug_get(const char* name, int64_t* value) {
     COGS_DEBUG_SWITCHES(COGS_DBG_GET)
 #undef COGS_DBG_GET
     if (strcmp(name, "gemm_last_body") == 0) { *value = g_cogs_debug.gemm_last_body; return COGS_OK; }
+    if (strcmp(name, "vit_last_streams") == 0) { *value = g_cogs_debug.vit_last_streams; return COGS_OK; }
     if (strcmp(name, "gemm_last_tile") == 0) { *value = g_cogs_debug.gemm_last_tile; return COGS_OK; }
     if (strcmp(name, "attn_last_kernel") == 0) { *value = g_cogs_debug.attn_last_kernel; return COGS_OK; }
     if (strcmp(name, "attn_last_rows") == 0) { *value = g_cogs_debug.attn_last_rows; return COGS_OK; }
@@ -101,6 +102,7 @@ const char* cogs_debug_list(void) {
         "attn_last_rows (read only): query rows per workgroup of the last prompt attention (kernel 5), 64 or 128\n"
         "attn_vit_last_end (read only): ragged end of the last pipelined ViT attention launch -- 10 x tiles behind the four-tile loop + "
         "32-key blocks of the last tile (41 .. 72: compile-time shape), 0 the run-time form\n"
+        "vit_last_streams (read only): streams the last cogs_vit_encode was queued on\n"
         "mla_last_waves (read only): waves per query tile of the last prompt attention of a described decoder in bf16, 4 or 8\n"
         "km_pp_last_launches (read only): kernels per centre of the last cogs_kmeans_pp, 1 or 3\n";
 }
@@ -369,7 +371,7 @@ static size_t vit_carve(const cogs_vit_weights& w, int64_t N, int nframes, Carve
 }
 
 cogs_status cogs_vit_set_streams(cogs_handle h, int streams) {
-    if (!h || streams < 1 || streams > 4) return COGS_E_INVALID;
+    if (!h || streams < 0 || streams > 4) return COGS_E_INVALID;
     h->vit_streams = streams;
     return COGS_OK;
 }
@@ -442,6 +444,7 @@ static cogs_status vit_encode_impl(cogs_handle h, cogs_stream stream, const void
     }
     const cogs_vit_weights& w = h->vit;
     auto whole = [&]() {
+        g_cogs_debug.vit_last_streams = 1;
         VitRange r{h, st, pixel_values, pix_dtype, std::vector<int64_t>(grid_sizes, grid_sizes + 3 * V),
                    std::vector<int64_t>(merge_sizes, merge_sizes + V), attn_mode, out_tokens, ws, ws_bytes};
         COGS_TRY(r.begin());
@@ -518,6 +521,7 @@ static cogs_status vit_encode_impl(cogs_handle h, cogs_stream stream, const void
     }
     if (!h->ev_fork && hipEventCreateWithFlags(&h->ev_fork, hipEventDisableTiming) != hipSuccess) return whole();
     if (hipEventRecord(h->ev_fork, st) != hipSuccess) return COGS_E_HIP;
+    g_cogs_debug.vit_last_streams = S;
     R[0].st = st;
     for (int r = 1; r < S; ++r) {
         R[r].st = h->aux_streams[r - 1];

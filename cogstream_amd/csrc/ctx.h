@@ -42,7 +42,7 @@ struct cogs_ctx {
     std::vector<hipStream_t> aux_streams;
     hipEvent_t ev_fork = nullptr;
     std::vector<hipEvent_t> ev_joins;
-    int vit_streams = 0;                  // cogs_vit_set_streams: 1 = never split; 0: two from VIT_SPLIT_MIN patches on
+    int vit_streams = 0;                  // cogs_vit_set_streams: 1 = never split; 0: by the clip's size (VIT_SPLIT_MIN)
     // optional per-kernel-class event profiling (bench/roofline only)
     bool prof_on = false;
     std::vector<hipEvent_t> prof_ev;      // pairs

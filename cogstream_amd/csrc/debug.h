@@ -72,6 +72,8 @@ struct CogsDebug {
     std::atomic<long long> attn_last_rows{0};
     // ... and which ragged end the last pipelined ViT launch had: 10 R + blocks of the last tile (41 .. 72), 0 = the run-time form
     std::atomic<long long> attn_vit_last_end{0};
+    // ... and the streams the last cogs_vit_encode was queued on
+    std::atomic<long long> vit_last_streams{0};
     // ... and the last prompt attention of a described decoder (bf16): waves per query tile, 4 or 8
     std::atomic<long long> mla_last_waves{0};
     // ... and the last cogs_kmeans_pp: kernels launched per centre, 1 or 3

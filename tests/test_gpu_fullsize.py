@@ -312,7 +312,7 @@ def test_share_sized_clip_is_bit_identical_on_1_to_4_streams(dev):
             L.check(L.lib.cogs_vit_set_streams(enc.handle.h, s))
             outs[s] = enc(pix, grid, merge).clone()
     finally:
-        L.check(L.lib.cogs_vit_set_streams(enc.handle.h, 2))
+        L.check(L.lib.cogs_vit_set_streams(enc.handle.h, 0))
     torch.cuda.synchronize()
     assert torch.isfinite(outs[1].float()).all()
     for s in (2, 3, 4):

@@ -55,7 +55,7 @@ def test_vit_bf16_pixel_input_and_frame_independence(dev):
 
 
 def test_frame_split_two_stream_encode_is_transparent(dev):
-    """cogs_vit_encode cuts a small clip at the frame boundary nearest to half its patches and encodes the halves on two
+    """told to, cogs_vit_encode cuts a small clip at the frame boundary nearest to half its patches and encodes the halves on two
     streams (frames are independent in block-diagonal mode). Three videos of different grids in ONE call -- the cut falls
     inside the second one, the halves see different video lists, the attention's uniform-segment shortcut is off -- must
     equal (bit for bit) the concatenation of one encode per video, and the oracle within bf16 tolerance; a workspace too
@@ -69,14 +69,20 @@ def test_frame_split_two_stream_encode_is_transparent(dev):
     merges = torch.tensor([2, 2, 2])
     rows = [int(t * a * b) for t, a, b in grids.tolist()]
     pix = (torch.rand(sum(rows), 588) * 2 - 1).bfloat16().to(dev)
-    whole = enc(pix, grids, merges)
-    parts, r0 = [], 0
-    for v in range(3):
-        parts.append(enc(pix[r0:r0 + rows[v]], grids[v:v + 1], merges[v:v + 1]))
-        r0 += rows[v]
-    assert torch.equal(whole, torch.cat(parts))
-    again = enc(pix, grids, merges)
-    assert torch.equal(whole, again)
+    request_streams = lambda n: L.check(L.lib.cogs_vit_set_streams(enc.handle.h, n))
+    try:
+        request_streams(2)
+        whole = enc(pix, grids, merges)
+        assert L.debug_get("vit_last_streams") == 2
+        parts, r0 = [], 0
+        for v in range(3):
+            parts.append(enc(pix[r0:r0 + rows[v]], grids[v:v + 1], merges[v:v + 1]))
+            r0 += rows[v]
+        assert torch.equal(whole, torch.cat(parts))
+        again = enc(pix, grids, merges)
+        assert torch.equal(whole, again)
+    finally:
+        request_streams(0)
     ref = ov.encode(st, pix.float().cpu(), grids, merges, heads=cfg.num_attention_heads, layers=cfg.num_hidden_layers, mode=0)
     assert rel_err(whole.float(), ref) < 3e-2
     # exactly the single-stream workspace (the query adds room for the second set of tables): still fine, same tokens
@@ -87,24 +93,52 @@ def test_frame_split_two_stream_encode_is_transparent(dev):
     out = torch.empty_like(whole)
     gs = (C.c_int64 * 9)(*[int(x) for x in grids.reshape(-1).tolist()])
     ms = (C.c_int64 * 3)(2, 2, 2)
-    rc = L.lib.cogs_vit_encode(enc.handle.h, L.current_stream(), pix.data_ptr(), L.dtype_code(pix.dtype), gs, ms, 3, 0,
-                               out.data_ptr(), ws.data_ptr(), ws.numel())
+    try:
+        request_streams(2)
+        rc = L.lib.cogs_vit_encode(enc.handle.h, L.current_stream(), pix.data_ptr(), L.dtype_code(pix.dtype), gs, ms, 3, 0,
+                                   out.data_ptr(), ws.data_ptr(), ws.numel())
+        assert L.debug_get("vit_last_streams") == 1
+    finally:
+        request_streams(0)
     torch.cuda.synchronize()
     assert rc == L.OK and torch.equal(out, whole)
     # split against UNSPLIT, explicitly: cogs_vit_set_streams(1) keeps the clip on the caller's stream
     try:
         L.check(L.lib.cogs_vit_set_streams(enc.handle.h, 1))
         single = enc(pix, grids, merges)
+        assert L.debug_get("vit_last_streams") == 1
     finally:
-        L.check(L.lib.cogs_vit_set_streams(enc.handle.h, 2))
+        L.check(L.lib.cogs_vit_set_streams(enc.handle.h, 0))
     assert torch.equal(single, whole)
     for streams in (3, 4):                       # three frame ranges (one per video here) / four (more ranges than videos)
         try:
             L.check(L.lib.cogs_vit_set_streams(enc.handle.h, streams))
             assert torch.equal(enc(pix, grids, merges), whole), streams
+            assert L.debug_get("vit_last_streams") == streams
         finally:
-            L.check(L.lib.cogs_vit_set_streams(enc.handle.h, 2))
-    assert L.lib.cogs_vit_set_streams(enc.handle.h, 5) == L.E_INVALID
+            L.check(L.lib.cogs_vit_set_streams(enc.handle.h, 0))
+    assert L.lib.cogs_vit_set_streams(enc.handle.h, 5) == L.E_INVALID and L.lib.cogs_vit_set_streams(enc.handle.h, -1) == L.E_INVALID
+
+
+@pytest.mark.parametrize("t,gh,gw,streams", [(18, 16, 16, 1), (3, 40, 40, 2), (1, 72, 72, 1)])
+def test_streams_of_a_clip_by_its_patches(dev, t, gh, gw, streams):
+    """where the caller has not said how many, or has given the choice back: one stream up to 4699 patches (4608 here), two from there on (4800),
+    one for one frame; the tokens are those of one stream"""
+    from cogstream_amd import _lib as L
+    from cogstream_amd.vision import VisionEncoder
+    from cogstream_amd.weights import VisionConfig, random_vit_state
+    vcfg = VisionConfig(hidden_size=576, intermediate_size=200, num_hidden_layers=2, num_attention_heads=8)
+    enc = VisionEncoder(random_vit_state(vcfg, seed=4, std=0.05), vcfg, dtype=torch.bfloat16, device=dev)
+    pix = (torch.rand(t * gh * gw, 588, generator=torch.Generator(device=dev).manual_seed(t), device=dev) * 2 - 1).bfloat16()
+    grid, merge = torch.tensor([[t, gh, gw]]), torch.tensor([2])
+    try:
+        L.check(L.lib.cogs_vit_set_streams(enc.handle.h, 1))
+        want = enc(pix, grid, merge)
+        assert L.debug_get("vit_last_streams") == 1
+    finally:
+        L.check(L.lib.cogs_vit_set_streams(enc.handle.h, 0))
+    assert torch.equal(enc(pix, grid, merge), want)
+    assert L.debug_get("vit_last_streams") == streams
 
 
 @pytest.mark.parametrize("dtype,tol", [(torch.float32, 1e-4), (torch.bfloat16, 2e-2)])
@@ -719,4 +753,4 @@ def test_encode_project_equals_encoder_then_projector_bit_for_bit(dev):
             assert torch.equal(tok2, tok), s
             assert torch.equal(got, want), (s, float((got.float() - want.float()).abs().max()))
     finally:
-        L.check(L.lib.cogs_vit_set_streams(enc.handle.h, 2))
+        L.check(L.lib.cogs_vit_set_streams(enc.handle.h, 0))
