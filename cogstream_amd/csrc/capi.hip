@@ -418,14 +418,14 @@ struct VitRange {
 // 64-frame clip 2.7 % (round 4, same box, interleaved: 60.8 -> 59.2 ms; 256 frames at 140 x 280: 47.3 -> 46.5 ms).
 // Shorter clips run on one stream unless the caller has said how many: their products leave CUs idle anyway, which then fetch weights
 // ahead (gemm_mid.hip), one launch of twice the rows against two that share the chip. One stream / two, us, frames x patches:
-//   8 x 256 3129 / 3227, 12 x 256 3706 / 4318, 14 x 256 4158 / 4423, 16 x 256 4823 / 4737, 18 x 256 5024 / 5275, 20 x 256 5575 / 5393,
-//   2 x 924 2972 / 3262, 4 x 924 4801 / 4752, 5 x 924 5639 / 5401, 6 x 924 6273 / 6329, 8 x 924 8674 / 7579, 2 x 1200 4064 / 4020, 3 x 1200
-//   4837 / 5032, 4 x 1200 6002 / 5880, 6 x 1200 8843 / 7731, 2 x 1600 4430 / 4778, 3 x 1600 6377 / 6025, 8 x 576 5195 / 5352, 9 x 576 5802 /
-//   5828, 20 x 200 4862 / 4705, 22 x 200 5037 / 5199, 24 x 200 5468 / 5444, 2 x 1936 5447 / 5451, 3 x 1936 7435 / 7176
+//   8 x 256 3198 / 3314, 12 x 256 3776 / 4428, 18 x 256 5258 / 5395, 20 x 256 5767 / 5454, 2 x 924 3066 / 3355, 4 x 924 4924 / 5333,
+//   5 x 924 5853 / 5967, 6 x 924 6469 / 6366, 2 x 1200 4065 / 4094, 3 x 1200 4952 / 5189, 4 x 1200 6159 / 5926, 5 x 1200 7303 / 6799,
+//   2 x 1600 4495 / 4882, 3 x 1600 6456 / 5967, 8 x 576 5355 / 5397, 9 x 576 5939 / 5979, 2 x 1936 5563 / 5689, 3 x 1936 7628 / 7410,
+//   16 x 924 14 544 / 13 465
 // Not while the per-kernel profiler is on: overlapping launches stretch every bracket, so bench.py's `roofline` and
 // `breakdown_ms` describe the kernels one at a time. cogs_vit_set_streams(h, 1) or the debug switch vit_split_max switch it off.
 
-constexpr int64_t VIT_SPLIT_MIN = 4610;      // patches
+constexpr int64_t VIT_SPLIT_MIN = 4700;      // patches
 
 static cogs_status cogs_project_rows(cogs_handle h, hipStream_t st, const void* tokens, int M, void* out, void* ws);
 
