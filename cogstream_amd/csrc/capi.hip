@@ -418,10 +418,10 @@ struct VitRange {
 // 64-frame clip 2.7 % (round 4, same box, interleaved: 60.8 -> 59.2 ms; 256 frames at 140 x 280: 47.3 -> 46.5 ms).
 // Shorter clips run on one stream unless the caller has said how many: their products leave CUs idle anyway, which then fetch weights
 // ahead (gemm_mid.hip), one launch of twice the rows against two that share the chip. One stream / two, us, frames x patches:
-//   8 x 256 3198 / 3314, 12 x 256 3776 / 4428, 18 x 256 5258 / 5395, 20 x 256 5767 / 5454, 2 x 924 3066 / 3355, 4 x 924 4924 / 5333,
-//   5 x 924 5853 / 5967, 6 x 924 6469 / 6366, 2 x 1200 4065 / 4094, 3 x 1200 4952 / 5189, 4 x 1200 6159 / 5926, 5 x 1200 7303 / 6799,
-//   2 x 1600 4495 / 4882, 3 x 1600 6456 / 5967, 8 x 576 5355 / 5397, 9 x 576 5939 / 5979, 2 x 1936 5563 / 5689, 3 x 1936 7628 / 7410,
-//   16 x 924 14 544 / 13 465
+//   8 x 256 3129 / 3227, 12 x 256 3706 / 4318, 16 x 256 4767 / 4807, 18 x 256 4986 / 5326, 19 x 256 5469 / 5542, 20 x 256 5558 / 5510,
+//   2 x 924 2972 / 3262, 4 x 924 4802 / 4916, 5 x 924 5616 / 5642, 8 x 924 8674 / 7579, 3 x 1200 4837 / 5032, 4 x 1200 6042 / 6063,
+//   6 x 1200 8843 / 7731, 2 x 1600 4430 / 4778, 3 x 1600 6312 / 6225, 8 x 576 5143 / 5496, 9 x 576 5802 / 5828, 20 x 200 4806 / 4801,
+//   23 x 200 5137 / 5484, 24 x 200 5413 / 5482, 2 x 1936 5447 / 5451, 3 x 1936 7435 / 7176, 16 x 924 14 544 / 13 465
 // Not while the per-kernel profiler is on: overlapping launches stretch every bracket, so bench.py's `roofline` and
 // `breakdown_ms` describe the kernels one at a time. cogs_vit_set_streams(h, 1) or the debug switch vit_split_max switch it off.
 
