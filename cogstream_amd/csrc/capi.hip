@@ -931,12 +931,18 @@ static cogs_status llm_forward_impl(cogs_handle h, cogs_stream stream, const voi
             g.rope_cos = rc; g.rope_sin = rs; g.rope_cols = qd_q + kvd; g.head_dim = hd;
             if (prescale_q) { g.q_scale = scale * 1.4426950408889634f; g.q_cols = qd_q; }
             if (fuse_norm) { g.rms_gamma = L.in_ln; g.rms_eps = w.rms_eps; }
-            if (kv) {             // new K / V rows go straight into the cache (or through C where the product's kernel cannot)
+            if (kv) {             // new K / V rows go straight into the cache where the product's kernel can
                 g.kv_k = (char*)kv->k + (((size_t)l * kv->max_len) + pos0) * kvd * es;
                 g.kv_v = (char*)kv->v + (((size_t)l * kv->max_len) + pos0) * kvd * es;
                 g.kv_col0 = qd_q; g.kv_dim = kvd;
             }
-            { PROF(COGS_PROF_GEMM); COGS_TRY(cogs_k_gemm(st, g)); }
+            bool kv_stored = true;
+            { PROF(COGS_PROF_GEMM); COGS_TRY(cogs_k_gemm(st, g, &kv_stored)); }
+            if (kv && !kv_stored) {
+                PROF(COGS_PROF_OTHER);
+                const char* k = (const char*)qkv + (size_t)qd_q * es;
+                COGS_TRY(cogs_k_kv_append(st, dt, k, k + (size_t)kvd * es, qd, g.kv_k, g.kv_v, kvd, S, kvd));
+            }
         }
         const char* kp = (const char*)qkv + (size_t)qd_q * es;
         const char* vp = kp + (size_t)kvd * es;

@@ -1307,10 +1307,9 @@ static int gemm_rows(hipStream_t st, const CogsGemm& g, bool* kv_stored) {
     return COGS_LAUNCH_CHECK();
 }
 
-int cogs_k_gemm(hipStream_t st, const CogsGemm& g) {
-    bool kv_stored = g.M == 1 || !g.kv_k;
-    const int rc = gemm_rows(st, g, &kv_stored);
-    if (rc != COGS_OK || kv_stored) return rc;
-    const char* k = (const char*)g.C + (size_t)g.kv_col0 * (g.dtype == COGS_DT_BF16 ? 2 : 4);
-    return cogs_k_kv_append(st, g.dtype, k, k + (size_t)g.kv_dim * (g.dtype == COGS_DT_BF16 ? 2 : 4), g.ldc, g.kv_k, g.kv_v, g.kv_dim, g.M, g.kv_dim);
+int cogs_k_gemm(hipStream_t st, const CogsGemm& g, bool* kv_stored) {
+    bool stored = g.M == 1;
+    const int rc = gemm_rows(st, g, &stored);
+    if (kv_stored) *kv_stored = stored;
+    return rc;
 }

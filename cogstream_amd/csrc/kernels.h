@@ -28,7 +28,7 @@ struct CogsGemm {
     const void* rms_gamma = nullptr;         // M == 1 only: RMS-normalise A on the fly with this weight
     float rms_eps = 0.f;
     // output columns [kv_col0, kv_col0 + kv_dim) go to rows of kv_dim at kv_k, the next kv_dim to kv_v (C may be left without them)
-    // (the single-row and the mid-size bf16 kernel store them themselves, behind the others they are copied)
+    // (the single-row and the mid-size bf16 kernel store them themselves; behind the others the caller copies them, see kv_stored)
     void* kv_k = nullptr; void* kv_v = nullptr; int kv_col0 = 0; int kv_dim = 0;
     // rope epilogues only: columns [0, q_cols) (the Q heads) are multiplied by q_scale before rounding
     float q_scale = 1.f; int q_cols = 0;
@@ -49,7 +49,7 @@ struct CogsGemm {
     // forms each row's factor itself, or cogs_k_ln_finalize runs first
     const float* ln_part = nullptr; float ln_eps = 0.f;
 };
-int cogs_k_gemm(hipStream_t st, const CogsGemm& g);
+int cogs_k_gemm(hipStream_t st, const CogsGemm& g, bool* kv_stored = nullptr);     // kv_stored (for a call with kv_k): false: the caller copies them from C
 int cogs_k_gemm_mid(hipStream_t st, const CogsGemm& g, int tile, bool alone);     // gemm_mid.hip; the caller (cogs_k_gemm) has checked the operands. alone: no other stream's products beside it
 void cogs_k_gemm_co_streams(int streams);   // streams fed with GEMMs of this size at once (thread-local): beside another stream a product of many tiles is not split, weights are not read ahead
 // (a, b) = (rstd, -rstd * mean) per row from the EPI_ROWSTAT partials [rows][tiles][2]: ab [rows][2]

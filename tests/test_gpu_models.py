@@ -183,6 +183,25 @@ def test_keys_and_values_stored_by_the_qkv_product(dev, tile, split):
             assert torch.equal(torch.cat(got), want[:sum(p.shape[0] for p in got)])
 
 
+@pytest.mark.parametrize("dtype,split,copies", [(torch.bfloat16, 1, 0), (torch.bfloat16, 0, 2), (torch.float32, 1, 2)])
+def test_copies_of_keys_and_values_are_no_product(dev, dtype, split, copies):
+    """profile classes of a prompt: what copies K and V behind a product that cannot store them is no time of the product's"""
+    import ctypes as C
+    from cogstream_amd import _lib as L
+    cfg, st, eng = _llm(dev, dtype)
+    x = torch.randn(300, cfg.hidden_size, generator=torch.Generator(device=dev).manual_seed(9), device=dev).to(dtype)
+    counts = []
+    for cache in (None, eng.new_cache(300)):
+        with L.debug_switch("gemm_split", split):
+            L.check(L.lib.cogs_profile_begin(eng.handle.h))
+            eng.forward(x, cache)
+            ms, n = (C.c_float * 4)(), (C.c_int * 4)()
+            L.check(L.lib.cogs_profile_end(eng.handle.h, L.current_stream(), ms, n))
+        counts.append(list(n))
+    assert cfg.num_hidden_layers == 2 and counts[0][0] == counts[1][0]
+    assert counts[1][3] - counts[0][3] == copies, counts
+
+
 @pytest.mark.parametrize("dtype,tol", [(torch.float32, 1e-4), (torch.bfloat16, 3e-2)])
 def test_llm_prefill_and_decode_vs_oracle(dev, dtype, tol):
     from oracle import qwen2 as oq
