@@ -84,6 +84,7 @@ cogs_status cogs_debug_get(const char* name, int64_t* value) {
     if (strcmp(name, "attn_last_kernel") == 0) { *value = g_cogs_debug.attn_last_kernel; return COGS_OK; }
     if (strcmp(name, "attn_last_rows") == 0) { *value = g_cogs_debug.attn_last_rows; return COGS_OK; }
     if (strcmp(name, "mla_last_waves") == 0) { *value = g_cogs_debug.mla_last_waves; return COGS_OK; }
+    if (strcmp(name, "preprocess_last_kernel") == 0) { *value = g_cogs_debug.preprocess_last_kernel; return COGS_OK; }
     if (strcmp(name, "km_pp_last_launches") == 0) { *value = g_cogs_debug.km_pp_last_launches; return COGS_OK; }
     if (strcmp(name, "attn_vit_last_end") == 0) { *value = g_cogs_debug.attn_vit_last_end; return COGS_OK; }
     return COGS_E_INVALID;
@@ -104,6 +105,8 @@ const char* cogs_debug_list(void) {
         "32-key blocks of the last tile (41 .. 72: compile-time shape), 0 the run-time form\n"
         "vit_last_streams (read only): streams the last cogs_vit_encode was queued on\n"
         "mla_last_waves (read only): waves per query tile of the last prompt attention of a described decoder in bf16, 4 or 8\n"
+        "preprocess_last_kernel (read only): kernel of the last cogs_preprocess_frames -- 1 two passes, 2 vector tiles, else matrix products: "
+        "100 x 64-byte steps of a row + 10 x patch rows of a band + 16-row tiles of its source rows\n"
         "km_pp_last_launches (read only): kernels per centre of the last cogs_kmeans_pp, 1 or 3\n";
 }
 

@@ -76,6 +76,9 @@ struct CogsDebug {
     std::atomic<long long> vit_last_streams{0};
     // ... and the last prompt attention of a described decoder (bf16): waves per query tile, 4 or 8
     std::atomic<long long> mla_last_waves{0};
+    // ... and the last cogs_preprocess_frames: 1 two passes, 2 vector tiles, else matrix products: 100 x 64-byte steps + 10 x patch rows of a band +
+    // 16-row tiles of its source rows
+    std::atomic<long long> preprocess_last_kernel{0};
     // ... and the last cogs_kmeans_pp: kernels launched per centre, 1 or 3
     std::atomic<long long> km_pp_last_launches{0};
 };

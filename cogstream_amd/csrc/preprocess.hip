@@ -7,11 +7,13 @@
 // built on the host by cogstream_amd.processing.resample_coeffs, uint8 rounding after each pass), so the uint8
 // image -- and, through the [3,256] value table (processing.pixel_value_table), pixel_values -- is bit-identical to the reference's host path.
 // resize_mfma_kernel does both passes as integer matrix products; resize_patchify_kernel does them with vector instructions where a patch's
-// taps span more than 48 source pixels or a band's more than 64 rows (shrinking by more than about 2.6), or a row has fewer pixels than the
-// products take; the two-pass kernels remain for shrinking by so much that a tile's intermediate rows do not fit the LDS, and for outputs
+// taps span more than 48 source pixels or a band's more than 64 rows (shrinking by more than about 2.6), a row has fewer pixels than the
+// products take, or large images come one or a few at a time (vector_is_faster); the two-pass kernels remain for shrinking by so much that a tile's intermediate rows do not fit the LDS, and for outputs
 // that are not aligned to a pair of elements.
 #include "common.h"
 #include "kernels.h"
+#include "debug.h"
+#include <algorithm>
 
 namespace {
 
@@ -379,7 +381,17 @@ inline double tap_span(int in_size, int out_size, int outputs) {
     const double scale = (double)in_size / out_size, wide = scale > 1.0 ? scale : 1.0;
     return (outputs - 1) * scale + 4 * wide + 3;
 }
-// false: sizes this kernel does not take (columns above 48 source pixels or more than the row has, bands above 64 source rows)
+// A wave's prologue, the taps in the order of its lanes, costs one and a half frames, and the waves of a large image by itself are more than the
+// chip holds: with few frames a wave and few taps an output the vector form is the faster. Times in ns a patch, the prologue over its frames
+// here, the taps' growth with the scale there, and 1.7 us more for a launch of that one. Vector / products, us: 1 x 1080 x 1920 -> 1078 x 1918
+// 19.8 / 33.6, two frames 33.2 / 43.8, three 44.5 / 53.9; 1 x 720 x 1280 -> 546 x 966 10.0 / 11.7, two 15.7 / 15.0; bands of two patches, 1 x
+// 1440 x 2560 -> 1428 x 2548 32.4 / 39.6, -> 1008 x 1792 23.9 / 21.7; 2 x 2160 x 3840 -> 2156 x 3836 91 / 102, 4 x 720 x 1280 -> 728 x 1288
+// 31.8 / 28.5. The other form taken costs 6 % at the most over 200 such launches, scales 0.8 to 1.5, one to three frames.
+bool vector_is_faster(long waves, int frames, int bp, double scale) {
+    const double patches = 1e-3 * waves * frames * bp;
+    return waves > MM_RESIDENT && (bp == 1 ? 0.92 : 0.65) * (1 + 1.5 / frames) * patches > ((scale > 1 ? scale : 1) + 0.05) * patches + 1.7;
+}
+// false: sizes this kernel does not take (columns above 48 source pixels or more than the row has, bands above 64 source rows) or is slower for
 template <typename TO>
 bool launch_mfma(hipStream_t st, const uint8_t* frames, TO* out, int T, int H, int W, int th, int tw, int ms, const int* bx, const int* kx, int ksx,
                  const int* by, const int* ky, int ksy, const float* table) {
@@ -399,6 +411,7 @@ bool launch_mfma(hipStream_t st, const uint8_t* frames, TO* out, int T, int H, i
     }
     const long units = columns * ((T + each - 1) / each), grid = (units + MM_WAVES - 1) / MM_WAVES;
     if (grid > 0x7fffffff) return false;
+    if (steps == 2 && ksx <= 7 && ksy <= 7 && vector_is_faster(units, each, bp, std::max((double)W / tw, (double)H / th))) return false;
     const int tiles = (int)((tap_span(H, th, 14 * bp) + 15) / 16);
 #define COGS_MM(KS, BP, RT) hipLaunchKernelGGL((resize_mfma_kernel<TO, KS, BP, RT>), dim3((unsigned)grid), dim3(64 * MM_WAVES), 0, st, frames, out, T, H, W, gh, gw, ms, each, bx, kx, ksx, by, ky, ksy, table)
     if (bp == 2) { if (tiles <= 3) COGS_MM(2, 2, 3); else COGS_MM(2, 2, 4); }
@@ -406,6 +419,7 @@ bool launch_mfma(hipStream_t st, const uint8_t* frames, TO* out, int T, int H, i
     else if (tiles <= 3) COGS_MM(3, 1, 3);
     else COGS_MM(3, 1, 4);
 #undef COGS_MM
+    g_cogs_debug.preprocess_last_kernel = 100 * steps + 10 * bp + (tiles <= 3 ? 3 : 4);
     return true;
 }
 
@@ -450,6 +464,7 @@ int cogs_k_preprocess(hipStream_t st, const uint8_t* frames, int T, int H, int W
             (out_dtype == COGS_DT_BF16 ? launch_mfma<bf16_t>(st, frames, (bf16_t*)out, T, H, W, th, tw, ms, bx, kx, ksx, by, ky, ksy, table)
                                        : launch_mfma<float>(st, frames, (float*)out, T, H, W, th, tw, ms, bx, kx, ksx, by, ky, ksy, table)))
             return COGS_LAUNCH_CHECK();
+        g_cogs_debug.preprocess_last_kernel = 2;
         if (lds <= 64 * 1024 && ksx <= 24 && (reinterpret_cast<size_t>(out) & (pair - 1)) == 0 && grid < 0x7fffffff) {
             if (out_dtype == COGS_DT_BF16)
                 dispatch_fused<bf16_t>(st, lds, (int)grid, frames, (bf16_t*)out, T, H, W, gh1, gw1, ms, band_p, max_rows, bx, kx, ksx, by, ky, ksy, table);
@@ -458,6 +473,7 @@ int cogs_k_preprocess(hipStream_t st, const uint8_t* frames, int T, int H, int W
             return COGS_LAUNCH_CHECK();
         }
     }
+    g_cogs_debug.preprocess_last_kernel = 1;
     const long rows = (long)T * H;
     hipLaunchKernelGGL(resize_h_kernel, dim3(grid_for(rows * tw)), dim3(256), 0, st, frames, tmp, rows, W, tw, bx, kx, ksx);
     const int gh = th / 14, gw = tw / 14;

@@ -1241,6 +1241,20 @@ def test_resize_as_matrix_products_equals_the_host_path(dev, t, h, w, merge, max
     test_fused_resize_equals_the_host_path(dev, t, h, w, merge, max_tokens, offset)
 
 
+@pytest.mark.parametrize("t,h,w,merge,max_tokens,want", [
+    (1, 602, 798, 1, 16384, 2),          # a large image by itself: more waves than the chip holds, a prologue each
+    (1, 728, 1288, 2, 16384, 2),         # bands of two patches
+    (1, 480, 640, 1, 16384, 223),        # as many waves as it holds
+    (3, 336, 518, 1, 16384, 223),        # several frames a wave
+    (4, 728, 1288, 2, 16384, 223),
+])
+def test_resize_of_large_images_takes_the_faster_form(dev, t, h, w, merge, max_tokens, want):
+    """matrix products or vector instructions, the bytes of the host path either way"""
+    from cogstream_amd import _lib as L2
+    test_fused_resize_equals_the_host_path(dev, t, h, w, merge, max_tokens, 1)
+    assert L2.debug_get("preprocess_last_kernel") == want
+
+
 def test_tap_tables_outlive_their_place_in_the_cache(dev):
     """a resize queued on a side stream, and tables that leave the cache before it runs: their memory, asked for again on the stream that
     made them, is not theirs until the resize is done. (Zeros in it would be tables of no taps: a black clip, no read out of place)"""
