@@ -1204,7 +1204,7 @@ def test_mid_size_gemm_tiles_of_two_slabs_and_of_160_rows(dev, tile):
 
 @pytest.mark.parametrize("t,h,w,merge,max_tokens,offset", [
     (1, 28, 28, 2, 16384, 0),        # one window, enlarged: the smallest
-    (1, 45, 61, 1, 16384, 1),        # odd grid (bands of one patch), frames that start off a word
+    (1, 45, 61, 1, 16384, 1),        # odd source sizes, frames that start off a word
     (2, 120, 214, 2, 16384, 2),      # a last tile of fewer than six patches
     (3, 333, 517, 2, 300, 3),        # shrunk by less than 2 (9 taps) and the clip's last bytes read one by one
     (2, 480, 854, 2, 120, 0),        # shrunk by about 3 (16 taps)
@@ -1228,17 +1228,24 @@ def test_fused_resize_equals_the_host_path(dev, t, h, w, merge, max_tokens, offs
         assert torch.equal(got["pixel_values"].cpu(), torch.from_numpy(ref["pixel_values"]).to(dtype))
 
 
-@pytest.mark.parametrize("t,h,w,merge,max_tokens,offset", [
-    (3, 70, 32, 1, 16384, 1),        # a row of exactly two steps of source bytes: the clip's last row is read byte by byte
-    (2, 57, 33, 1, 16384, 3),        # one pixel behind them
-    (2, 64, 34, 1, 16384, 2),        # two: whole words to the end
-    (3, 200, 300, 1, 90, 0),         # shrunk by about 1.8: three steps, bands of one patch
-    (70, 90, 120, 2, 2000, 1),       # frames in groups of several, the last one shorter
-    (1, 260, 90, 1, 40, 2),          # shrunk by about 1.7 one way, less the other
+@pytest.mark.parametrize("t,h,w,merge,max_tokens,offset,want", [
+    (3, 70, 32, 1, 16384, 1, 223),       # a row of exactly two steps of source bytes: the clip's last row is read byte by byte
+    (2, 57, 33, 1, 16384, 3, 223),       # one pixel behind them
+    (2, 64, 34, 1, 16384, 2, 223),       # two: whole words to the end
+    (3, 200, 300, 1, 90, 0, 2),          # shrunk by 3.6: more than three steps, the vector form
+    (70, 90, 120, 2, 2000, 1, 223),      # frames in groups of several, the last one shorter
+    (1, 260, 90, 1, 40, 2, 313),         # shrunk by 2.1 across, by 1.9 down: three steps, bands of one patch
+    (2, 180, 320, 1, 228, 3, 224),       # by 1.6: a band's rows are four tiles
+    (2, 75, 90, 1, 16384, 3, 213),       # an odd number of patch rows: bands of one patch
+    (1, 44, 1000, 1, 88, 1, 214),        # one patch row from 44 source rows, by 1.6 across: four tiles of one patch's rows
+    (1, 48, 700, 1, 43, 2, 314),         # the same from 48, by 2 across: three steps
 ])
-def test_resize_as_matrix_products_equals_the_host_path(dev, t, h, w, merge, max_tokens, offset):
-    """the sizes at which the matrix form's loads, steps and groups of frames change: the bytes of the host path"""
+def test_resize_as_matrix_products_equals_the_host_path(dev, t, h, w, merge, max_tokens, offset, want):
+    """the sizes at which the matrix form's loads, steps, bands, row tiles and groups of frames change, every instance of the kernel: the
+    bytes of the host path"""
+    from cogstream_amd import _lib as L2
     test_fused_resize_equals_the_host_path(dev, t, h, w, merge, max_tokens, offset)
+    assert L2.debug_get("preprocess_last_kernel") == want
 
 
 @pytest.mark.parametrize("t,h,w,merge,max_tokens,want", [
