@@ -260,6 +260,40 @@ def test_forms_and_kernels_agree(dev):
             assert rms_err(run(e, toks, [20, 380, *range(381, 400)]), lg) < TOL[torch.bfloat16], (name, value)
 
 
+@pytest.mark.parametrize("keys", [16384, 16385, 16600, 40000])
+def test_a_context_of_more_splits_than_are_combined(dev, keys):
+    """one sequence of up to 256 splits of two tiles (16 384 keys with the new one) and of more, which get longer ones, alone and between short ones.
+    Even weights, and cached rows that are zero but for one key tile (the first, the last and ones between): the logits show whether its
+    split was read once. Against the row-by-row kernel on the same rows"""
+    from cogstream_amd import _lib as L
+    cfg = config([dict(mixer(A, heads=20, dim=16, rot=32, vdim=32, kv_rank=64, scale=1e-7), ff=None)], width=64, vocab=96)
+    e = engine(cfg, state(cfg), torch.bfloat16)
+    g = torch.Generator(device=dev).manual_seed(keys)
+    for contexts in ([keys - 1], [37, keys - 1, 900]):
+        caches = [e.new_cache(n + 1) for n in contexts]
+        rows = caches[len(contexts) // 2]._blocks()[0]
+
+        def step(name, value):
+            for c, n in zip(caches, contexts):
+                c.reset(n)
+            with L.debug_switch(name, value):
+                return e.forward_batch(e.embed_tokens(torch.arange(len(contexts))), [1] * len(contexts), caches, list(range(len(contexts)))).cpu()
+
+        for c in caches:
+            c.k.zero_()
+        empty = step("mla_rowwise", 1)
+        for first in (0, 32 * 191, 32 * 192, keys // 2 // 32 * 32, (keys - 33) // 32 * 32, (keys - 1) // 32 * 32):
+            for c in caches:
+                c.k.zero_()
+            tile = rows[first:min(first + 32, keys - 1)]
+            if len(tile):
+                tile.copy_(torch.randn(64 + 32, generator=g, device=dev) * keys / len(tile))
+            want = step("mla_rowwise", 1)
+            assert not len(tile) or rms_err(empty, want) > 10 * TOL[torch.bfloat16], first
+            for keys_a_split in (0, 64):
+                assert rms_err(step("mla_split_keys", keys_a_split), want) < TOL[torch.bfloat16], (contexts, first, keys_a_split)
+
+
 @pytest.mark.parametrize("rows", [2, 16, 17, 32, 33, 64])
 @pytest.mark.parametrize("width,ff", [(70, 4100), (1100, 1030), (3140, 4100)])
 def test_sublayer_outputs_in_partial_sums(dev, rows, width, ff):
