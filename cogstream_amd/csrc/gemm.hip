@@ -1101,8 +1101,9 @@ void dispatch_f32(hipStream_t st, const GemmArgs& p, int grid, int mask, bool bi
 // All of them walk K in the same order, so the choice is by time alone. Time of a launch = rounds of tiles over the chip x (slabs x
 // time of a slab + the rest of a tile: prologue, epilogue), with a slab's time per tile size for one and, where the LDS has room for
 // them, two workgroups on a CU. The figures are a fit to launches of every tile at M = 48 .. 2048 and eleven weight shapes from 1152 x
-// 1152 to 37 888 x 3584 and 3584 x 18 944 (MI355X, weights from HBM); the tile they choose was the fastest or within 6 % of it at
-// each. They are those of a chip that is not full; two and three rounds are slower a slab (1281 x 11 264 x 2048: two rounds of 128x256
+// 1152 to 37 888 x 3584 and 3584 x 18 944 (MI355X, weights from HBM, nothing beside them). Over 884 products, M = 40 .. 4096 and 24 weight
+// shapes, the choice is 0.6 % slower than the best tile on the average, 4 % or more in 20 of them, 19 % at the most (64 x 28 416 x 3584: 64x64 56.0
+// us, 128x128 47.0; 160 x 11 264 x 2048 21.8, 128x128 19.7). They are those of a chip that is not full; two and three rounds are slower a slab (1281 x 11 264 x 2048: two rounds of 128x256
 // 61.6 us, one of ping-pong tiles and a row of small ones 52; 320 x 22 016 x 4096: two of 128x256 95.6, one of ping-pong 88; 180 x 37 888
 // x 3584: 64x64 108.9, 128x128 96.6).
 struct TileCost { int tile, tm, tn; float one, two, rest; };     // us; two = 0: one workgroup per CU
@@ -1124,10 +1125,12 @@ static int best_mid_tile(int M, int N, int K, bool ln_fold, bool alone, float* t
     int best = 0;
     for (const TileCost& t : MID_TILES) {
         const int tiles = (M + t.tm - 1) / t.tm * ((N + t.tn - 1) / t.tn);
-        // (160x64: its waves have more rows than lanes to hold their factors; three rounds of 150 x 37 888 x 3584 97 us, 128x128 88. Beside
+        // (160x64: its waves have more rows than lanes to hold their factors; three rounds of 150 x 37 888 x 3584 97 us, 128x128 88. One row of
+        // them shares no weights, 129 / 144 / 160 rows against 128x128, us: 11 264 x 2048 20.3 / 20.5 / 21.3 against 19.9 / 19.3 / 19.5, 12 352 x 4096
+        // 37.1 / 38.3 / 39.8 against 36.2 / 36.0 / 36.5, 16 384 x 2048 24.4 / 22.7 / 23.6 against 24.9 / 23.4 / 23.0. Beside
         // another stream, whose launch wants CUs too, its up to 256 workgroups of one to a CU leave none: 16 x 256 patches on two streams
         // 5171 us with it, 4792 without; 5 x 924 5988 / 5604, 4 x 924 5283 / 4876, 8 x 924 7661 / 7663)
-        if (t.tile == 7 && (ln_fold || !alone || tiles > PERSISTENT_WGS)) continue;
+        if (t.tile == 7 && (ln_fold || !alone || M <= t.tm || tiles > PERSISTENT_WGS)) continue;
         const float c = tile_time(tiles, K / 64, t.one, t.two, t.rest, MID_FULL);
         if (best == 0 || c < *time) { best = t.tile; *time = c; }
     }

@@ -1196,6 +1196,20 @@ def test_tiles_that_want_every_cu_are_not_chosen_beside_another_stream(dev, M, N
     assert torch.equal(alone, beside)
 
 
+@pytest.mark.parametrize("M,want", [(129, 4), (160, 4), (320, 7)])
+def test_one_row_of_160_row_tiles_is_not_chosen(dev, M, want):
+    """it would read every weight for itself, 64 columns a workgroup"""
+    from cogstream_amd import _lib as L2
+    ops = _ops()
+    g = torch.Generator(device=dev).manual_seed(M)
+    N = 11264 if M <= 160 else 6176
+    a, w = (torch.randn(*s, generator=g, device=dev).bfloat16() for s in ((M, 2048), (N, 2048)))
+    got = ops.gemm(a, w)
+    assert L2.debug_get("gemm_last_tile") == want
+    with L2.debug_switch("gemm_mid", 11 - want):
+        assert torch.equal(got, ops.gemm(a, w))
+
+
 @pytest.mark.parametrize("tile", [6, 7])
 def test_mid_size_gemm_tiles_of_two_slabs_and_of_160_rows(dev, tile):
     """the same edges for 128x64 with two slabs a slot and 160x64 (five row blocks a wave; a folded norm falls back to 128x64)"""
