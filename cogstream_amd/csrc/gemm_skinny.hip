@@ -146,7 +146,7 @@ void launch(hipStream_t st, const SkinnyArgs& p, int splits) {
         if (p.M <= 8) return launch1<MT, 1, NT, NW, D>(st, p, splits);
     launch1<MT, 2 * MT, NT, NW, D>(st, p, splits);
 }
-// columns at a time; the ring takes 64 to 144 KB, two workgroups a CU for the most used sizes
+// columns at a time; the ring takes 48 (up to eight rows, 16 columns) to 144 KB, two workgroups a CU for the most used sizes
 template <int MT>
 void launch_cols(hipStream_t st, const SkinnyArgs& p, int cols, int splits) {
     if (cols == 64) launch<MT, 4, 4, 2>(st, p, splits);

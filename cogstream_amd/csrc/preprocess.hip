@@ -187,8 +187,8 @@ __global__ __launch_bounds__(256) void resize_patchify_kernel(const uint8_t* __r
 // in a lane: one dword of the wave's transposed [channel][column][64 rows] in LDS, which is the vertical product's operand; that product
 // leaves four neighbouring columns of one output row in a lane, the order of pixel_values. The taps of both passes are in registers in the
 // order of the lanes, built once per wave from the tables.
-// 64 frames 480 x 854 -> 308 x 588: 61 us (the vector form above: 109); 149 MB of frames and pixel_values
-// take 30. 8 of them 32 -> 22 us, 64 x 720 x 1280 192 -> 108. What is left: some 700 vector and 90 matrix instructions a frame and wave.
+// 64 frames 480 x 854 -> 308 x 588: 61 us (the vector form above: 109) with the frames in the Infinity Cache, 111 (142) on frames that are not; 149 MB
+// of frames and pixel_values take 30. 8 of them 32 -> 22 us, 64 x 720 x 1280 192 -> 108. What is left: some 700 vector and 90 matrix instructions a frame and wave.
 constexpr int MM_ROWS = 64, MM_STRIDE = MM_ROWS + 16, MM_WAVES = 4, MM_RESIDENT = 2048;      // source rows of a band; bytes of a column of them in LDS
 
 // digits of a tap, each in the low byte
