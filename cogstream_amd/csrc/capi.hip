@@ -421,14 +421,15 @@ struct VitRange {
 // 64-frame clip 2.7 % (round 4, same box, interleaved: 60.8 -> 59.2 ms; 256 frames at 140 x 280: 47.3 -> 46.5 ms).
 // Shorter clips run on one stream unless the caller has said how many: their products leave CUs idle anyway, which then fetch weights
 // ahead (gemm_mid.hip), one launch of twice the rows against two that share the chip. One stream / two, us, frames x patches:
-//   8 x 256 3129 / 3227, 12 x 256 3706 / 4318, 16 x 256 4767 / 4807, 18 x 256 4986 / 5326, 19 x 256 5469 / 5542, 20 x 256 5558 / 5510,
+//   8 x 256 3129 / 3227, 12 x 256 3706 / 4318, 16 x 256 4767 / 4807, 18 x 256 4986 / 5326, 23 x 200 5137 / 5484, 8 x 576 5143 / 5496,
 //   2 x 924 2972 / 3262, 4 x 924 4802 / 4916, 5 x 924 5616 / 5642, 8 x 924 8674 / 7579, 3 x 1200 4837 / 5032, 4 x 1200 6042 / 6063,
-//   6 x 1200 8843 / 7731, 2 x 1600 4430 / 4778, 3 x 1600 6312 / 6225, 8 x 576 5143 / 5496, 9 x 576 5802 / 5828, 20 x 200 4806 / 4801,
-//   23 x 200 5137 / 5484, 24 x 200 5413 / 5482, 2 x 1936 5447 / 5451, 3 x 1936 7435 / 7176, 16 x 924 14 544 / 13 465
+//   6 x 1200 8843 / 7731, 2 x 1600 4430 / 4778, 3 x 1600 6312 / 6225, 2 x 1936 5447 / 5451, 3 x 1936 7435 / 7176, 16 x 924 14 544 / 13 465
+// and on a card whose clock falls earlier: 18 x 256 5382 / 5507, 23 x 200 5547 / 5653, 5 x 924 6123 / 5814, 4 x 1200 6401 / 6143, 3 x 1600
+//   6721 / 6307, 16 x 256 5137 / 4973. Up to 4608 patches, 18 row blocks, the QKV product's 14 columns of 256x256 tiles are one round.
 // Not while the per-kernel profiler is on: overlapping launches stretch every bracket, so bench.py's `roofline` and
 // `breakdown_ms` describe the kernels one at a time. cogs_vit_set_streams(h, 1) or the debug switch vit_split_max switch it off.
 
-constexpr int64_t VIT_SPLIT_MIN = 4700;      // patches
+constexpr int64_t VIT_SPLIT_MIN = 4609;      // patches
 
 static cogs_status cogs_project_rows(cogs_handle h, hipStream_t st, const void* tokens, int M, void* out, void* ws);
 

@@ -343,7 +343,7 @@ cogs_status cogs_vit_encode(cogs_handle h, cogs_stream stream, const void* pixel
  * and up to three the handle owns; frames are independent under per-frame attention, the tokens are bit-identical to a
  * one-stream encode): one range's kernels fill the partly empty last rounds of another's persistent GEMM launches. The
  * ranges are queued layer by layer in turn, so every stream starts within one layer of the first. streams = 1 keeps
- * everything on the caller's stream, 2 to 4 split every clip, 0 (the default) splits clips of 4700 patches and more in two. */
+ * everything on the caller's stream, 2 to 4 split every clip, 0 (the default) splits clips of 4609 patches and more in two. */
 cogs_status cogs_vit_set_streams(cogs_handle h, int streams);
 
 /* ----------------------------------------------------------------------- multi-GPU ------ */

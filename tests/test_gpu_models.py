@@ -120,9 +120,9 @@ def test_frame_split_two_stream_encode_is_transparent(dev):
     assert L.lib.cogs_vit_set_streams(enc.handle.h, 5) == L.E_INVALID and L.lib.cogs_vit_set_streams(enc.handle.h, -1) == L.E_INVALID
 
 
-@pytest.mark.parametrize("t,gh,gw,streams", [(18, 16, 16, 1), (3, 40, 40, 2), (1, 72, 72, 1)])
+@pytest.mark.parametrize("t,gh,gw,streams", [(18, 16, 16, 1), (5, 22, 42, 2), (3, 40, 40, 2), (1, 72, 72, 1)])
 def test_streams_of_a_clip_by_its_patches(dev, t, gh, gw, streams):
-    """where the caller has not said how many, or has given the choice back: one stream up to 4699 patches (4608 here), two from there on (4800),
+    """where the caller has not said how many, or has given the choice back: one stream up to 4608 patches, two from there on (4620, 4800),
     one for one frame; the tokens are those of one stream"""
     from cogstream_amd import _lib as L
     from cogstream_amd.vision import VisionEncoder
