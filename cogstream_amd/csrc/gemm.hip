@@ -1100,38 +1100,54 @@ void dispatch_f32(hipStream_t st, const GemmArgs& p, int grid, int mask, bool bi
 // ---- which kernel a bf16 product of two or more rows gets -------------------------------------------------------------------
 // All of them walk K in the same order, so the choice is by time alone. Time of a launch = rounds of tiles over the chip x (slabs x
 // time of a slab + the rest of a tile: prologue, epilogue), with a slab's time per tile size for one and, where the LDS has room for
-// them, two workgroups on a CU. The figures are a fit to launches of every tile at M = 48 .. 2048 and eleven weight shapes from 1152 x
-// 1152 to 37 888 x 3584 and 3584 x 18 944 (MI355X, weights from HBM, nothing beside them). Over 884 products, M = 40 .. 4096 and 24 weight
-// shapes, the choice is 0.6 % slower than the best tile on the average, 4 % or more in 20 of them, 19 % at the most (64 x 28 416 x 3584: 64x64 56.0
-// us, 128x128 47.0; 160 x 11 264 x 2048 21.8, 128x128 19.7). They are those of a chip that is not full; two and three rounds are slower a slab (1281 x 11 264 x 2048: two rounds of 128x256
-// 61.6 us, one of ping-pong tiles and a row of small ones 52; 320 x 22 016 x 4096: two of 128x256 95.6, one of ping-pong 88; 180 x 37 888
-// x 3584: 64x64 108.9, 128x128 96.6).
-struct TileCost { int tile, tm, tn; float one, two, rest; };     // us; two = 0: one workgroup per CU
+// them, two workgroups on a CU; a slab takes longer the fuller the chip is (from half of the CUs on, by `full` with all of them: power,
+// and the CUs that read weights ahead are gone). The figures are a fit to launches of every tile at M = 40 .. 4096 and 23 weight shapes from
+// 1152 x 1152 to 37 888 x 3584 and 3584 x 18 944 (MI355X, weights from HBM, nothing beside them): over those 805 products the choice
+// is 0.6 % slower than the best on the average, 5 % or more in 20 (64 x 28 416 x 3584: 64x64 46 us, 128x128 40; 512 x 2048 x 5632 26.5 / 23.9).
+//   * The steps between the sizes count: a product of 1.1 rounds takes two. 96x64, 160x128, 192x128 and 160x256 beside 32x64, 64x64, 128x64,
+//     160x64, 128x128 and 128x256 took, us: 2048 x 4304 x 1152 31.2 -> 24.6 (221 tiles of 160x256 for 272 of 128x256), 924 x 4352 x 1152 16.7
+//     -> 13.6, 1300 x 3584 x 18 944 205 -> 167, 300 x 3584 x 28 416 145 -> 115, 512 x 37 888 x 3584 160 -> 127; 3 % on the average of the 805.
+//   * More than a round of ping-pong tiles and not a whole number: whole rounds of them over some row and column blocks, what is left in one
+//     mid-size launch (strip of columns, ragged rows, or both). 4096 x 6176 x 2048 108 -> 60 + 41, 768 x 22 016 x 4096 148 -> 115. A strip
+//     of columns reads every weight once; rows that are left read all of them again, and where they are more than half of the 256 MB
+//     Infinity Cache they push the output out of it: 621 x 37 888 x 3584 (two row blocks and 109 rows) gained 5 us and the 18 944-wide
+//     product behind it lost 25; as a strip (three row blocks x 85 column blocks, 160x256) 163 -> 152 and 113 -> 108, 1000 rows 231 -> 202.
+struct TileCost { int tile, tm, tn; float one, two, rest, full; };     // us; two = 0: one workgroup per CU; full: a slab's surcharge on a full chip
 static constexpr TileCost MID_TILES[] = {
-    {1, 32, 64, 0.165f, 0.f, 1.8f},   {2, 64, 64, 0.218f, 0.409f, 1.8f}, {3, 128, 64, 0.309f, 0.637f, 2.3f}, {4, 128, 128, 0.387f, 0.f, 3.6f},
-    {5, 128, 256, 0.629f, 0.f, 4.8f}, {6, 128, 64, 0.292f, 0.f, 2.5f},   {7, 160, 64, 0.332f, 0.f, 3.8f}};
-static constexpr float MID_FULL = 1.25f, TWO_FULL = 1.15f, PP_FULL = 1.12f;         // slabs of launches of more than one round, against those
-static constexpr float PP_SLAB = 1.14f, PP_REST = 6.f, SECOND_LAUNCH = 2.f;
+    {1, 32, 64, 0.174f, 0.f, 0.9f, 0.14f},     {2, 64, 64, 0.213f, 0.381f, 2.2f, 0.08f}, {3, 128, 64, 0.311f, 0.569f, 2.1f, 0.14f},
+    {4, 128, 128, 0.379f, 0.f, 3.5f, 0.29f},   {5, 128, 256, 0.633f, 0.f, 5.3f, 0.36f},  {6, 128, 64, 0.271f, 0.f, 2.7f, 0.21f},
+    {7, 160, 64, 0.312f, 0.f, 3.2f, 0.28f},    {8, 96, 64, 0.238f, 0.f, 2.0f, 0.24f},    {9, 160, 128, 0.443f, 0.f, 4.6f, 0.39f},
+    {10, 192, 128, 0.502f, 0.f, 4.8f, 0.44f},  {11, 160, 256, 0.767f, 0.f, 4.9f, 0.42f}};
+static constexpr TileCost PP_TILE = {0, 256, 256, 1.127f, 0.f, 7.5f, 0.25f};
+static constexpr float SECOND_LAUNCH = 2.f, LN_FINALIZE = 5.f;                      // us
+static constexpr float REST_READ = 4.4e6f, REST_AGAIN = 128e6f;                     // weights of a second launch: bytes a us, and the most that are read again
+static constexpr int MIXED_ROUNDS = 4;                                              // (of more rounds the last one is little)
 
-static float tile_time(int tiles, int slabs, float one, float two, float rest, float full) {
-    const float t1 = slabs * one + rest, t2 = slabs * two + rest;
-    const int rounds = (tiles + PERSISTENT_WGS - 1) / PERSISTENT_WGS;
-    if (two == 0.f) return rounds > 1 ? rounds * (slabs * one * full + rest) : t1;
-    const int whole = tiles / (2 * PERSISTENT_WGS), left = tiles % (2 * PERSISTENT_WGS);
-    return whole * (whole > 1 ? slabs * two * TWO_FULL + rest : t2) + (left == 0 ? 0.f : left <= PERSISTENT_WGS ? t1 : t2);
+static float tile_time(int tiles, int slabs, const TileCost& t) {
+    constexpr int CUS = PERSISTENT_WGS, FREE = CUS / 2;
+    const float full = 1.f + t.full;
+    if (t.two == 0.f) {
+        const int left = tiles % CUS;
+        return tiles / CUS * (slabs * t.one * full + t.rest) + (left ? slabs * t.one * (1.f + t.full * max(left - FREE, 0) / (CUS - FREE)) + t.rest : 0.f);
+    }
+    const int left = tiles % (2 * CUS);
+    const float one = slabs * t.one * (1.f + t.full * max(left - FREE, 0) / (CUS - FREE)), two = slabs * t.two * (1.f + t.full * max(left - CUS, 0) / CUS);
+    return tiles / (2 * CUS) * (slabs * t.two * full + t.rest) + (left ? (left <= CUS ? one : two) + t.rest : 0.f);
 }
-// alone: no other stream's products beside this one
-static int best_mid_tile(int M, int N, int K, bool ln_fold, bool alone, float* time) {
+// alone: no other stream's products beside this one. rows0, cols0: the rectangle at the origin that another launch computes
+static int best_mid_tile(int M, int N, int K, bool alone, float* time, int rows0 = 0, int cols0 = 0) {
     int best = 0;
     for (const TileCost& t : MID_TILES) {
-        const int tiles = (M + t.tm - 1) / t.tm * ((N + t.tn - 1) / t.tn);
+        const int nbn = (N + t.tn - 1) / t.tn;
+        const int tiles = (M - rows0 + t.tm - 1) / t.tm * nbn + (rows0 + t.tm - 1) / t.tm * ((N - cols0 + t.tn - 1) / t.tn) * (cols0 > 0);
         // (160x64: its waves have more rows than lanes to hold their factors; three rounds of 150 x 37 888 x 3584 97 us, 128x128 88. One row of
         // them shares no weights, 129 / 144 / 160 rows against 128x128, us: 11 264 x 2048 20.3 / 20.5 / 21.3 against 19.9 / 19.3 / 19.5, 12 352 x 4096
         // 37.1 / 38.3 / 39.8 against 36.2 / 36.0 / 36.5, 16 384 x 2048 24.4 / 22.7 / 23.6 against 24.9 / 23.4 / 23.0. Beside
         // another stream, whose launch wants CUs too, its up to 256 workgroups of one to a CU leave none: 16 x 256 patches on two streams
         // 5171 us with it, 4792 without; 5 x 924 5988 / 5604, 4 x 924 5283 / 4876, 8 x 924 7661 / 7663)
-        if (t.tile == 7 && (ln_fold || !alone || M <= t.tm || tiles > PERSISTENT_WGS)) continue;
-        const float c = tile_time(tiles, K / 64, t.one, t.two, t.rest, MID_FULL);
+        if (t.tile == 8 && tiles > PERSISTENT_WGS - 8) continue;      // (its weights come too slowly with no CU to read them ahead: 768 x 2048 x 5632 32.2 us, 128x64 28.8)
+        if ((t.tile == 7 || t.tile == 9) && (!alone || M - rows0 <= t.tm || (t.tile == 7 && tiles > PERSISTENT_WGS))) continue;
+        const float c = tile_time(tiles, K / 64, t);
         if (best == 0 || c < *time) { best = t.tile; *time = c; }
     }
     return best;
@@ -1140,11 +1156,11 @@ static int best_mid_tile(int M, int N, int K, bool ln_fold, bool alone, float* t
 static int finish_ln(hipStream_t st, const CogsGemm& g) {
     return g.ln_part ? cogs_k_ln_finalize(st, g.ln_part, g.M, g.K / 64, g.K, g.ln_eps, const_cast<float*>(g.ln_ab)) : COGS_OK;
 }
-static int launch_mid(hipStream_t st, const CogsGemm& g, int tile, bool alone) {
+static int launch_mid(hipStream_t st, const CogsGemm& g, int tile, bool alone, int rows0 = 0, int cols0 = 0) {
     ++g_gemm_launches;
     g_cogs_debug.gemm_last_body = 2;
     g_cogs_debug.gemm_last_tile = tile;
-    return cogs_k_gemm_mid(st, g, tile, alone);
+    return cogs_k_gemm_mid(st, g, tile, alone, rows0, cols0);
 }
 
 // the mid-size kernel stores K and V columns straight into the cache where its waves' 32 or 64 columns do not straddle them
@@ -1171,7 +1187,7 @@ static int gemm_rows(hipStream_t st, const CogsGemm& g, bool* kv_stored) {
     const int S = env_co > 0 ? env_co : g_co_streams;
     float mid_time = 0.f;
     const int env_mid = (int)g_cogs_debug.gemm_mid;
-    const int mid = g.dtype != COGS_DT_BF16 ? 0 : env_mid > 0 ? env_mid : best_mid_tile(g.M, g.N, g.K, g.ln_ab != nullptr, S == 1, &mid_time);
+    const int mid = g.dtype != COGS_DT_BF16 ? 0 : env_mid > 0 ? env_mid : best_mid_tile(g.M, g.N, g.K, S == 1, &mid_time);
     const int n_pad = (g.N + BN3 - 1) / BN3 * BN3;
     const bool pp_fits = n_pad * 100 <= g.N * (int)g_cogs_debug.gemm_pad_pct;   // default: <= 12 % of the MFMAs spent on N padding
     // (the ping-pong kernel wants two slabs and, below a row block, wastes its tiles' rows)
@@ -1238,63 +1254,63 @@ static int gemm_rows(hipStream_t st, const CogsGemm& g, bool* kv_stored) {
         const int nb = count_tiles(g.M);
         p.ntiles = nb;
         const int rounds = nb / PERSISTENT_WGS, rem = nb % PERSISTENT_WGS;
-        int mb_main = -1;      // >= 0: row blocks that stay in this kernel (0 = none: all of the GEMM goes to the mid-size kernel)
-        if (!env_nosplit && !env_nostore && nb <= 2 * PERSISTENT_WGS) {
+        int mb_main = -1, cb_main = p.nbn;      // mb_main >= 0: row and column blocks that stay in this kernel (0 = none: all of the GEMM goes to the mid-size kernel)
+        int rest_tile = 0;
+        if (!env_nosplit && !env_nostore && nb <= (S == 1 && g.K >= 2048 ? MIXED_ROUNDS : 2) * PERSISTENT_WGS) {
             // Few tiles (a short clip, one rank's share of a frame-sharded one, a short prompt): the cheapest of this kernel, the
-            // mid-size one and one round here with the rest there -- each timed as if alone also when the encoder feeds two
+            // mid-size one and whole rounds here with the rest there -- each timed as if alone also when the encoder feeds two
             // streams. (Counting both streams' tiles as one launch picked larger tiles, which leave less for the other stream's
             // launch to run beside: 4 x 256 patches 3.09 against 2.58 ms, 16 x 256 5.46 / 4.92, 8 x 924 8.52 / 7.95.)
             const int slabs = g.K / 64;
-            float best = tile_time(nb, slabs, PP_SLAB, 0.f, PP_REST, PP_FULL);
+            const float ln = g.ln_part ? LN_FINALIZE : 0.f;
+            float best = tile_time(nb, slabs, PP_TILE) + ln;
             if (mid_time < best) { best = mid_time; mb_main = 0; }
-            if (rounds == 1 && rem > 0) {
-                const int mb = whole_blocks(PERSISTENT_WGS);           // whole row blocks inside the first round
-                const int rows_rem = g.M - mb * BM3;
-                if (mb > 0 && rows_rem > 0) {
-                    float rest;
-                    best_mid_tile(rows_rem, g.N, g.K, g.ln_ab != nullptr, S == 1, &rest);
-                    if (slabs * PP_SLAB + PP_REST + rest + SECOND_LAUNCH < best) mb_main = mb;
+            // row blocks x column blocks here (all columns: p.nbn, with the tall tiles), the L-shaped rest in one mid-size launch
+            auto consider = [&](int mb, int cb) {
+                const int rows = min(mb * BM3, g.M), cols = cb >= p.nbn ? g.N : cb * BN3;
+                if (mb <= 0 || cb <= 0 || (rows == g.M && cols == g.N) || (rows < g.M && 2.f * g.K * g.N > REST_AGAIN)) return;
+                float rest;
+                const int tile = best_mid_tile(g.M, g.N, g.K, S == 1, &rest, rows, cols);
+                rest = max(rest, 2.f * g.K * (rows < g.M ? g.N : g.N - cols) / REST_READ);
+                const float t = tile_time(cb >= p.nbn ? count_tiles(rows) : mb * cb, slabs, PP_TILE) + rest + SECOND_LAUNCH + ln;
+                if (t < best) { best = t; mb_main = mb; cb_main = min(cb, p.nbn); rest_tile = tile; }
+            };
+            if (rounds >= 1 && rem > 0) {
+                consider(whole_blocks(rounds * PERSISTENT_WGS), p.nbn);
+                if (S == 1) {
+                    consider(g.M / BM3, rounds * PERSISTENT_WGS / max(g.M / BM3, 1));
+                    consider(p.nbm, rounds * PERSISTENT_WGS / p.nbm);
                 }
             }
-        } else if (S == 1 && !env_nosplit && !env_nostore && g.K >= 2048 && rounds >= 2 && rem > 0 && rem * 100 < PERSISTENT_WGS * 45) {
+        }
+        if (mb_main < 0 && S == 1 && !env_nosplit && !env_nostore && g.K >= 2048 && rounds >= 2 && rem > 0 && rem * 100 < PERSISTENT_WGS * 45) {
             // (many tiles, one stream -- beside a second one a split launch costs the 64-frame clip 1 %: pays when a tile is long against a second launch and the last round is less than ~45 % full:
             // measured with the two-segment K loop at K = 1152: -2 %; K = 3584, last round 34 % full: +2 %; K = 18944,
             // 34 %: +6 %; K = 4352, 51 % full (ViT fc2): -2 %, so it no longer splits)
             const int mb = whole_blocks(rounds * PERSISTENT_WGS);    // whole row blocks within the full rounds
-            if (mb > 0 && g.M - mb * BM3 >= 512) mb_main = mb;
+            float rest;
+            if (mb > 0 && g.M - mb * BM3 >= 512) { mb_main = mb; rest_tile = best_mid_tile(g.M, g.N, g.K, true, &rest, mb * BM3, g.N); }
         }
         const bool env_choice = g_cogs_debug.gemm_choice != 0;      // diagnostics: which body each shape gets
-        if (env_choice) fprintf(stderr, "[gemm choice] M=%d N=%d K=%d: %d ping-pong tiles (%d rounds + %d), mb_main %d\n", g.M, g.N, g.K, nb, rounds, rem, mb_main);
-        if (mb_main >= 0) {
-            const int rows_main = mb_main * BM3;
+        if (env_choice) fprintf(stderr, "[gemm choice] M=%d N=%d K=%d: %d ping-pong tiles (%d rounds + %d), %d x %d here, rest in tiles %d\n", g.M, g.N, g.K, nb, rounds, rem, mb_main, cb_main, rest_tile);
+        if (mb_main == 0) {
+            *kv_stored = kv_in_epilogue(g);
+            return launch_mid(st, g, mid, S == 1);
+        }
+        if (mb_main > 0) {
+            const int rows = min(mb_main * BM3, g.M), cols = cb_main >= p.nbn ? g.N : cb_main * BN3;
+            if (const int rc_ln = finish_ln(st, g)) return rc_ln;
+            p.M = rows; p.nbm = mb_main;
+            if (cols < g.N) { p.nbn = cb_main; p.cf = p.group_m * cb_main; p.ntiles = mb_main * cb_main; }
+            else p.ntiles = count_tiles(rows);
+            dispatch_pp(st, p, p.ntiles, pp_mask);
+            const int rc2 = COGS_LAUNCH_CHECK();
+            if (rc2 != COGS_OK) return rc2;
             CogsGemm b = g;
-            b.M = g.M - rows_main;
-            b.A = (const char*)g.A + (size_t)rows_main * g.lda * es;
-            b.C = (char*)g.C + (size_t)rows_main * (g.hm_rows > 0 ? g.head_dim : g.ldc) * (g.out_f32 ? 4 : es);   // head-major: rows advance by head_dim inside every head block
-            if (g.residual) b.residual = (const char*)g.residual + (size_t)rows_main * g.ldr * es;
-            if (g.rope_rowpos) b.rope_rowpos = g.rope_rowpos + rows_main;
-            if (g.row_stats) b.row_stats = g.row_stats + (size_t)rows_main * (g.N / 64) * 2;
-            if (g.ln_ab) b.ln_ab = g.ln_ab + (size_t)rows_main * 2;
-            if (mb_main > 0) b.ln_part = nullptr;      // (finished below, in front of the first launch)
-            if (mb_main > 0) b.kv_k = b.kv_v = nullptr;
-            else *kv_stored = kv_in_epilogue(g);
-            if (g.rope_cos) {
-                const size_t per_row = (size_t)(g.head_dim / 2) * (g.rope_sin ? 1 : 2);
-                b.rope_cos = g.rope_cos + (size_t)rows_main * per_row;
-                if (g.rope_sin) b.rope_sin = g.rope_sin + (size_t)rows_main * per_row;
-            }
-            if (mb_main > 0) {
-                if (const int rc_ln = finish_ln(st, g)) return rc_ln;
-                p.M = rows_main; p.nbm = mb_main;
-                p.ntiles = count_tiles(rows_main);
-                dispatch_pp(st, p, p.ntiles, pp_mask);
-                const int rc2 = COGS_LAUNCH_CHECK();
-                if (rc2 != COGS_OK) return rc2;
-            }
-            // (straight to the kernel: a remainder may be one row, which cogs_k_gemm would take for a single-row product)
-            float rest = 0.f;
-            const int rc3 = launch_mid(st, b, mb_main > 0 ? best_mid_tile(b.M, b.N, b.K, g.ln_ab != nullptr, S == 1, &rest) : mid, S == 1);
-            if (mb_main > 0) g_cogs_debug.gemm_last_body = 5;
+            b.ln_part = nullptr;      // (finished)
+            b.kv_k = b.kv_v = nullptr;
+            const int rc3 = launch_mid(st, b, rest_tile, S == 1, rows, cols);
+            g_cogs_debug.gemm_last_body = 5;
             return rc3;
         }
         if (const int rc_ln = finish_ln(st, g)) return rc_ln;

@@ -1,6 +1,7 @@
 // Mid-size GEMM (bf16):  C[M,N] = epilogue( A[M,K] . W[N,K]^T ), same sums in the same order as the kernels of gemm.hip.
 //
-// For products whose 256-wide tiles would leave most of the chip idle. One tile per workgroup, tiles from 32x64 to 128x256; the
+// For products whose 256-wide tiles would leave most of the chip idle, and for what whole rounds of those leave of a product (rows0, cols0).
+// One tile per workgroup, tiles from 32x64 to 160x256, which size by what the chip makes of their number (gemm.hip); the
 // K slabs (64 elements: one whole 128-byte line a row; KS of them at a time) go by LDS-DMA into a ring of S slots, S - 1 of them in
 // flight ahead of the slabs being multiplied, one barrier and one counted vmcnt per KS slabs. While a slab is multiplied, the next
 // one's fragments are read and its slot is filled again.
@@ -16,7 +17,10 @@
 //   * A wave issues in order, so fragment reads and DMA in front of the matrix instructions leave the matrix pipe idle meanwhile: they
 //     stand between them, one behind each (621 x 3584 x 18944 at 160x64: 121 -> 109; 4096 x 2048 x 5632 at 128x256: 87.5 -> 84.2).
 //     128x64 with two workgroups a CU has sixteen waves to fill the gaps, and is the slower for it (24.7 -> 26.1): not there.
-//   * 32x64 is four waves of 16x32 (two of 32x32: 13.7 instead of 11.9): every SIMD has one.
+//   * 32x64 is four waves of 16x32 (two of 32x32: 13.7 instead of 11.9): every SIMD has one. 128x256 is eight of 64x64: four of 64x128 read a
+//     quarter less LDS and are slower, a wave alone on its SIMD waits for each DMA and read it issues (4096 x 2048 x 8192 139 us, 110;
+//     160x128 as four of 80x64 49 against 41). Where eight waves cannot share a slab's pieces evenly one of them fetches a few twice (2 to 9 %
+//     more DMA): 160x128, 160x256. 192x256 has no room for a third slot and spills.
 // Products split over K would need fewer bytes per CU, and give other bits.
 //
 // K is walked in order by one accumulator per output: a row's bits do not depend on which tile size, or which kernel of gemm.hip,
@@ -32,8 +36,10 @@ struct MidArgs {
     const char* A; long lda;   // bytes per row
     const char* W; long ldw;
     int M, N, KT;              // KT: 64-wide K slabs
-    int nbm, nbn;              // tiles; workgroups past them are prefetch_weights
-    int group;                 // row tiles that share a panel of weights
+    int rows0, cols0;          // the rectangle at the origin that is computed elsewhere (0, 0: none)
+    int nbm, nbn;              // tiles of the rows from rows0 on
+    int nbm0, nbn0;            // ... and of the columns from cols0 on of the rows in front of them; workgroups past both are prefetch_weights
+    int group, group0;         // row tiles that share a panel of weights
     const float* ln_part; int ln_tiles; float ln_inv_h, ln_eps;     // EPI_LNFOLD: row statistics still in partial sums (or null)
     int ln_staged;             // a tile's fit a ring slot
     char* kv_k; char* kv_v; int kv_col, kv_dim;      // EPI_ROPE, K and V columns into cache rows of kv_dim (or null)
@@ -104,12 +110,13 @@ template <int EPI, int MI, int NI, int WM, int WN, int S, int WPE, int KS, bool 
 __global__ __launch_bounds__(64 * WM * WN, WPE) void gemm_mid_kernel(MidArgs p) {
     extern __shared__ __attribute__((aligned(16))) char smem[];
     constexpr int TM = 16 * MI * WM, TN = 16 * NI * WN, WAVES = WM * WN;
-    constexpr int SUB = (TM + TN) * ROW_BYTES, SLAB = SUB * KS, P1 = SUB / 1024 / WAVES, P = P1 * KS;      // P: a wave's pieces per slot
-    static_assert(SUB % (1024 * WAVES) == 0, "every wave stages the same number of pieces");
+    constexpr int SUB = (TM + TN) * ROW_BYTES, SLAB = SUB * KS, PIECES = SUB / 1024, P1 = (PIECES + WAVES - 1) / WAVES, P = P1 * KS;      // P: a wave's pieces per slot
+    static_assert(SUB % 1024 == 0, "");
     const int lane = threadIdx.x & 63;
     const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int wm = wid / WN, wn = wid % WN;
-    if ((int)blockIdx.x >= p.nbm * p.nbn) {
+    const int rest_tiles = p.nbm * p.nbn, tiles = rest_tiles + p.nbm0 * p.nbn0;
+    if ((int)blockIdx.x >= tiles) {
         prefetch_weights(p, smem, TM, TN, WAVES, wid, lane);
         return;
     }
@@ -120,21 +127,27 @@ __global__ __launch_bounds__(64 * WM * WN, WPE) void gemm_mid_kernel(MidArgs p) 
     // panel of weights run on one XCD
     int m0, n0;
     {
-        const int nb = p.nbm * p.nbn, xcd = blockIdx.x & 7, q = nb >> 3, r = nb & 7;
-        const int bid = (xcd < r ? xcd * (q + 1) : r * (q + 1) + (xcd - r) * q) + (blockIdx.x >> 3);
-        const int per_group = p.group * p.nbn, first_m = bid / per_group * p.group, gsz = min(p.nbm - first_m, p.group);
-        m0 = (first_m + (bid % per_group) % gsz) * TM;
-        n0 = ((bid % per_group) / gsz) * TN;
+        const int xcd = blockIdx.x & 7, q = tiles >> 3, r = tiles & 7;
+        int bid = (xcd < r ? xcd * (q + 1) : r * (q + 1) + (xcd - r) * q) + (blockIdx.x >> 3);
+        const bool front = bid >= rest_tiles;                    // of the rows in front of rows0
+        if (front) bid -= rest_tiles;
+        const int group = front ? p.group0 : p.group, nbm = front ? p.nbm0 : p.nbm, per_group = group * (front ? p.nbn0 : p.nbn);
+        const int first_m = bid / per_group * group, gsz = min(nbm - first_m, group);
+        m0 = (first_m + (bid % per_group) % gsz) * TM + (front ? 0 : p.rows0);
+        n0 = ((bid % per_group) / gsz) * TN + (front ? p.cols0 : 0);
+        if (front) p.M = p.rows0;
     }
-    // piece pc of a slab: tile rows 8 pc .. +7 (A's rows, then W's); lane -> row + (lane >> 3), 16-byte chunk lane & 7, swizzled
+    // piece pc of a slab: tile rows 8 pc .. +7 (A's rows, then W's); lane -> row + (lane >> 3), 16-byte chunk lane & 7, swizzled. Every wave
+    // stages P1 of them (its waits count them); where they do not divide, the last wave writes some of its neighbour's again, the same bytes
+    const int first_piece = min(wid * P1, PIECES - P1);
     const char* src[P1];
 #pragma unroll
     for (int i = 0; i < P1; ++i) {
-        const int r = (wid * P1 + i) * 8 + (lane >> 3);
+        const int r = (first_piece + i) * 8 + (lane >> 3);
         const int c = (lane & 7) ^ (r & 7);
         src[i] = r < TM ? p.A + (long)min(m0 + r, p.M - 1) * p.lda + c * 16 : p.W + (long)min(n0 + r - TM, p.N - 1) * p.ldw + c * 16;
     }
-    char* const lds_wave = smem + wid * P1 * 1024;
+    char* const lds_wave = smem + first_piece * 1024;
     auto stage_piece = [&](int slot, int i, int u, int step) {
         glds16(src[i] + u * step, lds_wave + slot * SLAB + u * SUB + i * 1024);
     };
@@ -213,17 +226,17 @@ __global__ __launch_bounds__(64 * WM * WN, WPE) void gemm_mid_kernel(MidArgs p) 
     constexpr bool EARLY = NI == 2 && (EPI & EPI_GENERIC) == 0;
     EpiOperands<bf16_t, EPI, MI, NI> early;
     if constexpr (EARLY) early.load(p.epi, mb, nb, p.M, p.N, lane);
-    // EPI_LNFOLD: the factors of this wave's rows while the ring fills; lane l has row l of its 16 MI. Their partial sums, one run of memory
+    // EPI_LNFOLD: the factors of this wave's rows while the ring fills; lane l has rows l and l + 64 of its 16 MI. Their partial sums, one run of memory
     // for the tile's rows, come through the ring's last slot, ahead of the slabs: a lane reading its row's from memory is 64 lines a
     // load, 18 loads a wave, in front of the loop (M = 256 of the vision encoder: fc1 13.8 -> 12.5 us, QKV 11.2 -> 10.3)
-    float factor = 0.f;
+    constexpr int FACTORS = MI > 4 ? 2 : 1;
+    float factor[FACTORS];
     int filled = 0;
     auto fill = [&](int upto) {
         for (; filled < upto && filled < KT; ++filled) stage(filled, odd && filled == KT - 1);
     };
     if constexpr ((EPI & EPI_LNFOLD) != 0) {
-        static_assert(MI <= 4 && (MI & (MI - 1)) == 0, "a lane has one of the wave's rows");
-        const int in_tile = wm * 16 * MI + (lane & (16 * MI - 1));
+        auto in_tile = [&](int f) { return wm * 16 * MI + min(64 * f + lane, 16 * MI - 1); };
         if (p.ln_part && p.ln_staged) {
             char* const lds = smem + (S - 1) * SLAB;
             const long first = (long)m0 * p.ln_tiles * 8, last = (long)p.M * p.ln_tiles * 8 - 16;
@@ -233,14 +246,20 @@ __global__ __launch_bounds__(64 * WM * WN, WPE) void gemm_mid_kernel(MidArgs p) 
             wait_slabs<P, S - 1>(filled);
             __builtin_amdgcn_s_barrier();
             asm volatile("" ::: "memory");
-            factor = ln_row_factors(reinterpret_cast<const f32x2*>(lds) + min(in_tile, p.M - 1 - m0) * p.ln_tiles, p.ln_tiles, p.ln_inv_h, p.ln_eps)[0];
-            asm volatile("" : "+v"(factor));
+#pragma unroll
+            for (int f = 0; f < FACTORS; ++f) {
+                factor[f] = ln_row_factors(reinterpret_cast<const f32x2*>(lds) + min(in_tile(f), p.M - 1 - m0) * p.ln_tiles, p.ln_tiles, p.ln_inv_h, p.ln_eps)[0];
+                asm volatile("" : "+v"(factor[f]));
+            }
             __builtin_amdgcn_s_barrier();                        // every wave has read it
             asm volatile("" ::: "memory");
         } else {
             fill(S);
-            const long r = min(m0 + in_tile, p.M - 1);
-            factor = p.ln_part ? ln_row_factors(reinterpret_cast<const f32x2*>(p.ln_part) + r * p.ln_tiles, p.ln_tiles, p.ln_inv_h, p.ln_eps)[0] : p.epi.ln_ab[2 * r];
+#pragma unroll
+            for (int f = 0; f < FACTORS; ++f) {
+                const long r = min(m0 + in_tile(f), p.M - 1);
+                factor[f] = p.ln_part ? ln_row_factors(reinterpret_cast<const f32x2*>(p.ln_part) + r * p.ln_tiles, p.ln_tiles, p.ln_inv_h, p.ln_eps)[0] : p.epi.ln_ab[2 * r];
+            }
         }
     }
     fill(S);
@@ -308,8 +327,18 @@ __global__ __launch_bounds__(64 * WM * WN, WPE) void gemm_mid_kernel(MidArgs p) 
     if constexpr ((EPI & EPI_LNFOLD) != 0) {
         float rs[MI];
 #pragma unroll
-        for (int mi = 0; mi < MI; ++mi) rs[mi] = __shfl(factor, 16 * mi + (lane & 15));
+        for (int mi = 0; mi < MI; ++mi) rs[mi] = __shfl(factor[mi >> 2], 16 * (mi & 3) + (lane & 15));
         epilogue_tile<bf16_t, EPI, MI, NI>(p.epi, mb, nb, p.M, p.N, lane, acc, nullptr, rs, operands);
+    } else if constexpr (MI == 5 && NI == 4) {
+        f32x4 top[4][4], low[1][4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) top[i][j] = acc[i][j];
+            low[0][j] = acc[4][j];
+        }
+        epilogue_wave<bf16_t, EPI>(p.epi, mb, nb, p.M, p.N, lane, top);
+        epilogue_tile<bf16_t, EPI, 1, 4>(p.epi, mb + 64, nb, p.M, p.N, lane, low);
     } else if constexpr (MI == 4 && NI == 4) {
         epilogue_wave<bf16_t, EPI>(p.epi, mb, nb, p.M, p.N, lane, acc);
     } else if constexpr ((EPI & EPI_ROWSTAT) != 0 && NI == 2) {
@@ -350,14 +379,20 @@ void launch(hipStream_t st, MidArgs& p, bool alone) {
     static_assert(lds <= 160 * 1024, "");
     static std::atomic<uint64_t> attr_done{0};
     cogs_ensure_dyn_lds((const void*)gemm_mid_kernel<EPI, MI, NI, WM, WN, S, WPE, KS, IL>, lds, attr_done);
-    p.nbm = (p.M + TM - 1) / TM;
+    p.nbm = (p.M - p.rows0 + TM - 1) / TM;
     p.nbn = (p.N + TN - 1) / TN;
+    p.nbm0 = (p.rows0 + TM - 1) / TM;
+    p.nbn0 = (p.N - p.cols0 + TN - 1) / TN;
     // groups of row tiles as equal as they come: one row tile left over read every weight for itself, 9 row tiles of 1152 x 3456 x 1152
     // 69.6 us (with its XCD's prefetch, below) against 14.1 in one group
-    const int groups = (p.nbm + MAX_GROUP - 1) / MAX_GROUP;
-    p.group = (p.nbm + groups - 1) / groups;
+    auto group_of = [](int nbm) {
+        const int groups = (nbm + MAX_GROUP - 1) / MAX_GROUP;
+        return groups ? (nbm + groups - 1) / groups : 1;
+    };
+    p.group = group_of(p.nbm);
+    p.group0 = group_of(p.nbm0);
     p.ln_staged = (long)TM * p.ln_tiles * 8 <= KS * (TM + TN) * ROW_BYTES && ((long)p.M * p.ln_tiles) % 2 == 0;
-    const int tiles = p.nbm * p.nbn, extra = alone ? read_ahead_workgroups(tiles) : 0;
+    const int tiles = p.nbm * p.nbn + p.nbm0 * p.nbn0, extra = alone && p.rows0 == 0 ? read_ahead_workgroups(tiles) : 0;
     hipLaunchKernelGGL((gemm_mid_kernel<EPI, MI, NI, WM, WN, S, WPE, KS, IL>), dim3(tiles + extra), dim3(64 * WM * WN), lds, st, p);
 }
 
@@ -384,22 +419,23 @@ void dispatch_tile(hipStream_t st, MidArgs& p, int tile, bool alone) {
         case 4: launch<EPI, 4, 2, 2, 4, 4, 2, 1, true>(st, p, alone); break;          // 128 x 128
         case 5: launch<EPI, 4, 4, 2, 4, 3, 2, 1, true>(st, p, alone); break;          // 128 x 256
         case 6: launch<EPI, 2, 2, 4, 2, 3, 2, 2, true>(st, p, alone); break;          // 128 x 64, two slabs at a time
-        default:
-            if constexpr ((EPI & EPI_LNFOLD) == 0) launch<EPI, 5, 2, 2, 2, 5, 2, 1, true>(st, p, alone);          // 160 x 64
-            else launch<EPI, 2, 2, 4, 2, 3, 4, 1, false>(st, p, alone);
-            break;
+        case 7: launch<EPI, 5, 2, 2, 2, 5, 2, 1, true>(st, p, alone); break;          // 160 x 64
+        case 8: launch<EPI, 3, 2, 2, 2, 5, 2, 1, true>(st, p, alone); break;          // 96 x 64
+        case 9: launch<EPI, 5, 2, 2, 4, 4, 2, 1, true>(st, p, alone); break;          // 160 x 128
+        case 10: launch<EPI, 3, 4, 4, 2, 4, 2, 1, true>(st, p, alone); break;         // 192 x 128
+        default: launch<EPI, 5, 4, 2, 4, 3, 2, 1, true>(st, p, alone); break;         // 160 x 256
     }
 }
 
 }  // namespace
 
-int cogs_k_gemm_mid(hipStream_t st, const CogsGemm& g, int tile, bool alone) {
+int cogs_k_gemm_mid(hipStream_t st, const CogsGemm& g, int tile, bool alone, int rows0, int cols0) {
     MidArgs p;
     const int rc = cogs_fill_epi(g, &p.epi);
     if (rc != COGS_OK) return rc;
     p.A = (const char*)g.A; p.lda = g.lda * 2;
     p.W = (const char*)g.W; p.ldw = g.ldw * 2;
-    p.M = g.M; p.N = g.N; p.KT = g.K / 64;
+    p.M = g.M; p.N = g.N; p.KT = g.K / 64; p.rows0 = rows0; p.cols0 = cols0;
     p.kv_k = (char*)g.kv_k; p.kv_v = (char*)g.kv_v; p.kv_col = g.kv_col0; p.kv_dim = g.kv_dim;
     if (g.kv_k && (g.kv_col0 % 64 || g.kv_dim % 64)) p.kv_k = nullptr;      // (copied by the caller)
     p.ln_part = g.ln_part; p.ln_tiles = g.K / 64; p.ln_inv_h = 1.0f / (float)g.K; p.ln_eps = g.ln_eps;

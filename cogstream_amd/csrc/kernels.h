@@ -50,7 +50,8 @@ struct CogsGemm {
     const float* ln_part = nullptr; float ln_eps = 0.f;
 };
 int cogs_k_gemm(hipStream_t st, const CogsGemm& g, bool* kv_stored = nullptr);     // kv_stored (for a call with kv_k): false: the caller copies them from C
-int cogs_k_gemm_mid(hipStream_t st, const CogsGemm& g, int tile, bool alone);     // gemm_mid.hip; the caller (cogs_k_gemm) has checked the operands. alone: no other stream's products beside it
+int cogs_k_gemm_mid(hipStream_t st, const CogsGemm& g, int tile, bool alone, int rows0 = 0, int cols0 = 0);     // gemm_mid.hip; the caller (cogs_k_gemm) has checked the operands. alone: no other stream's products beside it.
+// rows0, cols0: without the outputs of the first rows0 rows and cols0 columns (multiples of 64), which another launch computes; no read-ahead then
 void cogs_k_gemm_co_streams(int streams);   // streams fed with GEMMs of this size at once (thread-local): beside another stream a product of many tiles is not split, weights are not read ahead
 // (a, b) = (rstd, -rstd * mean) per row from the EPI_ROWSTAT partials [rows][tiles][2]: ab [rows][2]
 int cogs_k_ln_finalize(hipStream_t st, const float* stat_part, int rows, int tiles, int H, float eps, float* ab);

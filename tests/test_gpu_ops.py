@@ -1216,6 +1216,46 @@ def test_mid_size_gemm_tiles_of_two_slabs_and_of_160_rows(dev, tile):
     test_mid_size_gemm_tiles_equal_each_other_and_fp64(dev, tile)
 
 
+@pytest.mark.parametrize("tile", [8, 9, 10, 11])
+def test_mid_size_gemm_tiles_of_96_160_and_192_rows(dev, tile):
+    """the same edges for 96x64, 160x128, 192x128 and 160x256: pieces of a slab that the waves do not share evenly, three and five row
+    blocks a wave (a folded norm's factors: fewer rows than lanes, more than lanes); and their groups of row tiles"""
+    test_mid_size_gemm_tiles_equal_each_other_and_fp64(dev, tile)
+    test_mid_size_gemm_groups_of_row_tiles(dev, tile, 1537, 1544, 128)
+
+
+@pytest.mark.parametrize("M,N,K", [(700, 25600, 512), (4096, 6176, 512), (1030, 16640, 512), (2100, 9000, 512)])
+def test_whole_rounds_and_an_l_shaped_rest_equal_one_launch(dev, M, N, K):
+    """gemm.hip: whole rounds of ping-pong tiles over some row and column blocks and the rest of the product in one mid-size launch
+    (a strip of columns; columns and rows; ragged in either) give the bits of the ping-pong kernel alone: with a residual that
+    is overwritten (a tile that two launches computed would add it twice), statistics, rotation, a folded norm, SwiGLU"""
+    from cogstream_amd import _lib as L2
+    ops = _ops()
+    g = torch.Generator(device=dev).manual_seed(M)
+    rnd = lambda *s: (torch.randn(*s, generator=g, device=dev) * 0.5).bfloat16()
+    a, w, b, r = rnd(M, K), rnd(N, K), rnd(N), rnd(M, N)
+    cases = [("bias", dict(bias=b)), ("residual", dict(residual=r)), ("swiglu", dict(act=L2.ACT_SWIGLU)), ("fp32", dict(out_f32=True))]
+    if N % 64 == 0:
+        fold = dict(ln_ab=torch.rand(M, 2, generator=g, device=dev) + 0.5, col_c=torch.randn(N, generator=g, device=dev))
+        cases += [("statistics", dict(bias=b, residual=r, row_stats=torch.empty(M, N // 64, 2, device=dev))), ("folded norm", fold),
+                  ("rotary", dict(rope_cos=torch.randn(M, 32, 2, generator=g, device=dev), rope_cols=128, head_dim=64, bias=b))]
+    for name, kw in cases:
+        outs = []
+        for split in (1, 0):
+            with L2.debug_switch("gemm_split", split):
+                stats, out = kw.get("row_stats"), None
+                if stats is not None:
+                    stats.fill_(-7.0)
+                if name == "residual":
+                    kw = dict(residual=r.clone())
+                    out = kw["residual"]
+                y = ops.gemm(a, w, out=out, **kw)
+                assert L2.debug_get("gemm_last_body") == (5 if split else 4), (name, split)
+                outs.append((y.clone(), None if stats is None else stats.clone()))
+        assert torch.equal(outs[0][0], outs[1][0]), name
+        assert outs[0][1] is None or torch.equal(outs[0][1], outs[1][1]), name
+
+
 @pytest.mark.parametrize("t,h,w,merge,max_tokens,offset", [
     (1, 28, 28, 2, 16384, 0),        # one window, enlarged: the smallest
     (1, 45, 61, 1, 16384, 1),        # odd source sizes, frames that start off a word
