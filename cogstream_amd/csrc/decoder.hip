@@ -47,6 +47,7 @@ struct CogsDecoder {
     long max_qlat = 0, max_olat = 0;
     int max_dqk = 0, max_dv = 0, max_dheads = 0;       // gated delta rule: kv_heads x dim, heads x vdim, heads
     bool att_tail = false;
+    bool normed_out = false;                           // a sublayer's output is normed on its way into the stream
 };
 
 void cogs_decoder_free(CogsDecoder* d) {
@@ -59,7 +60,7 @@ void cogs_decoder_free(CogsDecoder* d) {
 namespace {
 
 struct Work {
-    float* x; void *h, *y, *cq, *q, *att, *act, *hn, *ctx, *kvx, *qlat, *olat;
+    float* x; void *h, *y[COGS_CHAIN], *cq, *q, *att, *act, *hn, *ctx, *kvx, *qlat, *olat;
     float *ypart, *t32, *gate, *rope, *part, *dq, *dk, *dv, *dbg, *dout, *drec;
     CogsSeq* seqs; int *rowseq, *rowpos, *want;
     size_t bytes;
@@ -69,13 +70,16 @@ struct Work {
 inline bool token_step(int rows, int nseq) { return rows == nseq; }
 inline bool absorbed_step(int rows, int nseq) { return token_step(rows, nseq) && g_cogs_debug.mla_absorb != 0; }
 
+// hyper-connected streams that wait for several sublayers' outputs (norm.hip); an output that is normed first needs its row's factor, once
+inline bool chained(const CogsDecoder& d, int S) { return !d.normed_out && cogs_k_stream_chain_fits(d.w.streams, d.wp, S); }
+
 Work carve(const CogsDecoder& d, int S, int nseq, int64_t C, int n_want, void* ws, size_t cap) {
     Carver c(ws, cap);
     const size_t es = esize(d.w.dtype), n = (size_t)S;
     Work k{};
     k.x = (float*)c.take(n * d.wp * 4 * (d.w.streams > 0 ? d.w.streams : 1));
     k.h = c.take(n * d.wp * es);
-    k.y = c.take(n * d.wp * es);
+    for (int i = 0; i < (chained(d, S) ? COGS_CHAIN : 1); ++i) k.y[i] = c.take(n * d.wp * es);
     // few-row products into the residual stream; there for more rows too, so that a workspace sized for them serves fewer
     if (d.w.dtype == COGS_DT_BF16) k.ypart = (float*)c.take((size_t)(S < 64 ? S : 64) * d.wp * 4 * COGS_SKINNY_MAX_PARTS);
     k.t32 = (float*)c.take(n * d.max_t32 * 4);
@@ -128,7 +132,9 @@ struct Step {
     cogs_handle h; hipStream_t st; const CogsDecoder& d; Work k;
     const std::vector<CogsSeq>& seqs;
     int S, nseq, max_new, max_ctx; int64_t C;
-    int y_parts = 0;           // the sublayer's output is k.y, or so many partial sums in k.ypart
+    bool chain;                // the streams wait for sublayers' outputs: `waiting` has their base and the outputs since
+    CogsStreamChain waiting{};
+    int y_parts = 0;           // the sublayer's output is k.y[waiting.n], or so many partial sums in k.ypart
 
     const void* at(const void* p, size_t elems) const { return (const char*)p + elems * esize(d.w.dtype); }
 
@@ -141,9 +147,9 @@ struct Step {
         return cogs_k_gemm(st, g);
     }
 
-    // a sublayer's last product, C = k.y: partial sums where few rows leave too few workgroups otherwise
+    // a sublayer's last product, C = k.y[waiting.n]: partial sums where few rows leave too few workgroups otherwise
     int lin_out(CogsGemm& g) {
-        g.C = k.y; g.ldc = d.wp; g.M = S; g.N = d.wp;
+        g.C = k.y[waiting.n]; g.ldc = d.wp; g.M = S; g.N = d.wp;
         g.dtype = d.w.dtype;
         const int parts = g_cogs_debug.gemm_skinny != 0 && cogs_k_gemm_skinny_fits(g) ? cogs_k_gemm_skinny_parts(g.M, g.N, g.K) : 1;
         y_parts = parts > 1 ? parts : 0;
@@ -321,9 +327,10 @@ struct Step {
 
     // x from the embeddings, or x += norm(y) through the sublayer's (`from`) hyper-connections; then h = norm of what `to` reads
     int stream(const void* embeds, const float* y_gamma, const cogs_hyper* from, const cogs_hyper* to, const float* out_gamma, float* sum, const CogsAhead& next) {
+        if (chain) return stream_chain(embeds, from, to, out_gamma);
         CogsStreamNorm a;
         a.ahead = next;
-        a.x = k.x; a.embeds = embeds; a.y = embeds ? nullptr : y_parts ? (const void*)k.ypart : k.y; a.y_parts = embeds ? 0 : y_parts; a.y_gamma = y_gamma; a.out = out_gamma ? k.h : nullptr; a.out_gamma = out_gamma;
+        a.x = k.x; a.embeds = embeds; a.y = embeds ? nullptr : y_parts ? (const void*)k.ypart : k.y[0]; a.y_parts = embeds ? 0 : y_parts; a.y_gamma = y_gamma; a.out = out_gamma ? k.h : nullptr; a.out_gamma = out_gamma;
         a.rows = S; a.H = d.w.width; a.Hp = d.wp; a.eps = d.w.eps;
         if (embeds) { a.embed_scale = d.w.embed_scale; a.pos = d.w.pos; a.rowpos = k.rowpos; }
         a.streams = d.w.streams; a.sum = sum;
@@ -332,6 +339,36 @@ struct Step {
             if (to) a.in_w = to->in;
         }
         PROF(COGS_PROF_NORM);
+        return cogs_k_stream_norm(st, d.w.dtype, a);
+    }
+    int stream_chain(const void* embeds, const cogs_hyper* from, const cogs_hyper* to, const float* out_gamma) {
+        CogsStreamChain& w = waiting;
+        if (embeds) {
+            w.x = k.x; w.embeds = embeds; w.embed_scale = d.w.embed_scale; w.pos = d.w.pos; w.rowpos = k.rowpos;
+            w.rows = S; w.H = d.w.width; w.Hp = d.wp; w.eps = d.w.eps; w.streams = d.w.streams;
+        } else {
+            w.outs[w.n] = {k.y[w.n], from->mix, from->out};
+            ++w.n;
+        }
+        if (!to) return COGS_OK;                 // the last one: `wanted` mixes the rows that are asked for
+        CogsStreamChain a = w;
+        a.out = k.h; a.out_gamma = out_gamma; a.in_w = to->in; a.store = w.n == COGS_CHAIN;
+        if (a.store) { w.n = 0; w.embeds = nullptr; }
+        PROF(COGS_PROF_NORM);
+        return cogs_k_stream_chain(st, d.w.dtype, a);
+    }
+
+    // the normed rows of the logits that are asked for
+    int wanted(int n_want) {
+        PROF(COGS_PROF_NORM);
+        if (chain) {
+            CogsStreamChain a = waiting;
+            a.out = k.hn; a.out_gamma = d.w.final_norm; a.pick = k.want; a.rows = n_want;
+            return cogs_k_stream_chain(st, d.w.dtype, a);
+        }
+        CogsStreamNorm a;
+        a.x = k.x; a.streams = d.w.streams; a.out = k.hn; a.out_gamma = d.w.final_norm; a.pick = k.want; a.rows = n_want; a.H = d.w.width; a.Hp = d.wp; a.eps = d.w.eps;
+        a.ahead = ahead(d.w.head, n_want, d.vocabp);
         return cogs_k_stream_norm(st, d.w.dtype, a);
     }
 };
@@ -424,6 +461,7 @@ cogs_status cogs_decoder_load(cogs_handle h, const cogs_decoder_weights* w) {
         } else {
             return fail(COGS_E_INVALID);
         }
+        if (L.norm1b || (L.mlp.ff > 0 && L.norm2b)) d->normed_out = true;
         mx(d->max_o, oin);
         if (ocols != oin) d->att_tail = true;
         if (L.mlp.ff > 0) {
@@ -510,7 +548,7 @@ cogs_status cogs_decoder_forward(cogs_handle h, cogs_stream stream, const void* 
     if (!ws || ws_bytes < k.bytes) return COGS_E_WORKSPACE;
     COGS_TRY(stage_h2d(h, st, k.seqs, seqs.data(), nseq * sizeof(CogsSeq)));
     if (n_want > 0) COGS_TRY(stage_h2d(h, st, k.want, want, (size_t)n_want * sizeof(int32_t)));
-    Step s{h, st, d, k, seqs, S, nseq, max_new, max_ctx, C};
+    Step s{h, st, d, k, seqs, S, nseq, max_new, max_ctx, C, chained(d, S) && !streams};
     {
         PROF(COGS_PROF_OTHER);
         COGS_TRY(cogs_k_seq_rows(st, k.seqs, nseq, S, k.rowseq, k.rowpos));
@@ -535,10 +573,7 @@ cogs_status cogs_decoder_forward(cogs_handle h, cogs_stream stream, const void* 
     }
     for (int i = 0; i < nseq; ++i) kv[i]->len += lens[i];
     if (n_want > 0) {
-        CogsStreamNorm a;
-        a.x = k.x; a.streams = d.w.streams; a.out = k.hn; a.out_gamma = d.w.final_norm; a.pick = k.want; a.rows = n_want; a.H = d.w.width; a.Hp = d.wp; a.eps = d.w.eps;
-        a.ahead = s.ahead(d.w.head, n_want, d.vocabp);
-        { PROF(COGS_PROF_NORM); COGS_TRY(cogs_k_stream_norm(st, d.w.dtype, a)); }
+        COGS_TRY(s.wanted(n_want));
         CogsGemm g;
         g.A = k.hn; g.lda = d.wp; g.W = d.w.head; g.ldw = d.wp; g.C = logits; g.ldc = d.vocabp; g.M = n_want; g.N = d.vocabp; g.K = d.wp; g.out_f32 = 1;
         COGS_TRY(s.lin(g));

@@ -205,6 +205,15 @@ struct CogsStreamNorm {
     CogsAhead ahead;           // read beside hyper-connected streams of few rows (a workgroup of 1024 threads each), ignored elsewhere
 };
 int cogs_k_stream_norm(hipStream_t st, int dtype, const CogsStreamNorm& a);
+// the same for two to four hyper-connected streams of many rows, with the outputs of up to COGS_CHAIN sublayers, in turn, that x (or the
+// embeddings) does not have yet; x is written where `store` says so, untouched otherwise. y, y_parts, mix, out_w, sum: unused
+constexpr int COGS_CHAIN = 4;
+struct CogsStreamChain : CogsStreamNorm {
+    int n = 0; bool store = false;
+    struct Out { const void* y; const float *mix, *out_w; } outs[COGS_CHAIN];
+};
+bool cogs_k_stream_chain_fits(int streams, int Hp, int rows);
+int cogs_k_stream_chain(hipStream_t st, int dtype, const CogsStreamChain& a);
 int cogs_k_zero(hipStream_t st, void* p, size_t bytes);      // 16-byte multiples
 
 // multi-head latent attention (mla.hip)

@@ -453,6 +453,109 @@ __global__ __launch_bounds__(TPB) void stream_mix_kernel(CogsStreamNorm p) {
     }
 }
 
+// Many rows: HBM. A mix reads and writes every stream (4 x fp32) for one sublayer output of 16 bits, so it need not be done at once: what the next
+// sublayer reads is formed from the streams as they were and the outputs since, each mix in its turn with the arithmetic and the order of
+// stream_mix_kernel (the same bits), and only the COGS_CHAIN-th output has the streams written. The first ones start from the embeddings, one
+// 16-bit row for all streams, and the last ones are mixed for the rows that are asked for alone. 4096 rows of 4 x 2048, us (stream_mix_kernel
+// 66 each): 26, 27, 36, 53 from the embeddings, then 38, 37, 42, 61 in turn; 1109 -> 634 in a prompt of 16 sublayers. (A number of streams that is
+// not the template's made it 760, predicates and scalar loads one by one; rows walked by fewer workgroups 907. Longer chains cost what they save:
+// 20 multiplications an element and output.)
+template <typename T, int C, int NS>
+__global__ __launch_bounds__(256) void stream_chain_kernel(CogsStreamChain p) {
+    constexpr int TPB = 256;
+    typedef T raw_t __attribute__((ext_vector_type(4)));
+    __shared__ float red[TPB / 64];
+    const int tid = threadIdx.x;
+    const long row = p.pick ? p.pick[blockIdx.x] : blockIdx.x;
+    float* x = p.x + row * NS * p.Hp;
+    int at[C];
+#pragma unroll
+    for (int c = 0; c < C; ++c) at[c] = min((tid + TPB * c) * 4, p.Hp - 4);
+    f32x4 v[C][NS];
+    raw_t y[COGS_CHAIN][C];
+    if (p.embeds) {
+        const T* pos = p.pos ? reinterpret_cast<const T*>(p.pos) + (long)p.rowpos[row] * p.Hp : nullptr;
+#pragma unroll
+        for (int c = 0; c < C; ++c) {
+            f32x4 e = ld4_f<T>(reinterpret_cast<const T*>(p.embeds) + row * p.Hp + at[c]) * p.embed_scale;
+            if (pos) e += ld4_f<T>(pos + at[c]);
+#pragma unroll
+            for (int s = 0; s < NS; ++s) v[c][s] = e;
+        }
+    } else {
+#pragma unroll
+        for (int c = 0; c < C; ++c)
+#pragma unroll
+            for (int s = 0; s < NS; ++s) v[c][s] = *reinterpret_cast<const f32x4*>(x + (long)s * p.Hp + at[c]);
+    }
+#pragma unroll
+    for (int q = 0; q < COGS_CHAIN; ++q)
+        if (q < p.n)
+#pragma unroll
+            for (int c = 0; c < C; ++c) y[q][c] = *reinterpret_cast<const raw_t*>(reinterpret_cast<const T*>(p.outs[q].y) + row * p.Hp + at[c]);
+#pragma unroll
+    for (int q = 0; q < COGS_CHAIN; ++q) {
+        if (q >= p.n) continue;
+        float mix[NS * NS], out_w[NS];
+#pragma unroll
+        for (int s = 0; s < NS * NS; ++s) mix[s] = p.outs[q].mix[s];
+#pragma unroll
+        for (int s = 0; s < NS; ++s) out_w[s] = p.outs[q].out_w[s];
+#pragma unroll
+        for (int c = 0; c < C; ++c) {
+            const f32x4 yv = ld4_f<T>(reinterpret_cast<const T*>(&y[q][c]));
+            f32x4 w[NS];
+#pragma unroll
+            for (int t = 0; t < NS; ++t) {
+                w[t] = yv * out_w[t];
+#pragma unroll
+                for (int s = 0; s < NS; ++s) w[t] += v[c][s] * mix[s * NS + t];
+            }
+#pragma unroll
+            for (int t = 0; t < NS; ++t) v[c][t] = w[t];
+        }
+    }
+    f32x4 u[C];
+    float ss = 0.f;
+#pragma unroll
+    for (int c = 0; c < C; ++c) {
+        u[c] = f32x4{0.f, 0.f, 0.f, 0.f};
+        if ((tid + TPB * c) * 4 >= p.Hp) continue;
+#pragma unroll
+        for (int s = 0; s < NS; ++s) {
+            if (p.store) *reinterpret_cast<f32x4*>(x + (long)s * p.Hp + at[c]) = v[c][s];
+            u[c] += p.in_w ? v[c][s] * p.in_w[s] : v[c][s];
+        }
+#pragma unroll
+        for (int e = 0; e < 4; ++e) ss += u[c][e] * u[c][e];
+    }
+    ss = wave_sum(ss);
+    if ((tid & 63) == 0) red[tid >> 6] = ss;
+    __syncthreads();
+    ss = red[0];
+#pragma unroll
+    for (int w = 1; w < TPB / 64; ++w) ss += red[w];
+    const float rs = 1.f / sqrtf(ss / (float)p.H + p.eps);
+    T* o = reinterpret_cast<T*>(p.out) + (long)blockIdx.x * p.Hp;
+#pragma unroll
+    for (int c = 0; c < C; ++c)
+        if ((tid + TPB * c) * 4 < p.Hp) st4_f<T>(o + at[c], u[c] * rs * *reinterpret_cast<const f32x4*>(p.out_gamma + at[c]));
+}
+
+template <typename T>
+int launch_stream_chain(hipStream_t st, const CogsStreamChain& a) {
+#define COGS_CHAIN_CASE(C, NS) hipLaunchKernelGGL((stream_chain_kernel<T, C, NS>), dim3(a.rows), dim3(256), 0, st, a)
+#define COGS_CHAIN_STREAMS(NS) case NS: if (a.Hp <= 2048) COGS_CHAIN_CASE(2, NS); else COGS_CHAIN_CASE(4, NS); break;
+    switch (a.streams) {
+        COGS_CHAIN_STREAMS(2)
+        COGS_CHAIN_STREAMS(3)
+        COGS_CHAIN_STREAMS(4)
+    }
+#undef COGS_CHAIN_STREAMS
+#undef COGS_CHAIN_CASE
+    return COGS_LAUNCH_CHECK();
+}
+
 template <typename T, int NS>
 int launch_stream_mix(hipStream_t st, const CogsStreamNorm& a) {
     const int rows = a.rows, more = ahead_workgroups(a.ahead, rows);
@@ -519,6 +622,18 @@ int cogs_k_stream_norm(hipStream_t st, int dtype, const CogsStreamNorm& a) {
     if (a.y_parts != 0 && a.y_parts != 2 && a.y_parts != 4 && a.y_parts != 8) return COGS_E_INVALID;
     if (!a.x || a.Hp % 4 || a.H <= 0 || a.H > a.Hp || (a.out && !a.out_gamma) || (a.pick && (!a.out || a.y || a.embeds))) return COGS_E_INVALID;
     return dtype == COGS_DT_BF16 ? launch_stream_norm<bf16_t>(st, a) : launch_stream_norm<float>(st, a);
+}
+
+// more than 64 rows: fewer are latency (their own kernel, which reads weights ahead). The row is in the registers of 256 threads: up to 4096 columns
+bool cogs_k_stream_chain_fits(int streams, int Hp, int rows) { return streams >= 2 && streams <= 4 && Hp <= 4096 && rows > 64; }
+
+int cogs_k_stream_chain(hipStream_t st, int dtype, const CogsStreamChain& a) {
+    if (a.rows <= 0) return COGS_OK;
+    if (a.streams < 2 || a.streams > 4 || a.Hp > 4096 || a.Hp % 4 || a.H <= 0 || a.H > a.Hp || a.n < 0 || a.n > COGS_CHAIN) return COGS_E_INVALID;
+    if (!a.x || !a.out || !a.out_gamma || (a.pos && !a.rowpos) || (a.pick && a.store) || a.y || a.sum) return COGS_E_INVALID;
+    for (int q = 0; q < a.n; ++q)
+        if (!a.outs[q].y || !a.outs[q].mix || !a.outs[q].out_w) return COGS_E_INVALID;
+    return dtype == COGS_DT_BF16 ? launch_stream_chain<bf16_t>(st, a) : launch_stream_chain<float>(st, a);
 }
 
 int cogs_k_layernorm(hipStream_t st, int dtype, const void* x, void* y, const void* gamma, const void* beta,

@@ -404,6 +404,8 @@ class DecoderEngine(CausalEngine):
         nbytes = C.c_size_t()
         L.check(L.lib.cogs_decoder_workspace_bytes(self.handle.h, S, n, ctx, nw, C.byref(nbytes)), "cogs_decoder_workspace_bytes")
         ws = self.handle.workspace("decoder", nbytes.value)
+        if S > 64:
+            embeds.record_stream(torch.cuda.current_stream())      # (several layers of a prompt read it)
         logits = torch.empty(nw, self.packed.vocab_p, device=self.device, dtype=torch.float32) if nw else None
         kv = (C.POINTER(L.KV) * n)(*[C.pointer(c.struct) for c in caches])
         L.check(L.lib.cogs_decoder_forward(self.handle.h, L.current_stream(), embeds.data_ptr(), kv, (C.c_int32 * n)(*lens), n,
