@@ -261,13 +261,17 @@ cogs_status cogs_kmeans_pp_step(cogs_stream stream, int dtype, const void* feats
     if (!feats || !nearest2 || T <= 0) return COGS_E_INVALID;
     return cogs_k_kmeans_pp_step((hipStream_t)stream, dtype, feats, T, PD, row, first, nearest2, probs_host, (float*)ws, ns);
 }
-cogs_status cogs_kmeans_pp(cogs_stream stream, int dtype, const void* feats, int T, int64_t PD, int K, int first_row,
-                           const float* q_draws, int32_t* idx, int32_t* zero_flag, float* nearest2, void* ws, size_t ws_bytes) {
+cogs_status cogs_kmeans_pp_dist(cogs_stream stream, int dtype, const void* feats, int T, int64_t PD, int K, int first_row,
+                                const float* q_draws, int32_t* idx, int32_t* zero_flag, float* nearest2, float* dist2, void* ws, size_t ws_bytes) {
     int ns = 0;
     const size_t need = cogs_k_kmeans_ws(T, PD, 1, &ns);
     if (!ws || ws_bytes < need) return COGS_E_WORKSPACE;
     if (!feats || !q_draws || !idx || !zero_flag || !nearest2 || T <= 0 || K <= 0) return COGS_E_INVALID;
-    return cogs_k_kmeans_pp((hipStream_t)stream, dtype, feats, T, PD, K, first_row, q_draws, idx, zero_flag, nearest2, (float*)ws, ns);
+    return cogs_k_kmeans_pp((hipStream_t)stream, dtype, feats, T, PD, K, first_row, q_draws, idx, zero_flag, nearest2, dist2, (float*)ws, ns);
+}
+cogs_status cogs_kmeans_pp(cogs_stream stream, int dtype, const void* feats, int T, int64_t PD, int K, int first_row,
+                           const float* q_draws, int32_t* idx, int32_t* zero_flag, float* nearest2, void* ws, size_t ws_bytes) {
+    return cogs_kmeans_pp_dist(stream, dtype, feats, T, PD, K, first_row, q_draws, idx, zero_flag, nearest2, nullptr, ws, ws_bytes);
 }
 cogs_status cogs_kmeans_margins(cogs_stream stream, int T, int64_t PD, int K, void* ws, size_t ws_bytes, float* min_margin,
                                 int32_t* rows_below) {
@@ -275,16 +279,23 @@ cogs_status cogs_kmeans_margins(cogs_stream stream, int T, int64_t PD, int K, vo
     if (!ws || ws_bytes < need) return COGS_E_WORKSPACE;
     return cogs_k_kmeans_margins((hipStream_t)stream, T, PD, K, (float*)ws, min_margin, rows_below);
 }
-cogs_status cogs_kmeans_lloyd(cogs_stream stream, int dtype, const void* feats, const float* ts, int T, int64_t PD, int K,
-                              float alpha, int max_iter, float tol, const int32_t* reseed_pool, int pool_len,
-                              float* centres, float* centre_ts, int64_t* assign, int* iterations, int* reseeds_used,
-                              int* pool_exhausted, void* ws, size_t ws_bytes) {
+cogs_status cogs_kmeans_lloyd_dist(cogs_stream stream, int dtype, const void* feats, const float* ts, int T, int64_t PD, int K,
+                                   float alpha, int max_iter, float tol, const int32_t* reseed_pool, int pool_len,
+                                   float* centres, float* centre_ts, int64_t* assign, int* iterations, int* reseeds_used,
+                                   int* pool_exhausted, float* dist2, int known, void* ws, size_t ws_bytes) {
     int ns = 0;
     const size_t need = cogs_k_kmeans_ws(T, PD, K, &ns);
     if (!ws || ws_bytes < need) return COGS_E_WORKSPACE;
     if (!feats || !ts || !centres || !centre_ts || !assign || (pool_len > 0 && !reseed_pool)) return COGS_E_INVALID;
     return cogs_k_kmeans_lloyd((hipStream_t)stream, dtype, feats, ts, T, PD, K, alpha, max_iter, tol, reseed_pool, pool_len,
-                               centres, centre_ts, assign, iterations, reseeds_used, pool_exhausted, (float*)ws, ns);
+                               centres, centre_ts, assign, iterations, reseeds_used, pool_exhausted, dist2, known, (float*)ws, ns);
+}
+cogs_status cogs_kmeans_lloyd(cogs_stream stream, int dtype, const void* feats, const float* ts, int T, int64_t PD, int K,
+                              float alpha, int max_iter, float tol, const int32_t* reseed_pool, int pool_len,
+                              float* centres, float* centre_ts, int64_t* assign, int* iterations, int* reseeds_used,
+                              int* pool_exhausted, void* ws, size_t ws_bytes) {
+    return cogs_kmeans_lloyd_dist(stream, dtype, feats, ts, T, PD, K, alpha, max_iter, tol, reseed_pool, pool_len, centres, centre_ts,
+                                  assign, iterations, reseeds_used, pool_exhausted, nullptr, 0, ws, ws_bytes);
 }
 cogs_status cogs_pack_rows(cogs_stream stream, int in_dtype, int out_dtype, const void* in, int64_t ld_in, void* out,
                            int64_t ld_out, int rows, int cols_in, int cols_out) {

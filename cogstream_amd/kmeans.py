@@ -24,12 +24,12 @@ would flip its cluster (cogs_kmeans_margins; (d2 - d1) / mean(d1, d2) of the two
 equal); rows_below_1e-3 = (row, iteration) pairs under 1e-3, where the reference's own cdist rounding decides a row."""
 
 
-def _lloyd_from_rows(x, ts, rows, K: int, PD: int, alpha: float, max_iteration: int, tol: float, ws):
+def _lloyd_from_rows(x, ts, rows, K: int, PD: int, alpha: float, max_iteration: int, tol: float, ws, dist2=None):
     """Lloyd iterations (:71-131) from the centres x[rows], inside the library. Empty clusters are reseeded with
     random.randint(0, T-1) per cluster in ascending order (:116-120): the values are drawn AHEAD into a pool the device
     consumes in that order, and the generator is then put back to where the reference would have left it (state
     restored, the used number of draws replayed). -> (centres [K, PD] fp32, centre_ts, assign, iterations)"""
-    T = x.shape[0]
+    T, known = x.shape[0], 0 if dist2 is None else K - 1         # dist2 [T, K]: the seeding's squared distances to all of `rows` but the last
     centres = ops.pack_rows(x.index_select(0, rows), torch.float32, PD) if x.dtype != torch.float32 \
         else x.index_select(0, rows).contiguous()
     centre_ts = ts.index_select(0, rows).contiguous()
@@ -40,7 +40,8 @@ def _lloyd_from_rows(x, ts, rows, K: int, PD: int, alpha: float, max_iteration: 
     while left > 0:
         drawn.extend(random.randint(0, T - 1) for _ in range(pool_n))
         it, used, exhausted = ops.kmeans_lloyd(x, ts, centres, centre_ts, assign, float(alpha), left, float(tol),
-                                               drawn[used_total:], ws)
+                                               drawn[used_total:], ws, dist2, known)
+        known = 0
         done, left, used_total = done + it, left - it, used_total + used
         if not exhausted:
             break
@@ -80,10 +81,11 @@ def kmeans_with_time_min_max(features: torch.Tensor, timestamp, cluster_num: int
     q = torch.empty(K - 1, T, dtype=torch.float32)
     for row in q.unbind(0):
         row.exponential_(1)
-    idx_d, flag = ops.kmeans_pp(x, first, K, q.to(dev, non_blocking=True), ws)
+    dist2 = torch.empty(T, K, dtype=torch.float32, device=dev)
+    idx_d, flag = ops.kmeans_pp(x, first, K, q.to(dev, non_blocking=True), ws, dist2)
     # (no host read here: the Lloyd loop below starts from the device-resident rows; the flag is looked at after its
     # first synchronisation, and in the rare flagged case everything is redone step by step)
-    run = _lloyd_from_rows(x, ts, idx_d.to(torch.int64), K, PD, alpha, max_iteration, tol, ws)
+    run = _lloyd_from_rows(x, ts, idx_d.to(torch.int64), K, PD, alpha, max_iteration, tol, ws, dist2)
     if int(flag.item()) == 0:
         last_stats["kpp_path"] = "one call"
     else:

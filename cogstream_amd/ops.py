@@ -263,16 +263,17 @@ def kmeans_pp_step(feats, row: int, first: bool, nearest2: torch.Tensor, probs_h
                                     ptr(nearest2), ptr(probs_host), ptr(ws), ws.numel()), "cogs_kmeans_pp_step")
 
 
-def kmeans_pp(feats, first_row: int, K: int, q_draws: torch.Tensor, ws):
+def kmeans_pp(feats, first_row: int, K: int, q_draws: torch.Tensor, ws, dist2: Optional[torch.Tensor] = None):
     """cogs_kmeans_pp -> (centre rows int32 [K] on the device, zero-sum flag int32 [1] on the device). q_draws: device
-    fp32 [K-1, T] Exponential(1) draws of the CPU generator"""
+    fp32 [K-1, T] Exponential(1) draws of the CPU generator. dist2 (fp32 [T, K]) receives the squared distances to centres 0 .. K-2"""
     T, PD = feats.shape
+    assert dist2 is None or (dist2.is_cuda and dist2.dtype == torch.float32 and dist2.shape == (T, K) and dist2.is_contiguous())
     assert q_draws.is_cuda and q_draws.dtype == torch.float32 and q_draws.shape == (K - 1, T) and q_draws.is_contiguous()
     buf = torch.empty(K + 1, device=feats.device, dtype=torch.int32)       # [K] centre rows + the flag, one allocation
     idx, flag = buf[:K], buf[K:]
     nearest2 = torch.empty(T, device=feats.device, dtype=torch.float32)
-    check(L.lib.cogs_kmeans_pp(current_stream(), dtype_code(feats.dtype), ptr(feats), T, PD, int(K), int(first_row), ptr(q_draws),
-                               ptr(idx), ptr(flag), ptr(nearest2), ptr(ws), ws.numel()), "cogs_kmeans_pp")
+    check(L.lib.cogs_kmeans_pp_dist(current_stream(), dtype_code(feats.dtype), ptr(feats), T, PD, int(K), int(first_row), ptr(q_draws),
+                               ptr(idx), ptr(flag), ptr(nearest2), ptr(dist2), ptr(ws), ws.numel()), "cogs_kmeans_pp")
     return idx, flag
 
 
@@ -285,15 +286,18 @@ def kmeans_margins(T: int, PD: int, K: int, ws):
     return float(m.value), int(n.value)
 
 
-def kmeans_lloyd(feats, ts, centres, centre_ts, assign, alpha: float, max_iter: int, tol: float, pool, ws):
-    """cogs_kmeans_lloyd -> (iterations completed, reseeds used, pool exhausted). pool: python list of pre-drawn rows"""
+def kmeans_lloyd(feats, ts, centres, centre_ts, assign, alpha: float, max_iter: int, tol: float, pool, ws,
+                 dist2: Optional[torch.Tensor] = None, known: int = 0):
+    """cogs_kmeans_lloyd -> (iterations completed, reseeds used, pool exhausted). pool: python list of pre-drawn rows. dist2 (fp32
+    [T, K], overwritten): its first `known` columns are the squared distances to the first `known` centres as given"""
     T, PD = feats.shape
     K = centres.shape[0]
+    assert dist2 is None or (dist2.is_cuda and dist2.dtype == torch.float32 and dist2.shape == (T, K) and dist2.is_contiguous())
     arr = (C.c_int32 * max(len(pool), 1))(*pool)
     it, used, ex = C.c_int(0), C.c_int(0), C.c_int(0)
-    check(L.lib.cogs_kmeans_lloyd(current_stream(), dtype_code(feats.dtype), ptr(feats), ptr(ts), T, PD, K, float(alpha),
+    check(L.lib.cogs_kmeans_lloyd_dist(current_stream(), dtype_code(feats.dtype), ptr(feats), ptr(ts), T, PD, K, float(alpha),
                                   int(max_iter), float(tol), C.cast(arr, C.c_void_p), len(pool), ptr(centres), ptr(centre_ts),
-                                  ptr(assign), C.byref(it), C.byref(used), C.byref(ex), ptr(ws), ws.numel()),
+                                  ptr(assign), C.byref(it), C.byref(used), C.byref(ex), ptr(dist2), int(known), ptr(ws), ws.numel()),
           "cogs_kmeans_lloyd")
     return it.value, used.value, bool(ex.value)
 

@@ -249,6 +249,10 @@ cogs_status cogs_kmeans_pp_step(cogs_stream stream, int dtype, const void* feats
  * common divisor of all ratios. Workspace: cogs_kmeans_workspace_bytes(T, PD, 1). */
 cogs_status cogs_kmeans_pp(cogs_stream stream, int dtype, const void* feats, int T, int64_t PD, int K, int first_row,
                            const float* q_draws, int32_t* idx, int32_t* zero_flag, float* nearest2, void* ws, size_t ws_bytes);
+/* The same; dist2 (nullable, device fp32 [T][K]) also receives the squared distances to centres 0 .. K - 2 (its last column is not
+ * written), for cogs_kmeans_lloyd_dist from centres x[idx]. */
+cogs_status cogs_kmeans_pp_dist(cogs_stream stream, int dtype, const void* feats, int T, int64_t PD, int K, int first_row,
+                                const float* q_draws, int32_t* idx, int32_t* zero_flag, float* nearest2, float* dist2, void* ws, size_t ws_bytes);
 /* The whole Lloyd loop (:71-131) from given centres: per iteration distances -> assignment -> means / reseeds -> centre
  * shift, stopping after max_iter iterations or when the shift is <= tol. The library queues up to four iterations
  * between two synchronisations of the stream (it reads eight control words from host-mapped memory); every kernel of an
@@ -263,6 +267,12 @@ cogs_status cogs_kmeans_lloyd(cogs_stream stream, int dtype, const void* feats, 
                               float alpha, int max_iter, float tol, const int32_t* reseed_pool, int pool_len,
                               float* centres, float* centre_ts, int64_t* assign, int* iterations, int* reseeds_used,
                               int* pool_exhausted, void* ws, size_t ws_bytes);
+/* The same; dist2 (nullable unless known > 0, device fp32 [T][K], overwritten): its first `known` columns hold the squared distances
+ * to the first `known` centres as they come in, which are then not summed again. */
+cogs_status cogs_kmeans_lloyd_dist(cogs_stream stream, int dtype, const void* feats, const float* ts, int T, int64_t PD, int K,
+                                   float alpha, int max_iter, float tol, const int32_t* reseed_pool, int pool_len,
+                                   float* centres, float* centre_ts, int64_t* assign, int* iterations, int* reseeds_used,
+                                   int* pool_exhausted, float* dist2, int known, void* ws, size_t ws_bytes);
 /* How close the assignments of the LAST cogs_kmeans_lloyd call on this workspace were (host outputs; synchronises).
  * Per row and iteration: the relative change of the row's feature distances that would flip the decision between its
  * best and second-best cluster -- with every time term equal this is (d2 - d1) / mean(d1, d2) of the two nearest feature

@@ -1412,3 +1412,47 @@ def test_a_split_product_whose_remainder_is_one_row(dev, M, N, K, form):
         outs.append((out, None if stats is None else stats.clone()))
     (x, sx), (y, sy) = outs
     assert torch.equal(x, y) and (sx is None or torch.equal(sx, sy))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("T,K,PD,kind", [(40, 5, 520, "plain"), (150, 33, 1032, "plain"), (200, 70, 512, "plain"), (64, 6, 1024, "empty"),
+                                         (48, 4, 1024, "infinite"), (3, 2, 8, "plain")])
+def test_centres_that_stay_keep_their_distances_and_means(dev, T, K, PD, kind, dtype):
+    """csrc/kmeans.hip: the Lloyd loop sums distances and means only for centres whose rows have changed, and not those the seeding
+    has summed. Every iteration bit for bit against the same steps called one by one, which sum everything: more centres than one distance
+    launch holds, or than a wave, with clusters that run empty (duplicated centres, reseeded) and a row of infinities"""
+    ops = _ops()
+    g = torch.Generator(device=dev).manual_seed(T + K)
+    x = (torch.randn(max(2, K // 2), PD, generator=g, device=dev).repeat(T, 1)[:T] + 0.3 * torch.randn(T, PD, generator=g, device=dev)).to(dtype)
+    if kind == "infinite":
+        x[5, 3] = float("inf")
+    ts = torch.arange(T, device=dev, dtype=torch.float32)
+    ws = ops.kmeans_workspace(T, PD, K, dev)
+    q = torch.rand(K - 1, T, generator=g, device=dev) + 0.01
+    d2 = torch.full((T, K), -1.0, device=dev)
+    rows, flag = ops.kmeans_pp(x, 2, K, q, ws, d2)
+    known = K - 1 if kind == "plain" and int(flag) == 0 else 0
+    rows = rows.long()
+    if kind == "empty":
+        rows = torch.full((K,), 7, device=dev)
+        rows[0] = 11
+    pool = [int(v) for v in torch.randint(0, T, (400,), generator=torch.Generator().manual_seed(1))]
+    c0, t0 = x[rows].float().contiguous(), ts[rows].contiguous()
+    if known:                                  # the seeding's sums are those of the distance pass (fp64 over slices: the last place at most)
+        whole = ops.kmeans_sqdist(x, c0, None, K, ws)
+        assert bool(((d2[:, :known] - whole[:, :known]).abs() <= whole[:, :known] * 2.0 ** -23).all())
+    for iters in (1, 2, 3, 5, 9):
+        c, ct, used, done = c0.clone(), t0.clone(), 0, 0
+        for _ in range(iters):
+            a, _ = ops.kmeans_assign(ops.kmeans_sqdist(x, c, None, K, ws), ts, ct, 2.0)
+            empty = torch.bincount(a, minlength=K) == 0
+            reseed = torch.zeros(K, dtype=torch.int32, device=dev)
+            n = int(empty.sum())
+            reseed[empty] = torch.tensor(pool[used:used + n], dtype=torch.int32, device=dev)
+            used, done = used + n, done + 1
+            if float(ops.kmeans_update(x, ts, a, reseed, c, ct, ws)) <= 1e-4:
+                break
+        gc, gt, ga = c0.clone(), t0.clone(), torch.empty(T, dtype=torch.int64, device=dev)
+        got = ops.kmeans_lloyd(x, ts, gc, gt, ga, 2.0, iters, 1e-4, pool, ws, d2.clone() if known else None, known)
+        assert got == (done, used, False), (iters, got, done, used)
+        assert torch.equal(ga, a) and torch.equal(gt, ct) and torch.equal(gc.view(torch.int32), c.view(torch.int32)), iters
