@@ -934,8 +934,18 @@ static cogs_status llm_forward_impl(cogs_handle h, cogs_stream stream, const voi
     { PROF(COGS_PROF_OTHER); COGS_TRY(cogs_k_llm_rope_table(st, rc, rs, nseg > 0 ? pos_d : nullptr, pos0, S, h->llm_inv_freq, hd / 2)); }
     const float scale = 1.0f / sqrtf((float)hd);
     const bool prescale_q = dt == COGS_DT_BF16 && hd == 128;   // see cogs_vit_encode
+    const bool need_all = pooled_mean || hidden_out;
+    // Of the last layer nothing but the keys and values is used of the rows whose logits are not asked for: behind them it goes on with the
+    // last row's query tile (rows before that are a whole number of tiles, and two rows at the least are left, so that every row's sums are those
+    // of the whole prompt, bit for bit). 15 395 rows of 28 layers 190.6 -> 185.4 ms, 621 rows 9.76 -> 9.70.
+    const int last_from = nseg == 0 && !need_all && dt == COGS_DT_BF16 && S > 256 ? (S - 2) / 128 * 128 : 0;
     for (int l = 0; l < w.layers; ++l) {
         const cogs_llm_layer& L = h->llm_layers[l];
+        const int r0 = l == w.layers - 1 ? last_from : 0, R = S - r0;      // rows behind the keys and values
+        char* const xr = (char*)x + (size_t)r0 * H * es;
+        char* const lnr = (char*)ln + (size_t)r0 * H * es;
+        char* const qr = (char*)qkv + (size_t)r0 * qd * es;
+        char* const attr = (char*)att + (size_t)r0 * qd_q * es;
         const bool fuse_norm = (S == 1);   // single-token decode: RMSNorm runs inside the GEMV prologue
         const void* xin = (embeds_in_place && l == 0) ? embeds : (const void*)x;    // the residual stream entering this layer
         if (!fuse_norm) { PROF(COGS_PROF_NORM); COGS_TRY(cogs_k_rmsnorm(st, dt, x, ln, L.in_ln, S, H, w.rms_eps)); }
@@ -950,6 +960,14 @@ static cogs_status llm_forward_impl(cogs_handle h, cogs_stream stream, const voi
                 g.kv_k = (char*)kv->k + (((size_t)l * kv->max_len) + pos0) * kvd * es;
                 g.kv_v = (char*)kv->v + (((size_t)l * kv->max_len) + pos0) * kvd * es;
                 g.kv_col0 = qd_q; g.kv_dim = kvd;
+            }
+            if (r0 > 0 && S > 1024) {      // queries of those rows (fewer rows: two launches cost what one saves)
+                CogsGemm q = g;
+                q.A = lnr; q.C = qr; q.M = R; q.N = qd_q; q.rope_cols = qd_q; q.kv_k = q.kv_v = nullptr;
+                q.rope_cos = rc + (size_t)r0 * hd;
+                { PROF(COGS_PROF_GEMM); COGS_TRY(cogs_k_gemm(st, q)); }
+                g.W = (const char*)L.qkv_w + (size_t)qd_q * H * es; g.bias = L.qkv_b ? (const char*)L.qkv_b + (size_t)qd_q * es : nullptr;
+                g.C = (char*)qkv + (size_t)qd_q * es; g.N = 2 * kvd; g.rope_cols = kvd; g.q_scale = 1.f; g.q_cols = 0; g.kv_col0 = 0;
             }
             bool kv_stored = true;
             { PROF(COGS_PROF_GEMM); COGS_TRY(cogs_k_gemm(st, g, &kv_stored)); }
@@ -969,10 +987,10 @@ static cogs_status llm_forward_impl(cogs_handle h, cogs_stream stream, const voi
         }
         {
             CogsAttn a; a.dtype = dt;
-            a.Q = qkv; a.K = kp; a.V = vp; a.O = att;
+            a.Q = qr; a.K = kp; a.V = vp; a.O = attr;
             a.ldq = qd; a.ldk = ldkv; a.ldv = ldkv; a.ldo = qd_q;
-            a.q_len = S; a.kv_len = ctx; a.hq = w.heads; a.hkv = w.kv_heads; a.head_dim = hd; a.scale = scale;
-            a.causal = 1; a.q_pos0 = pos0; a.q_prescaled = prescale_q;
+            a.q_len = R; a.kv_len = ctx; a.hq = w.heads; a.hkv = w.kv_heads; a.head_dim = hd; a.scale = scale;
+            a.causal = 1; a.q_pos0 = pos0 + r0; a.q_prescaled = prescale_q;
             if (nseg > 0) { a.cu_seqlens = cu_d; a.nseg = nseg; a.max_seqlen = max_seg; }
             if (S == 1 && dt == COGS_DT_BF16 && hd == 128) {
                 a.nsplit = llm_nsplit(ctx); a.ws = split; a.ws_bytes = split_bytes;
@@ -981,22 +999,22 @@ static cogs_status llm_forward_impl(cogs_handle h, cogs_stream stream, const voi
         }
         {
             CogsGemm g; g.dtype = dt;
-            g.A = att; g.lda = qd_q; g.W = L.o_w; g.ldw = qd_q; g.C = x; g.ldc = H;
-            g.residual = xin; g.ldr = H; g.M = S; g.N = H; g.K = qd_q;
+            g.A = attr; g.lda = qd_q; g.W = L.o_w; g.ldw = qd_q; g.C = xr; g.ldc = H;
+            g.residual = r0 ? xr : xin; g.ldr = H; g.M = R; g.N = H; g.K = qd_q;
             { PROF(COGS_PROF_GEMM); COGS_TRY(cogs_k_gemm(st, g)); }
         }
-        if (!fuse_norm) { PROF(COGS_PROF_NORM); COGS_TRY(cogs_k_rmsnorm(st, dt, x, ln, L.post_ln, S, H, w.rms_eps)); }
+        if (!fuse_norm) { PROF(COGS_PROF_NORM); COGS_TRY(cogs_k_rmsnorm(st, dt, xr, lnr, L.post_ln, R, H, w.rms_eps)); }
         {
             CogsGemm g; g.dtype = dt;
-            g.A = fuse_norm ? x : ln; g.lda = H; g.W = L.gu_w; g.ldw = H; g.C = act; g.ldc = w.inter;
-            g.M = S; g.N = 2 * w.inter; g.K = H; g.act = COGS_ACT_SWIGLU;
+            g.A = fuse_norm ? x : lnr; g.lda = H; g.W = L.gu_w; g.ldw = H; g.C = act; g.ldc = w.inter;
+            g.M = R; g.N = 2 * w.inter; g.K = H; g.act = COGS_ACT_SWIGLU;
             if (fuse_norm) { g.rms_gamma = L.post_ln; g.rms_eps = w.rms_eps; }
             { PROF(COGS_PROF_GEMM); COGS_TRY(cogs_k_gemm(st, g)); }
         }
         {
             CogsGemm g; g.dtype = dt;
-            g.A = act; g.lda = w.inter; g.W = L.down_w; g.ldw = w.inter; g.C = x; g.ldc = H;
-            g.residual = x; g.ldr = H; g.M = S; g.N = H; g.K = w.inter;
+            g.A = act; g.lda = w.inter; g.W = L.down_w; g.ldw = w.inter; g.C = xr; g.ldc = H;
+            g.residual = xr; g.ldr = H; g.M = R; g.N = H; g.K = w.inter;
             { PROF(COGS_PROF_GEMM); COGS_TRY(cogs_k_gemm(st, g)); }
         }
     }
@@ -1011,7 +1029,6 @@ static cogs_status llm_forward_impl(cogs_handle h, cogs_stream stream, const voi
         }
         return COGS_OK;
     }
-    const bool need_all = pooled_mean || hidden_out;
     if (need_all) {
         void* hn = hidden_out ? hidden_out : ln;
         { PROF(COGS_PROF_NORM); COGS_TRY(cogs_k_rmsnorm(st, dt, x, hn, w.final_norm, S, H, w.rms_eps)); }

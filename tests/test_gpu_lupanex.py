@@ -450,6 +450,47 @@ def test_streams_that_wait_for_several_outputs(dev, streams, width, loop, dtype)
         assert rms_err(got[r], lg) < TOL[dtype]
 
 
+@pytest.mark.parametrize("past,n", [(0, 257), (0, 321), (90, 320), (3, 449)])
+@pytest.mark.parametrize("name", ["latent", "latent, nothing fed forward", "attention", "delta"])
+def test_rows_of_the_last_layer_that_nothing_reads(dev, name, past, n):
+    """decoder.hip: a prompt of one sequence goes on behind its last layer's keys, values and state with the query tiles from the first row
+    whose logits are asked for. Caches and states bit for bit those of a prompt that wants every row, logits those of its rows up to the
+    rounding of bfloat16 (other numbers of query tiles are taken by other forms of the attention), wherever the wanted rows lie"""
+    if name.startswith("latent"):
+        import pabalix_models as pm
+        from cogstream_amd.llm import DecoderEngine
+        layers = [pm.mixer(pm.A, heads=3), pm.mixer(pm.G, heads=4, kv_rank=56)]
+        if "nothing" in name:
+            layers[1] = dict(layers[1], ff=None)
+        cfg = pm.config(layers, width=136)
+        e = DecoderEngine(pm.state(cfg), pm.parse_config(cfg), dtype=torch.bfloat16, device="cuda:0")
+    else:
+        last = attention(heads=4, kv_heads=2, dim=64, vdim=32) if name == "attention" else delta(heads=2, kv_heads=1, dim=32, vdim=32)
+        cfg = config([delta(heads=2, kv_heads=1, dim=32, vdim=32), last], width=200, streams=4)
+        e = engine(cfg, state(cfg), torch.bfloat16)
+    toks = torch.tensor([(7 * i * i + 3 * i) % cfg["vocab"] for i in range(past + n + 1)])
+
+    def prompt(want):
+        c = e.new_cache(past + n + 1)
+        if past:
+            e.forward_batch(e.embed_tokens(toks[:past]), [past], [c], [])
+        got = e.forward_batch(e.embed_tokens(toks[past:past + n]), [n], [c], want)
+        return got, c.k.clone(), None if c.state is None else c.state.clone(), e.forward_batch(e.embed_tokens(toks[-1:]), [1], [c], [0])
+
+    every = prompt(list(range(n)))
+    for want in ([n - 1], [n - 66, n - 1], [n - 65, n - 2], [n - 1, 128], [127, n - 1], [129], []):
+        got, k, st, after = prompt(want)
+        at = 0
+        for w in e.packed.cache_widths:
+            size = w * (past + n + 1)
+            assert torch.equal(k[at:at + size].view(-1, w)[:past + n], every[1][at:at + size].view(-1, w)[:past + n]), want
+            at += size
+        assert st is None or torch.equal(st, every[2]), want
+        assert torch.equal(after, every[3]), want
+        if want:
+            assert rms_err(got, every[0][want].double().cpu()) < TOL[torch.bfloat16], want
+
+
 @pytest.mark.parametrize("dim,vdim", [(16, 16), (64, 48), (80, 16), (128, 128), (144, 32), (256, 16)])
 def test_chunked_delta_rule_at_the_edges_of_its_tiles(dev, dim, vdim):
     """every number of row tiles per wave, whole and ragged; chunks of one token, whole and ragged ones, one to four of them, from nothing

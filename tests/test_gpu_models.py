@@ -202,6 +202,31 @@ def test_copies_of_keys_and_values_are_no_product(dev, dtype, split, copies):
     assert counts[1][3] - counts[0][3] == copies, counts
 
 
+@pytest.mark.parametrize("kv", [True, False])
+@pytest.mark.parametrize("S", [257, 258, 384, 385, 386, 700, 1025, 1153, 1500])
+def test_rows_of_the_last_layer_that_no_logits_read(dev, S, kv):
+    """cogs_llm_forward: a prompt's last layer goes on behind its keys and values with the last row's query tile alone. Logits and cache bit
+    for bit those of the prompt brought in two parts of which the second is short enough for all its rows to go on; and without a cache"""
+    from cogstream_amd.llm import Qwen2Engine
+    from cogstream_amd.weights import LlmConfig, random_llm_state
+    cfg = LlmConfig(hidden_size=512, intermediate_size=768, num_hidden_layers=2, num_attention_heads=4, num_key_value_heads=2, vocab_size=640,
+                    image_token_index=600, eos_token_id=599)
+    eng = Qwen2Engine(random_llm_state(cfg, seed=4, std=0.05), cfg, dtype=torch.bfloat16)
+    emb = (torch.randn(S, 512, generator=torch.Generator().manual_seed(S)) * 0.5).bfloat16().to(dev)
+    ref = eng.new_cache(S)
+    eng.forward(emb[:S - 200], ref, want_logits=False)
+    want = eng.forward(emb[S - 200:], ref)["logits"]
+    if not kv:
+        assert torch.equal(eng.forward(emb)["logits"], want)
+        return
+    cache = eng.new_cache(S)
+    assert torch.equal(eng.forward(emb, cache)["logits"], want)
+    assert cache.len == S and torch.equal(cache.k, ref.k) and torch.equal(cache.v, ref.v)
+    some = eng.new_cache(S)
+    eng.forward(emb, some, want_logits=False)
+    assert torch.equal(some.k, ref.k) and torch.equal(some.v, ref.v)
+
+
 @pytest.mark.parametrize("dtype,tol", [(torch.float32, 1e-4), (torch.bfloat16, 3e-2)])
 def test_llm_prefill_and_decode_vs_oracle(dev, dtype, tol):
     from oracle import qwen2 as oq
