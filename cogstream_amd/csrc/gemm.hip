@@ -1144,9 +1144,11 @@ static int best_mid_tile(int M, int N, int K, bool alone, float* time, int rows0
         // them shares no weights, 129 / 144 / 160 rows against 128x128, us: 11 264 x 2048 20.3 / 20.5 / 21.3 against 19.9 / 19.3 / 19.5, 12 352 x 4096
         // 37.1 / 38.3 / 39.8 against 36.2 / 36.0 / 36.5, 16 384 x 2048 24.4 / 22.7 / 23.6 against 24.9 / 23.4 / 23.0. Beside
         // another stream, whose launch wants CUs too, its up to 256 workgroups of one to a CU leave none: 16 x 256 patches on two streams
-        // 5171 us with it, 4792 without; 5 x 924 5988 / 5604, 4 x 924 5283 / 4876, 8 x 924 7661 / 7663)
+        // 5171 us with it, 4792 without; 5 x 924 5988 / 5604, 4 x 924 5283 / 4876, 8 x 924 7661 / 7663. The four sizes behind it are no better there:
+        // 12 x 924 12 030 with them, 11 400 without, 3 x 1600 6790 / 6050, 16 x 924 14 430 / 13 800)
+        if (t.tile >= 7 && !alone) continue;
         if (t.tile == 8 && tiles > PERSISTENT_WGS - 8) continue;      // (its weights come too slowly with no CU to read them ahead: 768 x 2048 x 5632 32.2 us, 128x64 28.8)
-        if ((t.tile == 7 || t.tile == 9) && (!alone || M - rows0 <= t.tm || (t.tile == 7 && tiles > PERSISTENT_WGS))) continue;
+        if ((t.tile == 7 || t.tile == 9) && (M - rows0 <= t.tm || (t.tile == 7 && tiles > PERSISTENT_WGS))) continue;
         const float c = tile_time(tiles, K / 64, t);
         if (best == 0 || c < *time) { best = t.tile; *time = c; }
     }
@@ -1262,7 +1264,10 @@ static int gemm_rows(hipStream_t st, const CogsGemm& g, bool* kv_stored) {
             // streams. (Counting both streams' tiles as one launch picked larger tiles, which leave less for the other stream's
             // launch to run beside: 4 x 256 patches 3.09 against 2.58 ms, 16 x 256 5.46 / 4.92, 8 x 924 8.52 / 7.95.)
             const int slabs = g.K / 64;
-            const float ln = g.ln_part ? LN_FINALIZE : 0.f;
+            // (a folded norm's launch of its own is not counted against a mid-size launch of several rounds, whose longer epilogues -- rotation,
+            // head-major rows -- cost as much: 3072 x 3456 x 1152 of the encoder in two rounds of 192x128 46 us, here 35 and 5 in front)
+            const TileCost& m = MID_TILES[mid - 1];
+            const float ln = g.ln_part && (g.M + m.tm - 1) / m.tm * ((g.N + m.tn - 1) / m.tn) <= PERSISTENT_WGS ? LN_FINALIZE : 0.f;
             float best = tile_time(nb, slabs, PP_TILE) + ln;
             if (mid_time < best) { best = mid_time; mb_main = 0; }
             // row blocks x column blocks here (all columns: p.nbn, with the tall tiles), the L-shaped rest in one mid-size launch
