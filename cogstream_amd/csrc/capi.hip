@@ -282,20 +282,27 @@ cogs_status cogs_kmeans_margins(cogs_stream stream, int T, int64_t PD, int K, vo
 cogs_status cogs_kmeans_lloyd_dist(cogs_stream stream, int dtype, const void* feats, const float* ts, int T, int64_t PD, int K,
                                    float alpha, int max_iter, float tol, const int32_t* reseed_pool, int pool_len,
                                    float* centres, float* centre_ts, int64_t* assign, int* iterations, int* reseeds_used,
-                                   int* pool_exhausted, float* dist2, int known, void* ws, size_t ws_bytes) {
+                                   int* pool_exhausted, float* dist2, int known, const int32_t* watch, int32_t* watched,
+                                   float* min_margin, int32_t* rows_below, void* ws, size_t ws_bytes) {
     int ns = 0;
     const size_t need = cogs_k_kmeans_ws(T, PD, K, &ns);
     if (!ws || ws_bytes < need) return COGS_E_WORKSPACE;
     if (!feats || !ts || !centres || !centre_ts || !assign || (pool_len > 0 && !reseed_pool)) return COGS_E_INVALID;
-    return cogs_k_kmeans_lloyd((hipStream_t)stream, dtype, feats, ts, T, PD, K, alpha, max_iter, tol, reseed_pool, pool_len,
-                               centres, centre_ts, assign, iterations, reseeds_used, pool_exhausted, dist2, known, (float*)ws, ns);
+    CogsKmReport r;
+    const int rc = cogs_k_kmeans_lloyd((hipStream_t)stream, dtype, feats, ts, T, PD, K, alpha, max_iter, tol, reseed_pool, pool_len,
+                                       centres, centre_ts, assign, iterations, reseeds_used, pool_exhausted, dist2, known, watch, &r, (float*)ws, ns);
+    if (rc != COGS_OK) return rc;
+    if (watched) *watched = r.seen ? r.watched : -1;
+    if (min_margin) *min_margin = r.min_margin;
+    if (rows_below) *rows_below = r.rows_below;
+    return COGS_OK;
 }
 cogs_status cogs_kmeans_lloyd(cogs_stream stream, int dtype, const void* feats, const float* ts, int T, int64_t PD, int K,
                               float alpha, int max_iter, float tol, const int32_t* reseed_pool, int pool_len,
                               float* centres, float* centre_ts, int64_t* assign, int* iterations, int* reseeds_used,
                               int* pool_exhausted, void* ws, size_t ws_bytes) {
     return cogs_kmeans_lloyd_dist(stream, dtype, feats, ts, T, PD, K, alpha, max_iter, tol, reseed_pool, pool_len, centres, centre_ts,
-                                  assign, iterations, reseeds_used, pool_exhausted, nullptr, 0, ws, ws_bytes);
+                                  assign, iterations, reseeds_used, pool_exhausted, nullptr, 0, nullptr, nullptr, nullptr, nullptr, ws, ws_bytes);
 }
 cogs_status cogs_pack_rows(cogs_stream stream, int in_dtype, int out_dtype, const void* in, int64_t ld_in, void* out,
                            int64_t ld_out, int rows, int cols_in, int cols_out) {

@@ -140,9 +140,10 @@ int cogs_k_kmeans_pp_step(hipStream_t st, int dtype, const void* feats, int T, l
 int cogs_k_kmeans_pp(hipStream_t st, int dtype, const void* feats, int T, long PD, int K, int first_row, const float* q, int* idx,
                      int* zero_flag, float* nearest2, float* dist2, float* ws, int nslices);
 int cogs_k_kmeans_margins(hipStream_t st, int T, long PD, int K, float* ws, float* min_margin, int* rows_below);
+struct CogsKmReport { float min_margin; int rows_below, watched, seen; };      // as of the last iteration's read; seen: there was one
 int cogs_k_kmeans_lloyd(hipStream_t st, int dtype, const void* feats, const float* ts, int T, long PD, int K, float alpha,
                         int max_iter, float tol, const int* pool_host, int pool_len, float* centres, float* centre_ts,
-                        int64_t* assign, int* iterations, int* reseeds_used, int* exhausted, float* dist2, int known, float* ws, int nslices);
+                        int64_t* assign, int* iterations, int* reseeds_used, int* exhausted, float* dist2, int known, const int* watch, CogsKmReport* report, float* ws, int nslices);
 size_t cogs_k_kmeans_ws(int T, long PD, int K, int* nslices);
 int cogs_k_kmeans_assign(hipStream_t st, const float* dist2, const float* ts, const float* centre_ts, int T, int K,
                          float alpha, int64_t* assign, int* counts);

@@ -608,7 +608,7 @@ __global__ __launch_bounds__(UF_T) void update_final_kernel(const float* __restr
                                                            float* __restrict__ cts,
                                                            const float* __restrict__ shift_partial, int nblk,
                                                            float* __restrict__ scratch, float* __restrict__ shift_out,
-                                                           volatile int* __restrict__ status, int Tn_lds, float tol) {
+                                                           volatile int* __restrict__ status, int Tn_lds, float tol, const int* __restrict__ watch) {
     extern __shared__ __attribute__((aligned(16))) char smem_raw[];
     float* mts = reinterpret_cast<float*>(smem_raw);      // [Tn] time stamps in member order (0 floats when Tn_lds == 0)
     if (ctl && ctl[CTL_DONE]) return;                     // a speculatively queued iteration behind the converged one
@@ -654,6 +654,7 @@ __global__ __launch_bounds__(UF_T) void update_final_kernel(const float* __restr
         if (status) {      // host-mapped copy of the control words (one read per batch of iterations)
 #pragma unroll
             for (int i = 0; i < CTL_WORDS; ++i) status[i] = ctl ? ctl[i] : 0;
+            status[CTL_WORDS] = watch ? *watch : 0;
             __threadfence_system();
         }
     }
@@ -841,7 +842,7 @@ int launch_members(hipStream_t st, const int64_t* assign, int T, int K, const Km
     return COGS_LAUNCH_CHECK();
 }
 int launch_update(hipStream_t st, int dtype, const void* feats, const float* ts, int T, long PD, int K, const KmWs& w,
-                  int* ctl, float* centres, float* centre_ts, float* shift_out, volatile int* status, float tol = -1.f) {
+                  int* ctl, float* centres, float* centre_ts, float* shift_out, volatile int* status, float tol = -1.f, const int* watch = nullptr) {
     const int nblk = cogs_k_kmeans_update_blocks(PD);
     if (dtype == COGS_DT_BF16)
         hipLaunchKernelGGL(update_kernel<bf16_t>, dim3(nblk, K), dim3(256), 0, st, (const bf16_t*)feats, PD, K, w.offs, w.members,
@@ -851,7 +852,7 @@ int launch_update(hipStream_t st, int dtype, const void* feats, const float* ts,
                            w.reseed, ctl, centres, w.partial, ctl ? w.keep : nullptr);
     const int t_lds = T <= MEMB_T ? T : 0;       // member-ordered time stamps staged in LDS (64 KiB at most)
     hipLaunchKernelGGL(update_final_kernel, dim3(1), dim3(UF_T), (size_t)t_lds * 4, st, ts, K, w.offs, w.members, w.reseed, ctl,
-                       centre_ts, w.partial, nblk, w.scratch, shift_out, status, t_lds, tol);
+                       centre_ts, w.partial, nblk, w.scratch, shift_out, status, t_lds, tol, watch);
     return COGS_LAUNCH_CHECK();
 }
 }  // namespace
@@ -991,7 +992,7 @@ bool status_block(StatusBlock& b) {
 
 int cogs_k_kmeans_lloyd(hipStream_t st, int dtype, const void* feats, const float* ts, int T, long PD, int K, float alpha,
                         int max_iter, float tol, const int* pool_host, int pool_len, float* centres, float* centre_ts,
-                        int64_t* assign, int* iterations, int* reseeds_used, int* exhausted, float* dist2, int known, float* ws, int nslices) {
+                        int64_t* assign, int* iterations, int* reseeds_used, int* exhausted, float* dist2, int known, const int* watch, CogsKmReport* report, float* ws, int nslices) {
     if (T <= 0 || K <= 0 || PD % 8 || known < 0 || known > K || (known > 0 && !dist2) || max_iter < 0 || pool_len < 0 || pool_len > POOL_MAX) return COGS_E_INVALID;
     if (T > MEMB_T || (size_t)(T + K + 1) * 4 > 64 * 1024 || K > 4096) return COGS_E_UNSUPPORTED;   // T + K + 1 <= 16 384
     static thread_local StatusBlock sb;
@@ -999,6 +1000,7 @@ int cogs_k_kmeans_lloyd(hipStream_t st, int dtype, const void* feats, const floa
     if (iterations) *iterations = 0;
     if (reseeds_used) *reseeds_used = 0;
     if (exhausted) *exhausted = 0;
+    if (report) *report = CogsKmReport{INFINITY, 0, 0, 0};
     if (max_iter == 0) return COGS_OK;             // nothing to do
     const KmWs w = carve(ws, T, PD, K);
     if (hipMemsetAsync(w.ctl, 0, CTL_WORDS * sizeof(int), st) != hipSuccess) return COGS_E_HIP;     // margin word 0 = +inf
@@ -1007,7 +1009,7 @@ int cogs_k_kmeans_lloyd(hipStream_t st, int dtype, const void* feats, const floa
     if (known > 0 && hipMemsetAsync(w.keep, 1, (size_t)known * sizeof(int), st) != hipSuccess) return COGS_E_HIP;      // (anything but zero)
     int* pool_d = sb.d + 16;
     for (int i = 0; i < pool_len; ++i) sb.h[16 + i] = pool_host[i];        // plain host stores into the mapped block
-    for (int i = 0; i < CTL_WORDS; ++i) sb.h[i] = 0;
+    for (int i = 0; i <= CTL_WORDS; ++i) sb.h[i] = 0;
     int queued = 0, it = 0, used = 0, ex = 0;
     int rc = COGS_OK;
     while (queued < max_iter) {
@@ -1017,7 +1019,7 @@ int cogs_k_kmeans_lloyd(hipStream_t st, int dtype, const void* feats, const floa
             if (rc == COGS_OK) rc = launch_reduce_assign(st, w.partial, nslices, T, K, ts, centre_ts, alpha, dist2, assign, w.ctl, w.keep);
             if (rc == COGS_OK) rc = launch_members(st, assign, T, K, w, pool_d, pool_len, nullptr, w.ctl);
             if (rc == COGS_OK) rc = launch_update(st, dtype, feats, ts, T, PD, K, w, w.ctl, centres, centre_ts, (float*)(w.ctl + CTL_SHIFT),
-                                                  (volatile int*)sb.d, tol);
+                                                  (volatile int*)sb.d, tol, watch);
         }
         queued += batch;
         if (hipStreamSynchronize(st) != hipSuccess) return COGS_E_HIP;
@@ -1030,6 +1032,7 @@ int cogs_k_kmeans_lloyd(hipStream_t st, int dtype, const void* feats, const floa
     if (iterations) *iterations = it;
     if (reseeds_used) *reseeds_used = used;
     if (exhausted) *exhausted = ex;
+    if (report) *report = CogsKmReport{__builtin_bit_cast(float, 0x7f800000 - sb.h[CTL_MARGIN]), sb.h[CTL_NEAR], sb.h[CTL_WORDS], 1};
     return COGS_OK;
 }
 

@@ -24,7 +24,7 @@ would flip its cluster (cogs_kmeans_margins; (d2 - d1) / mean(d1, d2) of the two
 equal); rows_below_1e-3 = (row, iteration) pairs under 1e-3, where the reference's own cdist rounding decides a row."""
 
 
-def _lloyd_from_rows(x, ts, rows, K: int, PD: int, alpha: float, max_iteration: int, tol: float, ws, dist2=None):
+def _lloyd_from_rows(x, ts, rows, K: int, PD: int, alpha: float, max_iteration: int, tol: float, ws, dist2=None, watch=None, report=None):
     """Lloyd iterations (:71-131) from the centres x[rows], inside the library. Empty clusters are reseeded with
     random.randint(0, T-1) per cluster in ascending order (:116-120): the values are drawn AHEAD into a pool the device
     consumes in that order, and the generator is then put back to where the reference would have left it (state
@@ -40,7 +40,7 @@ def _lloyd_from_rows(x, ts, rows, K: int, PD: int, alpha: float, max_iteration: 
     while left > 0:
         drawn.extend(random.randint(0, T - 1) for _ in range(pool_n))
         it, used, exhausted = ops.kmeans_lloyd(x, ts, centres, centre_ts, assign, float(alpha), left, float(tol),
-                                               drawn[used_total:], ws, dist2, known)
+                                               drawn[used_total:], ws, dist2, known, watch, report)
         known = 0
         done, left, used_total = done + it, left - it, used_total + used
         if not exhausted:
@@ -85,8 +85,11 @@ def kmeans_with_time_min_max(features: torch.Tensor, timestamp, cluster_num: int
     idx_d, flag = ops.kmeans_pp(x, first, K, q.to(dev, non_blocking=True), ws, dist2)
     # (no host read here: the Lloyd loop below starts from the device-resident rows; the flag is looked at after its
     # first synchronisation, and in the rare flagged case everything is redone step by step)
-    run = _lloyd_from_rows(x, ts, idx_d.to(torch.int64), K, PD, alpha, max_iteration, tol, ws, dist2)
-    if int(flag.item()) == 0:
+    report: dict = {}
+    run = _lloyd_from_rows(x, ts, idx_d.to(torch.int64), K, PD, alpha, max_iteration, tol, ws, dist2, flag, report)
+    if report.get("watched", -1) < 0:          # no iteration was run
+        report["watched"] = int(flag.item())
+    if report["watched"] == 0:
         last_stats["kpp_path"] = "one call"
     else:
         random.setstate(py_state)
@@ -104,10 +107,10 @@ def kmeans_with_time_min_max(features: torch.Tensor, timestamp, cluster_num: int
                 new = int(torch.multinomial(probs / s, 1).item())        # CPU generator, like the reference
             idx.append(new)
         last_stats["kpp_path"] = "step by step (a zero-probability step)"
-        run = _lloyd_from_rows(x, ts, torch.tensor(idx, dtype=torch.int64, device=dev), K, PD, alpha, max_iteration, tol, ws)
+        run = _lloyd_from_rows(x, ts, torch.tensor(idx, dtype=torch.int64, device=dev), K, PD, alpha, max_iteration, tol, ws, report=report)
     centres, centre_ts, assign, done = run
     last_stats["kpp_passes"], last_stats["iterations"] = K - 1, done
-    last_stats["min_rel_margin"], last_stats["rows_below_1e-3"] = ops.kmeans_margins(T, PD, K, ws)
+    last_stats["min_rel_margin"], last_stats["rows_below_1e-3"] = report.get("margins", (float("inf"), 0))
     return centres.view(K, P, D), centre_ts, assign
 
 

@@ -287,18 +287,22 @@ def kmeans_margins(T: int, PD: int, K: int, ws):
 
 
 def kmeans_lloyd(feats, ts, centres, centre_ts, assign, alpha: float, max_iter: int, tol: float, pool, ws,
-                 dist2: Optional[torch.Tensor] = None, known: int = 0):
+                 dist2: Optional[torch.Tensor] = None, known: int = 0, watch: Optional[torch.Tensor] = None, report: Optional[dict] = None):
     """cogs_kmeans_lloyd -> (iterations completed, reseeds used, pool exhausted). pool: python list of pre-drawn rows. dist2 (fp32
-    [T, K], overwritten): its first `known` columns are the squared distances to the first `known` centres as given"""
+    [T, K], overwritten): its first `known` columns are the squared distances to the first `known` centres as given. report receives
+    "margins" (as kmeans_margins) and, of the int32 [1] tensor `watch`, "watched": its value behind the last iteration, -1 if there was none"""
     T, PD = feats.shape
     K = centres.shape[0]
     assert dist2 is None or (dist2.is_cuda and dist2.dtype == torch.float32 and dist2.shape == (T, K) and dist2.is_contiguous())
     arr = (C.c_int32 * max(len(pool), 1))(*pool)
     it, used, ex = C.c_int(0), C.c_int(0), C.c_int(0)
+    margin, near, seen = C.c_float(0), C.c_int32(0), C.c_int32(0)
     check(L.lib.cogs_kmeans_lloyd_dist(current_stream(), dtype_code(feats.dtype), ptr(feats), ptr(ts), T, PD, K, float(alpha),
                                   int(max_iter), float(tol), C.cast(arr, C.c_void_p), len(pool), ptr(centres), ptr(centre_ts),
-                                  ptr(assign), C.byref(it), C.byref(used), C.byref(ex), ptr(dist2), int(known), ptr(ws), ws.numel()),
-          "cogs_kmeans_lloyd")
+                                  ptr(assign), C.byref(it), C.byref(used), C.byref(ex), ptr(dist2), int(known), ptr(watch), C.byref(seen),
+                                  C.byref(margin), C.byref(near), ptr(ws), ws.numel()), "cogs_kmeans_lloyd")
+    if report is not None:
+        report["margins"], report["watched"] = (float(margin.value), int(near.value)), int(seen.value)
     return it.value, used.value, bool(ex.value)
 
 

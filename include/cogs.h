@@ -268,11 +268,14 @@ cogs_status cogs_kmeans_lloyd(cogs_stream stream, int dtype, const void* feats, 
                               float* centres, float* centre_ts, int64_t* assign, int* iterations, int* reseeds_used,
                               int* pool_exhausted, void* ws, size_t ws_bytes);
 /* The same; dist2 (nullable unless known > 0, device fp32 [T][K], overwritten): its first `known` columns hold the squared distances
- * to the first `known` centres as they come in, which are then not summed again. */
+ * to the first `known` centres as they come in, which are then not summed again. watch (nullable): a device word whose value behind the
+ * last iteration the call hands back in *watched (-1 if it ran none) -- cogs_kmeans_pp's zero_flag, without a read of its own;
+ * min_margin, rows_below (nullable): what cogs_kmeans_margins would say. */
 cogs_status cogs_kmeans_lloyd_dist(cogs_stream stream, int dtype, const void* feats, const float* ts, int T, int64_t PD, int K,
                                    float alpha, int max_iter, float tol, const int32_t* reseed_pool, int pool_len,
                                    float* centres, float* centre_ts, int64_t* assign, int* iterations, int* reseeds_used,
-                                   int* pool_exhausted, float* dist2, int known, void* ws, size_t ws_bytes);
+                                   int* pool_exhausted, float* dist2, int known, const int32_t* watch, int32_t* watched,
+                                   float* min_margin, int32_t* rows_below, void* ws, size_t ws_bytes);
 /* How close the assignments of the LAST cogs_kmeans_lloyd call on this workspace were (host outputs; synchronises).
  * Per row and iteration: the relative change of the row's feature distances that would flip the decision between its
  * best and second-best cluster -- with every time term equal this is (d2 - d1) / mean(d1, d2) of the two nearest feature
