@@ -126,12 +126,7 @@ __device__ __forceinline__ float lane_xor_dpp(float v) {
 // some order, and the operation is commutative), xor 8..1 through DPP (above). Same values, bit for bit, as the
 // __shfl_xor butterfly they replace.
 template <typename F>
-__device__ __forceinline__ float wave_butterfly(float v, F op) {
-    {
-        const unsigned b = __builtin_bit_cast(unsigned, v);
-        const auto r = __builtin_amdgcn_permlane32_swap(b, b, false, false);
-        v = op(__builtin_bit_cast(float, (unsigned)r[0]), __builtin_bit_cast(float, (unsigned)r[1]));
-    }
+__device__ __forceinline__ float half_wave_butterfly(float v, F op) {
     {
         const unsigned b = __builtin_bit_cast(unsigned, v);
         const auto r = __builtin_amdgcn_permlane16_swap(b, b, false, false);
@@ -142,6 +137,15 @@ __device__ __forceinline__ float wave_butterfly(float v, F op) {
     v = op(v, lane_xor_dpp<2>(v));
     v = op(v, lane_xor_dpp<1>(v));
     return v;
+}
+template <typename F>
+__device__ __forceinline__ float wave_butterfly(float v, F op) {
+    const unsigned b = __builtin_bit_cast(unsigned, v);
+    const auto r = __builtin_amdgcn_permlane32_swap(b, b, false, false);
+    return half_wave_butterfly(op(__builtin_bit_cast(float, (unsigned)r[0]), __builtin_bit_cast(float, (unsigned)r[1])), op);
+}
+__device__ __forceinline__ float half_wave_sum(float v) {      // of lanes 0 .. 31 in each of them, of 32 .. 63 in theirs
+    return half_wave_butterfly(v, [](float a, float b) { return a + b; });
 }
 __device__ __forceinline__ float wave_sum(float v) {
     return wave_butterfly(v, [](float a, float b) { return a + b; });

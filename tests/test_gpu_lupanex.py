@@ -491,6 +491,17 @@ def test_rows_of_the_last_layer_that_nothing_reads(dev, name, past, n):
             assert rms_err(got, every[0][want].double().cpu()) < TOL[torch.bfloat16], want
 
 
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("heads,vdim", [(1, 16), (2, 128), (3, 96), (7, 112), (17, 32), (33, 128), (9, 144)])
+def test_read_outs_of_one_head_or_two_a_wave(dev, heads, vdim, dtype):
+    """delta.hip, delta_out_kernel: fewer heads than a workgroup takes at a time, more, numbers that it does not divide, and heads wider than
+    half a wave's columns, against the oracle"""
+    cfg = config([delta(heads=heads, kv_heads=1, dim=16, vdim=vdim, ff=None)], width=192, streams=2)
+    st = state(cfg)
+    toks = tokens(cfg, 70)
+    assert rms_err(run(engine(cfg, st, dtype), toks), lo.forward(cfg, double(st), toks)[0]) < TOL[dtype]
+
+
 @pytest.mark.parametrize("dim,vdim", [(16, 16), (64, 48), (80, 16), (128, 128), (144, 32), (256, 16)])
 def test_chunked_delta_rule_at_the_edges_of_its_tiles(dev, dim, vdim):
     """every number of row tiles per wave, whole and ragged; chunks of one token, whole and ragged ones, one to four of them, from nothing
