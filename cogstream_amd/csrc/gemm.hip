@@ -1111,7 +1111,7 @@ void dispatch_f32(hipStream_t st, const GemmArgs& p, int grid, int mask, bool bi
 //     mid-size launch (strip of columns, ragged rows, or both). 4096 x 6176 x 2048 108 -> 60 + 41, 768 x 22 016 x 4096 148 -> 115. A strip
 //     of columns reads every weight once; rows that are left read all of them again, and where they are more than half of the 256 MB
 //     Infinity Cache they push the output out of it: 621 x 37 888 x 3584 (two row blocks and 109 rows) gained 5 us and the 18 944-wide
-//     product behind it lost 25; as a strip (three row blocks x 85 column blocks, 160x256) 163 -> 152 and 113 -> 108, 1000 rows 231 -> 202.
+//     product behind it lost 25 (of more rows than it holds nothing stays there anyway); as a strip (three row blocks x 85 column blocks, 160x256) 163 -> 152 and 113 -> 108, 1000 rows 231 -> 202.
 struct TileCost { int tile, tm, tn; float one, two, rest, full; };     // us; two = 0: one workgroup per CU; full: a slab's surcharge on a full chip
 static constexpr TileCost MID_TILES[] = {
     {1, 32, 64, 0.174f, 0.f, 0.9f, 0.14f},     {2, 64, 64, 0.213f, 0.381f, 2.2f, 0.08f}, {3, 128, 64, 0.311f, 0.569f, 2.1f, 0.14f},
@@ -1273,7 +1273,7 @@ static int gemm_rows(hipStream_t st, const CogsGemm& g, bool* kv_stored) {
             // row blocks x column blocks here (all columns: p.nbn, with the tall tiles), the L-shaped rest in one mid-size launch
             auto consider = [&](int mb, int cb) {
                 const int rows = min(mb * BM3, g.M), cols = cb >= p.nbn ? g.N : cb * BN3;
-                if (mb <= 0 || cb <= 0 || (rows == g.M && cols == g.N) || (rows < g.M && 2.f * g.K * g.N > REST_AGAIN)) return;
+                if (mb <= 0 || cb <= 0 || (rows == g.M && cols == g.N) || (rows < g.M && 2.f * g.K * g.N > REST_AGAIN && 2.f * g.M * ((float)g.K + g.N) < 2 * REST_AGAIN)) return;
                 float rest;
                 const int tile = best_mid_tile(g.M, g.N, g.K, S == 1, &rest, rows, cols);
                 rest = max(rest, 2.f * g.K * (rows < g.M ? g.N : g.N - cols) / REST_READ);
