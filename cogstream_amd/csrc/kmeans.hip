@@ -660,6 +660,14 @@ __global__ __launch_bounds__(UF_T) void update_final_kernel(const float* __restr
     }
 }
 
+// what a loop starts from: n words of zeros at a and one at b (nullable), ones and zeros at keep. One launch: a memset of a few words is one or two of
+// 3.4 us each (256 frames of 50 tokens: eleven of them 37 us)
+__global__ __launch_bounds__(256) void start_kernel(int* a, int n, int* b, int* keep, int K, int known) {
+    for (int i = threadIdx.x; i < n; i += 256) a[i] = 0;
+    if (b && threadIdx.x == 0) *b = 0;
+    for (int k = threadIdx.x; k < K; k += 256) keep[k] = k < known;
+}
+
 // one thread per row t from dist2 (the step-wise API, cogs_kmeans_assign); counts must be zero on entry
 __global__ __launch_bounds__(256) void assign_kernel(const float* __restrict__ dist2, const float* __restrict__ ts,
                                                      const float* __restrict__ cts, int Tn, int K, float alpha,
@@ -933,8 +941,7 @@ int cogs_k_kmeans_pp(hipStream_t st, int dtype, const void* feats, int T, long P
     const KmWs w = carve(ws, T, PD, 1);
     if (nslices != (int)((PD + SL - 1) / SL)) return COGS_E_WORKSPACE;
     const bool one = kpp_in_one_launch(dtype, T, PD);
-    if (hipMemsetAsync(zero_flag, 0, sizeof(int), st) != hipSuccess) return COGS_E_HIP;
-    if (one && hipMemsetAsync(w.ctl, 0, sizeof(int), st) != hipSuccess) return COGS_E_HIP;      // the counter of finished rows
+    hipLaunchKernelGGL(start_kernel, dim3(1), dim3(256), 0, st, w.ctl, one ? 1 : 0, zero_flag, nullptr, 0, 0);      // w.ctl: the counter of finished rows
     g_cogs_debug.km_pp_last_launches = one ? 1 : 3;
     const size_t lds = (size_t)nslices * 4;
     for (int m = 1; m < K; ++m) {
@@ -1003,10 +1010,8 @@ int cogs_k_kmeans_lloyd(hipStream_t st, int dtype, const void* feats, const floa
     if (report) *report = CogsKmReport{INFINITY, 0, 0, 0};
     if (max_iter == 0) return COGS_OK;             // nothing to do
     const KmWs w = carve(ws, T, PD, K);
-    if (hipMemsetAsync(w.ctl, 0, CTL_WORDS * sizeof(int), st) != hipSuccess) return COGS_E_HIP;     // margin word 0 = +inf
     if (!dist2) dist2 = w.dist2;
-    if (hipMemsetAsync(w.keep, 0, (size_t)K * sizeof(int), st) != hipSuccess) return COGS_E_HIP;
-    if (known > 0 && hipMemsetAsync(w.keep, 1, (size_t)known * sizeof(int), st) != hipSuccess) return COGS_E_HIP;      // (anything but zero)
+    hipLaunchKernelGGL(start_kernel, dim3(1), dim3(256), 0, st, w.ctl, (int)CTL_WORDS, nullptr, w.keep, K, known);        // margin word 0 = +inf
     int* pool_d = sb.d + 16;
     for (int i = 0; i < pool_len; ++i) sb.h[16 + i] = pool_host[i];        // plain host stores into the mapped block
     for (int i = 0; i <= CTL_WORDS; ++i) sb.h[i] = 0;
