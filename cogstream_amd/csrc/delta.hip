@@ -548,15 +548,17 @@ __global__ __launch_bounds__(256, NK > 2 ? 1 : 2) void delta_scan_kernel(CogsDel
     }
 }
 
-// read-outs -> the output product's operand: RMS norm over the head, weight, silu of the gate; half a wave or a wave per head
-template <typename T>
+// read-outs -> the output product's operand: RMS norm over the head, weight, silu of the gate; half a wave (HALF) or a wave per head. The squares
+// are written as fused operations, one after the other: left to the compiler, an unrolled sum rounds its second square by itself and
+// fuses the first one into it, and the two forms' bits differ
+template <typename T, bool HALF>
 __global__ __launch_bounds__(256) void delta_out_kernel(CogsDelta p) {
     const int row = blockIdx.x, lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
     const long nv = (long)p.heads * p.dvp;
     const float* gate = p.t + (long)row * p.ldt + 2L * p.kv_heads * p.dkp + nv;
     // heads of up to 128 columns: half a wave has one in its registers, all of its loads out together, two heads of each half at a time (a wave a
-    // head left half the lanes idle and read the row twice: 4096 rows of 16 heads of 128 27.5 us, 17.0; 84 MB. The sums in the same order)
-    if (p.dvp <= 128) {
+    // head left half the lanes idle and read the row twice: 4096 rows of 16 heads of 128 27.5 us, 17.0; 84 MB)
+    if constexpr (HALF) {
         constexpr int U = 2;
         const int d = min((lane & 31) * 4, p.dvp - 4);
         const bool in = (lane & 31) * 4 < p.dvp;
@@ -575,7 +577,7 @@ __global__ __launch_bounds__(256) void delta_out_kernel(CogsDelta p) {
                 float ss = 0.f;
                 if (in)
 #pragma unroll
-                    for (int e = 0; e < 4; ++e) ss += v[u][e] * v[u][e];
+                    for (int e = 0; e < 4; ++e) ss = fmaf(v[u][e], v[u][e], ss);
                 const float f = 1.f / sqrtf(half_wave_sum(ss) / (float)p.vdim + p.eps);
                 f32x4 r;
 #pragma unroll
@@ -591,7 +593,7 @@ __global__ __launch_bounds__(256) void delta_out_kernel(CogsDelta p) {
         for (int d = lane * 4; d < p.dvp; d += 256) {
             const f32x4 v = *reinterpret_cast<const f32x4*>(o + d);
 #pragma unroll
-            for (int e = 0; e < 4; ++e) ss += v[e] * v[e];
+            for (int e = 0; e < 4; ++e) ss = fmaf(v[e], v[e], ss);
         }
         const float f = 1.f / sqrtf(wave_sum(ss) / (float)p.vdim + p.eps);
         T* y = reinterpret_cast<T*>(p.att) + (long)row * p.ldo + (long)h * p.dvp;
@@ -862,8 +864,14 @@ int cogs_k_delta_prompt(hipStream_t st, int dtype, const CogsDelta& a, int rows,
     } else {
         hipLaunchKernelGGL(delta_recur_kernel, dim3((a.dvp + 63) / 64, a.heads, nseq), dim3(64), 0, st, a);
     }
-    if (dtype == COGS_DT_BF16) hipLaunchKernelGGL(delta_out_kernel<bf16_t>, dim3(rows), dim3(256), 0, st, a);
-    else hipLaunchKernelGGL(delta_out_kernel<float>, dim3(rows), dim3(256), 0, st, a);
+    const bool half = a.dvp <= 128 && g_cogs_debug.delta_out_wave == 0;
+    if (dtype == COGS_DT_BF16) {
+        if (half) hipLaunchKernelGGL((delta_out_kernel<bf16_t, true>), dim3(rows), dim3(256), 0, st, a);
+        else hipLaunchKernelGGL((delta_out_kernel<bf16_t, false>), dim3(rows), dim3(256), 0, st, a);
+    } else {
+        if (half) hipLaunchKernelGGL((delta_out_kernel<float, true>), dim3(rows), dim3(256), 0, st, a);
+        else hipLaunchKernelGGL((delta_out_kernel<float, false>), dim3(rows), dim3(256), 0, st, a);
+    }
     return COGS_LAUNCH_CHECK();
 }
 

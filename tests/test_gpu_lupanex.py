@@ -495,11 +495,19 @@ def test_rows_of_the_last_layer_that_nothing_reads(dev, name, past, n):
 @pytest.mark.parametrize("heads,vdim", [(1, 16), (2, 128), (3, 96), (7, 112), (17, 32), (33, 128), (9, 144)])
 def test_read_outs_of_one_head_or_two_a_wave(dev, heads, vdim, dtype):
     """delta.hip, delta_out_kernel: fewer heads than a workgroup takes at a time, more, numbers that it does not divide, and heads wider than
-    half a wave's columns, against the oracle"""
+    half a wave's columns, against the oracle; and, over more rows, the bits of a wave per head"""
+    from cogstream_amd import _lib as L
     cfg = config([delta(heads=heads, kv_heads=1, dim=16, vdim=vdim, ff=None)], width=192, streams=2)
     st = state(cfg)
     toks = tokens(cfg, 70)
-    assert rms_err(run(engine(cfg, st, dtype), toks), lo.forward(cfg, double(st), toks)[0]) < TOL[dtype]
+    e = engine(cfg, st, dtype)
+    assert rms_err(run(e, toks), lo.forward(cfg, double(st), toks)[0]) < TOL[dtype]
+    embeds = e.embed_tokens(torch.tensor(tokens(cfg, 500)))
+    logits = []
+    for wave in (0, 1):
+        with L.debug_switch("delta_out_wave", wave):
+            logits.append(e.forward_batch(embeds, [500], [e.new_cache(500)], list(range(500))))
+    assert torch.equal(*logits)
 
 
 @pytest.mark.parametrize("dim,vdim", [(16, 16), (64, 48), (80, 16), (128, 128), (144, 32), (256, 16)])
