@@ -381,6 +381,7 @@ struct Step {
         if (chain) {
             CogsStreamChain a = waiting;
             a.out = k.hn; a.out_gamma = d.w.final_norm; a.pick = k.want; a.rows = n_want;
+            a.ahead = ahead(d.w.head, n_want, d.vocabp);
             return cogs_k_stream_chain(st, d.w.dtype, a);
         }
         CogsStreamNorm a;

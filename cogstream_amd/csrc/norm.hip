@@ -459,10 +459,16 @@ __global__ __launch_bounds__(TPB) void stream_mix_kernel(CogsStreamNorm p) {
 // 16-bit row for all streams, and the last ones are mixed for the rows that are asked for alone. 4096 rows of 4 x 2048, us (stream_mix_kernel
 // 66 each): 26, 27, 36, 53 from the embeddings, then 38, 37, 42, 61 in turn; 1109 -> 634 in a prompt of 16 sublayers. (A number of streams that is
 // not the template's made it 760, predicates and scalar loads one by one; rows walked by fewer workgroups 907. Longer chains cost what they save:
-// 20 multiplications an element and output.)
-template <typename T, int C, int NS>
-__global__ __launch_bounds__(256) void stream_chain_kernel(CogsStreamChain p) {
-    constexpr int TPB = 256;
+// 20 multiplications an element and output.) Up to 64 wanted rows of more than 1024 columns are latency: 1024 threads each as in stream_mix_kernel, so
+// that a row's sum is that of a row mixed at once, and beside them the head's weights are read ahead.
+template <typename T, int C, int NS, int TPB>
+__global__ __launch_bounds__(TPB) void stream_chain_kernel(CogsStreamChain p) {
+    if constexpr (TPB == 1024) {
+        if ((int)blockIdx.x >= p.rows) {
+            read_ahead(p.ahead, p.rows);
+            return;
+        }
+    }
     typedef T raw_t __attribute__((ext_vector_type(4)));
     __shared__ float red[TPB / 64];
     const int tid = threadIdx.x;
@@ -544,8 +550,15 @@ __global__ __launch_bounds__(256) void stream_chain_kernel(CogsStreamChain p) {
 
 template <typename T>
 int launch_stream_chain(hipStream_t st, const CogsStreamChain& a) {
-#define COGS_CHAIN_CASE(C, NS) hipLaunchKernelGGL((stream_chain_kernel<T, C, NS>), dim3(a.rows), dim3(256), 0, st, a)
-#define COGS_CHAIN_STREAMS(NS) case NS: if (a.Hp <= 2048) COGS_CHAIN_CASE(2, NS); else COGS_CHAIN_CASE(4, NS); break;
+    const bool few = a.rows <= 64 && a.Hp > 1024;
+    const int more = few ? ahead_workgroups(a.ahead, a.rows) : 0;
+#define COGS_CHAIN_CASE(C, NS, TPB) hipLaunchKernelGGL((stream_chain_kernel<T, C, NS, TPB>), dim3(a.rows + more), dim3(TPB), 0, st, a)
+#define COGS_CHAIN_STREAMS(NS)                      \
+    case NS:                                        \
+        if (few) COGS_CHAIN_CASE(1, NS, 1024);      \
+        else if (a.Hp <= 2048) COGS_CHAIN_CASE(2, NS, 256); \
+        else COGS_CHAIN_CASE(4, NS, 256);           \
+        break;
     switch (a.streams) {
         COGS_CHAIN_STREAMS(2)
         COGS_CHAIN_STREAMS(3)
@@ -624,7 +637,7 @@ int cogs_k_stream_norm(hipStream_t st, int dtype, const CogsStreamNorm& a) {
     return dtype == COGS_DT_BF16 ? launch_stream_norm<bf16_t>(st, a) : launch_stream_norm<float>(st, a);
 }
 
-// more than 64 rows: fewer are latency (their own kernel, which reads weights ahead). The row is in the registers of 256 threads: up to 4096 columns
+// more than 64 rows: fewer are latency (their own kernel, which reads weights ahead). The row is in the registers of 256 or 1024 threads: up to 4096 columns
 bool cogs_k_stream_chain_fits(int streams, int Hp, int rows) { return streams >= 2 && streams <= 4 && Hp <= 4096 && rows > 64; }
 
 int cogs_k_stream_chain(hipStream_t st, int dtype, const CogsStreamChain& a) {

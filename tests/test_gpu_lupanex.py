@@ -429,7 +429,8 @@ def test_weights_read_beside_a_mix_of_streams(dev, rows, width, ff, vocab):
 def test_streams_that_wait_for_several_outputs(dev, streams, width, loop, dtype):
     """norm.hip: prompts of more than 64 rows mix the streams of up to four sublayers together and the last ones for the wanted rows
     alone. The bits are those of mixes done at once (asked for by wanting every layer's streams): two to four streams, rows of one to three
-    chunks of 1024 columns, chains that end anywhere (3 to 8 outputs), wanted rows anywhere, two sequences, against the oracle too"""
+    chunks of 1024 columns, chains that end anywhere (3 to 8 outputs), wanted rows anywhere, as few as a row has 1024 threads for and more,
+    two sequences, against the oracle too"""
     kw = dict(width=width, streams=streams, ff=128)
     if loop:
         kw["loop"] = loop
@@ -437,14 +438,14 @@ def test_streams_that_wait_for_several_outputs(dev, streams, width, loop, dtype)
     st = state(cfg)
     e = engine(cfg, st, dtype)
     toks = tokens(cfg, 131)
-    lens, want = [66, 65], [0, 64, 65, 66, 130]
+    lens = [66, 65]
     embeds = e.embed_tokens(torch.tensor(toks))
     runs = len(e.cfg.layers) if not loop else len(e.cfg.layers) + (loop[1] - loop[0]) * (loop[2] - 1)
     each = torch.empty(runs, 131, e.packed.width_p, device=dev)
-    at_once = e.forward_batch(embeds, lens, [e.new_cache(n) for n in lens], want, streams=each)
-    caches = [e.new_cache(n) for n in lens]
-    got = e.forward_batch(embeds, lens, caches, want)
-    assert torch.equal(got, at_once)
+    for want in (list(range(131)), list(range(65)), list(range(20, 84)), list(range(67, 131)), [0, 64, 65, 66, 130]):
+        at_once = e.forward_batch(embeds, lens, [e.new_cache(n) for n in lens], want, streams=each)
+        got = e.forward_batch(embeds, lens, [e.new_cache(n) for n in lens], want)
+        assert torch.equal(got, at_once), len(want)
     assert e.forward_batch(embeds[:65], [65], [e.new_cache(65)], []) is None
     for r, lg in ((slice(0, 3), lo.forward(cfg, double(st), toks[:66])[0][[0, 64, 65]]), (slice(3, 5), lo.forward(cfg, double(st), toks[66:])[0][[0, 64]])):
         assert rms_err(got[r], lg) < TOL[dtype]
