@@ -245,7 +245,7 @@ struct Step {
             a.Q = k.q; a.ldq = qcols; a.q_head = G.dq; a.q_rot = G.dk; a.K = k.kvx; a.ldk = G.kvcols; a.k_head = G.dn;
             a.KR = at(ctx, G.kvp); a.ldkr = G.kvw; a.V = at(k.kvx, (size_t)m.heads * G.dn); a.ldv = G.kvcols; a.v_head = G.dv;
             a.O = k.att; a.ldo = G.oin; a.o_head = G.dv; a.dn = G.dn; a.dr = G.dr; a.dv = G.dv; a.heads = m.heads;
-            a.sink = m.sink; a.gate = gate; a.seqs = tail; a.nseq = nseq; a.rowseq = k.rowseq; a.rows = S; a.max_new = new_rows;
+            a.sink = m.sink; a.gate = gate; a.seqs = tail; a.nseq = nseq; a.rowseq = k.rowseq; a.rows = S; a.max_new = new_rows; a.form_new = max_new;
             PROF(COGS_PROF_ATTN);
             COGS_TRY(cogs_k_mla_attention(st, dt, a));
         }
@@ -282,7 +282,7 @@ struct Step {
         } else {
             CogsMla a{};
             a.Q = k.q; a.ldq = (long)m.heads * G.dk; a.q_head = a.q_rot = G.dk; a.ldk = a.ldv = G.kvw; a.O = k.att; a.ldo = G.oin; a.o_head = G.dv;
-            a.dn = G.dk; a.dv = G.dv; a.heads = m.heads; a.seqs = tail; a.nseq = nseq; a.rowseq = k.rowseq; a.rows = S; a.max_new = new_rows;
+            a.dn = G.dk; a.dv = G.dv; a.heads = m.heads; a.seqs = tail; a.nseq = nseq; a.rowseq = k.rowseq; a.rows = S; a.max_new = new_rows; a.form_new = max_new;
             a.layer_off = run.cache_off; a.kvw = G.kvw; a.v_col = G.dk; a.rep = rep; a.bias = m.dist_bias; a.nb = m.dist_n;
             PROF(COGS_PROF_ATTN);
             COGS_TRY(cogs_k_mla_attention(st, dt, a));
@@ -368,7 +368,8 @@ struct Step {
     }
 
     // Nothing but what they leave in the cache and the state is used of the last layer's rows in front of the first one whose logits are asked for.
-    // Behind that the layer goes on with the rest: from a query tile's first row, and with more rows than the few-row kernels take. 4096
+    // Behind that the layer goes on with the rest: from a query tile's first row, and with more rows than the few-row kernels take; the attention in
+    // the whole prompt's order (CogsMla::form_new), so that every row's bits are those of a prompt that goes on with all rows. 4096
     // rows, width 2048: 9 latent layers 4.83 -> 4.55 ms, 8 layers the last of which is attention 5.32 -> 5.02.
     void last_layer_from(int first) {
         r0 = first; R = new_rows = S - first;

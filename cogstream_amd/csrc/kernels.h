@@ -242,6 +242,7 @@ struct CogsMla {
     const float* sink;                           // [heads] in log2 units, or null
     const float* gate;                           // [rows][heads], or null
     const CogsSeq* seqs; int nseq; const int* rowseq; int rows, max_new;     // (new rows of the longest sequence)
+    int form_new;                                // > max_new: rows of the whole prompt that these are the end of, whose order of sums they keep
     int absorbed; long layer_off; int kr_col;
     // kvw != 0: keys and values per head from the sequence's cache (K / KR / V unused): blocks [max_len][kvw] of heads / rep key / value
     // heads from column layer_off on, rows [key | value from v_col]; ldk = ldv = kvw, dr = 0, q_rot = q_head

@@ -968,13 +968,15 @@ int launch_prefill(hipStream_t st, const CogsMla& a) {
 // 32 x 16 behind 1000 2.98 / 3.15, 1 x 2048 + 3 x 64 3.94 / 4.04, + 63 x 32 5.83 / 6.63, 8 x 300 3.07 / 3.13.
 // Up to 128 query tiles of 128 rows are taken as tiles of 64, half the work in a key tile's chain on twice the CUs: passes of 128 rows 863 -> 829 us,
 // 400 1121 -> 1076, 800 1601 -> 1572 (16 heads), 400 of 28 heads 2145 -> 2119, of 32 1682 -> 1656; delta rule, 400 rows 1260 -> 1246.
+// The end of a prompt by itself is in halves where the whole prompt is: a row's keys are added up in the same order then (that of a tile's keys
+// does not depend on the rows of the tile).
 template <int KN, int KR, int DT>
 int launch_prefill_split(hipStream_t st, const CogsMla& a) {
-    const int nqt = (a.max_new + 127) / 128;
-    const long tiles = (long)nqt * a.heads * a.nseq;
+    const int nqt = (max(a.max_new, a.form_new) + 127) / 128;
+    const long pairs = (long)a.heads * a.nseq, tiles = nqt * pairs;
     const bool halves = tiles <= 256 || (tiles <= 512 && a.nseq == 1 && nqt >= a.heads);
     g_cogs_debug.mla_last_waves = halves ? 8 : 4;
-    if (tiles <= 128) return launch_prefill<KN, KR, DT, 2, 2, 1>(st, a);
+    if (halves && (a.max_new + 127) / 128 * pairs <= 128) return launch_prefill<KN, KR, DT, 2, 2, 1>(st, a);
     return halves ? launch_prefill<KN, KR, DT, 2, 2, 2>(st, a) : launch_prefill<KN, KR, DT, 2, 1, 2>(st, a);
 }
 

@@ -451,31 +451,32 @@ def test_streams_that_wait_for_several_outputs(dev, streams, width, loop, dtype)
         assert rms_err(got[r], lg) < TOL[dtype]
 
 
-@pytest.mark.parametrize("past,n", [(0, 257), (0, 321), (90, 320), (3, 449)])
+@pytest.mark.parametrize("past,n,heads", [(0, 257, 4), (0, 321, 4), (90, 320, 4), (3, 449, 4), (40, 449, 40), (0, 449, 80)])
 @pytest.mark.parametrize("name", ["latent", "latent, nothing fed forward", "attention", "delta"])
-def test_rows_of_the_last_layer_that_nothing_reads(dev, name, past, n):
+def test_rows_of_the_last_layer_that_nothing_reads(dev, name, past, n, heads):
     """decoder.hip: a prompt of one sequence goes on behind its last layer's keys, values and state with the query tiles from the first row
-    whose logits are asked for. Caches and states bit for bit those of a prompt that wants every row, logits those of its rows up to the
-    rounding of bfloat16 (other numbers of query tiles are taken by other forms of the attention), wherever the wanted rows lie"""
+    whose logits are asked for. Caches and states bit for bit those of a prompt that wants every row, logits bit for bit those of one that goes
+    on with every row (asked for by wanting every layer's streams), wherever the wanted rows lie and whichever form of the attention
+    the whole prompt's query tiles have: tiles of 64 rows, of 128 rows in halves, of 128 rows (4, 160 and 320 of them, and fewer for the rest)"""
     if name.startswith("latent"):
         import pabalix_models as pm
         from cogstream_amd.llm import DecoderEngine
-        layers = [pm.mixer(pm.A, heads=3), pm.mixer(pm.G, heads=4, kv_rank=56)]
+        layers = [pm.mixer(pm.A, heads=3), pm.mixer(pm.G, heads=heads, kv_rank=56)]
         if "nothing" in name:
             layers[1] = dict(layers[1], ff=None)
         cfg = pm.config(layers, width=136)
         e = DecoderEngine(pm.state(cfg), pm.parse_config(cfg), dtype=torch.bfloat16, device="cuda:0")
     else:
-        last = attention(heads=4, kv_heads=2, dim=64, vdim=32) if name == "attention" else delta(heads=2, kv_heads=1, dim=32, vdim=32)
+        last = attention(heads=heads, kv_heads=2, dim=64, vdim=32) if name == "attention" else delta(heads=2, kv_heads=1, dim=32, vdim=32)
         cfg = config([delta(heads=2, kv_heads=1, dim=32, vdim=32), last], width=200, streams=4)
         e = engine(cfg, state(cfg), torch.bfloat16)
     toks = torch.tensor([(7 * i * i + 3 * i) % cfg["vocab"] for i in range(past + n + 1)])
 
-    def prompt(want):
+    def prompt(want, streams=None):
         c = e.new_cache(past + n + 1)
         if past:
             e.forward_batch(e.embed_tokens(toks[:past]), [past], [c], [])
-        got = e.forward_batch(e.embed_tokens(toks[past:past + n]), [n], [c], want)
+        got = e.forward_batch(e.embed_tokens(toks[past:past + n]), [n], [c], want, streams=streams)
         return got, c.k.clone(), None if c.state is None else c.state.clone(), e.forward_batch(e.embed_tokens(toks[-1:]), [1], [c], [0])
 
     every = prompt(list(range(n)))
@@ -490,6 +491,7 @@ def test_rows_of_the_last_layer_that_nothing_reads(dev, name, past, n):
         assert torch.equal(after, every[3]), want
         if want:
             assert rms_err(got, every[0][want].double().cpu()) < TOL[torch.bfloat16], want
+            assert torch.equal(got, prompt(want, torch.empty(2, n, e.packed.width_p, device=dev))[0]), want
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
