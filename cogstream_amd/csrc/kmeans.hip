@@ -83,38 +83,32 @@ __global__ __launch_bounds__(256, 4) void sqdist_kernel(const T* __restrict__ x,
     extern __shared__ __attribute__((aligned(16))) char smem_raw[];
     float* cs = reinterpret_cast<float*>(smem_raw);
     if (ctl && (ctl[CTL_ABORT] | ctl[CTL_DONE])) return;   // speculatively queued iteration behind the last one
-    const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
-    const long j0 = (long)blockIdx.x * SL;
-    // the centres that have moved since their distances were last summed (keep null: all of them)
-    __shared__ int moved[KMAX + 4];
-    __shared__ int nmoved;
-    if (wid == 0) {
-        const bool mine = lane < K && !(keep && keep[k0 + lane]);
-        const unsigned long long m = __ballot(mine);
-        const int at = __popcll(m & ((1ull << lane) - 1ull)), n = __popcll(m);
-        if (mine) moved[at] = lane;
-        if (lane >= 60) moved[n + lane - 60] = 0;
-        if (lane == 0) nmoved = n;
-    }
-    __syncthreads();
-    K = nmoved;
-    if (K == 0) return;
-    const int KB = (K + 3) & ~3;
-    for (int i = tid; i < KB * 64; i += 256) {
-        const int l = i & 63, k = moved[i >> 6];
-        const long j = j0 + l * 8;
-        float v[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-        if ((i >> 6) < K && j < PD) {
-            if (centre_row >= 0) ld8_f<T>(x + (long)centre_row * PD + j, v);
-            else if (centre_rows) ld8_f<T>(x + (long)centre_rows[k0 + k] * PD + j, v);
-            else ld8_f<float>(centres + (long)(k0 + k) * PD + j, v);
-        }
-        *reinterpret_cast<f32x4*>(cs + (i >> 6) * SL + l * 4) = f32x4{v[0], v[1], v[2], v[3]};
-        *reinterpret_cast<f32x4*>(cs + (i >> 6) * SL + 256 + l * 4) = f32x4{v[4], v[5], v[6], v[7]};
-    }
-    __syncthreads();
-    const long j = j0 + lane * 8;
+    const int lane = threadIdx.x & 63, wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const long j = (long)blockIdx.x * SL + lane * 8;
     const bool in = j < PD;
+    // the centres that have moved since their distances were last summed (keep null: all of them), their list in a register of every wave: lane i has
+    // the i-th. (In LDS its 160 bytes took a workgroup's place on the CU, which the centres fill: launch_sqdist. 256 rows, us, in LDS / here: 18
+    // centres of 168, 301, 350, 448 slices 48.4 / 39.6, 82.1 / 68.2, 78.8 / 76.2, 110.7 / 89.7; 13 to 16 and more than 20 centres 3 to 6 % less)
+    const bool mine = lane < K && !(keep && keep[k0 + lane]);
+    const unsigned long long some = __ballot(mine);
+    const bool all = __popcll(some) == K;
+    K = __popcll(some);
+    if (K == 0) return;
+    const int before = __popcll(some & ((1ull << lane) - 1ull));
+    const int moved = __builtin_amdgcn_ds_permute(4 * (mine ? before : K + lane - before), lane);
+    const int KB = (K + 3) & ~3;
+    for (int i = wid; i < KB; i += 4) {
+        const int k = k0 + __builtin_amdgcn_readlane(moved, i);
+        float v[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+        if (i < K && in) {
+            if (centre_row >= 0) ld8_f<T>(x + (long)centre_row * PD + j, v);
+            else if (centre_rows) ld8_f<T>(x + (long)centre_rows[k] * PD + j, v);
+            else ld8_f<float>(centres + (long)k * PD + j, v);
+        }
+        *reinterpret_cast<f32x4*>(cs + i * SL + lane * 4) = f32x4{v[0], v[1], v[2], v[3]};
+        *reinterpret_cast<f32x4*>(cs + i * SL + 256 + lane * 4) = f32x4{v[4], v[5], v[6], v[7]};
+    }
+    __syncthreads();
     // Two rows per wave and step (rows t, t + 4: a centre's two LDS reads serve both), the NEXT step's global loads issued
     // before this step's arithmetic, and the centres taken FOUR at a time in a real loop: four accumulators per row are
     // exactly one unit of the transposing butterfly below, so nothing outlives a trip and the kernel needs ~80 VGPRs
@@ -148,8 +142,9 @@ __global__ __launch_bounds__(256, 4) void sqdist_kernel(const T* __restrict__ x,
         const bool live_b = t + 4 < r_hi;
         float* pa = partial + ((long)blockIdx.x * Tn + t) * Ktot + k0;
         float* pb = pa + 4 * (long)Ktot;
+        unsigned k = (unsigned)kperm;
 #pragma unroll 1
-        for (int m = 0; m < KB; m += 4) {
+        for (int m = 0; m < KB; m += 4, k += 4) {
             float a[4], b[4];
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
@@ -172,8 +167,8 @@ __global__ __launch_bounds__(256, 4) void sqdist_kernel(const T* __restrict__ x,
             // centre: row 0 -> m, row 1 -> m + 2, row 2 -> m + 1, row 3 -> m + 3
             const float ua = row16_sum(swap16_sum(swap32_sum(a[0], a[1]), swap32_sum(a[2], a[3])));
             const float ub = row16_sum(swap16_sum(swap32_sum(b[0], b[1]), swap32_sum(b[2], b[3])));
+            if (!all) k = (unsigned)__shfl(moved, m + kperm);
             if (writer && m + kperm < K) {
-                const int k = moved[m + kperm];
                 pa[k] = ua;
                 if (live_b) pb[k] = ub;
             }

@@ -38,6 +38,21 @@ def test_header_is_plain_c(tmp_path):
     assert r.returncode == 0, r.stderr
 
 
+def test_distance_pass_has_no_shared_memory_beside_its_centres(tmp_path):
+    """csrc/kmeans.hip sizes sqdist_kernel's grid for workgroups whose centres fill a CU's LDS (launch_sqdist): a few static bytes beside
+    them take one workgroup's place, and the grid runs a second, nearly empty round"""
+    import subprocess
+    from cogstream_amd import build
+    obj, readelf = build.OBJ / "kmeans.o", os.path.join(os.path.dirname(build.OBJDUMP), "llvm-readelf")
+    if not obj.exists() or not os.path.exists(readelf):
+        pytest.skip("no object file, or nothing to read it with")
+    (tmp_path / "kmeans.o").write_bytes(obj.read_bytes())
+    subprocess.run([build.OBJDUMP, "--offloading", "kmeans.o"], cwd=tmp_path, check=True, capture_output=True)
+    notes = subprocess.run([readelf, "--notes", *map(str, tmp_path.glob("*gfx950*"))], check=True, capture_output=True, text=True).stdout
+    sizes = re.findall(r"\.group_segment_fixed_size: (\d+)(?:(?!group_segment).)*?\.name: +\S*sqdist_kernel", notes, re.S)
+    assert sizes == ["0", "0"], sizes
+
+
 def test_no_cpu_fallback():
     """CPU tensors must be rejected loudly, never computed on the host"""
     if torch.cuda.is_available():
