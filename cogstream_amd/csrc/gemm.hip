@@ -1111,7 +1111,13 @@ void dispatch_f32(hipStream_t st, const GemmArgs& p, int grid, int mask, bool bi
 //     mid-size launch (strip of columns, ragged rows, or both). 4096 x 6176 x 2048 108 -> 60 + 41, 768 x 22 016 x 4096 148 -> 115. A strip
 //     of columns reads every weight once; rows that are left read all of them again, and where they are more than half of the 256 MB
 //     Infinity Cache they push the output out of it: 621 x 37 888 x 3584 (two row blocks and 109 rows) gained 5 us and the 18 944-wide
-//     product behind it lost 25 (of more rows than it holds nothing stays there anyway); as a strip (three row blocks x 85 column blocks, 160x256) 163 -> 152 and 113 -> 108, 1000 rows 231 -> 202.
+//     product behind it lost 25; as a strip (three row blocks x 85 column blocks, 160x256) 163 -> 152 and 113 -> 108, 1000 rows 231 -> 202. Of more
+//     rows than REST_ROWS (read and written) little stays there anyway. Two products of a feed-forward, rows left over / not, by bytes of rows:
+//     3584 x 37 888 and back 43 MB 1.15, 50 MB 1.14; 3584 x 28 416 49 .. 83 MB 1.09 .. 1.01, 93 MB 1.04, 120 MB 1.01; 4096 x 22 016 41 MB 1.03, 54 .. 140 MB
+//     0.97 .. 1.01; 9728 x 21 888 96 MB and 9472 x 21 824 140 MB 1.13 and 1.06; beyond, 13 376 x 6208 208 MB 0.94, 8256 x 8256 202 MB 0.96, 3584 x 18 944 210 .. 256 MB
+//     0.97 .. 1.0, 28 416 x 3584 295 MB 0.95. The line itself lies between 140 and 178 MB
+//     (13 696 x 7296 190 MB and 12 096 x 7232 178 MB 0.96); of weights of 500 MB it is as much as 2 % off (2706 x 20 544 x 19 392 0.98).
+//   * Up to MIXED_ROUNDS rounds this decides alone; of more, a last round that is less than 45 % full leaves its rows to a mid-size launch.
 struct TileCost { int tile, tm, tn; float one, two, rest, full; };     // us; two = 0: one workgroup per CU; full: a slab's surcharge on a full chip
 static constexpr TileCost MID_TILES[] = {
     {1, 32, 64, 0.174f, 0.f, 0.9f, 0.14f},     {2, 64, 64, 0.213f, 0.381f, 2.2f, 0.08f}, {3, 128, 64, 0.311f, 0.569f, 2.1f, 0.14f},
@@ -1120,7 +1126,8 @@ static constexpr TileCost MID_TILES[] = {
     {10, 192, 128, 0.502f, 0.f, 4.8f, 0.44f},  {11, 160, 256, 0.767f, 0.f, 4.9f, 0.42f}};
 static constexpr TileCost PP_TILE = {0, 256, 256, 1.127f, 0.f, 7.5f, 0.25f};
 static constexpr float SECOND_LAUNCH = 2.f, LN_FINALIZE = 5.f;                      // us
-static constexpr float REST_READ = 4.4e6f, REST_AGAIN = 128e6f;                     // weights of a second launch: bytes a us, and the most that are read again
+static constexpr float REST_READ = 4.4e6f;                                          // weights of a second launch: bytes a us
+static constexpr float REST_AGAIN = 128e6f, REST_ROWS = 160e6f;                     // the most that are read again beside fewer bytes of rows than that
 static constexpr int MIXED_ROUNDS = 4;                                              // (of more rounds the last one is little)
 
 static float tile_time(int tiles, int slabs, const TileCost& t) {
@@ -1273,7 +1280,7 @@ static int gemm_rows(hipStream_t st, const CogsGemm& g, bool* kv_stored) {
             // row blocks x column blocks here (all columns: p.nbn, with the tall tiles), the L-shaped rest in one mid-size launch
             auto consider = [&](int mb, int cb) {
                 const int rows = min(mb * BM3, g.M), cols = cb >= p.nbn ? g.N : cb * BN3;
-                if (mb <= 0 || cb <= 0 || (rows == g.M && cols == g.N) || (rows < g.M && 2.f * g.K * g.N > REST_AGAIN && 2.f * g.M * ((float)g.K + g.N) < 2 * REST_AGAIN)) return;
+                if (mb <= 0 || cb <= 0 || (rows == g.M && cols == g.N) || (rows < g.M && 2.f * g.K * g.N > REST_AGAIN && 2.f * g.M * ((float)g.K + g.N) < REST_ROWS)) return;
                 float rest;
                 const int tile = best_mid_tile(g.M, g.N, g.K, S == 1, &rest, rows, cols);
                 rest = max(rest, 2.f * g.K * (rows < g.M ? g.N : g.N - cols) / REST_READ);
@@ -1288,7 +1295,7 @@ static int gemm_rows(hipStream_t st, const CogsGemm& g, bool* kv_stored) {
                 }
             }
         }
-        if (mb_main < 0 && S == 1 && !env_nosplit && !env_nostore && g.K >= 2048 && rounds >= 2 && rem > 0 && rem * 100 < PERSISTENT_WGS * 45) {
+        if (nb > MIXED_ROUNDS * PERSISTENT_WGS && S == 1 && !env_nosplit && !env_nostore && g.K >= 2048 && rem > 0 && rem * 100 < PERSISTENT_WGS * 45) {
             // (many tiles, one stream -- beside a second one a split launch costs the 64-frame clip 1 %: pays when a tile is long against a second launch and the last round is less than ~45 % full:
             // measured with the two-segment K loop at K = 1152: -2 %; K = 3584, last round 34 % full: +2 %; K = 18944,
             // 34 %: +6 %; K = 4352, 51 % full (ViT fc2): -2 %, so it no longer splits)

@@ -1256,6 +1256,22 @@ def test_whole_rounds_and_an_l_shaped_rest_equal_one_launch(dev, M, N, K):
         assert outs[0][1] is None or torch.equal(outs[0][1], outs[1][1]), name
 
 
+@pytest.mark.parametrize("M,N,K,split", [(4707, 3584, 18944, True), (6117, 8256, 8256, True), (1514, 21888, 9728, False), (2242, 21824, 9472, False)])
+def test_rows_left_over_large_weights(dev, M, N, K, split):
+    """gemm.hip, REST_AGAIN and REST_ROWS: weights that half the last-level cache does not hold are read again for left-over rows only of products
+    whose rows do not stay there either; up to four rounds nothing else splits them. The bits of one launch"""
+    from cogstream_amd import _lib as L2
+    ops = _ops()
+    g = torch.Generator(device=dev).manual_seed(M)
+    a, w = (torch.randn(n, K, generator=g, device=dev).bfloat16() for n in (M, N))
+    outs = []
+    for on in (1, 0):
+        with L2.debug_switch("gemm_split", on):
+            outs.append(ops.gemm(a, w))
+            assert L2.debug_get("gemm_last_body") == (5 if split and on else 4)
+    assert torch.equal(*outs)
+
+
 @pytest.mark.parametrize("t,h,w,merge,max_tokens,offset", [
     (1, 28, 28, 2, 16384, 0),        # one window, enlarged: the smallest
     (1, 45, 61, 1, 16384, 1),        # odd source sizes, frames that start off a word
