@@ -161,7 +161,7 @@ def _llm(dev, dtype):
     return cfg, st, Qwen2Engine(st, cfg, dtype=dtype, device=dev)
 
 
-@pytest.mark.parametrize("tile,split", [(0, 1), (1, 1), (3, 1), (4, 1), (5, 1), (7, 1), (0, 0)])
+@pytest.mark.parametrize("tile,split", [(0, 1), (1, 1), (3, 1), (4, 1), (5, 1), (7, 1), (8, 1), (9, 1), (10, 1), (11, 1), (0, 0)])
 def test_keys_and_values_stored_by_the_qkv_product(dev, tile, split):
     """the QKV product's waves store their K and V columns into the cache (the ping-pong kernel's, split = 0, are copied): the same bits
     as without a cache, where attention reads the product's own rows, and behind a kept first part"""
@@ -181,6 +181,29 @@ def test_keys_and_values_stored_by_the_qkv_product(dev, tile, split):
             n = rows // 2 + 1
             got = [eng.forward(p, parts, want_logits=False, want_hidden=True)["hidden"] for p in (x[:n], x[n:]) if p.shape[0] > 1]
             assert torch.equal(torch.cat(got), want[:sum(p.shape[0] for p in got)])
+
+
+@pytest.mark.parametrize("width,heads,grids", [(576, 8, [(1, 1, 2), (1, 5, 7), (1, 13, 13), (1, 23, 23), (1, 20, 35)]), (1152, 16, [(1, 1, 3), (1, 9, 11), (2, 12, 15)]),
+                                               (3456, 48, [(1, 1, 2), (1, 11, 17)])])
+def test_norms_folded_into_the_products_of_every_tile(dev, width, heads, grids):
+    """gemm_mid.hip: a tile forms its rows' factors from statistics in partial sums, through a ring slot (two factors a lane with five row blocks a wave,
+    fewer rows than lanes with three) or, of an odd number of sums or more than a slot holds (54 a row), from memory. An encoder in bf16 with every
+    tile forced, of ragged numbers of patches: the bits of 64x64 tiles"""
+    from cogstream_amd import _lib as L2
+    from cogstream_amd.vision import VisionEncoder
+    from cogstream_amd.weights import VisionConfig, random_vit_state
+    cfg = VisionConfig(hidden_size=width, intermediate_size=200, num_hidden_layers=2, num_attention_heads=heads)
+    enc = VisionEncoder(random_vit_state(cfg, seed=2, std=0.05), cfg, dtype=torch.bfloat16, device=dev)
+    assert enc.packed.fold_ln
+    for t, h, w in grids:
+        pix = (torch.rand(t * h * w, 588, generator=torch.Generator().manual_seed(h)) * 2 - 1).bfloat16().to(dev)
+        out = {}
+        for tile in (2, 1, 3, 4, 5, 6, 7, 8, 9, 10, 11):
+            with L2.debug_switch("gemm_mid", tile):
+                out[tile] = enc(pix, torch.tensor([[t, h, w]]), torch.tensor([1])).clone()
+                assert L2.debug_get("gemm_last_tile") == tile
+            assert torch.equal(out[tile], out[2]), (tile, t, h, w)
+        assert bool(torch.isfinite(out[2].float()).all())
 
 
 @pytest.mark.parametrize("dtype,split,copies", [(torch.bfloat16, 1, 0), (torch.bfloat16, 0, 2), (torch.float32, 1, 2)])

@@ -1212,7 +1212,7 @@ def test_one_row_of_160_row_tiles_is_not_chosen(dev, M, want):
 
 @pytest.mark.parametrize("tile", [6, 7])
 def test_mid_size_gemm_tiles_of_two_slabs_and_of_160_rows(dev, tile):
-    """the same edges for 128x64 with two slabs a slot and 160x64 (five row blocks a wave; a folded norm falls back to 128x64)"""
+    """the same edges for 128x64 with two slabs a slot and 160x64 (five row blocks a wave)"""
     test_mid_size_gemm_tiles_equal_each_other_and_fp64(dev, tile)
 
 
