@@ -1432,11 +1432,12 @@ def test_a_split_product_whose_remainder_is_one_row(dev, M, N, K, form):
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("T,K,PD,kind", [(40, 5, 520, "plain"), (150, 33, 1032, "plain"), (200, 70, 512, "plain"), (64, 6, 1024, "empty"),
-                                         (48, 4, 1024, "infinite"), (3, 2, 8, "plain")])
+                                         (48, 4, 1024, "infinite"), (3, 2, 8, "plain"), (60, 7, 1032, "far"), (150, 33, 520, "far"), (90, 12, 1024, "dry")])
 def test_centres_that_stay_keep_their_distances_and_means(dev, T, K, PD, kind, dtype):
     """csrc/kmeans.hip: the Lloyd loop sums distances and means only for centres whose rows have changed, and not those the seeding
     has summed. Every iteration bit for bit against the same steps called one by one, which sum everything: more centres than one distance
-    launch holds, or than a wave, with clusters that run empty (duplicated centres, reseeded) and a row of infinities"""
+    launch holds, or than a wave, with clusters that run empty (duplicated centres; every other centre too late for any row, from the seeding's
+    distances; both reseeded), a pool that runs dry in a call that starts from those and is called again, and a row of infinities"""
     ops = _ops()
     g = torch.Generator(device=dev).manual_seed(T + K)
     x = (torch.randn(max(2, K // 2), PD, generator=g, device=dev).repeat(T, 1)[:T] + 0.3 * torch.randn(T, PD, generator=g, device=dev)).to(dtype)
@@ -1447,13 +1448,16 @@ def test_centres_that_stay_keep_their_distances_and_means(dev, T, K, PD, kind, d
     q = torch.rand(K - 1, T, generator=g, device=dev) + 0.01
     d2 = torch.full((T, K), -1.0, device=dev)
     rows, flag = ops.kmeans_pp(x, 2, K, q, ws, d2)
-    known = K - 1 if kind == "plain" and int(flag) == 0 else 0
+    known = K - 1 if kind in ("plain", "far", "dry") and int(flag) == 0 else 0
+    assert known or kind in ("empty", "infinite")
     rows = rows.long()
     if kind == "empty":
         rows = torch.full((K,), 7, device=dev)
         rows[0] = 11
     pool = [int(v) for v in torch.randint(0, T, (400,), generator=torch.Generator().manual_seed(1))]
     c0, t0 = x[rows].float().contiguous(), ts[rows].contiguous()
+    if kind in ("far", "dry"):
+        t0[1::2] = 10.0 * T
     if known:                                  # the seeding's sums are those of the distance pass (fp64 over slices: the last place at most)
         whole = ops.kmeans_sqdist(x, c0, None, K, ws)
         assert bool(((d2[:, :known] - whole[:, :known]).abs() <= whole[:, :known] * 2.0 ** -23).all())
@@ -1469,6 +1473,11 @@ def test_centres_that_stay_keep_their_distances_and_means(dev, T, K, PD, kind, d
             if float(ops.kmeans_update(x, ts, a, reseed, c, ct, ws)) <= 1e-4:
                 break
         gc, gt, ga = c0.clone(), t0.clone(), torch.empty(T, dtype=torch.int64, device=dev)
-        got = ops.kmeans_lloyd(x, ts, gc, gt, ga, 2.0, iters, 1e-4, pool, ws, d2.clone() if known else None, known)
+        mine, left = d2.clone() if known else None, known
+        if kind == "dry":
+            assert ops.kmeans_lloyd(x, ts, gc, gt, ga, 2.0, iters, 1e-4, pool[:K // 2 - 1], ws, mine, left) == (0, 0, True)
+            left = 0
+        got = ops.kmeans_lloyd(x, ts, gc, gt, ga, 2.0, iters, 1e-4, pool, ws, mine, left)
         assert got == (done, used, False), (iters, got, done, used)
+        assert used >= K // 2 or kind not in ("far", "dry")
         assert torch.equal(ga, a) and torch.equal(gt, ct) and torch.equal(gc.view(torch.int32), c.view(torch.int32)), iters
