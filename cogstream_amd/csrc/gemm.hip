@@ -1102,8 +1102,9 @@ void dispatch_f32(hipStream_t st, const GemmArgs& p, int grid, int mask, bool bi
 // time of a slab + the rest of a tile: prologue, epilogue), with a slab's time per tile size for one and, where the LDS has room for
 // them, two workgroups on a CU; a slab takes longer the fuller the chip is (from half of the CUs on, by `full` with all of them: power,
 // and the CUs that read weights ahead are gone). The figures are a fit to launches of every tile at M = 40 .. 4096 and 23 weight shapes from
-// 1152 x 1152 to 37 888 x 3584 and 3584 x 18 944 (MI355X, weights from HBM, nothing beside them): over those 805 products the choice
-// is 0.6 % slower than the best on the average, 5 % or more in 20 (64 x 28 416 x 3584: 64x64 46 us, 128x128 40; 512 x 2048 x 5632 26.5 / 23.9).
+// 1152 x 1152 to 37 888 x 3584 and 3584 x 18 944 (MI355X, weights from HBM, nothing beside them): over those 805 products the choice is
+// 1.1 % slower than the best single launch on the average, 5 % or more in 48 (64 x 28 416 x 3584: 64x64 46.6 us, 128x128 40.6; 1280 x 2048 x 5632:
+// 160x64 44.2, 128x128 38.1; 512 x 2048 x 5632: 64x64 26.4, 96x64 23.7), and as much faster where it mixes two.
 //   * The steps between the sizes count: a product of 1.1 rounds takes two. 96x64, 160x128, 192x128 and 160x256 beside 32x64, 64x64, 128x64,
 //     160x64, 128x128 and 128x256 took, us: 2048 x 4304 x 1152 31.2 -> 24.6 (221 tiles of 160x256 for 272 of 128x256), 924 x 4352 x 1152 16.7
 //     -> 13.6, 1300 x 3584 x 18 944 205 -> 167, 300 x 3584 x 28 416 145 -> 115, 512 x 37 888 x 3584 160 -> 127; 3 % on the average of the 805.
@@ -1120,7 +1121,7 @@ void dispatch_f32(hipStream_t st, const GemmArgs& p, int grid, int mask, bool bi
 //   * Up to MIXED_ROUNDS rounds this decides alone; of more, a last round that is less than 45 % full leaves its rows to a mid-size launch.
 struct TileCost { int tile, tm, tn; float one, two, rest, full; };     // us; two = 0: one workgroup per CU; full: a slab's surcharge on a full chip
 static constexpr TileCost MID_TILES[] = {
-    {1, 32, 64, 0.174f, 0.f, 0.9f, 0.14f},     {2, 64, 64, 0.213f, 0.381f, 2.2f, 0.08f}, {3, 128, 64, 0.311f, 0.569f, 2.1f, 0.14f},
+    {1, 32, 64, 0.174f, 0.f, 0.9f, 0.14f},     {2, 64, 64, 0.213f, 0.381f, 2.2f, 0.08f}, {3, 128, 64, 0.311f, 0.569f, 2.9f, 0.14f},
     {4, 128, 128, 0.379f, 0.f, 3.5f, 0.29f},   {5, 128, 256, 0.633f, 0.f, 5.3f, 0.36f},  {6, 128, 64, 0.271f, 0.f, 2.7f, 0.21f},
     {7, 160, 64, 0.312f, 0.f, 3.2f, 0.28f},    {8, 96, 64, 0.238f, 0.f, 2.0f, 0.24f},    {9, 160, 128, 0.443f, 0.f, 4.6f, 0.39f},
     {10, 192, 128, 0.502f, 0.f, 4.8f, 0.44f},  {11, 160, 256, 0.767f, 0.f, 4.9f, 0.42f}};

@@ -1256,6 +1256,20 @@ def test_whole_rounds_and_an_l_shaped_rest_equal_one_launch(dev, M, N, K):
         assert outs[0][1] is None or torch.equal(outs[0][1], outs[1][1]), name
 
 
+@pytest.mark.parametrize("M,N,K,tile", [(300, 4352, 1152, 6), (400, 3456, 1152, 6), (560, 3072, 768, 6), (384, 4096, 1024, 6)])
+def test_choice_between_tiles_of_64_columns(dev, M, N, K, tile):
+    """gemm.hip: 128x64 with one slab a slot is not taken where it has a CU to itself (two slabs are 4 to 10 % faster there), nor 96x64 on every
+    CU"""
+    from cogstream_amd import _lib as L2
+    ops = _ops()
+    g = torch.Generator(device=dev).manual_seed(M)
+    a, w = (torch.randn(n, K, generator=g, device=dev).bfloat16() for n in (M, N))
+    y = ops.gemm(a, w)
+    assert L2.debug_get("gemm_last_tile") == tile
+    with L2.debug_switch("gemm_mid", 2):
+        assert torch.equal(y, ops.gemm(a, w))
+
+
 @pytest.mark.parametrize("M,N,K,split", [(4707, 3584, 18944, True), (6117, 8256, 8256, True), (1514, 21888, 9728, False), (2242, 21824, 9472, False)])
 def test_rows_left_over_large_weights(dev, M, N, K, split):
     """gemm.hip, REST_AGAIN and REST_ROWS: weights that half the last-level cache does not hold are read again for left-over rows only of products
