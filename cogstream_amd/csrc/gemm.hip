@@ -1155,7 +1155,10 @@ static int best_mid_tile(int M, int N, int K, bool alone, float* time, int rows0
         // 5171 us with it, 4792 without; 5 x 924 5988 / 5604, 4 x 924 5283 / 4876, 8 x 924 7661 / 7663. The four sizes behind it are no better there:
         // 12 x 924 12 030 with them, 11 400 without, 3 x 1600 6790 / 6050, 16 x 924 14 430 / 13 800)
         if (t.tile >= 7 && !alone) continue;
-        if (t.tile == 8 && tiles > PERSISTENT_WGS - 8) continue;      // (its weights come too slowly with no CU to read them ahead: 768 x 2048 x 5632 32.2 us, 128x64 28.8)
+        // (96x64 on every CU, none left that reads weights ahead, only where the last row tile is far from full -- its rows are a third of them or less
+        // in what was timed: 300 x 4096 x 16 384 66.9 us, 128x64 79.4, 320 rows 70.6 / 81.1, 300 x 4096 x 11 008 47.6 / 54.9, 700 x 2048 x 5632 26.4 / 28.3, 1280
+        // x 1152 x 4352 21.5 / 23.7; full: 384 x 4096 x 16 384 85.2 / 81.1, 384 x 4096 x 11 008 63.9 / 59.8, 768 x 2048 x 5632 32.2 / 28.8, 768 x 2048 x 8192 41.4 / 39.5)
+        if (t.tile == 8 && tiles > PERSISTENT_WGS - 8 && ((M - rows0) % t.tm == 0 || (M - rows0) % t.tm > t.tm / 2)) continue;
         if ((t.tile == 7 || t.tile == 9) && (M - rows0 <= t.tm || (t.tile == 7 && tiles > PERSISTENT_WGS))) continue;
         const float c = tile_time(tiles, K / 64, t);
         if (best == 0 || c < *time) { best = t.tile; *time = c; }

@@ -1256,10 +1256,10 @@ def test_whole_rounds_and_an_l_shaped_rest_equal_one_launch(dev, M, N, K):
         assert outs[0][1] is None or torch.equal(outs[0][1], outs[1][1]), name
 
 
-@pytest.mark.parametrize("M,N,K,tile", [(300, 4352, 1152, 6), (400, 3456, 1152, 6), (560, 3072, 768, 6), (384, 4096, 1024, 6)])
+@pytest.mark.parametrize("M,N,K,tile", [(300, 4352, 1152, 6), (400, 3456, 1152, 6), (560, 3072, 768, 6), (300, 4096, 1024, 8), (700, 2048, 2048, 8), (384, 4096, 1024, 6)])
 def test_choice_between_tiles_of_64_columns(dev, M, N, K, tile):
-    """gemm.hip: 128x64 with one slab a slot is not taken where it has a CU to itself (two slabs are 4 to 10 % faster there), nor 96x64 on every
-    CU"""
+    """gemm.hip: 128x64 with one slab a slot is not taken where it has a CU to itself (two slabs are 4 to 10 % faster there), 96x64 on every CU only where
+    its last row tile is far from full"""
     from cogstream_amd import _lib as L2
     ops = _ops()
     g = torch.Generator(device=dev).manual_seed(M)
