@@ -655,8 +655,8 @@ __global__ __launch_bounds__(UF_T) void update_final_kernel(const float* __restr
     }
 }
 
-// what a loop starts from: n words of zeros at a and one at b (nullable), ones and zeros at keep. One launch: a memset of a few words is one or two of
-// 3.4 us each (256 frames of 50 tokens: eleven of them 37 us)
+// what a loop starts from: n words of zeros at a and one at b (nullable), ones and zeros at keep. One launch: memsets of a few words are one to three of 1 to
+// 5 us and a gap (256 frames of 50 tokens: 28 us in front of the Lloyd loop, 5 so)
 __global__ __launch_bounds__(256) void start_kernel(int* a, int n, int* b, int* keep, int K, int known) {
     for (int i = threadIdx.x; i < n; i += 256) a[i] = 0;
     if (b && threadIdx.x == 0) *b = 0;
@@ -962,8 +962,9 @@ int cogs_k_kmeans_pp(hipStream_t st, int dtype, const void* feats, int T, long P
 }
 
 // The Lloyd loop (kmeans_with_time.py:71-131). Centres that have not moved keep their distances (dist2) and means: a cluster that no row has joined
-// or left, and in the first iteration the `known` leading centres whose columns of dist2 the caller brings from the seeding. 256 frames of 179 200
-// bf16, 18 centres, two iterations that move and one that does not: distances 3 x 78 us -> 26 + 78 + 25, means 3 x 20 -> 21 + 8 + 5 (all of it 1059 -> 962).
+// or left, and in the first iteration the `known` leading centres whose columns of dist2 the caller brings from the seeding (the same fp32 slice sums,
+// added up in another fp64 order). 256 frames of 179 200 bf16, 18 centres, two iterations that move and one that does not: distances 3 x 76 us ->
+// 23 + 78 + 24, means 3 x 21 -> 20 + 8 + 5; with one launch and one read instead of several the whole clustering 948 -> 843.
 // The host queues up to LLOYD_BATCH iterations between two reads of the
 // control words (update_final copies them into host-mapped memory): every kernel of an iteration returns at once when an
 // earlier one has converged or run the reseed pool dry, so the iterations queued behind the last one change nothing.

@@ -268,7 +268,8 @@ cogs_status cogs_kmeans_lloyd(cogs_stream stream, int dtype, const void* feats, 
                               float* centres, float* centre_ts, int64_t* assign, int* iterations, int* reseeds_used,
                               int* pool_exhausted, void* ws, size_t ws_bytes);
 /* The same; dist2 (nullable unless known > 0, device fp32 [T][K], overwritten): its first `known` columns hold the squared distances
- * to the first `known` centres as they come in, which are then not summed again. watch (nullable): a device word whose value behind the
+ * to the first `known` centres as they come in, which are then not summed again (cogs_kmeans_pp_dist adds the same fp32 slice sums up in another
+ * fp64 order than the loop does: a distance may differ from the loop's own in its last place). watch (nullable): a device word whose value behind the
  * last iteration the call hands back in *watched (-1 if it ran none) -- cogs_kmeans_pp's zero_flag, without a read of its own;
  * min_margin, rows_below (nullable): what cogs_kmeans_margins would say. */
 cogs_status cogs_kmeans_lloyd_dist(cogs_stream stream, int dtype, const void* feats, const float* ts, int T, int64_t PD, int K,
@@ -549,8 +550,9 @@ cogs_status cogs_decoder_workspace_bytes(cogs_handle h, int rows, int nseq, int6
  * to back), at positions kv[i]->len ..; its cache rows are appended and kv[i]->len advances. No padding, any mix of lengths.
  * want (host [n_want], row numbers) -> logits fp32 [n_want][vocab_p]. streams, nullable: fp32 [layer runs][rows][width_p], the
  * residual stream (the sum of the streams) behind every layer run. Steps of one token per sequence take the absorbed form of
- * latent attention. The order of sums depends on the step's shape (rows, sequences, longest context): the same call gives the same
- * bits, the same tokens in another step the same values to rounding. The workspace size is that of this step's shape; of one
+ * latent attention. The order of sums depends on the step's shape (rows, sequences, longest context) and on the number of wanted rows,
+ * not on which they are or on `streams`: the same call gives the same bits, the same tokens in another step the same values to
+ * rounding. `embeds` is read until the step is done. The workspace size is that of this step's shape; of one
  * sequence, from two rows on, more rows never need less. */
 cogs_status cogs_decoder_forward(cogs_handle h, cogs_stream stream, const void* embeds, cogs_kv* const* kv, const int32_t* lens, int nseq,
                                  const int32_t* want, int n_want, float* logits, float* streams, void* ws, size_t ws_bytes);
