@@ -457,7 +457,7 @@ def test_rows_of_the_last_layer_that_nothing_reads(dev, name, past, n, heads):
     """decoder.hip: a prompt of one sequence goes on behind its last layer's keys, values and state with the query tiles from the first row
     whose logits are asked for. Caches and states bit for bit those of a prompt that wants every row, logits bit for bit those of one that goes
     on with every row (asked for by wanting every layer's streams), wherever the wanted rows lie and whichever form of the attention
-    the whole prompt's query tiles have: tiles of 64 rows, of 128 rows in halves, of 128 rows (4, 160 and 320 of them, and fewer for the rest)"""
+    the whole prompt's query tiles have: tiles of 64 rows, of 128 rows in halves, of 128 rows (12 to 16, 160 and 320 tiles, and fewer of the rest)"""
     if name.startswith("latent"):
         import pabalix_models as pm
         from cogstream_amd.llm import DecoderEngine
