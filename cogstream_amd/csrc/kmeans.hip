@@ -8,8 +8,8 @@
 //   update        per-cluster means (or the reseed row), centre shift                                (:107-125)
 //
 // HBM-bound by design: the features [T, P*D] (bf16 or fp32, 92/183 MB at T = 256) are read exactly once by sqdist and
-// once by update per Lloyd iteration, once per k-means++ step. Round 3 rebuilt the kernels around that bound (rocprofv3
-// at [256, 179 200] bf16, K = 18: sqdist 349 -> see DESIGN.md; the first version reduced every (row, centre) pair
+// once by update per Lloyd iteration, once per k-means++ step. The kernels are built around that bound (rocprofv3
+// at [256, 179 200] bf16, K = 18: sqdist 349 -> 76 us; the first version reduced every (row, centre) pair
 // across the wave on its own -- 12 cross-lane steps per pair -- and walked member lists one load at a time):
 //   * sqdist keeps one accumulator per centre in registers and reduces all of them across the wave in ONE
 //     transposing butterfly per row (v_permlane32_swap / v_permlane16_swap on register pairs, then DPP row sums):
@@ -21,7 +21,8 @@
 //   * update runs one workgroup per (column block, cluster) -- K times the parallelism -- with four member rows in
 //     flight per thread.
 // All sums run in a fixed order (reproducible run to run). Distances are DIRECT sums of (x - c)^2, fp32 within a
-// 512-column slice, fp64 across slices: DESIGN.md section 2 (near-tie study) says why not |x|^2 + |c|^2 - 2 x.c.
+// 512-column slice, fp64 across slices: |x|^2 + |c|^2 - 2 x.c cancels (|x|^2 is 200 times the nearest distances here, an ulp of it 1e-5 of them), and
+// more than a quarter of the rows whose two nearest centres lie within 1e-4 of one another were assigned by its rounding.
 #include "common.h"
 #include "kernels.h"
 #include "debug.h"
@@ -41,7 +42,7 @@ enum { CTL_USED = 0,      // reseed-pool entries consumed so far
        CTL_MARGIN = 6,    // bits(+inf) - bits(min over rows and iterations of the decision margin) (reduce_assign_kernel)
        CTL_NEAR = 7,      // rows (summed over iterations) whose margin is below NEAR_TIE
        CTL_WORDS = 8 };
-constexpr float NEAR_TIE = 1e-3f;   // DESIGN.md section 2: below this the reference's own sgemm rounding decides a row
+constexpr float NEAR_TIE = 1e-3f;   // below this the reference's own sgemm rounding decides a row
 
 constexpr int SL = 512;       // columns per slice
 constexpr int KMAX = 32;      // centres per sqdist launch (K itself is unbounded: 18 for 256 frames, 40 for 600)
@@ -59,7 +60,7 @@ __device__ __forceinline__ float swap16_sum(float a, float b) {
 }
 // sum over each 16-lane row, result in every lane of the row: four DPP adds (quad swaps, then the two mirrors). The
 // __shfl_xor form compiles to four DEPENDENT ds_bpermute round trips -- ~400 exposed cycles per call, more than the
-// arithmetic of the unit it closes (rocprofv3: 102 -> see DESIGN.md us per K = 18 pass).
+// arithmetic of the unit it closes (a pass of K = 18 took 102 us with it).
 template <int CTRL>
 __device__ __forceinline__ float dpp_mov(float v) {
     return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xf, 0xf, true));
@@ -266,7 +267,7 @@ __global__ __launch_bounds__(256) void reduce_assign_kernel(const float* __restr
     if (lane == 0) assign[t] = cand == 0x7fffffff ? 0 : cand;        // all-NaN row: cluster 0, like a serial first-minimum scan
     if (ctl && K > 1 && cand != 0x7fffffff) {
         // How close was the decision? Runner-up = the smallest final distance of any OTHER cluster. The margin is
-        // expressed in the unit the near-tie study uses: the RELATIVE change of the feature
+        // expressed in the unit the near-tie study (tests/golden/kmeans_tie_study.py) uses: the RELATIVE change of the feature
         // distances that would flip the order. A relative change e of d_k moves nf_k by d_k e / R (R = max - min of
         // the row) and the final distance sqrt(nf^2 + alpha nt^2) by (nf_k / fd_k) d_k e / R; with the winner moving up
         // and the runner-up down the gap closes at e* = gap / (s_1 + s_2); reported as 2 e*, which for a pure feature
@@ -1039,7 +1040,7 @@ int cogs_k_kmeans_lloyd(hipStream_t st, int dtype, const void* feats, const floa
 
 // how close the assignments of the last cogs_k_kmeans_lloyd call on this workspace were: the smallest relative margin
 // (second-best - best) / best of the final distance over all rows and iterations, and the number of (row, iteration)
-// pairs below 1e-3 -- below that the reference's own cdist rounding decides the row (DESIGN.md section 2)
+// pairs below 1e-3 -- below that the reference's own cdist rounding decides the row
 int cogs_k_kmeans_margins(hipStream_t st, int T, long PD, int K, float* ws, float* min_margin, int* rows_below) {
     const KmWs w = carve(ws, T, PD, K);
     int h[CTL_WORDS];

@@ -210,7 +210,7 @@ cogs_status cogs_cosine(cogs_stream stream, const float* a, const float* b, int 
 /* Time-aware k-means steps (model/kmeans_with_time.py:4-137); the host keeps the RNG draws.
  * feats [T, PD] (dtype), centres fp32 [K, PD], ts/centre_ts fp32. Any T and K (the reference has no limit: a
  * 600-frame session clusters into K = 40). Distances are direct sums of (x - c)^2, not torch.cdist's
- * |x|^2 + |c|^2 - 2 x.c: see DESIGN.md section 2 (near-tie study) for where the reference's own rounding decides. */
+ * |x|^2 + |c|^2 - 2 x.c, whose rounding decides rows that lie nearly as close to a second centre (cogs_kmeans_margins). */
 cogs_status cogs_kmeans_workspace_bytes(int T, int64_t PD, int K, size_t* bytes);
 /* dist2[T,K] = squared L2 distance to the centres; centre_rows (device int32 [K], nullable)
  * selects feature rows as centres instead of `centres` (k-means++ init, :46-50) */
@@ -280,7 +280,7 @@ cogs_status cogs_kmeans_lloyd_dist(cogs_stream stream, int dtype, const void* fe
 /* How close the assignments of the LAST cogs_kmeans_lloyd call on this workspace were (host outputs; synchronises).
  * Per row and iteration: the relative change of the row's feature distances that would flip the decision between its
  * best and second-best cluster -- with every time term equal this is (d2 - d1) / mean(d1, d2) of the two nearest feature
- * distances, the margin of the near-tie study; a decision the feature distances cannot flip is
+ * distances, the margin of the near-tie study (tests/golden/kmeans_tie_study.py); a decision the feature distances cannot flip is
  * +inf. *min_margin = the minimum over all rows and iterations, *rows_below = the number of (row, iteration) pairs
  * below 1e-3. Below that margin the reference's own torch.cdist rounding decides the row and no other summation order
  * reproduces it; at or above it the assignment equals the reference's. */
