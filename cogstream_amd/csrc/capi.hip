@@ -54,7 +54,7 @@ static bool cogs_debug_value_ok(const char* name, int64_t v) {
     static const Range ranges[] = {
         {"gemm_wgs", 0, 256}, {"gemm_mid", 0, 11}, {"gemm_pad_pct", 100, 400}, {"gemm_group_m", 0, 64}, {"gemm_co_streams", 0, 8},
         {"gemv_small_n", 0, 1 << 30}, {"attn_vit", 0, 2}, {"attn_uniform_hint", 0, 1 << 20}, {"attn_prio", 0, 2},
-        {"attn_nq", 0, 2}, {"vit_split_max", 0, INT64_MAX}, {"llm_split_keys", 0, 1 << 24}, {"mla_split_keys", 0, 1 << 24}, {"km_row_groups", 0, 1 << 16},
+        {"attn_nq", 0, 2}, {"vit_split_max", 0, INT64_MAX}, {"llm_split_keys", 0, 1 << 24}, {"mla_split_keys", 0, 1 << 24}, {"km_row_groups", 0, 1 << 16}, {"km_pp_form", 0, 3},
     };
     for (const Range& r : ranges)
         if (strcmp(name, r.name) == 0) return v >= r.lo && v <= r.hi;
@@ -107,7 +107,7 @@ const char* cogs_debug_list(void) {
         "mla_last_waves (read only): waves per query tile of the last prompt attention of a described decoder in bf16, 4 or 8\n"
         "preprocess_last_kernel (read only): kernel of the last cogs_preprocess_frames -- 1 two passes, 2 vector tiles, else matrix products: "
         "100 x 64-byte steps of a row + 10 x patch rows of a band + 16-row tiles of its source rows\n"
-        "km_pp_last_launches (read only): kernels per centre of the last cogs_kmeans_pp, 1 or 3\n";
+        "km_pp_last_launches (read only): form of the last cogs_kmeans_pp, 1 a row per workgroup, 3 by slices\n";
 }
 
 cogs_status cogs_create(int device, cogs_handle* out) {
@@ -267,7 +267,7 @@ cogs_status cogs_kmeans_pp_dist(cogs_stream stream, int dtype, const void* feats
     const size_t need = cogs_k_kmeans_ws(T, PD, 1, &ns);
     if (!ws || ws_bytes < need) return COGS_E_WORKSPACE;
     if (!feats || !q_draws || !idx || !zero_flag || !nearest2 || T <= 0 || K <= 0) return COGS_E_INVALID;
-    return cogs_k_kmeans_pp((hipStream_t)stream, dtype, feats, T, PD, K, first_row, q_draws, idx, zero_flag, nearest2, dist2, (float*)ws, ns);
+    return cogs_k_kmeans_pp((hipStream_t)stream, dtype, feats, T, PD, K, first_row, q_draws, idx, zero_flag, nearest2, dist2, (float*)ws, ws_bytes, ns);
 }
 cogs_status cogs_kmeans_pp(cogs_stream stream, int dtype, const void* feats, int T, int64_t PD, int K, int first_row,
                            const float* q_draws, int32_t* idx, int32_t* zero_flag, float* nearest2, void* ws, size_t ws_bytes) {

@@ -54,6 +54,7 @@
     X(delta_chunk, 1, "0: gated delta rule of prompts token by token instead of in chunks")                                 \
     X(delta_out_wave, 0, "1: read-outs of the gated delta rule normed by a wave per head at any width (same bits)")         \
     X(gemm_skinny, 1, "0: the decoder's few-row products through the general GEMM")                                         \
+    X(km_pp_form, 0, "> 0: k-means++ passes with 1 a row per workgroup (up to 300 rows), 3 by slices (0: chosen per size)")          \
     X(km_row_groups, 0, "> 0: row groups of the k-means distance pass (0: sized to fill the chip)")
 
 struct CogsDebug {
@@ -80,7 +81,7 @@ struct CogsDebug {
     // ... and the last cogs_preprocess_frames: 1 two passes, 2 vector tiles, else matrix products: 100 x 64-byte steps + 10 x patch rows of a band +
     // 16-row tiles of its source rows
     std::atomic<long long> preprocess_last_kernel{0};
-    // ... and the last cogs_kmeans_pp: kernels launched per centre, 1 or 3
+    // ... and the last cogs_kmeans_pp: 1 a row per workgroup, 3 by slices
     std::atomic<long long> km_pp_last_launches{0};
 };
 extern CogsDebug g_cogs_debug;     // capi.hip

@@ -1,7 +1,7 @@
 // Time-aware k-means device steps (model/kmeans_with_time.py:4-137). The host keeps the reference's RNG draws
 // (random.randint / torch.multinomial on the CPU generator); everything that touches the features runs here.
 //
-//   sqdist        partial[slice][t][k] = sum over the slice's 512 columns of (x[t,j]-c[k,j])^2   (:48,:73  torch.cdist)
+//   sqdist        partial[t][slice][k] = sum over the slice's 512 columns of (x[t,j]-c[k,j])^2   (:48,:73  torch.cdist)
 //   reduce+assign dist2 = sum of the slice partials (fp64), per-row min-max of feature/time distances,
 //                 sqrt(nf^2 + alpha nt^2), argmin                                                   (:76-104)
 //   members       member lists per cluster, empty clusters -> reseed rows from the host-drawn pool    (:107-120)
@@ -42,6 +42,14 @@ enum { CTL_USED = 0,      // reseed-pool entries consumed so far
        CTL_MARGIN = 6,    // bits(+inf) - bits(min over rows and iterations of the decision margin) (reduce_assign_kernel)
        CTL_NEAR = 7,      // rows (summed over iterations) whose margin is below NEAR_TIE
        CTL_WORDS = 8 };
+// ... and of the seeding (in the same place)
+constexpr int KPP_C = 4;      // rows a pass measures at most
+enum { KPP_DONE_ROWS = 0,     // rows measured so far (workgroups that have finished)
+       KPP_M = 1,             // centres drawn
+       KPP_END = 2,           // all of them
+       KPP_N = 3,             // rows of the next pass: the newest centre, then the guesses (the rest of them repeat the newest centre)
+       KPP_ROWS = 4 };        // ... KPP_ROWS + KPP_C words in all
+static_assert(KPP_ROWS + KPP_C <= CTL_WORDS, "");
 constexpr float NEAR_TIE = 1e-3f;   // below this the reference's own sgemm rounding decides a row
 
 constexpr int SL = 512;       // columns per slice
@@ -83,7 +91,7 @@ __global__ __launch_bounds__(256, 4) void sqdist_kernel(const T* __restrict__ x,
                                                         int Ktot, float* __restrict__ partial, const int* __restrict__ ctl, const int* __restrict__ keep) {
     extern __shared__ __attribute__((aligned(16))) char smem_raw[];
     float* cs = reinterpret_cast<float*>(smem_raw);
-    if (ctl && (ctl[CTL_ABORT] | ctl[CTL_DONE])) return;   // speculatively queued iteration behind the last one
+    if (ctl && (centre_rows ? ctl[KPP_END] : ctl[CTL_ABORT] | ctl[CTL_DONE])) return;   // queued behind the last iteration, or the last draw
     const int lane = threadIdx.x & 63, wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const long j = (long)blockIdx.x * SL + lane * 8;
     const bool in = j < PD;
@@ -141,8 +149,8 @@ __global__ __launch_bounds__(256, 4) void sqdist_kernel(const T* __restrict__ x,
         for (int e = 0; e < 8; ++e) xab[e] = f32x2{xn[0][e], xn[1][e]};
         if (t + 8 < r_hi) load_rows(t + 8);
         const bool live_b = t + 4 < r_hi;
-        float* pa = partial + ((long)blockIdx.x * Tn + t) * Ktot + k0;
-        float* pb = pa + 4 * (long)Ktot;
+        float* pa = partial + ((long)t * gridDim.x + blockIdx.x) * Ktot + k0;
+        float* pb = pa + 4 * (long)gridDim.x * Ktot;
         unsigned k = (unsigned)kperm;
 #pragma unroll 1
         for (int m = 0; m < KB; m += 4, k += 4) {
@@ -177,10 +185,10 @@ __global__ __launch_bounds__(256, 4) void sqdist_kernel(const T* __restrict__ x,
     }
 }
 
-// fp64 sum over the slices of partial[slice][t][k] for row t, by the lanes of one workgroup: lane (g, k) owns centre k
+// fp64 sum over the slices of partial[t][slice][k] for row t (one run of memory), by the lanes of one workgroup: lane (g, k) owns centre k
 // and slice group g; groups are combined in a fixed order. Result in d2s[k] (LDS, fp32 like torch.cdist's output).
 // keep[k] (keep nullable): the centre has not moved, kept[t][k] has its sum
-__device__ __forceinline__ void reduce_row(const float* __restrict__ partial, int nslices, int Tn, int K, int t,
+__device__ __forceinline__ void reduce_row(const float* __restrict__ partial, int nslices, int K, int t,
                                            float* d2s, double* scratch /* [groups][kp]: 256 doubles */, const int* __restrict__ keep, const float* kept) {
     const int tid = threadIdx.x;
     for (int kc = 0; kc < K; kc += 64) {
@@ -192,8 +200,8 @@ __device__ __forceinline__ void reduce_row(const float* __restrict__ partial, in
         double s = 0.0;
         const bool moved = k < Kc && !(keep && keep[kc + k]);
         if (moved) {
-            const float* pp = partial + (long)t * K + kc + k;
-            const long stride = (long)Tn * K;
+            const float* pp = partial + (long)t * nslices * K + kc + k;
+            const long stride = K;
             int sl = g;
             for (; sl + 7 * G < nslices; sl += 8 * G) {       // eight loads in flight, added in slice order
                 float v[8];
@@ -227,7 +235,7 @@ __global__ __launch_bounds__(256) void reduce_assign_kernel(const float* __restr
     if (ctl && (ctl[CTL_ABORT] | ctl[CTL_DONE])) return;
     float* d2s = reinterpret_cast<float*>(scratch + 256);            // [K]
     const int t = blockIdx.x;
-    reduce_row(partial, nslices, Tn, K, t, d2s, scratch, keep, dist2_out);
+    reduce_row(partial, nslices, K, t, d2s, scratch, keep, dist2_out);
     const int tid = threadIdx.x;
     if (dist2_out)
         for (int k = tid; k < K; k += 256) dist2_out[(long)t * K + k] = d2s[k];
@@ -297,153 +305,294 @@ __global__ __launch_bounds__(256) void reduce_assign_kernel(const float* __restr
     }
 }
 
-// k-means++ draw (:53-60) on the device: probs = (sqrt(nearest2))^2 as the reference computes them from cdist's distances,
+// The whole seeding, several centres a pass. A draw needs the distances to every centre in front of it, but which row it falls on can mostly be told
+// without the last of them: nearest2 only shrinks, and a new centre shrinks it for the rows of its own scene alone. So a pass over the features measures
+// the newest centre and, beside it, the rows that the next draws would fall on if nearest2 stayed as it is; the workgroup that finishes last draws
+// centres for as long as the newest one is among those measured, and leaves the next pass's rows. What is drawn, from which distances and in which
+// order is what a pass per centre draws: a guess that does not come true has been measured in vain. Passes queued behind the last draw return at once.
+// 256 frames of some twenty scenes, 18 centres: 5.4 passes of 4 rows on the average instead of 17.
+struct KppArgs {
+    int Tn, K;
+    float* nearest2; const float* q; int* idx; int* zero_flag;
+    int* state;
+    float* d2; int ldd2;            // the pass's distances [Tn][ldd2]
+    float* dist2;                   // nullable [Tn][K]
+};
+
+// sum or maximum over a wave in every lane, lanes 32, 16, 8, .. 1 apart (a register move each; through LDS a draw was 0.6 us longer)
+template <typename F>
+__device__ __forceinline__ void wave_join(F&& join) {
+    join([](unsigned v) { const auto r = __builtin_amdgcn_permlane32_swap(v, v, false, false); return (threadIdx.x & 32) ? (unsigned)r[0] : (unsigned)r[1]; });
+    join([](unsigned v) { const auto r = __builtin_amdgcn_permlane16_swap(v, v, false, false); return (threadIdx.x & 16) ? (unsigned)r[0] : (unsigned)r[1]; });
+    join([](unsigned v) { return __float_as_uint(lane_xor_dpp<8>(__uint_as_float(v))); });
+    join([](unsigned v) { return __float_as_uint(lane_xor_dpp<4>(__uint_as_float(v))); });
+    join([](unsigned v) { return __float_as_uint(lane_xor_dpp<2>(__uint_as_float(v))); });
+    join([](unsigned v) { return __float_as_uint(lane_xor_dpp<1>(__uint_as_float(v))); });
+}
+__device__ __forceinline__ double wave_sum_f64(double s) {
+    wave_join([&](auto&& other) {
+        const unsigned long long b = __builtin_bit_cast(unsigned long long, s);
+        s += __builtin_bit_cast(double, (unsigned long long)other((unsigned)(b >> 32)) << 32 | other((unsigned)b));
+    });
+    return s;
+}
+// a ratio and its row as one number: larger ratio first, NaN before all others like in torch.argmax, then the lower row; 0 is no row
+__device__ __forceinline__ unsigned long long ranked(float r, int t) {
+    const unsigned b = __float_as_uint(r + 0.f), up = r != r ? 0xffffffffu : b & 0x80000000u ? ~b : b | 0x80000000u;
+    return (unsigned long long)up << 32 | ~(unsigned)t;
+}
+__device__ __forceinline__ unsigned long long wave_max_u64(unsigned long long v) {
+    wave_join([&](auto&& other) {
+        const unsigned long long o = (unsigned long long)other((unsigned)(v >> 32)) << 32 | other((unsigned)v);
+        v = v > o ? v : o;
+    });
+    return v;
+}
+__device__ __forceinline__ int ranked_row(unsigned long long v, int none) { return v == 0 ? none : (int)~(unsigned)v; }
+
+// the rows that the draws behind centre m would fall on, a wave each (guess(t): what is known of row t's nearest2)
+template <typename F>
+__device__ __forceinline__ void kpp_guess(const KppArgs& p, int m, int newest, int tid, int waves, F&& guess) {
+    const int lane = tid & 63, wid = tid >> 6, n = max(1, min(min(KPP_C, p.ldd2), p.K - m));      // (the last centre's distances are not needed)
+    for (int j = wid; j < KPP_C; j += waves) {
+        unsigned long long best = 0;
+        if (j > 0 && j < n) {
+            const float* q = p.q + (long)(m + j - 2) * p.Tn;
+            for (int t = lane; t < p.Tn; t += 64) {
+                const float r = guess(t) / q[t];
+                if (t != newest && r > 0.f) best = max(best, ranked(r, t));
+            }
+            best = wave_max_u64(best);
+        }
+        if (lane == 0) p.state[KPP_ROWS + j] = ranked_row(best, newest);
+    }
+    if (tid == 0) p.state[KPP_N] = n;
+}
+
+// k-means++ draws (:53-60) on the device: probs = (sqrt(nearest2))^2 as the reference computes them from cdist's distances,
 // normalised by their sum; torch.multinomial(probs, 1) on the CPU IS argmax(probs / q), q ~ Exponential(1) one draw per
 // element from the CPU generator (ATen multinomial, n_sample == 1) -- the host hands those draws over. A zero sum (every
 // row coincides with a chosen centre) is the reference's random.randint branch: flagged, the host then takes the step-wise
 // path. The sum runs in fp64 in a fixed order (torch's own fp32 summation order is not reproduced: the sum
 // is a common divisor of all ratios and only moves the argmax between ratios closer than a few ulps).
-// Run by 256 threads, of kpp_select_kernel or of the workgroup that measured the last row (others wrote nearest2: read past the caches).
-__device__ __forceinline__ void kpp_select(float* nearest2, const float* __restrict__ q, int Tn, int* __restrict__ idx_out, int* __restrict__ zero_flag,
-                                           int tid, double* red, float* rv, int* ri) {
-    const int lane = tid & 63, wid = tid >> 6;
-    const bool on = tid < 256;
-    auto load = [&](int t) { return __hip_atomic_load(nearest2 + t, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); };
-    const float own = on && tid < Tn ? load(tid) : 0.f;          // a thread's first row; further ones are read twice
-    auto near_of = [&](int t) { return t == tid ? own : load(t); };
-    const float own_q = on && tid < Tn ? q[tid] : 1.f;
-    double sum = 0.0;
-    for (int t = on ? tid : Tn; t < Tn; t += 256) {
-        const float d = sqrtf(near_of(t));
-        sum += (double)__fmul_rn(d, d);
-    }
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) sum += __shfl_xor(sum, o, 64);
-    if (on && lane == 0) red[wid] = sum;
-    __syncthreads();
-    const float total = (float)((red[0] + red[1]) + (red[2] + red[3]));
-    if (total == 0.f) {
-        if (tid == 0) { *zero_flag = 1; *idx_out = 0; }
-        return;
-    }
-    float best = -INFINITY;
-    int bi = 0x7fffffff;
-    for (int t = on ? tid : Tn; t < Tn; t += 256) {       // ascending t per thread: the first maximum is kept
-        const float d = sqrtf(near_of(t));
-        const float r = __fdiv_rn(__fdiv_rn(__fmul_rn(d, d), total), t == tid ? own_q : q[t]);
-        if (r > best || (r != r && best == best)) { best = r; bi = t; }      // NaN counts as the maximum, like torch.argmax
-    }
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) {
-        const float ob = __shfl_xor(best, o, 64);
-        const int oi = __shfl_xor(bi, o, 64);
-        const bool take = (ob > best) || (ob != ob && best == best) || ((ob == best || (ob != ob && best != best)) && oi < bi);
-        if (take) { best = ob; bi = oi; }
-    }
-    if (on && lane == 0) { rv[wid] = best; ri[wid] = bi; }
-    __syncthreads();
-    if (tid == 0) {
-        float b = rv[0]; int i = ri[0];
-        for (int w = 1; w < 4; ++w) {
-            const float ob = rv[w]; const int oi = ri[w];
-            const bool take = (ob > b) || (ob != ob && b == b) || ((ob == b || (ob != ob && b != b)) && oi < i);
-            if (take) { b = ob; i = oi; }
-        }
-        *idx_out = i == 0x7fffffff ? 0 : i;
-    }
-}
-__global__ __launch_bounds__(256) void kpp_select_kernel(float* nearest2, const float* __restrict__ q, int Tn, int* idx_out, int* zero_flag, int first_row) {
+// Run by the workgroup that measured the last row (others wrote d2: read past the caches), the rows by its first 256 threads. It is all latency: what a
+// thread's first two rows need for the draws of a pass is loaded at once (in turn, with the waves' sums through LDS: 3.7 us a draw).
+template <int THREADS>
+__device__ __forceinline__ void kpp_draw(const KppArgs& p) {
     __shared__ double red[4];
-    __shared__ float rv[4];
-    __shared__ int ri[4];
-    if (first_row >= 0 && threadIdx.x == 0) idx_out[-1] = first_row;      // step 1 also records the caller's first centre
-    kpp_select(nearest2, q, Tn, idx_out, zero_flag, threadIdx.x, red, rv, ri);
+    __shared__ unsigned long long rv[4];
+    constexpr int R = 2;
+    __shared__ float near_s[256 * R], d2_s[KPP_C][256 * R], q_s[KPP_C][256 * R];        // (of rows that are all one thread's but in kpp_guess)
+    const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
+    const bool on = tid < 256;
+    int m = p.state[KPP_M], newest = p.state[KPP_ROWS], rows[KPP_C], c = 0;
+    const int n = p.state[KPP_N], m0 = m;
+#pragma unroll
+    for (int j = 0; j < KPP_C; ++j) rows[j] = p.state[KPP_ROWS + j];
+    auto load_d2 = [&](int t, int j) { return __hip_atomic_load(p.d2 + (long)t * p.ldd2 + j, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); };
+    if (on) {
+        float d2[R][KPP_C], q[R][KPP_C], near[R];
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            const int t = min(tid + 256 * r, p.Tn - 1);          // (rows and draws past the end repeat the last one and are not used)
+#pragma unroll
+            for (int j = 0; j < KPP_C; ++j) {
+                d2[r][j] = load_d2(t, min(j, n - 1));
+                q[r][j] = p.q[(long)min(m - 1 + j, p.K - 2) * p.Tn + t];
+            }
+            near[r] = m == 1 ? 0.f : p.nearest2[t];
+        }
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+#pragma unroll
+            for (int j = 0; j < KPP_C; ++j) {
+                d2_s[j][tid + 256 * r] = d2[r][j];
+                q_s[j][tid + 256 * r] = q[r][j];
+            }
+            near_s[tid + 256 * r] = near[r];
+        }
+    }
+    auto d2_of = [&](int t) { return t < 256 * R ? d2_s[c][t] : load_d2(t, c); };
+    auto q_of = [&](int t) { return t < 256 * R ? q_s[m - m0][t] : p.q[(long)(m - 1) * p.Tn + t]; };
+    auto near_of = [&](int t) -> float& { return t < 256 * R ? near_s[t] : p.nearest2[t]; };
+    bool end = false;
+    for (;;) {
+        double sum = 0.0;
+        for (int t = on ? tid : p.Tn; t < p.Tn; t += 256) {
+            const float d2 = d2_of(t), near = m > 1 ? fminf(near_of(t), d2) : d2;
+            near_of(t) = near;
+            if (p.dist2) p.dist2[(long)t * p.K + m - 1] = d2;
+            const float d = sqrtf(near);
+            sum += (double)__fmul_rn(d, d);
+        }
+        sum = wave_sum_f64(sum);
+        if (on && lane == 0) red[wid] = sum;
+        __syncthreads();
+        const float total = (float)((red[0] + red[1]) + (red[2] + red[3]));
+        if (total == 0.f) {                                      // nothing is drawn from here on
+            if (tid == 0) *p.zero_flag = 1;
+            for (int k = m + tid; k < p.K; k += THREADS) p.idx[k] = 0;
+            if (p.dist2)
+                for (int t = tid; t < p.Tn; t += THREADS)
+                    for (int k = m; k < p.K - 1; ++k) p.dist2[(long)t * p.K + k] = 0.f;
+            end = true;
+            break;
+        }
+        unsigned long long best = 0;
+        for (int t = on ? tid : p.Tn; t < p.Tn; t += 256) {
+            const float d = sqrtf(near_of(t));
+            best = max(best, ranked(__fdiv_rn(__fdiv_rn(__fmul_rn(d, d), total), q_of(t)), t));
+        }
+        best = wave_max_u64(best);
+        if (on && lane == 0) rv[wid] = best;
+        __syncthreads();
+        newest = ranked_row(max(max(rv[0], rv[1]), max(rv[2], rv[3])), 0);
+        if (tid == 0) p.idx[m] = newest;
+        if (++m == p.K) { end = true; break; }
+        c = -1;
+#pragma unroll
+        for (int j = KPP_C - 1; j >= 0; --j)
+            if (j < n && rows[j] == newest) c = j;
+        if (c < 0 || m - m0 == KPP_C) break;
+    }
+    if (tid == 0) {
+        p.state[KPP_M] = m;
+        p.state[KPP_END] = end;
+        p.state[KPP_DONE_ROWS] = 0;                              // for the next pass
+    }
+    if (end) return;
+    for (int t = tid; on && t < min(256 * R, p.Tn); t += 256) p.nearest2[t] = near_s[t];
+    __threadfence_block();                                       // (further rows of nearest2 were written by other threads of the workgroup)
+    __syncthreads();
+    kpp_guess(p, m, newest, tid, THREADS / 64, near_of);
 }
 
-// One k-means++ step (:46-60) of the whole-seeding call: workgroup t measures row t against the newest centre, a slice of 512
-// columns per wave at a time, folds the distance into nearest2[t], and the workgroup that finishes last draws the next centre. The sums are
-// those of sqdist_kernel and reduce_min_kernel, value by value: fp32 within a slice (lanes 32, 16, then 1, 2, 4, 8 apart), the
-// slices in fp64 by one wave's lanes. Bound by what a CU takes in (its row and the centre's, 60 bytes a nanosecond): a step of
-// [256, 179 200] bf16 is 23 us; partial sums by slices (sqdist), their reduction and the draw were three launches, 31 us.
+// the first pass's rows: no distance is known yet.
+__global__ __launch_bounds__(256) void kpp_start_kernel(KppArgs p, int first_row) {
+    if (threadIdx.x == 0) {
+        p.state[KPP_DONE_ROWS] = 0;
+        p.state[KPP_M] = 1;
+        p.state[KPP_END] = p.K < 2;
+        *p.zero_flag = 0;
+        p.idx[0] = first_row;
+    }
+    kpp_guess(p, 1, first_row, threadIdx.x, 4, [](int) { return 1.f; });
+}
+
+// One pass (:46-60) with a row per workgroup: workgroup t measures row t against up to KPP_C others, a slice of 512 columns per wave at a time. The sums
+// are those of sqdist_kernel and kpp_reduce_kernel, value by value: fp32 within a slice (lanes 32, 16, then 1, 2, 4, 8 apart), the
+// slices in fp64 by one wave's lanes. Bound by what a CU takes in (its row and the others', which its XCD's L2 has) and by the products' sums.
 constexpr int KPP_T = 1024;
-template <typename T>
-__global__ __launch_bounds__(KPP_T) void kpp_step_kernel(const T* __restrict__ x, int Tn, long PD, int nslices, const int* __restrict__ centre_from,
-                                                         int centre_row, int first, float* nearest2, const float* __restrict__ q, int* idx_out,
-                                                         int* zero_flag, int* done, float* dist2, int ldd) {
-    extern __shared__ __attribute__((aligned(16))) char smem_raw[];
-    float* const sums = reinterpret_cast<float*>(smem_raw);                                                     // [nslices]
-    __shared__ double red[4];
-    __shared__ float rv[4];
-    __shared__ int ri[4], last;
-    const int tid = threadIdx.x, lane = tid & 63, wid = __builtin_amdgcn_readfirstlane(tid >> 6);
-    constexpr int NW = KPP_T / 64, U = 4;
+template <typename T, int C>
+__device__ __forceinline__ void kpp_measure(const T* __restrict__ x, const KppArgs& p, long PD, int nslices, float* sums) {
+    const int lane = threadIdx.x & 63, wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    constexpr int NW = KPP_T / 64, U = C == 1 ? 4 : sizeof(T) == 2 ? 3 : 1;
     const T* xr = x + (long)blockIdx.x * PD + lane * 8;
-    const T* cr = x + (long)(centre_from ? *centre_from : centre_row) * PD + lane * 8;
+    const T* cr[C];
+#pragma unroll
+    for (int j = 0; j < C; ++j) cr[j] = x + (long)__builtin_amdgcn_readfirstlane(p.state[KPP_ROWS + j]) * PD + lane * 8;
+    const int row = lane >> 4, mine = ((row & 1) << 1) + (row >> 1);          // 16-lane row -> its row's sum: 0, 2, 1, 3
     // a row is a whole number of memory interleaves away from the next as often as not: every workgroup starts at another slice
     const int turn = (int)((unsigned)blockIdx.x * 61u % (unsigned)nslices);
     auto slice = [&](int i) { const int sl = i + turn; return sl < nslices ? sl : sl - nslices; };
     for (int s0 = wid; s0 < nslices; s0 += NW * U) {
-        float a[U][8], c[U][8];
+        float a[U][8], c[U][C][8];
 #pragma unroll
         for (int u = 0; u < U; ++u) {                            // (slices and columns past the end repeat what is there and are not used)
             const long j = (long)slice(min(s0 + NW * u, nslices - 1)) * SL;
             const long at = j + lane * 8 < PD ? j : PD - 8 - lane * 8;
             ld8_f<T>(xr + at, a[u]);
-            ld8_f<T>(cr + at, c[u]);
+#pragma unroll
+            for (int k = 0; k < C; ++k) ld8_f<T>(cr[k] + at, c[u][k]);
         }
 #pragma unroll
         for (int u = 0; u < U; ++u) {
             if (s0 + NW * u >= nslices) break;
             const int sl = slice(s0 + NW * u);
-            float s = 0.f;
+            float s[C];
 #pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const float d0 = a[u][e] - c[u][e], d1 = a[u][4 + e] - c[u][4 + e];
-                s = fmaf(d0, d0, s);
-                s = fmaf(d1, d1, s);
+            for (int k = 0; k < C; ++k) {
+                s[k] = 0.f;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const float d0 = a[u][e] - c[u][k][e], d1 = a[u][4 + e] - c[u][k][4 + e];
+                    s[k] = fmaf(d0, d0, s[k]);
+                    s[k] = fmaf(d1, d1, s[k]);
+                }
+                if ((long)sl * SL + lane * 8 >= PD) s[k] = 0.f;
             }
-            if ((long)sl * SL + lane * 8 >= PD) s = 0.f;
-            s = swap32_sum(s, s);
-            s = row16_sum(swap16_sum(s, s));
-            if (lane == 0) sums[sl] = s;
+            if constexpr (C == 1) {
+                float v = swap32_sum(s[0], s[0]);
+                v = row16_sum(swap16_sum(v, v));
+                if (lane == 0) sums[sl] = v;
+            } else {
+                const float v = row16_sum(swap16_sum(swap32_sum(s[0], s[1]), swap32_sum(s[2], s[3])));
+                if ((lane & 15) == 0) sums[mine * nslices + sl] = v;
+            }
         }
     }
     __syncthreads();
-    if (wid == 0) {
+    if (wid < C) {
         double d = 0.0;
-        for (int sl = lane; sl < nslices; sl += 64) d += (double)sums[sl];
-#pragma unroll
-        for (int o = 32; o > 0; o >>= 1) d += __shfl_xor(d, o, 64);
-        if (lane == 0) {
-            const float d2 = (float)d;
-            if (dist2) dist2[(long)blockIdx.x * ldd] = d2;
-            __hip_atomic_store(nearest2 + blockIdx.x, first ? d2 : fminf(nearest2[blockIdx.x], d2), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            last = __hip_atomic_fetch_add(done, 1, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) == Tn - 1;
-        }
+        for (int sl = lane; sl < nslices; sl += 64) d += (double)sums[wid * nslices + sl];
+        d = wave_sum_f64(d);
+        if (lane == 0) __hip_atomic_store(p.d2 + (long)blockIdx.x * p.ldd2 + wid, (float)d, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
+}
+
+// true in every thread of the workgroup that calls it last; d2 of all of them is there then
+__device__ __forceinline__ bool kpp_last(const KppArgs& p) {
+    __shared__ int last;
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");             // every wave's own stores (past the caches) have arrived
     __syncthreads();
-    if (!last) return;
-    if (tid == 0) {
-        *done = 0;                                               // for the next step's launch
-        if (first) idx_out[-1] = centre_row;                     // step 1 also records the caller's first centre
+    if (threadIdx.x == 0) last = __hip_atomic_fetch_add(p.state + KPP_DONE_ROWS, 1, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) == p.Tn - 1;
+    __syncthreads();
+    return last;
+}
+
+template <typename T>
+__global__ __launch_bounds__(KPP_T) void kpp_pass_kernel(const T* __restrict__ x, KppArgs p, long PD, int nslices) {
+    extern __shared__ __attribute__((aligned(16))) char smem_raw[];
+    float* const sums = reinterpret_cast<float*>(smem_raw);                                                     // [KPP_C][nslices]
+    if (p.state[KPP_END]) return;
+    if (p.state[KPP_N] == 1) kpp_measure<T, 1>(x, p, PD, nslices, sums);
+    else kpp_measure<T, KPP_C>(x, p, PD, nslices, sums);
+    if (kpp_last(p)) kpp_draw<KPP_T>(p);
+}
+
+// ... of a pass that sqdist_kernel has measured by slices, partial [row][slice][ldd2]: a workgroup per row, a wave per measured row, lanes over slices
+__global__ __launch_bounds__(256) void kpp_reduce_kernel(const float* __restrict__ partial, KppArgs p, int nslices) {
+    if (p.state[KPP_END]) return;
+    constexpr int U = 8;
+    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+    if (wid < p.ldd2) {
+        double s = 0.0;
+        for (int s0 = lane; s0 < nslices; s0 += 64 * U) {        // U loads in flight, added in slice order
+            float v[U];
+#pragma unroll
+            for (int u = 0; u < U; ++u) v[u] = s0 + 64 * u < nslices ? partial[((long)blockIdx.x * nslices + s0 + 64 * u) * p.ldd2 + wid] : 0.f;
+#pragma unroll
+            for (int u = 0; u < U; ++u) s += (double)v[u];
+        }
+        s = wave_sum_f64(s);
+        if (lane == 0) __hip_atomic_store(p.d2 + (long)blockIdx.x * p.ldd2 + wid, (float)s, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
-    kpp_select(nearest2, q, Tn, idx_out, zero_flag, tid, red, rv, ri);
+    if (kpp_last(p)) kpp_draw<256>(p);
 }
 
 // k-means++ step (:46-60): nearest2[t] = min(nearest2[t], dist2 to the newest centre) (first: plain store)
 __global__ __launch_bounds__(256) void reduce_min_kernel(const float* __restrict__ partial, int nslices, int Tn, int first,
-                                                         float* __restrict__ nearest2, float* __restrict__ dist2 = nullptr, int ldd = 0) {
+                                                         float* __restrict__ nearest2) {
     // one wave per row: lanes over slices, fp64 butterfly
     const int lane = threadIdx.x & 63;
     const int t = blockIdx.x * 4 + (threadIdx.x >> 6);
     if (t >= Tn) return;
     double s = 0.0;
-    for (int sl = lane; sl < nslices; sl += 64) s += (double)partial[(long)sl * Tn + t];
+    for (int sl = lane; sl < nslices; sl += 64) s += (double)partial[(long)t * nslices + sl];
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
     if (lane == 0) {
         const float d2 = (float)s;
-        if (dist2) dist2[(long)t * ldd] = d2;
         nearest2[t] = first ? d2 : fminf(nearest2[t], d2);
     }
 }
@@ -481,24 +630,33 @@ __global__ __launch_bounds__(1024) void members_kernel(const int64_t* __restrict
         before[t] = c;
     }
     __syncthreads();
-    if (tid == 0) {
+    // one wave: where every cluster's rows begin, and the empty clusters in ascending order, 64 clusters at a time
+    if (tid < 64) {
         int o = 0, ne = 0;
         const int used = ctl ? ctl[CTL_USED] : 0;
-        offs[0] = 0;
-        for (int k = 0; k < K; ++k) {
-            const int n = cnt[k];
-            if (n == 0) {
-                if (reseed_in) reseed_rows[k] = reseed_in[k];
-                else if (pool && used + ne < pool_len) reseed_rows[k] = pool[used + ne];
-                else reseed_rows[k] = 0;
-                if (keep) keep[k] = 0;
-                ++ne;
+        for (int k0 = 0; k0 < K; k0 += 64) {
+            const int k = k0 + tid, n = k < K ? cnt[k] : 0;
+            int upto = n;                                        // rows of the clusters up to this one
+#pragma unroll
+            for (int d = 1; d < 64; d *= 2) {
+                const int v = __shfl_up(upto, d, 64);
+                if (tid >= d) upto += v;
             }
-            cnt[k] = o;            // becomes the cluster's write cursor base
-            o += n;
-            offs[k + 1] = o;
+            const unsigned long long none = __ballot(k < K && n == 0);
+            if (k < K) {
+                if (n == 0) {
+                    const int e = used + ne + __popcll(none & ((1ull << tid) - 1ull));
+                    reseed_rows[k] = reseed_in ? reseed_in[k] : pool && e < pool_len ? pool[e] : 0;
+                    if (keep) keep[k] = 0;
+                }
+                cnt[k] = o + upto - n;                           // becomes the cluster's write cursor base
+                offs[k + 1] = o + upto;
+            }
+            o += __shfl(upto, 63, 64);
+            ne += __popcll(none);
         }
-        if (ctl) {
+        if (tid == 0) offs[0] = 0;
+        if (tid == 0 && ctl) {
             ctl[CTL_EMPTY] = ne;
             if (!reseed_in && ne > 0) {
                 if (!pool || used + ne > pool_len) ctl[CTL_ABORT] = 1;      // abort: this iteration must not commit
@@ -511,6 +669,7 @@ __global__ __launch_bounds__(1024) void members_kernel(const int64_t* __restrict
     for (int t = tid; t < Tn; t += nt) {
         const int c = a[t];
         int r = 0;
+#pragma unroll 8
         for (int u = 0; u < t; ++u) r += (a[u] == c) ? 1 : 0;
         members[cnt[c] + r] = t;
     }
@@ -597,7 +756,7 @@ __global__ __launch_bounds__(256) void update_kernel(const T* __restrict__ x, lo
 
 // one workgroup: centre times, shift norms (scratch [2K]: feature-shift norm, squared time shift), total movement.
 // status (nullable, host-mapped): {shift, reseeds used, abort, empty clusters} for the Lloyd loop's one read per iteration
-constexpr int UF_T = 1024;
+constexpr int UF_T = 1024, UF_K = 128;
 __global__ __launch_bounds__(UF_T) void update_final_kernel(const float* __restrict__ ts, int K,
                                                            const int* __restrict__ offs, const int* __restrict__ members,
                                                            const int* __restrict__ reseed_rows, int* __restrict__ ctl,
@@ -607,6 +766,7 @@ __global__ __launch_bounds__(UF_T) void update_final_kernel(const float* __restr
                                                            volatile int* __restrict__ status, int Tn_lds, float tol, const int* __restrict__ watch) {
     extern __shared__ __attribute__((aligned(16))) char smem_raw[];
     float* mts = reinterpret_cast<float*>(smem_raw);      // [Tn] time stamps in member order (0 floats when Tn_lds == 0)
+    __shared__ float moved[2 * UF_K];                     // as scratch, of the first UF_K clusters: what thread 0 adds up at the end, one after the other
     if (ctl && ctl[CTL_DONE]) return;                     // a speculatively queued iteration behind the converged one
     const bool aborted = ctl && ctl[CTL_ABORT];
     const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
@@ -620,7 +780,10 @@ __global__ __launch_bounds__(UF_T) void update_final_kernel(const float* __restr
             for (int b = lane; b < nblk; b += 64) s += (double)shift_partial[(long)b * K + k];
 #pragma unroll
             for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
-            if (lane == 0) scratch[k] = sqrtf((float)s);
+            if (lane == 0) {
+                const float v = scratch[k] = sqrtf((float)s);
+                if (k < UF_K) moved[k] = v;
+            }
         }
         for (int k = UF_T - 1 - (int)threadIdx.x; k < K; k += UF_T) {      // times: one thread per cluster, its members in order (the last waves first: they
             float tsum = 0.f;                                                       // have the fewest shifts to sum)
@@ -630,6 +793,7 @@ __global__ __launch_bounds__(UF_T) void update_final_kernel(const float* __restr
             const float nt = e0 > b0 ? tsum / (float)(e0 - b0) : ts[reseed_rows[k]];
             const float d = nt - cts[k];
             scratch[K + k] = d * d;
+            if (k < UF_K) moved[UF_K + k] = d * d;
             cts[k] = nt;
         }
     }
@@ -638,7 +802,7 @@ __global__ __launch_bounds__(UF_T) void update_final_kernel(const float* __restr
         float total = 0.f;
         if (!aborted) {
             float f = 0.f, tt = 0.f;
-            for (int i = 0; i < K; ++i) { f += scratch[i]; tt += scratch[K + i]; }
+            for (int i = 0; i < K; ++i) { f += i < UF_K ? moved[i] : scratch[i]; tt += i < UF_K ? moved[UF_K + i] : scratch[K + i]; }
             total = f + sqrtf(tt);
             shift_out[0] = total;
         }
@@ -656,11 +820,10 @@ __global__ __launch_bounds__(UF_T) void update_final_kernel(const float* __restr
     }
 }
 
-// what a loop starts from: n words of zeros at a and one at b (nullable), ones and zeros at keep. One launch: memsets of a few words are one to three of 1 to
+// what a loop starts from: zeros at ctl, ones and zeros at keep. One launch: memsets of a few words are one to three of 1 to
 // 5 us and a gap (256 frames of 50 tokens: 28 us in front of the Lloyd loop, 5 so)
-__global__ __launch_bounds__(256) void start_kernel(int* a, int n, int* b, int* keep, int K, int known) {
-    for (int i = threadIdx.x; i < n; i += 256) a[i] = 0;
-    if (b && threadIdx.x == 0) *b = 0;
+__global__ __launch_bounds__(256) void start_kernel(int* ctl, int* keep, int K, int known) {
+    if (threadIdx.x < CTL_WORDS) ctl[threadIdx.x] = 0;
     for (int k = threadIdx.x; k < K; k += 256) keep[k] = k < known;
 }
 
@@ -762,7 +925,7 @@ int cogs_k_select_near(hipStream_t st, const float* dist2, const int64_t* assign
     return COGS_LAUNCH_CHECK();
 }
 
-// ---- workspace: [A] max(sqdist slice partials [ns][T][K], update shift partials [nblk][K]) floats, then the member
+// ---- workspace: [A] max(sqdist slice partials [T][ns][K], update shift partials [nblk][K]) floats, then the member
 // lists (offs [K+1], members [T]), the update scratch [2K], and the Lloyd loop's own state: dist2 [T][K] floats,
 // reseed rows [K], ctl [CTL_WORDS], reseed pool [POOL_MAX], the last assignments [T], centres that have not moved [K] ints
 constexpr int POOL_MAX = 4096;
@@ -898,7 +1061,7 @@ int cogs_k_kmeans_pp_step(hipStream_t st, int dtype, const void* feats, int T, l
     const KmWs w = carve(ws, T, PD, 1);
     const int rc = sqdist_partials(st, dtype, feats, T, PD, nullptr, nullptr, row, 1, w.partial, nslices);
     if (rc != COGS_OK) return rc;
-    hipLaunchKernelGGL(reduce_min_kernel, dim3((T + 3) / 4), dim3(256), 0, st, w.partial, nslices, T, first, nearest2, nullptr, 0);
+    hipLaunchKernelGGL(reduce_min_kernel, dim3((T + 3) / 4), dim3(256), 0, st, w.partial, nslices, T, first, nearest2);
     if (COGS_LAUNCH_CHECK() != COGS_OK) return COGS_E_HIP;
     if (probs_host) {
         if (hipMemcpyAsync(probs_host, nearest2, (size_t)T * 4, hipMemcpyDeviceToHost, st) != hipSuccess) return COGS_E_HIP;
@@ -907,58 +1070,58 @@ int cogs_k_kmeans_pp_step(hipStream_t st, int dtype, const void* feats, int T, l
     return COGS_OK;
 }
 
-// Which form a centre of the whole seeding takes. One launch has a workgroup, and so a CU's intake, per row: it wins where rows are
-// about as many as CUs, or short. Fewer long rows leave CUs idle, more rows than CUs read the centre again for every round, where
-// sqdist keeps it in LDS. Time of three launches a centre over one (K = 18), by rows:        (MI355X; fp32 rows are twice as long)
-//                     T = 24    48    80   120   160   200   256   257   320   400
-//   bf16,  28 KB          1.7   1.6   1.6   1.4   1.2   1.2   1.1   1.2   1.05  1.1
-//   bf16,  84 KB          1.5   1.3   1.2   1.2   1.2   1.1   1.1   1.1   1.05  1.0
-//   bf16, 168 KB          1.2   1.0   1.1   1.1   1.2   1.2   1.1   0.95  0.88  0.94
-//   bf16, 350 KB          0.85  0.83  0.89  1.07  1.13  1.18  1.18  0.92  0.87  0.94
-//   bf16, 896 KB          0.55  0.69  0.82  1.01  1.11  1.20  1.18  0.82  0.77  0.86
-//   fp32, 168 KB          1.18  1.08  1.03  1.05  1.01  0.99  0.95  0.76  0.74  0.80
-//   fp32, 700 KB          0.65  0.63  0.81  0.94  1.02  1.09  1.09  0.78  0.80  0.75
+// Which form the passes of the whole seeding take. One launch has a workgroup, and so a CU's intake, per row: it wins where rows are
+// about as many as CUs, or short. Fewer long rows leave CUs idle, and long ones are read from L2 with up to four others by every workgroup, where
+// sqdist keeps those in LDS: [256, 179 200] bf16 35 to 39 us a pass, 21 and 15 in two launches; behind the last draw a pass is 2 us, or two of them.
+// Time of a seeding by slices over one by rows (18 centres of some scenes of twelve rows each, 6 up to 48 rows):        (MI355X)
+//                     T = 24    48    80   120   160   200   256   257   300
+//   bf16,  28 KB         1.32  1.24  1.28  1.35  1.38  1.40  1.40  1.35  1.32
+//   bf16,  84 KB         1.11  1.04  1.09  1.21  1.19  1.27  1.32  1.10  1.10
+//   bf16, 128 KB         0.94  1.00  0.99  1.08  1.11  1.14  1.20  0.99  0.99
+//   bf16, 168 KB         0.85  0.88  0.99  1.02  1.06  1.18  1.23  0.91  0.97
+//   bf16, 350 KB         0.62  0.68  0.76  0.86  0.94  1.00  1.05  0.73  0.82
+//   bf16, 896 KB         0.50  0.44  0.56  0.65  0.70  0.76  0.78  0.52  0.50
+//   fp32, 128 KB         1.07  1.03  1.06  1.08  1.01  1.07  1.12  1.02  0.99
+//   fp32, 350 KB         0.68  0.72  0.67  0.90  0.97  1.00  1.10  0.76  0.85
 static bool kpp_in_one_launch(int dtype, int T, long PD) {
     const long kb = PD * (dtype == COGS_DT_BF16 ? 2 : 4) >> 10;
-    if (dtype == COGS_DT_BF16) return T <= 256 ? kb <= 128 || (kb <= 1024 && T >= 120) : T <= 300 && kb <= 88;
-    return T <= 160 ? kb <= 176 : T <= 256 && kb >= 256 && kb <= 1024;
+    return kb <= 100 ? T <= 300 : T <= 256 && kb <= (T > 192 ? 512 : T >= 100 ? 224 : 128);
 }
 
-// The whole k-means++ seeding (kmeans_with_time.py:41-62) in one call, no host round trip per centre: step m measures
-// every row against the newest centre (row idx[m-1], read from device memory), folds it into nearest2 and draws centre m
-// as argmax(probs / q[m-1]) (kpp_select). q: device fp32 [K-1][T], the Exponential(1) draws the reference's K-1
+// The whole k-means++ seeding (kmeans_with_time.py:41-62) in one call, no host round trip per centre: up to K - 1 passes measure
+// every row against the newest centre and guesses of the next ones (rows read from device memory), fold it into nearest2 and draw centre m
+// as argmax(probs / q[m-1]) (kpp_draw). 256 frames of 179 200 bf16, 18 centres: 17 launches of 23 us were 388 us, now 205 (17 too, 12 of which return
+// at once). q: device fp32 [K-1][T], the Exponential(1) draws the reference's K-1
 // torch.multinomial calls would make on the CPU generator, made ahead by the host. idx: device int32 [K], idx[0] given.
 // dist2 (nullable) [T][K]: column m - 1 receives the squared distances to centre m - 1, the last column nothing.
 // *zero_flag (device int, zeroed here) is set when a step found all probabilities zero -- the reference's
 // random.randint branch; the indices from that step on are then meaningless and the caller redoes the seeding step by step.
 int cogs_k_kmeans_pp(hipStream_t st, int dtype, const void* feats, int T, long PD, int K, int first_row, const float* q, int* idx,
-                     int* zero_flag, float* nearest2, float* dist2, float* ws, int nslices) {
+                     int* zero_flag, float* nearest2, float* dist2, float* ws, size_t ws_bytes, int nslices) {
     if (T <= 0 || K <= 0 || PD % 8 || !q || !idx || !zero_flag || !nearest2 || first_row < 0 || first_row >= T) return COGS_E_INVALID;
-    const KmWs w = carve(ws, T, PD, 1);
     if (nslices != (int)((PD + SL - 1) / SL)) return COGS_E_WORKSPACE;
-    const bool one = kpp_in_one_launch(dtype, T, PD);
-    hipLaunchKernelGGL(start_kernel, dim3(1), dim3(256), 0, st, w.ctl, one ? 1 : 0, zero_flag, nullptr, 0, 0);      // w.ctl: the counter of finished rows
+    const int form = (int)g_cogs_debug.km_pp_form;
+    const bool one = form > 0 ? form == 1 && T <= 300 : kpp_in_one_launch(dtype, T, PD);
+    // rows a pass measures: what the workspace has room for (one centre's is accepted)
+    int C = KPP_C < K ? KPP_C : K;
+    while (C > 1 && cogs_k_kmeans_ws(T, PD, C, nullptr) > ws_bytes) --C;
+    const KmWs w = carve(ws, T, PD, one ? 1 : C);
+    static_assert(KPP_C * 300 <= POOL_MAX, "a row per workgroup: up to 300 rows, their distances in the pool's place");
+    if (one) C = KPP_C;
+    const KppArgs p{T, K, nearest2, q, idx, zero_flag, w.ctl, one ? (float*)w.pool : w.dist2, C, dist2};
+    hipLaunchKernelGGL(kpp_start_kernel, dim3(1), dim3(256), 0, st, p, first_row);
     g_cogs_debug.km_pp_last_launches = one ? 1 : 3;
-    const size_t lds = (size_t)nslices * 4;
+    const size_t lds = (size_t)nslices * KPP_C * 4;
     for (int m = 1; m < K; ++m) {
-        // step 1 measures against the caller's first centre (a kernel argument: nothing is uploaded), later steps against
-        // the row the previous step drew (read from device memory)
-        const int* from = m == 1 ? nullptr : idx + (m - 1);
-        const float* qm = q + (size_t)(m - 1) * T;
-        float* d2 = dist2 ? dist2 + (m - 1) : nullptr;
         if (!one) {
-            const int rc = sqdist_partials(st, dtype, feats, T, PD, nullptr, from, m == 1 ? first_row : -1, 1, w.partial, nslices);
+            const int rc = sqdist_partials(st, dtype, feats, T, PD, nullptr, w.ctl + KPP_ROWS, -1, C, w.partial, nslices, w.ctl);
             if (rc != COGS_OK) return rc;
-            hipLaunchKernelGGL(reduce_min_kernel, dim3((T + 3) / 4), dim3(256), 0, st, w.partial, nslices, T, m == 1 ? 1 : 0, nearest2, d2, K);
-            hipLaunchKernelGGL(kpp_select_kernel, dim3(1), dim3(256), 0, st, nearest2, qm, T, idx + m, zero_flag, m == 1 ? first_row : -1);
+            hipLaunchKernelGGL(kpp_reduce_kernel, dim3(T), dim3(256), 0, st, w.partial, p, nslices);
         } else if (dtype == COGS_DT_BF16)
-            hipLaunchKernelGGL(kpp_step_kernel<bf16_t>, dim3(T), dim3(KPP_T), lds, st, (const bf16_t*)feats, T, PD, nslices, from, first_row, m == 1, nearest2,
-                               qm, idx + m, zero_flag, w.ctl, d2, K);
+            hipLaunchKernelGGL(kpp_pass_kernel<bf16_t>, dim3(T), dim3(KPP_T), lds, st, (const bf16_t*)feats, p, PD, nslices);
         else
-            hipLaunchKernelGGL(kpp_step_kernel<float>, dim3(T), dim3(KPP_T), lds, st, (const float*)feats, T, PD, nslices, from, first_row, m == 1, nearest2,
-                               qm, idx + m, zero_flag, w.ctl, d2, K);
+            hipLaunchKernelGGL(kpp_pass_kernel<float>, dim3(T), dim3(KPP_T), lds, st, (const float*)feats, p, PD, nslices);
     }
-    if (K == 1 && hipMemcpyAsync(idx, &first_row, sizeof(int), hipMemcpyHostToDevice, st) != hipSuccess) return COGS_E_HIP;
     return COGS_LAUNCH_CHECK();
 }
 
@@ -1008,10 +1171,10 @@ int cogs_k_kmeans_lloyd(hipStream_t st, int dtype, const void* feats, const floa
     if (max_iter == 0) return COGS_OK;             // nothing to do
     const KmWs w = carve(ws, T, PD, K);
     if (!dist2) dist2 = w.dist2;
-    hipLaunchKernelGGL(start_kernel, dim3(1), dim3(256), 0, st, w.ctl, (int)CTL_WORDS, nullptr, w.keep, K, known);        // margin word 0 = +inf
     int* pool_d = sb.d + 16;
     for (int i = 0; i < pool_len; ++i) sb.h[16 + i] = pool_host[i];        // plain host stores into the mapped block
     for (int i = 0; i <= CTL_WORDS; ++i) sb.h[i] = 0;
+    hipLaunchKernelGGL(start_kernel, dim3(1), dim3(256), 0, st, w.ctl, w.keep, K, known);     // margin word 0 = +inf
     int queued = 0, it = 0, used = 0, ex = 0;
     int rc = COGS_OK;
     while (queued < max_iter) {

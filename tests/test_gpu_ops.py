@@ -1411,6 +1411,35 @@ def test_whole_seeding_equals_the_steps(dev, T, PD, K, dtype):
     assert int(flag) == 1
 
 
+@pytest.mark.parametrize("form", [1, 3])
+@pytest.mark.parametrize("T,PD,K,scenes", [(5, 8, 2, 2), (9, 520, 3, 3), (40, 1032, 39, 4), (255, 2048, 18, 21), (300, 512, 60, 1), (700, 1032, 30, 11)])
+def test_seeding_draws_several_centres_a_pass(dev, T, PD, K, scenes, form):
+    """a pass measures rows that the next draws are likely to fall on and draws while they do: the rows and distances of a pass per centre, where
+    guesses come true (rows of scenes), where most do not (more centres than scenes), for the last centres (fewer guesses), for more rows than
+    a workgroup keeps in LDS, and with a workspace of one centre"""
+    from cogstream_amd import _lib as L2
+    ops = _ops()
+    g = torch.Generator(device=dev).manual_seed(T + K)
+    x = (torch.randn(scenes, PD, generator=g, device=dev)[torch.arange(T, device=dev) * scenes // T] + 0.2 * torch.randn(T, PD, generator=g, device=dev)).bfloat16()
+    q = torch.empty(K - 1, T).exponential_(1, generator=torch.Generator().manual_seed(K))
+    ws = ops.kmeans_workspace(T, PD, K, x.device)
+    want, near, cols = [T // 3], torch.empty(T, device=dev), []
+    probs = torch.empty(T).pin_memory()
+    for m in range(K - 1):
+        ops.kmeans_pp_step(x, want[-1], m == 0, near, probs, ws)
+        one = torch.empty(T, device=dev)
+        ops.kmeans_pp_step(x, want[-1], True, one, None, ws)
+        cols.append(one)
+        p = probs.sqrt() ** 2
+        want.append(int((p / p.double().sum().float() / q[m]).argmax()))
+    for space in (ws, ops.kmeans_workspace(T, PD, 1, x.device)):
+        d2 = torch.full((T, K), -1.0, device=dev)
+        with L2.debug_switch("km_pp_form", form):
+            idx, flag = ops.kmeans_pp(x, T // 3, K, q.to(dev), space, d2)
+        assert idx.tolist() == want and int(flag) == 0
+        assert torch.equal(d2[:, :K - 1], torch.stack(cols, 1)) and bool((d2[:, K - 1] == -1).all())
+
+
 @pytest.mark.parametrize("M,N,K,form", [
     (4609, 3456, 1152, "rotary, head-major, folded norm"), (3841, 4352, 1152, "folded norm, gelu"), (13825, 1152, 1152, "residual, statistics"),
     (13825, 1152, 4352, "residual, statistics"), (3585, 4608, 3584, "rotary"), (4609, 3584, 3584, "residual"), (2049, 8192, 2048, "plain"),
