@@ -569,12 +569,20 @@ cogs_status cogs_decoder_forward(cogs_handle h, cogs_stream stream, const void* 
     for (int i = 0; i < n_want; ++i) first = want[i] < first ? want[i] : first;
     first = nseq == 1 && !streams && d.w.dtype == COGS_DT_BF16 && S > 256 ? first / 128 * 128 : 0;
     if (first > 0) seqs.push_back(CogsSeq{seqs[0].cache, seqs[0].state, seqs[0].max_len, first, S - first, seqs[0].pos0 + first, 0});
-    COGS_TRY(stage_h2d(h, st, k.seqs, seqs.data(), seqs.size() * sizeof(CogsSeq)));
-    if (n_want > 0) COGS_TRY(stage_h2d(h, st, k.want, want, (size_t)n_want * sizeof(int32_t)));
+    const int entries = (int)seqs.size();
+    CogsSeqTable table;
+    const bool in_args = entries <= COGS_INLINE_SEQS && n_want <= COGS_INLINE_WANT;
+    if (in_args) {
+        memcpy(table.seqs, seqs.data(), entries * sizeof(CogsSeq));
+        if (n_want > 0) memcpy(table.want, want, n_want * sizeof(int32_t));
+    } else {
+        COGS_TRY(stage_h2d(h, st, k.seqs, seqs.data(), entries * sizeof(CogsSeq)));
+        if (n_want > 0) COGS_TRY(stage_h2d(h, st, k.want, want, (size_t)n_want * sizeof(int32_t)));
+    }
     Step s{h, st, d, k, seqs, S, nseq, max_new, max_ctx, C, chained(d, S) && !streams};
     {
         PROF(COGS_PROF_OTHER);
-        COGS_TRY(cogs_k_seq_rows(st, k.seqs, nseq, S, k.rowseq, k.rowpos));
+        COGS_TRY(cogs_k_seq_rows(st, k.seqs, nseq, S, k.rowseq, k.rowpos, in_args ? &table : nullptr, entries, k.want, n_want));
         if (!d.sets.empty()) COGS_TRY(cogs_k_rope_sets(st, k.rope, d.sets_dev, (int)d.sets.size(), d.max_pairs, k.rowpos, S));
         if (d.att_tail) COGS_TRY(cogs_k_zero(st, k.att, align_up((size_t)S * d.max_o * esize(d.w.dtype))));
     }

@@ -183,7 +183,12 @@ struct CogsSeq {
     int pos0;            // rows already cached
     int ctx0;            // first row of its context (pos0 + len rows) in buffers that hold every sequence's context back to back
 };
-int cogs_k_seq_rows(hipStream_t st, const CogsSeq* seqs, int nseq, int rows, int* rowseq, int* rowpos);
+// a step's sequences and wanted rows as a kernel's argument: few of them need no copy of their own
+constexpr int COGS_INLINE_SEQS = 40, COGS_INLINE_WANT = 128;
+struct CogsSeqTable { CogsSeq seqs[COGS_INLINE_SEQS]; int want[COGS_INLINE_WANT]; };
+// rowseq, rowpos of the first nseq of `seqs`; with a table, its first `entries` sequences and n_want rows are stored at seqs and want first
+int cogs_k_seq_rows(hipStream_t st, CogsSeq* seqs, int nseq, int rows, int* rowseq, int* rowpos, const CogsSeqTable* table = nullptr, int entries = 0,
+                    int* want = nullptr, int n_want = 0);
 
 // (cos, sin) * mag of the pairs of a head, [rows][pairs][2] at table + off * rows: pairs first .. first + n - 1 turn with freq[i]
 // radians per position, the others stand still (1, 0). Angles are reduced in fp64. One launch for `nsets` such tables.

@@ -138,14 +138,25 @@ __global__ __launch_bounds__(1024) void topk_kernel(const float* __restrict__ lo
 }
 
 // sequence and position of every new row of a step
-__global__ __launch_bounds__(256) void seq_rows_kernel(const CogsSeq* __restrict__ seqs, int nseq, int rows, int* __restrict__ rowseq,
-                                                       int* __restrict__ rowpos) {
+__device__ __forceinline__ void seq_row(const CogsSeq* seqs, int nseq, int rows, int* __restrict__ rowseq, int* __restrict__ rowpos) {
     const int r = blockIdx.x * 256 + threadIdx.x;
     if (r >= rows) return;
     int lo = 0, hi = nseq;
     while (hi - lo > 1) { const int mid = (lo + hi) >> 1; if (seqs[mid].row0 <= r) lo = mid; else hi = mid; }
     rowseq[r] = lo;
     rowpos[r] = seqs[lo].pos0 + r - seqs[lo].row0;
+}
+__global__ __launch_bounds__(256) void seq_rows_kernel(const CogsSeq* __restrict__ seqs, int nseq, int rows, int* __restrict__ rowseq, int* __restrict__ rowpos) {
+    seq_row(seqs, nseq, rows, rowseq, rowpos);
+}
+// ... the sequences still in the launch's arguments: two copies of some hundred bytes were 2 to 5 us each, with a gap before each, in every step
+__global__ __launch_bounds__(256) void seq_table_kernel(const CogsSeqTable t, CogsSeq* __restrict__ seqs, int entries, int nseq, int rows, int* __restrict__ rowseq,
+                                                        int* __restrict__ rowpos, int* __restrict__ want, int n_want) {
+    if (blockIdx.x == 0) {
+        if (threadIdx.x < entries) seqs[threadIdx.x] = t.seqs[threadIdx.x];
+        if (threadIdx.x < n_want) want[threadIdx.x] = t.want[threadIdx.x];
+    }
+    seq_row(t.seqs, nseq, rows, rowseq, rowpos);
 }
 
 __global__ __launch_bounds__(256) void rope_sets_kernel(float* __restrict__ table, const CogsRopeSet* __restrict__ sets,
@@ -172,9 +183,12 @@ __global__ __launch_bounds__(256) void zero_kernel(u32x4* __restrict__ p, long n
 
 }  // namespace
 
-int cogs_k_seq_rows(hipStream_t st, const CogsSeq* seqs, int nseq, int rows, int* rowseq, int* rowpos) {
+int cogs_k_seq_rows(hipStream_t st, CogsSeq* seqs, int nseq, int rows, int* rowseq, int* rowpos, const CogsSeqTable* table, int entries, int* want, int n_want) {
     if (nseq <= 0 || rows <= 0) return COGS_E_INVALID;
-    hipLaunchKernelGGL(seq_rows_kernel, dim3((rows + 255) / 256), dim3(256), 0, st, seqs, nseq, rows, rowseq, rowpos);
+    if (table) {
+        if (entries < nseq || entries > COGS_INLINE_SEQS || n_want < 0 || n_want > COGS_INLINE_WANT) return COGS_E_INVALID;
+        hipLaunchKernelGGL(seq_table_kernel, dim3((rows + 255) / 256), dim3(256), 0, st, *table, seqs, entries, nseq, rows, rowseq, rowpos, want, n_want);
+    } else hipLaunchKernelGGL(seq_rows_kernel, dim3((rows + 255) / 256), dim3(256), 0, st, seqs, nseq, rows, rowseq, rowpos);
     return COGS_LAUNCH_CHECK();
 }
 

@@ -1524,3 +1524,24 @@ def test_centres_that_stay_keep_their_distances_and_means(dev, T, K, PD, kind, d
         assert got == (done, used, False), (iters, got, done, used)
         assert used >= K // 2 or kind not in ("far", "dry")
         assert torch.equal(ga, a) and torch.equal(gt, ct) and torch.equal(gc.view(torch.int32), c.view(torch.int32)), iters
+
+
+def test_token_ids_reach_the_device_as_they_were_at_the_call(dev):
+    """ops.token_ids: host ids behind work that is still running, their tensor rewritten as soon as the call returns; pinned ids, other types and shapes,
+    none at all; and a capture, which cannot hold a copy from the caller's memory, still refuses"""
+    ops = _ops()
+    d = torch.device("cuda", torch.cuda.current_device())
+    g = torch.Generator().manual_seed(3)
+    for n in (0, 1, 7, 4096):
+        for make in (lambda t: t, lambda t: t.int(), lambda t: t.pin_memory() if n else t, lambda t: t.reshape(1, -1), lambda t: t.to(dev)):
+            want = torch.randint(0, 1000, (n,), generator=g)
+            ids = make(want.clone())
+            torch.cuda._sleep(2_000_000)
+            got = ops.token_ids(ids, d)
+            if not ids.is_cuda:
+                ids.fill_(-1)
+            assert got.is_cuda and got.dtype == torch.int64 and torch.equal(got.cpu(), want)
+    with pytest.raises(RuntimeError), torch.cuda.graph(torch.cuda.CUDAGraph()):
+        ops.token_ids(torch.arange(8), d)
+    torch.cuda.synchronize()
+    assert ops.token_ids(torch.arange(8), d).tolist() == list(range(8))
