@@ -9,7 +9,7 @@
 // wave waits for its own loads alone. Matrix fragments straight from memory put sixteen rows of 16 bytes into every quarter of a load: the
 // vector-memory path then took in 39 B/ns a CU whatever was in flight, also of weights that sat in L2 (8 x 8192 x 2048: 7.4 us from
 // L2, 9.8 from HBM); whole lines come at 110 (4.6 and 8.0). The weights are read with the streaming hint: nothing reads them again before
-// the next step, and 5 to 10 % less time (11 264 x 2048, 16 rows: 11.6 -> 10.9). Columns are taken 64 or 32 at a time where that still
+// the next step, and 5 to 10 % less time (11 264 x 2048, 16 rows: 11.6 -> 10.9). Columns are taken 64, 48 or 32 at a time where that still
 // makes 160 workgroups: the batch rows come from L2 once per workgroup, as many bytes as the weights with NT = 1 and M = 16. Fragments
 // from memory -> ring, weights from HBM (us):
 //      rows    6176 x 2048    8192 x 2048    11 264 x 2048    32 768 x 2048    2048 x 8192    2048 x 5632    4096 x 11 008
@@ -150,12 +150,19 @@ void launch(hipStream_t st, const SkinnyArgs& p, int splits) {
 template <int MT>
 void launch_cols(hipStream_t st, const SkinnyArgs& p, int cols, int splits) {
     if (cols == 64) launch<MT, 4, 4, 2>(st, p, splits);
+    else if (cols == 48 && MT == 1) launch<1, 3, 4, 2>(st, p, splits);
     else if (cols == 32) launch<MT, 2, MT == 1 ? 8 : 4, 3>(st, p, splits);
     else launch<MT, 1, 4, MT == 1 ? 4 : MT == 2 ? 3 : 2>(st, p, splits);
 }
 
-// columns per workgroup of a product without partial sums
-int whole_cols(int N) { return N >= 64 * 160 ? 64 : N >= 32 * 160 ? 32 : 16; }
+// columns per workgroup of a product without partial sums. 48 instead of 64 where the CU with most workgroups then takes fewer columns in (with the 16
+// batch rows of each): 16 rows, us, 64 / 48 columns, 11 264 x 2048 10.7 / 10.3, 22 016 x 4096 36.8 / 30.3, 10 808 x 3584 15.7 / 14.1, and by the rule
+// with 64: 12 320 x 4096 19.3 / 24.3, 16 384 x 4096 25.6 / 27.4, 28 416 x 3584 32.9 / 36.3, 37 888 x 3584 46.5 / 47.5
+int whole_cols(int M, int N) {
+    if (N < 64 * 160) return N >= 32 * 160 ? 32 : 16;
+    auto taken = [N](int cols) { return ((N + cols - 1) / cols + 255) / 256 * (cols + 16); };
+    return M <= 16 && taken(48) < taken(64) ? 48 : 64;
+}
 
 }  // namespace
 
@@ -183,7 +190,7 @@ CogsAhead cogs_k_gemm_skinny_ahead(const void* W, long ldw, int M, int N, int K)
     g.dtype = COGS_DT_BF16; g.M = M; g.N = N; g.K = K; g.lda = K; g.ldw = ldw;
     if (!W || g_cogs_debug.gemm_skinny == 0 || !cogs_k_gemm_skinny_fits(g)) return a;
     const long lines = AHEAD_BYTES / (128L * N);
-    a.W = (const char*)W; a.ldw = ldw * 2; a.N = N; a.cols = whole_cols(N); a.groups = (N + a.cols - 1) / a.cols;
+    a.W = (const char*)W; a.ldw = ldw * 2; a.N = N; a.cols = whole_cols(M, N); a.groups = (N + a.cols - 1) / a.cols;
     a.lines = (int)(lines < K / 64 ? lines : K / 64);
     return a;
 }
@@ -198,7 +205,7 @@ int cogs_k_gemm_skinny(hipStream_t st, const CogsGemm& g, float* part) {
     g_cogs_debug.gemm_last_body = 7;
     const int parts = part ? cogs_k_gemm_skinny_parts(g.M, g.N, g.K) : 1;
     if (part && (g.act != COGS_ACT_NONE || g.residual || g.rope_cos || g.out_f32 || parts < 2)) return COGS_E_UNSUPPORTED;
-    const int cols = parts > 1 ? (g.K >= 4096 ? 64 : g.M <= 16 ? 16 : 32) : whole_cols(g.N);
+    const int cols = parts > 1 ? (g.K >= 4096 ? 64 : g.M <= 16 ? 16 : 32) : whole_cols(g.M, g.N);
     if (g.M <= 16) launch_cols<1>(st, p, cols, parts);
     else if (g.M <= 32) launch_cols<2>(st, p, cols, parts);
     else launch_cols<4>(st, p, cols, parts);

@@ -260,6 +260,21 @@ def test_forms_and_kernels_agree(dev):
             assert rms_err(run(e, toks, [20, 380, *range(381, 400)]), lg) < TOL[torch.bfloat16], (name, value)
 
 
+@pytest.mark.parametrize("rows", [2, 8, 9, 16, 17])
+def test_few_rows_by_48_and_64_columns(dev, rows):
+    """few-row products whose columns go 48 to a workgroup (10 240 to 12 288 of up to 16 rows: here the feed-forward's and the head's, the last group
+    ragged in both; 17 rows take 64): every row's logits against the oracle"""
+    cfg = config([mixer(A)], width=256, vocab=10811, ff=5632)
+    st = state(cfg)
+    e = engine(cfg, st, torch.bfloat16)
+    toks = [tokens(cfg, 4, seed=i) for i in range(rows)]
+    s = sequences(e)
+    s.step([(i, t[:3], []) for i, t in enumerate(toks)])
+    got = s.step([(i, t[3:], [0]) for i, t in enumerate(toks)])
+    want = torch.cat([po.forward(cfg, double(st), t)[0][3:] for t in toks])
+    assert rms_err(got, want) < TOL[torch.bfloat16]
+
+
 @pytest.mark.parametrize("keys", [16384, 16385, 16600, 40000])
 def test_a_context_of_more_splits_than_are_combined(dev, keys):
     """one sequence of up to 256 splits of two tiles (16 384 keys with the new one) and of more, which get longer ones, alone and between short ones.
