@@ -25,6 +25,7 @@
 //     four different 64-B bank quarters for the transposing read). 46 KiB per workgroup: 3 workgroups per CU.
 #include "common.h"
 #include "kernels.h"
+#include "weights_ahead.h"
 #include "debug.h"
 #include <stdlib.h>
 
@@ -45,9 +46,11 @@ struct VitAttnArgs {
     int uniform_len;           // > 0: every segment has this many rows and segment s starts at row s * uniform_len (one video:
                                // all frames alike) -- the bounds are then arithmetic on kernel arguments instead of two
                                // dependent scalar loads at the head of every workgroup (700-1 700 cycles of its 39 000)
+    CogsWeightsAhead next[2];  // pipe kernel: the workgroups from z = nseg on read these weights into L2 (weights_ahead.h)
 };
 
 constexpr float RESCALE_THR = 6.0f;
+constexpr int AHEAD_WGS = 64;      // workgroups that read weights ahead (one image: 32, 64, 96, 192: 1382, 1313, 1313, 1323 us)
 
 #if defined(COGS_ATTN_STAMPS) || defined(COGS_PIPE_STAMPS) || defined(COGS_PHASE_STAMPS)   // diagnostic builds (tools/micro/attn_vit_micro.cpp)
 __device__ unsigned long long g_attn_stamps[8];
@@ -442,6 +445,12 @@ __global__ __launch_bounds__(256, 2) void attn_vit_pipe_kernel(VitAttnArgs p) {
     PSTAMP();      // 0: kernel entry
     unsigned long long life0 = 0, life1 = 0;
     LIFE_NOW(life0);
+    if ((int)blockIdx.z >= p.nseg) {
+        const int per_xcd = gridDim.x >> 3, me = (((int)blockIdx.z - p.nseg) * gridDim.y + blockIdx.y) * per_xcd + (blockIdx.x >> 3);
+        const int of = ((int)gridDim.z - p.nseg) * gridDim.y * per_xcd;
+        read_weights_ahead(p.next[0], p.next[1], blockIdx.x & 7, me * NW + wid, of * NW, lane);
+        return;
+    }
     int seg, head, qb;                                           // XCD-aware 3-D grid, see attn_vit_kernel
     if (p.xcd_order) { qb = blockIdx.x >> 3; head = blockIdx.y * 8 + (blockIdx.x & 7); seg = blockIdx.z; }
     else { qb = blockIdx.x; head = blockIdx.y; seg = blockIdx.z; }
@@ -995,6 +1004,7 @@ int cogs_k_attention_vit(hipStream_t st, const CogsAttn& a) {
     const int variant = (int)g_cogs_debug.attn_vit;     // 1: unpipelined (A/B runs)
     const int env_early = (int)g_cogs_debug.attn_vit_early;
     p.early_prefetch = env_early;
+    p.next[0] = a.next[0]; p.next[1] = a.next[1];
     if (variant == 1 || a.ldk != a.ldv) { g_cogs_debug.attn_last_kernel = 2; hipLaunchKernelGGL(attn_vit_kernel<72>, grid, dim3(256), 0, st, p); }
     else {
         g_cogs_debug.attn_last_kernel = a.head_stride > 0 ? 8 : 3;
@@ -1002,7 +1012,10 @@ int cogs_k_attention_vit(hipStream_t st, const CogsAttn& a) {
         const int nt = (p.uniform_len + 63) >> 6;
         const int r = (g_cogs_debug.attn_vit_len != 0 && p.uniform_len > 0 && nt >= 4) ? 4 + ((nt - 4) & 3) : 0;
         const int nlb = p.uniform_len - 64 * (nt - 1) > 32 ? 2 : 1;
-#define COGS_AV_LAUNCH(R_, B_) hipLaunchKernelGGL((attn_vit_pipe_kernel<72, R_, B_>), grid, dim3(256), 0, st, p)
+        dim3 grid_ahead = grid;
+        const long slice = (long)grid.x * grid.y;
+        if (p.next[1].W && p.xcd_order && (p.nseg + 1) * slice <= 256) grid_ahead.z += max(1, min((int)(AHEAD_WGS / slice), (int)(256 / slice) - p.nseg));
+#define COGS_AV_LAUNCH(R_, B_) hipLaunchKernelGGL((attn_vit_pipe_kernel<72, R_, B_>), grid_ahead, dim3(256), 0, st, p)
         g_cogs_debug.attn_vit_last_end = r * 10 + (r ? nlb : 0);
         switch (r * 10 + (r ? nlb : 0)) {
             case 41: COGS_AV_LAUNCH(4, 1); break;   case 42: COGS_AV_LAUNCH(4, 2); break;

@@ -428,6 +428,7 @@ struct VitRange {
 
     cogs_status begin();
     cogs_status layer(int l);
+    CogsGemm qkv_product(int l) const, out_product(int l) const, fc1_product(int l) const, fc2_product(int l) const;
     cogs_status finish();
 };
 
@@ -685,6 +686,54 @@ cogs_status VitRange::begin() {
     return COGS_OK;
 }
 
+// the four products of a layer (what a launch in front reads ahead is what the product then gets)
+CogsGemm VitRange::qkv_product(int l) const {
+    const cogs_vit_weights& w = h->vit;
+    const cogs_vit_layer& L = h->vit_layers[l];
+    const int H = w.hidden;
+    CogsGemm g; g.dtype = w.dtype;
+    g.A = fold ? x : ln; g.lda = H; g.W = L.qkv_w; g.ldw = H; g.C = big; g.ldc = 3 * H;
+    g.M = (int)N; g.N = 3 * H; g.K = H;
+    if (fold) { g.ln_ab = ln_ab; g.ln_part = stat_part; g.ln_eps = w.ln_eps; g.col_c = L.qkv_c; }
+    else g.bias = L.qkv_b;
+    g.rope_cos = rc; g.rope_sin = rs; g.rope_cols = 2 * H; g.head_dim = H / w.heads;
+    if (prescale_q) { g.q_scale = scale * 1.4426950408889634f; g.q_cols = H; }
+    if (use_lut) { g.rope_lut = lut; g.rope_rowpos = lo; g.rope_maxpos = maxpos; }
+    if (head_major) { g.hm_rows = N; g.hm_cols = H; }
+    return g;
+}
+CogsGemm VitRange::out_product(int l) const {
+    const cogs_vit_weights& w = h->vit;
+    const cogs_vit_layer& L = h->vit_layers[l];
+    const int H = w.hidden;
+    CogsGemm g; g.dtype = w.dtype;
+    g.A = (char*)big + (size_t)N * 3 * H * esize(w.dtype); g.lda = H; g.W = L.o_w; g.ldw = H; g.C = x; g.ldc = H;
+    g.bias = L.o_b; g.residual = x; g.ldr = H; g.M = (int)N; g.N = H; g.K = H;
+    if (fold) g.row_stats = stat_part;
+    return g;
+}
+CogsGemm VitRange::fc1_product(int l) const {
+    const cogs_vit_weights& w = h->vit;
+    const cogs_vit_layer& L = h->vit_layers[l];
+    const int H = w.hidden;
+    CogsGemm g; g.dtype = w.dtype;
+    g.A = fold ? x : ln; g.lda = H; g.W = L.fc1_w; g.ldw = H; g.C = big; g.ldc = w.inter_pad;
+    g.M = (int)N; g.N = w.inter_pad; g.K = H; g.act = COGS_ACT_GELU_TANH;
+    if (fold) { g.ln_ab = ln_ab; g.ln_part = stat_part; g.ln_eps = w.ln_eps; g.col_c = L.fc1_c; }
+    else g.bias = L.fc1_b;
+    return g;
+}
+CogsGemm VitRange::fc2_product(int l) const {
+    const cogs_vit_weights& w = h->vit;
+    const cogs_vit_layer& L = h->vit_layers[l];
+    const int H = w.hidden;
+    CogsGemm g; g.dtype = w.dtype;
+    g.A = big; g.lda = w.inter_pad; g.W = L.fc2_w; g.ldw = w.inter_pad; g.C = x; g.ldc = H;
+    g.bias = L.fc2_b; g.residual = x; g.ldr = H; g.M = (int)N; g.N = H; g.K = w.inter_pad;
+    if (fold && l + 1 < w.layers) g.row_stats = stat_part;     // the last layer feeds post_layernorm (own kernel)
+    return g;
+}
+
 cogs_status VitRange::layer(int l) {
     const cogs_vit_weights& w = h->vit;
     const int dt = w.dtype;
@@ -694,18 +743,13 @@ cogs_status VitRange::layer(int l) {
     char* att = qkv + (size_t)N * 3 * H * es;
     const cogs_vit_layer& L = h->vit_layers[l];
     if (!fold) { PROF(COGS_PROF_NORM); COGS_TRY(cogs_k_layernorm(st, dt, x, ln, L.ln1_g, L.ln1_b, (int)N, H, w.ln_eps)); }
-    {
-        CogsGemm g; g.dtype = dt;
-        g.A = fold ? x : ln; g.lda = H; g.W = L.qkv_w; g.ldw = H; g.C = qkv; g.ldc = 3 * H;
-        g.M = (int)N; g.N = 3 * H; g.K = H;
-        if (fold) { g.ln_ab = ln_ab; g.ln_part = stat_part; g.ln_eps = w.ln_eps; g.col_c = L.qkv_c; }
-        else g.bias = L.qkv_b;
-        g.rope_cos = rc; g.rope_sin = rs; g.rope_cols = 2 * H; g.head_dim = hd;
-        if (prescale_q) { g.q_scale = scale * 1.4426950408889634f; g.q_cols = H; }
-        if (use_lut) { g.rope_lut = lut; g.rope_rowpos = lo; g.rope_maxpos = maxpos; }
-        if (head_major) { g.hm_rows = N; g.hm_cols = H; }
-        { PROF(COGS_PROF_GEMM); COGS_TRY(cogs_k_gemm(st, g)); }
+    CogsGemm qkv_g = qkv_product(l), out = out_product(l), fc1 = fc1_product(l), fc2 = fc2_product(l);
+    qkv_g.weights_read = l > 0 && cogs_k_gemm_weights_ahead(fc2).W && cogs_k_gemm_weights_ahead(qkv_g).W;
+    if (attn_mode != COGS_ATTN_REF_EAGER_GLOBAL && qkv_g.weights_read) {
+        qkv_g.next = cogs_k_gemm_weights_ahead(out);
+        out.weights_read = qkv_g.next.W != nullptr;
     }
+    { PROF(COGS_PROF_GEMM); COGS_TRY(cogs_k_gemm(st, qkv_g)); }
     {
         CogsAttn a; a.dtype = dt;
         a.Q = qkv; a.K = qkv + (size_t)H * es; a.V = qkv + (size_t)2 * H * es; a.O = att;
@@ -720,32 +764,19 @@ cogs_status VitRange::layer(int l) {
         else {
             a.cu_seqlens = cu; a.nseg = nframes; a.max_seqlen = max_seq;
             a.uniform_seqlen = uniform_seq;      // all frames alike (one video, or videos of one grid): see attn_vit.hip
+            if (!out.weights_read) a.next[0] = cogs_k_gemm_weights_ahead(out);
+            a.next[1] = cogs_k_gemm_weights_ahead(fc1);
+            fc1.weights_read = a.next[1].W != nullptr;
         }
         { PROF(COGS_PROF_ATTN); COGS_TRY(cogs_k_attention(st, a)); }
     }
-    {
-        CogsGemm g; g.dtype = dt;
-        g.A = att; g.lda = H; g.W = L.o_w; g.ldw = H; g.C = x; g.ldc = H;
-        g.bias = L.o_b; g.residual = x; g.ldr = H; g.M = (int)N; g.N = H; g.K = H;
-        if (fold) g.row_stats = stat_part;
-        { PROF(COGS_PROF_GEMM); COGS_TRY(cogs_k_gemm(st, g)); }
-    }
+    out.next = cogs_k_gemm_weights_ahead(fc2);
+    fc2.weights_read = out.next.W != nullptr;
+    { PROF(COGS_PROF_GEMM); COGS_TRY(cogs_k_gemm(st, out)); }
     if (!fold) { PROF(COGS_PROF_NORM); COGS_TRY(cogs_k_layernorm(st, dt, x, ln, L.ln2_g, L.ln2_b, (int)N, H, w.ln_eps)); }
-    {
-        CogsGemm g; g.dtype = dt;
-        g.A = fold ? x : ln; g.lda = H; g.W = L.fc1_w; g.ldw = H; g.C = big; g.ldc = w.inter_pad;
-        g.M = (int)N; g.N = w.inter_pad; g.K = H; g.act = COGS_ACT_GELU_TANH;
-        if (fold) { g.ln_ab = ln_ab; g.ln_part = stat_part; g.ln_eps = w.ln_eps; g.col_c = L.fc1_c; }
-        else g.bias = L.fc1_b;
-        { PROF(COGS_PROF_GEMM); COGS_TRY(cogs_k_gemm(st, g)); }
-    }
-    {
-        CogsGemm g; g.dtype = dt;
-        g.A = big; g.lda = w.inter_pad; g.W = L.fc2_w; g.ldw = w.inter_pad; g.C = x; g.ldc = H;
-        g.bias = L.fc2_b; g.residual = x; g.ldr = H; g.M = (int)N; g.N = H; g.K = w.inter_pad;
-        if (fold && l + 1 < w.layers) g.row_stats = stat_part;     // the last layer feeds post_layernorm (own kernel)
-        { PROF(COGS_PROF_GEMM); COGS_TRY(cogs_k_gemm(st, g)); }
-    }
+    { PROF(COGS_PROF_GEMM); COGS_TRY(cogs_k_gemm(st, fc1)); }
+    if (l + 1 < w.layers) fc2.next = cogs_k_gemm_weights_ahead(qkv_product(l + 1));
+    { PROF(COGS_PROF_GEMM); COGS_TRY(cogs_k_gemm(st, fc2)); }
     return COGS_OK;
 }
 

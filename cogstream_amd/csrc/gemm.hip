@@ -1165,6 +1165,19 @@ static int best_mid_tile(int M, int N, int K, bool alone, float* time, int rows0
     }
     return best;
 }
+// Up to 576 rows: more of them leave few CUs idle and wait for their rows rather than for weights. Encoder and projector, us, with / without: 144 patches 1249
+// / 1275, 256 1313 / 1372, 512 1626 / 1686; 663 1784 / 1772, 924 2228 / 2238, 1024 2104 / 2094.
+CogsWeightsAhead cogs_k_gemm_weights_ahead(const CogsGemm& g) {
+    constexpr int AHEAD_ROWS = 576;
+    CogsWeightsAhead a;
+    if (g.dtype != COGS_DT_BF16 || g.M < 2 || g.M > AHEAD_ROWS || g.K % 64 || g.N % 4 || g_co_streams != 1 || g_cogs_debug.gemm_co_streams > 1 || g_cogs_debug.gemm_mid > 0) return a;
+    float time = 0.f;
+    const TileCost& t = MID_TILES[best_mid_tile(g.M, g.N, g.K, true, &time) - 1];
+    const int nbm = (g.M + t.tm - 1) / t.tm, nbn = (g.N + t.tn - 1) / t.tn;
+    if (nbm > 12 || nbm * nbn > PERSISTENT_WGS) return a;        // (one group of row tiles: the runs of tiles are runs of columns)
+    a.W = (const char*)g.W; a.ldw = g.ldw * 2; a.N = g.N; a.KT = g.K / 64; a.nbm = nbm; a.nbn = nbn; a.tn = t.tn;
+    return a;
+}
 // the row factors of a folded LayerNorm for the kernels that read them finished (the mid-size one forms its rows' own)
 static int finish_ln(hipStream_t st, const CogsGemm& g) {
     return g.ln_part ? cogs_k_ln_finalize(st, g.ln_part, g.M, g.K / 64, g.K, g.ln_eps, const_cast<float*>(g.ln_ab)) : COGS_OK;

@@ -28,6 +28,7 @@
 #include "common.h"
 #include "kernels.h"
 #include "gemm_epilogue.h"
+#include "weights_ahead.h"
 #include "debug.h"
 
 namespace {
@@ -42,6 +43,8 @@ struct MidArgs {
     int group, group0;         // row tiles that share a panel of weights
     const float* ln_part; int ln_tiles; float ln_inv_h, ln_eps;     // EPI_LNFOLD: row statistics still in partial sums (or null)
     int ln_staged;             // a tile's fit a ring slot
+    CogsWeightsAhead next;     // the next product's
+    bool hot;                  // the launches in front have read this one's
     char* kv_k; char* kv_v; int kv_col, kv_dim;      // EPI_ROPE, K and V columns into cache rows of kv_dim (or null)
     EpiArgs epi;
 };
@@ -117,7 +120,8 @@ __global__ __launch_bounds__(64 * WM * WN, WPE) void gemm_mid_kernel(MidArgs p) 
     const int wm = wid / WN, wn = wid % WN;
     const int rest_tiles = p.nbm * p.nbn, tiles = rest_tiles + p.nbm0 * p.nbn0;
     if ((int)blockIdx.x >= tiles) {
-        prefetch_weights(p, smem, TM, TN, WAVES, wid, lane);
+        if (p.next.W) read_weights_ahead(p.next, CogsWeightsAhead{}, blockIdx.x & 7, (((int)blockIdx.x - tiles) >> 3) * WAVES + wid, (((int)gridDim.x - tiles) >> 3) * WAVES, lane);
+        else prefetch_weights(p, smem, TM, TN, WAVES, wid, lane);
         return;
     }
     const int KT = (p.KT + KS - 1) / KS;                         // slots' worth
@@ -370,7 +374,7 @@ __global__ __launch_bounds__(64 * WM * WN, WPE) void gemm_mid_kernel(MidArgs p) 
 }
 
 // CUs without a tile: up to four workgroups an XCD prefetch (one image, encoded over and over: 1561 us without, 1494 with two an XCD, 1371 with four,
-// 1374 with eight)
+// 1374 with eight). The next product's weights are read on all of them: with 32, 64, 112 of the 112 CUs that 256 x 1152 x 4352 leaves 1424, 1335, 1313 us
 int read_ahead_workgroups(int tiles) { return tiles >= MID_CUS ? 0 : tiles > MID_CUS - 32 ? (MID_CUS - tiles) / 8 * 8 : 32; }
 
 template <int EPI, int MI, int NI, int WM, int WN, int S, int WPE, int KS, bool IL>
@@ -392,7 +396,8 @@ void launch(hipStream_t st, MidArgs& p, bool alone) {
     p.group = group_of(p.nbm);
     p.group0 = group_of(p.nbm0);
     p.ln_staged = (long)TM * p.ln_tiles * 8 <= KS * (TM + TN) * ROW_BYTES && ((long)p.M * p.ln_tiles) % 2 == 0;
-    const int tiles = p.nbm * p.nbn + p.nbm0 * p.nbn0, extra = alone && p.rows0 == 0 ? read_ahead_workgroups(tiles) : 0;
+    const int tiles = p.nbm * p.nbn + p.nbm0 * p.nbn0;
+    const int extra = !alone || p.rows0 != 0 ? 0 : p.next.W ? max(MID_CUS - tiles, 0) / 8 * 8 : p.hot ? 0 : read_ahead_workgroups(tiles);
     hipLaunchKernelGGL((gemm_mid_kernel<EPI, MI, NI, WM, WN, S, WPE, KS, IL>), dim3(tiles + extra), dim3(64 * WM * WN), lds, st, p);
 }
 
@@ -436,6 +441,7 @@ int cogs_k_gemm_mid(hipStream_t st, const CogsGemm& g, int tile, bool alone, int
     p.A = (const char*)g.A; p.lda = g.lda * 2;
     p.W = (const char*)g.W; p.ldw = g.ldw * 2;
     p.M = g.M; p.N = g.N; p.KT = g.K / 64; p.rows0 = rows0; p.cols0 = cols0;
+    p.next = g.next; p.hot = g.weights_read;
     p.kv_k = (char*)g.kv_k; p.kv_v = (char*)g.kv_v; p.kv_col = g.kv_col0; p.kv_dim = g.kv_dim;
     if (g.kv_k && (g.kv_col0 % 64 || g.kv_dim % 64)) p.kv_k = nullptr;      // (copied by the caller)
     p.ln_part = g.ln_part; p.ln_tiles = g.K / 64; p.ln_inv_h = 1.0f / (float)g.K; p.ln_eps = g.ln_eps;

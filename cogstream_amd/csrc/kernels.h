@@ -10,6 +10,8 @@
 #define COGS_ACT_GELU_ERF 2
 #define COGS_ACT_SWIGLU 3
 
+struct CogsWeightsAhead { const char* W = nullptr; long ldw = 0; int N = 0, KT = 0, nbm = 0, nbn = 0, tn = 0; };      // ldw in bytes; KT slabs; tiles of tn columns
+
 struct CogsGemm {
     int dtype = 0;                 // COGS_DT_*
     const void* A = nullptr; long lda = 0;   // [M,K], elements per row
@@ -48,7 +50,11 @@ struct CogsGemm {
     // != null: ln_ab (then [M][2] of scratch) is not filled in yet, the statistics are in these partials [M][K/64][2]: the kernel
     // forms each row's factor itself, or cogs_k_ln_finalize runs first
     const float* ln_part = nullptr; float ln_eps = 0.f;
+    CogsWeightsAhead next;                   // read on idle CUs of a mid-size launch, instead of its own weights
+    bool weights_read = false;               // its weights were some launch's `next`
 };
+// the weights of product g as a launch in front of it reads them ahead (weights_ahead.h); none where they are no mid-size product's of one round
+CogsWeightsAhead cogs_k_gemm_weights_ahead(const CogsGemm& g);
 int cogs_k_gemm(hipStream_t st, const CogsGemm& g, bool* kv_stored = nullptr);     // kv_stored (for a call with kv_k): false: the caller copies them from C
 int cogs_k_gemm_mid(hipStream_t st, const CogsGemm& g, int tile, bool alone, int rows0 = 0, int cols0 = 0);     // gemm_mid.hip; the caller (cogs_k_gemm) has checked the operands. alone: no other stream's products beside it.
 // rows0, cols0: without the outputs of the first rows0 rows and cols0 columns (multiples of 64), which another launch computes; no read-ahead then
@@ -57,6 +63,7 @@ void cogs_k_gemm_co_streams(int streams);   // streams fed with GEMMs of this si
 int cogs_k_ln_finalize(hipStream_t st, const float* stat_part, int rows, int tiles, int H, float eps, float* ab);
 
 struct CogsAttn {
+    CogsWeightsAhead next[2];         // ViT kernel: read on the CUs that few workgroups leave idle
     int dtype = 0;
     const void* Q = nullptr; const void* K = nullptr; const void* V = nullptr; void* O = nullptr;
     long ldq = 0, ldk = 0, ldv = 0, ldo = 0;

@@ -1545,3 +1545,21 @@ def test_token_ids_reach_the_device_as_they_were_at_the_call(dev):
         ops.token_ids(torch.arange(8), d)
     torch.cuda.synchronize()
     assert ops.token_ids(torch.arange(8), d).tolist() == list(range(8))
+
+
+@pytest.mark.parametrize("grid", [(1, 2, 2), (1, 12, 11), (1, 16, 16), (2, 12, 23), (1, 24, 24), (1, 1, 577), (3, 14, 16)])
+def test_weights_read_ahead_change_nothing(dev, grid):
+    """the encoder's launches of up to 576 patches read the next products' weights on idle CUs: first and last layer, fewer columns than tiles, and sizes on both
+    sides of the line, bit for bit against launches that read none (as beside another stream)"""
+    from cogstream_amd import _lib as L2
+    from cogstream_amd.vision import VisionEncoder
+    from cogstream_amd.weights import VisionConfig, random_vit_state
+    cfg = VisionConfig(num_hidden_layers=3)
+    enc = VisionEncoder(random_vit_state(cfg, seed=1, device=dev, dtype=torch.bfloat16), cfg)
+    n = grid[0] * grid[1] * grid[2]
+    pix = (torch.rand(n, cfg.patch_dim, generator=torch.Generator(device=dev).manual_seed(n), device=dev) * 2 - 1).bfloat16()
+    run = lambda: enc(pix, torch.tensor([grid]), torch.tensor([1]))
+    got = run()
+    with L2.debug_switch("gemm_co_streams", 2):
+        want = run()
+    assert torch.isfinite(got.float()).all() and torch.equal(got, want)
