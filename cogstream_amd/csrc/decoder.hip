@@ -203,7 +203,7 @@ struct Step {
         {   // rotated queries in log2 score units
             CogsGemm g;
             g.A = row(k.cq, G.qrp); g.lda = G.qrp; g.W = m.q_w; g.ldw = G.qrp; g.C = row(k.q, qcols); g.ldc = qcols; g.M = this->R; g.N = qcols; g.K = G.qrp;
-            g.rope_cos = k.rope + R.off * S + (size_t)r0 * 2 * R.pairs; g.rope_cols = qcols; g.head_dim = G.dq;
+            g.rope_cos = k.rope + R.off * S + (size_t)r0 * 2 * R.pairs; g.rope_cols = qcols; g.head_dim = G.dq; g.rope_still = 2 * R.first;
             g.q_scale = m.scale * 1.4426950408889634f; g.q_cols = qcols;
             COGS_TRY(lin(g));
         }

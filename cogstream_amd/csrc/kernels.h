@@ -26,6 +26,7 @@ struct CogsGemm {
     const float* rope_sin = nullptr;
     int rope_cols = 0;
     int head_dim = 0;
+    int rope_still = 0;                      // leading columns of every head whose pairs the table leaves alone (cos 1, sin 0)
     int force_small_tile = 0;                // fp32: always the 128x128 kernel
     const void* rms_gamma = nullptr;         // M == 1 only: RMS-normalise A on the fly with this weight
     float rms_eps = 0.f;

@@ -260,6 +260,26 @@ def test_forms_and_kernels_agree(dev):
             assert rms_err(run(e, toks, [20, 380, *range(381, 400)]), lg) < TOL[torch.bfloat16], (name, value)
 
 
+@pytest.mark.parametrize("dim,rot", [(128, 64), (96, 64), (64, 32), (32, 64)])
+def test_columns_that_are_not_rotated(dev, dim, rot):
+    """the query product reads no factors for blocks of columns in front of a head's rotated part (64 columns a wave, 32 in the small tiles; heads where such
+    blocks cross into the rotated part or the next head): a prompt against the oracle, and the same bits with every tile size and with the ping-pong kernel"""
+    from cogstream_amd import _lib as L
+    cfg = config([mixer(B, heads=4, dim=dim, rot=rot, vdim=32, q_rank=128, kv_rank=64, gain=1.5), mixer(A, heads=4, dim=dim, rot=rot, vdim=32, q_rank=192, kv_rank=64, scaling=YARN)],
+                 width=128, ff=128)
+    st = state(cfg)
+    e = engine(cfg, st, torch.bfloat16)
+    toks = tokens(cfg, 300)
+    whole = lambda: run(e, toks)
+    first = whole()
+    assert rms_err(first, po.forward(cfg, double(st), toks)[0]) < TOL[torch.bfloat16]
+    for tile in range(1, 12):
+        with L.debug_switch("gemm_mid", tile):
+            assert torch.equal(whole(), first), tile
+    with L.debug_switch("gemm_split", 0):                # (what the ping-pong kernel can take is all its)
+        assert torch.equal(whole(), first)
+
+
 @pytest.mark.parametrize("rows", [2, 8, 9, 16, 17])
 def test_few_rows_by_48_and_64_columns(dev, rows):
     """few-row products whose columns go 48 to a workgroup (10 240 to 12 288 of up to 16 rows: here the feed-forward's and the head's, the last group
