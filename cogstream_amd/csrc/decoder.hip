@@ -189,23 +189,26 @@ struct Step {
             g.A = k.h; g.lda = d.wp; g.W = m.in_w; g.ldw = d.wp; g.C = k.t32; g.ldc = G.ldt; g.M = S; g.N = G.ldt; g.K = d.wp; g.out_f32 = 1;
             COGS_TRY(lin(g));
         }
-        {
-            CogsMlaLatent a{};
-            a.t = k.t32; a.ldt = G.ldt; a.qr = m.q_rank; a.qrp = G.qrp; a.kvr = m.kv_rank; a.kvp = G.kvp; a.dr = m.rot_dim; a.krc = G.rotc;
-            a.own_kv = G.own; a.gate_col = m.gated ? G.qrp + (G.own ? G.kvw : 0) : -1; a.heads = m.heads;
-            a.q_norm = m.q_norm; a.kv_norm = m.kv_norm; a.eps = d.w.eps;
-            a.rope = k.rope + R.off * S; a.rope_pairs = R.pairs; a.rope_first = R.first;
-            a.cq = k.cq; a.gate = k.gate; a.seqs = k.seqs; a.rowseq = k.rowseq; a.rowpos = k.rowpos; a.layer_off = run.cache_off;
-            PROF(COGS_PROF_NORM);
-            COGS_TRY(cogs_k_mla_latent(st, dt, a, S));
-        }
+        CogsMlaLatent lat{};
+        lat.t = k.t32; lat.ldt = G.ldt; lat.qr = m.q_rank; lat.qrp = G.qrp; lat.kvr = m.kv_rank; lat.kvp = G.kvp; lat.dr = m.rot_dim; lat.krc = G.rotc;
+        lat.own_kv = G.own; lat.gate_col = m.gated ? G.qrp + (G.own ? G.kvw : 0) : -1; lat.heads = m.heads;
+        lat.q_norm = m.q_norm; lat.kv_norm = m.kv_norm; lat.eps = d.w.eps;
+        lat.rope = k.rope + R.off * S; lat.rope_pairs = R.pairs; lat.rope_first = R.first;
+        lat.cq = k.cq; lat.gate = k.gate; lat.seqs = k.seqs; lat.rowseq = k.rowseq; lat.rowpos = k.rowpos; lat.layer_off = run.cache_off;
         const int qcols = m.heads * G.dq;
         {   // rotated queries in log2 score units
             CogsGemm g;
             g.A = row(k.cq, G.qrp); g.lda = G.qrp; g.W = m.q_w; g.ldw = G.qrp; g.C = row(k.q, qcols); g.ldc = qcols; g.M = this->R; g.N = qcols; g.K = G.qrp;
             g.rope_cos = k.rope + R.off * S + (size_t)r0 * 2 * R.pairs; g.rope_cols = qcols; g.head_dim = G.dq; g.rope_still = 2 * R.first;
             g.q_scale = m.scale * 1.4426950408889634f; g.q_cols = qcols;
-            COGS_TRY(lin(g));
+            g.dtype = dt;
+            if (r0 == 0 && cogs_k_gemm_skinny_latent_fits(g)) {
+                PROF(COGS_PROF_GEMM);
+                COGS_TRY(cogs_k_gemm_skinny_latent(st, g, lat));
+            } else {
+                { PROF(COGS_PROF_NORM); COGS_TRY(cogs_k_mla_latent(st, dt, lat, S)); }
+                COGS_TRY(lin(g));
+            }
         }
         const float* gate = m.gated ? k.gate : nullptr;
         if (absorbed_step(S, nseq)) {

@@ -22,6 +22,7 @@
 #include "common.h"
 #include "kernels.h"
 #include "gemm_epilogue.h"
+#include "mla_latent.h"
 #include "debug.h"
 
 namespace {
@@ -132,6 +133,143 @@ __global__ __launch_bounds__(64 * NW) void gemm_skinny_kernel(SkinnyArgs p) {
     }
 }
 
+// The query product of latent attention, up to 16 rows: A is the normed query latent, formed by every workgroup itself from the fused projection's fp32 rows
+// while its first weights are on their way (50 to 100 KB from L2 a workgroup), and kept in LDS; the workgroups behind the columns' norm and rotate a row's
+// key and value latent into its cache. A launch of 16 workgroups in front of this one cost 4.7 us of latency, and this one 2.7 more: 16 rows of 3072 x 768
+// 4.7 + 4.2 -> 6.9, a token of 16 requests 694 -> 684, of 3 553 -> 536. The norms have the bits of mla_latent_kernel (four waves share K, also of 32 columns).
+template <int AP, int J, int NT, int D>
+__global__ __launch_bounds__(256) void gemm_skinny_latent_kernel(SkinnyArgs p, CogsMlaLatent l) {
+    extern __shared__ __attribute__((aligned(16))) char smem[];
+    __shared__ __attribute__((aligned(16))) float red[16][4];
+    constexpr int NW = 4, P = 2 * NT, RING = D * P * 1024;
+    static_assert(NT * 1024 <= RING, "a wave's partial tile takes its ring's place");
+    const int tid = threadIdx.x, lane = tid & 63, li = lane & 15, g = lane >> 4;
+    const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int tiles = (p.N + 16 * NT - 1) / (16 * NT);
+    if ((int)blockIdx.x >= tiles) {
+        latent_row<bf16_t, false>(l, blockIdx.x - tiles, tid, &red[0][0]);
+        return;
+    }
+    const int n0 = blockIdx.x * (16 * NT);
+    char* const ring = smem + wid * RING;
+    char* const rows = smem + NW * RING;                         // [slice][AP pieces], as a ring slot would hold them
+    const int all = p.K >> 6, n = wid < all ? (all - wid + NW - 1) / NW : 0;
+    const int r = lane >> 3, c = (lane & 7) ^ r;
+    const bf16_t* w[2 * NT];
+#pragma unroll
+    for (int i = 0; i < 2 * NT; ++i) w[i] = p.W + (long)min(n0 + 8 * i + r, p.N - 1) * p.ldw + 8 * c;
+    auto stage = [&](int slot, int i) {                          // slice i of this wave (past its last: K's last once more)
+        const int k = 64 * min(wid + NW * i, all - 1);
+#pragma unroll
+        for (int q = 0; q < 2 * NT; ++q) piece16<2>(w[q] + k, ring + (slot * P + q) * 1024);
+    };
+    {
+        constexpr int R = 8 * AP;                                // a thread has four columns of every 1024 of each row
+        f32x4 v[R][J];
+#pragma unroll
+        for (int m = 0; m < R; ++m)
+#pragma unroll
+            for (int j = 0; j < J; ++j) v[m][j] = *reinterpret_cast<const f32x4*>(l.t + (long)min(m, p.M - 1) * l.ldt + min(tid * 4 + 1024 * j, p.K - 4));
+        f32x4 norm[J];
+#pragma unroll
+        for (int j = 0; j < J; ++j) norm[j] = *reinterpret_cast<const f32x4*>(l.q_norm + min(tid * 4 + 1024 * j, p.K - 4));
+#pragma unroll
+        for (int i = 0; i < D; ++i) stage(i, i);                 // (behind the rows' loads, and as many on every way here: those are waited for alone)
+#pragma unroll
+        for (int j = 0; j < J; ++j)
+            if (tid * 4 + 1024 * j >= p.K)
+#pragma unroll
+                for (int m = 0; m < R; ++m) v[m][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int m = 0; m < R; ++m) {
+            float sq = 0.f;
+#pragma unroll
+            for (int j = 0; j < J; ++j)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) sq += v[m][j][e] * v[m][j][e];
+            sq = wave_sum(sq);
+            if (lane == 0) red[m][wid] = sq;
+        }
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        // a row's factor by one lane each
+        const f32x4 sums = *reinterpret_cast<const f32x4*>(red[min(li, R - 1)]);
+        const float factor = 1.f / sqrtf(((sums[0] + sums[1]) + (sums[2] + sums[3])) / (float)l.qr + l.eps);
+#pragma unroll
+        for (int j = 0; j < J; ++j) {
+            const int col = tid * 4 + 1024 * j;
+            if (col >= p.K) continue;
+#pragma unroll
+            for (int m = 0; m < R; ++m) {
+                const float rq = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(factor), m));
+                u32x2 b;
+                b[0] = pack_bf2(v[m][j][0] * rq * norm[j][0], v[m][j][1] * rq * norm[j][1]);
+                b[1] = pack_bf2(v[m][j][2] * rq * norm[j][2], v[m][j][3] * rq * norm[j][3]);
+                *reinterpret_cast<u32x2*>(rows + ((col >> 6) * AP + (m >> 3)) * 1024 + (m & 7) * 128 + ((((col >> 3) & 7) ^ (m & 7)) << 4) + (col & 4) * 2) = b;
+            }
+        }
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+    }
+    f32x4 acc[NT];
+#pragma unroll
+    for (int t = 0; t < NT; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+    int off[2];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) off[h] = (li & 7) * 128 + (((4 * h + g) ^ (li & 7)) << 4);
+    int slot = 0;
+    for (int i = 0; i < n; ++i) {
+        wait_slices<P, D - 1>(min(D - 1, max(n, D) - 1 - i));
+        const char* d = ring + slot * (P * 1024);
+        const char* a = rows + ((wid + NW * i) * AP + min(li >> 3, AP - 1)) * 1024;
+        u32x4 wf[NT][2], af[2];
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+#pragma unroll
+            for (int t = 0; t < NT; ++t) wf[t][h] = *reinterpret_cast<const u32x4*>(d + (2 * t + (li >> 3)) * 1024 + off[h]);
+            af[h] = *reinterpret_cast<const u32x4*>(a + off[h]);
+        }
+#pragma unroll
+        for (int t = 0; t < NT; ++t) asm volatile("" : "+v"(wf[t][0]), "+v"(wf[t][1]));
+        asm volatile("" ::: "memory");
+        if (i + D < n) stage(slot, i + D);
+#pragma unroll
+        for (int q = 0; q < NT; ++q)
+#pragma unroll
+            for (int h = 0; h < 2; ++h)
+                acc[q] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, wf[q][h]), __builtin_bit_cast(bf16x8, af[h]), acc[q], 0, 0, 0);
+        slot = slot == D - 1 ? 0 : slot + 1;
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");             // (slices past the last)
+    auto part = [&](int wave, int t) { return reinterpret_cast<f32x4*>(smem + wave * RING) + t * 64 + lane; };
+#pragma unroll
+    for (int t = 0; t < NT; ++t) *part(wid, t) = acc[t];
+    __syncthreads();
+    for (int t = wid; t < NT; t += NW) {
+        f32x4 v = *part(0, t);
+#pragma unroll
+        for (int s = 1; s < NW; ++s) v += *part(s, t);
+        const int nn = n0 + 16 * t + 4 * g;
+        if (li < p.M && nn < p.N) epilogue4<bf16_t>(p.epi, li, nn, v);
+    }
+}
+
+template <int AP, int J, int NT, int D>
+void launch_latent(hipStream_t st, const SkinnyArgs& p, const CogsMlaLatent& l, int extra) {
+    static std::atomic<uint64_t> attr_done{0};
+    cogs_ensure_dyn_lds((const void*)gemm_skinny_latent_kernel<AP, J, NT, D>, 152 * 1024, attr_done);
+    const size_t lds = (size_t)4 * D * 2 * NT * 1024 + (size_t)(p.K / 64) * AP * 1024;
+    hipLaunchKernelGGL((gemm_skinny_latent_kernel<AP, J, NT, D>), dim3((p.N + 16 * NT - 1) / (16 * NT) + extra), dim3(256), lds, st, p, l);
+}
+template <int AP, int J>
+void launch_latent_cols(hipStream_t st, const SkinnyArgs& p, const CogsMlaLatent& l, int cols, int extra) {
+    if (cols >= 48) launch_latent<AP, J, 4, 2>(st, p, l, extra);
+    else if (cols == 32) launch_latent<AP, J, 2, 3>(st, p, l, extra);
+    else launch_latent<AP, J, 1, 3>(st, p, l, extra);
+}
+
 template <int MT, int AP, int NT, int NW, int D>
 void launch1(hipStream_t st, const SkinnyArgs& p, int splits) {
     constexpr int lds = NW * D * (2 * NT + AP) * 1024;
@@ -209,5 +347,22 @@ int cogs_k_gemm_skinny(hipStream_t st, const CogsGemm& g, float* part) {
     if (g.M <= 16) launch_cols<1>(st, p, cols, parts);
     else if (g.M <= 32) launch_cols<2>(st, p, cols, parts);
     else launch_cols<4>(st, p, cols, parts);
+    return COGS_LAUNCH_CHECK();
+}
+
+bool cogs_k_gemm_skinny_latent_fits(const CogsGemm& g) { return cogs_k_gemm_skinny_fits(g) && g.M <= 16 && g.K <= 2048 && g_cogs_debug.gemm_skinny != 0; }
+
+// g's rows are l's normed query latents (g.A is not read); l's key and value latents and gates go where cogs_k_mla_latent puts them
+int cogs_k_gemm_skinny_latent(hipStream_t st, const CogsGemm& g, const CogsMlaLatent& l) {
+    if (!cogs_k_gemm_skinny_latent_fits(g) || g.K != l.qrp || l.kvp % 4 || l.krc % 2 || l.ldt % 4 || l.dr % 2) return COGS_E_UNSUPPORTED;
+    SkinnyArgs p;
+    const int rc = cogs_fill_epi(g, &p.epi);
+    if (rc != COGS_OK) return rc;
+    p.A = nullptr; p.lda = 0; p.W = (const bf16_t*)g.W; p.ldw = g.ldw;
+    p.M = g.M; p.N = g.N; p.K = g.K; p.part = nullptr;
+    g_cogs_debug.gemm_last_body = 7;
+    const int extra = l.own_kv || l.gate_col >= 0 ? g.M : 0, cols = whole_cols(g.M, g.N);
+    if (g.M <= 8) g.K <= 1024 ? launch_latent_cols<1, 1>(st, p, l, cols, extra) : launch_latent_cols<1, 2>(st, p, l, cols, extra);
+    else g.K <= 1024 ? launch_latent_cols<2, 1>(st, p, l, cols, extra) : launch_latent_cols<2, 2>(st, p, l, cols, extra);
     return COGS_LAUNCH_CHECK();
 }

@@ -239,6 +239,9 @@ struct CogsMlaLatent {
     const CogsSeq* seqs; const int* rowseq; const int* rowpos; long layer_off;
 };
 int cogs_k_mla_latent(hipStream_t st, int dtype, const CogsMlaLatent& a, int rows);
+// ... and the query product behind it in one launch (bf16, up to 16 rows, query latents of up to 2048 columns)
+bool cogs_k_gemm_skinny_latent_fits(const CogsGemm& g);
+int cogs_k_gemm_skinny_latent(hipStream_t st, const CogsGemm& g, const CogsMlaLatent& a);
 int cogs_k_mla_gather(hipStream_t st, int dtype, const CogsSeq* seqs, int nseq, int max_ctx, long layer_off, int kvw, void* out);
 struct CogsHeadGemm {      // y[b][h][n] = gate[b][h] * sum_k x[b][h][k] W[h][n][k], then `tail` columns copied from x (zero past tail_n)
     const void* X; long ldxb; int ldxh; const void* W; void* Y; long ldyb; int ldyh; int B, heads, N, K;

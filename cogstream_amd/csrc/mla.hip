@@ -25,6 +25,7 @@
 // 32-multiple] = kvw columns.
 #include "common.h"
 #include "kernels.h"
+#include "mla_latent.h"
 #include "mla_place.h"
 #include "debug.h"
 #include <type_traits>
@@ -46,80 +47,11 @@ __device__ __forceinline__ void split_weights(float p0, float p1, uint32_t& hi, 
     lo = pack_bf2(p0 - bf_lo(hi), p1 - bf_hi(hi));
 }
 
-// sums of up to two values over a 256-thread workgroup, result in every thread; `red` holds 8 floats
-__device__ __forceinline__ void block_sum2(float& a, float& b, float* red) {
-    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-    a = wave_sum(a);
-    b = wave_sum(b);
-    if (lane == 0) { red[wid] = a; red[4 + wid] = b; }
-    __syncthreads();
-    a = (red[0] + red[1]) + (red[2] + red[3]);
-    b = (red[4] + red[5]) + (red[6] + red[7]);
-    __syncthreads();
-}
-
 // ------------------------------------------------------------------------------------------------ latents
-struct LatentArgs {
-    const float* t; long ldt;            // fused down projection, fp32: [q latent | kv latent | key part | gate logits]
-    int qr, qrp, kvr, kvp, dr, krc;      // true / padded query rank, true / padded kv rank, rotated key dims, cache columns of the key part
-    int own_kv, gate_col, heads;         // gate_col < 0: no gate
-    const float* q_norm; const float* kv_norm; float eps;
-    const float* rope; int rope_pairs, rope_first;     // table [rows][rope_pairs][2]; the rotated part starts at pair rope_first
-    void* cq; float* gate;
-    const CogsSeq* seqs; const int* rowseq; const int* rowpos; long layer_off;
-};
-
-// one workgroup per new row: RMS norm of the query latent, RMS norm of the kv latent and rotation of the shared key part
-// (both straight into the sequence's cache row), sigmoid of the gate logits
 template <typename T>
-__global__ __launch_bounds__(256) void mla_latent_kernel(LatentArgs p) {
+__global__ __launch_bounds__(256) void mla_latent_kernel(CogsMlaLatent p) {
     __shared__ float red[8];
-    const int row = blockIdx.x, tid = threadIdx.x;
-    const float* t = p.t + (long)row * p.ldt;
-    float sq = 0.f, skv = 0.f;
-    for (int i = tid * 4; i < p.qrp; i += 1024) {
-        const f32x4 v = *reinterpret_cast<const f32x4*>(t + i);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) sq += v[e] * v[e];
-    }
-    const float* tk = t + p.qrp;
-    if (p.own_kv)
-        for (int i = tid * 4; i < p.kvp; i += 1024) {
-            const f32x4 v = *reinterpret_cast<const f32x4*>(tk + i);
-#pragma unroll
-            for (int e = 0; e < 4; ++e) skv += v[e] * v[e];
-        }
-    block_sum2(sq, skv, red);
-    const float rq = 1.f / sqrtf(sq / (float)p.qr + p.eps);
-    T* cq = reinterpret_cast<T*>(p.cq) + (long)row * p.qrp;
-    for (int i = tid * 4; i < p.qrp; i += 1024) {
-        const f32x4 v = *reinterpret_cast<const f32x4*>(t + i), g = *reinterpret_cast<const f32x4*>(p.q_norm + i);
-        st4_f<T>(cq + i, f32x4{v[0] * rq * g[0], v[1] * rq * g[1], v[2] * rq * g[2], v[3] * rq * g[3]});
-    }
-    if (p.own_kv) {
-        const CogsSeq s = p.seqs[p.rowseq[row]];
-        const int kvw = p.kvp + p.krc;
-        T* c = reinterpret_cast<T*>(s.cache) + p.layer_off * s.max_len + (long)p.rowpos[row] * kvw;
-        const float rk = 1.f / sqrtf(skv / (float)p.kvr + p.eps);
-        for (int i = tid * 4; i < p.kvp; i += 1024) {
-            const f32x4 v = *reinterpret_cast<const f32x4*>(tk + i), g = *reinterpret_cast<const f32x4*>(p.kv_norm + i);
-            st4_f<T>(c + i, f32x4{v[0] * rk * g[0], v[1] * rk * g[1], v[2] * rk * g[2], v[3] * rk * g[3]});
-        }
-        const float* tr = tk + p.kvp;
-        const float* cs = p.rope + ((long)row * p.rope_pairs + p.rope_first) * 2;
-        for (int i = tid * 2; i < p.krc; i += 512) {
-            float a = 0.f, b = 0.f;
-            if (i < p.dr) {
-                const float u = tr[i], v = tr[i + 1], co = cs[i], si = cs[i + 1];
-                a = fmaf(-v, si, u * co);
-                b = fmaf(u, si, v * co);
-            }
-            st_f<T>(c + p.kvp + i, a);
-            st_f<T>(c + p.kvp + i + 1, b);
-        }
-    }
-    if (p.gate_col >= 0)
-        for (int i = tid; i < p.heads; i += 256) p.gate[(long)row * p.heads + i] = 1.f / (1.f + expf(-t[p.gate_col + i]));
+    latent_row<T, true>(p, blockIdx.x, threadIdx.x, red);
 }
 
 // cached rows of every sequence of the batch, back to back (the expansion GEMM's A operand when there is more than one)
@@ -994,13 +926,8 @@ int launch_decode(hipStream_t st, const MlaDecodeArgs& p, int nblk, int nsplit) 
 int cogs_k_mla_latent(hipStream_t st, int dtype, const CogsMlaLatent& a, int rows) {
     if (rows <= 0) return COGS_OK;
     if (a.qrp % 4 || a.kvp % 4 || a.krc % 2 || a.ldt % 4 || a.dr % 2) return COGS_E_INVALID;
-    LatentArgs p;
-    p.t = a.t; p.ldt = a.ldt; p.qr = a.qr; p.qrp = a.qrp; p.kvr = a.kvr; p.kvp = a.kvp; p.dr = a.dr; p.krc = a.krc;
-    p.own_kv = a.own_kv; p.gate_col = a.gate_col; p.heads = a.heads; p.q_norm = a.q_norm; p.kv_norm = a.kv_norm; p.eps = a.eps;
-    p.rope = a.rope; p.rope_pairs = a.rope_pairs; p.rope_first = a.rope_first; p.cq = a.cq; p.gate = a.gate;
-    p.seqs = a.seqs; p.rowseq = a.rowseq; p.rowpos = a.rowpos; p.layer_off = a.layer_off;
-    if (dtype == COGS_DT_BF16) hipLaunchKernelGGL(mla_latent_kernel<bf16_t>, dim3(rows), dim3(256), 0, st, p);
-    else hipLaunchKernelGGL(mla_latent_kernel<float>, dim3(rows), dim3(256), 0, st, p);
+    if (dtype == COGS_DT_BF16) hipLaunchKernelGGL(mla_latent_kernel<bf16_t>, dim3(rows), dim3(256), 0, st, a);
+    else hipLaunchKernelGGL(mla_latent_kernel<float>, dim3(rows), dim3(256), 0, st, a);
     return COGS_LAUNCH_CHECK();
 }
 

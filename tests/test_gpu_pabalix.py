@@ -260,6 +260,33 @@ def test_forms_and_kernels_agree(dev):
             assert rms_err(run(e, toks, [20, 380, *range(381, 400)]), lg) < TOL[torch.bfloat16], (name, value)
 
 
+@pytest.mark.parametrize("heads,q_rank", [(3, 40), (3, 64), (5, 1000), (3, 1024), (80, 1100), (3, 2048), (160, 300), (3, 2100)])
+@pytest.mark.parametrize("rows", [2, 8, 9, 16, 17])
+def test_query_products_that_norm_their_rows(dev, heads, q_rank, rows):
+    """one token of up to 16 sequences: the query product forms its rows' norms itself (up to 2048 columns of query latent; 17 rows and 2100 columns take the
+    launch in front), 16, 32 and 64 columns a workgroup, fewer slices of K than its waves have in flight and more; a layer with gates and one that borrows
+    its rows and has none, so that no workgroup is left for rows. Logits and the rows that went into the caches against the oracle and the launch of their own"""
+    from cogstream_amd import _lib as L
+    cfg = config([dict(mixer(G, heads=heads, q_rank=q_rank, dim=24, rot=16, vdim=16), ff=None), dict(mixer(A, heads=3, q_rank=q_rank, dim=24, rot=16), ff=None),
+                  dict(mixer(A, heads=3, q_rank=q_rank, dim=24, rot=16, kv_from=1), ff=None)], width=64, vocab=96)
+    st = state(cfg)
+    e = engine(cfg, st, torch.bfloat16)
+    toks = [tokens(cfg, 4 + i % 3, seed=i) for i in range(rows)]
+    s = sequences(e)
+    s.step([(i, t[:-1], []) for i, t in enumerate(toks)])
+    got = s.step([(i, t[-1:], [0]) for i, t in enumerate(toks)])
+    want = torch.cat([po.forward(cfg, double(st), t)[0][-1:] for t in toks])
+    assert rms_err(got, want) < TOL[torch.bfloat16]
+    other = sequences(e)
+    with L.debug_switch("gemm_skinny", 0):
+        other.step([(i, t[:-1], []) for i, t in enumerate(toks)])
+        other.step([(i, t[-1:], [0]) for i, t in enumerate(toks)])
+    for i, t in enumerate(toks):
+        for a, b in zip(s.caches[i]._blocks(), other.caches[i]._blocks()):
+            a, b = a[..., :len(t), :].float(), b[..., :len(t), :].float()
+            assert bool((a - b).abs().max() <= TOL[torch.bfloat16] * b.abs().max())
+
+
 @pytest.mark.parametrize("dim,rot", [(128, 64), (96, 64), (64, 32), (32, 64)])
 def test_columns_that_are_not_rotated(dev, dim, rot):
     """the query product reads no factors for blocks of columns in front of a head's rotated part (64 columns a wave, 32 in the small tiles; heads where such
