@@ -4,7 +4,7 @@
 //
 // Everything here is fp32, whatever the model's dtype: the fused projection's output t, the convolution's memory, S, and all products.
 //   prompts   delta_inputs (convolution, silu, unit vectors, beta, ln g) -> delta_chunk + delta_scan (32 tokens at a time on the fp32
-//             matrix instructions) -> delta_out (norm and gate); delta_tail keeps the convolution's last inputs
+//             matrix instructions; workgroups behind the scan's keep the convolution's last inputs) -> delta_out (norm and gate)
 //   decode    delta_step: one launch per layer does all of it
 // A token-by-token kernel (delta_recur) serves the sizes the chunked pair has no instance for.
 //
@@ -159,15 +159,16 @@ __global__ __launch_bounds__(256) void delta_inputs_any_kernel(CogsDelta p) {
 }
 
 // the last inputs of the convolution into the ring (behind every reader of the old ones)
-__global__ __launch_bounds__(256) void delta_tail_kernel(CogsDelta p) {
-    const CogsSeq s = p.seqs[blockIdx.y];
+__device__ __forceinline__ void conv_tail(const CogsDelta& p, const CogsSeq& s, int block, int blocks) {
     float* ring = s.state + p.state_off + (long)p.heads * p.dkp * p.dvp;
     const int n = min(s.len, p.taps);
-    for (int i = blockIdx.x * 256 + threadIdx.x; i < n * p.channels; i += gridDim.x * 256) {
+    for (int i = block * 256 + threadIdx.x; i < n * p.channels; i += blocks * 256) {
         const int r = s.len - n + i / p.channels, c = i % p.channels;
         ring[(long)((s.pos0 + r) % p.taps) * p.channels + c] = p.t[(long)(s.row0 + r) * p.ldt + c];
     }
 }
+
+__global__ __launch_bounds__(256) void delta_tail_kernel(CogsDelta p) { conv_tail(p, p.seqs[blockIdx.y], blockIdx.x, gridDim.x); }
 
 // token by token, a thread per column of S, S in memory
 __global__ __launch_bounds__(64) void delta_recur_kernel(CogsDelta p) {
@@ -332,13 +333,17 @@ struct ScanIn {
 // scan, 54 instead of 63 matrix instructions, two terms of V's size were rounded and cancelled: read-outs of 8 recurring pairs were off
 // by 1.2e-7 of them instead of 8.2e-8, values read back from the state by 1.2e-7 instead of 3.5e-8.) K S and Q S are two chains each, and
 // P U and the state's growth sums of their own: chained to what they are added to, they were rounded at its size.
+// The workgroups from `scan` on keep the convolution's last inputs, which nothing here reads: a launch for them alone, between the inputs and
+// the chunks, was 4.9 us a layer (prompts of 100 rows, width 2048 815 -> 793 us, of 4096 5048 -> 5022).
 template <int NK>
-__global__ __launch_bounds__(256, NK > 2 ? 1 : 2) void delta_scan_kernel(CogsDelta p) {
+__global__ __launch_bounds__(256, NK > 2 ? 1 : 2) void delta_scan_kernel(CogsDelta p, int scan) {
     __shared__ __attribute__((aligned(16))) f32x4 red[2][4][4][64];
-    // workgroups go round the XCDs: the columns of a head stay on one, whose L2 then serves its K and Q once
-    const int ng = p.dvp >> 4, place = blockIdx.x >> 3, h = (blockIdx.x & 7) + 8 * (place / ng), col0 = (place % ng) * 16, seq = blockIdx.z;
-    if (h >= p.heads) return;
+    const int seq = blockIdx.z;
     const CogsSeq s = p.seqs[seq];
+    if ((int)blockIdx.x >= scan) { conv_tail(p, s, blockIdx.x - scan, gridDim.x - scan); return; }
+    // workgroups go round the XCDs: the columns of a head stay on one, whose L2 then serves its K and Q once
+    const int ng = p.dvp >> 4, place = blockIdx.x >> 3, h = (blockIdx.x & 7) + 8 * (place / ng), col0 = (place % ng) * 16;
+    if (h >= p.heads) return;
     const int tid = threadIdx.x, lane = tid & 63, li = lane & 15, g = lane >> 4;
     const int wid = __builtin_amdgcn_readfirstlane(tid >> 6), half = wid & 1, fin = wid >> 1;
     const int kh = h / (p.heads / p.kv_heads);
@@ -853,15 +858,16 @@ size_t cogs_k_delta_rec_floats(int rows, int nseq, int heads) { return (size_t)(
 int cogs_k_delta_prompt(hipStream_t st, int dtype, const CogsDelta& a, int rows, int nseq, int max_new) {
     if (!sizes_ok(a) || rows <= 0 || nseq <= 0 || nseq > 65535 || a.heads > 65535) return COGS_E_INVALID;
     launch_inputs(st, a, rows, nseq, max_new);
-    const int keep = (max_new < a.taps ? max_new : a.taps) * a.channels;
-    hipLaunchKernelGGL(delta_tail_kernel, dim3((keep + 1023) / 1024, nseq), dim3(256), 0, st, a);
+    const int keep = (max_new < a.taps ? max_new : a.taps) * a.channels, tail = (keep + 1023) / 1024;
     if (a.dkp <= 256 && g_cogs_debug.delta_chunk != 0) {
         hipLaunchKernelGGL(delta_chunk_kernel, dim3((max_new + CH - 1) / CH, a.heads, nseq), dim3(256), 0, st, a);
-        const dim3 grid((a.heads + 7) / 8 * 8 * (a.dvp / 16), 1, nseq);
-        if (a.dkp <= 64) hipLaunchKernelGGL(delta_scan_kernel<1>, grid, dim3(256), 0, st, a);
-        else if (a.dkp <= 128) hipLaunchKernelGGL(delta_scan_kernel<2>, grid, dim3(256), 0, st, a);
-        else hipLaunchKernelGGL(delta_scan_kernel<4>, grid, dim3(256), 0, st, a);
+        const int scan = (a.heads + 7) / 8 * 8 * (a.dvp / 16);
+        const dim3 grid(scan + (tail + 7) / 8 * 8, 1, nseq);      // (a multiple of 8: the heads of every sequence keep their XCDs)
+        if (a.dkp <= 64) hipLaunchKernelGGL(delta_scan_kernel<1>, grid, dim3(256), 0, st, a, scan);
+        else if (a.dkp <= 128) hipLaunchKernelGGL(delta_scan_kernel<2>, grid, dim3(256), 0, st, a, scan);
+        else hipLaunchKernelGGL(delta_scan_kernel<4>, grid, dim3(256), 0, st, a, scan);
     } else {
+        hipLaunchKernelGGL(delta_tail_kernel, dim3(tail, nseq), dim3(256), 0, st, a);
         hipLaunchKernelGGL(delta_recur_kernel, dim3((a.dvp + 63) / 64, a.heads, nseq), dim3(64), 0, st, a);
     }
     const bool half = a.dvp <= 128 && g_cogs_debug.delta_out_wave == 0;
