@@ -61,7 +61,7 @@ namespace {
 
 struct Work {
     float* x; void *h, *y[COGS_CHAIN], *cq, *q, *att, *act, *hn, *ctx, *kvx, *qlat, *olat;
-    float *ypart, *t32, *gate, *rope, *part, *dq, *dk, *dv, *dbg, *dout, *drec;
+    float *ypart, *t32, *gate, *rope, *part, *dq, *dk, *dkt, *dv, *dbg, *dout, *drec;
     CogsSeq* seqs; int *rowseq, *rowpos, *want;
     size_t bytes;
 };
@@ -117,9 +117,11 @@ Work carve(const CogsDecoder& d, int S, int nseq, int64_t C, int n_want, void* w
         if (nseq > 1) k.ctx = c.take((size_t)C * d.max_kvw * es);
     }
     if (!token_step(S, nseq) && d.max_dheads > 0) {
-        k.dq = (float*)c.take(n * d.max_dqk * 4);
-        k.dk = (float*)c.take(n * d.max_dqk * 4);
-        k.dv = (float*)c.take(n * d.max_dv * 4);
+        const size_t tokens = (size_t)cogs_k_delta_slots(S, nseq) * 32;
+        k.dq = (float*)c.take(tokens * d.max_dqk * 4);
+        k.dk = (float*)c.take(tokens * d.max_dqk * 4);
+        k.dkt = (float*)c.take(tokens * d.max_dqk * 4);
+        k.dv = (float*)c.take(tokens * d.max_dv * 4);
         k.dout = (float*)c.take(n * d.max_dv * 4);
         k.dbg = (float*)c.take(n * d.max_dheads * 2 * 4);
         k.drec = (float*)c.take(cogs_k_delta_rec_floats(S, nseq, d.max_dheads) * 4);
@@ -302,7 +304,7 @@ struct Step {
             COGS_TRY(lin(g));
         }
         CogsDelta a{k.t32, G.ldt, m.heads, G.headsp, m.kv_heads, G.dk, G.dv, m.vdim, m.taps, G.channels, m.conv, m.neg_a, m.dt_bias, m.norm, d.w.eps,
-                    1.f / sqrtf((float)m.dim), S, k.dq, k.dk, k.dv, k.dbg, k.dout, k.drec, k.att, G.oin, k.seqs, k.rowseq, k.rowpos, run.state_off};
+                    1.f / sqrtf((float)m.dim), S, cogs_k_delta_slots(S, nseq), k.dq, k.dk, k.dkt, k.dv, k.dbg, k.dout, k.drec, k.att, G.oin, k.seqs, k.rowseq, k.rowpos, run.state_off};
         {
             PROF(COGS_PROF_ATTN);
             if (token_step(S, nseq)) COGS_TRY(cogs_k_delta_step(st, d.w.dtype, a, nseq));

@@ -16,9 +16,9 @@
 // exponentials do not depend on S: delta_chunk forms them for all chunks at once, T by forward substitution. delta_scan walks a
 // sequence's chunks: a workgroup owns 16 columns of S, its four waves the 16-row tiles of S in turn.
 // The scan's chunks follow one another, so what counts is the length of one: K S, a sum over the waves, the product with T, the new
-// state. Operands in the order of the lanes and buffer loads without address arithmetic took it from 2.1 to 1.45 us a chunk (4096
-// tokens, 16 heads of 128: scan 273 -> 188 us, delta_chunk 30). Two thirds of that are matrix instructions (63 of 14 ns), the rest LDS
-// exchange and the loads' share of issue.
+// state. Operands in the order of the lanes and buffer loads without address arithmetic took it from 2.1 to 1.4 us a chunk, 3400 cycles. 63 matrix
+// instructions are 2000 of them, the loads 300 (a chunk over and over in registers: 3100); the rest are some hundred vector instructions, which do not run
+// beside fp32 matrix instructions, and the exchange through LDS.
 // MFMA layout: a 16x16 accumulator holds rows 4 g + r in register r of lane group g, which is the B operand of the r-th of four
 // 4-deep steps if k is taken in the order 4 g + r -- so S, V - diag(e^G) K S and U go from product to product in their registers, and A operands are
 // 16-byte loads of four neighbouring k.
@@ -32,6 +32,38 @@ constexpr int CH = 32;                        // tokens of a chunk
 constexpr int TILE = 256;                     // floats of a 16x16 tile, row-major
 constexpr int EXPS = 6 * TILE;                // per chunk and head: P tiles (0,0) (1,0) (1,1) | T beta tiles | e^G | e^{G_last - G} | e^{G_last}, ..;
 constexpr int REC = EXPS + 3 * CH;            // P as A operands [4 steps][64 lanes], T beta as [64 lanes][4 steps]
+
+// Chunks have q, k and v as the operands of the scan's 16x16 tiles, [chunk][16 tokens a][16 columns t][64 lanes][4 floats]: q and k with a token per lane
+// (lane 16 g + li: token li, columns 4 g ..), k once more and v with a column per lane (column li, tokens 4 g ..). A sequence starts on a chunk of
+// its own, tokens past its end are zeros. An operand is one load of 1 KiB in a row, 25 of them a wave and chunk; as rows it was sixteen lines of 64 bytes, and those
+// with a column per lane four loads of 4 bytes a lane, 43 in all. 4096 rows, 16 heads of 128: scan 206 -> 198 us, 32 heads 242 -> 227 and the chunks
+// 57 -> 49; the inputs 31 -> 36 (k is written twice). Prompts of 4096 rows, width 2048 5021 -> 4963 us, of 700 1450 -> 1428, of 300, width 4096
+// 2101 -> 2081. (T, v and the exponentials, which all four waves read, through LDS instead of into each one's registers: 206 again.)
+__device__ __forceinline__ int token_major(int tiles, int a, int row, int c) {      // first of four columns c ..
+    return (a * tiles + (c >> 4)) * TILE + (((c & 15) >> 2) * 16 + row) * 4 + (c & 3);
+}
+__device__ __forceinline__ int column_major(int tiles, int a, int row, int c) {     // first of four rows
+    return (a * tiles + (c >> 4)) * TILE + ((row >> 2) * 16 + (c & 15)) * 4 + (row & 3);
+}
+// floats in front of a chunk of a head of n columns (a later sequence starts behind the chunks of an earlier one)
+__device__ __forceinline__ long chunk_at(const CogsDelta& p, const CogsSeq& s, int seq, int chunk, int head, int n) {
+    return ((long)head * p.slots + s.row0 / CH + seq + chunk) * CH * n;
+}
+// four lanes' four values each, transposed
+__device__ __forceinline__ void quad_transpose(f32x4& v, int lane) {
+#pragma unroll
+    for (int b = 1; b <= 2; b *= 2) {
+        const bool up = lane & b;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            if (i & b) continue;
+            const float lo = v[i], hi = v[i + b], give = up ? lo : hi;
+            const float got = b == 1 ? lane_xor_dpp<1>(give) : lane_xor_dpp<2>(give);
+            v[i] = up ? got : lo;
+            v[i + b] = up ? hi : got;
+        }
+    }
+}
 
 __device__ __forceinline__ float unit_scale(float ss) { return 1.f / sqrtf(ss + 1e-6f); }
 __device__ __forceinline__ float sigmoid_f(float x) { return 1.f / (1.f + expf(-x)); }
@@ -55,10 +87,11 @@ __device__ __forceinline__ float silu_q(float y) { return y * __builtin_amdgcn_r
 // the convolution's window in registers and the whole run's inputs requested ahead. E: 64-channel steps of a head; TAPS: taps, rounded up
 template <int E, int TAPS, int RUN>
 __global__ __launch_bounds__(256) void delta_inputs_kernel(CogsDelta p) {
-    const CogsSeq s = p.seqs[blockIdx.z];
+    const int seq = blockIdx.z;
+    const CogsSeq s = p.seqs[seq];
     const int lane = threadIdx.x & 63, wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int i0 = blockIdx.x * RUN, n = min(RUN, s.len - i0);
-    if (n <= 0) return;
+    if (i0 >= (s.len + CH - 1) / CH * CH) return;              // (runs of zeros behind the end belong to its chunk)
     const int nqk = 2 * p.kv_heads, nv = p.heads * p.dvp, units = nqk + (nv + 64 * E - 1) / (64 * E);
     const int unit = blockIdx.y * 4 + wid, v0 = nqk * p.dkp;
     const long row0 = s.row0 + i0;
@@ -83,52 +116,64 @@ __global__ __launch_bounds__(256) void delta_inputs_kernel(CogsDelta p) {
 #pragma unroll
     for (int r = 0; r < RUN; ++r)
 #pragma unroll
-        for (int e = 0; e < E; ++e) in[TAPS - 1 + r][e] = x[(long)min(r, n - 1) * p.ldt + ch[e]];
+        for (int e = 0; e < E; ++e) in[TAPS - 1 + r][e] = x[(long)min(r, n - 1) * p.ldt + ch[e]];      // (n <= 0: the sequence's last row)
 #pragma unroll
     for (int j = 1; j < TAPS; ++j)
 #pragma unroll
         for (int e = 0; e < E; ++e) {
             const int i = i0 - j, pos = s.pos0 + i;
             float v = 0.f;
-            if (j < p.taps && pos >= 0) v = i >= 0 ? x[ch[e] - (long)j * p.ldt] : ring[(long)(pos % p.taps) * p.channels + ch[e]];
+            if (j < p.taps && pos >= 0 && n > 0) v = i >= 0 ? x[ch[e] - (long)j * p.ldt] : ring[(long)(pos % p.taps) * p.channels + ch[e]];
             in[TAPS - 1 - j][e] = v;
         }
 #pragma unroll
     for (int j = 0; j < TAPS; ++j)
 #pragma unroll
         for (int e = 0; e < E; ++e) w[j][e] = j < p.taps ? p.conv[(long)(p.taps - 1 - j) * p.channels + ch[e]] : 0.f;
-    float* out[E];                                    // (v's pieces may cross heads)
-#pragma unroll
-    for (int e = 0; e < E; ++e) {
-        const int c = ch[e] - v0, hv = c / p.dvp;
-        out[e] = is_v ? p.v + ((long)hv * p.rows + row0) * p.dvp + (c - hv * p.dvp)
-                      : (unit < p.kv_heads ? p.q : p.k) + ((long)(unit % p.kv_heads) * p.rows + row0) * p.dkp + (ch[e] - c0);
-    }
-    const long ld = is_v ? p.dvp : p.dkp;
     const float scale = unit < p.kv_heads ? p.q_scale : 1.f;
+    f32x4 y[RUN / 4][E];
 #pragma unroll
     for (int r = 0; r < RUN; ++r) {
-        float y[E], ss = 0.f;
+        float ss = 0.f;
 #pragma unroll
         for (int e = 0; e < E; ++e) {
             float a = w[0][e] * in[TAPS - 1 + r][e];
 #pragma unroll
             for (int j = 1; j < TAPS; ++j) a = fmaf(w[j][e], in[TAPS - 1 + r - j][e], a);
-            y[e] = lane + 64 * e < size ? silu_q(a) : 0.f;
-            ss = fmaf(y[e], y[e], ss);
+            const float v = lane + 64 * e < size ? silu_q(a) : 0.f;
+            ss = fmaf(v, v, ss);
+            y[r >> 2][e][r & 3] = v;
         }
         const float f = is_v ? 1.f : unit_scale(wave_sum(ss)) * scale;
 #pragma unroll
-        for (int e = 0; e < E; ++e)
-            if (r < n && lane + 64 * e < size) out[e][r * ld] = y[e] * f;
+        for (int e = 0; e < E; ++e) y[r >> 2][e][r & 3] = r < n ? y[r >> 2][e][r & 3] * f : 0.f;
+    }
+    const int a = (i0 >> 4) & 1, first = i0 & 15;
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+        const bool mine = lane + 64 * e < size;
+        const int c = ch[e] - (is_v ? v0 : c0), width = is_v ? p.dvp : p.dkp, head = is_v ? c / width : unit % p.kv_heads, col = is_v ? c - head * width : c;
+        const long at = chunk_at(p, s, seq, i0 / CH, head, width);      // (v's pieces may cross heads)
+        float* const by_column = is_v ? p.v : p.kt;
+#pragma unroll
+        for (int q = 0; q < RUN / 4; ++q) {
+            f32x4 v = y[q][e];
+            if (mine && unit >= p.kv_heads) *reinterpret_cast<f32x4*>(by_column + at + column_major(width >> 4, a, first + 4 * q, col)) = v;
+            if (is_v) continue;
+            quad_transpose(v, lane);
+            if (mine) *reinterpret_cast<f32x4*>((unit < p.kv_heads ? p.q : p.k) + at + token_major(width >> 4, a, first + 4 * q + (lane & 3), col & ~3)) = v;
+        }
     }
 }
 
 // the same for any size: one workgroup per new row; a wave per q / k head
+template <bool TILES>
 __global__ __launch_bounds__(256) void delta_inputs_any_kernel(CogsDelta p) {
     const int row = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
     const int sq = p.rowseq[row], pos = p.rowpos[row];
     const CogsSeq s = p.seqs[sq];
+    const int i = row - s.row0, chunk = i / CH;
+    const int after = TILES && i == s.len - 1 ? (i / CH + 1) * CH - s.len : 0;       // rows of zeros that this one is followed by
     const float* x = p.t + (long)row * p.ldt;
     const float* ring = s.state + p.state_off + (long)p.heads * p.dkp * p.dvp;
     const int back = row - s.row0;
@@ -142,15 +187,32 @@ __global__ __launch_bounds__(256) void delta_inputs_any_kernel(CogsDelta p) {
         }
         float f = unit_scale(wave_sum(ss));
         if (j < p.kv_heads) f *= p.q_scale;
-        float* o = (j < p.kv_heads ? p.q : p.k) + ((long)(j % p.kv_heads) * p.rows + row) * p.dkp;
+        float* o = j < p.kv_heads ? p.q : p.k;
+        const int head = j % p.kv_heads;
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
             const int d = lane + 64 * e;
-            if (d < p.dkp) o[d] = v[e] * f;
+            if (d >= p.dkp) continue;
+            if constexpr (TILES) {
+                const long at = chunk_at(p, s, sq, chunk, head, p.dkp);
+                for (int z = 0; z <= after; ++z) {
+                    const int r = i + z, b = (r >> 4) & 1;
+                    const float y = z ? 0.f : v[e] * f;
+                    o[at + token_major(p.dkp >> 4, b, r & 15, d)] = y;
+                    if (j >= p.kv_heads) p.kt[at + column_major(p.dkp >> 4, b, r & 15, d)] = y;
+                }
+            } else o[((long)head * p.rows + row) * p.dkp + d] = v[e] * f;
         }
     }
     const int v0 = 2 * p.kv_heads * p.dkp, nv = p.heads * p.dvp;
-    for (int i = tid; i < nv; i += 256) p.v[((long)(i / p.dvp) * p.rows + row) * p.dvp + i % p.dvp] = conv_silu(p, x, ring, v0 + i, pos, back);
+    for (int c = tid; c < nv; c += 256) {
+        const float y = conv_silu(p, x, ring, v0 + c, pos, back);
+        const int head = c / p.dvp, d = c - head * p.dvp;
+        if constexpr (TILES) {
+            const long at = chunk_at(p, s, sq, chunk, head, p.dvp);
+            for (int z = 0; z <= after; ++z) p.v[at + column_major(p.dvp >> 4, ((i + z) >> 4) & 1, (i + z) & 15, d)] = z ? 0.f : y;
+        } else p.v[((long)head * p.rows + row) * p.dvp + d] = y;
+    }
     const float *tb = x + v0 + 2 * nv, *ta = tb + p.headsp;
     for (int h = tid; h < p.heads; h += 256) {
         p.bg[((long)row * p.heads + h) * 2] = sigmoid_f(tb[h]);
@@ -225,8 +287,8 @@ __global__ __launch_bounds__(256) void delta_chunk_kernel(CogsDelta p) {
     const int wid = (__builtin_amdgcn_readfirstlane(tid >> 6) + turn + blockIdx.x) & 3;
     const long row0 = s.row0 + chunk * CH;
     const int kh = h / (p.heads / p.kv_heads);
-    const float* K = p.k + ((long)kh * p.rows + row0) * p.dkp;
-    const float* Q = p.q + ((long)kh * p.rows + row0) * p.dkp;
+    const float* K = p.k + chunk_at(p, s, seq, chunk, kh, p.dkp);
+    const float* Q = p.q + chunk_at(p, s, seq, chunk, kh, p.dkp);
     float* rec = chunk_rec(p, s, seq, chunk, h);
     const int ta = wid > 0 ? 1 : 0, tb = wid == 2 ? 1 : 0;
     if (wid == 3 && lane < CH) {
@@ -244,16 +306,15 @@ __global__ __launch_bounds__(256) void delta_chunk_kernel(CogsDelta p) {
     }
     f32x4 kk = {0.f, 0.f, 0.f, 0.f}, qk = kk;
     if (wid < 3) {
-        const long ra = min(16 * ta + li, n - 1), rb = min(16 * tb + li, n - 1);
-        const float *ka = K + ra * p.dkp + 4 * g, *qa = Q + ra * p.dkp + 4 * g, *kb = K + rb * p.dkp + 4 * g;
+        const int da = 16 * p.dkp * ta + 4 * lane, db = 16 * p.dkp * tb + 4 * lane;
         for (int d = 0; d < p.dkp; d += 64) {          // four 16-wide steps in flight; steps past the end are not multiplied
             f32x4 a[4], b[4], q[4];
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
-                const int o = min(d + 16 * e, p.dkp - 16);
-                a[e] = *reinterpret_cast<const f32x4*>(ka + o);
-                b[e] = *reinterpret_cast<const f32x4*>(kb + o);
-                q[e] = *reinterpret_cast<const f32x4*>(qa + o);
+                const int o = 16 * min(d + 16 * e, p.dkp - 16);
+                a[e] = *reinterpret_cast<const f32x4*>(K + da + o);
+                b[e] = *reinterpret_cast<const f32x4*>(K + db + o);
+                q[e] = *reinterpret_cast<const f32x4*>(Q + da + o);
             }
             __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
@@ -363,36 +424,24 @@ __global__ __launch_bounds__(256, NK > 2 ? 1 : 2) void delta_scan_kernel(CogsDel
             for (int r = 0; r < 4; ++r) st[n][r] = S[(long)(16 * t + 4 * g + r) * p.dvp];
     }
     const int nc = (s.len + CH - 1) / CH;
-    // a lane's places in a chunk's rows (bytes)
-    int qo[2], to[2][4], vo[2][4], oo[2];
+    // a lane's places in a chunk's tiles and read-outs (bytes)
+    int oo[2];
     const int tmo = lane * 16, po = lane * 4 + wid * 256, ego = 16 * g;
     int zo = 0;
     asm("" : "+v"(zo));                          // (a scalar load would share its counter with LDS)
 #pragma unroll
     for (int r = 0; r < 2; ++r) oo[r] = ((16 * fin + 4 * g + 2 * half + r) * ldv + li) * 4;
-#pragma unroll
-    for (int a = 0; a < 2; ++a) {
-        qo[a] = ((16 * a + li) * ld + 4 * g) * 4;
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            to[a][r] = ((16 * a + 4 * g + r) * ld + li) * 4;
-            vo[a][r] = ((16 * a + 4 * g + r) * ldv + li) * 4;
-        }
-    }
-    // buffer loads: a scalar base per array and chunk, a lane's place, a scalar piece -- no address arithmetic per load; rows past the
-    // sequence's end, and K's columns of a tile past S's end, lie behind the buffer's size and read as zero
-    struct From { float *k, *q, *v, *rec; };
-    const From f0{p.k + ((long)kh * p.rows + s.row0) * ld, p.q + ((long)kh * p.rows + s.row0) * ld, p.v + ((long)h * p.rows + s.row0) * ldv + col0, chunk_rec(p, s, seq, 0, h)};
+    // buffer loads: a scalar base per array and chunk, a lane's place, a scalar piece -- no address arithmetic per load; K's columns of a tile
+    // past S's end lie behind the buffer's size and read as zero
+    struct From { float *k, *q, *kt, *v, *rec; };
+    const long qk0 = chunk_at(p, s, seq, 0, kh, ld);
+    const From f0{p.k + qk0, p.q + qk0, p.kt + qk0, p.v + chunk_at(p, s, seq, 0, h, ldv) + col0 * 16, chunk_rec(p, s, seq, 0, h)};
     From f = f0;
     constexpr int bytes_rec = REC * 4;
-    int bytes_q, bytes_v, bytes_k[NK];
-    auto sizes = [&](int rows) {
-        bytes_q = rows * ld * 4;
-        bytes_v = (rows - 1) * ldv * 4 + 64;
+    const int bytes_q = CH * ld * 4, bytes_v = CH * ldv * 4 - col0 * 64;
+    int bytes_k[NK];
 #pragma unroll
-        for (int n = 0; n < NK; ++n) bytes_k[n] = wid + 4 * n < tiles ? bytes_q : 0;
-    };
-    sizes(min(CH, s.len));
+    for (int n = 0; n < NK; ++n) bytes_k[n] = wid + 4 * n < tiles ? bytes_q : 0;
     auto at4 = [](float* base, int size, int lane_off, int off) {
         return __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(__builtin_amdgcn_make_buffer_rsrc(base, 0, size, 0x00020000), lane_off, off, 0));
     };
@@ -403,19 +452,19 @@ __global__ __launch_bounds__(256, NK > 2 ? 1 : 2) void delta_scan_kernel(CogsDel
     int at = 0;                                                // the chunk f points to
     auto advance = [&] {                                       // (the last chunk is loaded again rather than nothing)
         at = min(at + 1, nc - 1);
-        f = From{f0.k + at * step_k, f0.q + at * step_k, f0.v + at * step_v, f0.rec + at * step_rec};
-        sizes(min(CH, s.len - at * CH));
+        f = From{f0.k + at * step_k, f0.q + at * step_k, f0.kt + at * step_k, f0.v + at * step_v, f0.rec + at * step_rec};
     };
     // load i of a chunk, in the order of their use, the 16-byte ones first
-    constexpr int L_Q = 2 * NK, L_E = L_Q + 2 * NK, L_T = L_E + 4, L_V = L_T + 3, L_G = L_V + 8, L_KT = L_G + 1, L_PM = L_KT + 8 * NK, L_ALL = L_PM + 3;
+    constexpr int L_Q = 2 * NK, L_E = L_Q + 2 * NK, L_T = L_E + 4, L_V = L_T + 3, L_KT = L_V + 2, L_G = L_KT + 2 * NK, L_PM = L_G + 1, L_ALL = L_PM + 3;
     auto load = [&](ScanIn<NK>& in, int i) {
-        if (i < L_Q) in.k[i / NK][i % NK] = at4(f.k, bytes_q, qo[i / NK], 64 * tn[i % NK]);
-        else if (i < L_E) { const int j = i - L_Q; in.q[j / NK][j % NK] = at4(f.q, bytes_q, qo[j / NK], 64 * tn[j % NK]); }
+        auto tile = [&](int j) { return (j / NK * tiles + tn[j % NK]) * TILE * 4; };
+        if (i < L_Q) in.k[i / NK][i % NK] = at4(f.k, bytes_q, tmo, tile(i));
+        else if (i < L_E) { const int j = i - L_Q; in.q[j / NK][j % NK] = at4(f.q, bytes_q, tmo, tile(j)); }
         else if (i < L_T) { const int j = i - L_E; (j & 2 ? in.ec : in.eg)[j & 1] = at4(f.rec, bytes_rec, ego, (EXPS + (j & 2 ? CH : 0) + 16 * (j & 1)) * 4); }
         else if (i < L_V) in.tm[i - L_T] = at4(f.rec, bytes_rec, tmo, (3 + i - L_T) * TILE * 4);
-        else if (i < L_G) { const int j = i - L_V; in.v[j >> 2][j & 3] = at1(f.v, bytes_v, vo[j >> 2][j & 3], 0); }
-        else if (i < L_KT) in.gl = at1(f.rec, bytes_rec, zo, (EXPS + 2 * CH) * 4);
-        else if (i < L_PM) { const int j = i - L_KT; in.kt[(j >> 2) & 1][j >> 3][j & 3] = at1(f.k, bytes_k[j >> 3], to[(j >> 2) & 1][j & 3], 64 * tn[j >> 3]); }
+        else if (i < L_KT) { const int j = i - L_V; in.v[j] = at4(f.v, bytes_v, tmo, j * ldv * 64); }
+        else if (i < L_G) { const int j = i - L_KT; in.kt[j / NK][j % NK] = at4(f.kt, bytes_k[j % NK], tmo, tile(j)); }
+        else if (i < L_PM) in.gl = at1(f.rec, bytes_rec, zo, (EXPS + 2 * CH) * 4);
         else if (i < L_ALL) in.pm[i - L_PM] = at1(f.rec, bytes_rec, po, (i - L_PM) * TILE * 4);
     };
     const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
@@ -442,7 +491,7 @@ __global__ __launch_bounds__(256, NK > 2 ? 1 : 2) void delta_scan_kernel(CogsDel
     // chunk c from `in`, the next one into nx
     auto chunk = [&](int c, const ScanIn<NK>& in, ScanIn<NK>& nx) {
         constexpr int STEPS = 24 * NK + 12;                    // matrix instructions that bring loads with them
-        constexpr int LONG = L_V, WORK = L_ALL + LONG;         // the four waves' 16-byte loads take the time of two matrix instructions, the others half
+        constexpr int LONG = L_G, WORK = L_ALL + LONG;         // the four waves' 16-byte loads take the time of two matrix instructions, the others half
         static_assert(WORK <= 2 * STEPS);
         int step = 0, next = 0;
         auto due = [&] { return next < L_ALL && (next + min(next, LONG)) * STEPS < (step + 1) * WORK; };
@@ -839,11 +888,11 @@ int launch_step(hipStream_t st, const CogsDelta& p, int nseq) {
 
 void launch_inputs(hipStream_t st, const CogsDelta& a, int rows, int nseq, int max_new) {
     const int nv = a.heads * a.dvp;
-    const auto grid = [&](int e, int run) { return dim3((max_new + run - 1) / run, (2 * a.kv_heads + (nv + 64 * e - 1) / (64 * e) + 1 + 3) / 4, nseq); };
+    const auto grid = [&](int e, int run) { return dim3((max_new + CH - 1) / CH * (CH / run), (2 * a.kv_heads + (nv + 64 * e - 1) / (64 * e) + 1 + 3) / 4, nseq); };
     if (a.taps <= 4 && a.dkp <= 64) hipLaunchKernelGGL((delta_inputs_kernel<1, 4, 16>), grid(1, 16), dim3(256), 0, st, a);
     else if (a.taps <= 4 && a.dkp <= 128) hipLaunchKernelGGL((delta_inputs_kernel<2, 4, 16>), grid(2, 16), dim3(256), 0, st, a);
     else if (a.taps <= 8 && a.dkp <= 256) hipLaunchKernelGGL((delta_inputs_kernel<4, 8, 8>), grid(4, 8), dim3(256), 0, st, a);
-    else hipLaunchKernelGGL(delta_inputs_any_kernel, dim3(rows), dim3(256), 0, st, a);
+    else hipLaunchKernelGGL(delta_inputs_any_kernel<true>, dim3(rows), dim3(256), 0, st, a);
 }
 
 bool sizes_ok(const CogsDelta& a) {
@@ -853,13 +902,15 @@ bool sizes_ok(const CogsDelta& a) {
 
 }  // namespace
 
-size_t cogs_k_delta_rec_floats(int rows, int nseq, int heads) { return (size_t)(rows / CH + nseq) * heads * REC; }
+int cogs_k_delta_slots(int rows, int nseq) { return rows / CH + nseq; }
+size_t cogs_k_delta_rec_floats(int rows, int nseq, int heads) { return (size_t)cogs_k_delta_slots(rows, nseq) * heads * REC; }
 
 int cogs_k_delta_prompt(hipStream_t st, int dtype, const CogsDelta& a, int rows, int nseq, int max_new) {
     if (!sizes_ok(a) || rows <= 0 || nseq <= 0 || nseq > 65535 || a.heads > 65535) return COGS_E_INVALID;
-    launch_inputs(st, a, rows, nseq, max_new);
+    if (a.slots != cogs_k_delta_slots(rows, nseq)) return COGS_E_INVALID;
     const int keep = (max_new < a.taps ? max_new : a.taps) * a.channels, tail = (keep + 1023) / 1024;
     if (a.dkp <= 256 && g_cogs_debug.delta_chunk != 0) {
+        launch_inputs(st, a, rows, nseq, max_new);
         hipLaunchKernelGGL(delta_chunk_kernel, dim3((max_new + CH - 1) / CH, a.heads, nseq), dim3(256), 0, st, a);
         const int scan = (a.heads + 7) / 8 * 8 * (a.dvp / 16);
         const dim3 grid(scan + (tail + 7) / 8 * 8, 1, nseq);      // (a multiple of 8: the heads of every sequence keep their XCDs)
@@ -867,6 +918,7 @@ int cogs_k_delta_prompt(hipStream_t st, int dtype, const CogsDelta& a, int rows,
         else if (a.dkp <= 128) hipLaunchKernelGGL(delta_scan_kernel<2>, grid, dim3(256), 0, st, a, scan);
         else hipLaunchKernelGGL(delta_scan_kernel<4>, grid, dim3(256), 0, st, a, scan);
     } else {
+        hipLaunchKernelGGL(delta_inputs_any_kernel<false>, dim3(rows), dim3(256), 0, st, a);
         hipLaunchKernelGGL(delta_tail_kernel, dim3(tail, nseq), dim3(256), 0, st, a);
         hipLaunchKernelGGL(delta_recur_kernel, dim3((a.dvp + 63) / 64, a.heads, nseq), dim3(64), 0, st, a);
     }

@@ -293,11 +293,14 @@ struct CogsDelta {
     const float* t; long ldt;            // fused projection [q | k | v | gate | beta | a]
     int heads, headsp, kv_heads, dkp, dvp, vdim, taps, channels;
     const float *conv, *neg_a, *dt_bias, *norm; float eps, q_scale;
-    int rows;                            // prompts: q, k [kv_heads][rows][dkp], v [heads][rows][dvp], (beta, ln g) [rows][heads], read-outs like v, chunk records
-    float *q, *k, *v, *bg, *o, *rec;
+    // prompts: q, k, k by columns [kv_heads][slots][32][dkp] and v [heads][slots][32][dvp] as chunks of tiles (delta.hip; token by token as rows, [rows] in place
+    // of [slots][32]), (beta, ln g) [rows][heads], read-outs [heads][rows][dvp], chunk records
+    int rows, slots;
+    float *q, *k, *kt, *v, *bg, *o, *rec;
     void* att; long ldo;                 // [rows][heads x dvp], in `dtype`
     const CogsSeq* seqs; const int* rowseq; const int* rowpos; long state_off;      // floats
 };
+int cogs_k_delta_slots(int rows, int nseq);      // chunks of 32 rows of all sequences, each on chunks of its own, at the most
 size_t cogs_k_delta_rec_floats(int rows, int nseq, int heads);
 int cogs_k_delta_prompt(hipStream_t st, int dtype, const CogsDelta& a, int rows, int nseq, int max_new);
 int cogs_k_delta_step(hipStream_t st, int dtype, const CogsDelta& a, int nseq);      // one new row per sequence, row i = sequence i

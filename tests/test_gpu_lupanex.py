@@ -535,6 +535,23 @@ def test_chunked_delta_rule_at_the_edges_of_its_tiles(dev, dim, vdim):
     assert rms_err(out, lg[[n - 1 for n in lens]]) < TOL[torch.float32]
 
 
+@pytest.mark.parametrize("dim,vdim,conv", [(32, 80, 1), (128, 48, 3), (64, 16, 6), (256, 32, 8), (48, 130, 9), (144, 32, 11)])
+def test_tiles_of_chunks_from_every_convolution(dev, dim, vdim, conv):
+    """the kernels that form q, k and v as the scan's tiles (short and long convolutions, runs of 16 and 8 rows, a row at a time): prompts that end
+    at the edges of runs, of 16-row tiles and of chunks, together and behind cached tokens, against the oracle (fp32 sums in another order)"""
+    cfg = config([delta(heads=4, kv_heads=2, dim=dim, vdim=vdim, conv=conv, ff=None)], width=64)
+    st = state(cfg)
+    toks = tokens(cfg, 131)
+    lg = lo.forward(cfg, double(st), toks)[0]
+    e = engine(cfg, st, torch.float32)
+    lens = [2, 7, 8, 15, 16, 17, 31, 32, 33, 47, 49, 64, 65, 130]
+    s = sequences(e)
+    out = s.step([(i, toks[:n], [n - 1]) for i, n in enumerate(lens)])
+    assert rms_err(out, lg[[n - 1 for n in lens]]) < TOL[torch.float32]
+    out = s.step([(i, toks[n:131], [130 - n]) for i, n in enumerate(lens)])
+    assert rms_err(out, lg[[130] * len(lens)]) < TOL[torch.float32]
+
+
 @pytest.mark.parametrize("dim", [64, 128, 256])
 def test_the_chunked_delta_rule_keeps_what_recurs(dev, dim):
     """a few (key, value) pairs that come again and again: the state already predicts every value, so what a chunk writes is the rounding of
