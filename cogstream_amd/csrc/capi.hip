@@ -651,20 +651,17 @@ cogs_status VitRange::begin() {
             const int t = (int)grid_sizes[3 * v], gh = (int)grid_sizes[3 * v + 1], gw = (int)grid_sizes[3 * v + 2];
             const int per = gh * gw;
             if (per > max_seq) max_seq = per;
-            { PROF(COGS_PROF_OTHER); COGS_TRY(cogs_k_vit_rope_table(st, rc, rs, (int)row, t, gh, gw, (int)merge_sizes[v], h->vit_inv_freq, h->vit_nfreq)); }
-            if (use_lut) {   // `lo` is free in block-diagonal mode: per-row positions; the LUT itself once (first video)
-                PROF(COGS_PROF_OTHER);
-                COGS_TRY(cogs_k_vit_rope_lut(st, lo, (int)row, t, gh, gw, (int)merge_sizes[v], v == 0 ? lut : nullptr, maxpos,
-                                             h->vit_inv_freq, h->vit_nfreq));
-            }
-            { PROF(COGS_PROF_OTHER); COGS_TRY(cogs_k_vit_segments(st, cu, need_rows ? lo : nullptr, need_rows ? hi : nullptr, (int)row, frame0, t, per)); }
+            // `lo` is free in block-diagonal mode: per-row positions; the LUT and the patches' rows once (first video)
+            const CogsVitTables tables{rc, rs, (int)row, t, gh, gw, (int)merge_sizes[v], h->vit_inv_freq, h->vit_nfreq, use_lut ? lo : nullptr,
+                                       use_lut && v == 0 ? lut : nullptr, maxpos, cu, need_rows ? lo : nullptr, need_rows ? hi : nullptr, frame0};
+            PROF(COGS_PROF_OTHER);
+            COGS_TRY(cogs_k_vit_setup(st, tables, pix_dtype, dt, pixel_values, w.patch_dim, xpad, w.patch_pad, v == 0 ? (int)N : 0, w.patch_dim, w.patch_pad));
             row += (int64_t)t * per;
             frame0 += t;
         }
     }
 
     // patch embed: conv2d k=s=14 == GEMM over the 588-element rows (:202-210)
-    { PROF(COGS_PROF_OTHER); COGS_TRY(cogs_k_pack_rows(st, pix_dtype, dt, pixel_values, w.patch_dim, xpad, w.patch_pad, (int)N, w.patch_dim, w.patch_pad)); }
     {
         CogsGemm g; g.dtype = dt;
         g.A = xpad; g.lda = w.patch_pad; g.W = w.patch_w; g.ldw = w.patch_pad; g.C = x; g.ldc = H;
