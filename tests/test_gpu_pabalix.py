@@ -356,6 +356,29 @@ def test_a_context_of_more_splits_than_are_combined(dev, keys):
                 assert rms_err(step("mla_split_keys", keys_a_split), want) < TOL[torch.bfloat16], (contexts, first, keys_a_split)
 
 
+@pytest.mark.parametrize("kv_rank,heads,n", [(56, 32, 63), (56, 32, 64), (200, 16, 33)])
+def test_splits_combined_by_four_waves_or_by_one(dev, kv_rank, heads, n):
+    """one token of many sequences: 2016 workgroups of the combine (four waves each) and 2048 or more (a wave each), latents of 64 and of 208 columns, with
+    and without a sink, one split to more than 64, against the oracle"""
+    from cogstream_amd import _lib as L
+    cfg = config([mixer(k, heads=heads, dim=16, rot=16, vdim=16, q_rank=40, kv_rank=kv_rank) for k in (G, B)], width=96, vocab=64)
+    st = state(cfg)
+    e = engine(cfg, st, torch.bfloat16)
+    toks = tokens(cfg, 2100)
+    lg = po.forward(cfg, double(st), toks)[0]
+    lens = ([2099, 1, 2, 31, 32, 33, 63, 64, 65, 300, 511, 513] * 6)[:n]
+    lens = [m if i < 12 else min(m, 513) for i, m in enumerate(lens)]
+    s = sequences(e)
+    for i, m in enumerate(lens):
+        s.step([(i, toks[:m], [])])
+    for keys_a_split in (32, 0):
+        with L.debug_switch("mla_split_keys", keys_a_split):
+            got = s.step([(i, [toks[m]], [0]) for i, m in enumerate(lens)])
+        assert rms_err(got, lg[lens]) < TOL[torch.bfloat16], keys_a_split
+        for i, m in enumerate(lens):
+            s.caches[i].reset(m)
+
+
 @pytest.mark.parametrize("rows", [2, 16, 17, 32, 33, 64])
 @pytest.mark.parametrize("width,ff", [(70, 4100), (1100, 1030), (3140, 4100)])
 def test_sublayer_outputs_in_partial_sums(dev, rows, width, ff):
