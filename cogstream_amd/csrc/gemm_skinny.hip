@@ -350,7 +350,12 @@ int cogs_k_gemm_skinny(hipStream_t st, const CogsGemm& g, float* part) {
     return COGS_LAUNCH_CHECK();
 }
 
-bool cogs_k_gemm_skinny_latent_fits(const CogsGemm& g) { return cogs_k_gemm_skinny_fits(g) && g.M <= 16 && g.K <= 2048 && g_cogs_debug.gemm_skinny != 0; }
+// (one row too, which the single-row GEMV takes otherwise: one token of one request 567 -> 550 us, of width 4096 669 -> 661, of 3584 738 -> 730)
+bool cogs_k_gemm_skinny_latent_fits(const CogsGemm& g) {
+    CogsGemm two = g;
+    two.M = g.M == 1 ? 2 : g.M;
+    return cogs_k_gemm_skinny_fits(two) && g.M <= 16 && g.K <= 2048 && g_cogs_debug.gemm_skinny != 0;
+}
 
 // g's rows are l's normed query latents (g.A is not read); l's key and value latents and gates go where cogs_k_mla_latent puts them
 int cogs_k_gemm_skinny_latent(hipStream_t st, const CogsGemm& g, const CogsMlaLatent& l) {

@@ -287,6 +287,12 @@ def test_query_products_that_norm_their_rows(dev, heads, q_rank, rows):
             assert bool((a - b).abs().max() <= TOL[torch.bfloat16] * b.abs().max())
 
 
+@pytest.mark.parametrize("heads,q_rank", [(3, 40), (5, 1000), (3, 1024), (80, 1100), (3, 2048), (3, 2100)])
+def test_the_query_product_of_one_row_norms_it(dev, heads, q_rank):
+    """... one sequence (the sizes of the test above)"""
+    test_query_products_that_norm_their_rows(dev, heads, q_rank, 1)
+
+
 @pytest.mark.parametrize("dim,rot", [(128, 64), (96, 64), (64, 32), (32, 64)])
 def test_columns_that_are_not_rotated(dev, dim, rot):
     """the query product reads no factors for blocks of columns in front of a head's rotated part (64 columns a wave, 32 in the small tiles; heads where such
