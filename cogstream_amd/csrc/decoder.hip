@@ -144,11 +144,11 @@ struct Step {
     void* row(void* p, size_t width) const { return (char*)p + r0 * width * esize(d.w.dtype); }
     const void* at(const void* p, size_t elems) const { return (const char*)p + elems * esize(d.w.dtype); }
 
-    // C[rows, N] = A . W^T with an epilogue: few rows stream the weights, one row takes the GEMV, the rest the tiled kernels
+    // C[rows, N] = A . W^T with an epilogue: few rows stream the weights, one row of some sizes takes the GEMV, the rest the tiled kernels
     int lin(CogsGemm& g) {
         PROF(COGS_PROF_GEMM);
         g.dtype = d.w.dtype;
-        if (g_cogs_debug.gemm_skinny != 0 && cogs_k_gemm_skinny_fits(g)) return cogs_k_gemm_skinny(st, g);
+        if (g_cogs_debug.gemm_skinny != 0 && cogs_k_gemm_skinny_fits(g) && (g.M > 1 || cogs_k_gemm_skinny_one_row(g.N, g.K))) return cogs_k_gemm_skinny(st, g);
         if (g.K < 128) g.force_small_tile = 1;      // (fp32: products that short stay off the three-slab ring)
         return cogs_k_gemm(st, g);
     }

@@ -1,4 +1,4 @@
-// Few-row GEMM for batched decode:  C[M,N] = epilogue( A[M,K] . W[N,K]^T ),  2 <= M <= 64, bf16.
+// Few-row GEMM for batched decode:  C[M,N] = epilogue( A[M,K] . W[N,K]^T ),  1 <= M <= 64, bf16.
 //
 // HBM-bound like the single-row GEMV (gemv.hip): every weight byte is read once. A workgroup owns 16 NT output columns; its NW waves
 // take alternate 64-element slices of K, the batch rows are the columns of v_mfma_f32_16x16x32_bf16 (MT groups of 16), and the
@@ -305,8 +305,18 @@ int whole_cols(int M, int N) {
 }  // namespace
 
 bool cogs_k_gemm_skinny_fits(const CogsGemm& g) {
-    return g.dtype == COGS_DT_BF16 && g.M >= 2 && g.M <= 64 && g.K % 64 == 0 && g.N % 4 == 0 && g.lda % 8 == 0 && g.ldw % 8 == 0 &&
+    return g.dtype == COGS_DT_BF16 && g.M >= 1 && g.M <= 64 && g.K % 64 == 0 && g.N % 4 == 0 && g.lda % 8 == 0 && g.ldw % 8 == 0 &&
            !g.rms_gamma && !g.row_stats && !g.ln_ab && !g.kv_k && g.hm_rows == 0;
+}
+
+// One row, without partial sums: here where the columns come to whole rounds of workgroups, else by the GEMV, whose waves take four columns at a time
+// (GEMV / here, us: 32 768 x 2048 31.6 / 24.3, 22 016 x 4096 33.4 / 30.1, 28 416 x 3584 33.4 / 31.8, 10 808 x 3584 15.2 / 13.2, 16 384 x 4096 26.1 / 26.0;
+// not full 37 888 x 3584 42.5 / 45.2, 6144 x 4096 10.5 / 11.9, 1344 x 2048 3.9 / 4.5). With three quarters of the CUs busy a short K is still the
+// faster here, where latency counts: 3072 x 2048 5.4 / 4.7, 6176 x 2048 6.9 / 6.4, 5376 x 3584 9.4 / 8.3. Partial sums are always: 2048 x 2048 5.0 / 3.8,
+// 2048 x 5632 7.2 / 6.1, 3584 x 28 416 35.7 / 31.4.
+bool cogs_k_gemm_skinny_one_row(int N, int K) {
+    const int cols = whole_cols(1, N), wgs = (N + cols - 1) / cols, rounds = (wgs + 255) / 256;
+    return wgs * 5 >= rounds * 256 * 4 || (rounds == 1 && wgs >= 128 && K < 4096);
 }
 
 // how many partial sums a product of this size is stored as when its caller takes them (1: none). K shorter than 64 slices: two
@@ -326,7 +336,7 @@ CogsAhead cogs_k_gemm_skinny_ahead(const void* W, long ldw, int M, int N, int K)
     CogsAhead a;
     CogsGemm g;
     g.dtype = COGS_DT_BF16; g.M = M; g.N = N; g.K = K; g.lda = K; g.ldw = ldw;
-    if (!W || g_cogs_debug.gemm_skinny == 0 || !cogs_k_gemm_skinny_fits(g)) return a;
+    if (!W || g_cogs_debug.gemm_skinny == 0 || !cogs_k_gemm_skinny_fits(g) || (M == 1 && !cogs_k_gemm_skinny_one_row(N, K))) return a;
     const long lines = AHEAD_BYTES / (128L * N);
     a.W = (const char*)W; a.ldw = ldw * 2; a.N = N; a.cols = whole_cols(M, N); a.groups = (N + a.cols - 1) / a.cols;
     a.lines = (int)(lines < K / 64 ? lines : K / 64);
@@ -350,12 +360,8 @@ int cogs_k_gemm_skinny(hipStream_t st, const CogsGemm& g, float* part) {
     return COGS_LAUNCH_CHECK();
 }
 
-// (one row too, which the single-row GEMV takes otherwise: one token of one request 567 -> 550 us, of width 4096 669 -> 661, of 3584 738 -> 730)
-bool cogs_k_gemm_skinny_latent_fits(const CogsGemm& g) {
-    CogsGemm two = g;
-    two.M = g.M == 1 ? 2 : g.M;
-    return cogs_k_gemm_skinny_fits(two) && g.M <= 16 && g.K <= 2048 && g_cogs_debug.gemm_skinny != 0;
-}
+// (one row too: one token of one request, by the GEMV and a launch for its norms in front 567 us, 550 so; of width 4096 669, 661, of 3584 738, 730)
+bool cogs_k_gemm_skinny_latent_fits(const CogsGemm& g) { return cogs_k_gemm_skinny_fits(g) && g.M <= 16 && g.K <= 2048 && g_cogs_debug.gemm_skinny != 0; }
 
 // g's rows are l's normed query latents (g.A is not read); l's key and value latents and gates go where cogs_k_mla_latent puts them
 int cogs_k_gemm_skinny_latent(hipStream_t st, const CogsGemm& g, const CogsMlaLatent& l) {

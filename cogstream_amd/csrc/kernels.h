@@ -94,8 +94,9 @@ int cogs_k_attention(hipStream_t st, const CogsAttn& a);
 // L2 caches on CUs it leaves idle (norm.hip, read_ahead). lines = 0: nothing to read
 struct CogsAhead { const char* W = nullptr; long ldw = 0; int N = 0, cols = 0, groups = 0, lines = 0; };
 CogsAhead cogs_k_gemm_skinny_ahead(const void* W, long ldw, int M, int N, int K);       // bf16, ldw in elements
-// few-row GEMM (gemm_skinny.hip): bf16, 2 <= M <= 64; opt-in per call site (its summation order differs from cogs_k_gemm's)
+// few-row GEMM (gemm_skinny.hip): bf16, 1 <= M <= 64; opt-in per call site (its summation order differs from cogs_k_gemm's)
 bool cogs_k_gemm_skinny_fits(const CogsGemm& g);
+bool cogs_k_gemm_skinny_one_row(int N, int K);      // M = 1 without partial sums: not slower than the GEMV
 #define COGS_SKINNY_MAX_PARTS 8
 int cogs_k_gemm_skinny_parts(int M, int N, int K);
 // part != nullptr (plain products, with or without a bias): cogs_k_gemm_skinny_parts(..) (2, 4 or 8) partial sums fp32 [parts][M][N] instead of C

@@ -398,6 +398,12 @@ def test_few_row_products_at_the_edges_of_their_rings(dev, rows, width, ff):
     assert rms_err(got, lo.forward(cfg, double(st), toks)[0]) < TOL[torch.bfloat16]
 
 
+@pytest.mark.parametrize("width,ff", [(70, 10300), (1344, 5200)])
+def test_one_row_products_at_the_edges_of_their_rings(dev, width, ff):
+    """... a single row"""
+    test_few_row_products_at_the_edges_of_their_rings(dev, 1, width, ff)
+
+
 @pytest.mark.parametrize("dim,vdim,conv", [(16, 16, 1), (64, 256, 4), (256, 48, 5), (128, 128, 4), (130, 256, 8), (272, 16, 3), (16, 272, 9)])
 def test_one_token_delta_rule_at_the_edges_of_its_kernels(dev, dim, vdim, conv):
     """one to sixteen waves of 16 columns, whole and ragged rows a lane, more channels than threads, windows of one to nine taps that start

@@ -397,6 +397,23 @@ def test_sublayer_outputs_in_partial_sums(dev, rows, width, ff):
     assert rms_err(got, po.forward(cfg, double(st), toks)[0]) < TOL[torch.bfloat16]
 
 
+@pytest.mark.parametrize("width,ff", [(70, 4100), (1100, 1030), (3140, 4100)])
+def test_one_row_in_partial_sums(dev, width, ff):
+    """... of a single row, which the same kernel takes"""
+    test_sublayer_outputs_in_partial_sums(dev, 1, width, ff)
+
+
+@pytest.mark.parametrize("width,ff,vocab", [(64, 1000, 2032), (64, 2048, 4096), (200, 5200, 10496), (200, 2600, 13000), (64, 9000, 33000)])
+def test_one_row_by_the_few_row_product_or_the_gemv(dev, width, ff, vocab):
+    """products of one row, N on both sides of 128 workgroups, of four fifths of a round, of one and of two rounds: the logits of single tokens against the
+    oracle"""
+    cfg = config([mixer(G, heads=2, dim=16, rot=16, vdim=16), mixer(A, heads=3)], width=width, ff=ff, vocab=vocab)
+    st = state(cfg)
+    toks = tokens(cfg, 6)
+    got = run(engine(cfg, st, torch.bfloat16), toks, range(1, 6))
+    assert rms_err(got, po.forward(cfg, double(st), toks)[0]) < TOL[torch.bfloat16]
+
+
 @pytest.mark.parametrize("name", ["peaked", "mixed"])
 def test_a_query_tile_by_one_wave_or_by_two(dev, name):
     """many prompts at once (each query tile's keys are one wave's) and few (every second key tile is another wave's): prompts that end
