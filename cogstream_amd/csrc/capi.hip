@@ -215,6 +215,9 @@ cogs_status cogs_gather_rows(cogs_stream stream, int dtype, const void* ta, cons
                              void* out, int rows, int D) {
     return cogs_k_gather_rows((hipStream_t)stream, dtype, ta, tb, idx, out, rows, D);
 }
+cogs_status cogs_gather_rows_host(cogs_stream stream, int dtype, const void* ta, const void* tb, const int64_t* idx, void* out, int rows, int D) {
+    return cogs_k_gather_few((hipStream_t)stream, dtype, ta, tb, idx, out, rows, D);
+}
 cogs_status cogs_mean_rows(cogs_stream stream, int dtype, const void* x, int64_t ldx, int rows, int D, float* out) {
     return cogs_k_mean_rows((hipStream_t)stream, dtype, x, ldx, rows, D, out);
 }

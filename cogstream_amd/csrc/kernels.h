@@ -137,6 +137,8 @@ int cogs_k_mask_fix(hipStream_t st, uint8_t* mask, int t, int tokens_per_frame, 
 int cogs_k_frame_mean_to_slot0(hipStream_t st, int dtype, void* feats, int P, int D, const int* frames, int n_frames);
 int cogs_k_gather_rows(hipStream_t st, int dtype, const void* table_a, const void* table_b, const int64_t* idx,
                        void* out, int rows, int D);
+constexpr int COGS_GATHER_FEW = 128;
+int cogs_k_gather_few(hipStream_t st, int dtype, const void* table_a, const void* table_b, const int64_t* host_idx, void* out, int rows, int D);
 int cogs_k_mean_rows(hipStream_t st, int dtype, const void* x, long ldx, int rows, int D, float* out);
 int cogs_k_cosine(hipStream_t st, const float* a, const float* b, int n, int D, float* out);
 

@@ -319,7 +319,7 @@ class Qwen2Engine(CausalEngine):
         return KVCache(self.cfg, max_len, self.dtype, self.device)
 
     def embed_tokens(self, ids: torch.Tensor) -> torch.Tensor:
-        return ops.gather_rows(self.packed.embed, None, ops.token_ids(ids, self.device))
+        return ops.embed_rows(self.packed.embed, ids)
 
     def forward(self, embeds: torch.Tensor, cache: Optional[KVCache] = None, *, want_logits: bool = True,
                 want_pooled: bool = False, want_hidden: bool = False):
@@ -386,7 +386,7 @@ class DecoderEngine(CausalEngine):
         return DecoderCache(self.packed.cache_widths, self.packed.state_floats, max_len, self.dtype, self.device)
 
     def embed_tokens(self, ids: torch.Tensor) -> torch.Tensor:
-        return ops.gather_rows(self.packed.embed, None, ops.token_ids(ids, self.device))
+        return ops.embed_rows(self.packed.embed, ids)
 
     def forward_batch(self, embeds: torch.Tensor, lens: Sequence[int], caches: Sequence[KVCache], want: Sequence[int],
                       streams: Optional[torch.Tensor] = None) -> Optional[torch.Tensor]:

@@ -193,6 +193,19 @@ def token_ids(ids: torch.Tensor, device: torch.device) -> torch.Tensor:
     return ids.to(torch.int64).pin_memory().to(device, non_blocking=True)
 
 
+def embed_rows(table: torch.Tensor, ids: torch.Tensor) -> torch.Tensor:
+    """table rows of token ids. Up to 128 pageable host ids are the launch's arguments"""
+    ids = ids.reshape(-1)
+    if ids.is_cuda or not table.is_cuda or not 0 < ids.numel() <= 128 or ids.is_pinned() or torch.cuda.is_current_stream_capturing():
+        return gather_rows(table, None, token_ids(ids, table.device))
+    assert table.is_contiguous()
+    ids = ids.to(torch.int64).contiguous()
+    out = torch.empty(ids.numel(), table.shape[1], device=table.device, dtype=table.dtype)
+    check(L.lib.cogs_gather_rows_host(current_stream(), dtype_code(table.dtype), ptr(table), None, ids.data_ptr(), ptr(out),
+                                      ids.numel(), table.shape[1]), "cogs_gather_rows_host")
+    return out
+
+
 def mean_rows(x: torch.Tensor) -> torch.Tensor:
     _need_cuda(x)
     out = torch.empty(x.shape[1], device=x.device, dtype=torch.float32)

@@ -202,6 +202,9 @@ cogs_status cogs_frame_mean_to_slot0(cogs_stream stream, int dtype, void* feats,
 /* out[r] = idx[r] >= 0 ? table_a[idx[r]] : table_b[-idx[r]-1]   (embed_tokens + masked scatter, :567-572) */
 cogs_status cogs_gather_rows(cogs_stream stream, int dtype, const void* table_a, const void* table_b,
                              const int64_t* idx, void* out, int rows, int D);
+/* the same of up to 128 rows with idx in host memory, which is read before the call returns */
+cogs_status cogs_gather_rows_host(cogs_stream stream, int dtype, const void* table_a, const void* table_b,
+                                  const int64_t* idx, void* out, int rows, int D);
 /* out[D] (fp32) = mean over rows (torch.mean(last_hidden_state, dim=1), :317,323) */
 cogs_status cogs_mean_rows(cogs_stream stream, int dtype, const void* x, int64_t ldx, int rows, int D, float* out);
 /* out[i] = cos(a, b[i])  (F.cosine_similarity, :325) */

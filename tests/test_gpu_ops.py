@@ -1547,6 +1547,29 @@ def test_token_ids_reach_the_device_as_they_were_at_the_call(dev):
     assert ops.token_ids(torch.arange(8), d).tolist() == list(range(8))
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("n", [0, 1, 3, 4, 5, 127, 128, 129])
+def test_rows_of_few_tokens(dev, n, dtype):
+    """ops.embed_rows: up to 128 host ids as the launch's arguments, read before the call returns; more, pinned ones and those on the device as before;
+    a capture still refuses ids of the host"""
+    ops = _ops()
+    g = torch.Generator().manual_seed(n)
+    table = torch.randn(1000, 264, generator=g).to(dtype).to(dev)
+    for make in (lambda t: t, lambda t: t.int().reshape(1, -1), lambda t: t.repeat_interleave(2)[::2], lambda t: t.pin_memory() if n else t, lambda t: t.to(dev)):
+        want = torch.randint(0, 1000, (n,), generator=g)
+        want[-1:] = 999
+        ids = make(want.clone())
+        torch.cuda._sleep(1_000_000)
+        got = ops.embed_rows(table, ids)
+        if not ids.is_cuda:
+            ids.fill_(1)
+        assert torch.equal(got, table[want.to(dev)])
+    if n:
+        with pytest.raises(RuntimeError), torch.cuda.graph(torch.cuda.CUDAGraph()):
+            ops.embed_rows(table, want)
+        torch.cuda.synchronize()
+
+
 @pytest.mark.parametrize("grid", [(1, 2, 2), (1, 12, 11), (1, 16, 16), (2, 12, 23), (1, 24, 24), (1, 1, 577), (3, 14, 16)])
 def test_weights_read_ahead_change_nothing(dev, grid):
     """the encoder's launches of up to 576 patches read the next products' weights on idle CUs: first and last layer, fewer columns than tiles, and sizes on both
