@@ -75,6 +75,17 @@ class DecoderCache(KVCache):
             self.state.copy_(state)
         self.stale = False
 
+    def copy_rows_from(self, old: "KVCache", n: int):
+        """runs of blocks of one width at a time (a copy per block was 72 of 2.5 us where eight requests outgrew their prompts' caches)"""
+        at = i = 0
+        while i < len(self.widths):
+            w, count = self.widths[i], 1
+            while i + count < len(self.widths) and self.widths[i + count] == w:
+                count += 1
+            dst, src = (c.k[at * c.max_len:(at + count * w) * c.max_len].view(count, c.max_len, w) for c in (self, old))
+            dst[:, :n].copy_(src[:, :n])
+            at, i = at + count * w, i + count
+
     def _blocks(self) -> List[torch.Tensor]:
         out, at = [], 0
         for w in self.widths:
