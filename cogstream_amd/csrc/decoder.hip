@@ -3,6 +3,7 @@
 #include "ctx.h"
 #include "debug.h"
 
+#include <algorithm>
 #include <math.h>
 #include <new>
 
@@ -37,6 +38,7 @@ struct CogsDecoder {
     std::vector<Geom> geom;
     std::vector<Run> runs;
     std::vector<CogsRopeSet> sets;
+    std::vector<double> freq;                 // of all sets, one behind the other
     CogsRopeSet* sets_dev = nullptr;
     double* freq_dev = nullptr;
     int wp = 0, vocabp = 0, max_pairs = 0;
@@ -412,7 +414,7 @@ cogs_status cogs_decoder_load(cogs_handle h, const cogs_decoder_weights* w) {
     d->w.layer = d->layers.data();
     d->wp = up(w->width, 64);
     d->vocabp = up(w->vocab, 4);
-    std::vector<double> freq;
+    std::vector<double>& freq = d->freq;
     std::vector<size_t> freq_at;
     const bool hyper = w->streams > 0;
     auto hyper_ok = [&](const cogs_hyper& c) { return !hyper || (c.in && c.out && c.mix); };
@@ -513,6 +515,19 @@ cogs_status cogs_decoder_load(cogs_handle h, const cogs_decoder_weights* w) {
                 for (int t = 1; t < w->loop_times; ++t)
                     for (int m = w->loop_start; m < w->loop_stop; ++m) run(m);
         }
+    }
+    // another weight set with the same rotations, as where two engines take turns on a handle: the device tables stay. (To free them waits for all that
+    // is queued: one token of 16 requests, three engines in turn 813 -> 680 us, a prompt of 4096 4588 -> 4423)
+    CogsDecoder* const old = h->decoder;
+    auto same_set = [](const CogsRopeSet& a, const CogsRopeSet& b) { return a.off == b.off && a.pairs == b.pairs && a.first == b.first && a.n == b.n && a.mag == b.mag; };
+    if (old && !d->sets.empty() && old->sets.size() == d->sets.size() && old->freq.size() == freq.size() &&
+        std::equal(d->sets.begin(), d->sets.end(), old->sets.begin(), same_set) && memcmp(freq.data(), old->freq.data(), freq.size() * sizeof(double)) == 0) {
+        std::swap(d->freq_dev, old->freq_dev);
+        std::swap(d->sets_dev, old->sets_dev);
+        d->sets = old->sets;
+        cogs_decoder_free(old);
+        h->decoder = d;
+        return COGS_OK;
     }
     if (!d->sets.empty() && (hipMalloc(&d->freq_dev, freq.size() * sizeof(double)) != hipSuccess ||
                              hipMalloc(&d->sets_dev, d->sets.size() * sizeof(CogsRopeSet)) != hipSuccess)) return fail(COGS_E_HIP);

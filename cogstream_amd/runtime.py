@@ -16,6 +16,7 @@ class Handle:
         L.check(L.lib.cogs_create(device_index, C.byref(self._h)), "cogs_create")
         self._ws: Dict[str, torch.Tensor] = {}
         self._active: Dict[str, object] = {}   # which packed weight set ("vit" / "proj" / "llm") the handle points at
+        self._streams: Dict[str, set] = {}     # where it has been used since
 
     @property
     def h(self):
@@ -31,10 +32,16 @@ class Handle:
 
     def activate(self, kind: str, owner, load) -> None:
         """the handle keeps ONE pointer table per model kind; an engine re-points it before use when another
-        engine (a second adapter, another test model) was loaded in between"""
+        engine (a second adapter, another test model) was loaded in between. Engines of a kind share a workspace, so one that
+        comes behind another's calls on other streams waits for them; on the same stream nothing does"""
+        stream, used = L.current_stream(), self._streams.setdefault(kind, set())
         if self._active.get(kind) is not owner:
+            if used - {stream}:
+                torch.cuda.synchronize(self.device_index)
             load()
             self._active[kind] = owner
+            used.clear()
+        used.add(stream)
 
     def close(self):
         if self._h:

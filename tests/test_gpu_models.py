@@ -40,6 +40,33 @@ def test_vit_encode_vs_oracle(dev, dtype, tol, mode):
     assert rel_err(out.float(), ref) < tol
 
 
+def test_encoders_take_turns_on_a_handle(dev):
+    """two weight sets with heads of one size and one with others, in turn, on one stream and on another: each as by itself. (An encoder behind another's calls
+    on a second stream waits for them: they share a workspace)"""
+    from cogstream_amd.vision import VisionEncoder
+    from cogstream_amd.weights import VisionConfig, random_vit_state
+    grid, merge = torch.tensor([[6, 8, 10]]), torch.tensor([2])
+    pix = (torch.rand(480, 588, generator=torch.Generator().manual_seed(1)) * 2 - 1).bfloat16().to(dev)
+    encs = []
+    for seed, heads in ((1, 8), (2, 8), (3, 4)):
+        cfg = VisionConfig(**{**VIT, "num_attention_heads": heads})
+        encs.append(VisionEncoder(random_vit_state(cfg, seed=seed, std=0.05), cfg, dtype=torch.bfloat16, device=dev))
+    want = []
+    for e in encs:
+        want.append(e(pix, grid, merge).clone())
+        torch.cuda.synchronize()
+    assert not torch.equal(want[0], want[1])
+    side, main = torch.cuda.Stream(), torch.cuda.current_stream()
+    side.wait_stream(main)
+    got = []
+    for i, m in enumerate((0, 1, 0, 1, 2, 0, 2, 1)):
+        with torch.cuda.stream(side if i % 3 == 2 else main):
+            got.append((m, encs[m](pix, grid, merge)))
+    torch.cuda.synchronize()
+    for m, out in got:
+        assert torch.equal(out, want[m])
+
+
 def test_vit_bf16_pixel_input_and_frame_independence(dev):
     """block-diagonal mode: perturbing one frame must leave every other frame's tokens bit-identical
     (the property that makes frame sharding legal)"""

@@ -563,6 +563,26 @@ def test_two_models_share_a_handle(dev):
         assert rms_err(ra, a[4][lo:hi]) < TOL[torch.float32] and rms_err(rb, b[4][lo:hi]) < TOL[torch.bfloat16]
 
 
+def test_models_of_the_same_rotations_take_turns(dev):
+    """engines whose tables on the device are the same, whose rotations differ in a number or in their frequencies, and one without any, in turn on a handle:
+    each against its own oracle"""
+    models = []
+    for i, cfg in enumerate((CONFIGS["peaked"], CONFIGS["peaked"], config([mixer(G, heads=4), mixer(B, heads=4)], width=192, ff=128),
+                             config([mixer(G, heads=4, base=500.0), mixer(B, heads=4, base=500.0)], width=192, ff=128))):
+        st = state(cfg, seed=10 + i)
+        toks = tokens(cfg, 40, seed=i)
+        e = engine(cfg, st, torch.bfloat16)
+        models.append((e, toks, po.forward(cfg, double(st), toks)[0], sequences(e)))
+    for lo, hi in ((0, 20), (20, 21), (21, 40)):
+        for order in ((0, 1, 2, 3), (3, 1, 0, 2)):
+            for m in order:
+                e, toks, lg, s = models[m]
+                if order[0] == 3:
+                    s.caches["r"].reset(lo)
+                got = s.step([("r", toks[lo:hi], list(range(hi - lo)))])
+                assert rms_err(got, lg[lo:hi]) < TOL[torch.bfloat16], (m, lo)
+
+
 def test_command_lines(dev, tmp_path):
     """python -m cogstream_amd.generate and bin/trace_run in processes of their own"""
     cfg, st = _checkpoint(tmp_path, "peaked")
