@@ -36,7 +36,7 @@ class Handle:
         comes behind another's calls on other streams waits for them; on the same stream nothing does"""
         stream, used = L.current_stream(), self._streams.setdefault(kind, set())
         if self._active.get(kind) is not owner:
-            if used - {stream}:
+            if used - {stream} and not torch.cuda.is_current_stream_capturing():      # (a capture runs nothing, and cannot wait)
                 torch.cuda.synchronize(self.device_index)
             load()
             self._active[kind] = owner
