@@ -186,7 +186,7 @@ __global__ __launch_bounds__(256) void gemm_skinny_latent_kernel(SkinnyArgs p, C
 #pragma unroll
             for (int j = 0; j < J; ++j)
 #pragma unroll
-                for (int e = 0; e < 4; ++e) sq += v[m][j][e] * v[m][j][e];
+                for (int e = 0; e < 4; ++e) sq = fmaf(v[m][j][e], v[m][j][e], sq);      // (written out: left to the compiler, the first two swap places here)
             sq = wave_sum(sq);
             if (lane == 0) red[m][wid] = sq;
         }

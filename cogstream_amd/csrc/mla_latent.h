@@ -16,7 +16,8 @@ __device__ __forceinline__ void block_sum2(float& a, float& b, float* red) {
 }
 
 // One row by a workgroup of 256 threads: RMS norm of the query latent (QUERY), RMS norm of the kv latent and rotation of the shared key part
-// (both straight into the sequence's cache row), sigmoid of the gate logits. red: 8 floats
+// (both straight into the sequence's cache row), sigmoid of the gate logits. red: 8 floats. Squares are fused in the order of the columns, here and
+// in the query product: a row's norm has the same bits by either
 template <typename T, bool QUERY>
 __device__ __forceinline__ void latent_row(const CogsMlaLatent& p, int row, int tid, float* red) {
     const float* t = p.t + (long)row * p.ldt;
@@ -25,14 +26,14 @@ __device__ __forceinline__ void latent_row(const CogsMlaLatent& p, int row, int 
         for (int i = tid * 4; i < p.qrp; i += 1024) {
             const f32x4 v = *reinterpret_cast<const f32x4*>(t + i);
 #pragma unroll
-            for (int e = 0; e < 4; ++e) sq += v[e] * v[e];
+            for (int e = 0; e < 4; ++e) sq = fmaf(v[e], v[e], sq);
         }
     const float* tk = t + p.qrp;
     if (p.own_kv)
         for (int i = tid * 4; i < p.kvp; i += 1024) {
             const f32x4 v = *reinterpret_cast<const f32x4*>(tk + i);
 #pragma unroll
-            for (int e = 0; e < 4; ++e) skv += v[e] * v[e];
+            for (int e = 0; e < 4; ++e) skv = fmaf(v[e], v[e], skv);
         }
     block_sum2(sq, skv, red);
     if constexpr (QUERY) {

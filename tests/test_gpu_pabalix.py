@@ -293,6 +293,34 @@ def test_the_query_product_of_one_row_norms_it(dev, heads, q_rank):
     test_query_products_that_norm_their_rows(dev, heads, q_rank, 1)
 
 
+@pytest.mark.parametrize("rows,q_rank", [(16, 768), (8, 2048), (16, 2048), (3, 1024)])
+def test_query_norms_have_the_same_bits_by_either_kernel(dev, rows, q_rank):
+    """the query latents' norms formed inside the query product and by the launch in front, bit for bit. Every product's rows of weights have one entry of 1 or -1 (those
+    of the query latents a second one of 1/64, for values of more bits than a square in fp32 holds), so that no order of sums and no store of a partial one rounds: the norms
+    are all that could differ. A norm whose last bit is off moves one of some 65 000 of its bf16 values, so it takes thousands of rows to show"""
+    from cogstream_amd import _lib as L
+    cfg = config([dict(mixer(A, heads=q_rank // 32, q_rank=q_rank, dim=24, rot=16, vdim=8), ff=None)] * 2, width=256, vocab=1024)
+    st = state(cfg)
+    g = torch.Generator().manual_seed(rows)
+    for k, w in st.items():
+        if w.dim() == 2 and k.rsplit(".", 1)[-1] not in ("embed", "uk", "uv"):
+            st[k] = torch.zeros_like(w).scatter_(1, torch.randint(0, w.shape[1], (w.shape[0], 1), generator=g), torch.randint(0, 2, (w.shape[0], 1), generator=g) * 2.0 - 1)
+            if k.endswith(".dq"):
+                st[k] += torch.zeros_like(w).scatter_(1, torch.randint(0, w.shape[1], (w.shape[0], 1), generator=g), 2.0 ** -6)
+    e = engine(cfg, st, torch.bfloat16)
+    steps = 6000 // (2 * rows)
+    toks = [tokens(cfg, 4 + steps, seed=i) for i in range(rows)]
+
+    def logits():
+        s = sequences(e, 1024)
+        s.step([(i, t[:4], []) for i, t in enumerate(toks)])
+        return torch.stack([s.step([(i, [t[4 + n]], [0]) for i, t in enumerate(toks)]) for n in range(steps)])
+    got = logits()
+    with L.debug_switch("gemm_skinny", 0):
+        want = logits()
+    assert torch.equal(got, want)
+
+
 @pytest.mark.parametrize("dim,rot", [(128, 64), (96, 64), (64, 32), (32, 64)])
 def test_columns_that_are_not_rotated(dev, dim, rot):
     """the query product reads no factors for blocks of columns in front of a head's rotated part (64 columns a wave, 32 in the small tiles; heads where such
