@@ -16,7 +16,9 @@ class Handle:
         L.check(L.lib.cogs_create(device_index, C.byref(self._h)), "cogs_create")
         self._ws: Dict[str, torch.Tensor] = {}
         self._active: Dict[str, object] = {}   # which packed weight set ("vit" / "proj" / "llm") the handle points at
-        self._streams: Dict[str, set] = {}     # where it has been used since
+        self._queued: Dict[str, Dict[int, set]] = {}      # kind -> stream -> engines (ids) that have used it since the device was last waited for here
+        self._ran: Dict[str, object] = {}      # the engine of the last call that was no capture
+        self._captured: set = set()            # kinds that have been captured
 
     @property
     def h(self):
@@ -33,15 +35,21 @@ class Handle:
     def activate(self, kind: str, owner, load) -> None:
         """the handle keeps ONE pointer table per model kind; an engine re-points it before use when another
         engine (a second adapter, another test model) was loaded in between. Engines of a kind share a workspace, so one that
-        comes behind another's calls on other streams waits for them; on the same stream nothing does"""
-        stream, used = L.current_stream(), self._streams.setdefault(kind, set())
-        if self._active.get(kind) is not owner:
-            if used - {stream} and not torch.cuda.is_current_stream_capturing():      # (a capture runs nothing, and cannot wait)
+        finds another's calls on other streams, not waited for yet, waits for them; on the same stream nothing does. A capture runs nothing and
+        cannot wait: the call behind it does. Graphs are replayed on streams that are not seen here, so where a kind has any, an engine that
+        comes behind another waits wherever it was"""
+        stream, queued = L.current_stream(), self._queued.setdefault(kind, {})
+        if torch.cuda.is_current_stream_capturing():
+            self._captured.add(kind)
+        else:
+            if (kind in self._captured and self._ran.get(kind) is not owner) or any(s != stream and o != {id(owner)} for s, o in queued.items()):
                 torch.cuda.synchronize(self.device_index)
+                queued.clear()
+            queued.setdefault(stream, set()).add(id(owner))
+            self._ran[kind] = owner
+        if self._active.get(kind) is not owner:
             load()
             self._active[kind] = owner
-            used.clear()
-        used.add(stream)
 
     def close(self):
         if self._h:

@@ -209,3 +209,51 @@ def test_reference_plugin_names_resolve_through_auto_map(tmp_path):
     if os.path.isdir(ref):      # build container only: the reference's own files name exactly these classes
         assert auto._resolve(ref, "config.json", "AutoModelForCausalLM", "x.y") is Videollama3Qwen2ForCausalLM
         assert auto._resolve(ref, "preprocessor_config.json", "AutoProcessor", "x.y") is Videollama3Qwen2Processor
+
+
+def test_an_engine_waits_for_what_others_have_queued(monkeypatch):
+    """Handle.activate: engines of a kind share a workspace, so none may run while work of another is queued on another stream. Sequences of calls (engine,
+    stream, eager, captured, an engine that is made there, or the replay of an engine's graph somewhere) with a device that finishes nothing until it is
+    waited for; a capture must not wait, one engine on one stream never does, and engines that take turns on one do not either"""
+    import itertools
+    import random
+    from types import SimpleNamespace
+    from cogstream_amd import runtime
+    now = SimpleNamespace(stream=0, capturing=False, queued=[], waits=0)
+
+    def synchronize(device=None):
+        assert not now.capturing
+        now.waits += 1
+        now.queued.clear()
+    monkeypatch.setattr(runtime, "L", SimpleNamespace(lib=SimpleNamespace(cogs_create=lambda *a: 0, cogs_destroy=lambda *a: 0), check=lambda *a: None,
+                                                      current_stream=lambda: now.stream))
+    monkeypatch.setattr(torch.cuda, "synchronize", synchronize)
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: now.capturing)
+    engines = [object(), object(), object()]
+
+    def waits(*steps):
+        handle, points_at = runtime.Handle(0), []
+        now.queued, now.waits = [], 0
+        for engine, stream, how in steps:
+            if how == "replay":
+                now.queued.append((engine, "anywhere"))
+                continue
+            now.stream, now.capturing = stream, how == "capture"
+            handle.activate("vit", engines[engine], lambda: points_at.append(engine))
+            now.capturing = False
+            assert points_at[-1] == engine
+            if how == "eager":
+                assert all(e == engine or st == stream for e, st in now.queued), steps
+                now.queued.append((engine, stream))
+        return now.waits
+
+    assert waits((0, 1, "eager"), (1, 2, "capture"), (1, 2, "eager"), (1, 2, "eager")) == 1          # nothing is forgotten over a capture
+    assert waits((0, 1, "eager"), (1, 2, "capture"), (0, 1, "eager"), (1, 2, "eager")) >= 1
+    assert waits((0, 1, "eager"), (1, 1, "made"), (1, 2, "eager"), (1, 2, "eager")) == 1             # ... nor over an engine that is made in between
+    assert waits((0, 2, "eager"), (0, 3, "capture"), (0, 1, "replay"), (1, 2, "eager")) == 1
+    assert waits(*((i % 3, 1, "eager") for i in range(9))) == 0
+    assert waits(*((0, i % 3, "eager") for i in range(9))) == 0                                      # (its own calls are its caller's to order)
+    rng = random.Random(1)
+    moves = list(itertools.product(range(3), range(1, 4), ("eager", "eager", "capture", "made")))
+    for _ in range(3000):
+        waits(*(rng.choice(moves) for _ in range(rng.randint(2, 8))))

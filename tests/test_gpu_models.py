@@ -58,10 +58,26 @@ def test_encoders_take_turns_on_a_handle(dev):
     assert not torch.equal(want[0], want[1])
     side, main = torch.cuda.Stream(), torch.cuda.current_stream()
     side.wait_stream(main)
-    got = []
-    for i, m in enumerate((0, 1, 0, 1, 2, 0, 2, 1)):
-        with torch.cuda.stream(side if i % 3 == 2 else main):
+    got, behind = [], []
+
+    def encode(m, stream):
+        """every encode starts late: one that should have waited for it and has not would overlap it"""
+        with torch.cuda.stream(stream):
+            torch.cuda._sleep(4_000_000)
             got.append((m, encs[m](pix, grid, merge)))
+            assert all(e.query() for n, s, e in behind if n != m and s != stream)
+            behind.append((m, stream, torch.cuda.Event()))
+            behind[-1][2].record()
+    for i, m in enumerate((0, 1, 0, 1, 2, 0, 2, 1)):
+        encode(m, side if i % 3 == 2 else main)
+    # a capture in between waits for nothing, and what runs behind it still does
+    encode(0, main)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.stream(side):
+        graph.capture_begin(capture_error_mode="thread_local")
+        encs[1](pix, grid, merge)
+        graph.capture_end()
+    encode(1, side)
     torch.cuda.synchronize()
     for m, out in got:
         assert torch.equal(out, want[m])
