@@ -1014,7 +1014,11 @@ int cogs_k_attention_vit(hipStream_t st, const CogsAttn& a) {
         const int nlb = p.uniform_len - 64 * (nt - 1) > 32 ? 2 : 1;
         dim3 grid_ahead = grid;
         const long slice = (long)grid.x * grid.y;
-        if (p.next[1].W && p.xcd_order && (p.nseg + 1) * slice <= 256) grid_ahead.z += max(1, min((int)(AHEAD_WGS / slice), (int)(256 / slice) - p.nseg));
+        if (p.next[1].W && p.xcd_order && (p.nseg + 1) * slice <= 256) {
+            grid_ahead.z += max(1, min((int)(AHEAD_WGS / slice), (int)(256 / slice) - p.nseg));
+            if (a.next_read) *a.next_read = true;
+            g_cogs_debug.weights_ahead_read += 1 + (p.next[0].W != nullptr);
+        }
 #define COGS_AV_LAUNCH(R_, B_) hipLaunchKernelGGL((attn_vit_pipe_kernel<72, R_, B_>), grid_ahead, dim3(256), 0, st, p)
         g_cogs_debug.attn_vit_last_end = r * 10 + (r ? nlb : 0);
         switch (r * 10 + (r ? nlb : 0)) {

@@ -85,6 +85,8 @@ cogs_status cogs_debug_get(const char* name, int64_t* value) {
     if (strcmp(name, "attn_last_rows") == 0) { *value = g_cogs_debug.attn_last_rows; return COGS_OK; }
     if (strcmp(name, "mla_last_waves") == 0) { *value = g_cogs_debug.mla_last_waves; return COGS_OK; }
     if (strcmp(name, "preprocess_last_kernel") == 0) { *value = g_cogs_debug.preprocess_last_kernel; return COGS_OK; }
+    if (strcmp(name, "weights_ahead_read") == 0) { *value = g_cogs_debug.weights_ahead_read; return COGS_OK; }
+    if (strcmp(name, "weights_ahead_counted_on") == 0) { *value = g_cogs_debug.weights_ahead_counted_on; return COGS_OK; }
     if (strcmp(name, "km_pp_last_launches") == 0) { *value = g_cogs_debug.km_pp_last_launches; return COGS_OK; }
     if (strcmp(name, "attn_vit_last_end") == 0) { *value = g_cogs_debug.attn_vit_last_end; return COGS_OK; }
     return COGS_E_INVALID;
@@ -107,6 +109,8 @@ const char* cogs_debug_list(void) {
         "mla_last_waves (read only): waves per query tile of the last prompt attention of a described decoder in bf16, 4 or 8\n"
         "preprocess_last_kernel (read only): kernel of the last cogs_preprocess_frames -- 1 two passes, 2 vector tiles, else matrix products: "
         "100 x 64-byte steps of a row + 10 x patch rows of a band + 16-row tiles of its source rows\n"
+        "weights_ahead_read (read only): products whose weights a launch in front of them has read into L2\n"
+        "weights_ahead_counted_on (read only): mid-size products that left out their own read-ahead because of that\n"
         "km_pp_last_launches (read only): form of the last cogs_kmeans_pp, 1 a row per workgroup, 3 by slices\n";
 }
 
@@ -433,6 +437,7 @@ struct VitRange {
     float *rc = nullptr, *rs = nullptr, *lut = nullptr, *stat_part = nullptr, *ln_ab = nullptr;
     int32_t *cu = nullptr, *lo = nullptr, *hi = nullptr;
     bool fold = false, use_lut = false, prescale_q = false, head_major = false;
+    bool qkv_read = false;                // the layer in front has read this one's first weights ahead
     int maxpos = 0, max_seq = 0, uniform_seq = 0;
     float scale = 1.f;
 
@@ -751,10 +756,10 @@ cogs_status VitRange::layer(int l) {
     const cogs_vit_layer& L = h->vit_layers[l];
     if (!fold) { PROF(COGS_PROF_NORM); COGS_TRY(cogs_k_layernorm(st, dt, x, ln, L.ln1_g, L.ln1_b, (int)N, H, w.ln_eps)); }
     CogsGemm qkv_g = qkv_product(l), out = out_product(l), fc1 = fc1_product(l), fc2 = fc2_product(l);
-    qkv_g.weights_read = l > 0 && cogs_k_gemm_weights_ahead(fc2).W && cogs_k_gemm_weights_ahead(qkv_g).W;
+    qkv_g.weights_read = qkv_read;
     if (attn_mode != COGS_ATTN_REF_EAGER_GLOBAL && qkv_g.weights_read) {
         qkv_g.next = cogs_k_gemm_weights_ahead(out);
-        out.weights_read = qkv_g.next.W != nullptr;
+        qkv_g.next_read = &out.weights_read;
     }
     { PROF(COGS_PROF_GEMM); COGS_TRY(cogs_k_gemm(st, qkv_g)); }
     {
@@ -773,16 +778,20 @@ cogs_status VitRange::layer(int l) {
             a.uniform_seqlen = uniform_seq;      // all frames alike (one video, or videos of one grid): see attn_vit.hip
             if (!out.weights_read) a.next[0] = cogs_k_gemm_weights_ahead(out);
             a.next[1] = cogs_k_gemm_weights_ahead(fc1);
-            fc1.weights_read = a.next[1].W != nullptr;
         }
+        bool read = false;
+        a.next_read = &read;
         { PROF(COGS_PROF_ATTN); COGS_TRY(cogs_k_attention(st, a)); }
+        if (a.next[0].W) out.weights_read = read;
+        fc1.weights_read = read;
     }
     out.next = cogs_k_gemm_weights_ahead(fc2);
-    fc2.weights_read = out.next.W != nullptr;
+    out.next_read = &fc2.weights_read;
     { PROF(COGS_PROF_GEMM); COGS_TRY(cogs_k_gemm(st, out)); }
     if (!fold) { PROF(COGS_PROF_NORM); COGS_TRY(cogs_k_layernorm(st, dt, x, ln, L.ln2_g, L.ln2_b, (int)N, H, w.ln_eps)); }
     { PROF(COGS_PROF_GEMM); COGS_TRY(cogs_k_gemm(st, fc1)); }
     if (l + 1 < w.layers) fc2.next = cogs_k_gemm_weights_ahead(qkv_product(l + 1));
+    fc2.next_read = &qkv_read;
     { PROF(COGS_PROF_GEMM); COGS_TRY(cogs_k_gemm(st, fc2)); }
     return COGS_OK;
 }

@@ -81,6 +81,8 @@ struct CogsDebug {
     // ... and the last cogs_preprocess_frames: 1 two passes, 2 vector tiles, else matrix products: 100 x 64-byte steps + 10 x patch rows of a band +
     // 16-row tiles of its source rows
     std::atomic<long long> preprocess_last_kernel{0};
+    // products whose weights a launch in front has read into L2, and mid-size ones that left their own read-ahead out for it (never more)
+    std::atomic<long long> weights_ahead_read{0}, weights_ahead_counted_on{0};
     // ... and the last cogs_kmeans_pp: 1 a row per workgroup, 3 by slices
     std::atomic<long long> km_pp_last_launches{0};
 };

@@ -1357,6 +1357,7 @@ static int gemm_rows(hipStream_t st, const CogsGemm& g, bool* kv_stored) {
 
 int cogs_k_gemm(hipStream_t st, const CogsGemm& g, bool* kv_stored) {
     bool stored = g.M == 1;
+    if (g.next_read) *g.next_read = false;
     const int rc = gemm_rows(st, g, &stored);
     if (kv_stored) *kv_stored = stored;
     return rc;

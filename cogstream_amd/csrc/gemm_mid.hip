@@ -398,6 +398,7 @@ void launch(hipStream_t st, MidArgs& p, bool alone) {
     p.ln_staged = (long)TM * p.ln_tiles * 8 <= KS * (TM + TN) * ROW_BYTES && ((long)p.M * p.ln_tiles) % 2 == 0;
     const int tiles = p.nbm * p.nbn + p.nbm0 * p.nbn0;
     const int extra = !alone || p.rows0 != 0 ? 0 : p.next.W ? max(MID_CUS - tiles, 0) / 8 * 8 : p.hot ? 0 : read_ahead_workgroups(tiles);
+    if (extra == 0) p.next.W = nullptr;
     hipLaunchKernelGGL((gemm_mid_kernel<EPI, MI, NI, WM, WN, S, WPE, KS, IL>), dim3(tiles + extra), dim3(64 * WM * WN), lds, st, p);
 }
 
@@ -469,5 +470,8 @@ int cogs_k_gemm_mid(hipStream_t st, const CogsGemm& g, int tile, bool alone, int
         default: dispatch_tile<EPI_GENERIC>(st, p, tile, alone); break;
     }
 #undef COGS_MID_CASE
+    if (g.next_read) *g.next_read = p.next.W != nullptr;
+    g_cogs_debug.weights_ahead_read += p.next.W != nullptr;
+    g_cogs_debug.weights_ahead_counted_on += g.weights_read;
     return COGS_LAUNCH_CHECK();
 }

@@ -52,6 +52,7 @@ struct CogsGemm {
     // forms each row's factor itself, or cogs_k_ln_finalize runs first
     const float* ln_part = nullptr; float ln_eps = 0.f;
     CogsWeightsAhead next;                   // read on idle CUs of a mid-size launch, instead of its own weights
+    bool* next_read = nullptr;               // != null: set to whether it was (the launch may be of another kind, or leave no CU idle)
     bool weights_read = false;               // its weights were some launch's `next`
 };
 // the weights of product g as a launch in front of it reads them ahead (weights_ahead.h); none where they are no mid-size product's of one round
@@ -65,6 +66,7 @@ int cogs_k_ln_finalize(hipStream_t st, const float* stat_part, int rows, int til
 
 struct CogsAttn {
     CogsWeightsAhead next[2];         // ViT kernel: read on the CUs that few workgroups leave idle
+    bool* next_read = nullptr;        // != null: set to whether both were
     int dtype = 0;
     const void* Q = nullptr; const void* K = nullptr; const void* V = nullptr; void* O = nullptr;
     long ldq = 0, ldk = 0, ldv = 0, ldo = 0;

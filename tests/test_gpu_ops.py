@@ -1586,3 +1586,31 @@ def test_weights_read_ahead_change_nothing(dev, grid):
     with L2.debug_switch("gemm_co_streams", 2):
         want = run()
     assert torch.isfinite(got.float()).all() and torch.equal(got, want)
+
+
+@pytest.mark.parametrize("grid,heads,mode", [((1, 16, 16), 16, {}), ((16, 6, 6), 16, {}), ((9, 8, 8), 16, {}), ((2, 4, 4), 8, {}), ((1, 16, 16), 9, {}), ((1, 24, 24), 16, {}),
+                                             ((1, 16, 16), 16, {"attn_vit": 1}), ((1, 16, 16), 16, {"attn_vit": 0}), ((1, 16, 16), 16, {"gemm_mid": 3})])
+def test_read_ahead_is_counted_on_only_where_it_was(dev, grid, heads, mode):
+    """a product leaves out its own read-ahead of weights only where a launch in front has really read them: not behind an attention of many short frames, of heads whose number or size
+    its kernel has no such workgroups for, or of another kernel. Never more products than were read ahead, and of one image with 16 heads of 72 all four of a layer"""
+    import contextlib
+    from cogstream_amd import _lib as L2
+    from cogstream_amd.vision import VisionEncoder
+    from cogstream_amd.weights import VisionConfig, random_vit_state
+    layers = 3
+    cfg = VisionConfig(num_hidden_layers=layers, num_attention_heads=heads)
+    enc = VisionEncoder(random_vit_state(cfg, seed=1, device=dev, dtype=torch.bfloat16), cfg)
+    n = grid[0] * grid[1] * grid[2]
+    pix = (torch.rand(n, cfg.patch_dim, generator=torch.Generator(device=dev).manual_seed(n), device=dev) * 2 - 1).bfloat16()
+    with contextlib.ExitStack() as switches:
+        for name, value in mode.items():
+            switches.enter_context(L2.debug_switch(name, value))
+        before = [L2.debug_get(k) for k in ("weights_ahead_read", "weights_ahead_counted_on")]
+        out = enc(pix, torch.tensor([grid]), torch.tensor([1]))
+        read, counted = (L2.debug_get(k) - b for k, b in zip(("weights_ahead_read", "weights_ahead_counted_on"), before))
+    assert torch.isfinite(out.float()).all()
+    assert counted <= read
+    if grid == (1, 16, 16) and heads == 16 and not mode:
+        assert counted == read == 4 * layers - 1             # (the first layer's first weights are its own product's to read)
+    if grid == (16, 6, 6):
+        assert 0 < read < 4 * layers - 1
