@@ -1017,7 +1017,9 @@ int launch_update(hipStream_t st, int dtype, const void* feats, const float* ts,
     else
         hipLaunchKernelGGL(update_kernel<float>, dim3(nblk, K), dim3(256), 0, st, (const float*)feats, PD, K, w.offs, w.members,
                            w.reseed, ctl, centres, w.partial, ctl ? w.keep : nullptr);
-    const int t_lds = T <= MEMB_T ? T : 0;       // member-ordered time stamps staged in LDS (64 KiB at most)
+    const int t_lds = T <= MEMB_T ? T : 0;       // member-ordered time stamps staged in LDS: up to 64 KiB, and 1 KiB of the kernel's own beside them
+    static std::atomic<uint64_t> attr_done{0};
+    cogs_ensure_dyn_lds((const void*)update_final_kernel, MEMB_T * 4, attr_done);
     hipLaunchKernelGGL(update_final_kernel, dim3(1), dim3(UF_T), (size_t)t_lds * 4, st, ts, K, w.offs, w.members, w.reseed, ctl,
                        centre_ts, w.partial, nblk, w.scratch, shift_out, status, t_lds, tol, watch);
     return COGS_LAUNCH_CHECK();

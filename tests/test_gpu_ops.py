@@ -1614,3 +1614,30 @@ def test_read_ahead_is_counted_on_only_where_it_was(dev, grid, heads, mode):
         assert counted == read == 4 * layers - 1             # (the first layer's first weights are its own product's to read)
     if grid == (16, 6, 6):
         assert 0 < read < 4 * layers - 1
+
+
+@pytest.mark.parametrize("K", [2, 130])
+@pytest.mark.parametrize("T", [16127, 16128, 16129, 16251, 16381, 16384])
+def test_means_of_as_many_rows_as_the_loop_takes(dev, T, K):
+    """up to the documented limits (T + K + 1 <= 16 384 in the loop, no more than 16 384 staged time stamps in a step), where the last kernel of an update has 64 KiB of LDS and
+    more: centres of whole numbers, so that every sum is exact"""
+    from cogstream_amd import _lib as L2
+    ops = _ops()
+    a = torch.arange(T, device=dev) * 7 % K
+    x = (a[:, None] * 64 + torch.arange(8, device=dev)).float()
+    ts = (torch.arange(T, device=dev) % 13).float()
+    sums = torch.zeros(K, dtype=torch.float64, device=dev).index_add_(0, a, ts.double())
+    mean = sums.float() / torch.bincount(a, minlength=K).float()
+    start = lambda: (x[:K].clone().index_copy_(0, a[:K], x[:K]) + 1, torch.full((K,), 6.0, device=dev))
+    ws = ops.kmeans_workspace(T, 8, K, x.device)
+    c, ct = start()
+    ops.kmeans_update(x, ts, a, torch.zeros(K, dtype=torch.int32, device=dev), c, ct, ws)
+    assert torch.equal(ct, mean) and torch.equal(c, torch.arange(K, device=dev)[:, None] * 64 + torch.arange(8, device=dev).float())
+    c, ct = start()
+    got = torch.empty(T, dtype=torch.int64, device=dev)
+    if T + K + 1 > 16384:
+        with pytest.raises(L2.CogsError):
+            ops.kmeans_lloyd(x, ts, c, ct, got, 0.0, 4, 1e-4, [], ws)
+        return
+    assert ops.kmeans_lloyd(x, ts, c, ct, got, 0.0, 4, 1e-4, [], ws) == (2, 0, False)
+    assert torch.equal(got, a) and torch.equal(ct, mean) and torch.equal(c, torch.arange(K, device=dev)[:, None] * 64 + torch.arange(8, device=dev).float())
