@@ -1085,9 +1085,20 @@ int cogs_k_kmeans_pp_step(hipStream_t st, int dtype, const void* feats, int T, l
 //   bf16, 896 KB         0.50  0.44  0.56  0.65  0.70  0.76  0.78  0.52  0.50
 //   fp32, 128 KB         1.07  1.03  1.06  1.08  1.01  1.07  1.12  1.02  0.99
 //   fp32, 350 KB         0.68  0.72  0.67  0.90  0.97  1.00  1.10  0.76  0.85
+// and of nearly as many rows as CUs (fp32 rows are half as many values):
+//                     T = 193   200   224   240   256
+//   bf16, 400 KB         1.00  1.00  1.06  1.03  1.10
+//   bf16, 448 KB         0.94  0.97  1.01  1.03  1.07
+//   bf16, 512 KB         0.96  0.97  1.02  1.05  1.06
+//   bf16, 640 KB         0.92  0.94  0.98  0.98  1.03
+//   fp32, 350 KB         1.03  1.04  1.12  1.12  1.13
+//   fp32, 416 KB         0.93  0.94  1.00  0.99  1.03
+//   fp32, 448 KB         0.91  0.91  0.96  0.96  0.99
+//   fp32, 512 KB         0.90  0.91  0.94  0.96  0.99
 static bool kpp_in_one_launch(int dtype, int T, long PD) {
     const long kb = PD * (dtype == COGS_DT_BF16 ? 2 : 4) >> 10;
-    return kb <= 100 ? T <= 300 : T <= 256 && kb <= (T > 192 ? 512 : T >= 100 ? 224 : 128);
+    const bool bf = dtype == COGS_DT_BF16;
+    return kb <= 100 ? T <= 300 : T <= 256 && kb <= (T < 100 ? 128 : T <= 192 ? 224 : T < 224 ? (bf ? 400 : 352) : bf ? 512 : 416);
 }
 
 // The whole k-means++ seeding (kmeans_with_time.py:41-62) in one call, no host round trip per centre: up to K - 1 passes measure

@@ -1383,9 +1383,8 @@ def test_preprocessing_is_not_captured(dev):
 @pytest.mark.parametrize("T,PD,K", [(2, 8, 2), (5, 520, 4), (257, 1000, 9), (300, 4096, 12), (3, 6_300_000, 3), (130, 179_200, 4), (24, 179_200, 4),
                                     (256, 65_536, 3), (257, 65_536, 3), (160, 65_544, 3), (161, 65_536, 3)])
 def test_whole_seeding_equals_the_steps(dev, T, PD, K, dtype):
-    """cogs_kmeans_pp draws the rows that distances of cogs_kmeans_pp_step and the same exponentials give on the host, with one launch a
-    centre and with three: one slice and fewer, a ragged last slice, more rows than a workgroup's threads draw from at once, sizes on
-    both sides of the lines between the two; rows that all coincide raise the flag"""
+    """cogs_kmeans_pp draws the rows that distances of cogs_kmeans_pp_step and the same exponentials give on the host, by passes with a row per workgroup (form 1) and
+    by slices (form 3): one slice and fewer, a ragged last slice, more rows than a workgroup's threads draw from at once; rows that all coincide raise the flag"""
     from cogstream_amd import _lib as L2
     ops = _ops()
     g = torch.Generator(device=dev).manual_seed(T)
@@ -1409,6 +1408,35 @@ def test_whole_seeding_equals_the_steps(dev, T, PD, K, dtype):
     same = x[:1].expand(T, PD).contiguous()
     _, flag = ops.kmeans_pp(same, first, K, q.to(dev), ws)
     assert int(flag) == 1
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("T,kb,bf16,fp32", [(300, 100, 1, 1), (301, 100, 3, 3), (256, 101, 1, 1), (257, 101, 3, 3), (99, 128, 1, 1), (99, 129, 3, 3), (100, 129, 1, 1), (100, 224, 1, 1),
+                                            (100, 225, 3, 3), (192, 224, 1, 1), (192, 225, 3, 3), (193, 225, 1, 1), (193, 352, 1, 1), (193, 353, 1, 3), (223, 400, 1, 3),
+                                            (223, 401, 3, 3), (224, 401, 1, 1), (224, 416, 1, 1), (224, 417, 1, 3), (256, 512, 1, 3), (256, 513, 3, 3), (257, 512, 3, 3)])
+def test_forms_of_the_seeding_on_both_sides_of_their_lines(dev, T, kb, bf16, fp32, dtype):
+    """the form that rows and bytes a row choose, and the rows and distances it draws by: those of the other form, and of a step per centre"""
+    from cogstream_amd import _lib as L2
+    ops = _ops()
+    K, PD, form = 4, kb * 1024 // dtype.itemsize, bf16 if dtype == torch.bfloat16 else fp32
+    g = torch.Generator(device=dev).manual_seed(T + kb)
+    x = (torch.randn(5, PD, generator=g, device=dev)[torch.arange(T, device=dev) * 5 // T] + 0.2 * torch.randn(T, PD, generator=g, device=dev)).to(dtype)
+    q = torch.empty(K - 1, T).exponential_(1, generator=torch.Generator().manual_seed(T))
+    ws = ops.kmeans_workspace(T, PD, K, x.device)
+    got = []
+    for forced in (0, 1, 3):
+        d2 = torch.full((T, K), -1.0, device=dev)
+        with L2.debug_switch("km_pp_form", forced):
+            idx, flag = ops.kmeans_pp(x, T // 2, K, q.to(dev), ws, d2)
+        assert L2.debug_get("km_pp_last_launches") == (form if forced == 0 else 3 if T > 300 else forced)
+        got.append((idx.tolist(), int(flag), d2))
+    near, probs, want = torch.empty(T, device=dev), torch.empty(T).pin_memory(), [T // 2]
+    for m in range(K - 1):
+        ops.kmeans_pp_step(x, want[-1], m == 0, near, probs, ws)
+        p = probs.sqrt() ** 2
+        want.append(int((p / p.double().sum().float() / q[m]).argmax()))
+    for rows, zero, d2 in got:
+        assert rows == want and zero == 0 and torch.equal(d2, got[0][2])
 
 
 @pytest.mark.parametrize("form", [1, 3])
