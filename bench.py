@@ -137,8 +137,8 @@ def stage_rooflines(c3, mm3, dev, with_cpu=True):
     passes = st["kpp_passes"] + 2 * st["iterations"]
     out = [hbm_stage("kmeans_with_time_min_max (A8)", "sqdist_kernel / update_kernel (csrc/kmeans.hip)",
                      "model/kmeans_with_time.py:4-137", passes * T3 * P3 * D * es, t_km,
-                     f"[{T3},{P3 * D}] bf16 features, K={K}: {st['kpp_passes']} k-means++ passes + {st['iterations']} Lloyd "
-                     f"iterations x 2 passes (distances, means) over the features; wall time of the whole call (seeding in one "
+                     f"[{T3},{P3 * D}] bf16 features, K={K}: {st['kpp_passes']} k-means++ passes (at least: up to four "
+                     f"centres are drawn a pass) + {st['iterations']} Lloyd iterations x 2 passes (distances, means) over the features; wall time of the whole call (seeding in one "
                      f"library call from host-drawn exponentials, Lloyd iterations queued four at a time; {st.get('kpp_path', '')}). "
                      f"The algorithm itself re-reads the SAME {T3 * P3 * D * es / 1e6:.0f} MB of features on every pass, so all "
                      f"passes after the first are Infinity-Cache reads by construction -- not an artefact of the timing loop",

@@ -17,8 +17,10 @@ import torch
 
 from . import ops
 
+PP_DRAWS = 4          # centres a pass of cogs_kmeans_pp draws at most
 last_stats = {"kpp_passes": 0, "iterations": 0, "kpp_path": "", "min_rel_margin": float("inf"), "rows_below_1e-3": 0}
-"""of the most recent call (bytes moved per stage, how close the assignments were).
+"""of the most recent call (bytes moved per stage, how close the assignments were). kpp_passes = passes over the features that the seeding took:
+exact where it went step by step, else the fewest it can have taken (a pass draws up to PP_DRAWS centres; the device alone knows how many came true).
 min_rel_margin = over all rows and Lloyd iterations, the smallest relative change of a row's feature distances that
 would flip its cluster (cogs_kmeans_margins; (d2 - d1) / mean(d1, d2) of the two nearest centres when the time terms are
 equal); rows_below_1e-3 = (row, iteration) pairs under 1e-3, where the reference's own cdist rounding decides a row."""
@@ -109,7 +111,8 @@ def kmeans_with_time_min_max(features: torch.Tensor, timestamp, cluster_num: int
         last_stats["kpp_path"] = "step by step (a zero-probability step)"
         run = _lloyd_from_rows(x, ts, torch.tensor(idx, dtype=torch.int64, device=dev), K, PD, alpha, max_iteration, tol, ws, report=report)
     centres, centre_ts, assign, done = run
-    last_stats["kpp_passes"], last_stats["iterations"] = K - 1, done
+    last_stats["kpp_passes"] = -(-(K - 1) // PP_DRAWS) if last_stats["kpp_path"] == "one call" else K - 1
+    last_stats["iterations"] = done
     last_stats["min_rel_margin"], last_stats["rows_below_1e-3"] = report.get("margins", (float("inf"), 0))
     return centres.view(K, P, D), centre_ts, assign
 

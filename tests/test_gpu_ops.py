@@ -1669,3 +1669,14 @@ def test_means_of_as_many_rows_as_the_loop_takes(dev, T, K):
         return
     assert ops.kmeans_lloyd(x, ts, c, ct, got, 0.0, 4, 1e-4, [], ws) == (2, 0, False)
     assert torch.equal(got, a) and torch.equal(ct, mean) and torch.equal(c, torch.arange(K, device=dev)[:, None] * 64 + torch.arange(8, device=dev).float())
+
+
+@pytest.mark.parametrize("K,passes", [(2, 1), (5, 1), (6, 2), (18, 5)])
+def test_passes_of_a_seeding_are_not_overstated(dev, K, passes):
+    """last_stats counts the passes a seeding in one call takes at least (up to four centres each), and every one of a seeding step by step"""
+    from cogstream_amd import kmeans
+    x = torch.randn(40, 1, 64, generator=torch.Generator(device=dev).manual_seed(K), device=dev)
+    kmeans.kmeans_with_time_min_max(x, torch.arange(40.0), K)
+    assert kmeans.last_stats["kpp_path"] == "one call" and kmeans.last_stats["kpp_passes"] == passes
+    kmeans.kmeans_with_time_min_max(x[:1].expand(40, 1, 64).contiguous(), torch.arange(40.0), K)
+    assert kmeans.last_stats["kpp_path"].startswith("step by step") and kmeans.last_stats["kpp_passes"] == K - 1
