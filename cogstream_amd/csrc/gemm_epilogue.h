@@ -95,8 +95,13 @@ __device__ __forceinline__ float rowgroup_sum(float x) {
     return __builtin_bit_cast(float, (unsigned)b[0]) + __builtin_bit_cast(float, (unsigned)b[1]);
 }
 
-// columns nb .. nb + n - 1 are a head's, and none of them is turned
-__device__ __forceinline__ bool stands_still(const EpiArgs& p, int nb, int n) { return p.rope_still > 0 && nb % p.head_dim + n <= p.rope_still; }
+// columns nb .. nb + n - 1 are a head's, and none of them is turned. Asked where there is no bias, as with the queries of latent attention: with one, the rotary products of
+// the other models were the slower for the question alone (621 x 4608 x 3584 32.6 -> 33.3 us)
+template <int EPI>
+__device__ __forceinline__ bool stands_still(const EpiArgs& p, int nb, int n) {
+    if constexpr ((EPI & EPI_BIAS) != 0) return false;
+    return p.rope_still > 0 && nb % p.head_dim + n <= p.rope_still;
+}
 // (cos, sin) of the two rotary pairs pi, pi+1 of row m, from either table format
 __device__ __forceinline__ void rope_load(const EpiArgs& p, long m, int pi, f32x2& c, f32x2& s) {
     if (p.rope_sin) {
@@ -180,7 +185,7 @@ struct EpiOperands {
         for (int mi = 0; mi < MI; ++mi) {
             const int m = min(mb + (lane & 15) + 16 * mi, M - 1);
             if constexpr ((EPI & EPI_ROPE) != 0)
-                if (!stands_still(p, nb, 16 * NI))
+                if (!stands_still<EPI>(p, nb, 16 * NI))
 #pragma unroll
                 for (int ni = 0; ni < NI; ++ni) rope_load(p, m, (min(nb + 4 * g4 + 16 * ni, N - 4) % p.head_dim) >> 1, cs[mi][ni], sn[mi][ni]);
             if constexpr ((EPI & EPI_RES) != 0)
@@ -237,7 +242,7 @@ __device__ __forceinline__ void epilogue_tile(const EpiArgs& p, int mb, int nb, 
         // SwiGLU rows in whole 8- or 16-byte units: the wave's outputs all inside the row, rows and base aligned
         constexpr bool CAN_PACK = sizeof(T) == 2 && (EPI & ~EPI_BIAS) == EPI_SWIGLU;
         const bool packed = CAN_PACK && nb + 16 * NI <= N && (p.ldc & 7) == 0 && (reinterpret_cast<unsigned long>(p.C) & 15) == 0;
-        const bool still = (EPI & EPI_ROPE) != 0 && stands_still(p, nb, 16 * NI);
+        const bool still = (EPI & EPI_ROPE) != 0 && stands_still<EPI>(p, nb, 16 * NI);
         const int g4 = lane >> 4;
         const int wcol = 16 * (g4 & 1) + 8 * (g4 >> 1);   // this lane's 8 columns inside a 32-column tile pair
         f32x4 bias_v[NI];
@@ -539,7 +544,7 @@ __device__ __forceinline__ void epilogue_tile_fast(const EpiArgs& p, int mb, int
 // columns are such, and a rotary epilogue's factors are as many loads again as twice its stores (4096 x 3072 x 768 36 -> 33 us)
 template <typename... Accs>
 __device__ __forceinline__ bool scale_still(const EpiArgs& p, int nb, Accs&... accs) {
-    if (!stands_still(p, nb, 64)) return false;
+    if (!stands_still<0>(p, nb, 64)) return false;
     const float f = nb < p.q_cols ? p.q_scale : 1.f;
     auto scale = [f](f32x4 (&a)[4][4]) {
 #pragma unroll
