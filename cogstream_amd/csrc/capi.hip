@@ -54,7 +54,7 @@ static bool cogs_debug_value_ok(const char* name, int64_t v) {
     static const Range ranges[] = {
         {"gemm_wgs", 0, 256}, {"gemm_mid", 0, 11}, {"gemm_pad_pct", 100, 400}, {"gemm_group_m", 0, 64}, {"gemm_co_streams", 0, 8},
         {"gemv_small_n", 0, 1 << 30}, {"attn_vit", 0, 2}, {"attn_uniform_hint", 0, 1 << 20}, {"attn_prio", 0, 2},
-        {"attn_nq", 0, 2}, {"vit_split_max", 0, INT64_MAX}, {"llm_split_keys", 0, 1 << 24}, {"mla_split_keys", 0, 1 << 24}, {"km_row_groups", 0, 1 << 16}, {"km_pp_form", 0, 3},
+        {"attn_nq", 0, 2}, {"vit_split_max", 0, INT64_MAX}, {"llm_split_keys", 0, 1 << 24}, {"mla_split_keys", 0, 1 << 24}, {"km_row_groups", 0, 1 << 16}, {"km_pp_form", 0, 3}, {"delta_zeros", 0, 2},
     };
     for (const Range& r : ranges)
         if (strcmp(name, r.name) == 0) return v >= r.lo && v <= r.hi;

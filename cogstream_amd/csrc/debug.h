@@ -53,6 +53,7 @@
     X(mla_split_keys, 0, "> 0: keys per split of the latent decode attention (0: chosen from the batch and the context)")   \
     X(delta_chunk, 1, "0: gated delta rule of prompts token by token instead of in chunks")                                 \
     X(delta_out_wave, 0, "1: read-outs of the gated delta rule normed by a wave per head at any width (same bits)")         \
+    X(delta_zeros, 0, "tokens past the end of a chunk's sequence 1: stored as zeros, 2: masked where they are read (0: chosen per step, same bits)")          \
     X(gemm_skinny, 1, "0: the decoder's few-row products through the general GEMM")                                         \
     X(km_pp_form, 0, "> 0: k-means++ passes with 1 a row per workgroup (up to 300 rows), 3 by slices (0: chosen per size)")          \
     X(km_row_groups, 0, "> 0: row groups of the k-means distance pass (0: sized to fill the chip)")

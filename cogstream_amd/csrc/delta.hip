@@ -35,7 +35,7 @@ constexpr int REC = EXPS + 3 * CH;            // P as A operands [4 steps][64 la
 
 // Chunks have q, k and v as the operands of the scan's 16x16 tiles, [chunk][16 tokens a][16 columns t][64 lanes][4 floats]: q and k with a token per lane
 // (lane 16 g + li: token li, columns 4 g ..), k once more and v with a column per lane (column li, tokens 4 g ..). A sequence starts on a chunk of
-// its own, tokens past its end are zeros. An operand is one load of 1 KiB in a row, 25 of them a wave and chunk; as rows it was sixteen lines of 64 bytes, and those
+// its own; tokens past its end are zeros, or read as such (p.pad, cogs_k_delta_prompt). An operand is one load of 1 KiB in a row, 25 of them a wave and chunk; as rows it was sixteen lines of 64 bytes, and those
 // with a column per lane four loads of 4 bytes a lane, 43 in all. 4096 rows, 16 heads of 128: scan 206 -> 198 us, 32 heads 242 -> 227 and the chunks
 // 57 -> 49; the inputs 31 -> 36 (k is written twice). Prompts of 4096 rows, width 2048 5021 -> 4963 us, of 700 1450 -> 1428, of 300, width 4096
 // 2101 -> 2081. (T, v and the exponentials, which all four waves read, through LDS instead of into each one's registers: 206 again.)
@@ -91,7 +91,8 @@ __global__ __launch_bounds__(256) void delta_inputs_kernel(CogsDelta p) {
     const CogsSeq s = p.seqs[seq];
     const int lane = threadIdx.x & 63, wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int i0 = blockIdx.x * RUN, n = min(RUN, s.len - i0);
-    if (i0 >= (s.len + CH - 1) / CH * CH) return;              // (runs of zeros behind the end belong to its chunk)
+    if (n <= 0 && (!p.pad || i0 >= (s.len + CH - 1) / CH * CH)) return;      // (runs of zeros behind the end belong to its chunk)
+    const int stored = p.pad ? RUN : n;                        // tokens
     const int nqk = 2 * p.kv_heads, nv = p.heads * p.dvp, units = nqk + (nv + 64 * E - 1) / (64 * E);
     const int unit = blockIdx.y * 4 + wid, v0 = nqk * p.dkp;
     const long row0 = s.row0 + i0;
@@ -158,10 +159,10 @@ __global__ __launch_bounds__(256) void delta_inputs_kernel(CogsDelta p) {
 #pragma unroll
         for (int q = 0; q < RUN / 4; ++q) {
             f32x4 v = y[q][e];
-            if (mine && unit >= p.kv_heads) *reinterpret_cast<f32x4*>(by_column + at + column_major(width >> 4, a, first + 4 * q, col)) = v;
+            if (mine && 4 * q < stored && unit >= p.kv_heads) *reinterpret_cast<f32x4*>(by_column + at + column_major(width >> 4, a, first + 4 * q, col)) = v;
             if (is_v) continue;
             quad_transpose(v, lane);
-            if (mine) *reinterpret_cast<f32x4*>((unit < p.kv_heads ? p.q : p.k) + at + token_major(width >> 4, a, first + 4 * q + (lane & 3), col & ~3)) = v;
+            if (mine && 4 * q + (lane & 3) < stored) *reinterpret_cast<f32x4*>((unit < p.kv_heads ? p.q : p.k) + at + token_major(width >> 4, a, first + 4 * q + (lane & 3), col & ~3)) = v;
         }
     }
 }
@@ -173,7 +174,7 @@ __global__ __launch_bounds__(256) void delta_inputs_any_kernel(CogsDelta p) {
     const int sq = p.rowseq[row], pos = p.rowpos[row];
     const CogsSeq s = p.seqs[sq];
     const int i = row - s.row0, chunk = i / CH;
-    const int after = TILES && i == s.len - 1 ? (i / CH + 1) * CH - s.len : 0;       // rows of zeros that this one is followed by
+    const int after = TILES && i == s.len - 1 ? (p.pad ? (i / CH + 1) * CH - s.len : 3 - (i & 3)) : 0;       // rows of zeros that this one is followed by
     const float* x = p.t + (long)row * p.ldt;
     const float* ring = s.state + p.state_off + (long)p.heads * p.dkp * p.dvp;
     const int back = row - s.row0;
@@ -198,7 +199,7 @@ __global__ __launch_bounds__(256) void delta_inputs_any_kernel(CogsDelta p) {
                 for (int z = 0; z <= after; ++z) {
                     const int r = i + z, b = (r >> 4) & 1;
                     const float y = z ? 0.f : v[e] * f;
-                    o[at + token_major(p.dkp >> 4, b, r & 15, d)] = y;
+                    if (z == 0 || p.pad) o[at + token_major(p.dkp >> 4, b, r & 15, d)] = y;
                     if (j >= p.kv_heads) p.kt[at + column_major(p.dkp >> 4, b, r & 15, d)] = y;
                 }
             } else o[((long)head * p.rows + row) * p.dkp + d] = v[e] * f;
@@ -394,9 +395,10 @@ struct ScanIn {
 // scan, 54 instead of 63 matrix instructions, two terms of V's size were rounded and cancelled: read-outs of 8 recurring pairs were off
 // by 1.2e-7 of them instead of 8.2e-8, values read back from the state by 1.2e-7 instead of 3.5e-8.) K S and Q S are two chains each, and
 // P U and the state's growth sums of their own: chained to what they are added to, they were rounded at its size.
+// MASK: tokens past a sequence's end are not there, but for zeros up to the next fourth one (a lane's own); their lanes read behind the buffers' sizes.
 // The workgroups from `scan` on keep the convolution's last inputs, which nothing here reads: a launch for them alone, between the inputs and
 // the chunks, was 4.9 us a layer (prompts of 100 rows, width 2048 815 -> 793 us, of 4096 5048 -> 5022).
-template <int NK>
+template <int NK, bool MASK>
 __global__ __launch_bounds__(256, NK > 2 ? 1 : 2) void delta_scan_kernel(CogsDelta p, int scan) {
     __shared__ __attribute__((aligned(16))) f32x4 red[2][4][4][64];
     const int seq = blockIdx.z;
@@ -427,6 +429,16 @@ __global__ __launch_bounds__(256, NK > 2 ? 1 : 2) void delta_scan_kernel(CogsDel
     // a lane's places in a chunk's tiles and read-outs (bytes)
     int oo[2];
     const int tmo = lane * 16, po = lane * 4 + wid * 256, ego = 16 * g;
+    int tok[2] = {tmo, tmo}, col[2] = {tmo, tmo};      // ... of tiles with a token, and with a column per lane
+    auto mask = [&](int rows) {
+        if constexpr (MASK)
+#pragma unroll
+            for (int a = 0; a < 2; ++a) {
+                tok[a] = 16 * a + li < rows ? tmo : 1 << 30;
+                col[a] = 16 * a + 4 * g < rows ? tmo : 1 << 30;
+            }
+    };
+    mask(s.len);
     int zo = 0;
     asm("" : "+v"(zo));                          // (a scalar load would share its counter with LDS)
 #pragma unroll
@@ -453,17 +465,18 @@ __global__ __launch_bounds__(256, NK > 2 ? 1 : 2) void delta_scan_kernel(CogsDel
     auto advance = [&] {                                       // (the last chunk is loaded again rather than nothing)
         at = min(at + 1, nc - 1);
         f = From{f0.k + at * step_k, f0.q + at * step_k, f0.kt + at * step_k, f0.v + at * step_v, f0.rec + at * step_rec};
+        mask(s.len - at * CH);
     };
     // load i of a chunk, in the order of their use, the 16-byte ones first
     constexpr int L_Q = 2 * NK, L_E = L_Q + 2 * NK, L_T = L_E + 4, L_V = L_T + 3, L_KT = L_V + 2, L_G = L_KT + 2 * NK, L_PM = L_G + 1, L_ALL = L_PM + 3;
-    auto load = [&](ScanIn<NK>& in, int i) {
+    auto load = [&](ScanIn<NK>& in, int i) __attribute__((always_inline)) {
         auto tile = [&](int j) { return (j / NK * tiles + tn[j % NK]) * TILE * 4; };
-        if (i < L_Q) in.k[i / NK][i % NK] = at4(f.k, bytes_q, tmo, tile(i));
-        else if (i < L_E) { const int j = i - L_Q; in.q[j / NK][j % NK] = at4(f.q, bytes_q, tmo, tile(j)); }
+        if (i < L_Q) in.k[i / NK][i % NK] = at4(f.k, bytes_q, tok[i / NK], tile(i));
+        else if (i < L_E) { const int j = i - L_Q; in.q[j / NK][j % NK] = at4(f.q, bytes_q, tok[j / NK], tile(j)); }
         else if (i < L_T) { const int j = i - L_E; (j & 2 ? in.ec : in.eg)[j & 1] = at4(f.rec, bytes_rec, ego, (EXPS + (j & 2 ? CH : 0) + 16 * (j & 1)) * 4); }
         else if (i < L_V) in.tm[i - L_T] = at4(f.rec, bytes_rec, tmo, (3 + i - L_T) * TILE * 4);
-        else if (i < L_KT) { const int j = i - L_V; in.v[j] = at4(f.v, bytes_v, tmo, j * ldv * 64); }
-        else if (i < L_G) { const int j = i - L_KT; in.kt[j / NK][j % NK] = at4(f.kt, bytes_k[j % NK], tmo, tile(j)); }
+        else if (i < L_KT) { const int j = i - L_V; in.v[j] = at4(f.v, bytes_v, col[j], j * ldv * 64); }
+        else if (i < L_G) { const int j = i - L_KT; in.kt[j / NK][j % NK] = at4(f.kt, bytes_k[j % NK], col[j / NK], tile(j)); }
         else if (i < L_PM) in.gl = at1(f.rec, bytes_rec, zo, (EXPS + 2 * CH) * 4);
         else if (i < L_ALL) in.pm[i - L_PM] = at1(f.rec, bytes_rec, po, (i - L_PM) * TILE * 4);
     };
@@ -489,7 +502,7 @@ __global__ __launch_bounds__(256, NK > 2 ? 1 : 2) void delta_scan_kernel(CogsDel
     auto mine = [&](const f32x4& v) { return wid < 2 ? (wid == 0 ? v[0] : v[1]) : (wid == 2 ? v[2] : v[3]); };
     auto pin = [](f32x4 (&v)[4]) { asm volatile("" : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]), "+v"(v[3])); };      // (used from here on, no earlier)
     // chunk c from `in`, the next one into nx
-    auto chunk = [&](int c, const ScanIn<NK>& in, ScanIn<NK>& nx) {
+    auto chunk = [&](int c, const ScanIn<NK>& in, ScanIn<NK>& nx) __attribute__((always_inline)) {
         constexpr int STEPS = 24 * NK + 12;                    // matrix instructions that bring loads with them
         constexpr int LONG = L_G, WORK = L_ALL + LONG;         // the four waves' 16-byte loads take the time of two matrix instructions, the others half
         static_assert(WORK <= 2 * STEPS);
@@ -895,6 +908,12 @@ void launch_inputs(hipStream_t st, const CogsDelta& a, int rows, int nseq, int m
     else hipLaunchKernelGGL(delta_inputs_any_kernel<true>, dim3(rows), dim3(256), 0, st, a);
 }
 
+template <int NK>
+void launch_scan(hipStream_t st, const CogsDelta& a, dim3 grid, int scan) {
+    if (a.pad) hipLaunchKernelGGL((delta_scan_kernel<NK, false>), grid, dim3(256), 0, st, a, scan);
+    else hipLaunchKernelGGL((delta_scan_kernel<NK, true>), grid, dim3(256), 0, st, a, scan);
+}
+
 bool sizes_ok(const CogsDelta& a) {
     return a.heads > 0 && a.kv_heads > 0 && a.heads % a.kv_heads == 0 && a.taps > 0 && a.dkp % 16 == 0 && a.dvp % 16 == 0 && a.dkp <= 512 &&
            a.dvp <= 2048 && a.vdim > 0 && a.vdim <= a.dvp && a.channels == 2 * a.kv_heads * a.dkp + a.heads * a.dvp && a.ldt % 4 == 0 && a.ldo % 4 == 0;
@@ -905,7 +924,17 @@ bool sizes_ok(const CogsDelta& a) {
 int cogs_k_delta_slots(int rows, int nseq) { return rows / CH + nseq; }
 size_t cogs_k_delta_rec_floats(int rows, int nseq, int heads) { return (size_t)cogs_k_delta_slots(rows, nseq) * heads * REC; }
 
-int cogs_k_delta_prompt(hipStream_t st, int dtype, const CogsDelta& a, int rows, int nseq, int max_new) {
+// Short sequences: zeros for whole chunks would be up to 32 times their bytes. Without them the scan masks its loads, 0.3 to 0.8 % of a long prompt's
+// time: 4 to 8 ns a chunk, and the zeros 0.08 us a sequence. Widths 2048, 4096, us, zeros / masks: 128 prompts of 2 tokens 2021 / 1992, 4323 / 4112; 300
+// rows that join 16 requests 1315 / 1276, 2578 / 2550, 32 requests 1511 / 1477, 3010 / 2955; one prompt of 4096 4948 / 4987, 12 147 / 12 190
+static bool zeros_to_the_end(int nseq, int max_new) {
+    if (g_cogs_debug.delta_zeros > 0) return g_cogs_debug.delta_zeros == 1;
+    return nseq == 1 || nseq * 512L <= max_new;
+}
+
+int cogs_k_delta_prompt(hipStream_t st, int dtype, const CogsDelta& delta, int rows, int nseq, int max_new) {
+    CogsDelta a = delta;
+    a.pad = zeros_to_the_end(nseq, max_new);
     if (!sizes_ok(a) || rows <= 0 || nseq <= 0 || nseq > 65535 || a.heads > 65535) return COGS_E_INVALID;
     if (a.slots != cogs_k_delta_slots(rows, nseq)) return COGS_E_INVALID;
     const int keep = (max_new < a.taps ? max_new : a.taps) * a.channels, tail = (keep + 1023) / 1024;
@@ -914,9 +943,9 @@ int cogs_k_delta_prompt(hipStream_t st, int dtype, const CogsDelta& a, int rows,
         hipLaunchKernelGGL(delta_chunk_kernel, dim3((max_new + CH - 1) / CH, a.heads, nseq), dim3(256), 0, st, a);
         const int scan = (a.heads + 7) / 8 * 8 * (a.dvp / 16);
         const dim3 grid(scan + (tail + 7) / 8 * 8, 1, nseq);      // (a multiple of 8: the heads of every sequence keep their XCDs)
-        if (a.dkp <= 64) hipLaunchKernelGGL(delta_scan_kernel<1>, grid, dim3(256), 0, st, a, scan);
-        else if (a.dkp <= 128) hipLaunchKernelGGL(delta_scan_kernel<2>, grid, dim3(256), 0, st, a, scan);
-        else hipLaunchKernelGGL(delta_scan_kernel<4>, grid, dim3(256), 0, st, a, scan);
+        if (a.dkp <= 64) launch_scan<1>(st, a, grid, scan);
+        else if (a.dkp <= 128) launch_scan<2>(st, a, grid, scan);
+        else launch_scan<4>(st, a, grid, scan);
     } else {
         hipLaunchKernelGGL(delta_inputs_any_kernel<false>, dim3(rows), dim3(256), 0, st, a);
         hipLaunchKernelGGL(delta_tail_kernel, dim3(tail, nseq), dim3(256), 0, st, a);

@@ -303,6 +303,7 @@ struct CogsDelta {
     float *q, *k, *kt, *v, *bg, *o, *rec;
     void* att; long ldo;                 // [rows][heads x dvp], in `dtype`
     const CogsSeq* seqs; const int* rowseq; const int* rowpos; long state_off;      // floats
+    bool pad = false;                    // set by cogs_k_delta_prompt: whole chunks are stored, with zeros past a sequence's end
 };
 int cogs_k_delta_slots(int rows, int nseq);      // chunks of 32 rows of all sequences, each on chunks of its own, at the most
 size_t cogs_k_delta_rec_floats(int rows, int nseq, int heads);

@@ -558,6 +558,35 @@ def test_tiles_of_chunks_from_every_convolution(dev, dim, vdim, conv):
     assert rms_err(out, lg[[130] * len(lens)]) < TOL[torch.float32]
 
 
+@pytest.mark.parametrize("dim,vdim,conv", [(32, 80, 1), (128, 48, 3), (64, 16, 6), (256, 32, 8), (48, 130, 9), (144, 32, 11), (128, 128, 4)])
+def test_tokens_past_the_end_as_zeros_or_masked(dev, dim, vdim, conv):
+    """what lies past a sequence's end in its last chunk, stored as zeros (few or long sequences) or not stored and masked (many short ones): the same bits in logits and
+    states, whatever was in the workspace. Ends at every token of a lane's four, on both sides of 16 and of 32; together, one by itself, behind cached tokens"""
+    from cogstream_amd import _lib as L
+    cfg = config([delta(heads=4, kv_heads=2, dim=dim, vdim=vdim, conv=conv, ff=None)], width=64)
+    e = engine(cfg, state(cfg), torch.float32)
+    toks = tokens(cfg, 200)
+    lens = [1, 2, 3, 4, 5, 7, 8, 9, 13, 15, 16, 17, 18, 21, 30, 31, 32, 33, 36, 48, 49, 63, 64, 65, 130]
+
+    def results(poison):
+        out = []
+        for batch in (lens, [3], [65], [1, 64]):
+            s = sequences(e)
+            for parts in ((0, 1), (1, 2), (2, 3)):
+                cut = [[0, n, n + 1 + n % 7, 150][k] for n in batch for k in range(4)]
+                if poison:
+                    e.handle.workspace("decoder", 1).fill_(255)
+                out.append(s.step([(i, toks[cut[4 * i + parts[0]]:cut[4 * i + parts[1]]], [0]) for i in range(len(batch))]))
+            out += [s.caches[i].state for i in range(len(batch))]
+        return out
+    want = results(False)
+    assert all(torch.isfinite(x).all() for x in want)
+    for form in (0, 1, 2):
+        with L.debug_switch("delta_zeros", form):
+            for poison in (False, True):
+                assert all(torch.equal(a, b) for a, b in zip(results(poison), want)), (form, poison)
+
+
 @pytest.mark.parametrize("dim", [64, 128, 256])
 def test_the_chunked_delta_rule_keeps_what_recurs(dev, dim):
     """a few (key, value) pairs that come again and again: the state already predicts every value, so what a chunk writes is the rounding of
