@@ -1083,7 +1083,8 @@ __global__ __launch_bounds__(64) void attn_rowwise_kernel(AttnArgs p, int HD, in
 }  // namespace
 
 int cogs_k_attention(hipStream_t st, const CogsAttn& a) {
-    if (a.next_read) *a.next_read = false;
+    for (bool* read : a.next_read)
+        if (read) *read = false;
     if (a.q_len <= 0 || a.hq <= 0 || a.hkv <= 0 || a.hq % a.hkv != 0) return COGS_E_INVALID;
     if (a.head_dim > 256 || a.head_dim % 8 != 0) return COGS_E_UNSUPPORTED;
     AttnArgs p;

@@ -50,7 +50,7 @@ struct VitAttnArgs {
 };
 
 constexpr float RESCALE_THR = 6.0f;
-constexpr int AHEAD_WGS = 64;      // workgroups that read weights ahead (one image: 32, 64, 96, 192: 1382, 1313, 1313, 1323 us)
+constexpr int AHEAD_WGS = 64;      // workgroups that read weights ahead (one image, one encoder by itself: 32, 64, 96, 192: 1382, 1313, 1313, 1323 us)
 
 #if defined(COGS_ATTN_STAMPS) || defined(COGS_PIPE_STAMPS) || defined(COGS_PHASE_STAMPS)   // diagnostic builds (tools/micro/attn_vit_micro.cpp)
 __device__ unsigned long long g_attn_stamps[8];
@@ -1014,10 +1014,15 @@ int cogs_k_attention_vit(hipStream_t st, const CogsAttn& a) {
         const int nlb = p.uniform_len - 64 * (nt - 1) > 32 ? 2 : 1;
         dim3 grid_ahead = grid;
         const long slice = (long)grid.x * grid.y;
-        if (p.next[1].W && p.xcd_order && (p.nseg + 1) * slice <= 256) {
-            grid_ahead.z += max(1, min((int)(AHEAD_WGS / slice), (int)(256 / slice) - p.nseg));
-            if (a.next_read) *a.next_read = true;
-            g_cogs_debug.weights_ahead_read += 1 + (p.next[0].W != nullptr);
+        if (p.next[0].W && p.xcd_order && (p.nseg + 1) * slice <= 256) {
+            const int ahead = max(1, min((int)(AHEAD_WGS / slice), (int)(256 / slice) - p.nseg));
+            if (ahead_bytes(p.next[0]) + ahead_bytes(p.next[1]) > ahead * slice * WEIGHTS_AHEAD_BYTES) p.next[1].W = nullptr;      // (the first one's in any case)
+            grid_ahead.z += ahead;
+            for (int i = 0; i < 2; ++i) {
+                if (!p.next[i].W) continue;
+                if (a.next_read[i]) *a.next_read[i] = true;
+                g_cogs_debug.weights_ahead_read += 1;
+            }
         }
 #define COGS_AV_LAUNCH(R_, B_) hipLaunchKernelGGL((attn_vit_pipe_kernel<72, R_, B_>), grid_ahead, dim3(256), 0, st, p)
         g_cogs_debug.attn_vit_last_end = r * 10 + (r ? nlb : 0);

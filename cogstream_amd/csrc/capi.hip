@@ -776,21 +776,21 @@ cogs_status VitRange::layer(int l) {
         else {
             a.cu_seqlens = cu; a.nseg = nframes; a.max_seqlen = max_seq;
             a.uniform_seqlen = uniform_seq;      // all frames alike (one video, or videos of one grid): see attn_vit.hip
-            if (!out.weights_read) a.next[0] = cogs_k_gemm_weights_ahead(out);
-            a.next[1] = cogs_k_gemm_weights_ahead(fc1);
+            a.next[0] = cogs_k_gemm_weights_ahead(fc1);
+            a.next_read[0] = &fc1.weights_read;
+            if (!out.weights_read) {
+                a.next[1] = cogs_k_gemm_weights_ahead(out);
+                a.next_read[1] = &out.weights_read;
+            }
         }
-        bool read = false;
-        a.next_read = &read;
         { PROF(COGS_PROF_ATTN); COGS_TRY(cogs_k_attention(st, a)); }
-        if (a.next[0].W) out.weights_read = read;
-        fc1.weights_read = read;
     }
     out.next = cogs_k_gemm_weights_ahead(fc2);
     out.next_read = &fc2.weights_read;
     { PROF(COGS_PROF_GEMM); COGS_TRY(cogs_k_gemm(st, out)); }
     if (!fold) { PROF(COGS_PROF_NORM); COGS_TRY(cogs_k_layernorm(st, dt, x, ln, L.ln2_g, L.ln2_b, (int)N, H, w.ln_eps)); }
     { PROF(COGS_PROF_GEMM); COGS_TRY(cogs_k_gemm(st, fc1)); }
-    if (l + 1 < w.layers) fc2.next = cogs_k_gemm_weights_ahead(qkv_product(l + 1));
+    if (l + 1 < w.layers && fc2.weights_read) fc2.next = cogs_k_gemm_weights_ahead(qkv_product(l + 1));
     fc2.next_read = &qkv_read;
     { PROF(COGS_PROF_GEMM); COGS_TRY(cogs_k_gemm(st, fc2)); }
     return COGS_OK;

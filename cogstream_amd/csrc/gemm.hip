@@ -1165,8 +1165,8 @@ static int best_mid_tile(int M, int N, int K, bool alone, float* time, int rows0
     }
     return best;
 }
-// Up to 576 rows: more of them leave few CUs idle and wait for their rows rather than for weights. Encoder and projector, us, with / without: 144 patches 1249
-// / 1275, 256 1313 / 1372, 512 1626 / 1686; 663 1784 / 1772, 924 2228 / 2238, 1024 2104 / 2094.
+// Up to 576 rows: more of them leave few CUs idle and wait for their rows rather than for weights. Encoder and projector, one by itself, us, with / without: 144
+// patches 1249 / 1275, 256 1313 / 1372, 512 1626 / 1686; 663 1784 / 1772, 924 2228 / 2238, 1024 2104 / 2094.
 CogsWeightsAhead cogs_k_gemm_weights_ahead(const CogsGemm& g) {
     constexpr int AHEAD_ROWS = 576;
     CogsWeightsAhead a;

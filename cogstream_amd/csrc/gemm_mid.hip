@@ -397,7 +397,9 @@ void launch(hipStream_t st, MidArgs& p, bool alone) {
     p.group0 = group_of(p.nbm0);
     p.ln_staged = (long)TM * p.ln_tiles * 8 <= KS * (TM + TN) * ROW_BYTES && ((long)p.M * p.ln_tiles) % 2 == 0;
     const int tiles = p.nbm * p.nbn + p.nbm0 * p.nbn0;
-    const int extra = !alone || p.rows0 != 0 ? 0 : p.next.W ? max(MID_CUS - tiles, 0) / 8 * 8 : p.hot ? 0 : read_ahead_workgroups(tiles);
+    const int free = max(MID_CUS - tiles, 0) / 8 * 8;
+    if (ahead_bytes(p.next) > free * WEIGHTS_AHEAD_BYTES) p.next.W = nullptr;
+    const int extra = !alone || p.rows0 != 0 ? 0 : p.next.W ? free : p.hot ? 0 : read_ahead_workgroups(tiles);
     if (extra == 0) p.next.W = nullptr;
     hipLaunchKernelGGL((gemm_mid_kernel<EPI, MI, NI, WM, WN, S, WPE, KS, IL>), dim3(tiles + extra), dim3(64 * WM * WN), lds, st, p);
 }

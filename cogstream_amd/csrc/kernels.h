@@ -66,7 +66,7 @@ int cogs_k_ln_finalize(hipStream_t st, const float* stat_part, int rows, int til
 
 struct CogsAttn {
     CogsWeightsAhead next[2];         // ViT kernel: read on the CUs that few workgroups leave idle
-    bool* next_read = nullptr;        // != null: set to whether both were
+    bool* next_read[2] = {nullptr, nullptr};      // != null: set to whether it was
     int dtype = 0;
     const void* Q = nullptr; const void* K = nullptr; const void* V = nullptr; void* O = nullptr;
     long ldq = 0, ldk = 0, ldv = 0, ldo = 0;
